@@ -25,7 +25,8 @@ LATENT = {1024: (8, 512, 256), 2048: (16, 1024, 512)}         # width -> heads, 
 GATED_FF = {1024: 4096, 2048: 8192}
 PLAIN_FF = {1024: 6144, 2048: 12288}
 EXPERTS = {1024: (32, 4, 4, 2, 512, 1024), 2048: (64, 4, 8, 4, 1024, 2048)}   # experts, top, groups, kept, width, shared width
-LR, BETAS, ADAM_EPS, DECAY = 5e-5, (0.9, 0.999), 1e-8, 0.01
+# the learning rate of a warm-up: full steps of a fresh AdamW move every weight by as much, whichever way rounding tips the tiny gradients
+LR, BETAS, ADAM_EPS, DECAY = 1e-6, (0.9, 0.999), 1e-8, 0.01
 LIMIT, ALPHA, CAP, TEMP, DIFF = 7.0, 1.702, 30.0, (0.1, 4096), 0.5
 
 
