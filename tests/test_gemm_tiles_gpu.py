@@ -1,0 +1,77 @@
+"""Products of more than 32 rows on every tile the launcher chooses from, at the sizes where a tile can go wrong: its edges, ragged
+rows and columns, a K that is no multiple of a stage, one stage only, fewer stages than the ring holds, odd numbers of stages for
+the two groups of a 64 x 64 workgroup.  Against fp64 on the bf16 operands."""
+import math
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+BF, DEV = torch.bfloat16, "cuda"
+
+
+def rnd(*shape, seed, scale=1.0):
+    g = torch.Generator(device=DEV).manual_seed(seed)
+    return (torch.randn(*shape, generator=g, device=DEV) * scale).to(BF)
+
+
+def close(got, want, x, w, extra=0.0):
+    """A bf16 result of an fp32 sum: half an ulp of the result (2^-9 of it, twice where it is rounded ahead of a sum too) and the
+    fp32 sum's own error, at most K 2^-24 of the terms' magnitudes; tiny results have the spacing 2^-133."""
+    K = x.shape[1]
+    bound = 2.0 ** -8 * want.abs() + extra + K * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T) + 1e-30
+    assert torch.isfinite(got).all()
+    worst = ((got.double() - want).abs() / bound).max()
+    assert worst <= 1, float(worst)
+
+
+#: rows, columns, K: 64 x 64 tiles (one and two groups), 128 x 128, 256 x 128, 256 x 192, 256 x 256, K split over workgroups
+SHAPES = [(33, 8, 8), (63, 64, 64), (64, 72, 72), (65, 200, 136), (127, 64, 192), (129, 520, 200), (512, 768, 768), (300, 2304, 760),
+          (1000, 776, 320), (2111, 1032, 448), (1665, 3080, 128), (4096, 768, 3072), (4100, 1000, 1024), (8000, 1024, 1600),
+          (3000, 2048, 2048), (8193, 1030, 64), (9000, 776, 832), (130, 768, 6144), (257, 1024, 4160), (700, 1024, 6144)]
+
+
+@pytest.mark.parametrize("M,N,K", SHAPES)
+def test_linear_on_every_tile(M, N, K):
+    from vyomai_amd import ops
+    x, w, b, r = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5), rnd(N, seed=3), rnd(M, N, seed=4)
+    y = ops.linear(x, w)
+    close(y, x.double() @ w.double().T, x, w)
+    y = ops.linear(x, w, b, residual=r)
+    product = x.double() @ w.double().T + b.double()
+    close(y, product + r.double(), x, w, 2.0 ** -8 * product.abs())      # (the product is staged in bf16 ahead of the residual)
+
+
+@pytest.mark.parametrize("M,N,K", [(64, 768, 768), (333, 3072, 768), (512, 3080, 136), (1100, 2304, 768)])
+def test_activation_and_its_saved_derivative_on_small_tiles(M, N, K):
+    from vyomai_amd import ops, _lib
+    x, w, b = rnd(M, K, seed=5), rnd(N, K, seed=6, scale=K ** -0.5), rnd(N, seed=7)
+    y = torch.empty(M, (N + 7) // 8 * 8, dtype=BF, device=DEV)[:, :N]
+    pre = torch.empty(M, (N + 7) // 8 * 8, dtype=BF, device=DEV)[:, :N]
+    ops.linear(x, w, b, act=_lib.ACT_GELU_ERF, pre_out=pre, out=y)
+    z = x.double() @ w.double().T + b.double()
+    close(pre, z, x, w)
+    zb = pre.double()                                       # the activation is of the staged bf16 value
+    want = 0.5 * zb * (1 + torch.erf(zb / math.sqrt(2)))
+    assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()       # 1e-5: the epilogue's fast erf
+
+
+@pytest.mark.parametrize("B,L,h,hk", [(3, 37, 12, 12), (1, 65, 12, 4), (5, 333, 12, 4), (2, 1000, 12, 12)])
+def test_rotary_heads_on_small_tiles(B, L, h, hk):
+    from vyomai_amd import ops
+    K, N, pos0 = 768, (h + 2 * hk) * 64, 3
+    x, w, b = rnd(B, L, K, seed=8), rnd(N, K, seed=9, scale=K ** -0.5), rnd(N, seed=10)
+    cos, sin = ops.rope_tables(64, pos0 + L, DEV)
+    q = torch.empty(B, h, L, 64, dtype=BF, device=DEV)
+    cache = torch.zeros(2, B, hk, pos0 + L + 2, 64, dtype=BF, device=DEV)
+    k, v = cache[0, :, :, pos0:pos0 + L], cache[1, :, :, pos0:pos0 + L]
+    ops.qkv_rope(x, w, b, h, hk, 64, cos, sin, pos0, q, k, v)
+    y = (x.double() @ w.double().T + b.double()).view(B, L, -1, 64).transpose(1, 2)
+    c, s = (t[pos0:pos0 + L].double() for t in (cos, sin))
+    turn = lambda t: torch.cat([t[..., :32] * c - t[..., 32:] * s, t[..., 32:] * c + t[..., :32] * s], -1)
+    size = y.abs().amax(-1, keepdim=True)
+    # rounded to bf16: the projection, both factors, both products and their sum -- 2^-9 of at most |a| + |b| each
+    for got, want in ((q, turn(y[:, :h])), (k, turn(y[:, h:h + hk])), (v, y[:, h + hk:])):
+        assert ((got.double() - want).abs() <= 8 * 2.0 ** -9 * size.amax()).all()
+    assert float(cache[:, :, :, :pos0].abs().max()) == 0 and float(cache[:, :, :, pos0 + L:].abs().max()) == 0

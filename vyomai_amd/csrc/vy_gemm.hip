@@ -1,11 +1,11 @@
 // GEMM family for the projection / feed-forward path:  Y[M,N] = epi(X[M,K] . W[N,K]^T)
 //
 // bf16 kernels (the product path): MFMA, fp32 accumulate, LDS-DMA staging, by size of M:
-//   * M > ~2304 (training, prefill): 256 x 192 tiles with the X operand in a three-deep ring (gemm_nt_bf16_x3m16_kernel) or
-//     256 x 256 two-stage tiles where N >= 3072 (gemm_nt_bf16_m16_kernel), both on mfma_f32_16x16x32_bf16, 8 waves, one
-//     workgroup per CU; gemm_nt_bf16_kernel is the same tile family on mfma_f32_32x32x16_bf16 (A/B knob, 32 x 128 fallback);
-//   * 32 < M <= ~2304: 128 x 128 tiles (two workgroups per CU) or ONE all-rows tile of 256 / 320 x 128 for 128 < M <= 320,
-//     split over K when the tile grid leaves CUs idle (gemm_nt_bf16_m16_splitk_kernel + gemm_splitk_finish_kernel);
+//   * M > 32: the tile is chosen by what the shape costs on it (pick_tiling): 256 x 256 (gemm_nt_bf16_m16_kernel, two stages),
+//     256 x 192 or 256 x 128 (gemm_nt_bf16_x3m16_kernel, X in a three-deep ring), 128 x 128 (two workgroups per CU), 64 x 64 with a
+//     three-deep ring (gemm_nt_bf16_small_kernel), or K split over workgroups (gemm_nt_bf16_m16_splitk_kernel +
+//     gemm_splitk_finish_kernel; one row tile of 256 / 320 for 128 < M <= 320); all on mfma_f32_16x16x32_bf16.
+//     gemm_nt_bf16_kernel is the same tile family on mfma_f32_32x32x16_bf16 (A/B knob, 32 x 128 fallback);
 //   * M <= 32 (decode): weight-streaming kernels without LDS staging (gemm_skinny*), M <= 4: one wave per output column
 //     (gemv_bf16_kernel); the decode driver's straight-line versions are in vy_decode.hip;
 //   * both operands are K-contiguous ("NT"), so both MFMA fragments are 16-byte row reads
@@ -259,10 +259,6 @@ __device__ unsigned long long vy_gemm_clk[6];   // cycles, ticks, launches, prol
 // same-process A/B timing; not part of include/vyom_hip.h).  -1 = the default selection.
 int g_chains = 1;   // vy_set_concurrent_chains: launch chains the caller runs side by side
 int g_gemm_variant = -2;
-inline bool vy_m16_on() {   // VY_GEMM_M16=0: the two-stage 32 x 32 x 16 kernels instead of the 16 x 16 x 32 defaults
-  static const int v = [] { const char* e = getenv("VY_GEMM_M16"); return e ? atoi(e) : 1; }();
-  return v != 0;
-}
 inline int vy_gemm_variant() {
   if (g_gemm_variant == -2) { const char* e = getenv("VY_GEMM_VARIANT"); g_gemm_variant = e ? atoi(e) : -1; }
   return g_gemm_variant;
@@ -511,7 +507,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
           }
         }
     };
-    constexpr bool PFK = PF_OK && PASSES == 1 && BM * BN == 256 * 192 && (RP * CPR) % NT == 0;   // kernels that prefetch (the 256 x 256 tile has no registers to spare: +5 % on FFN1 with them reserved)
+    constexpr bool PFK = PF_OK && PASSES == 1 && (BM * BN == 256 * 192 || BM * BN == 64 * 64) && (RP * CPR) % NT == 0;   // kernels that prefetch (the 256 x 256 tile has no registers to spare: +5 % on FFN1 with them reserved)
     constexpr int ITERS = PFK ? (RP * CPR) / NT : 1;
     bf16x8 pre8[ITERS];
     const bool pf_on = PFK && pf_ptr != nullptr && ep.vec_ok && m0 + BM <= M && n0 + BN <= N;   // workgroup-uniform
@@ -1085,6 +1081,138 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
+// 64 x 64 tiles for outputs that give the big tiles too few workgroups: KG groups of 4 waves (2 x 2, 32 x 32 outputs each), each
+// with a ring of NBUF stages of its own, of which NBUF - 1 are on their way (counted vmcnt); group g multiplies the k-slices
+// g, g + KG, ... and the groups' accumulators are added through LDS at the end, in the order of the groups.
+// Bound by the chain of stages (0.3 us each: barrier, LDS reads, 8 products a wave), so many workgroups per CU and, where there is
+// at most one, two groups in it.  512 x 768 x 768: 12.4 -> 7.4 us against K split over workgroups and a second launch;
+// 512 x 3072 x 768: 21.3 -> 10.1; 1056 x 2304 x 768: 21.7 -> 12.5; 264 x 2048 x 2048: 24.7 -> 10.9.  (Four groups: no faster than
+// two on any shape; a fourth stage: level.)
+// ------------------------------------------------------------------------------------------
+template <int KG, int NBUF, int EPI, int ACT, bool GRAD>
+__global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
+    const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
+    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob) {
+  constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
+  constexpr int TM = 2, TN = 2, PER = 2;               // 16 x 16 blocks and 1 KiB pieces of either operand per wave
+  constexpr int STAGE = (BM + BN) * ROWB, RING = NBUF * STAGE;
+  constexpr int LDS_BYTES = vy_cmax(vy_cmax(KG * RING, (KG - 1) * BM * BN * 4), epi_lds_bytes(BM, BN, EPI, 1));
+  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
+
+  const int lane = threadIdx.x & 63;
+  const int wave_all = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int grp = wave_all / NW, wave = wave_all % NW;
+  const int wm = wave / WGN, wn = wave % WGN;
+  int tile_m, tile_n;
+  const int tiles_m = gridDim.x / tiles_n;
+  if (tiles_m < tiles_n) {   // the smaller operand is the one that every XCD reads
+    const int wg = xcd_remap(blockIdx.x, gridDim.x);
+    tile_n = wg / tiles_m;
+    tile_m = wg - tile_n * tiles_m;
+  } else {
+    tile_of(blockIdx.x, gridDim.x, tiles_n, !(knob & 32), tile_m, tile_n);
+  }
+  const int m0 = tile_m * BM, n0 = tile_n * BN;
+  char* ring = smem + grp * RING;
+
+  const int lrow = lane >> 3, slot = lane & 7;
+  const bf16 *xsrc[PER], *wsrc[PER];
+  int kcol[PER];
+#pragma unroll
+  for (int t = 0; t < PER; ++t) {
+    const int R = (wave + NW * t) * 8 + lrow;
+    const int g = slot ^ ((R >> 1) & 7);
+    int gm = m0 + R; gm = gm < M ? gm : M - 1;
+    int gn = n0 + R; gn = gn < N ? gn : N - 1;
+    xsrc[t] = X + (int64_t)gm * ldx + g * 8;
+    wsrc[t] = W + (int64_t)gn * ldw + g * 8;
+    kcol[t] = g * 8;
+  }
+  const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
+  const int KT = (K + BK - 1) / BK;
+  // slice kt of both operands -> buffer buf of the group's ring (columns from K on: zeros; slices from KT on: all of it, so that
+  // every group issues the same number of pieces)
+  auto stage = [&](int kt, int buf) {
+    char* xb = ring + buf * STAGE;
+    const int k0 = kt * BK;
+#pragma unroll
+    for (int t = 0; t < PER; ++t) {
+      const bool in = k0 + kcol[t] < K;
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(in ? xsrc[t] + k0 : zero), (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(in ? wsrc[t] + k0 : zero),
+                                       (VY_LDS void*)(xb + BM * ROWB + (wave + NW * t) * 1024), 16, 0, 0);
+    }
+  };
+
+  f32x4 acc[TN][TM];
+#pragma unroll
+  for (int i = 0; i < TN; ++i)
+#pragma unroll
+    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+
+  const int r16 = lane & 15, kq = lane >> 4, fsw = (r16 >> 1) & 7;
+  unsigned xa[2], wa[2];
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+    const int coff = (((ks * 4 + kq) ^ fsw) << 4);
+    xa[ks] = vy_lds_addr(ring) + (wm * 16 * TM + r16) * ROWB + coff;
+    wa[ks] = vy_lds_addr(ring) + BM * ROWB + (wn * 16 * TN + r16) * ROWB + coff;
+  }
+  const int n_it = (KT + KG - 1) / KG;
+#pragma unroll
+  for (int i = 0; i < NBUF - 1; ++i)
+    if (i < n_it) stage(i * KG + grp, i);
+  int buf = 0;
+  for (int it = 0; it < n_it; ++it) {
+    // the slice has landed for this wave, NBUF - 2 younger ones may still be on their way (near the end: wait for all) ...
+    if (it + NBUF - 2 < n_it) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER * (NBUF - 2)) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    // ... and, behind the barrier, for every wave; every wave has also finished with the buffer that is filled next
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (it + NBUF - 1 < n_it) stage((it + NBUF - 1) * KG + grp, buf == 0 ? NBUF - 1 : buf - 1);
+    const unsigned boff = (unsigned)buf * STAGE;
+    bf16x8 wf[2][TN], xf[2][TM];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+      vy_static_for<TN>([&](auto i_c) { constexpr int i = decltype(i_c)::value; wf[ks][i] = vy_lds_read128_off<i * 16 * ROWB>(wa[ks] + boff); });
+      vy_static_for<TM>([&](auto j_c) { constexpr int j = decltype(j_c)::value; xf[ks][j] = vy_lds_read128_off<j * 16 * ROWB>(xa[ks] + boff); });
+    }
+    vy_lgkm_wait<TN + TM>(wf[0][0], wf[0][1], xf[0][0], xf[0][1]);
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[0][i], xf[0][j], acc[i][j], 0, 0, 0);
+    vy_lgkm_wait<0>(wf[1][0], wf[1][1], xf[1][0], xf[1][1]);
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[1][i], xf[1][j], acc[i][j], 0, 0, 0);
+    buf = buf + 1 == NBUF ? 0 : buf + 1;
+  }
+  // what follows reuses the buffers: every wave is through with its reads
+  __syncthreads();
+  if constexpr (KG > 1) {
+    f32x4* part = reinterpret_cast<f32x4*>(smem) + (threadIdx.x & 255);
+    if (grp)
+#pragma unroll
+      for (int i = 0; i < TN * TM; ++i) part[((grp - 1) * TN * TM + i) * 256] = acc[i / TM][i % TM];
+    __syncthreads();
+    if (grp) return;   // (a barrier waits for the waves that are left)
+#pragma unroll
+    for (int g = 0; g < KG - 1; ++g)
+#pragma unroll
+      for (int i = 0; i < TN * TM; ++i) {
+        const f32x4 v = part[(g * TN * TM + i) * 256];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) acc[i / TM][i % TM][r] += v[r];
+      }
+    __syncthreads();
+  }
+  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq);
+}
+
+// ------------------------------------------------------------------------------------------
 // Split-K for mid-size M (32 < M <= ~2304 rows: a 264-row PaliGemma prefill, the 2112 rows of a captioning decoder).
 // A 264 x 2048 output is 48 tiles of 128 x 128 -- 48 of 256 CUs -- and with K = 16384 (Gemma's down-projection) each of
 // them walks 256 k-stages alone.  Here the K range is cut into S slices: tiles x S workgroups (~two per CU) each run the
@@ -1287,51 +1415,96 @@ struct WsEntry { hipStream_t st; void* p; int64_t bytes; };
 WsEntry g_ws[16];
 int g_ws_n = 0;
 std::mutex g_ws_mu;
-inline float* splitk_ws(hipStream_t st, int64_t need) {
+// scratch of a stream (vy_workspace_set): its size and, asked for by `need`, its address
+inline float* splitk_ws(hipStream_t st, int64_t need, int64_t* bytes) {
   std::lock_guard<std::mutex> lk(g_ws_mu);
   for (int i = 0; i < g_ws_n; ++i)
-    if (g_ws[i].st == st) return g_ws[i].bytes >= need ? (float*)g_ws[i].p : nullptr;
+    if (g_ws[i].st == st) {
+      if (bytes) *bytes = g_ws[i].bytes;
+      return g_ws[i].bytes >= need ? (float*)g_ws[i].p : nullptr;
+    }
+  if (bytes) *bytes = 0;
   return nullptr;
 }
-// slices for a tile grid: `target` workgroups in all (two per CU for the 128 x 128 tiles, one for the all-rows tiles), at least
-// two 64-deep stages per slice
+
+// ------------------------------------------------------------------------------------------
+// Tiles of a product of more than 32 rows.  What a shape costs depends on how its tiles fill the 256 CUs as much as on the tile's
+// own rate: 8192 x 2048 with K = 12288 is 352 tiles of 256 x 192 -- two rounds, the second a third full, 459 us -- or 256 tiles of
+// 256 x 256: 313 us; 8000 x 1024, K = 6144: 124 us on 256 x 192, 152 us on 256 x 256, 100 us on 256 x 128 (250 tiles).  So the
+// launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below; the constants
+// are fits to launches of 40 shapes from 48 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
+// output alone and so moves no choice).
+// ------------------------------------------------------------------------------------------
+enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_128x128_SPLIT, T_256x128_SPLIT, T_320x128_SPLIT };
+constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 128, 256, 320};
+constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 128, 128, 128};
+constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 256, 512, 512};
+struct Tiling { TileKind kind; int slices; };
+
+// slices of K for `tiles` workgroups per slice: a power of two (one slice per group of XCDs, splitk_block_of), about `target`
+// workgroups in all, at least two stages in a slice, none empty
 inline int splitk_slices(int64_t tiles, int KT, int target) {
-  static const int on = [] { const char* e = getenv("VY_SPLITK"); return e ? atoi(e) : 1; }();
-  // (measured, same box: 2 stages per slice at least -- configs[4] prefill 7.09 -> 6.88 ms, configs[3] step 19.1 -> 18.5 ms against 4)
-  static const int min_stages = [] { const char* e = getenv("VY_SPLITK_MIN_STAGES"); return e ? atoi(e) : 2; }();
-  if (!on || tiles * 3 >= target * 2 || g_chains != 1) return 1;
   int S = (int)((target + tiles / 2) / tiles);
-  if (S > KT / min_stages) S = KT / min_stages;
+  if (S > KT / 2) S = KT / 2;
   if (S > 16) S = 16;
   if (S < 2) return 1;
   int p2 = 2;
-  while (p2 * 2 <= S) p2 *= 2;   // a power of two: one slice per group of XCDs (splitk_block_of)
-  S = p2;
-  const int per = (KT + S - 1) / S;
-  return (KT + per - 1) / per;   // no empty slice
+  while (p2 * 2 <= S) p2 *= 2;
+  const int per = (KT + p2 - 1) / p2;
+  return (KT + per - 1) / per;
 }
 
-// mid-size M launch on BM x BN tiles: split over K when the tile grid leaves CUs idle and the stream has a workspace
+inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes) {
+  const int KT = (int)vy_cdiv(K, BK);
+  Tiling best{T_256x256, 1};
+  double least = 1e30;
+  auto offer = [&](TileKind kind, int slices, double us) {
+    if (us < least) { least = us; best = Tiling{kind, slices}; }
+  };
+  auto tiles_of = [&](TileKind k) { return vy_cdiv(M, TILE_M[k]) * vy_cdiv(N, TILE_N[k]); };
+  // `fixed` per round, `stage` per stage of a round; the stages of a last round that leaves CUs idle run up to 30 % faster
+  auto one_shot = [&](TileKind k, int per_cu, double launch, double fixed, double stage) {
+    const double r = (double)tiles_of(k) / (chip * per_cu), whole = (double)(int64_t)r, part = r - whole;
+    offer(k, 1, launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * stage * KT);
+  };
+  one_shot(T_256x256, 1, 2.5, 7.0, 1.55);
+  one_shot(T_256x192, 1, 2.3, 5.5, 1.30);
+  one_shot(T_256x128, 1, 4.5, 4.1, 0.97);
+  if (tiles_of(T_128x128) <= chip) offer(T_128x128, 1, 8.5 + 0.72 * KT);
+  else one_shot(T_128x128, 2, 3.5, 5.0, 1.0);     // (two of them share a CU)
+  const double load = (double)tiles_of(T_64x64) / chip;
+  offer(T_64x64, 1, 4.3 + KT * (0.22 * load > 0.295 ? 0.22 * load : 0.295));
+  offer(T_64x64_TWICE, 1, 3.0 + (double)vy_cdiv(tiles_of(T_64x64_TWICE), chip) * (2.2 + 0.44 * ((KT + 1) / 2)));
+  // K over several workgroups: the partial sums' way through memory (about 8 TB/s there and back: mostly the Infinity Cache) and a second launch.
+  // 128 < M <= 320: one row tile holds every row, so a weight crosses L2 -> LDS once
+  if (chip == 256 && ws_bytes > 0) {
+    const TileKind k = M > 256 && M <= 320 ? T_320x128_SPLIT : M > 128 && M <= 256 ? T_256x128_SPLIT : T_128x128_SPLIT;
+    const int64_t tiles = tiles_of(k);
+    const int S = splitk_slices(tiles, KT, k == T_128x128_SPLIT ? 448 : 256);
+    const double bytes = 4.0 * S * tiles * TILE_M[k] * TILE_N[k];
+    if (S > 1 && bytes <= (double)ws_bytes) {
+      const int per = (KT + S - 1) / S;
+      const double stage = k == T_128x128_SPLIT ? (tiles * S > chip ? 1.0 : 0.72) : 1.2 * TILE_M[k] / 256;
+      offer(k, S, 7.5 + (double)vy_cdiv(tiles * S, (int64_t)chip * (k == T_128x128_SPLIT ? 2 : 1)) * per * stage + 2 * bytes / 8e6);
+    }
+  }
+  return best;
+}
+
+// BM x BN tiles with K cut into S slices, whose partial sums the second launch adds up in the workspace's order
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD>
-void launch_mid(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K,
-                const EpiPlain<bf16>& ep, const EpiQkv<bf16>& eq, hipStream_t st, int target, int rot) {
-  constexpr int NT = 64 * WGM * WGN;
+void launch_split(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K, int S,
+                  const EpiPlain<bf16>& ep, const EpiQkv<bf16>& eq, hipStream_t st) {
   const int tn = (int)vy_cdiv(N, BN), tm = (int)vy_cdiv(M, BM);
   const int KT = (int)vy_cdiv(K, 64);
   const int tiles = tm * tn;
-  const int S = splitk_slices(tiles, KT, target);
-  float* ws = S > 1 ? splitk_ws(st, (int64_t)S * tiles * BM * BN * 4) : nullptr;
-  if (ws) {
-    const int per = (KT + S - 1) / S;
-    hipLaunchKernelGGL((gemm_nt_bf16_m16_splitk_kernel<BM, BN, WGM, WGN>), dim3(tiles * S), dim3(NT), 0, st, X, ldx, W, ldw,
-                       (int)M, (int)N, (int)K, tn, tiles, S, per, ws);
-    constexpr int TMB = BM / (16 * WGM);
-    hipLaunchKernelGGL((gemm_splitk_finish_kernel<BM, BN, WGM, WGN, EPI, ACT, GRAD>), dim3(tiles * WGM * WGN * TMB), dim3(64), 0,
-                       st, ws, (int)M, (int)N, tn, tiles, S, ep, eq);
-  } else {
-    hipLaunchKernelGGL((gemm_nt_bf16_m16_kernel<BM, BN, WGM, WGN, EPI, ACT, GRAD>), dim3(tiles), dim3(NT), 0,
-                       st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot);
-  }
+  float* ws = splitk_ws(st, (int64_t)S * tiles * BM * BN * 4, nullptr);
+  const int per = (KT + S - 1) / S;
+  hipLaunchKernelGGL((gemm_nt_bf16_m16_splitk_kernel<BM, BN, WGM, WGN>), dim3(tiles * S), dim3(64 * WGM * WGN), 0, st, X, ldx, W, ldw,
+                     (int)M, (int)N, (int)K, tn, tiles, S, per, ws);
+  constexpr int TMB = BM / (16 * WGM);
+  hipLaunchKernelGGL((gemm_splitk_finish_kernel<BM, BN, WGM, WGN, EPI, ACT, GRAD>), dim3(tiles * WGM * WGN * TMB), dim3(64), 0,
+                     st, ws, (int)M, (int)N, tn, tiles, S, ep, eq);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -2044,7 +2217,6 @@ template <int EPI, int ACT, bool GRAD>
 int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N,
                 int64_t K, const EpiPlain<bf16>& ep, const EpiQkv<bf16>& eq, hipStream_t st) {
   static const int rot = [] { const char* e = getenv("VY_GEMM_ROT"); return e ? atoi(e) : 0; }();  // rotated k order: measured 1-5 % slower
-  static const int mid_tiles = [] { const char* e = getenv("VY_GEMM_MID"); return e ? atoi(e) : 1; }();
   static const int gemv_on = [] { const char* e = getenv("VY_GEMV"); return e ? atoi(e) : 1; }();
   static const int skinny16_on = [] { const char* e = getenv("VY_SKINNY16"); return e ? atoi(e) : 1; }();
   static const int64_t skinny_max_n = [] { const char* e = getenv("VY_SKINNY_MAXN"); return e ? (int64_t)atoll(e) : (int64_t)8192; }();   // wider (the vocabulary): 32 x 128 tiles with X staged once per workgroup -- 15.5 vs 31.1 us at N = 50265
@@ -2066,49 +2238,36 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     const int tn = (int)vy_cdiv(N, 128), tm = (int)vy_cdiv(M, 32);
     hipLaunchKernelGGL((gemm_nt_bf16_kernel<32, 128, 1, 4, EPI, ACT, GRAD>), dim3(tm * tn), dim3(256), 0,
                        st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot);
-  } else if (M <= 1024 || (mid_tiles && vy_cdiv(M, 256) * vy_cdiv(N, 192) * g_chains < 160)) {
-    // mid-size M: also whenever the 256 x 192 grid would leave more than a third of the CUs without a tile
-    // (M = 2112 rows of a captioning decoder x N = 768: 36 tiles of 256 x 192, 102 of 128 x 128)
-    const int tn = (int)vy_cdiv(N, 128), tm = (int)vy_cdiv(M, 128);
-    static const int mid16 = [] { const char* e = getenv("VY_GEMM_MID16"); return e ? atoi(e) : 1; }();
-    // 128 < M <= 320 (a 256-patch vision tower, a 264-row PaliGemma prefill): ONE row tile holds every row, so each weight
-    // element crosses L2 -> LDS once per launch and the 8 rows past 256 do not cost a third row of 128 x 128 tiles
-    // (all-rows tiles of 256 or 320 x 128, 8 waves, one workgroup per CU; VY_GEMM_ROWS=0: the 128 x 128 tiles)
-    static const int rows_on = [] { const char* e = getenv("VY_GEMM_ROWS"); return e ? atoi(e) : 1; }();
-    if (mid16 && rows_on && M > 128 && M <= 320) {
-      if (M <= 256) launch_mid<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, ep, eq, st, 256, rot);
-      else launch_mid<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, ep, eq, st, 256, rot);
-    } else if (mid16)
-      launch_mid<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, ep, eq, st, 448, rot);
-    else
-      hipLaunchKernelGGL((gemm_nt_bf16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>), dim3(tm * tn), dim3(256), 0,
-                         st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot);
   } else {
-    const int tn = (int)vy_cdiv(N, 192), tm = (int)vy_cdiv(M, 256);
-    // Large M.  256 x 192 tiles divide N in {768, 2304} x M = 16384 into whole multiples of the 256 CUs (X operand in a
-    // three-deep ring: gemm_nt_bf16_x3m16_kernel); 256 x 256 (fewer L2 bytes per FLOP) where N is wide enough for whole
-    // rounds anyway (FFN1, the dgrad of FFN2, the vocabulary projection).  Both on mfma_f32_16x16x32_bf16.
-    // VY_GEMM_VARIANT (A/B runs in one process, tools/exp_gemm.py): 8 / 9 force the 256 x 256 / 256 x 192 tiles of the
-    // two-stage 32 x 32 x 16 kernel, 40 / 41 force the two default kernels whatever N.  The experimental kernels of rounds
-    // 1-2 (persistent pipelined epilogue, two 4-wave workgroups per CU, 4- and 5-slot rings of 32-wide slices, the
-    // 32 x 32 x 16 X-ring) measured level or behind these on every box and were removed in round 3.
-    const int var = vy_gemm_variant();
-    const bool wide = (N >= 3072);
-    if (var == 8 || (var != 9 && var != 40 && var != 41 && !vy_m16_on() && wide)) {
-      const int tn2 = (int)vy_cdiv(N, 256);
-      hipLaunchKernelGGL((gemm_nt_bf16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>), dim3(tm * tn2), dim3(512), 0,
-                         st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn2, ep, eq, rot);
-    } else if (var == 9 || (var != 40 && var != 41 && !vy_m16_on())) {
-      hipLaunchKernelGGL((gemm_nt_bf16_kernel<256, 192, 4, 2, EPI, ACT, GRAD>), dim3(tm * tn), dim3(512), 0,
-                         st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot);
-    } else if (var == 41 || (var != 40 && wide)) {
-      const int tn2 = (int)vy_cdiv(N, 256);
-      hipLaunchKernelGGL((gemm_nt_bf16_m16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>), dim3(tm * tn2), dim3(512), 0,
-                         st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn2, ep, eq, rot);
-    } else {
-      hipLaunchKernelGGL((gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>), dim3(tm * tn), dim3(512), 0,
-                         st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot);
+    int var = vy_gemm_variant();   // 8 / 9: the 256 x 256 / 256 x 192 tiles of the 32 x 32 x 16 kernel (tests, A/B runs); -1: by cost
+    if (EPI != 0 || GRAD || M < 1025) var = -1;
+    const int chip = 256 / g_chains;
+    Tiling t{};
+    if (var < 0) {
+      int64_t ws_bytes;
+      splitk_ws(st, 0, &ws_bytes);
+      t = pick_tiling(M, N, K, chip, ws_bytes);
     }
+    const int bm = var >= 0 ? 256 : TILE_M[t.kind], bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
+    const int tn = (int)vy_cdiv(N, bn), tiles = (int)vy_cdiv(M, bm) * tn, threads = var >= 0 ? 512 : TILE_THREADS[t.kind];
+#define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot)
+    if (var >= 0) {
+      if constexpr (EPI == 0 && !GRAD) {
+        if (var == 8) VY_TILES(gemm_nt_bf16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>);
+        else VY_TILES(gemm_nt_bf16_kernel<256, 192, 4, 2, EPI, ACT, GRAD>);
+      }
+    } else switch (t.kind) {
+      case T_256x256: VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>); break;
+      case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>); break;
+      case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, EPI, ACT, GRAD>); break;
+      case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
+      case T_64x64: VY_TILES(gemm_nt_bf16_small_kernel<1, 3, EPI, ACT, GRAD>); break;
+      case T_64x64_TWICE: VY_TILES(gemm_nt_bf16_small_kernel<2, 3, EPI, ACT, GRAD>); break;
+      case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
+      case T_256x128_SPLIT: launch_split<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
+      case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
+    }
+#undef VY_TILES
   }
   return 0;
 }
