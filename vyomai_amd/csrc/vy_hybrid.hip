@@ -19,6 +19,10 @@ int vy_parallel_decode(const vy_hybrid_plan* p, const vy_hybrid_layer* L, const 
 int vy_dec_gemv1_act(const void* x, const void* w, const void* bias, int act, float act_arg, void* y, int N, int K, hipStream_t st);
 int vy_rows_linear(const void* x, const void* w, const void* bias, int act, float act_arg, void* y, int64_t ldy, int64_t M, int64_t N,
                    int64_t K, hipStream_t st);
+int vy_rows_parts(const void* x, const void* w, float* parts, int64_t M, int64_t N, int64_t K, hipStream_t st);
+int vy_residual_norm_parts(float* x, int64_t ldx, const float* parts, int slices, const float* w_post, const float* w_pre, float eps,
+                           void* h, int64_t ldh, int64_t M, int64_t N, int64_t NP, int rms, int* advance, const int* slots, int n_adv,
+                           hipStream_t st);
 int vy_dec_gemv1_gated(const void* x, const void* wgu, void* y, int I, int K, int act, int prescaled, float eps, hipStream_t st);
 int vy_gemv_gated(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* norm_w, float eps, void* y, int64_t ldy,
                   int64_t M, int64_t I, int64_t K, int act, void* stream);
@@ -74,6 +78,9 @@ int product(const vy_hybrid_plan* p, const void* x, const void* w, void* y, int6
   return vy_linear_fwd(x, K, w, K, bias, nullptr, 0, y, ldy, nullptr, p->B, N, K, act, p->dtype, stream);
 }
 
+constexpr int MOST_PARTS = 8;   // of vy_rows_parts
+int64_t parts_bytes(const vy_hybrid_plan* p) { return p->dtype == VY_BF16 && p->B >= 5 && p->B <= 32 ? MOST_PARTS * (int64_t)p->B * p->dp * 4 : 0; }
+
 // packed [gate | up] rows -> activation rows
 int activation(const vy_hybrid_plan* p, const vy_hybrid_layer& L, const void* gu, int64_t ldg, void* act, int64_t lda, void* stream) {
   if (L.clamped) return vy_clamped_act_fwd(gu, ldg, act, lda, p->B, L.ff, L.limit, L.alpha, p->dtype, stream);
@@ -99,7 +106,7 @@ extern "C" int64_t vy_hybrid_ws_bytes(const vy_hybrid_plan* p) {
   const int64_t e = p->dtype == VY_BF16 ? 2 : 4, B = p->B;
   return up(B * p->dp * 4) + 2 * up(B * p->dp * e) + up(B * s.in * e) + up(B * s.q * e) + up(B * s.cq * e) +
          up(B * s.ao * e) + up(B * s.o * e) + up(B * s.gu * e) + up(B * s.ff * e) + up(s.mix_ws) + up(B * s.top * p->dp * e) +
-         3 * up(B * s.top * 4) + up(s.moe_ws) + up(B * s.values * e);
+         3 * up(B * s.top * 4) + up(s.moe_ws) + up(B * s.values * e) + up(parts_bytes(p));
 }
 
 extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* ids, const int32_t* slots, int32_t* lengths,
@@ -129,12 +136,22 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
   float* ew = (float*)take(B * s.top * 4);
   void* ews = take(s.moe_ws);
   void* values = take(B * s.values * e);
+  float* parts = (float*)take(parts_bytes(p));
   const vy_hybrid_layer* values_of = nullptr;   // the layer that filled them
   int rc;
   auto norm = [&](const void* yy, const vy_routed_rows* routed, const float* post, const float* pre, bool last) {
     return vy_residual_norm_ex(x, dp, yy, dp, p->embed, dp, yy || routed ? nullptr : ids, p->vocab, p->err, p->embed_scale, routed,
                                post, p->eps, pre, p->eps, h, dp, B, p->d, dp, p->rms, last ? lengths : nullptr, slots,
                                last ? (int)B : 0, p->dtype, stream);
+  };
+  // the stream += norm(in W^T), then its next norm: with few rows the product leaves slices that the norm adds up
+  auto into_stream = [&](const void* xin, const void* weight, int64_t K, const float* post, const float* pre, bool last) {
+    const int n = parts_bytes(p) ? vy_rows_parts(xin, weight, parts, B, dp, K, (hipStream_t)stream) : 0;
+    if (n)
+      return vy_residual_norm_parts(x, dp, parts, n, post, pre, p->eps, h, dp, B, p->d, dp, p->rms, last ? lengths : nullptr, slots,
+                                    last ? (int)B : 0, (hipStream_t)stream);
+    const int bad = product(p, xin, weight, y, dp, dp, K, stream);
+    return bad ? bad : norm(y, nullptr, post, pre, last);
   };
   if ((rc = norm(nullptr, nullptr, nullptr, p->layers[0].norm1, false))) return rc;
   for (int l = 0; l < p->num_layers; ++l) {
@@ -209,25 +226,31 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
       if ((rc = norm(y, routed, L.norm1b, next, last))) return rc;
       continue;
     }
-    if ((rc = product(p, ao, L.w_o, y, dp, dp, nv, stream))) return rc;
     if (!L.ff && !L.moe) {
-      if ((rc = norm(y, nullptr, L.norm1b, next, last))) return rc;
+      if ((rc = into_stream(ao, L.w_o, nv, L.norm1b, next, last))) return rc;
       continue;
     }
     // few tokens: the choice of experts comes with the residual sum
     bool chosen = false;
     if (L.moe) {
+      if ((rc = product(p, ao, L.w_o, y, dp, dp, nv, stream))) return rc;
       rc = vy_moe_few(L.moe, nullptr, 0, B, nullptr, nullptr, 0, nullptr, 0, p->dtype, stream);
       if (rc == VY_OK)
         rc = vy_residual_route(x, dp, y, dp, L.norm1b, L.norm2, p->eps, h, dp, B, p->d, dp, p->rms, L.moe, eids, ew, p->dtype, stream);
       if (rc && rc != VY_ERR_UNSUPPORTED) return rc;
       chosen = rc == VY_OK;
+      if (!chosen && (rc = norm(y, nullptr, L.norm1b, L.norm2, false))) return rc;
+    } else if ((rc = into_stream(ao, L.w_o, nv, L.norm1b, L.norm2, false))) {
+      return rc;
     }
-    if (!chosen && (rc = norm(y, nullptr, L.norm1b, L.norm2, false))) return rc;
     if (L.ff) {
       if (L.w_up) rc = product(p, h, L.w_up, act, L.ff, L.ff, dp, stream, nullptr, p->act);
       else rc = gated(p, L, h, gu, act, stream);
       if (rc) return rc;
+      if (!L.moe) {
+        if ((rc = into_stream(act, L.w_down, L.ff, L.norm2b, next, last))) return rc;
+        continue;
+      }
       if ((rc = product(p, act, L.w_down, y, dp, dp, L.ff, stream))) return rc;
     }
     if (chosen) {

@@ -82,7 +82,7 @@ __device__ __forceinline__ float finish(const Dense& a, float v, int n) {
 
 // rows 16 NT tile .. + 16 NT - 1 of W against all of X
 template <int MB, int NW = 4, int NT = 1>
-__device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile) {
+__device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int K) {   // K: columns of x and w that count
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const bf16* ws[NT];
 #pragma unroll
@@ -91,7 +91,7 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile) {
 #pragma unroll
   for (int j = 0; j < MB; ++j) xs[j] = a.x + (int64_t)min(16 * j + r16, a.M - 1) * a.ldx + 8 * kq;
   f32x4 acc[NT][MB];
-  stream<NT, MB, true, NW>(ws, xs, a.K, acc, red);
+  stream<NT, MB, true, NW>(ws, xs, K, acc, red);
   if (threadIdx.x >= 64) return;
 #pragma unroll
   for (int i = 0; i < NT * MB; ++i) {
@@ -114,6 +114,9 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile) {
     }
   }
 }
+
+template <int MB, int NW = 4, int NT = 1>
+__device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile) { dense<MB, NW, NT>(a, red, tile, a.K); }
 
 // ---- one row of X: a wave per two weight rows ---------------------------------------------------
 // Whole 1 KiB pieces of a row per instruction and no sharing between waves: many small, even pieces of work, which a single

@@ -11,6 +11,17 @@ __global__ __launch_bounds__(64 * NW) void rows_linear_kernel(Dense a) {
   vy_rows::dense<MB, NW, NT>(a, red, blockIdx.x);
 }
 
+// K cut into slices of `len` columns: fp32 partial sums [slice][M][N]
+template <int MB, int NT>
+__global__ __launch_bounds__(256) void rows_parts_kernel(Dense a, int len, int tiles) {
+  __shared__ f32x4 red[vy_rows::RED<NT, MB>];
+  const int slice = blockIdx.x / tiles, tile = blockIdx.x - slice * tiles, k0 = slice * len;
+  a.x += k0;
+  a.w += k0;
+  a.y = (float*)a.y + (int64_t)slice * a.M * a.N;
+  vy_rows::dense<MB, 4, NT>(a, red, tile, min(len, a.K - k0));
+}
+
 template <int MB>
 void rows_go(const Dense& a, hipStream_t st) {
   const unsigned tiles = (unsigned)((a.N + 15) / 16);
@@ -33,4 +44,23 @@ int vy_rows_linear(const void* x, const void* w, const void* bias, int act, floa
   else rows_go<2>(a, st);
   VY_CHECK_LAUNCH("vy_rows_linear");
   return VY_OK;
+}
+
+// internal (vy_hybrid.hip): the product of a sublayer's output, whose rows vy_residual_norm_parts adds to the stream: fp32 partial sums
+// parts[slice][M][N] of K cut into that many slices (returned; 0: other sizes).  A product with as few columns as the stream has 32
+// or 64 workgroups of 32 columns, and what one CU takes in (25 to 40 GB/s) sets its time; slices bring the workgroups to 256, and
+// wider tiles halve the times x is read.  32 rows, 1024 x 6144: 23.3 -> 7.7 us; 2048 x 12288: 43.2 -> 19.8; 1024 x 1024: 6.1 -> 4.4;
+// 8 rows: 13.3 -> 5.7, 24.8 -> 14.6, 4.2 -> 4.6 (weights from HBM).  A slice keeps at least 128 columns: 8 waves' lines.
+int vy_rows_parts(const void* x, const void* w, float* parts, int64_t M, int64_t N, int64_t K, hipStream_t st) {
+  if (M < 5 || M > 32 || N < 512 || N > 4096 || K > INT32_MAX || K < 1024 || K % 8 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
+      (uintptr_t)parts % 16)
+    return 0;
+  const int slices = N <= 1024 ? 8 : N <= 2048 ? (K >= 8192 ? 8 : 4) : 2;
+  const int len = (int)((K + slices - 1) / slices + 63) / 64 * 64;
+  if ((slices - 1) * (int64_t)len >= K) return 0;
+  const int tiles = (int)((N + 31) / 32);
+  const Dense a{(const bf16*)x, K, (int)M, (const bf16*)w, (int)N, (int)K, parts, N, 1, nullptr, VY_ACT_NONE, 0.f};
+  if (M <= 16) hipLaunchKernelGGL((rows_parts_kernel<1, 2>), dim3(tiles * slices), dim3(256), 0, st, a, len, tiles);
+  else hipLaunchKernelGGL((rows_parts_kernel<2, 2>), dim3(tiles * slices), dim3(256), 0, st, a, len, tiles);
+  return slices;
 }
