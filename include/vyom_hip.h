@@ -147,6 +147,28 @@ int vy_layernorm_fwd(const void* x, int64_t ldx, const void* gamma, const void* 
                      int64_t ldy, float* mean, float* rstd, int64_t M, int64_t N, float eps,
                      int dtype, void* stream);
 
+/* vy_text_layer_fwd: one post-LN layer of the text and vision models without gradients, the calls above in a row:
+ *   a = LN1(attention(x Wqkv^T + bqkv) Wo^T + bo + x) ;  y = LN2(act(a W1^T + b1) W2^T + b2 + x)
+ * replaces: EncoderLayer / DecoderLayer.forward (VyomAI/models/encoder.py:60-64, models/decoder.py:241-250,
+ *   models/vision_encoder.py:49-53).  x and y are [B][L][h dh], contiguous, weights [out][in] contiguous.  New keys and values are
+ * written to k_new / v_new ([B][hk][L][dh] by the strides), attention reads S keys from k / v; mask_kind, start_pos and keypad as for
+ * vy_attn_fwd (no additive mask); L = 1 without a mask is vy_attn_decode.  ws: vy_text_layer_ws_bytes. */
+typedef struct vy_text_layer {
+  int32_t h, hk, dh, ffn, act, mask_kind, dtype;
+  float eps1, eps2;
+  const void *wqkv, *bqkv, *wo, *bo, *ln1_w, *ln1_b, *w1, *b1, *w2, *b2, *ln2_w, *ln2_b;
+  const float *cos_tab, *sin_tab;
+  int64_t pos0;
+  void *k_new, *v_new;
+  int64_t kn_sb, kn_sh, kn_sl, vn_sb, vn_sh, vn_sl;
+  const void *k, *v;
+  int64_t k_sb, k_sh, k_sl, v_sb, v_sh, v_sl, S, start_pos;
+  const uint8_t* keypad;
+  int64_t kp_sb;
+} vy_text_layer;
+int64_t vy_text_layer_ws_bytes(int64_t B, int64_t L, int32_t h, int32_t dh, int32_t ffn, int dtype);
+int vy_text_layer_fwd(const vy_text_layer* l, const void* x, void* y, int64_t B, int64_t L, void* ws, int64_t ws_bytes, void* stream);
+
 /* vy_rmsnorm_fwd: y = x * rsqrt(mean(x^2) + eps) * (w_offset + w); Gemma uses w_offset = 1
  * (Examples/paligemma.ipynb cell 11, GemmaRMSNorm).  Statistics in fp32. */
 int vy_rmsnorm_fwd(const void* x, int64_t ldx, const void* w, void* y, int64_t ldy, int64_t M,

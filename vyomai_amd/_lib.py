@@ -32,6 +32,7 @@ PROTOTYPES = {
     "vy_attn_fwd": [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
                     _p, _i64, _i64, _p, _i, _i64, _p, _i64, _p, _i64, _i64,
                     _i64, _i, _i, _i64, _i64, _i, _f, _i, _p],
+    "vy_text_layer_fwd": [_p, _p, _p, _i64, _i64, _p, _i64, _p],
     "vy_attn_decode": [_p, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
                        _p, _i64, _i64, _i, _i, _i64, _i, _f, _i, _p],
     "vy_layernorm_fwd": [_p, _i64, _p, _p, _p, _i64, _p, _p, _i64, _i64, _f, _i, _p],
@@ -95,7 +96,7 @@ PROTOTYPES = {
     "vy_set_concurrent_chains": [_i],
     "vy_workspace_set": [_p, _p, _i64],
 }
-OTHER_SYMBOLS = ["vy_last_error", "vy_abi_version", "vy_layernorm_bwd_ws_rows", "vy_decode_ws_bytes",
+OTHER_SYMBOLS = ["vy_last_error", "vy_text_layer_ws_bytes", "vy_abi_version", "vy_layernorm_bwd_ws_rows", "vy_decode_ws_bytes",
                  "vy_gemma_ws_bytes", "vy_ddp_world", "vy_ddp_rank", "vy_latent_decode_ws_bytes", "vy_decay_attn_ws_bytes",
                  "vy_hybrid_ws_bytes", "vy_window_decode_ws_bytes", "vy_moe_ws_bytes", "vy_gated_attn_ws_bytes"]
 DECAY_CHUNK = 64   # VY_DECAY_CHUNK
@@ -142,6 +143,15 @@ class VyomHipError(RuntimeError):
     pass
 
 
+class VyTextLayer(C.Structure):
+    """vy_text_layer (include/vyom_hip.h)"""
+    _fields_ = [(n, C.c_int32) for n in ("h", "hk", "dh", "ffn", "act", "mask_kind", "dtype")] + [("eps1", _f), ("eps2", _f)] + \
+               [(n, _p) for n in ("wqkv", "bqkv", "wo", "bo", "ln1_w", "ln1_b", "w1", "b1", "w2", "b2", "ln2_w", "ln2_b", "cos_tab",
+                                  "sin_tab")] + [("pos0", _i64), ("k_new", _p), ("v_new", _p)] + \
+               [(n, _i64) for n in ("kn_sb", "kn_sh", "kn_sl", "vn_sb", "vn_sh", "vn_sl")] + [("k", _p), ("v", _p)] + \
+               [(n, _i64) for n in ("k_sb", "k_sh", "k_sl", "v_sb", "v_sh", "v_sl", "S", "start_pos")] + [("keypad", _p), ("kp_sb", _i64)]
+
+
 _lib: Optional[C.CDLL] = None
 
 
@@ -165,6 +175,8 @@ def load() -> C.CDLL:
     lib.vy_abi_version.restype = C.c_int
     lib.vy_layernorm_bwd_ws_rows.restype = C.c_int64
     lib.vy_layernorm_bwd_ws_rows.argtypes = [_i64]
+    lib.vy_text_layer_ws_bytes.restype = C.c_int64
+    lib.vy_text_layer_ws_bytes.argtypes = [_i64, _i64, C.c_int32, C.c_int32, C.c_int32, _i]
     lib.vy_decode_ws_bytes.restype = C.c_int64
     lib.vy_decode_ws_bytes.argtypes = [C.c_int32] * 7
     for name, argtypes in (("vy_latent_decode_ws_bytes", [_i, _i, _i]),
@@ -178,7 +190,7 @@ def load() -> C.CDLL:
 
 
 def call(name: str, *args) -> None:
-    lib = load()
+    lib = _lib if _lib is not None else load()
     rc = getattr(lib, name)(*args)
     if rc != 0:
         raise VyomHipError(f"{name} failed ({rc}): {lib.vy_last_error().decode()}")

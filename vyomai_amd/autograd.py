@@ -16,15 +16,15 @@ from typing import Optional
 
 import torch
 
-from . import ops
+from . import _lib, ops
 from ._lib import VyomHipError
+from .layers.attention import AttentionSelfOutput, _shadow as _param_shadow
+from .layers.ffn import FeedForward
 from .layers.mask import AttnMask
 from .layers.positional_embeddings import resolve_freqs
 
 
-def _shadow(param: Optional[torch.Tensor], dtype: torch.dtype) -> Optional[torch.Tensor]:
-    from .layers.attention import _shadow as s
-    return s(param, dtype)
+_shadow = _param_shadow
 
 
 def _wants_grad(*ts) -> bool:
@@ -119,7 +119,7 @@ def self_attention_block(mod, x, attention_mask, freqs, cache, cache_index, star
     else:
         kw = torch.empty((B, hk, L, dh), dtype=dt, device=dev)
         vw = torch.empty_like(kw)
-    sw, sb = mod._packed_shadow(dt)
+    sw, sb = mod._packed_shadow(dt, (w, b))
     ops.qkv_rope(x, sw, sb, h, hk, dh, cos, sin, pos0, q, kw, vw)
     if cache is not None:
         k_all, v_all = cache.commit() if cache_index is None else cache.commit(cache_index)
@@ -132,6 +132,61 @@ def self_attention_block(mod, x, attention_mask, freqs, cache, cache_index, star
         o = ops.attention(q, k_all, v_all, **_mask_args(attention_mask, B, L, S, dev))
     return linear_residual_layernorm(o, x, aso.dense.weight, aso.dense.bias, aso.layernorm.weight,
                                      aso.layernorm.bias, aso.layernorm.eps, aso.dropout.p, aso.training)
+
+
+_GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks)
+
+
+def layer_forward(att, ff, x, mask, freqs, cache=None, cache_index: Optional[int] = None, start_pos: int = 0):
+    """ff(att(x), x) of one post-LN layer without gradients as ONE native call (vy_text_layer_fwd), the same launches in the same order:
+    a layer of a few short texts is 50 us of GPU work, and four times that in Python.  None: the modules are to be called one by one --
+    a module of another class or with a hook, active dropout, a dense mask, rows that are not contiguous."""
+    if type(ff) is not FeedForward or "_whole_layer" not in type(att).__dict__ or type(att.out) is not AttentionSelfOutput \
+            or not (mask is None or isinstance(mask, AttnMask)):
+        return None
+    aso = att.out
+    if any(_GLOBAL_HOOKS) or any(m._forward_hooks or m._forward_pre_hooks for m in (att, aso, ff)):
+        return None
+    if not x.is_cuda or x.dim() != 3 or not x.is_contiguous() or ops._Lanes.active or torch.is_grad_enabled() or type(x) is not torch.Tensor:
+        return None
+    if (aso.training and aso.dropout.p > 0.0) or (ff.training and ff.dropout.p > 0.0):
+        return None
+    dt, dev = x.dtype, x.device
+    if dt is not torch.bfloat16 and dt is not torch.float32:
+        return None
+    B, L, d = x.shape
+    h, hk, dh = att.num_attention_heads, att.num_key_value_heads, att.head_dim
+    if d != h * dh or 0 in x.shape:
+        return None
+    w, b = att._packed_shadow(dt)
+    keep = [w, b] + [_shadow(p, dt) for p in (aso.dense.weight, aso.dense.bias, aso.layernorm.weight, aso.layernorm.bias, ff.intermediate.weight,
+                                              ff.intermediate.bias, ff.out.weight, ff.out.bias, ff.layernorm.weight, ff.layernorm.bias)]
+    inner = ff.intermediate.weight.shape[0]
+    if any(t is not None and (t.device != dev or not t.is_contiguous()) for t in keep) or w.shape != ((h + 2 * hk) * dh, d) \
+            or keep[2].shape != (d, d) or keep[6].shape != (inner, d) or keep[8].shape != (d, inner):
+        return None
+    cos, sin, pos0 = resolve_freqs(freqs, dev)
+    if cache is None:
+        kv = torch.empty((2, B, hk, L, dh), dtype=dt, device=dev)
+        k_new, v_new = kv[0], kv[1]
+        k, v = k_new, v_new
+    else:
+        k_new, v_new = cache.reserve(B, hk, L, dh, start_pos, dt, dev) if cache_index is None else \
+            cache.reserve(cache_index, B, hk, L, dh, start_pos, dt, dev)
+        k, v = cache.commit() if cache_index is None else cache.commit(cache_index)
+    assert k_new.stride(3) == 1 and v_new.stride(3) == 1
+    S = k.shape[2]
+    m = _mask_args(mask, B, L, S, dev)
+    kp = m["keypad"]
+    kind = (_lib.MASK_CAUSAL if m["causal"] else 0) | (_lib.MASK_KEYPAD if kp is not None else 0)
+    if kp is not None:
+        assert kp.dtype == torch.uint8 and kp.shape == (B, S) and kp.stride(1) == 1
+    p = [ops._ptr(t) for t in keep]
+    desc = _lib.VyTextLayer(h, hk, dh, inner, ff.act, kind, _lib.dtype_code(dt), aso.layernorm.eps, ff.layernorm.eps, *p, ops._ptr(cos),
+                            ops._ptr(sin), pos0, k_new.data_ptr(), v_new.data_ptr(), *k_new.stride()[:3], *v_new.stride()[:3], k.data_ptr(),
+                            v.data_ptr(), *k.stride()[:3], *v.stride()[:3], S, m["start_pos"], ops._ptr(kp),
+                            kp.stride(0) if kp is not None else 0)
+    return ops.text_layer(desc, x)
 
 
 def _split(x2: torch.Tensor, heads: int, dh: int) -> torch.Tensor:

@@ -113,7 +113,7 @@ class DecodePlan:
 
     def _launch(self, x_ptr, pos, pos_dev_ptr, hidden_ptr, logits_ptr):
         _lib.call("vy_decoder_step", C.byref(self.plan), x_ptr, pos, pos_dev_ptr, hidden_ptr, logits_ptr,
-                  self.ldv, torch.cuda.current_stream().cuda_stream)
+                  self.ldv, ops._raw_stream())
 
     def _capture(self, x: torch.Tensor, pos: int):
         """Run this step eagerly on a side stream (also the warm-up) and record the same launches
@@ -250,7 +250,7 @@ class GemmaDecodePlan:
             raise ValueError(f"position {pos} exceeds the cache size {self.capacity} (max_cache_len)")
         logits = torch.empty((self.batch, self.ldv), dtype=self.dtype, device=self.device)
         _lib.call("vy_gemma_decoder_step", C.byref(self.plan), x.data_ptr(), int(pos), logits.data_ptr(), self.ldv,
-                  torch.cuda.current_stream().cuda_stream)
+                  ops._raw_stream())
         return logits[:, : self.vocab]
 
 
@@ -387,5 +387,5 @@ class HybridDecodePlan:
         logits = torch.empty((self.batch, self.ldv), dtype=self.dtype, device=self.device)
         _lib.call("vy_hybrid_decoder_step", C.byref(self.plan), ids.data_ptr(), batch.slots.data_ptr(),
                   batch.start.data_ptr(), int(batch.max_keys), logits.data_ptr(), self.ldv,
-                  torch.cuda.current_stream().cuda_stream)
+                  ops._raw_stream())
         return logits[:, : self.vocab]

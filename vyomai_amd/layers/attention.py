@@ -130,16 +130,16 @@ class _SelfAttentionBase(nn.Module):
         self._plain_projections()
         if self._fused_qkv:
             return self.qkv.weight, self.qkv.bias
-        ws = [self.query.weight, self.key.weight, self.value.weight]
+        ws = [self._modules[n].weight for n in ("query", "key", "value")]
         packed = getattr(self, "_packed_w", None)
         ok = packed is not None and packed.device == ws[0].device and packed.dtype == ws[0].dtype
         if ok:
-            off = 0
+            at, row = packed.data_ptr(), packed.element_size() * packed.shape[1]
             for w in ws:
-                if w.data_ptr() != packed.data_ptr() + off * packed.element_size() * packed.shape[1]:
+                if w.data_ptr() != at:
                     ok = False
                     break
-                off += w.shape[0]
+                at += w.shape[0] * row
         if not ok:
             with torch.no_grad():
                 packed = torch.cat([w.detach() for w in ws], dim=0).contiguous()
@@ -181,7 +181,7 @@ class _SelfAttentionBase(nn.Module):
         whose weight lives at `.linear.weight` (VyomAI/layers/adapters.py:21-24, 58-62) -- would be ignored (or crash on
         a missing attribute).  Adapters are outside SURVEY section 8; say so instead of computing without them."""
         for name in (("qkv",) if self._fused_qkv else ("query", "key", "value")):
-            m = getattr(self, name)
+            m = self._modules[name] if name in self._modules else getattr(self, name)
             if not isinstance(m, nn.Linear):
                 raise VyomHipError(
                     f"attention.{name} is a {type(m).__name__}, not an nn.Linear: the MI355X attention path reads the "
@@ -189,13 +189,13 @@ class _SelfAttentionBase(nn.Module):
                     "Adapter wrappers (LoRA / DoRA) are out of scope here -- merge the low-rank update into "
                     f"`{name}.weight` (W + alpha * B A) and restore the nn.Linear before running on the HIP path.")
 
-    def _packed_shadow(self, dtype: torch.dtype) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    def _packed_shadow(self, dtype: torch.dtype, packed=None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
         """_packed() in the compute dtype.  The packed buffer has a version counter of its own that
         in-place writes to query/key/value.weight (optimizer.step() of a torch optimizer,
         load_state_dict) never bump, so the copy is keyed on the MEMBER parameters' versions (as the
         transposed copy for the backward GEMMs is).  Entry: (key, w, b, packed data_ptr, pinned);
         pinned = views of the trainer's shadow arena, refreshed in place (see _shadow)."""
-        w, b = self._packed()
+        w, b = self._packed() if packed is None else packed     # (packed: what _packed() has just returned)
         if w.dtype == dtype:
             return w, b
         if self._fused_qkv:
@@ -237,6 +237,7 @@ class _SelfAttentionBase(nn.Module):
 
 class EncoderAttention(_SelfAttentionBase):
     """forward(hidden_state, attention_mask, freqs=None) -> Tensor.  Reference :75-133."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()
@@ -248,6 +249,7 @@ class EncoderAttention(_SelfAttentionBase):
 
 class EncoderAttentionGqa(_SelfAttentionBase):
     """Grouped-query encoder attention (num_key_value_heads default 4).  Reference :136-215."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()
@@ -260,6 +262,7 @@ class EncoderAttentionGqa(_SelfAttentionBase):
 class DecoderAttention(_SelfAttentionBase):
     """Decoder self-attention with the cache attached as ``self.cache`` (model._setup_cache()).
     forward(hidden_state, attention_mask, freqs, use_cache, start_pos).  Reference :218-289."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()
@@ -277,6 +280,7 @@ class DecoderAttention(_SelfAttentionBase):
 
 class DecoderAttentionGqa(_SelfAttentionBase):
     """Reference :292-379."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()
@@ -294,6 +298,7 @@ class DecoderAttentionGqa(_SelfAttentionBase):
 
 class VisionAttention(_SelfAttentionBase):
     """ViT attention with one fused ``qkv`` Linear.  Reference :576-624."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()

@@ -17,6 +17,7 @@ from ..layers.attention import _SelfAttentionBase
 from ..layers.ffn import FeedForward
 from ..layers.kv_cache import DynamicCacheOne, StaticCacheOne
 from ..layers.mask import AttnMask
+from ..autograd import layer_forward
 from ..autograd_train import defer_residual_grads as _defer
 from .common import LMHead, PositionMixin
 
@@ -36,6 +37,7 @@ class CLMOutput(object):
 class DecoderAttention(_SelfAttentionBase):
     """forward(hidden_state, attention_mask, freqs, use_cache, kv_cache, start_pos)
     -> (hidden_state, kv_cache).  Reference :44-113."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()
@@ -52,6 +54,7 @@ class DecoderAttention(_SelfAttentionBase):
 
 class DecoderAttentionGqa(_SelfAttentionBase):
     """Reference :116-201 (K/V projections of num_key_value_heads heads, default 4)."""
+    _whole_layer = True
 
     def __init__(self, config, layer_idx: int) -> None:
         super().__init__()
@@ -81,6 +84,11 @@ class DecoderLayer(nn.Module):
 
     def forward(self, hidden_state, attention_mask, freqs=None, use_cache: Optional[bool] = False,
                 kv_cache=None, start_pos: Optional[int] = 0):
+        if not torch.is_grad_enabled() and (kv_cache is not None or not use_cache):
+            y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs,
+                              kv_cache if use_cache else None, self.attention.layer_idx, start_pos)
+            if y is not None:
+                return y, kv_cache
         _defer(hidden_state)  # training: its residual-path gradients are added in the QKV dgrad epilogue
         out, kv_cache = self.attention(hidden_state=hidden_state, attention_mask=attention_mask, freqs=freqs,
                                        use_cache=use_cache, kv_cache=kv_cache, start_pos=start_pos)

@@ -9,6 +9,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
+from ..autograd import layer_forward
 from ..autograd_train import defer_residual_grads as _defer
 from ..layers.attention import DecoderAttention, DecoderAttentionGqa
 from ..layers.ffn import FeedForward
@@ -36,6 +37,10 @@ class DecoderLayer(nn.Module):
 
     def forward(self, hidden_state, attention_mask, freqs=None, use_cache: Optional[bool] = False,
                 start_pos: Optional[int] = 0) -> torch.Tensor:
+        if not torch.is_grad_enabled() and not use_cache:
+            y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
+            if y is not None:
+                return y
         _defer(hidden_state)  # training: its residual-path gradients are added in the QKV dgrad epilogue
         out = self.attention(hidden_state=hidden_state, attention_mask=attention_mask, freqs=freqs,
                              use_cache=use_cache, start_pos=start_pos)

@@ -18,6 +18,12 @@ from ._lib import call, dtype_code
 Tensor = torch.Tensor
 
 
+def _raw_stream() -> int:
+    """The current stream's handle (torch.cuda.current_stream().cuda_stream, without building a Stream object: a tenth of the
+    3 us, on every launch)."""
+    return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 # ------------------------------------------------------------------------------------------
 # Two lanes: the training forward as two batch halves on two HIP streams.
 #
@@ -92,8 +98,8 @@ def _lanes_join() -> None:
 def _lane_plan(rows: Optional[int] = None, batches: Optional[int] = None, keep=()):
     """-> [(first, count, stream)] over rows (of a (B*L, .) view) or batches: one entry when the op runs whole, two
     when it is split over the lanes."""
-    main = torch.cuda.current_stream()
     if _Lanes.active:
+        main = torch.cuda.current_stream()
         if rows is not None and rows == _Lanes.B * _Lanes.L:
             cut, n = _Lanes.B0 * _Lanes.L, rows
         elif batches is not None and batches == _Lanes.B:
@@ -109,13 +115,14 @@ def _lane_plan(rows: Optional[int] = None, batches: Optional[int] = None, keep=(
             return [(0, cut, main.cuda_stream), (cut, n - cut, _Lanes.side.cuda_stream)]
         _lanes_join()
     n = rows if rows is not None else batches
-    return [(0, n, main.cuda_stream)]
+    return [(0, n, _raw_stream())]
 
 
 def _stream() -> int:
     """The stream of an op that always runs whole (inside a lane region: after the main stream has joined lane 1)."""
-    _lanes_join()
-    return torch.cuda.current_stream().cuda_stream
+    if _Lanes.active:
+        _lanes_join()
+    return _raw_stream()
 
 
 _WS = {}
@@ -127,11 +134,10 @@ def _mid_ws(rows: int) -> None:
     (vy_workspace_set: one buffer per stream, registered once; the library never allocates device memory)."""
     if rows <= 32 or rows > 4096 or _Lanes.active:
         return
-    st = torch.cuda.current_stream()
-    key = (st.device_index, st.cuda_stream)
+    key = torch._C._cuda_getDevice(), _raw_stream()
     if key not in _WS:
-        buf = torch.empty(_WS_BYTES, dtype=torch.uint8, device=torch.device("cuda", st.device_index))
-        call("vy_workspace_set", st.cuda_stream, buf.data_ptr(), _WS_BYTES)
+        buf = torch.empty(_WS_BYTES, dtype=torch.uint8, device=torch.device("cuda", key[0]))
+        call("vy_workspace_set", key[1], buf.data_ptr(), _WS_BYTES)
         _WS[key] = buf
 
 
@@ -139,6 +145,8 @@ def _at(t: Optional[Tensor], first: int):
     """data pointer of t[first:] (None stays None)."""
     if t is None:
         return None
+    if first == 0:
+        return t.data_ptr()
     return t.data_ptr() + first * t.stride(0) * t.element_size()
 
 
@@ -182,8 +190,10 @@ def linear(x: Tensor, w: Tensor, bias: Optional[Tensor] = None, act: int = _lib.
         # row stride padded to 8 elements so every row is 16-byte aligned (N = vocab is odd)
         ldy = (N + 7) // 8 * 8
         buf = torch.empty((M, ldy), dtype=x.dtype, device=x.device)
-        y2 = buf[:, :N]
-        ret = buf.view(*x.shape[:-1], ldy)[..., :N]
+        y2 = buf if ldy == N else buf[:, :N]
+        ret = buf if ldy == N and x.dim() == 2 else buf.view(*x.shape[:-1], ldy)
+        if ldy != N:
+            ret = ret[..., :N]
     else:
         y2 = _rows(out)
         ret = out
@@ -276,6 +286,17 @@ def attention(q: Tensor, k: Tensor, v: Tensor, *, causal: bool = False, start_po
              _at(keypad, b0), keypad.stride(0) if keypad is not None else 0,
              _ptr(addmask), am_sb, am_sl, nb, h, hk, L, S, dh, float(scale), dtype_code(q.dtype), st)
     return out
+
+
+def text_layer(desc: "_lib.VyTextLayer", x: Tensor) -> Tensor:
+    """One layer without gradients: desc (dtype, mask and key fields are filled in), x (B, L, d) contiguous.  (vy_text_layer_fwd)"""
+    B, L, _ = x.shape
+    _mid_ws(B * L)
+    y = torch.empty_like(x)
+    n = _lib.load().vy_text_layer_ws_bytes(B, L, desc.h, desc.dh, desc.ffn, desc.dtype)
+    ws = torch.empty(n, dtype=torch.uint8, device=x.device)
+    call("vy_text_layer_fwd", C.addressof(desc), x.data_ptr(), y.data_ptr(), B, L, ws.data_ptr(), n, _stream())
+    return y
 
 
 def attention_decode(q: Tensor, k: Tensor, v: Tensor, S: int, scale: Optional[float] = None) -> Tensor:
