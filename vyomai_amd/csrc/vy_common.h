@@ -172,19 +172,21 @@ __device__ __forceinline__ float vy_act_grad(float x) {
   else return 1.0f;
 }
 
-// sum / maximum over the 64 lanes, in every lane: rotations inside the rows of 16 (DPP) and the two half-swaps of gfx950 -- six
-// vector instructions, where a shuffle is an LDS round trip per step (a residual sum with its two layer norms, one row: 3.8 -> 2.9 us)
+// sum / maximum over the 64 lanes, in every lane: the two half-swaps of gfx950 and rotations inside the rows of 16 (DPP) -- six
+// vector instructions, where a shuffle is an LDS round trip per step (a residual sum with its two layer norms, one row: 3.8 -> 2.8 us,
+// with the norms' weights requested ahead).  The order is the butterfly's over lane ^ 32, 16, 8, 4, 2, 1: behind the step of 8 a row
+// repeats itself every 8 lanes, so a rotation by 4 is lane ^ 4, and so on.
 template <typename F> __device__ __forceinline__ float vy_wave_fold(float v, F f) {
-  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false)));   // row_ror:8
-  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xf, 0xf, false)));   // row_ror:4
-  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x122, 0xf, 0xf, false)));   // row_ror:2
-  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false)));   // row_ror:1
+  const unsigned w = __builtin_bit_cast(unsigned, v);
+  auto s32 = __builtin_amdgcn_permlane32_swap(w, w, false, false);
+  v = f(__builtin_bit_cast(float, (unsigned)s32[0]), __builtin_bit_cast(float, (unsigned)s32[1]));
   const unsigned u = __builtin_bit_cast(unsigned, v);
   auto s16 = __builtin_amdgcn_permlane16_swap(u, u, false, false);
   v = f(__builtin_bit_cast(float, (unsigned)s16[0]), __builtin_bit_cast(float, (unsigned)s16[1]));
-  const unsigned w = __builtin_bit_cast(unsigned, v);
-  auto s32 = __builtin_amdgcn_permlane32_swap(w, w, false, false);
-  return f(__builtin_bit_cast(float, (unsigned)s32[0]), __builtin_bit_cast(float, (unsigned)s32[1]));
+  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x128, 0xf, 0xf, false)));   // row_ror:8
+  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x124, 0xf, 0xf, false)));   // row_ror:4
+  v = f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x122, 0xf, 0xf, false)));   // row_ror:2
+  return f(v, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, v), 0x121, 0xf, 0xf, false)));   // row_ror:1
 }
 __device__ __forceinline__ float vy_wave_sum(float v) { return vy_wave_fold(v, [](float a, float b) { return a + b; }); }
 __device__ __forceinline__ float vy_wave_max(float v) { return vy_wave_fold(v, [](float a, float b) { return fmaxf(a, b); }); }
