@@ -1,0 +1,89 @@
+"""Decode steps of 1 to 4 sequences, whose products make their operand rows themselves (vyomai_amd/csrc/vy_few.hip): every number of
+rows, the widths that have kernels, padded widths, odd vocabularies and layers without a feed-forward, against steps that run the
+norms and products one by one."""
+import pytest
+import torch
+
+from tests.test_decode_lean_gpu import _plan, _step
+
+pytestmark = pytest.mark.gpu
+BF, DEV = torch.bfloat16, "cuda"
+
+
+def decoder(width, pos_kind, kv_heads, dtype, layers=2):
+    import vyomai_amd as V
+    from vyomai_amd import recipe
+    cfg = V.EncoderConfig(hidden_size=width, num_attention_heads=width // 64, num_hidden_layers=layers, max_position_embeddings=256,
+                          intermediate_size=4 * width, hidden_dropout_prob=0.0, vocab_size=1003)
+    if kv_heads:
+        cfg.num_key_value_heads = kv_heads
+    m = V.DecoderModel(cfg, pos_kind, "gqa" if kv_heads else None)
+    recipe.load_recipe_(m)
+    return cfg, m.to(DEV).to(dtype).eval()
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 4])
+@pytest.mark.parametrize("width,pos_kind,kv_heads", [(512, "rope", None), (768, "rope", 4), (768, "absolute", None), (1024, "rope", 2)])
+def test_decoder_step(B, width, pos_kind, kv_heads):
+    """Against the fp32 step on the same weights.  A layer rounds seven rows to bf16 (operand, q / k / v, attention, both sums, the
+    normalised sum, the feed-forward's middle), the head three; each adds at most 2^-8 relative to what comes out of a norm."""
+    g = torch.Generator().manual_seed(width + B)
+    cfg, m = decoder(width, pos_kind, kv_heads, BF)
+    x = (torch.randn(B, width, generator=g) * 0.5).to(BF).to(DEV)
+    plan, cache = _plan(cfg, m, B, BF)
+    got = _step(plan, cache, x, 37, 1)
+    for lean in (0, 1):   # the general launchers; the same kernels again, from the state that the first call left
+        other, its = _plan(cfg, m, B, BF)
+        same = _step(other, its, x, 37, lean)
+        for (k, v), (ok, ov) in zip(got[2], same[2]):
+            assert (k - ok).norm() <= 14 * 2.0 ** -8 * ok.norm() and (v - ov).norm() <= 14 * 2.0 ** -8 * ov.norm()
+    assert torch.equal(got[0], same[0]) and torch.equal(got[1], same[1])
+    cfg32, m32 = decoder(width, pos_kind, kv_heads, torch.float32)
+    plan32, cache32 = _plan(cfg32, m32, B, torch.float32)
+    want = _step(plan32, cache32, x.float(), 37, 1)
+    # (this plan's cache holds the unrounded rows: one more rounding)
+    for a, b, n in ((got[1], want[1], 15), (got[0], want[0], 18)):
+        assert torch.isfinite(a).all() and (a - b).norm() <= n * 2.0 ** -8 * b.norm(), float((a - b).norm() / b.norm())
+
+
+def gisitar(width):
+    from vyomai_amd import GisitarConfig, GisitarModel
+    lig = {"type": "lightning", "mixer": {"heads": 8, "dim": 64, "vdim": 64, "decay": [0.9] * 8}}
+    lat = {"type": "latent_attention", "mixer": {"heads": 4, "dim": 64, "vdim": 64, "q_rank": 256, "kv_rank": 128, "scale": 0.125}}
+    ff = {"kind": "dense", "ff": 1496}
+    return GisitarModel(GisitarConfig(vocab=1003, width=width, layers=[{**lig, "mlp": None}, {**lat, "mlp": ff}, {**lig, "mlp": ff},
+                                                                       {**lat, "mlp": None}]))
+
+
+def biruvik(width):
+    from tests import biruvik_cases as K
+    from vyomai_amd import BiruvikConfig, BiruvikModel
+    return BiruvikModel(BiruvikConfig.from_dict(K.config([K.hgrn2(4, 64, 64, mlp=K.dense(1500)), K.latent(4, 64, 64, 128, 64),
+                                                          K.attention(4, 2, 64, 128, mlp=K.dense(768))], width=width, vocab=1003)))
+
+
+@pytest.mark.parametrize("B", [1, 2, 3, 4])
+@pytest.mark.parametrize("make,width", [(gisitar, 1024), (gisitar, 1020), (gisitar, 2048), (gisitar, 1032), (biruvik, 1024),
+                                        (biruvik, 2044)])
+def test_hybrid_step(make, width, B):
+    """A next token through the step and through the prompt path (other product and norm kernels): the logits agree within bf16
+    roundings of the sublayers' inputs, 2^-9 relative each, at most eight per layer and a vocabulary product."""
+    torch.manual_seed(width)
+    with torch.device(DEV):
+        torch.set_default_dtype(BF)
+        try:
+            m = make(width).eval()
+        finally:
+            torch.set_default_dtype(torch.float32)
+    ids = torch.randint(0, 1003, (B, 6), device=DEV, generator=torch.Generator(device=DEV).manual_seed(B))
+    cache = m.new_cache(B + 2, 8)
+    cache.allocate(2)   # (slots that are not the rows numbers)
+    slots = cache.allocate(B)
+    m.prefill(ids[:, :2].contiguous(), [2] * B, cache, slots)
+    for t in range(2, 6):
+        got = m.decode(ids[:, t].contiguous(), cache, slots).double()
+        other = m.new_cache(B, 8)
+        s = other.allocate(B)
+        want = m.logits(m.prefill(ids[:, :t + 1].contiguous(), [t + 1] * B, other, s)[:, -1]).double()
+        assert torch.isfinite(got).all()
+        assert (got - want).norm() <= 8 * len(m.layers) * 2.0 ** -9 * want.norm(), float((got - want).norm() / want.norm())

@@ -1,0 +1,271 @@
+// Decode steps of 1 to 4 sequences: matrix-vector products that make their operand rows themselves.
+//
+// Such a step is a chain of launches that each move a few MB and take 2 to 4 us, of which the norm between two products is one: a
+// single workgroup that waits for the product before it, reduces a row and writes it for the next.  Here every workgroup of the next
+// product redoes that norm -- a row is 1.5 to 8 KB out of L2, a wave per row, reductions in registers -- while its weights, which it
+// has requested first, are on their way; so the norm costs a launch's tail instead of a launch.  A wave takes R = 1 or 2 weight rows
+// (rotary pairs and gate / up pairs are the two rows of a wave) in whole 1 KB pieces.
+//
+// 12 layers of 768, one sequence behind 70 tokens: 334 -> 249 us a step (62 launches instead of 75, and no products for 32 rows);
+// 8 layers of width 1024 (latent and lightning attention), 700 tokens: 302 -> 267 us, 2 / 4 rows 414 -> 308 / 482 -> 398 us.
+#include "vy_few.h"
+
+namespace vy_few {
+namespace {
+
+__device__ __forceinline__ float dot8(const bf16x8 a, const bf16x8 b, float s) {
+#pragma unroll
+  for (int i = 0; i < 8; i += 2) s = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{a[i], a[i + 1]}, bf16x2{b[i], b[i + 1]}, s, false);
+  return s;
+}
+__device__ __forceinline__ float rsqrt_refined(float ms) {
+  const float r = rsqrtf(ms);
+  return r * (1.5f - 0.5f * ms * r * r);
+}
+
+// (v - mean) rstd of a row of which a lane holds the quads 64 c + lane, over its first n columns (v = 0 in the padding of a LayerNorm
+// is not assumed)
+template <int KC>
+__device__ __forceinline__ void stats(const float (&v)[KC][4], int lane, int n, bool rms, float eps, float& mean, float& rstd) {
+  mean = 0.f;
+  if (!rms) {
+    float s = 0.f;
+#pragma unroll
+    for (int c = 0; c < KC; ++c)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) s += v[c][e];
+    mean = vy_wave_sum(s) / (float)n;
+  }
+  float q = 0.f;
+#pragma unroll
+  for (int c = 0; c < KC; ++c)
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      const float d = (64 * c + lane) * 4 + e < n ? v[c][e] - mean : 0.f;
+      q += d * d;
+    }
+  rstd = rsqrt_refined(vy_wave_sum(q) / (float)n + eps);
+}
+
+template <int EPI, int PRO, int MR, int KC>
+__global__ __launch_bounds__(256) void few_kernel(Args a) {
+  constexpr int K = 256 * KC, R = (EPI != STORE || KC % 2) ? 2 : 1, P = KC * R / 2;   // columns; weight rows and pieces per wave
+  __shared__ __attribute__((aligned(16))) bf16 hs[PRO == PLAIN ? 8 : MR * K];
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int units = EPI == STORE ? (a.N + R - 1) / R : EPI == QKV ? a.N / 2 : a.N;   // of R weight rows
+  const int step = gridDim.x * 4;
+  int u = blockIdx.x * 4 + wave;
+
+  auto row_of = [&](int unit, int r) {
+    if constexpr (EPI == QKV) return (unit >> 5) * 64 + (unit & 31) + 32 * r;
+    else if constexpr (EPI == GATED) return unit + r * a.N;
+    else { const int n = unit * R + r; return n < a.N ? n : a.N - 1; }
+  };
+  // chunk (8 columns) of piece p: which of the wave's rows, and which columns
+  bf16x8 w[P];
+  auto request = [&](int unit) {
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int c = 64 * p + lane, r = R == 1 ? 0 : (c >= 32 * KC);
+      const bf16x8* at = reinterpret_cast<const bf16x8*>(a.w + (int64_t)row_of(unit, r) * K + (c - r * 32 * KC) * 8);
+      if (a.once) w[p] = __builtin_nontemporal_load(at);
+      else w[p] = *at;
+    }
+  };
+  if (u < units) request(u);
+
+  if constexpr (PRO != PLAIN) {
+    if (a.advance && blockIdx.x == 0)
+      for (int i = threadIdx.x; i < a.n_adv; i += 256) a.advance[a.slots ? a.slots[i] : i] += 1;
+    if (wave < a.M) {
+      const int m = wave;
+      float v[KC][4], g[KC][4], b[KC][4];
+      if constexpr (PRO == LAYER) {
+        bf16x4 v4[KC], g4[KC], b4[KC];
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          const int col = (64 * c + lane) * 4;
+          v4[c] = *reinterpret_cast<const bf16x4*>(a.x + m * a.ldx + col);
+          g4[c] = *reinterpret_cast<const bf16x4*>(a.ln_g + col);
+          b4[c] = *reinterpret_cast<const bf16x4*>(a.ln_b + col);
+        }
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { v[c][e] = (float)v4[c][e]; g[c][e] = (float)g4[c][e]; b[c][e] = (float)b4[c][e]; }
+      } else {
+        f32x4 s4[KC], p4[KC], g4[KC];
+        bf16x4 y4[KC];
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          const int col = (64 * c + lane) * 4;
+          s4[c] = *reinterpret_cast<const f32x4*>(a.s_in + m * a.lds + col);
+          if (a.x) y4[c] = *reinterpret_cast<const bf16x4*>(a.x + m * a.ldx + col);
+          if (a.w_post) p4[c] = *reinterpret_cast<const f32x4*>(a.w_post + col);
+          if (a.w_pre) g4[c] = *reinterpret_cast<const f32x4*>(a.w_pre + col);
+        }
+        if (a.x) {
+          float mean = 0.f, rstd = 1.f, y[KC][4];
+#pragma unroll
+          for (int c = 0; c < KC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) y[c][e] = (float)y4[c][e];
+          if (a.w_post) stats<KC>(y, lane, a.n, a.rms, a.eps, mean, rstd);
+#pragma unroll
+          for (int c = 0; c < KC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[c][e] = s4[c][e] + (a.w_post ? (y[c][e] - mean) * rstd * p4[c][e] : y[c][e]);
+        } else {
+#pragma unroll
+          for (int c = 0; c < KC; ++c)
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[c][e] = s4[c][e];
+        }
+        if (a.s_out && blockIdx.x == 0)
+#pragma unroll
+          for (int c = 0; c < KC; ++c) *reinterpret_cast<f32x4*>(a.s_out + m * a.lds + (64 * c + lane) * 4) = f32x4{v[c][0], v[c][1], v[c][2], v[c][3]};
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) { g[c][e] = a.w_pre ? g4[c][e] : 1.f; b[c][e] = 0.f; }
+      }
+      float mean = 0.f, rstd = 1.f;
+      if (PRO == LAYER || a.w_pre) stats<KC>(v, lane, PRO == LAYER ? K : a.n, PRO == STREAM && a.rms, a.eps, mean, rstd);
+#pragma unroll
+      for (int c = 0; c < KC; ++c) {
+        const int col = (64 * c + lane) * 4;
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (bf16)((v[c][e] - mean) * rstd * g[c][e] + b[c][e]);
+        *reinterpret_cast<bf16x4*>(hs + m * K + col) = o;
+        if (a.h && blockIdx.x == 0) *reinterpret_cast<bf16x4*>(a.h + m * a.ldh + col) = o;
+      }
+    }
+    __syncthreads();
+  }
+
+  for (; u < units; u += step) {
+    // what the epilogue reads besides the product: one lane per (weight row, operand row)
+    const int er = R == 1 ? 0 : lane / MR, em = R == 1 ? lane : lane % MR;
+    const bool mine = lane < R * MR && em < a.M;
+    const int n = row_of(u, mine ? er : 0);
+    const bool real = mine && (EPI != STORE || u * R + er < a.N);
+    float bias = 0.f, res = 0.f;
+    if (mine && EPI != GATED && a.bias) bias = (float)a.bias[n];
+    if (EPI == STORE && mine && a.residual) res = (float)a.residual[em * a.ldr + n];
+    float cs = 0.f, sn = 0.f;
+    int pos = 0;
+    if constexpr (EPI == QKV) {
+      pos = a.pos_dev ? *a.pos_dev : a.pos;
+      if (a.cos_tab && mine) {
+        cs = a.cos_tab[(int64_t)pos * 32 + (n & 31)];
+        sn = a.sin_tab[(int64_t)pos * 32 + (n & 31)];
+      }
+    }
+    float acc[R][MR];
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int m = 0; m < MR; ++m) acc[r][m] = 0.f;
+    bf16x8 wv[P];
+#pragma unroll
+    for (int p = 0; p < P; ++p) wv[p] = w[p];
+    if (u + step < units) request(u + step);
+#pragma unroll
+    for (int p = 0; p < P; ++p) {
+      const int c = 64 * p + lane;
+      const bool second = R == 2 && c >= 32 * KC;
+      const int col = (c - (second ? 32 * KC : 0)) * 8;
+#pragma unroll
+      for (int m = 0; m < MR; ++m) {
+        const bf16x8 xv = PRO == PLAIN ? *reinterpret_cast<const bf16x8*>(a.x + min(m, a.M - 1) * a.ldx + col)
+                                       : *reinterpret_cast<const bf16x8*>(hs + m * K + col);
+        if (R == 1 || 64 * (p + 1) <= 32 * KC) acc[0][m] = dot8(wv[p], xv, acc[0][m]);
+        else if (64 * p >= 32 * KC) acc[R - 1][m] = dot8(wv[p], xv, acc[R - 1][m]);
+        else {   // the piece that holds the end of one row and the start of the other
+          const float d = dot8(wv[p], xv, 0.f);
+          acc[0][m] += second ? 0.f : d;
+          acc[R - 1][m] += second ? d : 0.f;
+        }
+      }
+    }
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int m = 0; m < MR; ++m) acc[r][m] = vy_wave_sum(acc[r][m]);
+    float own = 0.f, other = 0.f;
+#pragma unroll
+    for (int r = 0; r < R; ++r)
+#pragma unroll
+      for (int m = 0; m < MR; ++m)
+        if (er == r && em == m) { own = acc[r][m]; other = acc[R - 1 - r][m]; }
+    if constexpr (EPI == STORE) {
+      float v = own + bias;
+      if (a.act == VY_ACT_GELU_ERF) v = vy_act_fwd_fast<VY_ACT_GELU_ERF>(v);
+      else if (a.act == VY_ACT_GELU_TANH) v = vy_act_fwd_fast<VY_ACT_GELU_TANH>(v);
+      else if (a.act == VY_ACT_RELU2) v = vy_act_fwd<VY_ACT_RELU2>(v);
+      else if (a.act == VY_ACT_SOFTCAP) v = vy_act_fwd<VY_ACT_SOFTCAP>(v, a.act_arg);
+      if (real) a.y[em * a.ldy + n] = (bf16)(v + res);
+    } else if constexpr (EPI == GATED) {
+      const float g = vy_round_bf16(own), up = vy_round_bf16(other);   // (lanes of row 0: own is the gate's)
+      if (real && er == 0) a.y[em * a.ldy + u] = (bf16)((a.act == VY_ACT_SILU ? vy_silu(g) : vy_gelu_tanh(g)) * up);
+    } else {
+      // (the other column of the pair needs its own bias)
+      const float ob = a.bias && mine ? (float)a.bias[n ^ 32] : 0.f;
+      float v = own + bias;
+      if (a.cos_tab && n < a.nq + a.nkv) {
+        const float c = vy_round_bf16(cs), s = vy_round_bf16(sn);
+        const float t = vy_round_bf16(vy_round_bf16(other + ob) * s), m0 = vy_round_bf16(vy_round_bf16(v) * c);
+        v = er ? m0 + t : m0 - t;
+      }
+      if (real) {
+        const int hd = n >> 6, d = n & 63, hq = a.nq >> 6, hkv = a.nkv >> 6;
+        bf16* dst;
+        if (hd < hq) dst = a.q + (int64_t)em * a.nq + n;
+        else if (hd < hq + hkv) dst = a.k + em * a.c_sb + (hd - hq) * a.c_sh + (int64_t)pos * a.c_sl + d;
+        else dst = a.v + em * a.c_sb + (hd - hq - hkv) * a.c_sh + (int64_t)pos * a.c_sl + d;
+        *dst = (bf16)v;
+      }
+    }
+  }
+}
+
+template <int EPI, int PRO, int KC>
+void go_rows(const Args& a, hipStream_t st) {
+  constexpr int R = (EPI != STORE || KC % 2) ? 2 : 1;
+  const int units = EPI == STORE ? (a.N + R - 1) / R : EPI == QKV ? a.N / 2 : a.N;
+  // every workgroup redoes the operand rows, so there are no more of them than fit on the chip at once (by registers): the waves of
+  // wide products loop, with the next rows' weights requested ahead
+  const int most = PRO != STREAM ? 2048 : KC <= 4 ? 1024 : 512;
+  const int grid = (units + 3) / 4 < most ? (units + 3) / 4 : most;
+  if (a.M == 1) hipLaunchKernelGGL((few_kernel<EPI, PRO, 1, KC>), dim3(grid), dim3(256), 0, st, a);
+  else if (a.M == 2) hipLaunchKernelGGL((few_kernel<EPI, PRO, 2, KC>), dim3(grid), dim3(256), 0, st, a);
+  else hipLaunchKernelGGL((few_kernel<EPI, PRO, 4, KC>), dim3(grid), dim3(256), 0, st, a);
+}
+
+}  // namespace
+
+bool few_k(int epi, int pro, int64_t K) {
+  if (K % 256) return false;
+  const int kc = (int)(K / 256);
+  if (pro == PLAIN) return epi == QKV ? kc >= 2 && kc <= 4 : epi == STORE && (kc == 2 || kc == 3 || kc == 4 || kc == 8 || kc == 12 || kc == 16);
+  if (pro == LAYER) return epi != GATED && kc >= 2 && kc <= 4;
+  return epi != QKV && (kc == 4 || kc == 8);
+}
+
+int few_go(int epi, int pro, const Args& a, int64_t K, hipStream_t st) {
+  if (!few_k(epi, pro, K) || a.M < 1 || a.M > 4 || a.N < 1) return VY_ERR_UNSUPPORTED;
+  const int kc = (int)(K / 256);
+#define FEW(E, P, KC_) case KC_: go_rows<E, P, KC_>(a, st); break
+  if (pro == PLAIN && epi == QKV) switch (kc) { FEW(QKV, PLAIN, 2); FEW(QKV, PLAIN, 3); FEW(QKV, PLAIN, 4); }
+  else if (pro == PLAIN) switch (kc) { FEW(STORE, PLAIN, 2); FEW(STORE, PLAIN, 3); FEW(STORE, PLAIN, 4); FEW(STORE, PLAIN, 8); FEW(STORE, PLAIN, 12); FEW(STORE, PLAIN, 16); }
+  else if (pro == LAYER && epi == QKV) switch (kc) { FEW(QKV, LAYER, 2); FEW(QKV, LAYER, 3); FEW(QKV, LAYER, 4); }
+  else if (pro == LAYER) switch (kc) { FEW(STORE, LAYER, 2); FEW(STORE, LAYER, 3); FEW(STORE, LAYER, 4); }
+  else if (epi == STORE) switch (kc) { FEW(STORE, STREAM, 4); FEW(STORE, STREAM, 8); }
+  else switch (kc) { FEW(GATED, STREAM, 4); FEW(GATED, STREAM, 8); }
+#undef FEW
+  VY_CHECK_LAUNCH("few_kernel");
+  return VY_OK;
+}
+
+}  // namespace vy_few

@@ -3,6 +3,8 @@
 // linear attention over its fp32 state, or windowed or differential attention over its ring), dense or routed feed-forward behind
 // or beside the mixer, final norm and vocabulary product.  See include/vyom_hip.h (vy_hybrid_decoder_step).
 #include "vy_common.h"
+#include "vy_few.h"
+#include <utility>
 
 int vy_residual_norm_ex(float* x, int64_t ldx, const void* y, int64_t ldy, const void* table, int64_t ldt, const int64_t* ids,
                         int64_t V, int32_t* err, float table_scale, const vy_routed_rows* routed, const float* w_post,
@@ -70,6 +72,13 @@ int product(const vy_hybrid_plan* p, const void* x, const void* w, void* y, int6
     const int rc = vy_dec_gemv1_act(x, w, bias, act, cap, y, (int)N, (int)K, (hipStream_t)stream);
     if (rc != VY_ERR_UNSUPPORTED) return rc;
   }
+  if (p->dtype == VY_BF16 && p->B <= 4 && N <= INT32_MAX / 2 && vy_few::few_k(vy_few::STORE, vy_few::PLAIN, K) &&
+      (act == VY_ACT_NONE || act == VY_ACT_RELU2 || act == VY_ACT_SOFTCAP) && (uintptr_t)w % 16 == 0) {
+    vy_few::Args a{};
+    a.M = (int)p->B; a.x = (const bf16*)x; a.ldx = K; a.w = (const bf16*)w; a.N = (int)N; a.bias = (const bf16*)bias; a.act = act;
+    a.act_arg = cap; a.y = (bf16*)y; a.ldy = ldy;
+    return vy_few::few_go(vy_few::STORE, vy_few::PLAIN, a, K, (hipStream_t)stream);
+  }
   if (p->dtype == VY_BF16) {
     const int rc = vy_rows_linear(x, w, bias, act, cap, y, ldy, p->B, N, K, (hipStream_t)stream);
     if (rc != VY_ERR_UNSUPPORTED) return rc;
@@ -104,7 +113,7 @@ extern "C" int64_t vy_hybrid_ws_bytes(const vy_hybrid_plan* p) {
   if (!p || !p->layers) return -1;
   const Sizes s = sizes_of(p);
   const int64_t e = p->dtype == VY_BF16 ? 2 : 4, B = p->B;
-  return up(B * p->dp * 4) + 2 * up(B * p->dp * e) + up(B * s.in * e) + up(B * s.q * e) + up(B * s.cq * e) +
+  return 2 * up(B * p->dp * 4) + 2 * up(B * p->dp * e) + up(B * s.in * e) + up(B * s.q * e) + up(B * s.cq * e) +
          up(B * s.ao * e) + up(B * s.o * e) + up(B * s.gu * e) + up(B * s.ff * e) + up(s.mix_ws) + up(B * s.top * p->dp * e) +
          3 * up(B * s.top * 4) + up(s.moe_ws) + up(B * s.values * e) + up(parts_bytes(p));
 }
@@ -120,6 +129,7 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
   char* w = (char*)p->ws;
   auto take = [&](int64_t bytes) { char* r = w; w += up(bytes); return r; };
   float* x = (float*)take(B * dp * 4);
+  float* x2 = (float*)take(B * dp * 4);   // the stream behind a norm that a product has made (workgroups that read x may still run)
   void* h = take(B * dp * e);
   void* y = take(B * dp * e);
   void* in = take(B * s.in * e);
@@ -144,8 +154,41 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
                                post, p->eps, pre, p->eps, h, dp, B, p->d, dp, p->rms, last ? lengths : nullptr, slots,
                                last ? (int)B : 0, p->dtype, stream);
   };
-  // the stream += norm(in W^T), then its next norm: with few rows the product leaves slices that the norm adds up
-  auto into_stream = [&](const void* xin, const void* weight, int64_t K, const float* post, const float* pre, bool last) {
+  // 1 to 4 rows: the norm in front of a product is the product's own (STREAM of vy_few.hip)
+  struct { const float *post, *pre; bool last, due; } later{};
+  auto settle = [&]() {
+    if (!later.due) return (int)VY_OK;
+    later.due = false;
+    return norm(y, nullptr, later.post, later.pre, later.last);
+  };
+  // out = epilogue(h W^T + bias) behind whatever norm is due
+  auto from_stream = [&](int epi, const void* weight, const void* bias, int act, float cap, void* out, int64_t ldo, int64_t N) {
+    if (!later.due) return (int)VY_ERR_UNSUPPORTED;
+    const bool known = epi == vy_few::GATED ? act == VY_ACT_SILU || act == VY_ACT_GELU_TANH
+                                            : act == VY_ACT_NONE || act == VY_ACT_RELU2 || act == VY_ACT_SOFTCAP;
+    if (!known || !vy_few::few_k(epi, vy_few::STREAM, dp) || N > INT32_MAX / 2 || (uintptr_t)weight % 16 || (uintptr_t)later.post % 16 ||
+        (uintptr_t)later.pre % 16) {
+      const int bad = settle();
+      return bad ? bad : (int)VY_ERR_UNSUPPORTED;
+    }
+    vy_few::Args a{};
+    a.M = (int)B; a.x = (const bf16*)y; a.ldx = dp; a.s_in = x; a.s_out = x2; a.lds = dp;
+    a.w_post = later.post; a.w_pre = later.pre; a.n = p->d; a.rms = p->rms; a.eps = p->eps;
+    if (later.last) { a.advance = lengths; a.slots = slots; a.n_adv = (int)B; }
+    a.w = (const bf16*)weight; a.N = (int)N; a.bias = (const bf16*)bias; a.act = act; a.act_arg = cap; a.y = (bf16*)out; a.ldy = ldo;
+    later.due = false;
+    const int bad = vy_few::few_go(epi, vy_few::STREAM, a, dp, (hipStream_t)stream);
+    std::swap(x, x2);
+    return bad;
+  };
+  // the stream += norm(in W^T), then its next norm: with few rows the product leaves slices that the norm adds up, or the norm waits
+  // for the product that reads it (`own`: such a product is the next launch)
+  auto into_stream = [&](const void* xin, const void* weight, int64_t K, const float* post, const float* pre, bool last, bool own) {
+    if (own && p->dtype == VY_BF16 && B <= 4) {
+      const int bad = product(p, xin, weight, y, dp, dp, K, stream);
+      later = {post, pre, last, true};
+      return bad;
+    }
     const int n = parts_bytes(p) ? vy_rows_parts(xin, weight, parts, B, dp, K, (hipStream_t)stream) : 0;
     if (n)
       return vy_residual_norm_parts(x, dp, parts, n, post, pre, p->eps, h, dp, B, p->d, dp, p->rms, last ? lengths : nullptr, slots,
@@ -158,6 +201,7 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
     const vy_hybrid_layer& L = p->layers[l];
     const bool last = l + 1 == p->num_layers, parallel = L.form == VY_FORM_PARALLEL;
     const float* next = last ? p->final_norm : p->layers[l + 1].norm1;
+    const bool own = last || p->layers[l + 1].form != VY_FORM_PARALLEL;
     const int64_t nv = (int64_t)L.heads * L.vdim, nk = (int64_t)L.heads * L.dim, na = nv + (parallel ? L.ff : 0);
     if (parallel) {   // windowed attention beside clamped feed-forwards: the pieces of the layer share launches
       rc = vy_parallel_decode(p, &L, h, in, ao, y, erows, eids, ew, ews, s.moe_ws, slots, lengths, max_keys, mws, s.mix_ws, stream);
@@ -168,7 +212,9 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
       }
       if (rc != VY_ERR_UNSUPPORTED) return rc;
     }
-    if ((rc = product(p, h, L.w_in, in, L.n_in, L.n_in, dp, stream, L.b_in))) return rc;
+    rc = from_stream(vy_few::STORE, L.w_in, L.b_in, VY_ACT_NONE, 0.f, in, L.n_in, L.n_in);
+    if (rc == VY_ERR_UNSUPPORTED) rc = product(p, h, L.w_in, in, L.n_in, L.n_in, dp, stream, L.b_in);
+    if (rc) return rc;
     if (L.mixer == VY_MIX_LATENT) {
       if (!L.ring && max_keys > L.cap) VY_FAIL(VY_ERR_ARG, "%s: %ld keys exceed the cache capacity %d", who, (long)max_keys, L.cap);
       const int64_t nq = L.w_uq ? L.q_rank_p : nk;   // columns ahead of the key/value latent: the queries' latent, or the queries
@@ -227,7 +273,7 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
       continue;
     }
     if (!L.ff && !L.moe) {
-      if ((rc = into_stream(ao, L.w_o, nv, L.norm1b, next, last))) return rc;
+      if ((rc = into_stream(ao, L.w_o, nv, L.norm1b, next, last, own))) return rc;
       continue;
     }
     // few tokens: the choice of experts comes with the residual sum
@@ -240,15 +286,20 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
       if (rc && rc != VY_ERR_UNSUPPORTED) return rc;
       chosen = rc == VY_OK;
       if (!chosen && (rc = norm(y, nullptr, L.norm1b, L.norm2, false))) return rc;
-    } else if ((rc = into_stream(ao, L.w_o, nv, L.norm1b, L.norm2, false))) {
+    } else if ((rc = into_stream(ao, L.w_o, nv, L.norm1b, L.norm2, false, true))) {
       return rc;
     }
     if (L.ff) {
-      if (L.w_up) rc = product(p, h, L.w_up, act, L.ff, L.ff, dp, stream, nullptr, p->act);
-      else rc = gated(p, L, h, gu, act, stream);
+      if (L.w_up) {
+        rc = from_stream(vy_few::STORE, L.w_up, nullptr, p->act, 0.f, act, L.ff, L.ff);
+        if (rc == VY_ERR_UNSUPPORTED) rc = product(p, h, L.w_up, act, L.ff, L.ff, dp, stream, nullptr, p->act);
+      } else {
+        rc = from_stream(vy_few::GATED, L.w_gu, nullptr, L.clamped ? VY_ACT_NONE : p->act, 0.f, act, L.ff, L.ff);
+        if (rc == VY_ERR_UNSUPPORTED) rc = gated(p, L, h, gu, act, stream);
+      }
       if (rc) return rc;
       if (!L.moe) {
-        if ((rc = into_stream(act, L.w_down, L.ff, L.norm2b, next, last))) return rc;
+        if ((rc = into_stream(act, L.w_down, L.ff, L.norm2b, next, last, own))) return rc;
         continue;
       }
       if ((rc = product(p, act, L.w_down, y, dp, dp, L.ff, stream))) return rc;
@@ -262,5 +313,7 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
     if (rc) return rc;
     if ((rc = norm(L.ff ? y : nullptr, routed, L.norm2b, next, last))) return rc;
   }
-  return product(p, h, p->head, logits, ldv, p->vocab, dp, stream, nullptr, p->softcap > 0.f ? VY_ACT_SOFTCAP : VY_ACT_NONE, p->softcap);
+  const int cap = p->softcap > 0.f ? VY_ACT_SOFTCAP : VY_ACT_NONE;
+  rc = from_stream(vy_few::STORE, p->head, nullptr, cap, p->softcap, logits, ldv, p->vocab);
+  return rc == VY_ERR_UNSUPPORTED ? product(p, h, p->head, logits, ldv, p->vocab, dp, stream, nullptr, cap, p->softcap) : rc;
 }

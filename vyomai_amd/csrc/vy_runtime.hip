@@ -1,6 +1,7 @@
 // Native decode driver (host code): chains the kernel launchers for one single-token step so the
 // Python side makes ONE call per generated token.  See include/vyom_hip.h (vy_decoder_step).
 #include "vy_common.h"
+#include "vy_few.h"
 #include <stdlib.h>
 
 int vy_qkv_rope_fwd_ex(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,
@@ -69,6 +70,84 @@ extern "C" int64_t vy_decode_ws_bytes(int32_t B, int32_t d, int32_t h, int32_t h
          up((vy_splitk_ws_floats(d) > 24 * 32 * (int64_t)d ? vy_splitk_ws_floats(d) : 24 * 32 * (int64_t)d) * 4) + 4096;
 }
 
+// Do the kernels of vy_few.hip take the step's sizes and operands?  (whole 256-column pieces, weights on 16 bytes, norms on 8)
+static bool few_operands(const vy_decode_plan* p, const void* x, const void* logits) {
+  using namespace vy_few;
+  if (!few_k(QKV, PLAIN, p->d) || !few_k(QKV, LAYER, p->d) || !few_k(STORE, PLAIN, p->d) || !few_k(STORE, LAYER, p->d) ||
+      !few_k(STORE, PLAIN, p->ffn) || p->dh != 64 || p->h * 64 != p->d ||
+      (p->act != VY_ACT_NONE && p->act != VY_ACT_GELU_ERF && p->act != VY_ACT_GELU_TANH))
+    return false;
+  uintptr_t w = (uintptr_t)x, n = 0;
+  for (int l = 0; l < p->num_layers; ++l) {
+    const vy_decode_layer& L = p->layers[l];
+    w |= (uintptr_t)L.wqkv | (uintptr_t)L.wo | (uintptr_t)L.w1 | (uintptr_t)L.w2;
+    n |= (uintptr_t)L.ln1_w | (uintptr_t)L.ln1_b | (uintptr_t)L.ln2_w | (uintptr_t)L.ln2_b;
+  }
+  if (logits) {
+    w |= (uintptr_t)p->head_wd | (uintptr_t)p->head_wv;
+    n |= (uintptr_t)p->head_ln_w | (uintptr_t)p->head_ln_b;
+  }
+  return w % 16 == 0 && n % 8 == 0;
+}
+
+// The step of 1 to 4 sequences on the kernels of vy_few.hip: five launches per layer, LayerNorms inside the products behind them.
+static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos, const int32_t* pos_dev, void* hidden_out, void* logits,
+                            int64_t ldv, hipStream_t st) {
+  using namespace vy_few;
+  const int64_t e = 2;
+  const int B = p->B, d = p->d, h = p->h, hk = p->hk;
+  char* w = (char*)p->ws;
+  auto take = [&](int64_t n) { char* r = w; w += up(n * e); return (bf16*)r; };
+  bf16 *q = take(B * (int64_t)d), *ao = take(B * (int64_t)d), *s1 = take(B * (int64_t)d), *s2 = take(B * (int64_t)d);
+  bf16* hb[2] = {take(B * (int64_t)d), take(B * (int64_t)d)};
+  bf16* mid = take(B * (int64_t)p->ffn);
+  const bf16* cur = (const bf16*)x;   // the layer's input rows: of the first layer x, of the others LN2 of the layer before
+  const vy_decode_layer* before = nullptr;
+  int rc;
+  for (int l = 0; l < p->num_layers; ++l) {
+    const vy_decode_layer& L = p->layers[l];
+    Args a{};
+    a.M = B; a.w = (const bf16*)L.wqkv; a.bias = (const bf16*)L.bqkv; a.N = (h + 2 * hk) * 64;
+    a.q = q; a.k = (bf16*)L.kcache; a.v = (bf16*)L.vcache; a.c_sb = L.c_sb; a.c_sh = L.c_sh; a.c_sl = L.c_sl;
+    a.cos_tab = p->cos_tab; a.sin_tab = p->sin_tab; a.pos_dev = pos_dev; a.pos = (int)pos; a.nq = h * 64; a.nkv = hk * 64;
+    if (before) {
+      a.x = s2; a.ldx = d; a.ln_g = (const bf16*)before->ln2_w; a.ln_b = (const bf16*)before->ln2_b; a.eps = p->eps_ffn;
+      a.h = hb[l & 1]; a.ldh = d;
+      cur = hb[l & 1];
+    } else {
+      a.x = cur; a.ldx = d;
+    }
+    if ((rc = few_go(QKV, before ? LAYER : PLAIN, a, d, st))) return rc;
+    if ((rc = vy_attn_decode_ex(q, d, 64, L.kcache, L.c_sb, L.c_sh, L.c_sl, L.vcache, L.c_sb, L.c_sh, L.c_sl, ao, d, B, h, hk, pos + 1,
+                                pos_dev, 64, 0.125f, VY_BF16, st))) return rc;
+    Args o{};
+    o.M = B; o.x = ao; o.ldx = d; o.w = (const bf16*)L.wo; o.bias = (const bf16*)L.bo; o.N = d; o.residual = cur; o.ldr = d;
+    o.y = s1; o.ldy = d;
+    if ((rc = few_go(STORE, PLAIN, o, d, st))) return rc;
+    Args f{};
+    f.M = B; f.x = s1; f.ldx = d; f.ln_g = (const bf16*)L.ln1_w; f.ln_b = (const bf16*)L.ln1_b; f.eps = p->eps_attn;
+    f.w = (const bf16*)L.w1; f.bias = (const bf16*)L.b1; f.N = p->ffn; f.act = p->act; f.y = mid; f.ldy = p->ffn;
+    if ((rc = few_go(STORE, LAYER, f, d, st))) return rc;
+    Args g{};
+    g.M = B; g.x = mid; g.ldx = p->ffn; g.w = (const bf16*)L.w2; g.bias = (const bf16*)L.b2; g.N = d; g.residual = cur; g.ldr = d;
+    g.y = s2; g.ldy = d;
+    if ((rc = few_go(STORE, PLAIN, g, p->ffn, st))) return rc;
+    before = &L;
+  }
+  if (!logits)
+    return hidden_out ? vy_layernorm_fwd(s2, d, before->ln2_w, before->ln2_b, hidden_out, d, nullptr, nullptr, B, d, p->eps_ffn, VY_BF16, st)
+                      : VY_OK;
+  Args a{};
+  a.M = B; a.x = s2; a.ldx = d; a.ln_g = (const bf16*)before->ln2_w; a.ln_b = (const bf16*)before->ln2_b; a.eps = p->eps_ffn;
+  a.h = (bf16*)hidden_out; a.ldh = d; a.w = (const bf16*)p->head_wd; a.bias = (const bf16*)p->head_bd; a.N = d; a.act = VY_ACT_GELU_ERF;
+  a.y = s1; a.ldy = d;
+  if ((rc = few_go(STORE, LAYER, a, d, st))) return rc;
+  Args v{};
+  v.M = B; v.x = s1; v.ldx = d; v.ln_g = (const bf16*)p->head_ln_w; v.ln_b = (const bf16*)p->head_ln_b; v.eps = p->eps_head;
+  v.w = (const bf16*)p->head_wv; v.once = 1; v.bias = (const bf16*)p->head_bias; v.N = p->vocab; v.y = (bf16*)logits; v.ldy = ldv;
+  return few_go(STORE, LAYER, v, d, st);
+}
+
 extern "C" int vy_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos, const int32_t* pos_dev,
                                void* hidden_out, void* logits, int64_t ldv, void* stream) {
   const char* who = "vy_decoder_step";
@@ -96,6 +175,8 @@ extern "C" int vy_decoder_step(const vy_decode_plan* p, const void* x, int64_t p
   if (g_decode_lean < 0) { const char* e = getenv("VY_DECODE_LEAN"); g_decode_lean = e ? atoi(e) : 1; }
   const bool lean = g_decode_lean && vy_dec_supported(B, d, h, hk, dh, p->ffn, p->dtype);
   hipStream_t hst = (hipStream_t)stream;
+  if (lean && B <= 4 && p->num_layers > 0 && (pos_dev || pos >= 0) && few_operands(p, x, logits))
+    return few_decoder_step(p, x, pos, pos_dev, hidden_out, logits, ldv, hst);
   const void* cur = x;
   for (int l = 0; l < p->num_layers; ++l) {
     const vy_decode_layer& L = p->layers[l];
