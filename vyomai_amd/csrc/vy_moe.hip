@@ -11,7 +11,7 @@
 // Few tokens (decode): expert_rows_kernel streams the weights of the experts in use straight into MFMA operands (vy_rows.h), one
 // workgroup per 16 or 32 weight rows of an expert; which experts and tokens, every workgroup reads from the choice itself.
 // Many tokens (prefill): tokens are sorted by expert (ranks from the choice kernel, offsets in the scatter kernel) and
-// grouped_gemm_kernel runs 128 x 128 tiles over the experts' row ranges, gathering its rows of h on the way into LDS.
+// grouped_gemm_kernel runs 128 x 128 or 256 x 256 tiles over the experts' row ranges, gathering its rows of h on the way into LDS.
 // fp32 takes the same way with a plain tile kernel.  A row's result does not depend on its place or on other rows.
 #include "vy_moe.h"
 
@@ -194,21 +194,23 @@ __device__ __forceinline__ bool grouped_tile(const GroupedArgs& a, int tiles_n, 
 
 constexpr int BK = 64, ROWB = BK * 2;
 
-// 128 x 128 x 64 tiles, two LDS stages, four waves of 64 x 64 on mfma_f32_16x16x32_bf16 (the structure of
-// gemm_nt_bf16_m16_kernel).  GU: rows gathered, activation in the epilogue, half as many output columns.
-template <int KIND>
-__global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedArgs a) {
-  constexpr int BM = 128, BN = 128, NW = 4, TM = 4, TN = 4, GX = BM / 8 / NW, GW = BN / 8 / NW;
+// BM x BN x 64 tiles, two LDS stages, waves of 16 TM x 16 TN on mfma_f32_16x16x32_bf16 (the structure of gemm_nt_bf16_m16_kernel):
+// 128 x 128 with four waves, two workgroups on a CU, or 256 x 256 with eight (tile_rows).  Bound as that kernel is, by loads and
+// products of a stage that overlap in part; 64 experts of 2048 -> 2 x 1024 -> 2048 over 32772 rows: 741 / 679 TFLOP/s on 128 x 128,
+// 866 / 791 on 256 x 256.  GATE_UP: rows gathered, activation in the epilogue, half as many output columns.
+template <int KIND, int BM, int BN, int WGM, int WGN>
+__global__ __launch_bounds__(64 * WGM * WGN) void grouped_gemm_kernel(GroupedArgs a) {
+  constexpr int NW = WGM * WGN, TM = BM / (16 * WGM), TN = BN / (16 * WGN), GX = BM / 8 / NW, GW = BN / 8 / NW;
   constexpr int STAGE = (BM + BN) * ROWB, ON = KIND == GATE_UP ? BN / 2 : BN, OROW = ON * 2 + 16;
-  static_assert(BM * OROW <= 2 * STAGE, "the output tile fits");
-  __shared__ __attribute__((aligned(16))) char smem[2 * STAGE];
+  __shared__ __attribute__((aligned(16))) char smem[BM * OROW > 2 * STAGE ? BM * OROW : 2 * STAGE];
   int e, mt, nt;
   if (!grouped_tile(a, (a.N + BN - 1) / BN, e, mt, nt)) return;
   const int rows = a.count[e] - mt * BM, row0 = a.offset[e] + mt * BM, n0 = nt * BN;
   const int N = a.N, K = a.K;
   const bf16* W = (const bf16*)a.w + (int64_t)e * N * K;
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave >> 1, wn = wave & 1;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), wm = wave / WGN, wn = wave % WGN;
+  const bool live = wm * 16 * TM < rows;   // (the waves behind an expert's last row only load)
   const int lrow = lane >> 3, slot = lane & 7;
   const bf16* xsrc[GX]; int xk[GX];
   const bf16* wsrc[GW]; int wk[GW];
@@ -234,6 +236,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedArgs a) {
     const int k0 = kt * BK;
 #pragma unroll
     for (int t = 0; t < GX; ++t) {
+      if ((wave + NW * t) * 8 >= rows) continue;   // (rows of the image that nobody stores)
       const bf16* s = xsrc[t] + k0;
       if (ktail && k0 + xk[t] >= K) s = zero;
       __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
@@ -282,22 +285,31 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedArgs a) {
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
-  read_frags(wa[0], xa[0], wf[0], xf[0]);
-  for (int kt = 0; kt < KT; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < KT) stage(kt + 1, cur ^ 1);
-    const unsigned boff = cur * STAGE;
-    read_frags(wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TN + TM) : "memory");
-    tie_frags(wf[0], xf[0]);
-    mma(wf[0], xf[0]);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    tie_frags(wf[1], xf[1]);
-    mma(wf[1], xf[1]);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
+  if (live) {
+    read_frags(wa[0], xa[0], wf[0], xf[0]);
+    for (int kt = 0; kt < KT; ++kt) {
+      const int cur = kt & 1;
+      if (kt + 1 < KT) stage(kt + 1, cur ^ 1);
+      const unsigned boff = cur * STAGE;
+      read_frags(wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TN + TM) : "memory");
+      tie_frags(wf[0], xf[0]);
+      mma(wf[0], xf[0]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      tie_frags(wf[1], xf[1]);
+      mma(wf[1], xf[1]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
+    }
+  } else {   // (the same barriers)
+    for (int kt = 0; kt < KT; ++kt) {
+      if (kt + 1 < KT) stage(kt + 1, (kt & 1) ^ 1);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+    }
   }
   // every wave is behind the loop's last barrier: the stages are free.  Lane: token r16 of block j, columns 4 kq .. of block i
 #pragma unroll
@@ -322,7 +334,7 @@ __global__ __launch_bounds__(256) void grouped_gemm_kernel(GroupedArgs a) {
   __syncthreads();
   constexpr int CPR = ON / 8;
   const int NO = KIND == GATE_UP ? N / 2 : N, c0 = KIND == GATE_UP ? n0 / 2 : n0;
-  for (int i = tid; i < BM * CPR; i += 256) {
+  for (int i = tid; i < BM * CPR; i += 64 * NW) {
     const int r = i / CPR, ch = (i % CPR) * 8;
     if (r < rows && c0 + ch < NO)
       *reinterpret_cast<bf16x8*>((bf16*)a.y + (int64_t)(row0 + r) * a.ldy + c0 + ch) = *reinterpret_cast<const bf16x8*>(smem + r * OROW + ch * 2);
@@ -414,10 +426,29 @@ bool few(const vy_moe* d, int64_t M, int dtype) {
   const int64_t n = M * d->top;
   return dtype == VY_BF16 && n <= MAX_ENTRIES && (M <= 64 || n <= 24 * (int64_t)d->experts);
 }
-int tile_rows(int dtype) { return dtype == VY_BF16 ? 128 : 64; }
-int64_t max_tiles(const vy_moe* d, int64_t M, int dtype) {   // every expert in use may end with a partial tile
+// Rows (and columns) of a tile: the size on which both products take the shorter time, in rounds over the 256 CUs.  A round of 256
+// x 256 takes 1.55 us a stage, one of 128 x 128 -- two on a CU, half the outputs -- 1.0; the rows that fill up an expert's last tile
+// (half a tile each, of as many experts as rows can reach) and a last round that leaves CUs idle (up to 30 % faster) decide.
+// Both products, 128 / 256, width 2048 and 64 experts of 1024: 512 rows an expert 573 / 491 us, 256 rows 351 / 341, 125 rows
+// 241 / 265; width 1024 and 32 experts of 512: 1024 rows 186 / 171, 512 rows 109 / 114, 256 rows 74 / 63, 125 rows 43 / 55.
+int tile_rows(const vy_moe* d, int64_t M, int dtype) {
+  if (dtype != VY_BF16) return 64;
+  const double n = (double)M * d->top, experts = n < d->experts ? n : d->experts;
+  auto cost = [&](int t, int per_cu, double stage, double fixed) {
+    double rows = n / t + experts / 2, us = 0;
+    if (rows < experts) rows = experts;
+    const int64_t NK[2][2] = {{(d->act == VY_MOE_CLAMPED ? 2 : 1) * (int64_t)d->ff, d->width}, {d->width, d->ff}};
+    for (auto& s : NK) {
+      const double r = rows * (double)vy_cdiv(s[0], t) / (256 * per_cu), whole = floor(r), part = r - whole;
+      us += (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0)) * stage * (double)vy_cdiv(s[1], 64);
+    }
+    return us;
+  };
+  return cost(256, 1, 1.55, 8.0) < cost(128, 2, 1.0, 5.0) ? 256 : 128;
+}
+int64_t max_tiles(const vy_moe* d, int64_t M, int rows) {   // every expert in use may end with a partial tile
   const int64_t n = M * d->top, e = n < d->experts ? n : d->experts;
-  return n / tile_rows(dtype) + e;
+  return n / rows + e;
 }
 
 struct Parts { float* logits; char* act; int* counts; int* rank; int* token; int* offset; int* rows; int* ntiles; Tile* tiles; };
@@ -434,7 +465,7 @@ int64_t lay_out(const vy_moe* d, int64_t M, int dtype, char* ws, Parts& p) {
   p.offset = (int*)take(d->experts * 4);
   p.rows = (int*)take(d->experts * 4);
   p.ntiles = (int*)take(4);
-  p.tiles = (Tile*)take(max_tiles(d, M, dtype) * (int64_t)sizeof(Tile));
+  p.tiles = (Tile*)take(max_tiles(d, M, dtype == VY_BF16 ? 128 : 64) * (int64_t)sizeof(Tile));
   return at - ws;
 }
 
@@ -527,17 +558,23 @@ extern "C" int vy_moe_fwd(const vy_moe* d, const void* h, int64_t ldh, int64_t M
     VY_CHECK_LAUNCH(who);
     return VY_OK;
   }
-  const int bm = tile_rows(dtype);
+  const int bm = tile_rows(d, M, dtype);
   SortArgs s{ids, p.rank, p.counts, n, d->top, E, bm, pos, p.token, p.offset, p.rows, p.tiles, p.ntiles};
   hipLaunchKernelGGL(sort_kernel, dim3((unsigned)vy_cdiv(n, 256)), block, 0, st, s);
   GroupedArgs g{h, ldh, p.token, p.offset, p.rows, p.tiles, p.ntiles, d->w_gu, up_rows, K, p.act, d->ff, d->limit, d->alpha};
   GroupedArgs o{p.act, d->ff, nullptr, p.offset, p.rows, p.tiles, p.ntiles, d->w_down, K, d->ff, rows, ldr, 0.f, 0.f};
-  const int64_t tiles = max_tiles(d, M, dtype);
+  const int64_t tiles = max_tiles(d, M, bm);
   const dim3 ggrid((unsigned)(tiles * vy_cdiv(g.N, bm))), ogrid((unsigned)(tiles * vy_cdiv(o.N, bm)));
   if (dtype == VY_BF16) {
-    if (gated) hipLaunchKernelGGL((grouped_gemm_kernel<GATE_UP>), ggrid, block, 0, st, g);
-    else hipLaunchKernelGGL((grouped_gemm_kernel<UP>), ggrid, block, 0, st, g);
-    hipLaunchKernelGGL((grouped_gemm_kernel<DOWN>), ogrid, block, 0, st, o);
+    if (bm == 256) {
+      if (gated) hipLaunchKernelGGL((grouped_gemm_kernel<GATE_UP, 256, 256, 4, 2>), ggrid, dim3(512), 0, st, g);
+      else hipLaunchKernelGGL((grouped_gemm_kernel<UP, 256, 256, 4, 2>), ggrid, dim3(512), 0, st, g);
+      hipLaunchKernelGGL((grouped_gemm_kernel<DOWN, 256, 256, 4, 2>), ogrid, dim3(512), 0, st, o);
+    } else {
+      if (gated) hipLaunchKernelGGL((grouped_gemm_kernel<GATE_UP, 128, 128, 2, 2>), ggrid, block, 0, st, g);
+      else hipLaunchKernelGGL((grouped_gemm_kernel<UP, 128, 128, 2, 2>), ggrid, block, 0, st, g);
+      hipLaunchKernelGGL((grouped_gemm_kernel<DOWN, 128, 128, 2, 2>), ogrid, block, 0, st, o);
+    }
   } else {
     if (gated) hipLaunchKernelGGL((grouped_gemm_f32_kernel<GATE_UP>), ggrid, block, 0, st, g);
     else hipLaunchKernelGGL((grouped_gemm_f32_kernel<UP>), ggrid, block, 0, st, g);
