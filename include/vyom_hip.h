@@ -81,6 +81,11 @@ int vy_linear_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const 
 /* vy_linear_softcap_fwd: Y = cap * tanh(X . W^T / cap), a vocabulary product whose logits stay within +-cap. */
 int vy_linear_softcap_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t M, int64_t N,
                           int64_t K, float cap, int dtype, void* stream);
+/* vy_linear_gated_fwd: Y[M,I] = act(X . Wg^T) * (X . Wu^T), W = [Wg; Wu] (2 I rows), both products rounded to bf16 first: what
+ * vy_linear_fwd and vy_gated_act_fwd compute, in one launch.  act: VY_ACT_SILU or VY_ACT_GELU_TANH.  VY_ERR_UNSUPPORTED, with nothing
+ * launched and no message: f32, M <= 32, I % 8 != 0, other activations, and shapes that are faster with K split. */
+int vy_linear_gated_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t M, int64_t I,
+                        int64_t K, int act, int dtype, void* stream);
 
 /* ------------------------------------------------------------------------------------------
  * vy_qkv_rope_fwd: fused Q/K/V projection + bias + rotary embedding + head split.

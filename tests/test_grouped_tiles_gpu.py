@@ -11,8 +11,8 @@ BF = torch.bfloat16
 @pytest.mark.parametrize("width,ff", [(136, 200), (1096, 1032)])
 @pytest.mark.parametrize("counts", [[0, 1, 128, 129], [190, 190, 190, 197], [0, 1, 256, 511], [257, 700, 64, 65], [0, 1, 9000, 257]])
 def test_rows_of_uneven_experts(act, width, ff, counts):
-    """One expert per token, forced by the token's first columns.  A row's activations and its outputs are rounded to bf16, 2^-9
-    relative each, the sums are fp32."""
+    """One expert per token, forced by the token's first columns.  A row's activations and its outputs are rounded to bf16 (half a unit in the
+    last of 8 bits: at most 2^-8 of the value), the sums are fp32."""
     from vyomai_amd.layers.ffn import MixtureFeedForward
     E, M = len(counts), sum(counts)
     g = torch.Generator().manual_seed(M + width)
@@ -43,5 +43,5 @@ def test_rows_of_uneven_experts(act, width, ff, counts):
         else:
             a = torch.nn.functional.gelu(u)
         want = a @ weights["down"][e].T
-        bound = 2.0 ** -9 * (a.abs() @ weights["down"][e].abs().T + want.abs()) * 1.01 + 1e-4
+        bound = 2.0 ** -8 * (a.abs() @ weights["down"][e].abs().T + want.abs()) * 1.01 + 1e-4
         assert ((rows[want_ids == e] - want).abs() <= bound).all(), e

@@ -15,6 +15,7 @@ LIB_PATH = os.environ.get("VY_LIB_PATH") or os.path.join(_HERE, "lib", "libvyom_
 
 VY_F32, VY_BF16 = 0, 1
 ACT_NONE, ACT_GELU_ERF, ACT_GELU_TANH, ACT_SILU, ACT_RELU2 = 0, 1, 2, 3, 4
+ERR_UNSUPPORTED = -2
 ACT_SAVE_DERIV = 0x100   # saved tensor = act'(pre) instead of pre (include/vyom_hip.h)
 MOE_CLAMPED, MOE_GELU = 0, 1
 SCORE_SOFTMAX, SCORE_SIGMOID = 0, 1
@@ -37,6 +38,7 @@ PROTOTYPES = {
                        _p, _i64, _i64, _i, _i, _i64, _i, _f, _i, _p],
     "vy_layernorm_fwd": [_p, _i64, _p, _p, _p, _i64, _p, _p, _i64, _i64, _f, _i, _p],
     "vy_rmsnorm_fwd": [_p, _i64, _p, _p, _i64, _i64, _i64, _f, _f, _i, _p],
+    "vy_linear_gated_fwd": [_p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i64, _i, _i, _p],
     "vy_gated_act_fwd": [_p, _i64, _p, _i64, _i64, _i64, _i, _i, _p],
     "vy_rope_fwd": [_p, _i64, _i64, _i64, _p, _p, _i64, _i64, _i, _i64, _i, _i, _i, _p],
     "vy_linear_dgrad": [_p, _i64, _p, _i64, _p, _i64, _i, _p, _i64, _p, _i64, _p, _i64, _i64, _i64, _i64, _i, _p],

@@ -309,6 +309,18 @@ constexpr int epi_lds_bytes(int BM, int BN, int EPI, int PASSES) {
 }
 constexpr int vy_cmax(int a, int b) { return a > b ? a : b; }
 
+// Row of W behind row R of a tile's image.  EPI 2 (W = [gate; up], N = 2 I): blocks of 16 gate rows and the 16 up rows of the same
+// outputs in turn, so that a lane's accumulators of neighbouring blocks are the two factors of its outputs.
+template <int EPI>
+__device__ __forceinline__ int w_row(int n0, int R, int N) {
+  if constexpr (EPI == 2) {
+    const int I = N >> 1, j = (n0 >> 1) + ((R >> 5) << 4) + (R & 15);
+    return ((R >> 4) & 1) * I + (j < I ? j : I - 1);
+  } else {
+    return n0 + R < N ? n0 + R : N - 1;
+  }
+}
+
 // ---- shared epilogue of the bf16 kernels ------------------------------------------------------
 // PASSES > 1: the staged tile does not fit next to a second resident workgroup's LDS, so it goes out in
 // PASSES row bands of BM / PASSES rows (each band is owned by whole wave rows: WGM % PASSES == 0).
@@ -352,6 +364,33 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
     for (int e = 0; e < 4; ++e) w[e] = (bf16)v[e];
     *reinterpret_cast<bf16x4*>(et + (row - my_pass * RP) * EROW + col * 2) = w;
   };
+  if constexpr (EPI == 2) {
+    // act(gate) * up of the two roundings, half as many columns as the tile has rows of W
+    constexpr int TM16 = BM / (16 * WGM), TN16 = BN / (16 * WGN), GROW = BN + 16, GPR = BN / 16;
+    static_assert(MF16 && TN16 % 2 == 0, "gate and up blocks of a wave come in pairs");
+    const int r16 = lane & 15, kq = lane >> 4;
+#pragma unroll
+    for (int i = 0; i < TN16; i += 2)
+#pragma unroll
+      for (int j = 0; j < TM16; ++j) {
+        bf16x4 o;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (bf16)(vy_act_fwd<ACT>(vy_round_bf16(acc[i][j][e])) * vy_round_bf16(acc[i + 1][j][e]));
+        *reinterpret_cast<bf16x4*>(et + (wm * 16 * TM16 + 16 * j + r16) * GROW + (wn * 8 * TN16 + 8 * i + 4 * kq) * 2) = o;
+      }
+    __syncthreads();
+    const int I = N >> 1, j0 = n0 >> 1;
+    for (int c = tid; c < BM * GPR; c += NT) {
+      const int row = c / GPR, ch = (c - row * GPR) * 8;
+      if (m0 + row < M && j0 + ch < I) {   // (I is a multiple of 8)
+        const bf16x8 o = *reinterpret_cast<const bf16x8*>(et + row * GROW + ch * 2);
+        bf16* at = ep.y + (int64_t)(m0 + row) * ep.ldy + j0 + ch;
+        if (ep.wt_store) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(at), "v"(o) : "memory");
+        else *reinterpret_cast<bf16x8*>(at) = o;
+      }
+    }
+    return;
+  }
   // bias of a register quad (depends on the lane half only); loaded at use, not kept live
   const bf16* biasp = EPI == 0 ? ep.bias : eq.bias;
   const bool bias_vec = (reinterpret_cast<uintptr_t>(biasp) & 7) == 0;
@@ -541,7 +580,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
       flush_plain(ep.y, true, dual, pass);
       if (pass + 1 < PASSES) __syncthreads();
     }
-  } else {
+  } else if constexpr (EPI == 1) {
     // QKV: bias in registers; RoPE and the head-split scatter in phase 2, where a rotary pair
     // (d, d+32) is two 16-byte chunks 64 bytes apart in the same staged row.  The staged values
     // are the bf16-rounded projections, so the rotation reproduces the reference's op order
@@ -862,8 +901,7 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
   for (int t = 0; t < GW; ++t) {
     const int R = (wave + NW * t) * 8 + lrow;
     const int g = slot ^ ((R >> 1) & 7);
-    int gn = n0 + R; gn = gn < N ? gn : N - 1;
-    wsrc[t] = W + (int64_t)gn * ldw + g * 8;
+    wsrc[t] = W + (int64_t)w_row<EPI>(n0, R, N) * ldw + g * 8;
     wk[t] = g * 8;
   }
   const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
@@ -996,8 +1034,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   for (int t = 0; t < GW; ++t) {
     const int R = (wave + NW * t) * 8 + lrow;
     const int g = slot ^ ((R >> 1) & 7);
-    int gn = n0 + R; gn = gn < N ? gn : N - 1;
-    wsrc[t] = W + (int64_t)gn * ldw + g * 8;
+    wsrc[t] = W + (int64_t)w_row<EPI>(n0, R, N) * ldw + g * 8;
     wk[t] = g * 8;
   }
   const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
@@ -1123,9 +1160,8 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     const int R = (wave + NW * t) * 8 + lrow;
     const int g = slot ^ ((R >> 1) & 7);
     int gm = m0 + R; gm = gm < M ? gm : M - 1;
-    int gn = n0 + R; gn = gn < N ? gn : N - 1;
     xsrc[t] = X + (int64_t)gm * ldx + g * 8;
-    wsrc[t] = W + (int64_t)gn * ldw + g * 8;
+    wsrc[t] = W + (int64_t)w_row<EPI>(n0, R, N) * ldw + g * 8;
     kcol[t] = g * 8;
   }
   const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
@@ -2272,6 +2308,29 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
   return 0;
 }
 
+// act(X Wg^T) * (X Wu^T), W = [Wg; Wu]: the products of more than 32 rows whose tiles hold both factors of an output.  Against the
+// product and a pass over its result (bound by memory: 400 MB at 8192 x 8192), 8192 x 2 x 8192, K = 2048: 589 -> 501 us;
+// 8000 x 2 x 4096, K = 1024: 163 -> 134; 700 x 2 x 4096, K = 1024: 25.8 -> 20.6; 100 rows: 10.3 -> 6.8.
+template <int ACT>
+int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K, const EpiPlain<bf16>& ep, hipStream_t st) {
+  int64_t ws_bytes;
+  splitk_ws(st, 0, &ws_bytes);
+  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes);
+  const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, TILE_M[t.kind]) * tn;
+#define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
+  switch (t.kind) {
+    case T_256x256: VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, 2, ACT, false>); break;
+    case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, 2, ACT, false>); break;
+    case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, 2, ACT, false>); break;
+    case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, 2, ACT, false>); break;
+    case T_64x64: VY_TILES(gemm_nt_bf16_small_kernel<1, 3, 2, ACT, false>); break;
+    case T_64x64_TWICE: VY_TILES(gemm_nt_bf16_small_kernel<2, 3, 2, ACT, false>); break;
+    default: return VY_ERR_UNSUPPORTED;   // (K split over workgroups)
+  }
+#undef VY_TILES
+  return VY_OK;
+}
+
 template <int EPI, int ACT, bool GRAD>
 int launch_f32(const float* X, int64_t ldx, const float* W, int64_t ldw, int64_t M, int64_t N,
                int64_t K, const EpiPlain<float>& ep, const EpiQkv<float>& eq, hipStream_t st) {
@@ -2424,6 +2483,23 @@ extern "C" int vy_linear_softcap_fwd(const void* x, int64_t ldx, const void* w, 
   if (dtype == VY_F32)
     return linear_impl<float>(x, ldx, w, ldw, nullptr, nullptr, 0, nullptr, 0, y, ldy, nullptr, M, N, K, VY_ACT_SOFTCAP, false, st, who, nullptr, 0, VyDrop{}, cap);
   VY_FAIL(VY_ERR_ARG, "%s: bad dtype %d", who, dtype);
+}
+
+extern "C" int vy_linear_gated_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, void* y, int64_t ldy, int64_t M, int64_t I,
+                                   int64_t K, int act, int dtype, void* stream) {
+  const char* who = "vy_linear_gated_fwd";
+  if (dtype != VY_BF16 || M <= 32 || I < 8 || I % 8 || I > INT32_MAX / 2 || (act != VY_ACT_SILU && act != VY_ACT_GELU_TANH))
+    return VY_ERR_UNSUPPORTED;
+  if (int rc = check_operands<bf16>(who, x, ldx, w, ldw, M, 2 * I, K)) return rc;
+  if (!y || ldy < I || ldy % 8 || !aligned_to(y, 16)) VY_FAIL(VY_ERR_ARG, "%s: output rows must be 16-byte aligned (ldy=%ld)", who, (long)ldy);
+  EpiPlain<bf16> ep{};
+  ep.y = (bf16*)y; ep.ldy = ldy;
+  ep.wt_store = M * I * 2 >= (16 << 20);
+  const int rc = act == VY_ACT_SILU ? launch_gated<VY_ACT_SILU>((const bf16*)x, ldx, (const bf16*)w, ldw, M, 2 * I, K, ep, (hipStream_t)stream)
+                                    : launch_gated<VY_ACT_GELU_TANH>((const bf16*)x, ldx, (const bf16*)w, ldw, M, 2 * I, K, ep, (hipStream_t)stream);
+  if (rc) return rc;
+  VY_CHECK_LAUNCH(who);
+  return VY_OK;
 }
 
 extern "C" int vy_linear_dropout_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,

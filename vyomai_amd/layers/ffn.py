@@ -78,7 +78,8 @@ class GatedFeedForward(nn.Module):
 
     def forward(self, h: torch.Tensor) -> torch.Tensor:
         p = self.packed()
-        return ops.linear(self.activation(ops.linear(h, p.w_gu)), p.w_down)
+        mid = ops.gated_linear(h, p.w_gu, self.act) if not self.clamped else self.activation(ops.linear(h, p.w_gu))
+        return ops.linear(mid, p.w_down)
 
     # what a layer asks of its feed-forward: the part that runs on every token, and the routed rows beside it
     @property

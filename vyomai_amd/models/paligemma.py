@@ -146,8 +146,7 @@ class GemmaMLP(nn.Module):
 
     def forward(self, x, residual=None):
         w, _ = _packed([self.gate_proj, self.up_proj], self, "_gu")
-        gu = ops.linear(x, w)                       # one GEMM for [gate | up]
-        act = ops.gated_act(gu, ACT_GELU_TANH)      # gelu_tanh(gate) * up
+        act = ops.gated_linear(x, w, ACT_GELU_TANH)   # gelu_tanh(gate) * up, one GEMM for [gate | up]
         return ops.linear(act, self.down_proj.weight, residual=residual)
 
 

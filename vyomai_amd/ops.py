@@ -229,6 +229,26 @@ def linear_softcap(x: Tensor, w: Tensor, cap: float) -> Tensor:
     return y[:, :N]
 
 
+def gated_linear(x: Tensor, w: Tensor, act: int) -> Tensor:
+    """act(x @ wg.T) * (x @ wu.T), w = [wg; wu], both products rounded first.  (vy_linear_gated_fwd; where that does not cover the
+    call, linear and gated_act)"""
+    I = w.shape[0] // 2
+    if not _Lanes.active and x.dtype == torch.bfloat16 and w.dtype == x.dtype and I % 8 == 0 and w.shape[0] == 2 * I:
+        _need_gpu(x, w)
+        x2 = _rows(x)
+        M, K = x2.shape
+        assert w.shape[1] == K and w.stride(1) == 1
+        _mid_ws(M)
+        out = torch.empty((M, I), dtype=x.dtype, device=x.device)
+        rc = _lib.load().vy_linear_gated_fwd(x2.data_ptr(), x2.stride(0), w.data_ptr(), w.stride(0), out.data_ptr(), I, M, I, K, act,
+                                             dtype_code(x.dtype), _stream())
+        if rc == 0:
+            return out.view(*x.shape[:-1], I)
+        if rc != _lib.ERR_UNSUPPORTED:
+            raise _lib.VyomHipError(f"vy_linear_gated_fwd failed ({rc}): {_lib.load().vy_last_error().decode()}")
+    return gated_act(linear(x, w), act)
+
+
 def qkv_rope(x: Tensor, w_packed: Tensor, b_packed: Optional[Tensor], h: int, hk: int, dh: int,
              cos: Optional[Tensor], sin: Optional[Tensor], pos0: int,
              q: Tensor, k: Tensor, v: Tensor) -> None:
