@@ -321,6 +321,53 @@ __device__ __forceinline__ int w_row(int n0, int R, int N) {
   }
 }
 
+// ---- activations by table ----------------------------------------------------------------------
+// An activation's input is a bf16 -- the rounded product -- so its values are looked up: every workgroup of a 256-row tile fills a
+// table in LDS while its first stage is on its way, with the very expressions that it replaces (the same bits), for 2^-20 <= |x| < 16
+// and both signs; a wave with any other value in its chunk evaluates them.  Evaluated, the erf GELU's 21 vector instructions an element
+// (two at a quarter of the rate) were 9 of the 15 us that the epilogue of a 256 x 256 tile took next to a loop of 19 us (K = 768).
+// Tile sizes whose stages leave no room for it (256 x 192, and the smaller ones that share a CU) evaluate.
+// 16384 x 3072, K = 768: 107 -> 95 us, with the derivative saved 112 -> 95; 30500 rows 195 -> 171 and 218 -> 181; gated SiLU (there the
+// division), 8192 x 2 x 8192, K = 2048: 508 -> 501 us, 8192 x 2 x 4096, K = 1024: 135 -> 132.
+constexpr unsigned ACT_TAB_LOW = (127 - 20) << 7, ACT_TAB_HALF = 24 << 7;   // first magnitude's bits, entries per sign
+constexpr bool act_has_table(int BM, int BN, int EPI, int ACT, bool GRAD) {
+  return BM == 256 && BN != 192 && !GRAD && (EPI == 0 ? ACT == VY_ACT_GELU_ERF || ACT == VY_ACT_GELU_TANH : EPI == 2);
+}
+constexpr int act_table_bytes(int BM, int BN, int EPI, int ACT, bool GRAD) {
+  return act_has_table(BM, BN, EPI, ACT, GRAD) ? 2 * ACT_TAB_HALF * 4 : 0;
+}
+// the bf16 value of act and, above it, of its derivative
+template <int ACT>
+__device__ __forceinline__ unsigned act_pair(float x, bool deriv) {
+  union { bf16 v[2]; unsigned u; } o;
+  if constexpr (ACT == VY_ACT_GELU_ERF) {   // both out of one evaluation of Phi and the Gaussian
+    float cdf, gs;
+    vy_phi_fast(x, cdf, gs);
+    o.v[1] = (bf16)(cdf + x * 0.39894228040143267794f * gs);
+    o.v[0] = (bf16)(x * cdf);
+  } else {
+    o.v[1] = deriv ? (bf16)vy_act_grad_fast<ACT>(x) : (bf16)0.f;
+    o.v[0] = (bf16)vy_act_fwd_fast<ACT>(x);
+  }
+  return o.u;
+}
+// EPI 0: act_pair; EPI 2: act as fp32, a factor of the gated product
+template <int EPI, int ACT>
+__device__ __forceinline__ void fill_act_table(unsigned* tab, bool deriv) {
+  for (unsigned i = threadIdx.x; i < 2 * ACT_TAB_HALF; i += blockDim.x) {
+    const unsigned bits = i < ACT_TAB_HALF ? ACT_TAB_LOW + i : 0x8000u + ACT_TAB_LOW + (i - ACT_TAB_HALF);
+    const float x = __builtin_bit_cast(float, bits << 16);
+    if constexpr (EPI == 0) tab[i] = act_pair<ACT>(x, deriv);
+    else tab[i] = __builtin_bit_cast(unsigned, vy_act_fwd<ACT>(x));
+  }
+}
+// entry of a bf16 (its bits in the low half of u); far: grows beyond ACT_TAB_HALF where there is none
+__device__ __forceinline__ unsigned act_entry(unsigned u, unsigned& far) {
+  const unsigned k = (u & 0x7fffu) - ACT_TAB_LOW;
+  far = k > far ? k : far;
+  return k + ((u >> 15) & 1) * ACT_TAB_HALF;
+}
+
 // ---- shared epilogue of the bf16 kernels ------------------------------------------------------
 // PASSES > 1: the staged tile does not fit next to a second resident workgroup's LDS, so it goes out in
 // PASSES row bands of BM / PASSES rows (each band is owned by whole wave rows: WGM % PASSES == 0).
@@ -337,7 +384,8 @@ template <int BM, int BN, int WGM, int WGN, bool MF16> struct AccTile {
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD, int PASSES = 1, bool PF_OK = true, bool MF16 = false>
 __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN, MF16>::type& acc, char* smem,
                                               int m0, int n0, int M, int N, const EpiPlain<bf16>& ep,
-                                              const EpiQkv<bf16>& eq) {
+                                              const EpiQkv<bf16>& eq, const unsigned* tab = nullptr) {
+  constexpr bool TAB = MF16 && act_has_table(BM, BN, EPI, ACT, GRAD);
   static_assert(!MF16 || PASSES == 1, "the 16 x 16 accumulator layout is staged in one pass");
   constexpr int NW = WGM * WGN, NT = 64 * NW;
   constexpr int TM = BM / (32 * WGM), TN = BN / (32 * WGN);
@@ -374,8 +422,24 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
 #pragma unroll
       for (int j = 0; j < TM16; ++j) {
         bf16x4 o;
+        float f[4];
+        bool known = false;
+        if constexpr (TAB) {
+          unsigned at[4], far = 0;
 #pragma unroll
-        for (int e = 0; e < 4; ++e) o[e] = (bf16)(vy_act_fwd<ACT>(vy_round_bf16(acc[i][j][e])) * vy_round_bf16(acc[i + 1][j][e]));
+          for (int e = 0; e < 4; ++e) at[e] = act_entry(__builtin_bit_cast(unsigned, vy_round_bf16(acc[i][j][e])) >> 16, far);
+          known = !__any(far >= ACT_TAB_HALF);
+          if (known) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) f[e] = __builtin_bit_cast(float, tab[at[e]]);
+          }
+        }
+        if (!known) {
+#pragma unroll
+          for (int e = 0; e < 4; ++e) f[e] = vy_act_fwd<ACT>(vy_round_bf16(acc[i][j][e]));
+        }
+#pragma unroll
+        for (int e = 0; e < 4; ++e) o[e] = (bf16)(f[e] * vy_round_bf16(acc[i + 1][j][e]));
         *reinterpret_cast<bf16x4*>(et + (wm * 16 * TM16 + 16 * j + r16) * GROW + (wn * 8 * TN16 + 8 * i + 4 * kq) * 2) = o;
       }
     __syncthreads();
@@ -453,12 +517,39 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
     const bf16* pf_ptr = GRAD ? (ep.gradpre ? ep.gradpre : ep.residual) : ep.residual;
     const int64_t pf_ld = GRAD ? (ep.gradpre ? ep.ldg : ep.ldr) : ep.ldr;
     const bool pf_is_gradpre = GRAD && ep.gradpre != nullptr;
+    const bool by_table = TAB && ep.vec_ok && !ep.residual && !ep.drop.thr;
     auto do_chunk = [&](bf16* __restrict__ dst, bool dual, int pass, int c, bool pf, const bf16x8& p8) {
         const int row = c / CPR, cc = c - row * CPR;
         const int64_t m = m0 + pass * RP + row;
         const int n = n0 + cc * 8;
         if (m >= M || n >= N) return;
         const bf16x8 sv = *reinterpret_cast<const bf16x8*>(et + row * EROW + cc * 16);
+        if constexpr (TAB) {
+          if (by_table && n + 8 <= N) {
+            const u32x4 u = __builtin_bit_cast(u32x4, sv);
+            unsigned at[8], far = 0;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) at[e] = act_entry(u[e >> 1] >> (16 * (e & 1)), far);
+            if (!__any(far >= ACT_TAB_HALF)) {
+              unsigned t[8];
+              u32x4 o, d;
+#pragma unroll
+              for (int e = 0; e < 8; ++e) t[e] = tab[at[e]];
+#pragma unroll
+              for (int e = 0; e < 4; ++e) {
+                o[e] = __builtin_amdgcn_perm(t[2 * e + 1], t[2 * e], 0x05040100);
+                d[e] = __builtin_amdgcn_perm(t[2 * e + 1], t[2 * e], 0x07060302);
+              }
+              if (dual) {
+                if (ep.pre_deriv) __builtin_nontemporal_store(d, reinterpret_cast<u32x4*>(ep.pre + m * ep.ldy + n));
+                else *reinterpret_cast<bf16x8*>(ep.pre + m * ep.ldy + n) = sv;
+              }
+              if (ep.wt_store) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 1" ::"v"(dst + m * ep.ldy + n), "v"(o) : "memory");
+              else *reinterpret_cast<u32x4*>(dst + m * ep.ldy + n) = o;
+              return;
+            }
+          }
+        }
         float v[8];
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = (float)sv[e];
@@ -876,8 +967,9 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
   static_assert(GX * NW == PX && GW * NW == PW, "pieces must divide over the waves");
   constexpr int XT = BM * ROWB, WT = BN * ROWB;
   constexpr int WOFF = 3 * XT;
-  constexpr int LDS_BYTES = vy_cmax(3 * XT + 2 * WT, epi_lds_bytes(BM, BN, EPI, 1));
-  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
+  constexpr int LDS_BYTES = vy_cmax(3 * XT + 2 * WT, epi_lds_bytes(BM, BN, EPI, 1)), TABLE = act_table_bytes(BM, BN, EPI, ACT, GRAD);
+  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES + TABLE];
+  unsigned* tab = reinterpret_cast<unsigned*>(smem + LDS_BYTES);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -966,6 +1058,10 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
   stage_x(0);
   stage_w(0);
   if (KT > 1) stage_x(1);
+  if constexpr (TABLE > 0) {
+    fill_act_table<EPI, ACT>(tab, ep.pre_deriv);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
   if (KT > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GX) : "memory");
   else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
@@ -990,7 +1086,7 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
     xbuf = xbuf == 2 ? 0 : xbuf + 1;
     if (kt + 1 < KT) read_frags(wa[0] + (WT - wo), xa[0] + xbuf * XT, wf[0], xf[0]);
   }
-  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq);
+  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq, tab);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1009,8 +1105,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   constexpr int GX = PX / NW, GW = PW / NW;
   static_assert(GX * NW == PX && GW * NW == PW, "pieces must divide over the waves");
   constexpr int STAGE = (BM + BN) * ROWB;
-  constexpr int LDS_BYTES = vy_cmax(2 * STAGE, epi_lds_bytes(BM, BN, EPI, 1));
-  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
+  constexpr int LDS_BYTES = vy_cmax(2 * STAGE, epi_lds_bytes(BM, BN, EPI, 1)), TABLE = act_table_bytes(BM, BN, EPI, ACT, GRAD);
+  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES + TABLE];
+  unsigned* tab = reinterpret_cast<unsigned*>(smem + LDS_BYTES);
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1094,6 +1191,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   };
 
   stage(0, 0);
+  if constexpr (TABLE > 0) {
+    fill_act_table<EPI, ACT>(tab, ep.pre_deriv);
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
@@ -1114,7 +1215,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     asm volatile("" ::: "memory");
     if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
   }
-  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq);
+  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq, tab);
 }
 
 // ------------------------------------------------------------------------------------------
