@@ -381,10 +381,40 @@ template <int BM, int BN, int WGM, int WGN, bool MF16> struct AccTile {
   typedef std::conditional_t<MF16, T16, T32> type;
 };
 
-template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD, int PASSES = 1, bool PF_OK = true, bool MF16 = false>
+// The second operand of a plain epilogue -- residual, or the pre-activation of a dgrad -- in the registers of the threads that will
+// combine it (16-byte chunks tid, tid + NT, ... of the tile), requested before the accumulators are staged: loaded in the loop over the
+// chunks, every iteration waits a full memory latency for it (22 k cycles per tile against 12 k without the operand).
+constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, bool GRAD) {
+  return EPI == 0 && (BM * BN == 256 * 192 || BM * BN == 64 * 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
+}
+template <int BM, int BN, int NW, int EPI, bool GRAD>
+struct EpiAhead {
+  static constexpr bool ON = epi_prefetches(BM, BN, NW, EPI, GRAD);
+  static constexpr int ITERS = ON ? BM * BN / 8 / (64 * NW) : 1;
+  bf16x8 v[ITERS];
+  bool on = false;
+  __device__ __forceinline__ void request(const EpiPlain<bf16>& ep, int m0, int n0, int M, int N) {
+    const bool pre = GRAD && ep.gradpre != nullptr;
+    const bf16* p = pre ? ep.gradpre : ep.residual;
+    on = ON && p != nullptr && ep.vec_ok && m0 + BM <= M && n0 + BN <= N;   // workgroup-uniform
+    if constexpr (ON) {
+      if (on) {
+        const int64_t ld = pre ? ep.ldg : ep.ldr;
+#pragma unroll
+        for (int it = 0; it < ITERS; ++it) {
+          const int c = (int)threadIdx.x + it * 64 * NW, row = c / (BN / 8);
+          v[it] = *reinterpret_cast<const bf16x8*>(p + (int64_t)(m0 + row) * ld + n0 + (c - row * (BN / 8)) * 8);
+        }
+      }
+    }
+  }
+};
+
+template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD, int PASSES = 1, bool MF16 = false>
 __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN, MF16>::type& acc, char* smem,
                                               int m0, int n0, int M, int N, const EpiPlain<bf16>& ep,
-                                              const EpiQkv<bf16>& eq, const unsigned* tab = nullptr) {
+                                              const EpiQkv<bf16>& eq, const EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>& ahead = EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>{},
+                                              const unsigned* tab = nullptr) {
   constexpr bool TAB = MF16 && act_has_table(BM, BN, EPI, ACT, GRAD);
   static_assert(!MF16 || PASSES == 1, "the 16 x 16 accumulator layout is staged in one pass");
   constexpr int NW = WGM * WGN, NT = 64 * NW;
@@ -510,12 +540,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
     // values -- what the reference's bf16 Linear -> GELU computes -- and, when the caller wants the
     // pre-activation saved for backward (dual), it is stored from the same chunk: one pass over the
     // tile, no second staging pass, no GELU chains among the accumulator registers.
-    // one 16-byte chunk of the staged band.  pf: the chunk's second operand (residual, or the pre-activation of a
-    // dgrad) was requested BEFORE the accumulators were staged and is handed in as p8 -- loaded here, inside the
-    // loop, every iteration waits a full memory latency for it (the residual epilogue measured 22 k cycles per
-    // tile against 12 k without the residual)
-    const bf16* pf_ptr = GRAD ? (ep.gradpre ? ep.gradpre : ep.residual) : ep.residual;
-    const int64_t pf_ld = GRAD ? (ep.gradpre ? ep.ldg : ep.ldr) : ep.ldr;
+    // one 16-byte chunk of the staged band.  pf: its second operand is p8 (EpiAhead)
     const bool pf_is_gradpre = GRAD && ep.gradpre != nullptr;
     const bool by_table = TAB && ep.vec_ok && !ep.residual && !ep.drop.thr;
     auto do_chunk = [&](bf16* __restrict__ dst, bool dual, int pass, int c, bool pf, const bf16x8& p8) {
@@ -637,26 +662,11 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
           }
         }
     };
-    constexpr bool PFK = PF_OK && PASSES == 1 && (BM * BN == 256 * 192 || BM * BN == 64 * 64) && (RP * CPR) % NT == 0;   // kernels that prefetch (the 256 x 256 tile has no registers to spare: +5 % on FFN1 with them reserved)
-    constexpr int ITERS = PFK ? (RP * CPR) / NT : 1;
-    bf16x8 pre8[ITERS];
-    const bool pf_on = PFK && pf_ptr != nullptr && ep.vec_ok && m0 + BM <= M && n0 + BN <= N;   // workgroup-uniform
-    if constexpr (PFK) {
-      if (pf_on) {
+    auto flush_plain = [&](bf16* __restrict__ dst, bool dual, int pass) {
+      if constexpr (PASSES == 1 && EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>::ON) {
+        if (ahead.on) {
 #pragma unroll
-        for (int it = 0; it < ITERS; ++it) {
-          const int c = tid + it * NT;
-          const int row = c / CPR, cc = c - row * CPR;
-          pre8[it] = *reinterpret_cast<const bf16x8*>(pf_ptr + (int64_t)(m0 + row) * pf_ld + n0 + cc * 8);
-        }
-      }
-    }
-    auto flush_plain = [&](bf16* __restrict__ dst, bool final_pass, bool dual, int pass) {
-      (void)final_pass;
-      if constexpr (PFK) {
-        if (pf_on) {
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) do_chunk(dst, dual, pass, tid + it * NT, true, pre8[it]);
+          for (int it = 0; it < (RP * CPR) / NT; ++it) do_chunk(dst, dual, pass, tid + it * NT, true, ahead.v[it]);
           return;
         }
       }
@@ -668,7 +678,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
     for (int pass = 0; pass < PASSES; ++pass) {
       stage_all(pass);
       __syncthreads();
-      flush_plain(ep.y, true, dual, pass);
+      flush_plain(ep.y, dual, pass);
       if (pass + 1 < PASSES) __syncthreads();
     }
   } else if constexpr (EPI == 1) {
@@ -1086,7 +1096,9 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
     xbuf = xbuf == 2 ? 0 : xbuf + 1;
     if (kt + 1 < KT) read_frags(wa[0] + (WT - wo), xa[0] + xbuf * XT, wf[0], xf[0]);
   }
-  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq, tab);
+  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
+  ahead.request(ep, m0, n0, M, N);
+  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1215,7 +1227,9 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     asm volatile("" ::: "memory");
     if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
   }
-  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq, tab);
+  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
+  ahead.request(ep, m0, n0, M, N);
+  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1346,7 +1360,9 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
       }
     __syncthreads();
   }
-  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq);
+  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
+  ahead.request(ep, m0, n0, M, N);
+  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1543,7 +1559,7 @@ __global__ __launch_bounds__(64) void gemm_splitk_finish_kernel(
 #pragma unroll
       for (int i = 0; i < TN; ++i) acc[i][0] = acc[i][0] + part[sidx][i];   // slice order: deterministic
     }
-  gemm_epilogue<16, SN, 1, 1, EPI, ACT, GRAD, 1, true, true>(acc, smem, m0, n0, M, N, ep, eq);
+  gemm_epilogue<16, SN, 1, 1, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq);
 }
 
 // Workspaces for the split-K launches, registered per stream by the caller (the library never allocates device memory):
