@@ -59,7 +59,7 @@ template <int BN, int BKW, int MS, int NS, bool MF16 = false>
 __device__ __forceinline__ void wgrad_tn_bf16_body(
     const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
     float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
-    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag, int wg) {
+    int M, int N, int K, int tiles_k, int m_chunk, int diag, int split, int t2) {
   constexpr int NW = BN / 32;                 // waves: (BN/64) x 2
   constexpr int WKT = BKW / 2, TJ = WKT / 32; // k extent of a wave, 32-wide fragments along k
   constexpr int AROW = BN * 2, BROW = BKW * 2;  // LDS row bytes of the dY and X tiles
@@ -73,7 +73,6 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wn = wave >> 1, wk = wave & 1;
-  const int split = wg / tiles_nk, t2 = wg - split * tiles_nk;
   const int tile_n = t2 / tiles_k, tile_k = t2 - tile_n * tiles_k;
   const int n0 = tile_n * BN, k0 = tile_k * BKW;
   const int m_begin = split * m_chunk;
@@ -404,9 +403,21 @@ template <int BN, int BKW, int MS, int NS, bool MF16 = false>
 __global__ __launch_bounds__(BN * 2, BN == 128 ? 2 : 1) void wgrad_tn_bf16_kernel(
     const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
     float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
-    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag) {
-  wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, tiles_k, tiles_nk, m_chunk,
-                                      diag, xcd_remap(blockIdx.x, gridDim.x));
+    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag, int whole, int tail_chunk) {
+  // the first `whole` workgroups: chunks of m_chunk rows, tile by tile; the others: chunks of tail_chunk rows of the tiles from `whole` on
+  int split, t2, chunk;
+  if ((int)blockIdx.x < whole) {
+    const int wg = xcd_remap(blockIdx.x, whole);
+    split = wg / tiles_nk;
+    t2 = wg - split * tiles_nk;
+    chunk = m_chunk;
+  } else {
+    const int wg = xcd_remap(blockIdx.x - whole, gridDim.x - whole), tail = tiles_nk - whole;
+    split = wg / tail;
+    t2 = whole + wg - split * tail;
+    chunk = tail_chunk;
+  }
+  wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, tiles_k, chunk, diag, split, t2);
 }
 
 // Several weight gradients in ONE launch (vy_linear_wgrad_grouped): the four GEMMs of a transformer layer
@@ -432,7 +443,7 @@ __global__ __launch_bounds__(BN * 2, 1) void wgrad_tn_bf16_grouped_kernel(WgradG
   for (int i = 1; i < 8; ++i)
     if (d == i) it = grp.g[i];
   wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(it.dY, it.lddy, it.X, it.ldx, it.dW, it.lddw, it.db, nullptr, it.M, it.N, it.K,
-                                      it.tiles_k, it.tiles_nk, it.m_chunk, diag, id - it.item0);
+                                      it.tiles_k, it.m_chunk, diag, (id - it.item0) / it.tiles_nk, (id - it.item0) % it.tiles_nk);
 }
 
 // db[n] += sum_m dY[m,n]: block = 64 lanes x 8 columns, 256 rows per block
@@ -1067,15 +1078,23 @@ extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int6
   if (splits < 1) splits = 1;
   int64_t m_chunk = vy_cdiv(vy_cdiv(M, splits), 64) * 64;
   splits = vy_cdiv(M, m_chunk);
+  // One workgroup per CU: where the tiles end in a round of at most half the chip, that round's tiles are cut in two along M (two
+  // contributions to a zeroed gradient: their order does not show).  50265 x 768 over 16384 rows, 591 tiles: 1389 -> 1260 us; 8192 rows 733 -> 654.
+  int64_t whole = tiles * splits, tail_chunk = m_chunk, grid = whole;
+  if (big && splits == 1 && tiles > 256 && tiles % 256 > 0 && tiles % 256 <= 128) {
+    whole = tiles / 256 * 256;
+    tail_chunk = vy_cdiv(vy_cdiv(M, 2), 64) * 64;
+    grid = whole + (tiles - whole) * vy_cdiv(M, tail_chunk);
+  }
   static const int ns = [] { const char* e = getenv("VY_WGRAD_STAGES"); return e ? atoi(e) : 2; }();
 #define WG_GO(BN_, BK_, MS_, NS_)                                                                          \
-  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_>), dim3((unsigned)(tiles * splits)), dim3(BN_ * 2), 0, \
+  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_>), dim3((unsigned)grid), dim3(BN_ * 2), 0, \
                      st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
-                     (int)K, tiles_k, tiles, (int)m_chunk, diag)
+                     (int)K, tiles_k, tiles, (int)m_chunk, diag, (int)whole, (int)tail_chunk)
 #define WG_GO16(BN_, BK_, MS_, NS_)                                                                        \
-  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_, true>), dim3((unsigned)(tiles * splits)), dim3(BN_ * 2), 0, \
+  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_, true>), dim3((unsigned)grid), dim3(BN_ * 2), 0, \
                      st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
-                     (int)K, tiles_k, tiles, (int)m_chunk, diag)
+                     (int)K, tiles_k, tiles, (int)m_chunk, diag, (int)whole, (int)tail_chunk)
   // 16 x 16 x 32 MFMAs: 3 % faster on the 256 x 256 tiles (vocabulary projection 1.62 -> 1.57 ms, +0.25 % on the training
   // step), 2-8 % SLOWER on the 128 x 128 tiles (these kernels are bound by the transposing LDS reads and the atomic
   // epilogue, not by the matrix pipe): 1 = the wide tiles only (default), 2 = everywhere, 0 = off
