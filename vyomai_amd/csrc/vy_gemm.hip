@@ -1234,21 +1234,23 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
 
 // ------------------------------------------------------------------------------------------
 // 64 x 64 tiles for outputs that give the big tiles too few workgroups: KG groups of 4 waves (2 x 2, 32 x 32 outputs each), each
-// with a ring of NBUF stages of its own, of which NBUF - 1 are on their way (counted vmcnt); group g multiplies the k-slices
-// g, g + KG, ... and the groups' accumulators are added through LDS at the end, in the order of the groups.
+// with a ring of NBUF stages of its own, of which NBUF - 1 are on their way (counted vmcnt).  The sums of every `per` stages are added
+// up in order (sum_slices: as many as where K is split over workgroups, so that the result does not hang on the kernel); two groups
+// take half of the two or four slices each and add them up through LDS at the end.
 // Bound by the chain of stages (0.3 us each: barrier, LDS reads, 8 products a wave), so many workgroups per CU and, where there is
-// at most one, two groups in it.  512 x 768 x 768: 12.4 -> 7.4 us against K split over workgroups and a second launch;
-// 512 x 3072 x 768: 21.3 -> 10.1; 1056 x 2304 x 768: 21.7 -> 12.5; 264 x 2048 x 2048: 24.7 -> 10.9.  (Four groups: no faster than
-// two on any shape; a fourth stage: level.)
+// at most one, two groups in it.  512 x 768 x 768: 12.4 -> 8.5 us against K split over workgroups and a second launch;
+// 512 x 3072 x 768: 21.4 -> 10.5; 1056 x 2304 x 768: 22.0 -> 11.7; 264 x 2048 x 2048: 24.9 -> 17.9.  (Adding the slices up in order
+// takes 0.8 us of that, eight and more slices the second group too.  Four groups: no faster than two on any shape; a fourth stage: level.)
 // ------------------------------------------------------------------------------------------
 template <int KG, int NBUF, int EPI, int ACT, bool GRAD>
 __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
-    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob) {
+    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob, int per) {
   constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
   constexpr int TM = 2, TN = 2, PER = 2;               // 16 x 16 blocks and 1 KiB pieces of either operand per wave
   constexpr int STAGE = (BM + BN) * ROWB, RING = NBUF * STAGE;
-  constexpr int LDS_BYTES = vy_cmax(vy_cmax(KG * RING, (KG - 1) * BM * BN * 4), epi_lds_bytes(BM, BN, EPI, 1));
+  static_assert(KG <= 2 && (KG - 1) * 2 * BM * BN * 4 <= KG * RING, "the second group's two slices lie in the rings");
+  constexpr int LDS_BYTES = vy_cmax(KG * RING, epi_lds_bytes(BM, BN, EPI, 1));
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
 
   const int lane = threadIdx.x & 63;
@@ -1309,55 +1311,76 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     xa[ks] = vy_lds_addr(ring) + (wm * 16 * TM + r16) * ROWB + coff;
     wa[ks] = vy_lds_addr(ring) + BM * ROWB + (wn * 16 * TN + r16) * ROWB + coff;
   }
-  const int n_it = (KT + KG - 1) / KG;
+  const bool four = KG > 1 && KT > 2 * per;               // (two groups: 2 or 4 slices)
+  const int n_it = KG == 1 ? KT : four ? 2 * per : per;   // of a group
+  const int first = grp * n_it;
+  f32x4 sum[TN][TM];   // of the slices behind
 #pragma unroll
   for (int i = 0; i < NBUF - 1; ++i)
-    if (i < n_it) stage(i * KG + grp, i);
-  int buf = 0;
-  for (int it = 0; it < n_it; ++it) {
-    // the slice has landed for this wave, NBUF - 2 younger ones may still be on their way (near the end: wait for all) ...
-    if (it + NBUF - 2 < n_it) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER * (NBUF - 2)) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    // ... and, behind the barrier, for every wave; every wave has also finished with the buffer that is filled next
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    if (it + NBUF - 1 < n_it) stage((it + NBUF - 1) * KG + grp, buf == 0 ? NBUF - 1 : buf - 1);
-    const unsigned boff = (unsigned)buf * STAGE;
-    bf16x8 wf[2][TN], xf[2][TM];
+    if (i < n_it) stage(first + i, i);
+  int buf = 0, it = 0;
+  for (;;) {
+    const int end = it + per < n_it ? it + per : n_it;
+    for (; it < end; ++it) {
+      // the slice has landed for this wave, NBUF - 2 younger ones may still be on their way (near the end: wait for all) ...
+      if (it + NBUF - 2 < n_it) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER * (NBUF - 2)) : "memory");
+      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // ... and, behind the barrier, for every wave; every wave has also finished with the buffer that is filled next
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (it + NBUF - 1 < n_it) stage(first + it + NBUF - 1, buf == 0 ? NBUF - 1 : buf - 1);
+      const unsigned boff = (unsigned)buf * STAGE;
+      bf16x8 wf[2][TN], xf[2][TM];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
-      vy_static_for<TN>([&](auto i_c) { constexpr int i = decltype(i_c)::value; wf[ks][i] = vy_lds_read128_off<i * 16 * ROWB>(wa[ks] + boff); });
-      vy_static_for<TM>([&](auto j_c) { constexpr int j = decltype(j_c)::value; xf[ks][j] = vy_lds_read128_off<j * 16 * ROWB>(xa[ks] + boff); });
+      for (int ks = 0; ks < 2; ++ks) {
+        vy_static_for<TN>([&](auto i_c) { constexpr int i = decltype(i_c)::value; wf[ks][i] = vy_lds_read128_off<i * 16 * ROWB>(wa[ks] + boff); });
+        vy_static_for<TM>([&](auto j_c) { constexpr int j = decltype(j_c)::value; xf[ks][j] = vy_lds_read128_off<j * 16 * ROWB>(xa[ks] + boff); });
+      }
+      vy_lgkm_wait<TN + TM>(wf[0][0], wf[0][1], xf[0][0], xf[0][1]);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[0][i], xf[0][j], acc[i][j], 0, 0, 0);
+      vy_lgkm_wait<0>(wf[1][0], wf[1][1], xf[1][0], xf[1][1]);
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[1][i], xf[1][j], acc[i][j], 0, 0, 0);
+      buf = buf + 1 == NBUF ? 0 : buf + 1;
     }
-    vy_lgkm_wait<TN + TM>(wf[0][0], wf[0][1], xf[0][0], xf[0][1]);
+    if (it == n_it) break;
+    const bool begun = it > per;
 #pragma unroll
     for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[0][i], xf[0][j], acc[i][j], 0, 0, 0);
-    vy_lgkm_wait<0>(wf[1][0], wf[1][1], xf[1][0], xf[1][1]);
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[1][i], xf[1][j], acc[i][j], 0, 0, 0);
-    buf = buf + 1 == NBUF ? 0 : buf + 1;
+      for (int j = 0; j < TM; ++j) {
+        sum[i][j] = begun ? sum[i][j] + acc[i][j] : acc[i][j];
+        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+      }
   }
   // what follows reuses the buffers: every wave is through with its reads
   __syncthreads();
+  if (grp == 0 && n_it > per)
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j] + acc[i][j];
   if constexpr (KG > 1) {
     f32x4* part = reinterpret_cast<f32x4*>(smem) + (threadIdx.x & 255);
     if (grp)
 #pragma unroll
-      for (int i = 0; i < TN * TM; ++i) part[((grp - 1) * TN * TM + i) * 256] = acc[i / TM][i % TM];
+      for (int i = 0; i < TN * TM; ++i) {
+        if (four) part[(TN * TM + i) * 256] = sum[i / TM][i % TM];
+        part[i * 256] = acc[i / TM][i % TM];
+      }
     __syncthreads();
     if (grp) return;   // (a barrier waits for the waves that are left)
 #pragma unroll
-    for (int g = 0; g < KG - 1; ++g)
-#pragma unroll
-      for (int i = 0; i < TN * TM; ++i) {
-        const f32x4 v = part[(g * TN * TM + i) * 256];
-#pragma unroll
-        for (int r = 0; r < 4; ++r) acc[i / TM][i % TM][r] += v[r];
-      }
+    for (int i = 0; i < TN * TM; ++i) {
+      f32x4& a = acc[i / TM][i % TM];
+      if (four) a = a + part[(TN * TM + i) * 256];
+      a = a + part[i * 256];
+    }
     __syncthreads();
   }
   EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
@@ -1594,9 +1617,16 @@ constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 128, 128, 128};
 constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 256, 512, 512};
 struct Tiling { TileKind kind; int slices; };
 
-// slices of K for `tiles` workgroups per slice: a power of two (one slice per group of XCDs, splitk_block_of), about `target`
-// workgroups in all, at least two stages in a slice, none empty
-inline int splitk_slices(int64_t tiles, int KT, int target) {
+// Slices of K whose sums a product adds up, in order: what fills the chip where every slice is a workgroup of its own (as many as
+// `target` workgroups in all, a power of two -- one per group of XCDs, splitk_block_of -- of at least two stages, none empty).  The
+// kernels below add up the same sums in the same order, so a result does not hang on which of them the shape takes (in training the
+// rounding of one product decides the noise of every gradient behind it).
+inline int sum_slices(int64_t M, int64_t N, int64_t K, int64_t ws_bytes) {
+  if (g_chains != 1 || (M > 1024 && vy_cdiv(M, 256) * vy_cdiv(N, 192) >= 160)) return 1;
+  const int bm = M > 128 && M <= 256 ? 256 : M > 256 && M <= 320 ? 320 : 128, target = bm == 128 ? 448 : 256;
+  const int64_t tiles = vy_cdiv(M, bm) * vy_cdiv(N, 128);
+  const int KT = (int)vy_cdiv(K, BK);
+  if (tiles * 3 >= target * 2) return 1;
   int S = (int)((target + tiles / 2) / tiles);
   if (S > KT / 2) S = KT / 2;
   if (S > 16) S = 16;
@@ -1604,43 +1634,42 @@ inline int splitk_slices(int64_t tiles, int KT, int target) {
   int p2 = 2;
   while (p2 * 2 <= S) p2 *= 2;
   const int per = (KT + p2 - 1) / p2;
-  return (KT + per - 1) / per;
+  S = (KT + per - 1) / per;
+  return S * tiles * bm * 128 * 4 <= ws_bytes ? S : 1;
 }
 
 inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes) {
-  const int KT = (int)vy_cdiv(K, BK);
-  Tiling best{T_256x256, 1};
+  const int KT = (int)vy_cdiv(K, BK), S = sum_slices(M, N, K, ws_bytes);
+  Tiling best{T_256x256, S};
   double least = 1e30;
-  auto offer = [&](TileKind kind, int slices, double us) {
-    if (us < least) { least = us; best = Tiling{kind, slices}; }
+  auto offer = [&](TileKind kind, double us) {
+    if (us < least) { least = us; best.kind = kind; }
   };
   auto tiles_of = [&](TileKind k) { return vy_cdiv(M, TILE_M[k]) * vy_cdiv(N, TILE_N[k]); };
   // `fixed` per round, `stage` per stage of a round; the stages of a last round that leaves CUs idle run up to 30 % faster
   auto one_shot = [&](TileKind k, int per_cu, double launch, double fixed, double stage) {
     const double r = (double)tiles_of(k) / (chip * per_cu), whole = (double)(int64_t)r, part = r - whole;
-    offer(k, 1, launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * stage * KT);
+    offer(k, launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * stage * KT);
   };
-  one_shot(T_256x256, 1, 2.5, 7.0, 1.55);
-  one_shot(T_256x192, 1, 2.3, 5.5, 1.30);
-  one_shot(T_256x128, 1, 4.5, 4.1, 0.97);
-  if (tiles_of(T_128x128) <= chip) offer(T_128x128, 1, 8.5 + 0.72 * KT);
-  else one_shot(T_128x128, 2, 3.5, 5.0, 1.0);     // (two of them share a CU)
   const double load = (double)tiles_of(T_64x64) / chip;
-  offer(T_64x64, 1, 4.3 + KT * (0.22 * load > 0.295 ? 0.22 * load : 0.295));
-  offer(T_64x64_TWICE, 1, 3.0 + (double)vy_cdiv(tiles_of(T_64x64_TWICE), chip) * (2.2 + 0.44 * ((KT + 1) / 2)));
+  offer(T_64x64, 4.3 + KT * (0.22 * load > 0.295 ? 0.22 * load : 0.295));
+  if (S == 1) {
+    one_shot(T_256x256, 1, 2.5, 7.0, 1.55);
+    one_shot(T_256x192, 1, 2.3, 5.5, 1.30);
+    one_shot(T_256x128, 1, 4.5, 4.1, 0.97);
+    if (tiles_of(T_128x128) <= chip) offer(T_128x128, 8.5 + 0.72 * KT);
+    else one_shot(T_128x128, 2, 3.5, 5.0, 1.0);     // (two of them share a CU)
+    return best;
+  }
+  if (S == 2 || S == 4) offer(T_64x64_TWICE, 3.0 + (double)vy_cdiv(tiles_of(T_64x64_TWICE), chip) * (2.2 + 0.44 * ((KT + 1) / 2)));
   // K over several workgroups: the partial sums' way through memory (about 8 TB/s there and back: mostly the Infinity Cache) and a second launch.
   // 128 < M <= 320: one row tile holds every row, so a weight crosses L2 -> LDS once
-  if (chip == 256 && ws_bytes > 0) {
-    const TileKind k = M > 256 && M <= 320 ? T_320x128_SPLIT : M > 128 && M <= 256 ? T_256x128_SPLIT : T_128x128_SPLIT;
-    const int64_t tiles = tiles_of(k);
-    const int S = splitk_slices(tiles, KT, k == T_128x128_SPLIT ? 448 : 256);
-    const double bytes = 4.0 * S * tiles * TILE_M[k] * TILE_N[k];
-    if (S > 1 && bytes <= (double)ws_bytes) {
-      const int per = (KT + S - 1) / S;
-      const double stage = k == T_128x128_SPLIT ? (tiles * S > chip ? 1.0 : 0.72) : 1.2 * TILE_M[k] / 256;
-      offer(k, S, 7.5 + (double)vy_cdiv(tiles * S, (int64_t)chip * (k == T_128x128_SPLIT ? 2 : 1)) * per * stage + 2 * bytes / 8e6);
-    }
-  }
+  const TileKind k = M > 256 && M <= 320 ? T_320x128_SPLIT : M > 128 && M <= 256 ? T_256x128_SPLIT : T_128x128_SPLIT;
+  const int64_t tiles = tiles_of(k);
+  const double bytes = 4.0 * S * tiles * TILE_M[k] * TILE_N[k];
+  const int per = (KT + S - 1) / S;
+  const double stage = k == T_128x128_SPLIT ? (tiles * S > chip ? 1.0 : 0.72) : 1.2 * TILE_M[k] / 256;
+  offer(k, 7.5 + (double)vy_cdiv(tiles * S, (int64_t)chip * (k == T_128x128_SPLIT ? 2 : 1)) * per * stage + 2 * bytes / 8e6);
   return best;
 }
 
@@ -2403,7 +2432,9 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     }
     const int bm = var >= 0 ? 256 : TILE_M[t.kind], bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
     const int tn = (int)vy_cdiv(N, bn), tiles = (int)vy_cdiv(M, bm) * tn, threads = var >= 0 ? 512 : TILE_THREADS[t.kind];
+    const int KT = (int)vy_cdiv(K, BK), per = t.slices ? (KT + t.slices - 1) / t.slices : KT;
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot)
+#define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot, per)
     if (var >= 0) {
       if constexpr (EPI == 0 && !GRAD) {
         if (var == 8) VY_TILES(gemm_nt_bf16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>);
@@ -2414,13 +2445,14 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
       case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>); break;
       case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, EPI, ACT, GRAD>); break;
       case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
-      case T_64x64: VY_TILES(gemm_nt_bf16_small_kernel<1, 3, EPI, ACT, GRAD>); break;
-      case T_64x64_TWICE: VY_TILES(gemm_nt_bf16_small_kernel<2, 3, EPI, ACT, GRAD>); break;
+      case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, EPI, ACT, GRAD>); break;
+      case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, EPI, ACT, GRAD>); break;
       case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
       case T_256x128_SPLIT: launch_split<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
       case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
     }
 #undef VY_TILES
+#undef VY_SMALL
   }
   return 0;
 }
@@ -2434,17 +2466,20 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
   splitk_ws(st, 0, &ws_bytes);
   const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes);
   const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, TILE_M[t.kind]) * tn;
+  const int KT = (int)vy_cdiv(K, BK), per = (KT + t.slices - 1) / t.slices;
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
+#define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0, per)
   switch (t.kind) {
     case T_256x256: VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, 2, ACT, false>); break;
     case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, 2, ACT, false>); break;
     case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, 2, ACT, false>); break;
     case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, 2, ACT, false>); break;
-    case T_64x64: VY_TILES(gemm_nt_bf16_small_kernel<1, 3, 2, ACT, false>); break;
-    case T_64x64_TWICE: VY_TILES(gemm_nt_bf16_small_kernel<2, 3, 2, ACT, false>); break;
+    case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 2, ACT, false>); break;
+    case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, ACT, false>); break;
     default: return VY_ERR_UNSUPPORTED;   // (K split over workgroups)
   }
 #undef VY_TILES
+#undef VY_SMALL
   return VY_OK;
 }
 
