@@ -420,6 +420,8 @@ typedef struct vy_wgrad_desc {
   int64_t M, N, K;
 } vy_wgrad_desc;
 int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
+/* vy_linear_wgrad_batch: the same for up to 12. */
+int vy_linear_wgrad_batch(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
 
 /* LayerNorm backward: dx = rstd*(g - mean(g) - xhat*mean(g*xhat)), g = dy*gamma;
  * dgamma/dbeta fp32 [N] accumulated (beta) from per-block partials in `ws`

@@ -30,3 +30,46 @@ def test_against_fp64(M, N, K, accumulate):
         size = d.abs().T.contiguous() @ x.double().abs() + 1.0
         assert ((dw[n0:n0 + 8192].double() - want).abs() <= M * 2.0 ** -24 * size).all()
         assert ((db[n0:n0 + 8192].double() - d.sum(0) - (-0.25 if accumulate else 0.0)).abs() <= M * 2.0 ** -24 * (d.abs().sum(0) + 1.0)).all()
+
+
+@pytest.mark.parametrize("n", [9, 12])
+def test_more_than_a_layer_in_one_launch(n):
+    """Gradients of several layers, ragged and of different rows, in one launch (one piece a tile, or several): against fp64."""
+    from vyomai_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(n)
+    items = []
+    for i in range(n):
+        M, N, K = (2112, 2200)[i % 2] + i, (768, 520, 1032)[i % 3], (768, 264, 1024)[i % 3 - 1]
+        dy = torch.randn(M, (N + 7) // 8 * 8, device=DEV, generator=g).to(BF)[:, :N]
+        x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+        items.append((dy, x, torch.full((N, K), 0.5, device=DEV), torch.full((N,), -0.25, device=DEV) if i % 4 else None))
+    ops.linear_wgrad_grouped(items)
+    for dy, x, dw, db in items:
+        M, d = dy.shape[0], dy.double()
+        size = d.abs().T.contiguous() @ x.double().abs() + 1.0
+        assert ((dw.double() - (d.T.contiguous() @ x.double() + 0.5)).abs() <= M * 2.0 ** -24 * size).all()
+        if db is not None:
+            assert ((db.double() - (d.sum(0) - 0.25)).abs() <= M * 2.0 ** -24 * (d.abs().sum(0) + 1.0)).all()
+
+
+def test_pending_gradients_fill_a_launch_and_no_more():
+    """autograd_train._WgradGroup: a launch takes the gradients whose tiles the chip has CUs for; the next one starts the next launch."""
+    from vyomai_amd import autograd_train as AT
+    sizes = []
+    real = AT.ops.linear_wgrad_grouped
+    AT.ops.linear_wgrad_grouped = lambda items: sizes.append(sum(-(-i[2].shape[0] // 256) * -(-i[2].shape[1] // 256) for i in items))
+    try:
+        group = AT._WgradGroup()
+        group.armed = True   # (no backward pass to flush it)
+        for layer in range(5):
+            for N, K in ((768, 3072), (3072, 768), (768, 768), (2304, 768)):
+                group.add_tensors(None, None, torch.empty(N, K, device="meta"), None, [])
+        assert sizes == [252, 252] and group.tiles == 36
+        group.flush()
+        for _ in range(13):
+            group.add_tensors(None, None, torch.empty(512, 512, device="meta"), None, [])
+        assert sizes == [252, 252, 36, 48] and len(group.items) == 1
+        group.add_tensors(None, None, torch.empty(8191, 8192, device="meta"), None, [])   # alone more than the chip
+        assert sizes == [252, 252, 36, 48, 4, 1024] and not group.items
+    finally:
+        AT.ops.linear_wgrad_grouped = real

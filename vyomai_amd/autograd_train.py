@@ -133,11 +133,12 @@ class _WgradGroup:
     """Weight gradients that accumulate straight into the gradient arena do not have to be launched where
     autograd reaches them: the projections of a layer are small wgrad problems (9-36 tiles of 256 x 256),
     and one at a time each needs M-splits -- fp32 atomic traffic -- to fill the chip.  They are collected
-    here and go out as ONE launch per ~layer (vy_linear_wgrad_grouped); the parameters are reported ready
+    here and go out as ONE launch per chip of tiles, ~2 layers (ops.linear_wgrad_grouped); the parameters are reported ready
     (DDP buckets, per-bucket AdamW) when that launch has been enqueued.  Whatever is still pending when
     the backward pass ends is flushed by an autograd-engine callback."""
 
-    TILES = int(os.environ.get("VY_WGRAD_GROUP_TILES", "100"))   # flush once this many 256 x 256 output tiles are pending (one post-LN layer: 108)
+    TILES = int(os.environ.get("VY_WGRAD_GROUP_TILES", "256"))   # most 256 x 256 output tiles of a launch: a CU each (a post-LN layer of 768: 108)
+    MOST = 12                                                    # gradients of a launch
 
     def __init__(self):
         self.items, self.tiles, self.armed = [], 0, False
@@ -154,16 +155,19 @@ class _WgradGroup:
     def add_tensors(self, dy, x, dw, db, members) -> None:
         """dw / db: the fp32 gradient tensors the launch accumulates into (views of the arena); members: the
         parameters to report ready once it has been enqueued (a packed projection has several)."""
+        tiles = -(-dw.shape[0] // 256) * -(-dw.shape[1] // 256)
+        if self.tiles + tiles > self.TILES:
+            self.flush()
         self.items.append((dy, x, dw, db, members))
         # autograd's own post-accumulate hook fires for these parameters as soon as this backward function
         # returns -- the reducer must not take that for "gradient written" (training.BucketReducer._hook)
         for p in members:
             p._vy_deferred = True
-        self.tiles += -(-dw.shape[0] // 256) * -(-dw.shape[1] // 256)
+        self.tiles += tiles
         if not self.armed:
             torch.autograd.Variable._execution_engine.queue_callback(self._end_of_backward)
             self.armed = True
-        if self.tiles >= self.TILES or len(self.items) == 8:
+        if self.tiles >= self.TILES or len(self.items) == self.MOST:
             self.flush()
 
     def flush(self) -> None:

@@ -420,27 +420,29 @@ __global__ __launch_bounds__(BN * 2, BN == 128 ? 2 : 1) void wgrad_tn_bf16_kerne
   wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, tiles_k, chunk, diag, split, t2);
 }
 
-// Several weight gradients in ONE launch (vy_linear_wgrad_grouped): the four GEMMs of a transformer layer
+// Several weight gradients in ONE launch (vy_linear_wgrad_grouped, vy_linear_wgrad_batch): the four GEMMs of a transformer layer
 // have 9-36 tiles of 256 x 256 each -- alone, a launch needs 7 M-splits to fill 256 CUs (66 MB of fp32
-// atomics); together they are 108 tiles and need 2.  The table travels in the kernel arguments.
+// atomics); together they are 108 tiles and need 2 (216 work items), and nine GEMMs of neighbouring layers are 252 tiles that need no
+// splits: per 108 tiles over 16384 rows 258 -> 226 us, over 2112 rows 72 -> 46 us.  The table travels in the kernel arguments.
 struct WgradItem {
   const bf16* dY; const bf16* X; float* dW; float* db;
   int64_t lddy, ldx, lddw;
   int M, N, K, tiles_k, tiles_nk, m_chunk, item0;   // item0: first work item of this GEMM
 };
-struct WgradGroup { WgradItem g[8]; int n; };
+constexpr int MOST_WGRADS = 12;
+struct WgradGroup { WgradItem g[MOST_WGRADS]; int n; };
 
 template <int BN, int BKW, int MS, int NS, bool MF16 = false>
 __global__ __launch_bounds__(BN * 2, 1) void wgrad_tn_bf16_grouped_kernel(WgradGroup grp, int diag) {
   const int id = xcd_remap(blockIdx.x, gridDim.x);
   int d = 0;
 #pragma unroll
-  for (int i = 1; i < 8; ++i)
+  for (int i = 1; i < MOST_WGRADS; ++i)
     if (i < grp.n && id >= grp.g[i].item0) d = i;
   // (selected with a uniform loop: the descriptor lives in SGPRs after this)
   WgradItem it = grp.g[0];
 #pragma unroll
-  for (int i = 1; i < 8; ++i)
+  for (int i = 1; i < MOST_WGRADS; ++i)
     if (d == i) it = grp.g[i];
   wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(it.dY, it.lddy, it.X, it.ldx, it.dW, it.lddw, it.db, nullptr, it.M, it.N, it.K,
                                       it.tiles_k, it.m_chunk, diag, (id - it.item0) / it.tiles_nk, (id - it.item0) % it.tiles_nk);
@@ -1113,10 +1115,9 @@ extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int6
   return VY_OK;
 }
 
-extern "C" int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream) {
-  const char* who = "vy_linear_wgrad_grouped";
+static int wgrad_together(const char* who, const vy_wgrad_desc* descs, int32_t n, int32_t most, int dtype, void* stream) {
   if (dtype != VY_BF16 && dtype != VY_F32) VY_FAIL(VY_ERR_ARG, "%s: bad dtype %d", who, dtype);
-  if (!descs || n <= 0 || n > 8) VY_FAIL(VY_ERR_ARG, "%s: 1..8 descriptors", who);
+  if (!descs || n <= 0 || n > most) VY_FAIL(VY_ERR_ARG, "%s: 1..%d descriptors", who, most);
   if (dtype == VY_F32) {   // the parity path: one plain launch per descriptor
     for (int i = 0; i < n; ++i) {
       const vy_wgrad_desc& d = descs[i];
@@ -1153,7 +1154,7 @@ extern "C" int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, in
     it.tiles_k = (int)tiles_k; it.tiles_nk = (int)tiles; it.m_chunk = (int)m_chunk; it.item0 = (int)items;
     items += tiles * splits;
   }
-  for (int i = n; i < 8; ++i) grp.g[i] = grp.g[0];
+  for (int i = n; i < MOST_WGRADS; ++i) grp.g[i] = grp.g[0];
   // 16 x 16 x 32 MFMAs: 3 % faster on the 256 x 256 tiles (vocabulary projection 1.62 -> 1.57 ms, +0.25 % on the training
   // step), 2-8 % SLOWER on the 128 x 128 tiles (these kernels are bound by the transposing LDS reads and the atomic
   // epilogue, not by the matrix pipe): 1 = the wide tiles only (default), 2 = everywhere, 0 = off
@@ -1166,6 +1167,14 @@ extern "C" int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, in
                        grp, diag);
   VY_CHECK_LAUNCH(who);
   return VY_OK;
+}
+
+extern "C" int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream) {
+  return wgrad_together("vy_linear_wgrad_grouped", descs, n, 8, dtype, stream);
+}
+
+extern "C" int vy_linear_wgrad_batch(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream) {
+  return wgrad_together("vy_linear_wgrad_batch", descs, n, MOST_WGRADS, dtype, stream);
 }
 
 // ------------------------------------------------------------------------------------------

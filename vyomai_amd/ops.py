@@ -416,12 +416,12 @@ def linear_wgrad(dy: Tensor, x: Tensor, dw: Tensor, db: Optional[Tensor], accumu
 
 
 def linear_wgrad_grouped(items) -> None:
-    """items: up to 8 tuples (dy, x, dw, db|None): dw += dy^T @ x, db += colsum(dy), ONE launch
-    (vy_linear_wgrad_grouped).  The tensors must stay alive until the launch has been enqueued (they do:
+    """items: up to 12 tuples (dy, x, dw, db|None): dw += dy^T @ x, db += colsum(dy), ONE launch
+    (vy_linear_wgrad_grouped, vy_linear_wgrad_batch).  The tensors must stay alive until the launch has been enqueued (they do:
     the caller holds them)."""
     import ctypes as C
     n = len(items)
-    assert 1 <= n <= 8
+    assert 1 <= n <= 12
     arr = (_lib.VyWgradDesc * n)()
     dt = None
     for i, (dy, x, dw, db) in enumerate(items):
@@ -437,7 +437,7 @@ def linear_wgrad_grouped(items) -> None:
         a.dy, a.lddy, a.x, a.ldx = d2.data_ptr(), d2.stride(0), x2.data_ptr(), x2.stride(0)
         a.dw, a.lddw, a.db = dw.data_ptr(), dw.stride(0), _ptr(db)
         a.M, a.N, a.K = M, N, K
-    call("vy_linear_wgrad_grouped", C.cast(arr, C.c_void_p), n, dtype_code(dt), _stream())
+    call("vy_linear_wgrad_grouped" if n <= 8 else "vy_linear_wgrad_batch", C.cast(arr, C.c_void_p), n, dtype_code(dt), _stream())
 
 
 def layernorm_bwd(dy: Tensor, x: Tensor, gamma: Tensor, mean: Tensor, rstd: Tensor, dgamma: Tensor,
