@@ -23,21 +23,16 @@ using namespace vy_decay;
 
 constexpr int BT = 16, NB = C / BT;     // tokens per block, blocks per chunk
 
-// gates, written keys (and queries) of the 16 tokens of block s, channels c and c + 1
-struct Gates { float f[BT][2], k[BT][2], q[BT][2]; };
-template <bool Q>
+// gates and written keys of the 16 tokens of block s, channels c and c + 1
+struct Gates { float f[BT][2], k[BT][2]; };
 __device__ __forceinline__ void load_gates(const DecayArgs& a, const bf16* P, int head, int s, int c, int m, Gates& g) {
-  bf16x2 z[BT], q[BT];
+  bf16x2 z[BT];
   const bool in = c < a.dk;
   const int64_t at = (int64_t)head * a.dk + (in ? c : 0);
 #pragma unroll
   for (int t = 0; t < BT; ++t) {
-    z[t] = q[t] = bf16x2{(bf16)0.f, (bf16)0.f};
-    if (in && BT * s + t < m) {
-      const bf16* row = P + (int64_t)(BT * s + t) * a.ldp + at;
-      z[t] = *reinterpret_cast<const bf16x2*>(row + a.ok);
-      if constexpr (Q) q[t] = *reinterpret_cast<const bf16x2*>(row + a.oq);
-    }
+    z[t] = bf16x2{(bf16)0.f, (bf16)0.f};
+    if (in && BT * s + t < m) z[t] = *reinterpret_cast<const bf16x2*>(P + (int64_t)(BT * s + t) * a.ldp + at + a.ok);
   }
 #pragma unroll
   for (int e = 0; e < 2; ++e) {
@@ -47,7 +42,6 @@ __device__ __forceinline__ void load_gates(const DecayArgs& a, const bf16* P, in
       g.f[t][e] = 1.f;
       g.k[t][e] = 0.f;
       if (in && BT * s + t < m) forget_gate((float)z[t][e] + b, lower, g.f[t][e], g.k[t][e]);
-      if constexpr (Q) g.q[t][e] = activate((float)q[t][e], a.silu);
     }
   }
 }
@@ -89,7 +83,7 @@ __global__ __launch_bounds__(256) void gated_kv_kernel(DecayArgs a) {
   fetch(0);
   float sfx[2] = {1.f, 1.f};
   if (it < ITEMS) {
-    load_gates<false>(a, P, head, s, c, m, g);
+    load_gates(a, P, head, s, c, m, g);
 #pragma unroll
     for (int t = BT - 1; t >= 0; --t)
 #pragma unroll
@@ -181,24 +175,29 @@ __device__ __forceinline__ void share_out(float (&a)[24], int lane) {
   half(std::integral_constant<int, 3>{}, 8);
 }
 
-// grid (chunks, B * h): wave w computes rows 16 w .. + 15 of the chunk, block w
+// grid (chunks, B * h): wave w computes rows 16 w .. + 15 of the chunk, block w.
+// Bound by the latency of its phases, so two workgroups share a CU: channels are taken HC = 64 at a time, which halves the fp32 images
+// of gates, keys and queries, and with 64 channels a wave's phases up to the products between blocks touch its own block alone (no
+// barriers).  16 heads of 128 x 128, 8192 tokens: 183 -> 128 us against all channels at once, one workgroup on a CU.
 template <int DKP>
-__global__ __launch_bounds__(256, 1) void gated_out_kernel(DecayArgs a) {
+__global__ __launch_bounds__(256, 2) void gated_out_kernel(DecayArgs a) {
   static_assert(NB == 4, "one block per wave");
-  constexpr int KP = (DKP + 8) * 2, VP = (64 + 8) * 2, PAIRS = DKP / 2, ITEMS = NB * PAIRS;
-  constexpr int KS = DKP / 32, QP = DKP + 4, AP = 20;   // QP, AP: pitches in floats
+  constexpr int HC = DKP < 64 ? DKP : 64, NP = DKP / HC;   // channels of a pass, passes
+  constexpr bool OWN = HC == 64;                           // a wave's items are its block's
+  constexpr int KP = (HC + 8) * 2, VP = (64 + 8) * 2;
+  constexpr int KS = DKP / 32, KH = HC / 32, QP = HC + 4, AP = 20;   // QP, AP: pitches in floats
   constexpr int RAW = C * QP * 4;                       // bytes of an fp32 image
   constexpr int SN = DKP * 16 / 256;                    // quads of S per thread and value block
-  static_assert(2 * DKP * VP + C * VP <= 2 * RAW, "the state and value tiles fit over the raw gates and keys");
-  __shared__ __attribute__((aligned(16))) char smem[3 * RAW + 2 * C * KP + NB * BT * AP * 4 + NB * DKP * 4];
+  constexpr int TILES = 2 * DKP * VP + C * VP, IMAGES = 3 * RAW + 2 * C * KP;
+  __shared__ __attribute__((aligned(16))) char smem[(TILES > IMAGES ? TILES : IMAGES) + NB * BT * AP * 4 + NB * HC * 4];
   float* qs = reinterpret_cast<float*>(smem);           // queries, then times their prefix
   float* fs = reinterpret_cast<float*>(smem + RAW);
   float* ks = reinterpret_cast<float*>(smem + 2 * RAW);
   char* kh = smem + 3 * RAW;                            // keys times their suffix, hi and lo
   char* kl = kh + C * KP;
-  float* A = reinterpret_cast<float*>(kl + C * KP);     // [block][i][j] inside a block
+  float* A = reinterpret_cast<float*>(smem + (TILES > IMAGES ? TILES : IMAGES));   // [block][i][j] inside a block
   float* F = A + NB * BT * AP;                          // [block][channel]
-  char* sh = smem + RAW;                                // over fs and ks: state tile hi, lo, value tile
+  char* sh = smem;                                      // over the images: state tile hi, lo, value tile
   char* sl = sh + DKP * VP;
   char* vt = sl + DKP * VP;
   const int lane = threadIdx.x & 63;
@@ -225,142 +224,175 @@ __global__ __launch_bounds__(256, 1) void gated_out_kernel(DecayArgs a) {
       v8[i] = load8(P + (int64_t)t * a.ldp + a.ov + head * a.dv + v0 + d, t < m && v0 + d < a.dv, 0);
     }
   };
-  // ---- gates, keys, queries
-  const int it = threadIdx.x, s = it / PAIRS, c = (it % PAIRS) * 2;
-  static_assert(ITEMS <= 256, "one item per thread");
-  {
-    Gates g;
-    if (it < ITEMS) load_gates<true>(a, P, head, s, c, m, g);
-    fetch(0);
-    if (it < ITEMS) {
+  // one item a thread: block s, channel c of the pass
+  const int it = threadIdx.x, s = it / HC, c = it % HC;
+  const bool item = it < NB * HC;
+  bf16 z[BT], q[BT];
+  auto request = [&](int c0) {
+    const bool in = item && c0 + c < a.dk;
+#pragma unroll
+    for (int t = 0; t < BT; ++t) {
+      z[t] = q[t] = (bf16)0.f;
+      if (in && BT * s + t < m) {
+        const bf16* row = P + (int64_t)(BT * s + t) * a.ldp + (int64_t)head * a.dk + c0 + c;
+        z[t] = row[a.ok];
+        q[t] = row[a.oq];
+      }
+    }
+  };
+  auto block_sync = [&]() {
+    if constexpr (OWN) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // the wave's own rows
+    else __syncthreads();
+  };
+  bf16x8 qh[KS], ql[KS];
+  f32x4 sc[NB];
+#pragma unroll
+  for (int J = 0; J < NB; ++J) sc[J] = f32x4{0.f, 0.f, 0.f, 0.f};
+  float part[24];
+#pragma unroll
+  for (int i = 0; i < 24; ++i) part[i] = 0.f;
+  request(0);
+#pragma unroll
+  for (int pass = 0; pass < NP; ++pass) {
+    const int c0 = pass * HC;
+    // ---- gates, keys, queries
+    if (item) {
+      const bool in = c0 + c < a.dk;
+      const int64_t at = (int64_t)head * a.dk + (in ? c0 + c : 0);
+      const float bias = a.f_bias ? a.f_bias[at] : 0.f, lower = a.f_lower[at];
 #pragma unroll
       for (int t = 0; t < BT; ++t) {
-        const int at = (BT * s + t) * QP + c;
-        *reinterpret_cast<float2*>(qs + at) = make_float2(g.q[t][0], g.q[t][1]);
-        *reinterpret_cast<float2*>(fs + at) = make_float2(g.f[t][0], g.f[t][1]);
-        *reinterpret_cast<float2*>(ks + at) = make_float2(g.k[t][0], g.k[t][1]);
+        float f = 1.f, k = 0.f;
+        if (in && BT * s + t < m) forget_gate((float)z[t] + bias, lower, f, k);
+        const int x = (BT * s + t) * QP + c;
+        qs[x] = activate((float)q[t], a.silu);
+        fs[x] = f;
+        ks[x] = k;
       }
     }
-  }
-  __syncthreads();
-  // ---- A inside the wave's block: lane (jp, dg) has keys jp and jp + 8, DKP / 8 channels
-  {
-    constexpr int DG = DKP / 8;
-    const int jp = lane & 7, d0 = (lane >> 3) * DG;
-    float k0[DG], k1[DG], w0[DG], w1[DG], part[24];
-    auto row = [&](const float* p, int t, float (&v)[DG]) {
+    if (pass + 1 < NP) request(c0 + HC);
+    else fetch(0);
+    block_sync();
+    // ---- A inside the wave's block: lane (jp, dg) has keys jp and jp + 8, HC / 8 channels
+    {
+      constexpr int DG = HC / 8;
+      const int jp = lane & 7, d0 = (lane >> 3) * DG;
+      float k0[DG], k1[DG], w0[DG], w1[DG];
+      auto row = [&](const float* p, int t, float (&v)[DG]) {
 #pragma unroll
-      for (int e = 0; e < DG; e += 4) {
-        const f32x4 x = *reinterpret_cast<const f32x4*>(p + (BT * wave + t) * QP + d0 + e);
+        for (int e = 0; e < DG; e += 4) {
+          const f32x4 x = *reinterpret_cast<const f32x4*>(p + (BT * wave + t) * QP + d0 + e);
 #pragma unroll
-        for (int i = 0; i < 4; ++i) v[e + i] = x[i];
-      }
-    };
-    row(ks, jp, k0);
-    row(ks, jp + 8, k1);
-#pragma unroll
-    for (int e = 0; e < DG; ++e) w0[e] = w1[e] = 0.f;
-#pragma unroll
-    for (int i = 0; i < BT; ++i) {
-      float f[DG], q[DG], p0 = 0.f, p1 = 0.f;
-      row(fs, i, f);
-      row(qs, i, q);
-#pragma unroll
-      for (int e = 0; e < DG; ++e) {
-        w0[e] *= f[e];
-        if (i < 8) w0[e] = i == jp ? k0[e] : w0[e];
-        p0 = fmaf(q[e], w0[e], p0);
-        if (i >= 8) {
-          w1[e] *= f[e];
-          w1[e] = i - 8 == jp ? k1[e] : w1[e];
-          p1 = fmaf(q[e], w1[e], p1);
+          for (int i = 0; i < 4; ++i) v[e + i] = x[i];
         }
+      };
+      row(ks, jp, k0);
+      row(ks, jp + 8, k1);
+#pragma unroll
+      for (int e = 0; e < DG; ++e) w0[e] = w1[e] = 0.f;
+#pragma unroll
+      for (int i = 0; i < BT; ++i) {
+        float f[DG], x[DG], p0 = 0.f, p1 = 0.f;
+        row(fs, i, f);
+        row(qs, i, x);
+#pragma unroll
+        for (int e = 0; e < DG; ++e) {
+          w0[e] *= f[e];
+          if (i < 8) w0[e] = i == jp ? k0[e] : w0[e];
+          p0 = fmaf(x[e], w0[e], p0);
+          if (i >= 8) {
+            w1[e] *= f[e];
+            w1[e] = i - 8 == jp ? k1[e] : w1[e];
+            p1 = fmaf(x[e], w1[e], p1);
+          }
+        }
+        part[i] += p0;
+        if (i >= 8) part[8 + i] += p1;
       }
-      part[i] = p0;
-      if (i >= 8) part[8 + i] = p1;
+#pragma unroll
+      for (int i = 0; i < 24; ++i) asm volatile("" : "+v"(part[i]));   // (summed here, not where they are used: the rows' registers)
     }
+    block_sync();
+    // ---- queries times their prefix, keys times their suffix, products of whole blocks
+    if (item) {
+      float f[BT], p0 = 1.f, s0 = 1.f;
+#pragma unroll
+      for (int t = 0; t < BT; ++t) {
+        const int x = (BT * s + t) * QP + c;
+        f[t] = fs[x];
+        p0 *= f[t];
+        qs[x] *= p0;
+      }
+      F[s * HC + c] = p0;
+#pragma unroll
+      for (int t = BT - 1; t >= 0; --t) {
+        bf16 hi, lo;
+        split_bf16(ks[(BT * s + t) * QP + c] * s0, hi, lo);
+        const int x = (BT * s + t) * KP + c * 2;
+        *reinterpret_cast<bf16*>(kh + x) = hi;
+        *reinterpret_cast<bf16*>(kl + x) = lo;
+        s0 *= f[t];
+      }
+    }
+    __syncthreads();
+    // ---- A between blocks; the query operand takes in one block's gates after the other, at last the whole prefix of the chunk
+    float qv[KH][8];
+    bf16x8 th[KH], tl[KH];
+    auto split_q = [&]() {
+#pragma unroll
+      for (int k = 0; k < KH; ++k)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) { bf16 x, y; split_bf16(qv[k][e], x, y); th[k][e] = x; tl[k][e] = y; }
+    };
+#pragma unroll
+    for (int k = 0; k < KH; ++k)
+#pragma unroll
+      for (int hf = 0; hf < 2; ++hf) {
+        const f32x4 x = *reinterpret_cast<const f32x4*>(qs + (BT * wave + r16) * QP + 32 * k + 16 * hf + 4 * kq);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qv[k][4 * hf + e] = x[e];
+      }
+#pragma unroll
+    for (int J = NB - 2; J >= 0; --J) {
+      if (J < wave) {   // wave-uniform
+        split_q();
+#pragma unroll
+        for (int k = 0; k < KH; ++k) {
+          union { struct { bf16x4 a, b; } h; bf16x8 v; } h8, l8;
+          const int at = (BT * J + r16) * KP + (32 * k + 4 * kq) * 2;
+          h8.h.a = *reinterpret_cast<const bf16x4*>(kh + at);
+          h8.h.b = *reinterpret_cast<const bf16x4*>(kh + at + 32);
+          l8.h.a = *reinterpret_cast<const bf16x4*>(kl + at);
+          l8.h.b = *reinterpret_cast<const bf16x4*>(kl + at + 32);
+          sc[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l8.v, th[k], sc[J], 0, 0, 0);
+          sc[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h8.v, tl[k], sc[J], 0, 0, 0);
+          sc[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h8.v, th[k], sc[J], 0, 0, 0);
+        }
+#pragma unroll
+        for (int k = 0; k < KH; ++k)
+#pragma unroll
+          for (int hf = 0; hf < 2; ++hf) {
+            const f32x4 x = *reinterpret_cast<const f32x4*>(F + J * HC + 32 * k + 16 * hf + 4 * kq);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) qv[k][4 * hf + e] *= x[e];
+          }
+      }
+    }
+    split_q();
+#pragma unroll
+    for (int k = 0; k < KH; ++k) { qh[pass * KH + k] = th[k]; ql[pass * KH + k] = tl[k]; }
+    __syncthreads();   // the next pass, or the tiles, overwrite the images
+  }
+  {
     share_out(part, lane);
-    const int first = (lane & 32 ? 12 : 0) + (lane & 16 ? 6 : 0) + (lane & 8 ? 3 : 0);
+    const int first = (lane & 32 ? 12 : 0) + (lane & 16 ? 6 : 0) + (lane & 8 ? 3 : 0), jp = lane & 7;
 #pragma unroll
     for (int v = 0; v < 3; ++v) {
       const int x = first + v, i = x < 16 ? x : x - 8, j = x < 16 ? jp : jp + 8;
       A[(wave * BT + i) * AP + j] = part[v];
     }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (read by this wave alone)
   }
-  __syncthreads();
-  // ---- queries times their prefix, keys times their suffix, products of whole blocks
-  if (it < ITEMS) {
-    float2 f[BT];
-    float p0 = 1.f, p1 = 1.f;
-#pragma unroll
-    for (int t = 0; t < BT; ++t) {
-      const int at = (BT * s + t) * QP + c;
-      f[t] = *reinterpret_cast<const float2*>(fs + at);
-      float2 q = *reinterpret_cast<const float2*>(qs + at);
-      p0 *= f[t].x;
-      p1 *= f[t].y;
-      *reinterpret_cast<float2*>(qs + at) = make_float2(q.x * p0, q.y * p1);
-    }
-    F[s * DKP + c] = p0;
-    F[s * DKP + c + 1] = p1;
-    float s0 = 1.f, s1 = 1.f;
-#pragma unroll
-    for (int t = BT - 1; t >= 0; --t) {
-      const float2 k = *reinterpret_cast<const float2*>(ks + (BT * s + t) * QP + c);
-      const int at = (BT * s + t) * KP + c * 2;
-      store_split2(kh + at, kl + at, k.x * s0, k.y * s1);
-      s0 *= f[t].x;
-      s1 *= f[t].y;
-    }
-  }
-  __syncthreads();
-  // ---- A between blocks; the query operand takes in one block's gates after the other, at last the whole prefix of the chunk
-  float qv[KS][8];
-  bf16x8 qh[KS], ql[KS];
-  auto split_q = [&]() {
-#pragma unroll
-    for (int k = 0; k < KS; ++k)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { bf16 x, y; split_bf16(qv[k][e], x, y); qh[k][e] = x; ql[k][e] = y; }
-  };
-#pragma unroll
-  for (int k = 0; k < KS; ++k)
-#pragma unroll
-    for (int hf = 0; hf < 2; ++hf) {
-      const f32x4 x = *reinterpret_cast<const f32x4*>(qs + (BT * wave + r16) * QP + 32 * k + 16 * hf + 4 * kq);
-#pragma unroll
-      for (int e = 0; e < 4; ++e) qv[k][4 * hf + e] = x[e];
-    }
-  f32x4 sc[NB];
-#pragma unroll
-  for (int J = 0; J < NB; ++J) sc[J] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-  for (int J = NB - 2; J >= 0; --J) {
-    if (J < wave) {   // wave-uniform
-      split_q();
-#pragma unroll
-      for (int k = 0; k < KS; ++k) {
-        union { struct { bf16x4 a, b; } h; bf16x8 v; } h8, l8;
-        const int at = (BT * J + r16) * KP + (32 * k + 4 * kq) * 2;
-        h8.h.a = *reinterpret_cast<const bf16x4*>(kh + at);
-        h8.h.b = *reinterpret_cast<const bf16x4*>(kh + at + 32);
-        l8.h.a = *reinterpret_cast<const bf16x4*>(kl + at);
-        l8.h.b = *reinterpret_cast<const bf16x4*>(kl + at + 32);
-        sc[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(l8.v, qh[k], sc[J], 0, 0, 0);
-        sc[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h8.v, ql[k], sc[J], 0, 0, 0);
-        sc[J] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(h8.v, qh[k], sc[J], 0, 0, 0);
-      }
-#pragma unroll
-      for (int k = 0; k < KS; ++k)
-#pragma unroll
-        for (int hf = 0; hf < 2; ++hf) {
-          const f32x4 x = *reinterpret_cast<const f32x4*>(F + J * DKP + 32 * k + 16 * hf + 4 * kq);
-#pragma unroll
-          for (int e = 0; e < 4; ++e) qv[k][4 * hf + e] *= x[e];
-        }
-    }
-  }
-  split_q();
   const f32x4 own = *reinterpret_cast<const f32x4*>(A + (wave * BT + r16) * AP + 4 * kq);
   bf16x8 ph[NB / 2], pl[NB / 2];
 #pragma unroll
