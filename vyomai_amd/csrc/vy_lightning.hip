@@ -21,10 +21,22 @@ namespace {
 using namespace vy_decay;
 
 // ---- chunked form ----------------------------------------------------------------------------
-// eight key columns d .. of a chunk's token t: rotated and scaled (ROT), else as loaded
+// Both kernels of a chunk request everything they read before they use any of it, and take `span` value columns, 64 at a time, so
+// that keys, queries and scores are made once for all of them and the next tile is on its way while one is multiplied.  Bound by
+// memory then (the states and q, k, v once are 54 us of chunk_out at 8 x 1024 tokens and 16 heads of 128 x 128, 40 us of chunk_kv):
+// 135 -> 68 and 79 -> 50 us against a workgroup per 64 columns that loaded piece after piece.
+__device__ __forceinline__ bf16x8 raw8(const bf16* p, bool ok) { return ok ? *reinterpret_cast<const bf16x8*>(p) : bf16x8{}; }
+__device__ __forceinline__ bf16x8 act8(bf16x8 r, int silu) {   // (zero stays zero)
+  if (silu) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) r[e] = (bf16)vy_silu((float)r[e]);
+  }
+  return r;
+}
+// eight key columns d .. of a chunk's token: rotated and scaled (ROT), else as loaded
 template <bool ROT>
-__device__ __forceinline__ void key8(const DecayArgs& a, const bf16* p, bool ok, int pos, int d, float (&v)[8]) {
-  const bf16x8 k8 = load8(p, ok, a.silu);
+__device__ __forceinline__ void key8(const DecayArgs& a, bf16x8 raw, int pos, int d, float (&v)[8]) {
+  const bf16x8 k8 = act8(raw, a.silu);
 #pragma unroll
   for (int e = 0; e < 8; ++e) v[e] = (float)k8[e];
   if constexpr (ROT) {
@@ -34,10 +46,11 @@ __device__ __forceinline__ void key8(const DecayArgs& a, const bf16* p, bool ok,
   }
 }
 
-// grid (chunks, value blocks of 64, B * h)
+// grid (chunks, value columns / span, B * h)
 template <int DKP, bool ROT>
-__global__ __launch_bounds__(256) void chunk_kv_kernel(DecayArgs a) {
-  constexpr int KP = (DKP + 8) * 2, VP = (64 + 8) * 2;
+__global__ __launch_bounds__(256) void chunk_kv_kernel(DecayArgs a, int span) {
+  constexpr int KP = (DKP + 8) * 2, VP = (64 + 8) * 2, KN = C * (DKP / 8) / 256;
+  static_assert(C * 8 == 512 && KN * 256 == C * (DKP / 8), "whole pieces per thread");
   __shared__ __attribute__((aligned(16))) char smem[C * (2 * KP + VP)];
   char* kh = smem;
   char* kl = smem + C * KP;
@@ -46,71 +59,90 @@ __global__ __launch_bounds__(256) void chunk_kv_kernel(DecayArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
   const int ch = blockIdx.x, bh = blockIdx.z, b = bh / a.h, head = bh - b * a.h;
-  const int v0 = (int)blockIdx.y * 64;
+  const int first_v = (int)blockIdx.y * span, end_v = min(a.dv, first_v + span);
   const int n = a.count ? min(a.count[b], a.L) : a.L;
   const int m = max(0, min(C, n - ch * C));            // tokens of this chunk
   const int first = ROT ? a.start[a.slots ? a.slots[b] : b] + ch * C : 0;
   const float* pw = a.pow + (int64_t)head * (C + 1);
   const bf16* P = (const bf16*)a.p + ((int64_t)b * a.L + ch * C) * a.ldp;
-  for (int i = threadIdx.x; i < C * (DKP / 8); i += 256) {
-    const int t = i / (DKP / 8), d = (i % (DKP / 8)) * 8;
-    const bool ok = t < m && d < a.dk;
-    float k8[8];
-    key8<ROT>(a, P + (int64_t)t * a.ldp + a.ok + head * a.dk + d, ok, first + t, d, k8);
-    const float w = t < m ? pw[m - 1 - t] : 0.f;
+  bf16x8 k8[KN], v8[2];
+  float w[KN];
+  auto fetch = [&](int v0) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = threadIdx.x + 256 * i, t = x >> 3, d = v0 + (x & 7) * 8;
+      v8[i] = raw8(P + (int64_t)t * a.ldp + a.ov + head * a.dv + d, t < m && d < a.dv);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < KN; ++i) {
+    const int x = threadIdx.x + 256 * i, t = x / (DKP / 8), d = (x % (DKP / 8)) * 8;
+    k8[i] = raw8(P + (int64_t)t * a.ldp + a.ok + head * a.dk + d, t < m && d < a.dk);
+    w[i] = t < m ? pw[m - 1 - t] : 0.f;
+  }
+  fetch(first_v);
+#pragma unroll
+  for (int i = 0; i < KN; ++i) {
+    const int x = threadIdx.x + 256 * i, t = x / (DKP / 8), d = (x % (DKP / 8)) * 8;
+    float v[8];
+    key8<ROT>(a, k8[i], first + t, d, v);
     bf16x8 hi, lo;
 #pragma unroll
-    for (int e = 0; e < 8; ++e) { bf16 x, y; split_bf16(k8[e] * w, x, y); hi[e] = x; lo[e] = y; }
+    for (int e = 0; e < 8; ++e) { bf16 p, q; split_bf16(v[e] * w[i], p, q); hi[e] = p; lo[e] = q; }
     *reinterpret_cast<bf16x8*>(kh + t * KP + d * 2) = hi;
     *reinterpret_cast<bf16x8*>(kl + t * KP + d * 2) = lo;
   }
-  for (int i = threadIdx.x; i < C * 8; i += 256) {
-    const int t = i >> 3, d = (i & 7) * 8;
-    const bool ok = t < m && v0 + d < a.dv;
-    *reinterpret_cast<bf16x8*>(vt + t * VP + d * 2) = load8(P + (int64_t)t * a.ldp + a.ov + head * a.dv + v0 + d, ok, a.silu);
-  }
-  __syncthreads();
   float* U = a.U + ((int64_t)bh * a.nc + ch) * a.dk * a.dv;
   const int lr = 4 * kq + (r16 >> 2), lc = (4 * (r16 & 3)) * 2;
   const unsigned khb = vy_lds_addr(kh) + lr * KP + lc, klb = vy_lds_addr(kl) + lr * KP + lc, vb = vy_lds_addr(vt) + lr * VP + lc;
-  for (int blk = wave; blk < DKP / 16; blk += 4) {      // 16 key rows of the state
-    if (blk * 16 >= a.dk) break;
-    f32x4 acc[4];
+  for (int v0 = first_v; v0 < end_v; v0 += 64) {
 #pragma unroll
-    for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int tt = 0; tt < C / 32; ++tt) {
-      bf16x8 fh = tr_frag<0>(khb + tt * 32 * KP + blk * 32, KP), fl = tr_frag<0>(klb + tt * 32 * KP + blk * 32, KP);
-      bf16x8 fv[4];
-      vy_static_for<4>([&](auto i_c) {
-        constexpr int i = decltype(i_c)::value;
-        fv[i] = tr_frag<i * 32>(vb + tt * 32 * VP, VP);
-      });
-      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-      vy_tie(fh);
-      vy_tie(fl);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        vy_tie(fv[i]);
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl, fv[i], acc[i], 0, 0, 0);
-        acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh, fv[i], acc[i], 0, 0, 0);
-      }
+    for (int i = 0; i < 2; ++i) {
+      const int x = threadIdx.x + 256 * i;
+      *reinterpret_cast<bf16x8*>(vt + (x >> 3) * VP + (x & 7) * 16) = act8(v8[i], a.silu);
     }
+    __syncthreads();
+    if (v0 + 64 < end_v) fetch(v0 + 64);
+    for (int blk = wave; blk < DKP / 16; blk += 4) {      // 16 key rows of the state
+      if (blk * 16 >= a.dk) break;
+      f32x4 acc[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i)
+      for (int i = 0; i < 4; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        const int r = blk * 16 + 4 * kq + e, c = v0 + 16 * i + r16;
-        if (r < a.dk && c < a.dv) U[(int64_t)r * a.dv + c] = acc[i][e];
+      for (int tt = 0; tt < C / 32; ++tt) {
+        bf16x8 fh = tr_frag<0>(khb + tt * 32 * KP + blk * 32, KP), fl = tr_frag<0>(klb + tt * 32 * KP + blk * 32, KP);
+        bf16x8 fv[4];
+        vy_static_for<4>([&](auto i_c) {
+          constexpr int i = decltype(i_c)::value;
+          fv[i] = tr_frag<i * 32>(vb + tt * 32 * VP, VP);
+        });
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        vy_tie(fh);
+        vy_tie(fl);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          vy_tie(fv[i]);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl, fv[i], acc[i], 0, 0, 0);
+          acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh, fv[i], acc[i], 0, 0, 0);
+        }
       }
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int r = blk * 16 + 4 * kq + e, c = v0 + 16 * i + r16;
+          if (r < a.dk && c < a.dv) U[(int64_t)r * a.dv + c] = acc[i][e];
+        }
+    }
+    __syncthreads();   // the tile has been read
   }
 }
 
-// grid (chunks, value blocks of 64, B * h): wave w computes rows 16 w .. + 15 of the chunk (C = 64)
+// grid (chunks, value columns / span, B * h): wave w computes rows 16 w .. + 15 of the chunk (C = 64)
 template <int DKP, bool ROT>
-__global__ __launch_bounds__(256) void chunk_out_kernel(DecayArgs a) {
+__global__ __launch_bounds__(256, 2) void chunk_out_kernel(DecayArgs a, int span) {
   static_assert(C == 64, "one 16-row block per wave");
-  constexpr int KP = (DKP + 8) * 2, VP = (64 + 8) * 2;
+  constexpr int KP = (DKP + 8) * 2, VP = (64 + 8) * 2, KN = C * (DKP / 8) / 256, SN = DKP * 16 / 256;
   constexpr int KS = DKP / 32, KB = ROT ? 2 : 1;        // key images: hi, lo
   __shared__ __attribute__((aligned(16))) char smem[C * (KB * KP + VP) + 2 * DKP * VP + (C + 1) * 4];
   char* kt = smem;
@@ -122,98 +154,98 @@ __global__ __launch_bounds__(256) void chunk_out_kernel(DecayArgs a) {
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
   const int ch = blockIdx.x, bh = blockIdx.z, b = bh / a.h, head = bh - b * a.h;
-  const int v0 = (int)blockIdx.y * 64;
+  const int first_v = (int)blockIdx.y * span, end_v = min(a.dv, first_v + span);
   const int rows = min(C, a.L - ch * C);
   const bf16* P = (const bf16*)a.p + ((int64_t)b * a.L + ch * C) * a.ldp;
   const float* Sg = a.U + ((int64_t)bh * a.nc + ch) * a.dk * a.dv;
   const int first = ROT ? a.start[a.slots ? a.slots[b] : b] + ch * C : 0;
-  for (int i = threadIdx.x; i < C * (DKP / 8); i += 256) {
-    const int t = i / (DKP / 8), d = (i % (DKP / 8)) * 8;
-    const bf16* src = P + (int64_t)t * a.ldp + a.ok + head * a.dk + d;
-    const bool ok = t < rows && d < a.dk;
-    if constexpr (ROT) {
-      float k8[8];
-      key8<true>(a, src, ok, first + t, d, k8);
-      bf16x8 hi, lo;
-#pragma unroll
-      for (int e = 0; e < 8; ++e) { bf16 x, y; split_bf16(k8[e], x, y); hi[e] = x; lo[e] = y; }
-      *reinterpret_cast<bf16x8*>(kt + t * KP + d * 2) = hi;
-      *reinterpret_cast<bf16x8*>(kt + C * KP + t * KP + d * 2) = lo;
-    } else {
-      *reinterpret_cast<bf16x8*>(kt + t * KP + d * 2) = load8(src, ok, a.silu);
-    }
-  }
-  for (int i = threadIdx.x; i < C * 8; i += 256) {
-    const int t = i >> 3, d = (i & 7) * 8;
-    *reinterpret_cast<bf16x8*>(vt + t * VP + d * 2) =
-        load8(P + (int64_t)t * a.ldp + a.ov + head * a.dv + v0 + d, t < rows && v0 + d < a.dv, a.silu);
-  }
-  for (int i = threadIdx.x; i < DKP * 16; i += 256) {
-    const int r = i >> 4, c = (i & 15) * 4;
-    union { struct { bf16x4 hi, lo; } h; f32x4 f; } w;
-    w.f = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (r < a.dk && v0 + c < a.dv) w.f = *reinterpret_cast<const f32x4*>(Sg + (int64_t)r * a.dv + v0 + c);
-    *reinterpret_cast<bf16x4*>(sh + r * VP + c * 2) = w.h.hi;
-    *reinterpret_cast<bf16x4*>(sl + r * VP + c * 2) = w.h.lo;
-  }
-  for (int i = threadIdx.x; i <= C; i += 256) pw[i] = a.pow[(int64_t)head * (C + 1) + i];
   // the wave's query rows, in the k order of the transposed state fragments (4 kq .. and 16 + 4 kq ..)
   const int qi = 16 * wave + r16;
-  bf16x8 qf[KS], ql[ROT ? KS : 1];
+  bf16x8 k8[KN], v8[2];
+  bf16x4 q4[KS][2];
+  f32x4 s4[SN];
+  auto fetch = [&](int v0) {
+#pragma unroll
+    for (int i = 0; i < SN; ++i) {
+      const int x = threadIdx.x + 256 * i, r = x >> 4, c = v0 + (x & 15) * 4;
+      s4[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (r < a.dk && c < a.dv) s4[i] = *reinterpret_cast<const f32x4*>(Sg + (int64_t)r * a.dv + c);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = threadIdx.x + 256 * i, t = x >> 3, d = v0 + (x & 7) * 8;
+      v8[i] = raw8(P + (int64_t)t * a.ldp + a.ov + head * a.dv + d, t < rows && d < a.dv);
+    }
+  };
+  auto put = [&]() {   // what fetch has brought
+#pragma unroll
+    for (int i = 0; i < SN; ++i) {
+      const int x = threadIdx.x + 256 * i, at = (x >> 4) * VP + (x & 15) * 8;
+      union { struct { bf16x4 hi, lo; } h; f32x4 f; } w;
+      w.f = s4[i];
+      *reinterpret_cast<bf16x4*>(sh + at) = w.h.hi;
+      *reinterpret_cast<bf16x4*>(sl + at) = w.h.lo;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const int x = threadIdx.x + 256 * i;
+      *reinterpret_cast<bf16x8*>(vt + (x >> 3) * VP + (x & 7) * 16) = act8(v8[i], a.silu);
+    }
+  };
+#pragma unroll
+  for (int i = 0; i < KN; ++i) {
+    const int x = threadIdx.x + 256 * i, t = x / (DKP / 8), d = (x % (DKP / 8)) * 8;
+    k8[i] = raw8(P + (int64_t)t * a.ldp + a.ok + head * a.dk + d, t < rows && d < a.dk);
+  }
   {
     const bf16* Q = P + (int64_t)min(qi, rows - 1) * a.ldp + a.oq + head * a.dk;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
+    for (int ks = 0; ks < KS; ++ks)
 #pragma unroll
       for (int hf = 0; hf < 2; ++hf) {
         const int d = 32 * ks + 16 * hf + 4 * kq;
-        bf16x4 q4 = {};
-        if (d < a.dk) q4 = *reinterpret_cast<const bf16x4*>(Q + d);
-        if constexpr (ROT) {
-          float v[4];
+        q4[ks][hf] = d < a.dk ? *reinterpret_cast<const bf16x4*>(Q + d) : bf16x4{};
+      }
+  }
+  fetch(first_v);
+  if (threadIdx.x <= C) pw[threadIdx.x] = a.pow[(int64_t)head * (C + 1) + threadIdx.x];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = activate((float)q4[e], a.silu);
-          if (a.half) rotate(trig_row(a, first + qi), a.half, d, v);
+  for (int i = 0; i < KN; ++i) {
+    const int x = threadIdx.x + 256 * i, t = x / (DKP / 8), d = (x % (DKP / 8)) * 8;
+    if constexpr (ROT) {
+      float v[8];
+      key8<true>(a, k8[i], first + t, d, v);
+      bf16x8 hi, lo;
 #pragma unroll
-          for (int e = 0; e < 4; ++e) { bf16 x, y; split_bf16(v[e], x, y); qf[ks][4 * hf + e] = x; ql[ks][4 * hf + e] = y; }
-        } else {
+      for (int e = 0; e < 8; ++e) { bf16 p, q; split_bf16(v[e], p, q); hi[e] = p; lo[e] = q; }
+      *reinterpret_cast<bf16x8*>(kt + t * KP + d * 2) = hi;
+      *reinterpret_cast<bf16x8*>(kt + C * KP + t * KP + d * 2) = lo;
+    } else {
+      *reinterpret_cast<bf16x8*>(kt + t * KP + d * 2) = act8(k8[i], a.silu);
+    }
+  }
+  bf16x8 qf[KS], ql[ROT ? KS : 1];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) qf[ks][4 * hf + e] = (bf16)activate((float)q4[e], a.silu);
-        }
+  for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+    for (int hf = 0; hf < 2; ++hf) {
+      const int d = 32 * ks + 16 * hf + 4 * kq;
+      if constexpr (ROT) {
+        float v[4];
+#pragma unroll
+        for (int e = 0; e < 4; ++e) v[e] = activate((float)q4[ks][hf][e], a.silu);
+        if (a.half) rotate(trig_row(a, first + qi), a.half, d, v);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) { bf16 x, y; split_bf16(v[e], x, y); qf[ks][4 * hf + e] = x; ql[ks][4 * hf + e] = y; }
+      } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) qf[ks][4 * hf + e] = (bf16)activate((float)q4[ks][hf][e], a.silu);
       }
     }
-  }
+  put();
   __syncthreads();
-  const int lr = 4 * kq + (r16 >> 2), lc = (4 * (r16 & 3)) * 2;
-  const unsigned shb = vy_lds_addr(sh) + lr * VP + lc, slb = vy_lds_addr(sl) + lr * VP + lc, vb = vy_lds_addr(vt) + lr * VP + lc;
-  f32x4 o[4];
-#pragma unroll
-  for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
-  // O^T += S^T Q^T
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    bf16x8 fh[4], fl[4];
-    vy_static_for<4>([&](auto i_c) {
-      constexpr int i = decltype(i_c)::value;
-      fh[i] = tr_frag<i * 32>(shb + ks * 32 * VP, VP);
-      fl[i] = tr_frag<i * 32>(slb + ks * 32 * VP, VP);
-    });
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      vy_tie(fh[i]);
-      vy_tie(fl[i]);
-      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl[i], qf[ks], o[i], 0, 0, 0);
-      if constexpr (ROT) o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh[i], ql[ks], o[i], 0, 0, 0);
-      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh[i], qf[ks], o[i], 0, 0, 0);
-    }
-  }
-  const float dq = pw[qi + 1];
-#pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int e = 0; e < 4; ++e) o[i][e] *= dq;
-  // O^T += V^T (decayed scores)^T over 32 keys at a time
+  // decayed scores, transposed, 32 keys at a time
+  bf16x8 ph[C / 32], pl[C / 32];
 #pragma unroll
   for (int tt = 0; tt < C / 32; ++tt) {
     if (32 * tt > 16 * wave + 15) break;
@@ -237,7 +269,6 @@ __global__ __launch_bounds__(256) void chunk_out_kernel(DecayArgs a) {
         sc[blk] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(kf.v, qf[ks], sc[blk], 0, 0, 0);
       }
     }
-    bf16x8 ph, pl;
 #pragma unroll
     for (int blk = 0; blk < 2; ++blk)
 #pragma unroll
@@ -246,33 +277,76 @@ __global__ __launch_bounds__(256) void chunk_out_kernel(DecayArgs a) {
         const float s = kj <= qi ? sc[blk][r] * pw[qi - kj] : 0.f;
         bf16 x, y;
         split_bf16(s, x, y);
-        ph[4 * blk + r] = x;
-        pl[4 * blk + r] = y;
+        ph[tt][4 * blk + r] = x;
+        pl[tt][4 * blk + r] = y;
       }
-    bf16x8 fv[4];
-    vy_static_for<4>([&](auto i_c) {
-      constexpr int i = decltype(i_c)::value;
-      fv[i] = tr_frag<i * 32>(vb + tt * 32 * VP, VP);
-    });
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      vy_tie(fv[i]);
-      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fv[i], pl, o[i], 0, 0, 0);
-      o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fv[i], ph, o[i], 0, 0, 0);
-    }
   }
-  if (qi < rows) {
-    bf16* O = (bf16*)a.out + ((int64_t)b * a.L + ch * C + qi) * a.ldo + head * a.dv + v0;
+  const float dq = pw[qi + 1];
+  const int lr = 4 * kq + (r16 >> 2), lc = (4 * (r16 & 3)) * 2;
+  const unsigned shb = vy_lds_addr(sh) + lr * VP + lc, slb = vy_lds_addr(sl) + lr * VP + lc, vb = vy_lds_addr(vt) + lr * VP + lc;
+  for (int v0 = first_v; v0 < end_v; v0 += 64) {
+    const bool more = v0 + 64 < end_v;
+    if (more) fetch(v0 + 64);
+    f32x4 o[4];
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int c = 16 * i + 4 * kq;
-      if (v0 + c < a.dv) {
-        bf16x4 w;
+    for (int i = 0; i < 4; ++i) o[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    // O^T += S^T Q^T
 #pragma unroll
-        for (int e = 0; e < 4; ++e) w[e] = (bf16)o[i][e];
-        *reinterpret_cast<bf16x4*>(O + c) = w;
+    for (int ks = 0; ks < KS; ++ks) {
+      bf16x8 fh[4], fl[4];
+      vy_static_for<4>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        fh[i] = tr_frag<i * 32>(shb + ks * 32 * VP, VP);
+        fl[i] = tr_frag<i * 32>(slb + ks * 32 * VP, VP);
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        vy_tie(fh[i]);
+        vy_tie(fl[i]);
+        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fl[i], qf[ks], o[i], 0, 0, 0);
+        if constexpr (ROT) o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh[i], ql[ks], o[i], 0, 0, 0);
+        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fh[i], qf[ks], o[i], 0, 0, 0);
       }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < 4; ++e) o[i][e] *= dq;
+    // O^T += V^T (decayed scores)^T
+#pragma unroll
+    for (int tt = 0; tt < C / 32; ++tt) {
+      if (32 * tt > 16 * wave + 15) break;
+      bf16x8 fv[4];
+      vy_static_for<4>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        fv[i] = tr_frag<i * 32>(vb + tt * 32 * VP, VP);
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        vy_tie(fv[i]);
+        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fv[i], pl[tt], o[i], 0, 0, 0);
+        o[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(fv[i], ph[tt], o[i], 0, 0, 0);
+      }
+    }
+    if (qi < rows) {
+      bf16* O = (bf16*)a.out + ((int64_t)b * a.L + ch * C + qi) * a.ldo + head * a.dv + v0;
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const int c = 16 * i + 4 * kq;
+        if (v0 + c < a.dv) {
+          bf16x4 w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = (bf16)o[i][e];
+          *reinterpret_cast<bf16x4*>(O + c) = w;
+        }
+      }
+    }
+    if (more) {
+      __syncthreads();   // the tiles have been read
+      put();
+      __syncthreads();
     }
   }
 }
@@ -301,13 +375,16 @@ extern "C" int vy_decay_attn(const void* p, int64_t ldp, int64_t oq, int64_t ok,
               (int)vy_cdiv(L, C), (float*)ws, (const float2*)rope, rope_dims / 2, rope_len > 0 ? rope_len : 1, k_scale, nullptr, nullptr, nullptr};
   if (chunked(L, dk, dtype)) {
     if (!ws || ws_bytes < vy_decay_attn_ws_bytes(B, L, h, dk, dv, dtype)) VY_FAIL(VY_ERR_ARG, "%s: workspace too small", who);
-    const dim3 grid(a.nc, (unsigned)vy_cdiv(dv, 64), (unsigned)(B * h)), block(256);
+    // all value columns in one workgroup where every CU gets one (heads of 128 x 128, chunk_out: 2048 workgroups 68 us, 4096 of 64
+    // columns 89; 256 and 512: 14.0 and 14.8; 88 and 176: 12.5 and 10.0)
+    const int span = B * h * a.nc >= 256 ? (int)vy_cdiv(dv, 64) * 64 : 64;
+    const dim3 grid(a.nc, (unsigned)vy_cdiv(dv, span), (unsigned)(B * h)), block(256);
     const dim3 sgrid((unsigned)vy_cdiv((int64_t)dk * dv, 1024), (unsigned)(B * h));
 #define CH_GO(D, ROT)                                                           \
   do {                                                                          \
-    hipLaunchKernelGGL((chunk_kv_kernel<D, ROT>), grid, block, 0, st, a);       \
+    hipLaunchKernelGGL((chunk_kv_kernel<D, ROT>), grid, block, 0, st, a, span); \
     hipLaunchKernelGGL(chunk_scan_kernel<false>, sgrid, block, 0, st, a);              \
-    hipLaunchKernelGGL((chunk_out_kernel<D, ROT>), grid, block, 0, st, a);      \
+    hipLaunchKernelGGL((chunk_out_kernel<D, ROT>), grid, block, 0, st, a, span); \
   } while (0)
     const bool rot = a.half || k_scale != 1.f;
     if (dk <= 32) { if (rot) CH_GO(32, true); else CH_GO(32, false); }
