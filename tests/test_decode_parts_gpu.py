@@ -45,3 +45,10 @@ def test_a_step_equals_the_same_rows_as_a_prompt(B, width, ff, heads, dim):
         a, b = a.double(), b.double()
         assert torch.isfinite(a).all()
         assert (a - b).norm() <= 24 * 2.0 ** -9 * b.norm(), float((a - b).norm() / b.norm())
+
+
+@pytest.mark.parametrize("B", [5, 16, 17, 32])
+@pytest.mark.parametrize("ff", [1400, 2603, 4096, 5203, 8003])
+def test_a_step_through_wide_products(B, ff):
+    """[gate; up] products of 2800 to 16016 columns: 16, 24, 32, 48 and 64 weight rows a workgroup, the last ones ragged."""
+    test_a_step_equals_the_same_rows_as_a_prompt(B, 520, ff, 8, 128)

@@ -13,7 +13,8 @@ template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3
 
 // acc[t][j] (in wave 0 only) = 16 rows ws[t] x 16 rows xs[j]; a lane's pointers are its row (lane & 15) + 8 (lane >> 4).
 // D: a lane owns row lane & 15 of X and rows 4 (lane >> 4) .. + 3 of W.
-template <int NT, int MB, bool ONCE = true, int NW = 4>
+// HALF: the last 16 weight rows are 8.
+template <int NT, int MB, bool ONCE = true, int NW = 4, bool HALF = false>
 __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB],
                                        f32x4* red) {
   constexpr int U = STEPS<NT, MB>;
@@ -33,8 +34,9 @@ __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* 
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
-        if constexpr (ONCE) w[u][t] = in ? __builtin_nontemporal_load(at) : zero8;
-        else w[u][t] = in ? *at : zero8;
+        const bool row = in && (!HALF || t < NT - 1 || (lane & 15) < 8);
+        if constexpr (ONCE) w[u][t] = row ? __builtin_nontemporal_load(at) : zero8;
+        else w[u][t] = row ? *at : zero8;
       }
 #pragma unroll
       for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
@@ -80,23 +82,24 @@ __device__ __forceinline__ float finish(const Dense& a, float v, int n) {
   return v;
 }
 
-// rows 16 NT tile .. + 16 NT - 1 of W against all of X
-template <int MB, int NW = 4, int NT = 1>
+// rows R tile .. + R - 1 of W against all of X, R = 16 NT (HALF: - 8)
+template <int MB, int NW = 4, int NT = 1, bool HALF = false>
 __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int K) {   // K: columns of x and w that count
+  constexpr int R = 16 * NT - (HALF ? 8 : 0);
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const bf16* ws[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) ws[t] = a.w + (int64_t)min(16 * (NT * tile + t) + r16, a.N - 1) * a.K + 8 * kq;
+  for (int t = 0; t < NT; ++t) ws[t] = a.w + (int64_t)min(R * tile + 16 * t + r16, a.N - 1) * a.K + 8 * kq;
   const bf16* xs[MB];
 #pragma unroll
   for (int j = 0; j < MB; ++j) xs[j] = a.x + (int64_t)min(16 * j + r16, a.M - 1) * a.ldx + 8 * kq;
   f32x4 acc[NT][MB];
-  stream<NT, MB, true, NW>(ws, xs, K, acc, red);
+  stream<NT, MB, true, NW, HALF>(ws, xs, K, acc, red);
   if (threadIdx.x >= 64) return;
 #pragma unroll
   for (int i = 0; i < NT * MB; ++i) {
-    const int m = 16 * (i % MB) + r16, n = 16 * (NT * tile + i / MB) + 4 * kq;
-    if (m >= a.M) continue;
+    const int m = 16 * (i % MB) + r16, n = R * tile + 16 * (i / MB) + 4 * kq;
+    if (m >= a.M || (HALF && i / MB == NT - 1 && kq >= 2)) continue;
     const f32x4 v = acc[i / MB][i % MB];
     if (a.f32) {
 #pragma unroll

@@ -5,10 +5,10 @@ namespace {
 
 using vy_rows::Dense;
 
-template <int MB, int NW, int NT>
+template <int MB, int NW, int NT, bool HALF = false>
 __global__ __launch_bounds__(64 * NW) void rows_linear_kernel(Dense a) {
   __shared__ f32x4 red[vy_rows::RED<NT, MB, NW>];
-  vy_rows::dense<MB, NW, NT>(a, red, blockIdx.x);
+  vy_rows::dense<MB, NW, NT, HALF>(a, red, blockIdx.x, a.K);
 }
 
 // K cut into slices of `len` columns: fp32 partial sums [slice][M][N]
@@ -22,13 +22,35 @@ __global__ __launch_bounds__(256) void rows_parts_kernel(Dense a, int len, int t
   vy_rows::dense<MB, 4, NT>(a, red, tile, min(len, a.K - k0));
 }
 
+// Weight rows of a workgroup.  What one CU takes in (25 to 40 GB/s) sets the time, and a workgroup reads x -- 16 MB rows of K -- beside
+// its weights: so the rows that make the fullest CU read least.  24 are one workgroup a CU where 16 are two on half of them.  32 rows:
+// 6144 x 1024 9.7 -> 8.6 us on 24 (16 at first), 6144 x 2048 16.9 -> 12.9, 12288 x 2048 24.7 -> 19.4 on 48, 16384 x 2048 26.9 -> 25.7
+// on 64 (32), 32000 x 2048 47.3 -> 44.6 on 64 (32); 8192 x 1024 stays on 32 (9.3; 24: 12.5).  Up to 16 rows x weighs half and wide products
+// stream from HBM, so only 24 in place of 16 pays, up to 16384: 8 rows, 6144 x 2048 10.4 -> 9.2, 12288 x 2048 15.9 -> 14.4, 32000 x 1024
+// 16.7 (24: 18.0).
 template <int MB>
 void rows_go(const Dense& a, hipStream_t st) {
-  const unsigned tiles = (unsigned)((a.N + 15) / 16);
-  // few workgroups with long rows: twice the waves each; many: two tiles each, for half the traffic of x
-  if (a.N <= 4096 && a.K >= 2048) hipLaunchKernelGGL((rows_linear_kernel<MB, 8, 1>), dim3(tiles), dim3(512), 0, st, a);
-  else if (MB == 1 || a.N < 8192) hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 1>), dim3(tiles), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 2>), dim3((tiles + 1) / 2), dim3(256), 0, st, a);
+  // few workgroups with long rows: twice the waves each
+  if (a.N <= 4096 && a.K >= 2048) {
+    hipLaunchKernelGGL((rows_linear_kernel<MB, 8, 1>), dim3((unsigned)vy_cdiv(a.N, 16)), dim3(512), 0, st, a);
+    return;
+  }
+  auto rounds = [&](int r) { return vy_cdiv(vy_cdiv(a.N, r), 256); };
+  int best = 16;
+  if constexpr (MB == 1) {
+    if (a.N <= 16384 && rounds(24) < rounds(16)) best = 24;
+  } else {
+    for (const int r : {24, 32, 48, 64})
+      if (rounds(r) * (16 * MB + r) < rounds(best) * (16 * MB + best)) best = r;
+  }
+  const dim3 grid((unsigned)vy_cdiv(a.N, best)), block(256);
+  if (best == 16) hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 1>), grid, block, 0, st, a);
+  else if (best == 24) hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 2, true>), grid, block, 0, st, a);
+  else if constexpr (MB > 1) {
+    if (best == 32) hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 2>), grid, block, 0, st, a);
+    else if (best == 48) hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 3>), grid, block, 0, st, a);
+    else hipLaunchKernelGGL((rows_linear_kernel<MB, 4, 4>), grid, block, 0, st, a);
+  }
 }
 
 }  // namespace
