@@ -104,15 +104,21 @@ __device__ __forceinline__ void attn_rotate8(const AttnParams& p, int b, int qi,
 // ------------------------------------------------------------------------------------------
 // MFMA flash forward (bf16).  EXT = 1: per-sequence start positions and the sigmoid output gate; 2: also the sliding window,
 // the sink and the queries' rotary positions.
+// dh = 128: one wave's softmax and MFMAs cannot overlap each other, so it takes two waves on a SIMD to keep the matrix cores
+// busy.  Two K/V tiles in LDS (66 KB) and eight K, then eight V^T fragments in registers at a time (245 VGPRs) let two workgroups share
+// a CU; three tiles (98 KB) and all fragments at once (370 registers) left one wave on each SIMD.  Causal, before -> after: 1 x 16
+// heads x 8192 417 -> 301 us (914 TFLOP/s of the visible half), 3 x 16 x 2731 172 -> 114, 8 x 16 x 1024 81 -> 52, 32 x 16 x 250
+// 53 -> 31, 1 x 8 x 100 13.7 -> 10.5.
 // ------------------------------------------------------------------------------------------
 template <int DH, int EXT = 0>
-__global__ __launch_bounds__(256, DH == 64 ? 3 : 1) void attn_fwd_mfma_kernel(AttnParams p) {
+__global__ __launch_bounds__(256, DH == 64 ? 3 : 2) void attn_fwd_mfma_kernel(AttnParams p) {
   constexpr int RB = DH * 2;            // bytes per K/V row
   constexpr int TILE = 64 * RB;         // bytes per 64-key tile
   constexpr int NP = TILE / 1024 / 4;   // 1-KiB LDS-DMA pieces per wave per tile
   constexpr int KS = DH / 16;           // k-steps of the QK^T contraction
   constexpr int ND = DH / 32;           // 32-wide d blocks of O^T
-  constexpr int NS = 3;                 // K/V tiles in the LDS ring: NS - 1 tiles of loads in flight (4: no gain)
+  // K/V tiles in the LDS ring: NS - 1 tiles of loads in flight (dh = 64: 4 no gain; dh = 128: two rings of two share a CU)
+  constexpr int NS = DH == 64 ? 3 : 2;
   constexpr int KPW = 256;              // key-padding visibility words (64 keys each): S <= 16384
   // ONE shared object (a second one makes hipcc wait vmcnt(0) before every ds_read while LDS-DMA
   // is in flight): K ring, V ring, then 4 flag words for the block-wide OR below
@@ -262,40 +268,53 @@ __global__ __launch_bounds__(256, DH == 64 ? 3 : 1) void attn_fwd_mfma_kernel(At
     // fragment i only (lgkmcnt counts in order) and the V^T fragments are requested two at a time behind each QK^T
     // MFMA, so they land under the remaining MFMAs and the softmax.  (With compiler-visible K reads every QK^T MFMA
     // sat behind an lgkmcnt(0) that also drained the V^T reads just issued.)
-    bf16x8 kfr[2 * KS];
-    unsigned ka[KS];
+    unsigned ka[KS], vbase[ND];
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) ka[ks] = k_lds[ks] + buf * TILE;
-    vy_static_for<2 * KS>([&](auto i_c) {
-      constexpr int i = decltype(i_c)::value;
-      kfr[i] = vy_lds_read128_off<(i / KS) * 32 * RB>(ka[i % KS]);
-    });
-    unsigned vbase[ND];
 #pragma unroll
     for (int n = 0; n < ND; ++n) vbase[n] = v_lds[n] + buf * TILE;
-    bf16x8 vfr[4 * ND];
-    auto vread = [&](auto f_c) {
-      constexpr int f = decltype(f_c)::value;
-      if constexpr (f < 4 * ND) {
-        constexpr int n = f >> 2, kb = (f >> 1) & 1, s_ = f & 1;
-        vfr[f] = vy_lds_tr16_pair_off<NS * TILE + (32 * kb + 16 * s_) * RB, NS * TILE + (32 * kb + 16 * s_ + 8) * RB>(vbase[n]);
-      }
+    auto kread = [&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      return vy_lds_read128_off<(i / KS) * 32 * RB>(ka[i % KS]);
     };
+    // V^T fragment f: column f >> 2, keys 32 ((f >> 1) & 1) + 16 (f & 1) ..
+    auto vload = [&](auto f_c) {
+      constexpr int f = decltype(f_c)::value, n = f >> 2, kb = (f >> 1) & 1, s_ = f & 1;
+      return vy_lds_tr16_pair_off<NS * TILE + (32 * kb + 16 * s_) * RB, NS * TILE + (32 * kb + 16 * s_ + 8) * RB>(vbase[n]);
+    };
+    constexpr bool FEW = DH != 64;           // registers for two waves on a SIMD: K fragments eight, V^T fragments eight at a time
+    bf16x8 kfr[FEW ? KS : 2 * KS], vfr[FEW ? 8 : 4 * ND];
+    vy_static_for<FEW ? KS : 2 * KS>([&](auto i_c) { constexpr int i = decltype(i_c)::value; kfr[i] = kread(i_c); });
 #pragma unroll
     for (int r = 0; r < 16; ++r) { st[0][r] = 0.f; st[1][r] = 0.f; }
-    // V^T requests per QK^T MFMA: 4 ND fragments (two ds_read_b64_tr each) spread over the 2 KS MFMAs
-    constexpr int VPM = (4 * ND + 2 * KS - 1) / (2 * KS);
-    // (lgkmcnt is a 4-bit counter: where the exact count exceeds 15 the wait is for 15, i.e. stricter -- dh = 128)
-    vy_static_for<2 * KS>([&](auto i_c) {
-      constexpr int i = decltype(i_c)::value;
-      // outstanding before this wait: K fragments i .. 2KS-1 and the 2 VPM i tr reads issued so far
-      constexpr int allow = (2 * KS - 1 - i) + 2 * VPM * i;
-      if constexpr (allow <= 15) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(allow) : "memory");
-      else asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
-      vy_tie(kfr[i]);
-      st[i / KS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[i], qf[i % KS], st[i / KS], 0, 0, 0);
-      vy_static_for<VPM>([&](auto j_c) { vread(std::integral_constant<int, i * VPM + decltype(j_c)::value>{}); });
-    });
+    if constexpr (FEW) {
+      static_assert(KS == 8 || DH == 64, "eight k-steps");
+      vy_static_for<2 * KS>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        constexpr int allow = i < KS ? KS - 1 : 2 * KS - 1 - i;   // requested behind fragment i
+        asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(allow) : "memory");
+        vy_tie(kfr[i % KS]);
+        st[i / KS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[i % KS], qf[i % KS], st[i / KS], 0, 0, 0);
+        if constexpr (i < KS) kfr[i] = kread(std::integral_constant<int, i + KS>{});
+      });
+      vy_static_for<4>([&](auto f_c) { constexpr int f = decltype(f_c)::value; vfr[f] = vload(f_c); });
+    } else {
+      // V^T requests per QK^T MFMA: 4 ND fragments (two ds_read_b64_tr each) spread over the 2 KS MFMAs
+      constexpr int VPM = (4 * ND + 2 * KS - 1) / (2 * KS);
+      vy_static_for<2 * KS>([&](auto i_c) {
+        constexpr int i = decltype(i_c)::value;
+        // outstanding before this wait: K fragments i .. 2KS-1 and the 2 VPM i tr reads issued so far
+        constexpr int allow = (2 * KS - 1 - i) + 2 * VPM * i;
+        if constexpr (allow <= 15) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(allow) : "memory");
+        else asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
+        vy_tie(kfr[i]);
+        st[i / KS] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[i], qf[i % KS], st[i / KS], 0, 0, 0);
+        vy_static_for<VPM>([&](auto j_c) {
+          constexpr int f = i * VPM + decltype(j_c)::value;
+          if constexpr (f < 4 * ND) vfr[f] = vload(std::integral_constant<int, f>{});
+        });
+      });
+    }
     unsigned long long vis = ~0ull;
     if (haskp) vis = kpbits[tile];
     const bool need_mask = hasadd || (k0 + 64 > p.S) || (causal && k0 + 63 > start + wave_first) || vis != ~0ull ||
@@ -375,12 +394,32 @@ __global__ __launch_bounds__(256, DH == 64 ? 3 : 1) void attn_fwd_mfma_kernel(At
       for (int s = 0; s < 2; ++s)
 #pragma unroll
         for (int j = 0; j < 8; ++j) pf[kb][s][j] = (bf16)st[kb][8 * s + j];
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    if constexpr (FEW) {
+      vy_static_for<ND>([&](auto n_c) {
+        constexpr int n = decltype(n_c)::value, at = 4 * (n & 1), next = 4 - at;
+        if constexpr (n + 1 < ND) {
+          vy_static_for<4>([&](auto f_c) {
+            constexpr int f = decltype(f_c)::value;
+            vfr[next + f] = vload(std::integral_constant<int, 4 * (n + 1) + f>{});
+          });
+          asm volatile("s_waitcnt lgkmcnt(8)" ::: "memory");
+        } else {
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        }
 #pragma unroll
-    for (int f = 0; f < 4 * ND; ++f) vy_tie(vfr[f]);
+        for (int f = 0; f < 4; ++f) vy_tie(vfr[at + f]);
 #pragma unroll
-    for (int f = 0; f < 4 * ND; ++f)
-      o[f >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[f], pf[(f >> 1) & 1][f & 1], o[f >> 2], 0, 0, 0);
+        for (int f = 0; f < 4; ++f)
+          o[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[at + f], pf[f >> 1][f & 1], o[n], 0, 0, 0);
+      });
+    } else {
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+      for (int f = 0; f < 4 * ND; ++f) vy_tie(vfr[f]);
+#pragma unroll
+      for (int f = 0; f < 4 * ND; ++f)
+        o[f >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[f], pf[(f >> 1) & 1][f & 1], o[f >> 2], 0, 0, 0);
+    }
   };
 
   // Loads run NS-1 tiles ahead of the MFMAs: a tile is waited for with a COUNTED vmcnt (its own
