@@ -5,10 +5,10 @@
 // never wraps: row = position; vy_qkv_rows has put the new tokens there): rows [key 1 | key 2 | value] per key/value head.  So a
 // prompt behind a past needs no copy of it.  Decode steps are vy_window_decode's.
 //
-// All kernels walk the keys once for both maps: one fetch of a row, one value fragment for two products.  Difference and norm are
-// part of the epilogue, in fp32, on accumulators that were never rounded.
+// All kernels walk the keys once for both maps: one fetch of a row from memory.  Difference and norm are part of the epilogue, in
+// fp32, on accumulators that were never rounded.
 //   diff_mfma_kernel  bf16, heads whose two key maps together are as wide as their values, 64 or 128: attn_fwd_mfma_kernel's
-//                     structure (vy_attn.hip) -- 128 query rows per workgroup, 64-key tiles through a three-deep LDS-DMA ring,
+//                     structure (vy_attn.hip) -- 128 query rows per workgroup, four waves a map, 64-key tiles through a three-deep LDS-DMA ring,
 //                     swapped products on mfma_f32_32x32x16, probabilities in registers, transposing reads of the values
 //   diff_gen_kernel   bf16, any widths up to 256: attn_fwd_gen_kernel's structure, 64 query rows, one tile in LDS
 //   diff_row_kernel   fp32 and wider heads: a workgroup per query row and head, 256 keys at a time
@@ -31,49 +31,47 @@ struct DiffArgs {
 };
 
 // ---- two maps of DV / 2 columns, values of DV -------------------------------------------------
+// A wave's softmax and matrix instructions do not overlap each other, so the matrix cores want two waves on a SIMD: the maps have
+// waves of their own (211 registers at DV = 128, 127 at 64), which read the same tiles from LDS.  With both maps in one wave its
+// sums alone were 128 registers, a SIMD had one wave, and the sums were copied at each of the two rescales.  The value fragments
+// are read from LDS twice for it.  Before -> after: 8192 tokens, 16 heads of 128 541 -> 425 us (970 TFLOP/s of the visible half),
+// 3000 x 24 138 -> 111, 32 x 250 x 16 58 -> 51; 8192 tokens, 32 heads of 64 770 -> 488.  Both maps in a wave with fewer fragments
+// at a time, two workgroups on a CU: heads of 64 551, heads of 128 spilled (526, and 34 for 2 x 700 x 16, 28 before, 22 now).
 template <int DV>
-__global__ __launch_bounds__(256, 1) void diff_mfma_kernel(DiffArgs p) {
+__global__ __launch_bounds__(512, 2) void diff_mfma_kernel(DiffArgs p) {
   constexpr int RB = DV * 2;            // bytes per key pair / value row
   constexpr int TILE = 64 * RB;         // bytes per 64-key tile
-  constexpr int NP = TILE / 1024 / 4;   // 1-KiB LDS-DMA pieces per wave per tile
-  constexpr int KS = DV / 16;           // k-steps of both maps' contractions together
-  constexpr int KM = KS / 2;            // of one
+  constexpr int NP = TILE / 1024 / 8;   // 1-KiB LDS-DMA pieces per wave per tile
+  constexpr int RPP = 1024 / RB;        // rows per piece
+  constexpr int KM = DV / 32;           // k-steps of one map's contraction
   constexpr int ND = DV / 32;           // 32-wide blocks of O^T (2 or 4)
   constexpr int NS = 3;                 // tiles in the ring
-  __shared__ __attribute__((aligned(16))) char smem[2 * NS * TILE];
+  __shared__ __attribute__((aligned(256))) char smem[2 * NS * TILE];
   const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), map = wave >> 2, rows = wave & 3;   // waves 0 .. 3: map 1, 4 .. 7: map 2
   const int head = (int)blockIdx.x % p.h, b = (int)blockIdx.x / p.h;   // (heaviest query blocks of every head first)
   const int q0 = ((int)gridDim.y - 1 - (int)blockIdx.y) * 128;
   const int fr = lane & 31, fh = lane >> 5;
-  const int qi = q0 + wave * 32 + fr, qrow = min(qi, p.L - 1);
+  const int qi = q0 + rows * 32 + fr, qrow = min(qi, p.L - 1);
   const int slot = p.slots ? p.slots[b] : b;
   const int start = p.start[slot], S = start + (p.count ? min(p.count[b], p.L) : p.L);
   const int64_t W = 2 * DV;             // a row of the ring
-  const bf16* Q = (const bf16*)p.q + ((int64_t)b * p.L + qrow) * p.ldq + head * DV;
+  const bf16* Q = (const bf16*)p.q + ((int64_t)b * p.L + qrow) * p.ldq + head * DV + map * (DV / 2);
   const bf16* Kb = (const bf16*)p.ring + (int64_t)slot * p.r_ss + (int64_t)(head / (p.h / p.hk)) * p.r_sh;
-  const bf16* Vb = Kb + DV;
 
-  // LDS-DMA source geometry: piece pc covers LDS bytes [pc * 1024, + 1024); swizzles as in attn_fwd_mfma_kernel
-  int ld_row[NP], ld_koff[NP], ld_voff[NP];
-#pragma unroll
-  for (int t = 0; t < NP; ++t) {
-    const int P = (wave * NP + t) * 1024 + lane * 16;
-    const int row = P / RB, off = P % RB;
-    const int ksw = RB == 128 ? (row >> 1) & 7 : row & 15;
-    const int vsw = RB == 128 ? ((row >> 1) & 1) << 6 : (row & 3) << 6;
-    ld_row[t] = row;
-    ld_koff[t] = (((off >> 4) ^ ksw) << 4) >> 1;
-    ld_voff[t] = (off ^ vsw) >> 1;
-  }
+  // LDS-DMA source geometry: piece pc covers LDS bytes [pc * 1024, + 1024); swizzles as in attn_fwd_mfma_kernel.  Piece t of a
+  // wave lies t RPP rows further down: its keys' swizzle differs by 4 t chunks of 16 bytes, its values' does not.
+  const int ld_off = lane * 16 % RB, ld_row = wave * NP * RPP + lane * 16 / RB;
+  const int ld_koff = (((ld_off >> 4) ^ (RB == 128 ? (ld_row >> 1) & 7 : ld_row & 15)) << 4) >> 1;
+  const int ld_voff = (ld_off ^ (RB == 128 ? ((ld_row >> 1) & 1) << 6 : (ld_row & 3) << 6)) >> 1;
   auto stage = [&](int tile, int buf) {
     const int k0 = tile * 64;
 #pragma unroll
     for (int t = 0; t < NP; ++t) {
-      const bf16* row = Kb + (int64_t)min(k0 + ld_row[t], S - 1) * W;   // (rows past the end: the last one, weight 0)
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(row + ld_koff[t]),
+      const bf16* row = Kb + (int64_t)min(k0 + ld_row + t * RPP, max(S - 1, 0)) * W;   // (rows past the end: the last one, weight 0)
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(row + (ld_koff ^ (32 * t))),
                                        (VY_LDS void*)(smem + buf * TILE + (wave * NP + t) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(row + DV + ld_voff[t]),
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(row + DV + ld_voff),
                                        (VY_LDS void*)(smem + (NS + buf) * TILE + (wave * NP + t) * 1024), 16, 0, 0);
     }
   };
@@ -81,125 +79,90 @@ __global__ __launch_bounds__(256, 1) void diff_mfma_kernel(DiffArgs p) {
   const int li = lane & 15, g16 = (lane >> 4) & 1;
   const int v_sw = RB == 128 ? ((li >> 3) & 1) << 6 : ((li >> 2) & 3) << 6;
   const int v_lane_row = 4 * fh + (li >> 2), v_lane_off = 32 * g16 + 8 * (li & 3);
-  unsigned k_lds[KS], v_lds[ND];
-#pragma unroll
-  for (int ks = 0; ks < KS; ++ks) k_lds[ks] = vy_lds_addr(smem) + fr * RB + (((2 * ks + fh) ^ k_sw) << 4);
-#pragma unroll
-  for (int n = 0; n < ND; ++n) v_lds[n] = vy_lds_addr(smem) + v_lane_row * RB + ((64 * n + v_lane_off) ^ v_sw);
+  // k-step k of a key row, block n of a value row: XORs of k << 5 and n << 6, bits that only the swizzles touch
+  const unsigned k_lds = (vy_lds_addr(smem) + fr * RB + ((fh ^ k_sw) << 4)) ^ (map * KM << 5);
+  const unsigned v_lds = vy_lds_addr(smem) + v_lane_row * RB + (v_lane_off ^ v_sw);
 
-  f32x16 o[2][ND];
-  float m_run[2], l_run[2];
+  f32x16 o[ND];
 #pragma unroll
-  for (int m = 0; m < 2; ++m) {
-    m_run[m] = -FLT_MAX;
-    l_run[m] = 0.f;
+  for (int n = 0; n < ND; ++n)
 #pragma unroll
-    for (int n = 0; n < ND; ++n)
-#pragma unroll
-      for (int r = 0; r < 16; ++r) o[m][n][r] = 0.f;
-  }
+    for (int r = 0; r < 16; ++r) o[n][r] = 0.f;
+  float m_run = -FLT_MAX, l_run = 0.f;
   const float c = p.scale * LOG2E;
   const int nt = max(1, (min(S, start + q0 + 128) + 63) / 64);
-  const int wave_first = q0 + wave * 32, wave_last = wave_first + 31;
-  bf16x8 qf[KS];
+  const int wave_first = q0 + rows * 32, wave_last = wave_first + 31;
+  bf16x8 qf[KM];
 
   auto compute = [&](int tile, int buf) {
     const int k0 = tile * 64;
-    if (k0 > start + wave_last) return;   // wave-uniform: wholly above this wave's diagonal
-    // Hidden (asm) LDS reads retired by counted waits: map 1's key fragments first; behind each of its products one of map 2's is
-    // requested, behind those the values'.  The products of map 1's probabilities with the values run under map 2's softmax.
+    // Hidden (asm) LDS reads retired by counted waits: the key fragments, behind each of their products some of the values'.
+    const unsigned ka = k_lds + buf * TILE, va = v_lds + buf * TILE;
     f32x16 st[2];
-    bf16x8 kfr[2][KS];                    // [map][KM kb + k]
-    auto kread = [&](auto m_c, auto i_c) {
-      constexpr int m = decltype(m_c)::value, i = decltype(i_c)::value;
-      kfr[m][i] = vy_lds_read128_off<(i / KM) * 32 * RB>(k_lds[m * KM + i % KM] + buf * TILE);
-    };
-    vy_static_for<KS>([&](auto i_c) { kread(std::integral_constant<int, 0>{}, i_c); });
-    bf16x8 vfr[4 * ND];
-    auto vread = [&](auto f_c) {
-      constexpr int f = decltype(f_c)::value;
-      if constexpr (f < 4 * ND) {
-        constexpr int n = f >> 2, kb = (f >> 1) & 1, s_ = f & 1;
-        vfr[f] = vy_lds_tr16_pair_off<NS * TILE + (32 * kb + 16 * s_) * RB, NS * TILE + (32 * kb + 16 * s_ + 8) * RB>(v_lds[n] + buf * TILE);
-      }
-    };
-    constexpr int VPM = (4 * ND + KS - 1) / KS;   // value fragments requested behind each product of map 2
-    const bool need_mask = k0 + 64 > S || k0 + 63 > start + wave_first;
-    const int klim = min(S - 1, qi + start) - k0 - 4 * fh;   // register r of block kb: key k0 + 4 fh + 32 kb + (r & 3) + 8 (r >> 2)
-    float neg_m;
-    auto scores = [&](auto m_c) {
-      constexpr int m = decltype(m_c)::value;
+    bf16x8 kfr[2 * KM], vfr[4 * ND];          // [KM kb + k], [4 n + 2 kb + half]
+    vy_static_for<2 * KM>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      kfr[i] = vy_lds_read128_off<(i / KM) * 32 * RB>(ka ^ ((i % KM) << 5));
+    });
 #pragma unroll
-      for (int kb = 0; kb < 2; ++kb)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) st[kb][r] = 0.f;
-      vy_static_for<KS>([&](auto i_c) {
-        constexpr int i = decltype(i_c)::value;
-        constexpr int allow = (KS - 1 - i) + (m == 0 ? i : 2 * VPM * i);   // requested behind fragment i so far
-        if constexpr (allow <= 15) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(allow) : "memory");
-        else asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
-        vy_tie(kfr[m][i]);
-        st[i / KM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[m][i], qf[m * KM + i % KM], st[i / KM], 0, 0, 0);
-        if constexpr (m == 0) kread(std::integral_constant<int, 1>{}, i_c);
-        else vy_static_for<VPM>([&](auto j_c) { vread(std::integral_constant<int, i * VPM + decltype(j_c)::value>{}); });
+      for (int r = 0; r < 16; ++r) st[kb][r] = 0.f;
+    constexpr int VPM = 4 * ND / (2 * KM);    // value fragments requested behind each product
+    static_assert(VPM * 2 * KM == 4 * ND, "all of them");
+    vy_static_for<2 * KM>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      constexpr int allow = (2 * KM - 1 - i) + 2 * VPM * i;   // requested behind fragment i so far
+      if constexpr (allow <= 15) asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(allow) : "memory");
+      else asm volatile("s_waitcnt lgkmcnt(15)" ::: "memory");
+      vy_tie(kfr[i]);
+      st[i / KM] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[i], qf[i % KM], st[i / KM], 0, 0, 0);
+      vy_static_for<VPM>([&](auto j_c) {
+        constexpr int f = i * VPM + decltype(j_c)::value, n = f >> 2, kb = (f >> 1) & 1, s_ = f & 1;
+        vfr[f] = vy_lds_tr16_pair_off<NS * TILE + (32 * kb + 16 * s_) * RB, NS * TILE + (32 * kb + 16 * s_ + 8) * RB>(va ^ (n << 6));
       });
-      if (need_mask) {
-#pragma unroll
-        for (int kb = 0; kb < 2; ++kb)
-#pragma unroll
-          for (int r = 0; r < 16; ++r) st[kb][r] = 32 * kb + (r & 3) + 8 * (r >> 2) > klim ? -INFINITY : st[kb][r];
-      }
-      float tmax = -INFINITY;
+    });
+    if (k0 + 64 > S || k0 + 63 > start + wave_first) {
+      const int klim = min(S - 1, qi + start) - k0 - 4 * fh;   // register r of block kb: key k0 + 4 fh + 32 kb + (r & 3) + 8 (r >> 2)
 #pragma unroll
       for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, st[kb][r]);
-      tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
-      const float tmax_s = tmax * c;
-      if (__any(tmax_s > m_run[m] + 8.f)) {   // lazy rescale: exp2 arguments stay <= 8
-        const float m_new = fmaxf(m_run[m], tmax_s);
-        const float alpha = __builtin_amdgcn_exp2f(m_run[m] - m_new);
-        m_run[m] = m_new;
-        l_run[m] *= alpha;
+        for (int r = 0; r < 16; ++r) st[kb][r] = 32 * kb + (r & 3) + 8 * (r >> 2) > klim ? -INFINITY : st[kb][r];
+    }
+    float tmax = -INFINITY;
 #pragma unroll
-        for (int n = 0; n < ND; ++n)
+    for (int kb = 0; kb < 2; ++kb)
 #pragma unroll
-          for (int r = 0; r < 16; ++r) o[m][n][r] *= alpha;
-      }
-      neg_m = -m_run[m];
-    };
-    bf16x8 pf[2][4];                          // [map][2 kb + half]
-    auto weigh = [&](auto m_c, int i, float& rs) {   // probabilities i and i + 1 of the lane's 32
-      constexpr int m = decltype(m_c)::value;
+      for (int r = 0; r < 16; ++r) tmax = fmaxf(tmax, st[kb][r]);
+    tmax = fmaxf(tmax, __shfl_xor(tmax, 32, 64));
+    const float tmax_s = tmax * c;
+    if (__any(tmax_s > m_run + 8.f)) {        // lazy rescale: exp2 arguments stay <= 8
+      const float m_new = fmaxf(m_run, tmax_s);
+      const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
+      m_run = m_new;
+      l_run *= alpha;
+#pragma unroll
+      for (int n = 0; n < ND; ++n)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) o[n][r] *= alpha;
+    }
+    bf16x8 pf[4];                             // [2 kb + half]
+    const float neg_m = -m_run;
+    float rs = 0.f;
+#pragma unroll
+    for (int i = 0; i < 32; i += 2) {
       const float e0 = __builtin_amdgcn_exp2f(fmaf(st[i >> 4][i & 15], c, neg_m));
       const float e1 = __builtin_amdgcn_exp2f(fmaf(st[i >> 4][(i & 15) + 1], c, neg_m));
       rs += e0 + e1;
-      pf[m][i >> 3][i & 7] = (bf16)e0;
-      pf[m][i >> 3][(i & 7) + 1] = (bf16)e1;
-    };
-    constexpr std::integral_constant<int, 0> map0{};
-    constexpr std::integral_constant<int, 1> map1{};
-    scores(map0);
-    float rs = 0.f;
-#pragma unroll
-    for (int i = 0; i < 32; i += 2) weigh(map0, i, rs);
-    l_run[0] += rs;                           // this half's keys; the halves are added at the end
-    scores(map1);
+      pf[i >> 3][i & 7] = (bf16)e0;
+      pf[i >> 3][(i & 7) + 1] = (bf16)e1;
+    }
+    l_run += rs;                              // this half's keys; the halves are added at the end
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
     for (int f = 0; f < 4 * ND; ++f) vy_tie(vfr[f]);
-    rs = 0.f;
-    vy_static_for<16>([&](auto i_c) {
-      constexpr int i = decltype(i_c)::value;
-      weigh(map1, 2 * i, rs);
-      vy_static_for<ND / 4 + (ND % 4 && (i & 1) ? 1 : 0)>([&](auto j_c) {
-        constexpr int f = ND >= 4 ? i * (ND / 4) + decltype(j_c)::value : i >> 1;
-        o[0][f >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[f], pf[0][f & 3], o[0][f >> 2], 0, 0, 0);
-      });
-    });
-    l_run[1] += rs;
 #pragma unroll
-    for (int f = 0; f < 4 * ND; ++f) o[1][f >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[f], pf[1][f & 3], o[1][f >> 2], 0, 0, 0);
+    for (int f = 0; f < 4 * ND; ++f) o[f >> 2] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vfr[f], pf[f & 3], o[f >> 2], 0, 0, 0);
   };
   auto wait_tile = [&](int younger) {   // `younger` tiles (2 NP LDS-DMA instructions each) may stay in flight
     if (younger >= 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * NP) : "memory");
@@ -209,48 +172,69 @@ __global__ __launch_bounds__(256, 1) void diff_mfma_kernel(DiffArgs p) {
   for (int s_ = 0; s_ < NS - 1; ++s_)
     if (s_ < nt) stage(s_, s_);
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) qf[ks] = *reinterpret_cast<const bf16x8*>(Q + ks * 16 + fh * 8);
+  for (int k = 0; k < KM; ++k) qf[k] = *reinterpret_cast<const bf16x8*>(Q + k * 16 + fh * 8);
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) asm volatile("" ::"v"(qf[ks]));   // retired here: a wait inside the loop would drain the ring
-  for (int t = 0; t < nt; ++t) {
+  for (int k = 0; k < KM; ++k) asm volatile("" ::"v"(qf[k]));   // retired here: a wait inside the loop would drain the ring
+  auto next_tile = [&](int t) {
     wait_tile(min(NS - 2, nt - 1 - t));
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     if (t + NS - 1 < nt) stage(t + NS - 1, (t + NS - 1) % NS);   // the buffer tile t - 1 was read from
+  };
+  const int mine = min(nt, (start + wave_last) / 64 + 1);   // the further tiles lie wholly above this wave's diagonal
+  int t = 0;
+  for (; t < mine; ++t) {
+    next_tile(t);
     compute(t, t % NS);
   }
-  const float i1 = 1.f / (l_run[0] + __shfl_xor(l_run[0], 32, 64));
-  const float i2 = p.lambda / (l_run[1] + __shfl_xor(l_run[1], 32, 64));
+  for (; t < nt; ++t) next_tile(t);
+
+  // Map 2's sums go to the wave with the same rows of map 1, lane by lane, through the (now idle) ring.
+  constexpr int PART = ND * 16 * 64 * 4;   // bytes of a wave's sums
+  static_assert(4 * PART + 4 * 64 * 4 <= 2 * NS * TILE, "map 2's sums fit over the ring");
+  float* sums = reinterpret_cast<float*>(smem + rows * PART) + lane;
+  float* totals = reinterpret_cast<float*>(smem + 4 * PART) + rows * 64 + lane;
+  const float l_tot = l_run + __shfl_xor(l_run, 32, 64);
+  __syncthreads();
+  if (map) {
+#pragma unroll
+    for (int n = 0; n < ND; ++n)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) sums[(n * 16 + r) * 64] = o[n][r];
+    *totals = l_tot;
+  }
+  __syncthreads();
+  if (map) return;
+  const float i1 = 1.f / l_tot, i2 = p.lambda / *totals;
   float sq = 0.f;
 #pragma unroll
   for (int n = 0; n < ND; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-      const float d = o[0][n][r] * i1 - o[1][n][r] * i2;
-      o[0][n][r] = d;
+      const float d = o[n][r] * i1 - sums[(n * 16 + r) * 64] * i2;
+      o[n][r] = d;
       sq = fmaf(d, d, sq);   // (padded value columns are zero)
     }
   sq += __shfl_xor(sq, 32, 64);
   const float f = rms_factor(sq, p.n_v, p.eps) * p.out_scale;
-  // through LDS: whole 16-byte pieces of rows to memory
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
+  // through LDS, over the sums that this wave alone has read: whole 16-byte pieces of rows to memory
   constexpr int OROW = RB + 16, LPR = RB / 16;
-  static_assert(4 * 32 * OROW <= 2 * NS * TILE, "the waves' rows fit over the ring");
-  char* ot = smem + wave * (32 * OROW);
+  static_assert(32 * OROW <= PART, "a wave's rows fit over its sums");
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+  char* ot = smem + rows * PART;
 #pragma unroll
   for (int n = 0; n < ND; ++n)
 #pragma unroll
     for (int rg = 0; rg < 4; ++rg) {
       bf16x4 w;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) w[e] = (bf16)(o[0][n][4 * rg + e] * f);
+      for (int e = 0; e < 4; ++e) w[e] = (bf16)(o[n][4 * rg + e] * f);
       *reinterpret_cast<bf16x4*>(ot + fr * OROW + (32 * n + 8 * rg + 4 * fh) * 2) = w;
     }
   asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // wave-private
 #pragma unroll
   for (int it = 0; it < 32 * LPR / 64; ++it) {
-    const int r = (it * 64 + lane) / LPR, ch = (it * 64 + lane) % LPR, row = q0 + wave * 32 + r;
+    const int r = (it * 64 + lane) / LPR, ch = (it * 64 + lane) % LPR, row = q0 + rows * 32 + r;
     const bf16x8 v = *reinterpret_cast<const bf16x8*>(ot + r * OROW + ch * 16);
     if (row < p.L) *reinterpret_cast<bf16x8*>((bf16*)p.out + ((int64_t)b * p.L + row) * p.ldo + head * DV + ch * 8) = v;
   }
@@ -536,8 +520,8 @@ extern "C" int vy_diff_attn_fwd(const void* q, int64_t ldq, const void* ring, in
   const dim3 block(256);
   if (dtype == VY_BF16 && L > 1 && dim == vdim && (vdim == 64 || vdim == 128)) {
     const dim3 grid((unsigned)(h * B), (unsigned)((L + 127) / 128));
-    if (vdim == 64) hipLaunchKernelGGL(diff_mfma_kernel<64>, grid, block, 0, st, a);
-    else hipLaunchKernelGGL(diff_mfma_kernel<128>, grid, block, 0, st, a);
+    if (vdim == 64) hipLaunchKernelGGL(diff_mfma_kernel<64>, grid, dim3(512), 0, st, a);
+    else hipLaunchKernelGGL(diff_mfma_kernel<128>, grid, dim3(512), 0, st, a);
   } else if (dtype == VY_BF16 && L > 1 && a.dim <= 256 && vdim <= 256) {
     const dim3 grid((unsigned)(h * B), (unsigned)((L + 63) / 64));
     if (a.dim <= 32) gen_go<32>(a, grid, st);
