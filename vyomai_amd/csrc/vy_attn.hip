@@ -240,20 +240,37 @@ __global__ __launch_bounds__(256, DH == 64 ? 3 : 2) void attn_fwd_mfma_kernel(At
   if (EXT == 2 && window) t0 = max(0, start + q0 - window + 1) >> 6;
   // tiles of kept keys ahead of them: step u of the walk takes tile tile_at(u), steps u0 .. nt - 1
   const int keep = EXT == 2 && window ? p.keep : 0;
-  const int kept = EXT == 2 ? min((keep + 63) >> 6, t0) : 0, u0 = t0 - kept;
+  const int kept = EXT == 2 ? min((keep + 63) >> 6, t0) : 0;
+  int u0 = t0 - kept;
   auto tile_at = [&](int u) { return EXT == 2 && u < t0 ? u - u0 : u; };
 
   // key-padding mask -> one 64-bit visibility word per key tile, built once (an ordinary load inside
-  // the tile loop would make the compiler drain the LDS-DMA ring with vmcnt(0) every tile)
+  // the tile loop would make the compiler drain the LDS-DMA ring with vmcnt(0) every tile).  The walk goes from the first tile
+  // with a visible key to the last: hidden keys weigh 0, and the padding of a batch is at its sequences' ends.  61 sequences of
+  // 167 .. 500 of 500 tokens, 12 heads of 64: 82 -> 65 us; all 500 long 77.5 -> 78.6.
   unsigned long long* kpbits = reinterpret_cast<unsigned long long*>(smem + 2 * NS * TILE + 64);
   if (haskp) {
+    int* ends = reinterpret_cast<int*>(smem + 2 * NS * TILE) + 8;   // [wave] first, [wave] one past the last
+    int first = nt, last = 0;
     for (int t = wave; t < nt; t += 4) {
       const int kj = t * 64 + lane;
       const bool vis = kj < p.S && kp[kj < p.S ? kj : 0] != 0;
       const unsigned long long bits = __ballot(vis);
       if (lane == 0) kpbits[t] = bits;
+      if (bits) {
+        first = min(first, t);
+        last = t + 1;
+      }
+    }
+    if (lane == 0) {
+      ends[wave] = first;
+      ends[4 + wave] = last;
     }
     __syncthreads();
+    if (EXT == 0) {
+      u0 = __builtin_amdgcn_readfirstlane(min(min(ends[0], ends[1]), min(ends[2], ends[3])));
+      nt = __builtin_amdgcn_readfirstlane(max(max(ends[4], ends[5]), max(ends[6], ends[7])));   // (no visible key: 0, below u0)
+    }
   }
 
   auto compute = [&](int tile, int buf) {

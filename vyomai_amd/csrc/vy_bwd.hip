@@ -540,7 +540,7 @@ __device__ __forceinline__ unsigned long long range_bits64(int lo, int hi) {
 // forward kernel); masks are per-lane bit words, P is recomputed as exp2(fma(s, c, -lse*log2e)).
 __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
   constexpr int DH = 64, RB = 128, TILE = 64 * RB, NS = 3, KPW = 256;
-  __shared__ __attribute__((aligned(16))) char smem[2 * NS * TILE + KPW * 8];  // K ring, V ring, key-padding words
+  __shared__ __attribute__((aligned(16))) char smem[2 * NS * TILE + KPW * 8 + 32];  // K ring, V ring, key-padding words, their ends
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int nqb = (p.L + 127) / 128;
@@ -629,15 +629,30 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
   if (causal) nt = max(1, min(nt, (min(p.S, p.start_pos + q0 + 128) + 63) / 64));
   const int wave_first = q0 + wave * 32, wave_last = wave_first + 31;
 
+  // only the tiles from the first with a visible key to the last: hidden keys pass nothing on (with the dK/dV kernel's hidden blocks,
+  // 61 sequences of 167 .. 500 of 500 tokens, 12 heads: 258 -> 219 us for both kernels; 16 of 600 .. 2000 834 -> 657)
   unsigned long long* kpbits = reinterpret_cast<unsigned long long*>(smem + 2 * NS * TILE);
+  int u0 = 0;
   if (haskp) {
+    int* ends = reinterpret_cast<int*>(smem + 2 * NS * TILE + KPW * 8);   // [wave] first, [wave] one past the last
+    int first = nt, last = 0;
     for (int t = wave; t < nt; t += 4) {
       const int kj = t * 64 + lane;
       const bool vis = kj < p.S && kp[kj < p.S ? kj : 0] != 0;
       const unsigned long long bits = __ballot(vis);
       if (lane == 0) kpbits[t] = bits;
+      if (bits) {
+        first = min(first, t);
+        last = t + 1;
+      }
+    }
+    if (lane == 0) {
+      ends[wave] = first;
+      ends[4 + wave] = last;
     }
     __syncthreads();
+    u0 = __builtin_amdgcn_readfirstlane(min(min(ends[0], ends[1]), min(ends[2], ends[3])));
+    nt = __builtin_amdgcn_readfirstlane(max(max(ends[4], ends[5]), max(ends[6], ends[7])));   // (no visible key: 0, below u0)
   }
 
   auto compute = [&](int tile, int buf) {
@@ -710,17 +725,17 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
   // becomes a vmcnt(0) inside the loop and drains the ring every tile)
 #pragma unroll
   for (int s_ = 0; s_ < NS - 1; ++s_)
-    if (s_ < nt) stage(s_, s_);
+    if (u0 + s_ < nt) stage(u0 + s_, s_);
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) { vy_tie(qf[ks]); vy_tie(gf[ks]); }
   vy_tie(neg_lse); vy_tie(neg_delta);
-  for (int t = 0; t < nt; ++t) {
+  for (int t = u0; t < nt; ++t) {
     if (t + 1 < nt) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + NS - 1 < nt) stage(t + NS - 1, (t + NS - 1) % NS);
-    compute(t, t % NS);
+    if (t + NS - 1 < nt) stage(t + NS - 1, (t - u0 + NS - 1) % NS);
+    compute(t, (t - u0) % NS);
   }
   if (qi < p.L) {
     bf16* D = p.dq + (int64_t)b * p.dq_sb + (int64_t)head * p.dq_sh + (int64_t)qi * p.dq_sl;
@@ -748,7 +763,7 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
 __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
   constexpr int DH = 64, RB = 128, QR = 64, QT = QR * RB, NS = 3;  // one 64-row tile = 8 KiB
   constexpr int ST_OFF = 2 * NS * QT;                              // NS x [lse 64 floats][-delta 64 floats]
-  __shared__ __attribute__((aligned(16))) char smem[2 * NS * QT + NS * 512];
+  __shared__ __attribute__((aligned(16))) char smem[2 * NS * QT + NS * 512 + 16];   // .., a word per wave
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   // grid (hk*B, key blocks): key block 0 sees every query row under a causal mask -> all of them first
@@ -769,7 +784,15 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
   const bool causal = p.mask_kind & VY_MASK_CAUSAL;
   const bool haskp = p.mask_kind & VY_MASK_KEYPAD;
   const bool key_dead = (kj >= p.S) || (haskp && !p.keypad[(int64_t)b * p.kp_sb + krow]);
-  const bool any_dead = __any(key_dead);
+  const bool any_dead = __any(key_dead), all_dead = __all(key_dead);
+  // hidden keys get zero gradients: a block of them sweeps no query row, a wave of them multiplies nothing
+  bool block_dead = false;
+  if (haskp) {
+    int* dead = reinterpret_cast<int*>(smem + ST_OFF + NS * 512);
+    if (lane == 0) dead[wave] = all_dead;
+    __syncthreads();
+    block_dead = __builtin_amdgcn_readfirstlane(dead[0] & dead[1] & dead[2] & dead[3]) != 0;
+  }
   const float c = p.scale * LOG2E;
 
   f32x16 dk[2], dv[2];
@@ -785,7 +808,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
     const int first_row = kblk * 128 - p.start_pos;
     qt_first = first_row > 0 ? first_row / QR : 0;
   }
-  const int per_head = nqt > qt_first ? nqt - qt_first : 0;
+  const int per_head = nqt > qt_first && !block_dead ? nqt - qt_first : 0;
   const int total = per_head * n_rep;
 
   // LDS-DMA: tile = 8 pieces of 1 KiB; wave w loads pieces 2w, 2w+1 of the Q tile and of the dO tile
@@ -830,6 +853,7 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
     }
 
   auto compute = [&](int it, int buf) {
+    if (all_dead) return;
     const int hh = it / per_head, qt = qt_first + (it - hh * per_head);
     const char* qb_ = smem + buf * QT;
     const char* gb_ = smem + (NS + buf) * QT;
