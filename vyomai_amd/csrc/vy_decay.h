@@ -156,6 +156,94 @@ __global__ __launch_bounds__(256) void decay_recurrent_kernel(DecayArgs a) {
   }
 }
 
+// One token a sequence: workgroup = 32 value columns of one (b, head), thread (rg, quad) the rows rg, rg + 32, ... of four columns.
+// Bound by the state's read and write, for few sequences by the round trips: the token's row and the state are requested together,
+// 16 bytes a lane and whole 128-byte lines a row (16 columns: 2 to 3 times the time of 32; 64: as fast for 32 sequences, 0.3 us more
+// for one).  Heads of 128 x 128, one column a lane -> this: 1 x 8 heads 4.1 -> 3.1 us, 8 x 8 6.1 -> 3.6, 32 x 8 10.6 -> 6.2 (5.4 TB/s
+// of state), 64 x 16 27.3 -> 21.8; 4 x 8 of 256 x 256 9.9 -> 4.6.
+template <typename T, int RPT, bool GATED>
+__global__ __launch_bounds__(256) void decay_step_kernel(DecayArgs a) {
+  constexpr int COLS = 32, QUADS = COLS / 4, RG = 256 / QUADS, DK = RG * RPT;
+  static_assert(DK <= 256, "a thread per row");
+  __shared__ float qs[DK], ks[DK], fs[GATED ? DK : 1];
+  __shared__ __attribute__((aligned(16))) float vs[COLS], red[4][COLS];
+  const int tid = threadIdx.x, quad = tid % QUADS, rg = tid / QUADS;
+  const int head = blockIdx.y, b = blockIdx.z, c0 = (int)blockIdx.x * COLS, vc = c0 + 4 * quad;
+  const int slot = a.slots ? a.slots[b] : b, first = a.start[slot];
+  T* O = (T*)a.out + (int64_t)b * a.ldo + head * a.dv;
+  const bool some = !a.count || a.count[b] > 0;   // else: the state stays, zeros for whatever reads whole batches
+  const T* P = (const T*)a.p + (int64_t)b * a.ldp;
+  // the token's row first, the state behind it: the row's wait leaves the state in flight
+  const bool ok = tid < a.dk, vok = tid < COLS && c0 + tid < a.dv;
+  const T* row = P + (int64_t)head * a.dk + (ok ? tid : 0);
+  float q = VyT<T>::ld(row + a.oq), k = VyT<T>::ld(row + a.ok), v = vok ? VyT<T>::ld(P + a.ov + head * a.dv + c0 + tid) : 0.f;
+  const bool turned = !GATED && ok && tid < 2 * a.half;
+  const int to = turned ? (tid & 1 ? -1 : 1) : 0;   // the other column of the pair
+  float qx = 0.f, kx = 0.f, bias = 0.f, lower = 0.f;
+  float2 cs = {1.f, 0.f};
+  if constexpr (GATED) {
+    const int64_t at = (int64_t)head * a.dk + (ok ? tid : 0);
+    if (a.f_bias) bias = a.f_bias[at];
+    lower = a.f_lower[at];
+  } else if (turned) {
+    qx = VyT<T>::ld(row + a.oq + to);
+    kx = VyT<T>::ld(row + a.ok + to);
+    cs = trig_row(a, first)[tid >> 1];
+  }
+  const float decay = GATED ? 0.f : a.pow[(int64_t)head * (C + 1) + 1];
+  float* S = a.state + ((int64_t)slot * a.h + head) * a.dk * a.dv + vc;
+  f32x4 s[RPT];
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int r = rg + RG * i;
+    s[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (r < a.dk && vc < a.dv) s[i] = *reinterpret_cast<const f32x4*>(S + (int64_t)r * a.dv);
+  }
+  if (tid < DK) {
+    float f = 1.f;
+    if constexpr (GATED) {
+      float kk = 0.f;
+      if (ok) forget_gate(k + bias, lower, f, kk);
+      k = kk;
+      q = activate(q, a.silu);
+      fs[tid] = f;
+    } else {
+      q = activate(q, a.silu);
+      k = activate(k, a.silu);
+      if (turned) {
+        const float sn = tid & 1 ? cs.y : -cs.y;
+        q = q * cs.x + activate(qx, a.silu) * sn;
+        k = k * cs.x + activate(kx, a.silu) * sn;
+      }
+      k *= a.k_scale;
+    }
+    qs[tid] = ok ? q : 0.f;
+    ks[tid] = ok ? k : 0.f;
+  }
+  if (tid < COLS) vs[tid] = activate(v, GATED ? 0 : a.silu);
+  __syncthreads();
+  const f32x4 v4 = *reinterpret_cast<const f32x4*>(vs + 4 * quad);
+  f32x4 o = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < RPT; ++i) {
+    const int r = rg + RG * i;
+    const float f = GATED ? fs[r] : decay, kr = ks[r], qr = qs[r];
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      s[i][e] = fmaf(f, first == 0 ? 0.f : s[i][e], kr * v4[e]);   // an empty slot's state is zero, whatever lies there
+      o[e] = fmaf(s[i][e], qr, o[e]);
+    }
+    if (some && r < a.dk && vc < a.dv) *reinterpret_cast<f32x4*>(S + (int64_t)r * a.dv) = s[i];
+  }
+#pragma unroll
+  for (int e = 0; e < 4; ++e)
+#pragma unroll
+    for (int x = QUADS; x < 64; x *= 2) o[e] += __shfl_xor(o[e], x, 64);
+  if ((tid & 63) < QUADS) *reinterpret_cast<f32x4*>(&red[tid >> 6][4 * quad]) = o;
+  __syncthreads();
+  if (vok) VyT<T>::st(O + c0 + tid, some ? (red[0][tid] + red[1][tid]) + (red[2][tid] + red[3][tid]) : 0.f);
+}
+
 // ---- chunked form ----------------------------------------------------------------------------
 __device__ __forceinline__ bf16x8 load8(const bf16* p, bool ok, int silu) {
   bf16x8 r = {};
@@ -233,11 +321,12 @@ template <typename T, bool GATED>
 int recurrent_go(const DecayArgs& a, hipStream_t st) {
   const dim3 grid((unsigned)vy_cdiv(a.dv, 16), a.h, a.B), block(256);
   if (a.L == 1) {
-    // a decode step streams the state: whole 256-byte row pieces where enough workgroups remain, else narrow columns
-    const int64_t wide = vy_cdiv(a.dv, 64) * a.h * a.B;
-    const dim3 wgrid((unsigned)vy_cdiv(a.dv, 64), a.h, a.B);
-    if (wide >= 512 && a.dk <= 64) hipLaunchKernelGGL((decay_recurrent_kernel<T, 64, 16, 1, GATED>), wgrid, block, 0, st, a);
-    else if (wide >= 512 && a.dk <= 128) hipLaunchKernelGGL((decay_recurrent_kernel<T, 64, 32, 1, GATED>), wgrid, block, 0, st, a);
+    // (states that 16-byte pieces do not reach, and wider heads: a column a lane)
+    const dim3 sgrid((unsigned)vy_cdiv(a.dv, 32), a.h, a.B);
+    const bool quads = a.dv % 4 == 0 && (uintptr_t)a.state % 16 == 0;
+    if (quads && a.dk <= 64) hipLaunchKernelGGL((decay_step_kernel<T, 2, GATED>), sgrid, block, 0, st, a);
+    else if (quads && a.dk <= 128) hipLaunchKernelGGL((decay_step_kernel<T, 4, GATED>), sgrid, block, 0, st, a);
+    else if (quads && a.dk <= 256) hipLaunchKernelGGL((decay_step_kernel<T, 8, GATED>), sgrid, block, 0, st, a);
     else if (a.dk <= 64) hipLaunchKernelGGL((decay_recurrent_kernel<T, 16, 4, 1, GATED>), grid, block, 0, st, a);
     else if (a.dk <= 128) hipLaunchKernelGGL((decay_recurrent_kernel<T, 16, 8, 1, GATED>), grid, block, 0, st, a);
     else if (a.dk <= 256) hipLaunchKernelGGL((decay_recurrent_kernel<T, 16, 16, 1, GATED>), grid, block, 0, st, a);
