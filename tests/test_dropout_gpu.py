@@ -319,3 +319,34 @@ def test_gemm_tile_variants_agree_with_the_default_selection(variant):
             assert torch.allclose(y1.double(), want, atol=3e-2, rtol=1e-2)
     finally:
         lib.vy_debug_set_gemm_variant(-1)
+
+
+@pytest.mark.parametrize("variant", [0, 5, 12, 40, 41, 1000, -7])
+def test_gemm_tile_variants_of_other_numbers(variant):
+    """40 / 41 choose a tile of the default kernels, other numbers nothing: the same k order, so the same bits, in every column -- plain,
+    dgrad and rotary products, output widths that the tiles of 192 and 256 columns do not divide."""
+    import ctypes as C
+    from vyomai_amd import ops, _lib
+    lib = _lib.load()
+    lib.vy_debug_set_gemm_variant.argtypes = [C.c_int]
+
+    def all_of(M, N, K, heads):
+        x = rnd(M, K, seed=1).to(BF).to(DEV)
+        w = rnd(N, K, seed=2, scale=1 / math.sqrt(K)).to(BF).to(DEV)
+        b = rnd(N, seed=3, scale=0.1).to(BF).to(DEV)
+        y = torch.full((M, N), float("nan"), dtype=BF, device=DEV)
+        dx = torch.full((M, N), float("nan"), dtype=BF, device=DEV)
+        q, k, v = (torch.full((1, heads, M, 64), float("nan"), dtype=BF, device=DEV) for _ in range(3))
+        ops.linear(x, w, b, out=y)
+        ops.linear_dgrad(x, w, out=dx)
+        ops.qkv_rope(x.view(1, M, K), w[: 3 * heads * 64].contiguous(), None, heads, heads, 64, None, None, 0, q, k, v)
+        return y, dx, q, k, v
+    try:
+        for M, N, K, heads in ((16385, 768, 256, 4), (12608, 3080, 64, 16)):
+            lib.vy_debug_set_gemm_variant(-1)
+            want = all_of(M, N, K, heads)
+            lib.vy_debug_set_gemm_variant(variant)
+            got = all_of(M, N, K, heads)
+            assert all(torch.isfinite(a).all() and torch.equal(a, e) for a, e in zip(got, want))
+    finally:
+        lib.vy_debug_set_gemm_variant(-1)

@@ -1,5 +1,5 @@
 """The three dgrad launches of a layer + the FFN2 dgrad with the GELU derivative (B=32 x 512 rows, d=768), per
-GEMM variant:  python tools/bench_dgrad.py [variants...]   (VY_GEMM_VARIANT values; -1 = default selection)"""
+GEMM tile:  python tools/bench_dgrad.py [variants...]   (VY_GEMM_VARIANT: 40 / 41 = 256 x 192 / 256 x 256 tiles; -1 = by cost)"""
 import ctypes as C, math, os, sys
 import torch
 sys.path.insert(0, os.path.dirname(os.path.dirname(os.path.abspath(__file__))))

@@ -2421,14 +2421,17 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     hipLaunchKernelGGL((gemm_nt_bf16_kernel<32, 128, 1, 4, EPI, ACT, GRAD>), dim3(tm * tn), dim3(256), 0,
                        st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot);
   } else {
-    int var = vy_gemm_variant();   // 8 / 9: the 256 x 256 / 256 x 192 tiles of the 32 x 32 x 16 kernel (tests, A/B runs); -1: by cost
-    if (EPI != 0 || GRAD || M < 1025) var = -1;
+    // Tests and A/B runs, more than 1024 rows: 8 / 9 take the 256 x 256 / 256 x 192 tiles of the 32 x 32 x 16 kernel (plain products
+    // alone), 40 / 41 the 256 x 192 / 256 x 256 tiles below where K is not sliced.  Every other value: by cost.
+    const int variant = M > 1024 ? vy_gemm_variant() : -1;
+    const int var = EPI == 0 && !GRAD && (variant == 8 || variant == 9) ? variant : -1;
     const int chip = 256 / g_chains;
     Tiling t{};
     if (var < 0) {
       int64_t ws_bytes;
       splitk_ws(st, 0, &ws_bytes);
       t = pick_tiling(M, N, K, chip, ws_bytes);
+      if (t.slices == 1 && (variant == 40 || variant == 41)) t.kind = variant == 40 ? T_256x192 : T_256x256;
     }
     const int bm = var >= 0 ? 256 : TILE_M[t.kind], bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
     const int tn = (int)vy_cdiv(N, bn), tiles = (int)vy_cdiv(M, bm) * tn, threads = var >= 0 ? 512 : TILE_THREADS[t.kind];
