@@ -77,3 +77,40 @@ def test_rotary_heads_on_small_tiles(B, L, h, hk):
     for got, want in ((q, turn(y[:, :h])), (k, turn(y[:, h:h + hk])), (v, y[:, h + hk:])):
         assert ((got.double() - want).abs() <= 8 * 2.0 ** -9 * size.amax()).all()
     assert float(cache[:, :, :, :pos0].abs().max()) == 0 and float(cache[:, :, :, pos0 + L:].abs().max()) == 0
+
+
+def test_workspaces_that_come_and_go():
+    """Another thread registers the stream's workspace and takes it back (the memory itself stays) while products are launched: each is
+    cut into slices or is not, and has the bits of one of the two."""
+    import threading
+    from vyomai_amd import ops
+    from vyomai_amd._lib import call
+    g = torch.Generator(device=DEV).manual_seed(3)
+    x, w = (torch.randn(n, 8192, device=DEV, generator=g).to(BF) for n in (264, 1024))
+    st, size = torch.cuda.current_stream().cuda_stream, 64 << 20
+    buf = torch.empty(size, dtype=torch.uint8, device=DEV)
+    register = ops._mid_ws
+    ops._mid_ws = lambda rows: None
+    done = threading.Event()
+
+    def turn():
+        while not done.is_set():
+            call("vy_workspace_set", st, None, 0)
+            call("vy_workspace_set", st, buf.data_ptr(), size)
+    other = threading.Thread(target=turn)
+    try:
+        call("vy_workspace_set", st, None, 0)
+        whole = ops.linear(x, w)
+        call("vy_workspace_set", st, buf.data_ptr(), size)
+        sliced = ops.linear(x, w)
+        assert not torch.equal(whole, sliced)
+        other.start()
+        got = [ops.linear(x, w) for _ in range(400)]
+        done.set()
+        other.join()
+        assert all(torch.equal(y, whole) or torch.equal(y, sliced) for y in got)
+    finally:
+        done.set()
+        ops._mid_ws = register
+        call("vy_workspace_set", st, None, 0)
+        ops._WS.pop((torch.cuda.current_device(), st), None)

@@ -1591,16 +1591,13 @@ struct WsEntry { hipStream_t st; void* p; int64_t bytes; };
 WsEntry g_ws[16];
 int g_ws_n = 0;
 std::mutex g_ws_mu;
-// scratch of a stream (vy_workspace_set): its size and, asked for by `need`, its address
-inline float* splitk_ws(hipStream_t st, int64_t need, int64_t* bytes) {
+// scratch of a stream (vy_workspace_set).  A launch looks it up once: slices are chosen for the very buffer that they are written to
+struct Scratch { float* p; int64_t bytes; };
+inline Scratch splitk_ws(hipStream_t st) {
   std::lock_guard<std::mutex> lk(g_ws_mu);
   for (int i = 0; i < g_ws_n; ++i)
-    if (g_ws[i].st == st) {
-      if (bytes) *bytes = g_ws[i].bytes;
-      return g_ws[i].bytes >= need ? (float*)g_ws[i].p : nullptr;
-    }
-  if (bytes) *bytes = 0;
-  return nullptr;
+    if (g_ws[i].st == st) return {(float*)g_ws[i].p, g_ws[i].bytes};
+  return {nullptr, 0};
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1673,14 +1670,14 @@ inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_
   return best;
 }
 
-// BM x BN tiles with K cut into S slices, whose partial sums the second launch adds up in the workspace's order
+// BM x BN tiles with K cut into S slices, whose partial sums the second launch adds up in the workspace's order (ws: sum_slices has
+// seen that they fit)
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD>
 void launch_split(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K, int S,
-                  const EpiPlain<bf16>& ep, const EpiQkv<bf16>& eq, hipStream_t st) {
+                  float* ws, const EpiPlain<bf16>& ep, const EpiQkv<bf16>& eq, hipStream_t st) {
   const int tn = (int)vy_cdiv(N, BN), tm = (int)vy_cdiv(M, BM);
   const int KT = (int)vy_cdiv(K, 64);
   const int tiles = tm * tn;
-  float* ws = splitk_ws(st, (int64_t)S * tiles * BM * BN * 4, nullptr);
   const int per = (KT + S - 1) / S;
   hipLaunchKernelGGL((gemm_nt_bf16_m16_splitk_kernel<BM, BN, WGM, WGN>), dim3(tiles * S), dim3(64 * WGM * WGN), 0, st, X, ldx, W, ldw,
                      (int)M, (int)N, (int)K, tn, tiles, S, per, ws);
@@ -2426,11 +2423,10 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     const int variant = M > 1024 ? vy_gemm_variant() : -1;
     const int var = EPI == 0 && !GRAD && (variant == 8 || variant == 9) ? variant : -1;
     const int chip = 256 / g_chains;
+    const Scratch ws = splitk_ws(st);
     Tiling t{};
     if (var < 0) {
-      int64_t ws_bytes;
-      splitk_ws(st, 0, &ws_bytes);
-      t = pick_tiling(M, N, K, chip, ws_bytes);
+      t = pick_tiling(M, N, K, chip, ws.bytes);
       if (t.slices == 1 && (variant == 40 || variant == 41)) t.kind = variant == 40 ? T_256x192 : T_256x256;
     }
     const int bm = var >= 0 ? 256 : TILE_M[t.kind], bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
@@ -2450,9 +2446,9 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
       case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
       case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, EPI, ACT, GRAD>); break;
       case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, EPI, ACT, GRAD>); break;
-      case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
-      case T_256x128_SPLIT: launch_split<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
-      case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ep, eq, st); break;
+      case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
+      case T_256x128_SPLIT: launch_split<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
+      case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
     }
 #undef VY_TILES
 #undef VY_SMALL
@@ -2465,9 +2461,7 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
 // 8000 x 2 x 4096, K = 1024: 163 -> 134; 700 x 2 x 4096, K = 1024: 25.8 -> 20.6; 100 rows: 10.3 -> 6.8.
 template <int ACT>
 int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K, const EpiPlain<bf16>& ep, hipStream_t st) {
-  int64_t ws_bytes;
-  splitk_ws(st, 0, &ws_bytes);
-  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes);
+  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, splitk_ws(st).bytes);
   const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, TILE_M[t.kind]) * tn;
   const int KT = (int)vy_cdiv(K, BK), per = (KT + t.slices - 1) / t.slices;
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
