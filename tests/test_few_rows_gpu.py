@@ -87,3 +87,76 @@ def test_hybrid_step(make, width, B):
         want = m.logits(m.prefill(ids[:, :t + 1].contiguous(), [t + 1] * B, other, s)[:, -1]).double()
         assert torch.isfinite(got).all()
         assert (got - want).norm() <= 8 * len(m.layers) * 2.0 ** -9 * want.norm(), float((got - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("B", [1, 2, 4])
+def test_what_a_step_refuses(B):
+    """Vocabulary weights that are not there and logits rows narrower than the vocabulary: errors, as from the general launchers, and the
+    plan works again afterwards."""
+    from vyomai_amd._lib import VyomHipError
+    cfg, m = decoder(512, "rope", None, BF, layers=1)
+    x = torch.randn(B, 512, device=DEV, generator=torch.Generator(device=DEV).manual_seed(B)).to(BF)
+    plan, cache = _plan(cfg, m, B, BF)
+    want = _step(plan, cache, x, 5, 1)[0]
+    keep, ldv = plan.plan.head_wv, plan.ldv
+    plan.plan.head_wv = None
+    with pytest.raises(VyomHipError, match="null operand"):
+        plan.step(x, 6)
+    plan.plan.head_wv, plan.ldv = keep, 1000
+    with pytest.raises(VyomHipError, match="1000"):
+        plan.step(x, 6)
+    plan.ldv = ldv
+    assert torch.equal(_step(plan, cache, x, 5, 1)[0], want)
+
+
+@pytest.mark.parametrize("B", [2, 4])
+def test_what_a_hybrid_step_refuses(B):
+    from vyomai_amd import _lib, decode_plan
+    torch.manual_seed(3)
+    with torch.device(DEV):
+        torch.set_default_dtype(BF)
+        try:
+            m = gisitar(1024).eval()
+        finally:
+            torch.set_default_dtype(torch.float32)
+    ids = torch.randint(0, 1003, (B, 3), device=DEV)
+    cache = m.new_cache(B, 8)
+    slots = cache.allocate(B)
+    m.prefill(ids[:, :2].contiguous(), [2] * B, cache, slots)
+    plans, real = [], decode_plan.HybridDecodePlan.step
+
+    def seen(self, *a):
+        plans.append((self, a))
+        return real(self, *a)
+    decode_plan.HybridDecodePlan.step = seen
+    try:
+        m.decode(ids[:, 2].contiguous(), cache, slots)
+    finally:
+        decode_plan.HybridDecodePlan.step = real
+    plan, args = plans[0]
+    head, ldv = plan.plan.head, plan.ldv
+    plan.plan.head = None
+    with pytest.raises(_lib.VyomHipError, match="null operand"):
+        real(plan, *args)
+    plan.plan.head, plan.ldv = head, 1000
+    with pytest.raises(_lib.VyomHipError, match="ldy < N"):
+        real(plan, *args)
+    plan.plan.head, plan.ldv = head, ldv
+
+
+def test_hidden_rows_at_any_address():
+    """vy_decoder_step leaves the hidden state wherever it is asked to: two bytes off a 16-byte line the general launchers take the step."""
+    import ctypes as C
+    from vyomai_amd import _lib, ops
+    cfg, m = decoder(768, "rope", 4, BF)
+    x = torch.randn(2, 768, device=DEV, generator=torch.Generator(device=DEV).manual_seed(9)).to(BF)
+    plan, cache = _plan(cfg, m, 2, BF)
+    logits, want = plan.step(x, 5, want_hidden=True)
+    want = want.clone()
+    for off in (0, 1, 4):
+        room = torch.zeros(2 * 768 + 16, dtype=BF, device=DEV)
+        for logits_ptr in (logits.data_ptr(), None):
+            _lib.call("vy_decoder_step", C.byref(plan.plan), x.data_ptr(), 5, None, room.data_ptr() + 2 * off, logits_ptr, plan.ldv,
+                      ops._raw_stream())
+            got = room[off:off + 2 * 768].view(2, 768).float()
+            assert (got - want.float()).norm() <= 18 * 2.0 ** -8 * want.float().norm() and room[:off].eq(0).all() and room[off + 1536:].eq(0).all()

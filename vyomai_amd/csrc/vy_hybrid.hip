@@ -73,7 +73,7 @@ int product(const vy_hybrid_plan* p, const void* x, const void* w, void* y, int6
     if (rc != VY_ERR_UNSUPPORTED) return rc;
   }
   if (p->dtype == VY_BF16 && p->B <= 4 && N <= INT32_MAX / 2 && vy_few::few_k(vy_few::STORE, vy_few::PLAIN, K) &&
-      (act == VY_ACT_NONE || act == VY_ACT_RELU2 || act == VY_ACT_SOFTCAP) && (uintptr_t)w % 16 == 0) {
+      (act == VY_ACT_NONE || act == VY_ACT_RELU2 || act == VY_ACT_SOFTCAP) && w && (uintptr_t)w % 16 == 0 && ldy >= N) {
     vy_few::Args a{};
     a.M = (int)p->B; a.x = (const bf16*)x; a.ldx = K; a.w = (const bf16*)w; a.N = (int)N; a.bias = (const bf16*)bias; a.act = act;
     a.act_arg = cap; a.y = (bf16*)y; a.ldy = ldy;
@@ -166,8 +166,8 @@ extern "C" int vy_hybrid_decoder_step(const vy_hybrid_plan* p, const int64_t* id
     if (!later.due) return (int)VY_ERR_UNSUPPORTED;
     const bool known = epi == vy_few::GATED ? act == VY_ACT_SILU || act == VY_ACT_GELU_TANH
                                             : act == VY_ACT_NONE || act == VY_ACT_RELU2 || act == VY_ACT_SOFTCAP;
-    if (!known || !vy_few::few_k(epi, vy_few::STREAM, dp) || N > INT32_MAX / 2 || (uintptr_t)weight % 16 || (uintptr_t)later.post % 16 ||
-        (uintptr_t)later.pre % 16) {
+    if (!known || !vy_few::few_k(epi, vy_few::STREAM, dp) || N > INT32_MAX / 2 || ldo < N || !weight || (uintptr_t)weight % 16 ||
+        (uintptr_t)later.post % 16 || (uintptr_t)later.pre % 16) {
       const int bad = settle();
       return bad ? bad : (int)VY_ERR_UNSUPPORTED;
     }

@@ -3,6 +3,7 @@
 #include "vy_common.h"
 #include "vy_few.h"
 #include <stdlib.h>
+#include <initializer_list>
 
 int vy_qkv_rope_fwd_ex(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,
                        const float* cos_tab, const float* sin_tab, int64_t pos0, const int* pos_dev, void* q,
@@ -70,24 +71,27 @@ extern "C" int64_t vy_decode_ws_bytes(int32_t B, int32_t d, int32_t h, int32_t h
          up((vy_splitk_ws_floats(d) > 24 * 32 * (int64_t)d ? vy_splitk_ws_floats(d) : 24 * 32 * (int64_t)d) * 4) + 4096;
 }
 
-// Do the kernels of vy_few.hip take the step's sizes and operands?  (whole 256-column pieces, weights on 16 bytes, norms on 8)
-static bool few_operands(const vy_decode_plan* p, const void* x, const void* logits) {
+// Do the kernels of vy_few.hip take the step's sizes and operands?  (whole 256-column pieces, weights and the hidden rows on 16 bytes,
+// norms on 8; a null weight or norm is the general launchers' to refuse or to leave out)
+static bool few_operands(const vy_decode_plan* p, const void* x, const void* hidden_out, const void* logits) {
   using namespace vy_few;
   if (!few_k(QKV, PLAIN, p->d) || !few_k(QKV, LAYER, p->d) || !few_k(STORE, PLAIN, p->d) || !few_k(STORE, LAYER, p->d) ||
       !few_k(STORE, PLAIN, p->ffn) || p->dh != 64 || p->h * 64 != p->d ||
       (p->act != VY_ACT_NONE && p->act != VY_ACT_GELU_ERF && p->act != VY_ACT_GELU_TANH))
     return false;
-  uintptr_t w = (uintptr_t)x, n = 0;
+  uintptr_t all = (uintptr_t)hidden_out;   // the low bits of every address
+  bool given = true;
+  auto need = [&](std::initializer_list<const void*> weights, std::initializer_list<const void*> norms) {
+    for (const void* w : weights) { all |= (uintptr_t)w; given = given && w; }
+    for (const void* n : norms) { all |= (uintptr_t)n << 1; given = given && n; }
+  };
+  need({x}, {});
   for (int l = 0; l < p->num_layers; ++l) {
     const vy_decode_layer& L = p->layers[l];
-    w |= (uintptr_t)L.wqkv | (uintptr_t)L.wo | (uintptr_t)L.w1 | (uintptr_t)L.w2;
-    n |= (uintptr_t)L.ln1_w | (uintptr_t)L.ln1_b | (uintptr_t)L.ln2_w | (uintptr_t)L.ln2_b;
+    need({L.wqkv, L.wo, L.w1, L.w2}, {L.ln1_w, L.ln1_b, L.ln2_w, L.ln2_b});
   }
-  if (logits) {
-    w |= (uintptr_t)p->head_wd | (uintptr_t)p->head_wv;
-    n |= (uintptr_t)p->head_ln_w | (uintptr_t)p->head_ln_b;
-  }
-  return w % 16 == 0 && n % 8 == 0;
+  if (logits) need({p->head_wd, p->head_wv}, {p->head_ln_w, p->head_ln_b});
+  return given && all % 16 == 0 && (!logits || p->vocab > 0);
 }
 
 // The step of 1 to 4 sequences on the kernels of vy_few.hip: five launches per layer, LayerNorms inside the products behind them.
@@ -154,6 +158,7 @@ extern "C" int vy_decoder_step(const vy_decode_plan* p, const void* x, int64_t p
   if (!p || !x || !p->layers || !p->ws) VY_FAIL(VY_ERR_ARG, "%s: null plan/input/workspace", who);
   if (p->ws_bytes < vy_decode_ws_bytes(p->B, p->d, p->h, p->hk, p->dh, p->ffn, p->dtype))
     VY_FAIL(VY_ERR_ARG, "%s: workspace too small", who);
+  if (logits && ldv < p->vocab) VY_FAIL(VY_ERR_ARG, "%s: logits rows of %ld for a vocabulary of %d", who, (long)ldv, p->vocab);
   const int64_t e = esize(p->dtype);
   const int B = p->B, d = p->d, h = p->h, hk = p->hk, dh = p->dh;
   char* w = (char*)p->ws;
@@ -175,7 +180,7 @@ extern "C" int vy_decoder_step(const vy_decode_plan* p, const void* x, int64_t p
   if (g_decode_lean < 0) { const char* e = getenv("VY_DECODE_LEAN"); g_decode_lean = e ? atoi(e) : 1; }
   const bool lean = g_decode_lean && vy_dec_supported(B, d, h, hk, dh, p->ffn, p->dtype);
   hipStream_t hst = (hipStream_t)stream;
-  if (lean && B <= 4 && p->num_layers > 0 && (pos_dev || pos >= 0) && few_operands(p, x, logits))
+  if (lean && B <= 4 && p->num_layers > 0 && (pos_dev || pos >= 0) && few_operands(p, x, hidden_out, logits))
     return few_decoder_step(p, x, pos, pos_dev, hidden_out, logits, ldv, hst);
   const void* cur = x;
   for (int l = 0; l < p->num_layers; ++l) {
