@@ -403,21 +403,24 @@ template <int BN, int BKW, int MS, int NS, bool MF16 = false>
 __global__ __launch_bounds__(BN * 2, BN == 128 ? 2 : 1) void wgrad_tn_bf16_kernel(
     const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
     float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
-    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag, int whole, int tail_chunk) {
-  // the first `whole` workgroups: chunks of m_chunk rows, tile by tile; the others: chunks of tail_chunk rows of the tiles from `whole` on
-  int split, t2, chunk;
-  if ((int)blockIdx.x < whole) {
-    const int wg = xcd_remap(blockIdx.x, whole);
-    split = wg / tiles_nk;
-    t2 = wg - split * tiles_nk;
-    chunk = m_chunk;
-  } else {
-    const int wg = xcd_remap(blockIdx.x - whole, gridDim.x - whole), tail = tiles_nk - whole;
-    split = wg / tail;
-    t2 = whole + wg - split * tail;
-    chunk = tail_chunk;
-  }
-  wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, tiles_k, chunk, diag, split, t2);
+    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag) {
+  const int wg = xcd_remap(blockIdx.x, gridDim.x), split = wg / tiles_nk;
+  wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, tiles_k, m_chunk, diag, split,
+                                            wg - split * tiles_nk);
+}
+
+// The 256 x 256 tiles (tiles_k of them side by side) from `first` on, four workgroups of 128 x 128 each, two on a CU.  An element is
+// still one sum over all rows in the same order, added to the gradient once: the bits of a whole tile, whatever the gradient holds.
+// (Two halves of the rows are quicker, 1424 us below, but their two contributions to a gradient that is not zero come in either order.)
+__global__ __launch_bounds__(256, 2) void wgrad_quarters_kernel(
+    const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
+    float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
+    int M, int N, int K, int tiles_k, int first, int m_chunk, int diag) {
+  const int wg = xcd_remap(blockIdx.x, gridDim.x), t = first + (wg >> 2), tile = t / tiles_k;
+  const int tile_n = 2 * tile + ((wg >> 1) & 1), tile_k = 2 * (t - tile * tiles_k) + (wg & 1);
+  if (tile_n * 128 >= N || tile_k * 128 >= K) return;
+  wgrad_tn_bf16_body<128, 128, 64, 2, true>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, 2 * tiles_k, m_chunk, diag, 0,
+                                            tile_n * 2 * tiles_k + tile_k);
 }
 
 // Several weight gradients in ONE launch (vy_linear_wgrad_grouped, vy_linear_wgrad_batch): the four GEMMs of a transformer layer
@@ -1104,27 +1107,23 @@ extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int6
   if (splits < 1) splits = 1;
   int64_t m_chunk = vy_cdiv(vy_cdiv(M, splits), 64) * 64;
   splits = vy_cdiv(M, m_chunk);
-  // One workgroup per CU: where the tiles end in a round of at most half the chip, that round's tiles are cut in two along M (two
-  // contributions to a zeroed gradient: their order does not show).  50265 x 768 over 16384 rows, 591 tiles: 1389 -> 1260 us; 8192 rows 733 -> 654.
-  int64_t whole = tiles * splits, tail_chunk = m_chunk, grid = whole;
-  if (big && splits == 1 && tiles > 256 && tiles % 256 > 0 && tiles % 256 <= 128) {
-    whole = tiles / 256 * 256;
-    tail_chunk = vy_cdiv(vy_cdiv(M, 2), 64) * 64;
-    grid = whole + (tiles - whole) * vy_cdiv(M, tail_chunk);
-  }
   static const int ns = [] { const char* e = getenv("VY_WGRAD_STAGES"); return e ? atoi(e) : 2; }();
-#define WG_GO(BN_, BK_, MS_, NS_)                                                                          \
-  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_>), dim3((unsigned)grid), dim3(BN_ * 2), 0, \
-                     st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
-                     (int)K, tiles_k, tiles, (int)m_chunk, diag, (int)whole, (int)tail_chunk)
-#define WG_GO16(BN_, BK_, MS_, NS_)                                                                        \
-  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_, true>), dim3((unsigned)grid), dim3(BN_ * 2), 0, \
-                     st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
-                     (int)K, tiles_k, tiles, (int)m_chunk, diag, (int)whole, (int)tail_chunk)
   // 16 x 16 x 32 MFMAs: 3 % faster on the 256 x 256 tiles (vocabulary projection 1.62 -> 1.57 ms, +0.25 % on the training
   // step), 2-8 % SLOWER on the 128 x 128 tiles (these kernels are bound by the transposing LDS reads and the atomic
   // epilogue, not by the matrix pipe): 1 = the wide tiles only (default), 2 = everywhere, 0 = off
   static const int w16 = [] { const char* e = getenv("VY_WGRAD_M16"); return e ? atoi(e) : 1; }();
+  // One workgroup per CU: where the tiles end in a round of at most half the chip, that round's tiles go out in quarters behind
+  // the others.  50265 x 768 over 16384 rows, 591 tiles: 1543 -> 1478 us; 8192 rows 742 -> 700; 22016 x 768 over 8192 rows, 258 tiles:
+  // 461 -> 380; 11008 x 2048, 344 tiles: 482 -> 411.  (Halves of 256 x 128, one on a CU: 1490, 712, 410, 427.)
+  const int whole = var == 8 && w16 && splits == 1 && tiles > 256 && tiles % 256 > 0 && tiles % 256 <= 128 ? tiles / 256 * 256 : tiles;
+#define WG_GO(BN_, BK_, MS_, NS_)                                                                          \
+  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_>), dim3((unsigned)(whole * splits)), dim3(BN_ * 2), 0, \
+                     st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
+                     (int)K, tiles_k, whole, (int)m_chunk, diag)
+#define WG_GO16(BN_, BK_, MS_, NS_)                                                                        \
+  hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_, true>), dim3((unsigned)(whole * splits)), dim3(BN_ * 2), 0, \
+                     st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
+                     (int)K, tiles_k, whole, (int)m_chunk, diag)
   if (var == 1) { if (ns == 3) WG_GO(256, 128, 64, 3); else WG_GO(256, 128, 64, 2); }
   else if (var == 2) WG_GO(128, 256, 32, 2);
   else if (var == 4) WG_GO(128, 256, 32, 3);
@@ -1135,6 +1134,9 @@ extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int6
   else { if (ns == 3) WG_GO(128, 128, 64, 3); else if (w16 >= 2) WG_GO16(128, 128, 64, 2); else WG_GO(128, 128, 64, 2); }
 #undef WG_GO
 #undef WG_GO16
+  if (whole < tiles)
+    hipLaunchKernelGGL(wgrad_quarters_kernel, dim3((unsigned)(4 * (tiles - whole))), dim3(256), 0, st, (const bf16*)dy, lddy,
+                       (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, (int)K, tiles_k, whole, (int)m_chunk, diag);
   VY_CHECK_LAUNCH(who);
   return VY_OK;
 }
