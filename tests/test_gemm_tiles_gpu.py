@@ -80,8 +80,7 @@ def test_rotary_heads_on_small_tiles(B, L, h, hk):
 
 
 def test_workspaces_that_come_and_go():
-    """Another thread registers the stream's workspace and takes it back (the memory itself stays) while products are launched: each is
-    cut into slices or is not, and has the bits of one of the two."""
+    """Another thread registers the stream's workspace and takes it back (the memory itself stays) while products are launched."""
     import threading
     from vyomai_amd import ops
     from vyomai_amd._lib import call
@@ -99,18 +98,57 @@ def test_workspaces_that_come_and_go():
             call("vy_workspace_set", st, buf.data_ptr(), size)
     other = threading.Thread(target=turn)
     try:
-        call("vy_workspace_set", st, None, 0)
-        whole = ops.linear(x, w)
         call("vy_workspace_set", st, buf.data_ptr(), size)
-        sliced = ops.linear(x, w)
-        assert not torch.equal(whole, sliced)
+        want = ops.linear(x, w)
         other.start()
         got = [ops.linear(x, w) for _ in range(400)]
         done.set()
         other.join()
-        assert all(torch.equal(y, whole) or torch.equal(y, sliced) for y in got)
+        assert all(torch.equal(y, want) for y in got)
     finally:
         done.set()
         ops._mid_ws = register
         call("vy_workspace_set", st, None, 0)
         ops._WS.pop((torch.cuda.current_device(), st), None)
+
+
+@pytest.mark.parametrize("M,N,K,act", [(5000, 768, 768, 1), (4097, 256, 4104, 0), (8192, 512, 2048, 0), (12001, 128, 1536, 0),
+                                       (4096, 768, 3072, 0), (2112, 768, 768, 1), (264, 1024, 8192, 0), (200, 1152, 4304, 1),
+                                       (33, 64, 1000, 0), (512, 768, 3080, 0)])
+def test_bits_before_and_behind_a_smaller_product(M, N, K, act):
+    """The first product on a stream, the same one behind a product for which the stream gets a workspace, the same one on a stream
+    with a workspace that is too small: equal bits, as plain, gated and rotary products."""
+    from vyomai_amd import ops
+    from vyomai_amd._lib import call
+    x, w = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=1 / math.sqrt(K))
+    heads = N // 192
+
+    def products():
+        out = [ops.linear(x, w, act=act), ops.gated_linear(x, w, 3)]
+        if heads:
+            qkv = [torch.empty(1, heads, M, 64, dtype=BF, device=DEV) for _ in range(3)]
+            ops.qkv_rope(x.view(1, M, K), w[:192 * heads].contiguous(), None, heads, heads, 64, None, None, 0, *qkv)
+            out += qkv
+        return out
+    torch.cuda.synchronize()
+    stream = torch.cuda.Stream()
+    with torch.cuda.stream(stream):
+        st, key = stream.cuda_stream, (torch.cuda.current_device(), stream.cuda_stream)
+        register, small = ops._mid_ws, torch.empty(1 << 16, dtype=torch.uint8, device=DEV)
+        try:
+            ops._mid_ws = lambda rows: None
+            call("vy_workspace_set", st, None, 0)     # (torch hands streams out again)
+            ops._WS.pop(key, None)
+            first = products()
+            call("vy_workspace_set", st, small.data_ptr(), 1 << 16)
+            narrow = products()
+            ops._mid_ws = register
+            ops.linear(rnd(64, 512, seed=3), rnd(64, 512, seed=4))
+            assert key in ops._WS
+            behind = products()
+            stream.synchronize()
+        finally:
+            ops._mid_ws = register
+            call("vy_workspace_set", st, None, 0)
+            ops._WS.pop(key, None)
+    assert all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(first, behind, narrow))

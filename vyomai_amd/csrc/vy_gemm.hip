@@ -1586,7 +1586,8 @@ __global__ __launch_bounds__(64) void gemm_splitk_finish_kernel(
 }
 
 // Workspaces for the split-K launches, registered per stream by the caller (the library never allocates device memory):
-// vy_workspace_set(stream, ptr, bytes).  Launches on a stream without one simply do not split.
+// vy_workspace_set(stream, ptr, bytes).  Launches on a stream without one take 64 x 64 tiles, which add
+// the slices up in registers.
 struct WsEntry { hipStream_t st; void* p; int64_t bytes; };
 WsEntry g_ws[16];
 int g_ws_n = 0;
@@ -1616,10 +1617,12 @@ struct Tiling { TileKind kind; int slices; };
 
 // Slices of K whose sums a product adds up, in order: what fills the chip where every slice is a workgroup of its own (as many as
 // `target` workgroups in all, a power of two -- one per group of XCDs, splitk_block_of -- of at least two stages, none empty).  The
-// kernels below add up the same sums in the same order, so a result does not hang on which of them the shape takes (in training the
-// rounding of one product decides the noise of every gradient behind it).
-inline int sum_slices(int64_t M, int64_t N, int64_t K, int64_t ws_bytes) {
-  if (g_chains != 1 || (M > 1024 && vy_cdiv(M, 256) * vy_cdiv(N, 192) >= 160)) return 1;
+// kernels below add up the same sums in the same order, so a result hangs neither on which of them the shape takes nor on a workspace
+// that the stream has or has not (in training the rounding of one product decides the noise of every gradient behind it).  Above 4096
+// rows, where the host layer registers none, K is not cut, and nothing is lost (two slices -> whole: 4200 x 1024, K = 6144, 92 -> 85 us;
+// 8192 x 512, K = 2048, 36 -> 29; 5000 x 768, K = 3072, 39.5 -> 39.8; the others of 15 shapes level or faster).
+inline int sum_slices(int64_t M, int64_t N, int64_t K) {
+  if (g_chains != 1 || M > 4096 || (M > 1024 && vy_cdiv(M, 256) * vy_cdiv(N, 192) >= 160)) return 1;
   const int bm = M > 128 && M <= 256 ? 256 : M > 256 && M <= 320 ? 320 : 128, target = bm == 128 ? 448 : 256;
   const int64_t tiles = vy_cdiv(M, bm) * vy_cdiv(N, 128);
   const int KT = (int)vy_cdiv(K, BK);
@@ -1631,12 +1634,11 @@ inline int sum_slices(int64_t M, int64_t N, int64_t K, int64_t ws_bytes) {
   int p2 = 2;
   while (p2 * 2 <= S) p2 *= 2;
   const int per = (KT + p2 - 1) / p2;
-  S = (KT + per - 1) / per;
-  return S * tiles * bm * 128 * 4 <= ws_bytes ? S : 1;
+  return (KT + per - 1) / per;
 }
 
 inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes) {
-  const int KT = (int)vy_cdiv(K, BK), S = sum_slices(M, N, K, ws_bytes);
+  const int KT = (int)vy_cdiv(K, BK), S = sum_slices(M, N, K);
   Tiling best{T_256x256, S};
   double least = 1e30;
   auto offer = [&](TileKind kind, double us) {
@@ -1664,13 +1666,14 @@ inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_
   const TileKind k = M > 256 && M <= 320 ? T_320x128_SPLIT : M > 128 && M <= 256 ? T_256x128_SPLIT : T_128x128_SPLIT;
   const int64_t tiles = tiles_of(k);
   const double bytes = 4.0 * S * tiles * TILE_M[k] * TILE_N[k];
+  if (bytes > (double)ws_bytes) return best;
   const int per = (KT + S - 1) / S;
   const double stage = k == T_128x128_SPLIT ? (tiles * S > chip ? 1.0 : 0.72) : 1.2 * TILE_M[k] / 256;
   offer(k, 7.5 + (double)vy_cdiv(tiles * S, (int64_t)chip * (k == T_128x128_SPLIT ? 2 : 1)) * per * stage + 2 * bytes / 8e6);
   return best;
 }
 
-// BM x BN tiles with K cut into S slices, whose partial sums the second launch adds up in the workspace's order (ws: sum_slices has
+// BM x BN tiles with K cut into S slices, whose partial sums the second launch adds up in the workspace's order (ws: pick_tiling has
 // seen that they fit)
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD>
 void launch_split(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K, int S,
@@ -2709,7 +2712,7 @@ extern "C" int vy_workspace_set(void* stream, void* ws, int64_t bytes) {
       return VY_OK;
     }
   if (!ws || !bytes) return VY_OK;
-  if (g_ws_n == 16) {   // full: the oldest entry goes (its stream's later launches run unsplit -- speed only)
+  if (g_ws_n == 16) {   // full: the oldest entry goes (its stream's later launches take other tiles -- speed only)
     for (int i = 1; i < 16; ++i) g_ws[i - 1] = g_ws[i];
     --g_ws_n;
   }

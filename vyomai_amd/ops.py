@@ -130,8 +130,8 @@ _WS_BYTES = 64 << 20
 
 
 def _mid_ws(rows: int) -> None:
-    """Mid-size GEMMs (32 < rows <= 4096) split K over workgroups and need scratch for their fp32 partial tiles
-    (vy_workspace_set: one buffer per stream, registered once; the library never allocates device memory)."""
+    """Mid-size GEMMs (32 < rows <= 4096) split K over workgroups where the stream has scratch for their fp32 partial tiles
+    (vy_workspace_set: one buffer per stream, registered once; the library never allocates device memory).  Speed only."""
     if rows <= 32 or rows > 4096 or _Lanes.active:
         return
     key = torch._C._cuda_getDevice(), _raw_stream()
