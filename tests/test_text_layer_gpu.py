@@ -111,3 +111,26 @@ def test_what_the_native_layer_does_not_take():
         assert layer_forward(l.attention, l.feed_forward, x, None, None) is None                          # another forward
     l.attention.__class__ = Mine.__mro__[1]
     assert layer_forward(l.attention, l.feed_forward, x, None, None) is None                              # gradients wanted
+
+
+@pytest.mark.parametrize("which", ["attention", "feed_forward"])
+def test_a_forward_set_on_a_module_is_called(which):
+    """As profilers and quantisers wrap modules: layer.feed_forward.forward = wrapped."""
+    import vyomai_amd as V
+    torch.manual_seed(6)
+    m = V.EncoderModel(config(), "rope", None).to(DEV, BF).eval()
+    ids = torch.randint(3, 97, (2, 9), device=DEV)
+    keep = torch.ones_like(ids)
+    with torch.no_grad():
+        want = m(ids, keep).logits
+        module, calls = getattr(m.all_layer[1], which), []
+        inner = module.forward
+
+        def wrapped(*a, **k):
+            calls.append(1)
+            return inner(*a, **k) * 2
+        module.forward = wrapped
+        twice = m(ids, keep).logits
+        assert len(calls) == 1 and not torch.equal(twice, want)
+        del module.forward
+        assert torch.equal(m(ids, keep).logits, want) and len(calls) == 1

@@ -140,12 +140,12 @@ _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules
 def layer_forward(att, ff, x, mask, freqs, cache=None, cache_index: Optional[int] = None, start_pos: int = 0):
     """ff(att(x), x) of one post-LN layer without gradients as ONE native call (vy_text_layer_fwd), the same launches in the same order:
     a layer of a few short texts is 50 us of GPU work, and four times that in Python.  None: the modules are to be called one by one --
-    a module of another class or with a hook, active dropout, a dense mask, rows that are not contiguous."""
+    a module of another class, with a hook or with a forward of its own, active dropout, a dense mask, rows that are not contiguous."""
     if type(ff) is not FeedForward or "_whole_layer" not in type(att).__dict__ or type(att.out) is not AttentionSelfOutput \
             or not (mask is None or isinstance(mask, AttnMask)):
         return None
     aso = att.out
-    if any(_GLOBAL_HOOKS) or any(m._forward_hooks or m._forward_pre_hooks for m in (att, aso, ff)):
+    if any(_GLOBAL_HOOKS) or any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (att, aso, ff)):
         return None
     if not x.is_cuda or x.dim() != 3 or not x.is_contiguous() or ops._Lanes.active or torch.is_grad_enabled() or type(x) is not torch.Tensor:
         return None
