@@ -134,3 +134,22 @@ def test_a_forward_set_on_a_module_is_called(which):
         assert len(calls) == 1 and not torch.equal(twice, want)
         del module.forward
         assert torch.equal(m(ids, keep).logits, want) and len(calls) == 1
+
+
+def test_an_attention_of_the_users_own():
+    """A layer calls whatever module stands in its place, without asking it for a layer number."""
+    import vyomai_amd as V
+    torch.manual_seed(8)
+    cfg = config()
+    l = V.DecoderModel(cfg, "rope", None).to(DEV, BF).eval().all_layer[0]
+
+    class Halves(torch.nn.Module):
+        def forward(self, hidden_state, attention_mask, freqs=None, use_cache=False, kv_cache=None, start_pos=0):
+            return hidden_state / 2, kv_cache
+    l.attention = Halves()
+    x = torch.randn(2, 8, 128, device=DEV, generator=torch.Generator(device=DEV).manual_seed(8)).to(BF)
+    cache = V.DynamicCacheOne(cfg)
+    with torch.no_grad():
+        for kw in ({}, dict(use_cache=True, kv_cache=cache, start_pos=3)):
+            y, kept = l(x, None, None, **kw)
+            assert torch.equal(y, l.feed_forward(x / 2, x)) and kept is kw.get("kv_cache")

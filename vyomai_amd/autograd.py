@@ -137,7 +137,7 @@ def self_attention_block(mod, x, attention_mask, freqs, cache, cache_index, star
 _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks)
 
 
-def layer_forward(att, ff, x, mask, freqs, cache=None, cache_index: Optional[int] = None, start_pos: int = 0):
+def layer_forward(att, ff, x, mask, freqs, cache=None, start_pos: int = 0):
     """ff(att(x), x) of one post-LN layer without gradients as ONE native call (vy_text_layer_fwd), the same launches in the same order:
     a layer of a few short texts is 50 us of GPU work, and four times that in Python.  None: the modules are to be called one by one --
     a module of another class, with a hook or with a forward of its own, active dropout, a dense mask, rows that are not contiguous."""
@@ -171,9 +171,8 @@ def layer_forward(att, ff, x, mask, freqs, cache=None, cache_index: Optional[int
         k_new, v_new = kv[0], kv[1]
         k, v = k_new, v_new
     else:
-        k_new, v_new = cache.reserve(B, hk, L, dh, start_pos, dt, dev) if cache_index is None else \
-            cache.reserve(cache_index, B, hk, L, dh, start_pos, dt, dev)
-        k, v = cache.commit() if cache_index is None else cache.commit(cache_index)
+        k_new, v_new = cache.reserve(att.layer_idx, B, hk, L, dh, start_pos, dt, dev)
+        k, v = cache.commit(att.layer_idx)
     assert k_new.stride(3) == 1 and v_new.stride(3) == 1
     S = k.shape[2]
     m = _mask_args(mask, B, L, S, dev)

@@ -86,7 +86,7 @@ class DecoderLayer(nn.Module):
                 kv_cache=None, start_pos: Optional[int] = 0):
         if not torch.is_grad_enabled() and (kv_cache is not None or not use_cache):
             y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs,
-                              kv_cache if use_cache else None, self.attention.layer_idx, start_pos)
+                              kv_cache if use_cache else None, start_pos)
             if y is not None:
                 return y, kv_cache
         _defer(hidden_state)  # training: its residual-path gradients are added in the QKV dgrad epilogue
