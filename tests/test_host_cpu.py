@@ -251,6 +251,41 @@ def test_deferred_weight_gradient_bookkeeping():
     assert seen == [p]
 
 
+def test_exchanged_weight_gradients_go_out_layer_by_layer(monkeypatch):
+    """A reducer that exchanges its buckets gets a layer's gradients as soon as the layer's backward is through; without an exchange a
+    launch fills the chip."""
+    import torch.distributed as dist
+    from vyomai_amd import autograd_train as AT
+    from vyomai_amd.training import BucketReducer, FlatArena
+    shapes = ((768, 3072), (3072, 768), (768, 768), (2304, 768))
+
+    def launches(exchange):
+        m = torch.nn.ModuleList(torch.nn.Linear(8, 8) for _ in range(5))
+        if exchange:
+            monkeypatch.setenv("VY_DDP_FORCE_COLLECTIVES", "1")
+            dist.init_process_group("gloo", store=dist.HashStore(), rank=0, world_size=1)
+        try:
+            reducer = BucketReducer(FlatArena(m))
+        finally:
+            if exchange:
+                dist.destroy_process_group()
+        sizes, ready = [], []
+        monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", lambda items: sizes.append(len(items)))
+        group = AT._WgradGroup()
+        group.armed = True   # (no backward pass to flush it)
+        for p in reducer.arena.params:
+            p._vy_ready = ready.append
+        for layer in m:
+            for N, K in shapes:
+                group.add_tensors(None, None, torch.empty(N, K, device="meta"), None, [layer.weight] if (N, K) == shapes[-1] else [layer.bias])
+            if exchange:
+                assert not group.items and ready[-1] is layer.weight
+        group.flush()
+        return sizes
+    assert launches(True) == [4] * 5
+    assert launches(False) == [9, 9, 2]
+
+
 def test_bench_starts_its_own_ranks_and_never_misreports_n_gpus():
     """`python bench.py --gpus N` without a launcher used to run ONE rank and print n_gpus: 1.  Now it starts
     the N ranks itself (a child torch.distributed.run), and refuses a world size that differs from --gpus."""

@@ -134,11 +134,14 @@ class _WgradGroup:
     autograd reaches them: the projections of a layer are small wgrad problems (9-36 tiles of 256 x 256),
     and one at a time each needs M-splits -- fp32 atomic traffic -- to fill the chip.  They are collected
     here and go out as ONE launch per chip of tiles, ~2 layers (ops.linear_wgrad_grouped); the parameters are reported ready
-    (DDP buckets, per-bucket AdamW) when that launch has been enqueued.  Whatever is still pending when
-    the backward pass ends is flushed by an autograd-engine callback."""
+    (per-bucket AdamW) when that launch has been enqueued, and its operands live until then (0.4 GB a layer at 16384 rows of
+    768).  Parameters whose gradients are exchanged between ranks (training.BucketReducer) go out layer by layer: their buckets
+    wait for the launch, and the exchange is what has to begin early.  Whatever is still pending when the backward pass ends is
+    flushed by an autograd-engine callback."""
 
     TILES = int(os.environ.get("VY_WGRAD_GROUP_TILES", "256"))   # most 256 x 256 output tiles of a launch: a CU each (a post-LN layer of 768: 108)
     MOST = 12                                                    # gradients of a launch
+    EXCHANGED, EXCHANGED_MOST = 100, 8                           # exchanged gradients: as many tiles or gradients end a launch
 
     def __init__(self):
         self.items, self.tiles, self.armed = [], 0, False
@@ -156,7 +159,8 @@ class _WgradGroup:
         """dw / db: the fp32 gradient tensors the launch accumulates into (views of the arena); members: the
         parameters to report ready once it has been enqueued (a packed projection has several)."""
         tiles = -(-dw.shape[0] // 256) * -(-dw.shape[1] // 256)
-        if self.tiles + tiles > self.TILES:
+        exchanged = any(getattr(p, "_vy_exchanged", False) for p in members)
+        if self.tiles + tiles > self.TILES and not exchanged:
             self.flush()
         self.items.append((dy, x, dw, db, members))
         # autograd's own post-accumulate hook fires for these parameters as soon as this backward function
@@ -167,7 +171,11 @@ class _WgradGroup:
         if not self.armed:
             torch.autograd.Variable._execution_engine.queue_callback(self._end_of_backward)
             self.armed = True
-        if self.tiles >= self.TILES or len(self.items) == self.MOST:
+        if exchanged:
+            full = self.tiles >= min(self.TILES, self.EXCHANGED) or len(self.items) >= self.EXCHANGED_MOST
+        else:
+            full = self.tiles >= self.TILES or len(self.items) >= self.MOST
+        if full:
             self.flush()
 
     def flush(self) -> None:

@@ -252,6 +252,7 @@ class BucketReducer:
         # all-reduce (work, None when world == 1) has been enqueued -- the trainer steps the bucket
         for p in arena.params:
             p._vy_ready = self.mark_ready
+            p._vy_exchanged = self.world > 1 or self.force   # (autograd_train._WgradGroup: how long its gradient may wait)
             if p.requires_grad:
                 # gradients produced by torch autograd itself (embedding tables) arrive through the tape
                 p.register_post_accumulate_grad_hook(self._hook)
