@@ -269,3 +269,23 @@ int few_go(int epi, int pro, const Args& a, int64_t K, hipStream_t st) {
 }
 
 }  // namespace vy_few
+
+// test aid, not part of include/vyom_hip.h: one product by itself on contiguous rows.  a, b: gamma and beta of LAYER (bf16), w_post and
+// w_pre of STREAM (fp32); y: QKV's queries [M][nq], k and v [M][nkv]
+extern "C" int vy_debug_few(int epi, int pro, const void* x, const void* a, const void* b, const float* s_in, float* s_out, void* h, int n,
+                            int rms, float eps, const void* w, const void* bias, int act, float act_arg, const void* residual, void* y,
+                            int64_t ldy, void* k, void* v, int nq, int nkv, const float* cos_tab, const float* sin_tab, int pos, int M,
+                            int N, int64_t K, void* stream) {
+  vy_few::Args f{};
+  f.x = (const bf16*)x; f.ldx = K;
+  if (pro == vy_few::LAYER) { f.ln_g = (const bf16*)a; f.ln_b = (const bf16*)b; }
+  else { f.w_post = (const float*)a; f.w_pre = (const float*)b; }
+  f.s_in = s_in; f.s_out = s_out; f.lds = K; f.n = n; f.rms = rms; f.eps = eps; f.h = (bf16*)h; f.ldh = K;
+  f.w = (const bf16*)w; f.N = N; f.M = M; f.bias = (const bf16*)bias; f.act = act; f.act_arg = act_arg;
+  f.residual = (const bf16*)residual; f.ldr = N; f.y = (bf16*)y; f.ldy = ldy;
+  if (epi == vy_few::QKV) {   // (one cache row a sequence: `pos` turns, the rows lie at 0)
+    f.q = (bf16*)y; f.k = (bf16*)k - (int64_t)pos * nkv; f.v = (bf16*)v - (int64_t)pos * nkv; f.c_sb = nkv; f.c_sh = 64; f.c_sl = nkv;
+    f.cos_tab = cos_tab; f.sin_tab = sin_tab; f.pos = pos; f.nq = nq; f.nkv = nkv;
+  }
+  return vy_few::few_go(epi, pro, f, K, (hipStream_t)stream);
+}
