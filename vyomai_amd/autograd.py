@@ -145,8 +145,11 @@ def layer_forward(att, ff, x, mask, freqs, cache=None, start_pos: int = 0):
             or not (mask is None or isinstance(mask, AttnMask)):
         return None
     aso = att.out
-    if any(_GLOBAL_HOOKS) or any(m._forward_hooks or m._forward_pre_hooks or "forward" in m.__dict__ for m in (att, aso, ff)):
+    if _GLOBAL_HOOKS[0] or _GLOBAL_HOOKS[1]:
         return None
+    for d in (att.__dict__, aso.__dict__, ff.__dict__):
+        if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
+            return None
     if not x.is_cuda or x.dim() != 3 or not x.is_contiguous() or ops._Lanes.active or torch.is_grad_enabled() or type(x) is not torch.Tensor:
         return None
     if (aso.training and aso.dropout.p > 0.0) or (ff.training and ff.dropout.p > 0.0):
