@@ -57,7 +57,8 @@ int vy_abi_version(void);
 /* Launch-sizing hint: the caller is about to run `n` independent launch chains side by side on `n` streams (the
  * training forward as two batch halves, vyomai_amd/ops.py `lanes`), so each launch should size its grid for 1/n of
  * the 256 CUs: a 128-tile launch of 256 x 192 tiles is then a full share, not a half-empty chip.  n = 1 (the default)
- * restores whole-chip sizing.  Process-global, read on the host when a launch is sized; results never depend on it. */
+ * restores whole-chip sizing.  Process-global, read on the host when a launch is sized; n > 1 also leaves K in one piece where a lone
+ * chain cuts it into slices (vy_workspace_set), so results may differ by the order of fp32 sums over K. */
 int vy_set_concurrent_chains(int n);
 
 /* Scratch for the launches on `stream` (the library never allocates device memory): GEMMs of 33 to 4096 rows and fewer

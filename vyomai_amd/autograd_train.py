@@ -201,7 +201,9 @@ class _WgradGroup:
 
 _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
-_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # measured on configs[3] (2112 decoder rows): -6 %
+_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 116 us one by one,
+# 73 in a launch of their own, 46 of one with its neighbours'.  (So it pays below as well, 1665 rows 109 / 67 / 41 and 1030 rows 94 / 60 / 35:
+# the line dates from launches of one layer.)
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group
 _wgrad_group = _WgradGroup()
 
