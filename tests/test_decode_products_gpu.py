@@ -212,7 +212,7 @@ def test_rows_of_wide_products(M, N, K, act, extras):
 
 
 @pytest.mark.parametrize("M", [5, 16, 17, 32])
-@pytest.mark.parametrize("N,K,slices", [(512, 1024, 8), (520, 1400, 8), (1000, 6144, 8), (520, 1032, 0), (1024, 1096, 0), (1032, 4104, 4), (2048, 8200, 8),
+@pytest.mark.parametrize("N,K,slices", [(512, 1024, 8), (520, 1400, 8), (1000, 6144, 8), (520, 1032, 0), (1024, 1096, 0), (1032, 4104, 4), (2048, 8200, 8), (2001, 8200, 8),
                                         (2048, 1024, 4), (2056, 12288, 2), (4096, 1400, 2), (504, 1024, 0), (4104, 1024, 0),
                                         (1024, 1016, 0)])
 def test_rows_in_slices(M, N, K, slices):

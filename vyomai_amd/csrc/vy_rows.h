@@ -9,16 +9,14 @@
 namespace vy_rows {
 
 template <int NT, int MB, int NW = 4> constexpr int RED = (NW - 1) * NT * MB * 64;   // f32x4 of LDS that stream() needs
+template <int NT, int MB, int NW = 4> constexpr int DENSE_RED = NW * NT * MB * 64;   // and dense()
 template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3 ? 8 : 4;
 
-// acc[t][j] (in wave 0 only) = 16 rows ws[t] x 16 rows xs[j]; a lane's pointers are its row (lane & 15) + 8 (lane >> 4).
+// acc[t][j] = 16 rows ws[t] x 16 rows xs[j] over the wave's share of K; a lane's pointers are its row (lane & 15) + 8 (lane >> 4).
 // D: a lane owns row lane & 15 of X and rows 4 (lane >> 4) .. + 3 of W.
-// HALF: the last 16 weight rows are 8.
-template <int NT, int MB, bool ONCE = true, int NW = 4, bool HALF = false>
-__device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB],
-                                       f32x4* red) {
-  constexpr int U = STEPS<NT, MB>;
-  const int lane = threadIdx.x & 63, kq = lane >> 4;
+template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>>
+__device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB]) {
+  const int kq = (threadIdx.x & 63) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bf16x8 zero8 = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
 #pragma unroll
@@ -27,19 +25,30 @@ __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* 
     for (int j = 0; j < MB; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int k0 = 64 * wave; k0 < K; k0 += 32 * NW * U) {
     bf16x8 w[U][NT], x[U][MB];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int k = k0 + 64 * NW * (u >> 1) + 32 * (u & 1);
-      const bool in = k + 8 * kq < K;
+    auto request = [&](int u, int k) {
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
-        const bool row = in && (!HALF || t < NT - 1 || (lane & 15) < 8);
-        if constexpr (ONCE) w[u][t] = row ? __builtin_nontemporal_load(at) : zero8;
-        else w[u][t] = row ? *at : zero8;
+        if constexpr (ONCE) w[u][t] = __builtin_nontemporal_load(at);
+        else w[u][t] = *at;
       }
 #pragma unroll
-      for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
+      for (int j = 0; j < MB; ++j) x[u][j] = *reinterpret_cast<const bf16x8*>(xs[j] + k);
+    };
+    // (all of the pass inside K, the common case: loads behind conditions of their own come one branch after the other)
+    if (k0 + 64 * NW * ((U - 1) >> 1) + 64 <= K) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) request(u, k0 + 64 * NW * (u >> 1) + 32 * (u & 1));
+    } else {
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + 64 * NW * (u >> 1) + 32 * (u & 1);
+#pragma unroll
+        for (int t = 0; t < NT; ++t) w[u][t] = zero8;
+#pragma unroll
+        for (int j = 0; j < MB; ++j) x[u][j] = zero8;
+        if (k + 8 * kq < K) request(u, k);
+      }
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -48,6 +57,15 @@ __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* 
 #pragma unroll
         for (int j = 0; j < MB; ++j) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][t], x[u][j], acc[t][j], 0, 0, 0);
   }
+}
+
+// share() and, in wave 0, the waves' sums
+template <int NT, int MB, bool ONCE = true, int NW = 4>
+__device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB],
+                                       f32x4* red) {
+  const int lane = threadIdx.x & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  share<NT, MB, ONCE, NW>(ws, xs, K, acc);
   __syncthreads();   // (red may still be read from the pass before)
   if (wave)
 #pragma unroll
@@ -72,48 +90,77 @@ struct Dense {
   const bf16* x; int64_t ldx; int M;   // M <= 16 MB
   const bf16* w; int N, K;             // [N][K]
   void* y; int64_t ldy; int f32;       // f32: fp32 results
-  const bf16* bias; int act; float act_arg;   // of bf16 results: act(x W^T + bias), act none, VY_ACT_RELU2 or VY_ACT_SOFTCAP
+  const bf16* bias; float act_arg;     // of bf16 results: act(x W^T + bias)
 };
 
-__device__ __forceinline__ float finish(const Dense& a, float v, int n) {
-  if (a.bias) v += (float)a.bias[n];
-  if (a.act == VY_ACT_RELU2) v = vy_act_fwd<VY_ACT_RELU2>(v);
-  else if (a.act == VY_ACT_SOFTCAP) v = vy_act_fwd<VY_ACT_SOFTCAP>(v, a.act_arg);
-  return v;
-}
-
-// rows R tile .. + R - 1 of W against all of X, R = 16 NT (HALF: - 8)
-template <int MB, int NW = 4, int NT = 1, bool HALF = false>
+// rows R tile .. + R - 1 of W against all of X, R = 16 NT (HALF: - 8, the last eight lanes' rows twice).  What the waves add up goes through
+// LDS, and each wave finishes blocks of its own, biases requested ahead of the stream: finished by the first wave alone, element by
+// element with a wait for each bias and a switch over the activations, a workgroup ran through 3300 instructions behind its last
+// product, 3 of 8.6 us (32 rows, 6144 x 1024).
+template <int MB, int NW = 4, int NT = 1, bool HALF = false, int ACT = VY_ACT_NONE, int U = STEPS<NT, MB>>
 __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int K) {   // K: columns of x and w that count
-  constexpr int R = 16 * NT - (HALF ? 8 : 0);
+  constexpr int R = 16 * NT - (HALF ? 8 : 0), BLOCKS = NT * MB, MINE = (BLOCKS + NW - 1) / NW;
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bf16* ws[NT];
 #pragma unroll
-  for (int t = 0; t < NT; ++t) ws[t] = a.w + (int64_t)min(R * tile + 16 * t + r16, a.N - 1) * a.K + 8 * kq;
+  for (int t = 0; t < NT; ++t) {
+    const int r = HALF && t == NT - 1 ? r16 & 7 : r16;
+    ws[t] = a.w + (int64_t)min(R * tile + 16 * t + r, a.N - 1) * a.K + 8 * kq;
+  }
   const bf16* xs[MB];
 #pragma unroll
   for (int j = 0; j < MB; ++j) xs[j] = a.x + (int64_t)min(16 * j + r16, a.M - 1) * a.ldx + 8 * kq;
+  float bias[MINE][4];
+  if (a.bias) {   // (uniform)
+#pragma unroll
+    for (int b = 0; b < MINE; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) bias[b][r] = (float)a.bias[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
+  }
   f32x4 acc[NT][MB];
-  stream<NT, MB, true, NW, HALF>(ws, xs, K, acc, red);
-  if (threadIdx.x >= 64) return;
+  share<NT, MB, true, NW, U>(ws, xs, K, acc);
+  __syncthreads();   // (red may still be read from the pass before)
 #pragma unroll
-  for (int i = 0; i < NT * MB; ++i) {
-    const int m = 16 * (i % MB) + r16, n = R * tile + 16 * (i / MB) + 4 * kq;
-    if (m >= a.M || (HALF && i / MB == NT - 1 && kq >= 2)) continue;
-    const f32x4 v = acc[i / MB][i % MB];
+  for (int i = 0; i < BLOCKS; ++i) red[(wave * BLOCKS + i) * 64 + lane] = acc[i / MB][i % MB];
+  __syncthreads();
+#pragma unroll
+  for (int b = 0; b < MINE; ++b) {
+    const int i = wave + NW * b, m = 16 * (i % MB) + r16, n = R * tile + 16 * (i / MB) + 4 * kq;
+    if (i >= BLOCKS || m >= a.M || n >= a.N || (HALF && i / MB == NT - 1 && kq >= 2)) continue;
+    f32x4 v = red[i * 64 + lane];
+#pragma unroll
+    for (int s = 1; s < NW; ++s) {
+      const f32x4 p = red[(s * BLOCKS + i) * 64 + lane];
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[r] += p[r];
+    }
     if (a.f32) {
+      float* y = (float*)a.y + (int64_t)m * a.ldy + n;
+      if (n + 4 <= a.N && (uintptr_t)y % 16 == 0) {
+        *reinterpret_cast<f32x4*>(y) = v;
+      } else {
 #pragma unroll
-      for (int r = 0; r < 4; ++r)
-        if (n + r < a.N) ((float*)a.y)[(int64_t)m * a.ldy + n + r] = v[r];
-    } else if (n + 4 <= a.N) {
-      bf16x4 w4;
+        for (int r = 0; r < 4; ++r)
+          if (n + r < a.N) y[r] = v[r];
+      }
+      continue;
+    }
+    bf16x4 w4;
 #pragma unroll
-      for (int r = 0; r < 4; ++r) w4[r] = (bf16)finish(a, v[r], n + r);
-      *reinterpret_cast<bf16x4*>((bf16*)a.y + (int64_t)m * a.ldy + n) = w4;
+    for (int r = 0; r < 4; ++r) {
+      float z = v[r];
+      if (a.bias) z += bias[b][r];
+      if constexpr (ACT != VY_ACT_NONE) z = vy_act_fwd<ACT>(z, a.act_arg);
+      w4[r] = (bf16)z;
+    }
+    bf16* y = (bf16*)a.y + (int64_t)m * a.ldy + n;
+    if (n + 4 <= a.N) {
+      *reinterpret_cast<bf16x4*>(y) = w4;
     } else {
 #pragma unroll
       for (int r = 0; r < 4; ++r)
-        if (n + r < a.N) ((bf16*)a.y)[(int64_t)m * a.ldy + n + r] = (bf16)finish(a, v[r], n + r);
+        if (n + r < a.N) y[r] = w4[r];
     }
   }
 }
