@@ -72,7 +72,25 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
       else w[p] = *at;
     }
   };
+  // what the epilogue reads besides the product, one lane per (weight row, operand row), and none of it hangs on the product: requested
+  // behind the norm's operands (behind the norm, the position and then the rotary factors were two more trips to memory)
+  const int er = R == 1 || lane >= R * MR ? 0 : lane / MR, em = R == 1 ? lane : lane % MR;
+  float e_bias = 0.f, e_other = 0.f, e_res = 0.f, e_cos = 0.f, e_sin = 0.f;
+  int pos = 0;
+  auto request_rest = [&](int unit) {
+    if (lane >= R * MR || em >= a.M) return;
+    const int n = row_of(unit, er);
+    if (EPI != GATED && a.bias) e_bias = (float)a.bias[n];
+    if (EPI == STORE && a.residual) e_res = (float)a.residual[em * a.ldr + n];
+    if (EPI == QKV && a.bias) e_other = (float)a.bias[n ^ 32];   // (of the pair's other column)
+    if (EPI == QKV && a.cos_tab) {
+      e_cos = a.cos_tab[(int64_t)pos * 32 + (n & 31)];
+      e_sin = a.sin_tab[(int64_t)pos * 32 + (n & 31)];
+    }
+  };
+  if constexpr (EPI == QKV) pos = a.pos_dev ? *a.pos_dev : a.pos;
   if (u < units) request(u);
+  if (u < units && (PRO == PLAIN || wave >= a.M)) request_rest(u);
 
   if constexpr (PRO != PLAIN) {
     if (a.advance && blockIdx.x == 0)
@@ -89,6 +107,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
           g4[c] = *reinterpret_cast<const bf16x4*>(a.ln_g + col);
           b4[c] = *reinterpret_cast<const bf16x4*>(a.ln_b + col);
         }
+        if (u < units) request_rest(u);
 #pragma unroll
         for (int c = 0; c < KC; ++c)
 #pragma unroll
@@ -104,6 +123,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
           if (a.w_post) p4[c] = *reinterpret_cast<const f32x4*>(a.w_post + col);
           if (a.w_pre) g4[c] = *reinterpret_cast<const f32x4*>(a.w_pre + col);
         }
+        if (u < units) request_rest(u);
         if (a.x) {
           float mean = 0.f, rstd = 1.f, y[KC][4];
 #pragma unroll
@@ -145,23 +165,10 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   }
 
   for (; u < units; u += step) {
-    // what the epilogue reads besides the product: one lane per (weight row, operand row)
-    const int er = R == 1 ? 0 : lane / MR, em = R == 1 ? lane : lane % MR;
     const bool mine = lane < R * MR && em < a.M;
-    const int n = row_of(u, mine ? er : 0);
+    const int n = row_of(u, er);
     const bool real = mine && (EPI != STORE || u * R + er < a.N);
-    float bias = 0.f, res = 0.f;
-    if (mine && EPI != GATED && a.bias) bias = (float)a.bias[n];
-    if (EPI == STORE && mine && a.residual) res = (float)a.residual[em * a.ldr + n];
-    float cs = 0.f, sn = 0.f;
-    int pos = 0;
-    if constexpr (EPI == QKV) {
-      pos = a.pos_dev ? *a.pos_dev : a.pos;
-      if (a.cos_tab && mine) {
-        cs = a.cos_tab[(int64_t)pos * 32 + (n & 31)];
-        sn = a.sin_tab[(int64_t)pos * 32 + (n & 31)];
-      }
-    }
+    const float bias = e_bias, other_bias = e_other, res = e_res, cs = e_cos, sn = e_sin;
     float acc[R][MR];
 #pragma unroll
     for (int r = 0; r < R; ++r)
@@ -170,7 +177,10 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
     bf16x8 wv[P];
 #pragma unroll
     for (int p = 0; p < P; ++p) wv[p] = w[p];
-    if (u + step < units) request(u + step);
+    if (u + step < units) {
+      request(u + step);
+      request_rest(u + step);
+    }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
       const int c = 64 * p + lane;
@@ -210,12 +220,10 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
       const float g = vy_round_bf16(own), up = vy_round_bf16(other);   // (lanes of row 0: own is the gate's)
       if (real && er == 0) a.y[em * a.ldy + u] = (bf16)((a.act == VY_ACT_SILU ? vy_silu(g) : vy_gelu_tanh(g)) * up);
     } else {
-      // (the other column of the pair needs its own bias)
-      const float ob = a.bias && mine ? (float)a.bias[n ^ 32] : 0.f;
       float v = own + bias;
       if (a.cos_tab && n < a.nq + a.nkv) {
         const float c = vy_round_bf16(cs), s = vy_round_bf16(sn);
-        const float t = vy_round_bf16(vy_round_bf16(other + ob) * s), m0 = vy_round_bf16(vy_round_bf16(v) * c);
+        const float t = vy_round_bf16(vy_round_bf16(other + other_bias) * s), m0 = vy_round_bf16(vy_round_bf16(v) * c);
         v = er ? m0 + t : m0 - t;
       }
       if (real) {
