@@ -384,12 +384,12 @@ template <int BM, int BN, int WGM, int WGN, bool MF16> struct AccTile {
 // The second operand of a plain epilogue -- residual, or the pre-activation of a dgrad -- in the registers of the threads that will
 // combine it (16-byte chunks tid, tid + NT, ... of the tile), requested before the accumulators are staged: loaded in the loop over the
 // chunks, every iteration waits a full memory latency for it (22 k cycles per tile against 12 k without the operand).
-constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, bool GRAD) {
-  return EPI == 0 && (BM * BN == 256 * 192 || BM * BN == 64 * 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
+constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, int ACT, bool GRAD) {
+  return EPI == 0 && (GRAD || ACT == VY_ACT_NONE) && (BM * BN == 256 * 192 || BM * BN == 64 * 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
 }
-template <int BM, int BN, int NW, int EPI, bool GRAD>
+template <int BM, int BN, int NW, int EPI, int ACT, bool GRAD>
 struct EpiAhead {
-  static constexpr bool ON = epi_prefetches(BM, BN, NW, EPI, GRAD);
+  static constexpr bool ON = epi_prefetches(BM, BN, NW, EPI, ACT, GRAD);
   static constexpr int ITERS = ON ? BM * BN / 8 / (64 * NW) : 1;
   bf16x8 v[ITERS];
   bool on = false;
@@ -413,7 +413,7 @@ struct EpiAhead {
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD, int PASSES = 1, bool MF16 = false>
 __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN, MF16>::type& acc, char* smem,
                                               int m0, int n0, int M, int N, const EpiPlain<bf16>& ep,
-                                              const EpiQkv<bf16>& eq, const EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>& ahead = EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>{},
+                                              const EpiQkv<bf16>& eq, const EpiAhead<BM, BN, WGM * WGN, EPI, ACT, GRAD>& ahead = EpiAhead<BM, BN, WGM * WGN, EPI, ACT, GRAD>{},
                                               const unsigned* tab = nullptr) {
   constexpr bool TAB = MF16 && act_has_table(BM, BN, EPI, ACT, GRAD);
   static_assert(!MF16 || PASSES == 1, "the 16 x 16 accumulator layout is staged in one pass");
@@ -498,6 +498,27 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
       for (int e = 0; e < 4; ++e) bq[e] = (biasp && n + e < N) ? (float)biasp[n + e] : 0.f;
     }
   };
+  // (16 x 16 blocks, all columns there: the wave's biases requested together -- a quad at a time, each behind a condition, they were
+  // as many trips to L2 one after the other as the wave has column blocks)
+  constexpr int QUADS = MF16 ? BN / (16 * WGN) : 1;
+  const bool bias_all = MF16 && biasp && bias_vec && n0 + BN <= N;
+  bf16x4 bias4[QUADS];
+  if constexpr (MF16) {
+#pragma unroll
+    for (int i = 0; i < QUADS; ++i) bias4[i] = bf16x4{(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
+    if (bias_all) {
+#pragma unroll
+      for (int i = 0; i < QUADS; ++i) bias4[i] = *reinterpret_cast<const bf16x4*>(biasp + n0 + wn * 16 * QUADS + 16 * i + 4 * (lane >> 4));
+    } else if (biasp) {
+#pragma unroll
+      for (int i = 0; i < QUADS; ++i)
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+          const int n = n0 + wn * 16 * QUADS + 16 * i + 4 * (lane >> 4) + e;
+          bias4[i][e] = biasp[n < N ? n : N - 1];
+        }
+    }
+  }
   // phase 1 of a pass: every quad of the wave's sub-tile that lies in the pass's row band, + bias, -> LDS
   auto stage_all = [&](int pass) {
     if constexpr (!MF16) {
@@ -522,13 +543,11 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
       const int r16 = lane & 15, kq = lane >> 4;
 #pragma unroll
       for (int i = 0; i < TN16; ++i) {
-        float bq[4];
-        bias_quad(n0 + wn * 16 * TN16 + 16 * i + 4 * kq, bq);
 #pragma unroll
         for (int j = 0; j < TM16; ++j) {
           float v[4];
 #pragma unroll
-          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + bq[e];
+          for (int e = 0; e < 4; ++e) v[e] = acc[i][j][e] + (float)bias4[i][e];
           stage_quad(wm * 16 * TM16 + 16 * j + r16, wn * 16 * TN16 + 16 * i + 4 * kq, v);
         }
       }
@@ -543,14 +562,15 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
     // one 16-byte chunk of the staged band.  pf: its second operand is p8 (EpiAhead)
     const bool pf_is_gradpre = GRAD && ep.gradpre != nullptr;
     const bool by_table = TAB && ep.vec_ok && !ep.residual && !ep.drop.thr;
-    auto do_chunk = [&](bf16* __restrict__ dst, bool dual, int pass, int c, bool pf, const bf16x8& p8) {
+    // whole: the tile lies inside the output and chunks are vectors
+    auto do_chunk = [&](auto whole_c, bf16* __restrict__ dst, bool dual, int pass, int c, const bf16x8& sv, bool pf, const bf16x8& p8) {
+        constexpr bool whole = decltype(whole_c)::value;
         const int row = c / CPR, cc = c - row * CPR;
         const int64_t m = m0 + pass * RP + row;
         const int n = n0 + cc * 8;
-        if (m >= M || n >= N) return;
-        const bf16x8 sv = *reinterpret_cast<const bf16x8*>(et + row * EROW + cc * 16);
+        if (!whole && (m >= M || n >= N)) return;
         if constexpr (TAB) {
-          if (by_table && n + 8 <= N) {
+          if (by_table && (whole || n + 8 <= N)) {
             const u32x4 u = __builtin_bit_cast(u32x4, sv);
             unsigned at[8], far = 0;
 #pragma unroll
@@ -579,7 +599,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = (float)sv[e];
         if (dual && !ep.pre_deriv) {
-          if (ep.vec_ok && n + 8 <= N) {
+          if (whole || (ep.vec_ok && n + 8 <= N)) {
             *reinterpret_cast<bf16x8*>(ep.pre + m * ep.ldy + n) = sv;
           } else {
             for (int e = 0; e < 8 && n + e < N; ++e) ep.pre[m * ep.ldy + n + e] = sv[e];
@@ -602,7 +622,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
                 v[e] = vy_act_fwd_fast<ACT>(v[e], ep.act_arg);
               }
             }
-            if (ep.vec_ok && n + 8 <= N) {
+            if (whole || (ep.vec_ok && n + 8 <= N)) {
               // read again only by the backward pass, milliseconds later: streamed, so that it does not take the place of
               // the activation written beside it (FFN2's operand) in the Infinity Cache
               __builtin_nontemporal_store(d8, reinterpret_cast<bf16x8*>(ep.pre + m * ep.ldy + n));
@@ -622,7 +642,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
             for (int e = 0; e < 8; ++e) v[e] = vy_drop_keep(ep.drop, lots, e) ? v[e] * ep.drop.scale : 0.f;
           }
         }
-        if (ep.vec_ok && n + 8 <= N) {
+        if (whole || (ep.vec_ok && n + 8 <= N)) {
           if constexpr (GRAD) {
             if (ep.gradpre) {
               const bf16x8 g = pf ? p8 : *reinterpret_cast<const bf16x8*>(ep.gradpre + m * ep.ldg + n);
@@ -662,16 +682,36 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
           }
         }
     };
+    // Tiles inside the output go out without conditions, several chunks out of LDS at a time.  With the biases requested together:
+    // 30500 x 768, K = 3072, 130.7 -> 128.0 us; 30500 x 3072, K = 768, GELU 206 -> 199; 16384 x 2304, K = 768, 65.4 -> 63.6.
+    const bool inside = ep.vec_ok && m0 + BM <= M && n0 + BN <= N;   // (workgroup-uniform)
+    auto staged = [&](int c) { const int row = c / CPR; return *reinterpret_cast<const bf16x8*>(et + row * EROW + (c - row * CPR) * 16); };
     auto flush_plain = [&](bf16* __restrict__ dst, bool dual, int pass) {
-      if constexpr (PASSES == 1 && EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>::ON) {
+      constexpr int ITERS = RP * CPR / NT, G = ITERS % 4 == 0 ? 4 : ITERS % 3 == 0 ? 3 : ITERS % 2 == 0 ? 2 : 1;
+      const std::integral_constant<bool, true> whole{};
+      const std::integral_constant<bool, false> ragged{};
+      const bf16x8 none{};
+      if constexpr (PASSES == 1 && EpiAhead<BM, BN, WGM * WGN, EPI, ACT, GRAD>::ON) {
         if (ahead.on) {
 #pragma unroll
-          for (int it = 0; it < (RP * CPR) / NT; ++it) do_chunk(dst, dual, pass, tid + it * NT, true, ahead.v[it]);
+          for (int it = 0; it < ITERS; ++it) do_chunk(whole, dst, dual, pass, tid + it * NT, staged(tid + it * NT), true, ahead.v[it]);
           return;
         }
       }
-      const bf16x8 none{};
-      for (int c = tid; c < RP * CPR; c += NT) do_chunk(dst, dual, pass, c, false, none);
+      if constexpr (ITERS * NT == RP * CPR) {
+        if (inside) {
+#pragma unroll 1
+          for (int it = 0; it < ITERS; it += G) {
+            bf16x8 sv[G];
+#pragma unroll
+            for (int g = 0; g < G; ++g) sv[g] = staged(tid + (it + g) * NT);
+#pragma unroll
+            for (int g = 0; g < G; ++g) do_chunk(whole, dst, dual, pass, tid + (it + g) * NT, sv[g], false, none);
+          }
+          return;
+        }
+      }
+      for (int c = tid; c < RP * CPR; c += NT) do_chunk(ragged, dst, dual, pass, c, staged(c), false, none);
     };
     const bool dual = !GRAD && ep.pre != nullptr;   // (the GRAD path never sets ep.pre)
 #pragma unroll 1
@@ -741,7 +781,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
       const int n = n0 + cc * 8;
       if (m >= M || n >= N) continue;
       const unsigned t = l0 + (unsigned)(pass * RP + row);
-      const unsigned tq = t / Lu;
+      const unsigned tq = Lu >= (unsigned)BM ? (t >= Lu ? 1u : 0u) : t / Lu;   // (l0 < Lu)
       const int64_t b = b0 + tq, l = t - tq * Lu;
       bf16x8 sv = *reinterpret_cast<const bf16x8*>(et + row * EROW + cc * 16);
       if (eq.rope && n < eq.nq + eq.nkv) {
@@ -1096,7 +1136,7 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
     xbuf = xbuf == 2 ? 0 : xbuf + 1;
     if (kt + 1 < KT) read_frags(wa[0] + (WT - wo), xa[0] + xbuf * XT, wf[0], xf[0]);
   }
-  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
+  EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
   gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
 }
@@ -1227,7 +1267,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     asm volatile("" ::: "memory");
     if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
   }
-  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
+  EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
   gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
 }
@@ -1383,7 +1423,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     }
     __syncthreads();
   }
-  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
+  EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
   gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead);
 }
