@@ -361,11 +361,19 @@ __device__ __forceinline__ void fill_act_table(unsigned* tab, bool deriv) {
     else tab[i] = __builtin_bit_cast(unsigned, vy_act_fwd<ACT>(x));
   }
 }
-// entry of a bf16 (its bits in the low half of u); far: grows beyond ACT_TAB_HALF where there is none
-__device__ __forceinline__ unsigned act_entry(unsigned u, unsigned& far) {
-  const unsigned k = (u & 0x7fffu) - ACT_TAB_LOW;
-  far = k > far ? k : far;
-  return k + ((u >> 15) & 1) * ACT_TAB_HALF;
+// byte offsets of the entries of two bf16 (u), in 16-bit halves up to the last step; far: grows beyond ACT_TAB_HALF where there is none
+typedef unsigned short u16x2 __attribute__((ext_vector_type(2)));
+__device__ __forceinline__ void act_entries(unsigned u, u16x2& far, unsigned& lo, unsigned& hi) {
+  const u16x2 x = __builtin_bit_cast(u16x2, u), low = (u16x2)((unsigned short)ACT_TAB_LOW), half = (u16x2)((unsigned short)ACT_TAB_HALF);
+  const u16x2 k = (x & (u16x2)((unsigned short)0x7fff)) - low;
+  far = __builtin_elementwise_max(far, k);
+  const unsigned at = __builtin_bit_cast(unsigned, (u16x2)((k + (x >> (u16x2)((unsigned short)15)) * half) << (u16x2)((unsigned short)2)));
+  lo = at & 0xffffu;
+  hi = at >> 16;
+}
+__device__ __forceinline__ bool act_far(u16x2 far) { return far[0] >= ACT_TAB_HALF || far[1] >= ACT_TAB_HALF; }
+__device__ __forceinline__ unsigned act_at(const unsigned* tab, unsigned offset) {
+  return *reinterpret_cast<const unsigned*>(reinterpret_cast<const char*>(tab) + offset);
 }
 
 // ---- shared epilogue of the bf16 kernels ------------------------------------------------------
@@ -455,13 +463,17 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
         float f[4];
         bool known = false;
         if constexpr (TAB) {
-          unsigned at[4], far = 0;
+          unsigned at[4];
+          u16x2 far = {0, 0};
 #pragma unroll
-          for (int e = 0; e < 4; ++e) at[e] = act_entry(__builtin_bit_cast(unsigned, vy_round_bf16(acc[i][j][e])) >> 16, far);
-          known = !__any(far >= ACT_TAB_HALF);
+          for (int e = 0; e < 4; e += 2) {
+            const bf16x2 x2 = {(bf16)acc[i][j][e], (bf16)acc[i][j][e + 1]};
+            act_entries(__builtin_bit_cast(unsigned, x2), far, at[e], at[e + 1]);
+          }
+          known = !__any(act_far(far));
           if (known) {
 #pragma unroll
-            for (int e = 0; e < 4; ++e) f[e] = __builtin_bit_cast(float, tab[at[e]]);
+            for (int e = 0; e < 4; ++e) f[e] = __builtin_bit_cast(float, act_at(tab, at[e]));
           }
         }
         if (!known) {
@@ -572,14 +584,15 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
         if constexpr (TAB) {
           if (by_table && (whole || n + 8 <= N)) {
             const u32x4 u = __builtin_bit_cast(u32x4, sv);
-            unsigned at[8], far = 0;
+            unsigned at[8];
+            u16x2 far = {0, 0};
 #pragma unroll
-            for (int e = 0; e < 8; ++e) at[e] = act_entry(u[e >> 1] >> (16 * (e & 1)), far);
-            if (!__any(far >= ACT_TAB_HALF)) {
+            for (int e = 0; e < 4; ++e) act_entries(u[e], far, at[2 * e], at[2 * e + 1]);
+            if (!__any(act_far(far))) {
               unsigned t[8];
               u32x4 o, d;
 #pragma unroll
-              for (int e = 0; e < 8; ++e) t[e] = tab[at[e]];
+              for (int e = 0; e < 8; ++e) t[e] = act_at(tab, at[e]);
 #pragma unroll
               for (int e = 0; e < 4; ++e) {
                 o[e] = __builtin_amdgcn_perm(t[2 * e + 1], t[2 * e], 0x05040100);
