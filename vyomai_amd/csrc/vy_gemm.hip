@@ -1289,21 +1289,21 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
 // 64 x 64 tiles for outputs that give the big tiles too few workgroups: KG groups of 4 waves (2 x 2, 32 x 32 outputs each), each
 // with a ring of NBUF stages of its own, of which NBUF - 1 are on their way (counted vmcnt).  The sums of every `per` stages are added
 // up in order (sum_slices: as many as where K is split over workgroups, so that the result does not hang on the kernel); two groups
-// take half of the two or four slices each and add them up through LDS at the end.
-// Bound by the chain of stages (0.3 us each: barrier, LDS reads, 8 products a wave), so many workgroups per CU and, where there is
-// at most one, two groups in it.  512 x 768 x 768: 12.4 -> 8.5 us against K split over workgroups and a second launch;
-// 512 x 3072 x 768: 21.4 -> 10.5; 1056 x 2304 x 768: 22.0 -> 11.7; 264 x 2048 x 2048: 24.9 -> 17.9.  (Adding the slices up in order
-// takes 0.8 us of that, eight and more slices the second group too.  Four groups: no faster than two on any shape; a fourth stage: level.)
+// take half of the slices each -- up to MOST -- and keep each by itself in registers; the second group's go through LDS at the end.
+// Bound by the chain of stages (0.33 us each: barrier, LDS reads, 8 products a wave), so many workgroups per CU and, where there is
+// at most one, two groups in it (0.24 us a stage).  Weights out of the Infinity Cache: 512 x 768 x 768 8.1 us in one group, 6.6 in two;
+// 700 x 1024 x 1024, eight slices, 10.7 and 8.4; sixteen slices, 512 x 768 x 3072: 16.4 (K over workgroups and a second launch 18.1);
+// 256 x 2048 x 2048: 13.2 (18.4).  Four groups: no faster than two on any shape; a fourth and fifth stage: level.
 // ------------------------------------------------------------------------------------------
-template <int KG, int NBUF, int EPI, int ACT, bool GRAD>
+template <int KG, int NBUF, int MOST, int EPI, int ACT, bool GRAD>
 __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
     int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob, int per) {
   constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
   constexpr int TM = 2, TN = 2, PER = 2;               // 16 x 16 blocks and 1 KiB pieces of either operand per wave
   constexpr int STAGE = (BM + BN) * ROWB, RING = NBUF * STAGE;
-  static_assert(KG <= 2 && (KG - 1) * 2 * BM * BN * 4 <= KG * RING, "the second group's two slices lie in the rings");
-  constexpr int LDS_BYTES = vy_cmax(KG * RING, epi_lds_bytes(BM, BN, EPI, 1));
+  static_assert(KG <= 2, "one group, or two");
+  constexpr int LDS_BYTES = vy_cmax(vy_cmax(KG * RING, (KG - 1) * MOST * BM * BN * 4), epi_lds_bytes(BM, BN, EPI, 1));   // (MOST slices of the second group)
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES];
 
   const int lane = threadIdx.x & 63;
@@ -1364,16 +1364,14 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     xa[ks] = vy_lds_addr(ring) + (wm * 16 * TM + r16) * ROWB + coff;
     wa[ks] = vy_lds_addr(ring) + BM * ROWB + (wn * 16 * TN + r16) * ROWB + coff;
   }
-  const bool four = KG > 1 && KT > 2 * per;               // (two groups: 2 or 4 slices)
-  const int n_it = KG == 1 ? KT : four ? 2 * per : per;   // of a group
+  const int slices = (KT + per - 1) / per, half = (slices + 1) / 2;   // two groups: the first `half` slices, and the others
+  const int n_it = KG == 1 ? KT : half * per;                        // of a group
   const int first = grp * n_it;
-  f32x4 sum[TN][TM];   // of the slices behind
 #pragma unroll
   for (int i = 0; i < NBUF - 1; ++i)
     if (i < n_it) stage(first + i, i);
   int buf = 0, it = 0;
-  for (;;) {
-    const int end = it + per < n_it ? it + per : n_it;
+  auto stages_to = [&](int end) __attribute__((always_inline)) {
     for (; it < end; ++it) {
       // the slice has landed for this wave, NBUF - 2 younger ones may still be on their way (near the end: wait for all) ...
       if (it + NBUF - 2 < n_it) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER * (NBUF - 2)) : "memory");
@@ -1401,39 +1399,61 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
         for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[1][i], xf[1][j], acc[i][j], 0, 0, 0);
       buf = buf + 1 == NBUF ? 0 : buf + 1;
     }
-    if (it == n_it) break;
-    const bool begun = it > per;
+  };
+  if constexpr (KG == 1) {
+    f32x4 sum[TN][TM];   // of the slices behind
+    for (;;) {
+      stages_to(it + per < n_it ? it + per : n_it);
+      if (it == n_it) break;
+      const bool begun = it > per;
 #pragma unroll
-    for (int i = 0; i < TN; ++i)
+      for (int i = 0; i < TN; ++i)
 #pragma unroll
-      for (int j = 0; j < TM; ++j) {
-        sum[i][j] = begun ? sum[i][j] + acc[i][j] : acc[i][j];
-        acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int j = 0; j < TM; ++j) {
+          sum[i][j] = begun ? sum[i][j] + acc[i][j] : acc[i][j];
+          acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    }
+    __syncthreads();   // what follows reuses the buffers: every wave is through with its reads
+    if (n_it > per)
+#pragma unroll
+      for (int i = 0; i < TN; ++i)
+#pragma unroll
+        for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j] + acc[i][j];
+  } else {
+    f32x4 part[MOST][TN * TM];   // each slice of the group by itself
+#pragma unroll
+    for (int s = 0; s < MOST; ++s)
+      if (s < half) {
+        stages_to((s + 1) * per);
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) {
+          part[s][i] = acc[i / TM][i % TM];
+          acc[i / TM][i % TM] = f32x4{0.f, 0.f, 0.f, 0.f};
+        }
       }
-  }
-  // what follows reuses the buffers: every wave is through with its reads
-  __syncthreads();
-  if (grp == 0 && n_it > per)
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j) acc[i][j] = sum[i][j] + acc[i][j];
-  if constexpr (KG > 1) {
-    f32x4* part = reinterpret_cast<f32x4*>(smem) + (threadIdx.x & 255);
+    __syncthreads();
+    f32x4* other = reinterpret_cast<f32x4*>(smem) + (threadIdx.x & 255);   // the second group's, [slice][block][thread]
     if (grp)
 #pragma unroll
-      for (int i = 0; i < TN * TM; ++i) {
-        if (four) part[(TN * TM + i) * 256] = sum[i / TM][i % TM];
-        part[i * 256] = acc[i / TM][i % TM];
-      }
+      for (int s = 0; s < MOST; ++s)
+        if (s < slices - half)
+#pragma unroll
+          for (int i = 0; i < TN * TM; ++i) other[(s * TN * TM + i) * 256] = part[s][i];
     __syncthreads();
     if (grp) return;   // (a barrier waits for the waves that are left)
 #pragma unroll
-    for (int i = 0; i < TN * TM; ++i) {
-      f32x4& a = acc[i / TM][i % TM];
-      if (four) a = a + part[(TN * TM + i) * 256];
-      a = a + part[i * 256];
-    }
+    for (int i = 0; i < TN * TM; ++i) acc[i / TM][i % TM] = part[0][i];
+#pragma unroll
+    for (int s = 1; s < MOST; ++s)
+      if (s < half)
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) acc[i / TM][i % TM] = acc[i / TM][i % TM] + part[s][i];
+#pragma unroll
+    for (int s = 0; s < MOST; ++s)
+      if (s < slices - half)
+#pragma unroll
+        for (int i = 0; i < TN * TM; ++i) acc[i / TM][i % TM] = acc[i / TM][i % TM] + other[(s * TN * TM + i) * 256];
     __syncthreads();
   }
   EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
@@ -1659,15 +1679,53 @@ inline Scratch splitk_ws(hipStream_t st) {
 // own rate: 8192 x 2048 with K = 12288 is 352 tiles of 256 x 192 -- two rounds, the second a third full, 459 us -- or 256 tiles of
 // 256 x 256: 313 us; 8000 x 1024, K = 6144: 124 us on 256 x 192, 152 us on 256 x 256, 100 us on 256 x 128 (250 tiles).  So the
 // launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below; the constants
-// are fits to launches of 40 shapes from 48 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
-// output alone and so moves no choice).
+// are fits to launches of 130 shapes from 40 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
+// output alone and so moves no choice), up to 4096 rows in graphs that walk through 170 MB of weights, as a model's layers do: products
+// that find their weights in L2, as a loop over one product does, made one launch look shorter than two groups in it.  90 shapes of
+// 40 to 4096 rows: the fastest kernel for 83, within 10 % of it for the others.
 // ------------------------------------------------------------------------------------------
-enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_128x128_SPLIT, T_256x128_SPLIT, T_320x128_SPLIT };
-constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 128, 256, 320};
-constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 128, 128, 128};
-constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 256, 512, 512};
+enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_64x64_MANY, T_128x128_SPLIT, T_256x128_SPLIT, T_320x128_SPLIT };
+constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 64, 128, 256, 320};
+constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 64, 128, 128, 128};
+constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 512, 256, 512, 512};
 struct Tiling { TileKind kind; int slices; };
 
+// what a shape costs on a tile, S slices of K added up
+template <TileKind kind>
+inline double tile_cost(int64_t M, int64_t N, int KT, int S, int chip) {
+  const int64_t tiles = vy_cdiv(M, TILE_M[kind]) * vy_cdiv(N, TILE_N[kind]);
+  const double load = (double)tiles / chip;
+  // `fixed` per round, `stage` per stage of a round; the stages of a last round that leaves CUs idle run up to 30 % faster
+  auto one_shot = [&](int per_cu, double launch, double fixed, double stage) {
+    const double r = load / per_cu, whole = (double)(int64_t)r, part = r - whole;
+    return launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * stage * KT;
+  };
+  switch (kind) {
+    case T_256x256: return one_shot(1, 2.5, 7.0, 1.55);
+    case T_256x192: return one_shot(1, 2.3, 5.5, 1.30);
+    case T_256x128: return one_shot(1, 4.5, 4.1, 0.97);
+    case T_128x128: return load <= 1 ? 8.5 + 0.72 * KT : one_shot(2, 3.5, 5.0, 1.0);     // (two of them share a CU)
+    case T_64x64: return (S > 1 ? 4.1 : 3.2) + (load > 1 ? 0.8 : 0.0) + KT * (0.25 * load > 0.335 ? 0.25 * load : 0.335);
+    case T_64x64_TWICE: case T_64x64_MANY: return 1.2 + (double)(int64_t)(load + 0.999) * (2.0 + 0.245 * KT + 0.13 * (S - 2));
+    default: {   // K over several workgroups: the partial sums' way through memory (about 6 TB/s there and back) and a second launch
+      const double bytes = 4.0 * S * tiles * TILE_M[kind] * TILE_N[kind];
+      const int per = (KT + S - 1) / S;
+      const double sums = 7.5 + 2 * bytes / 6e6;
+      if (kind != T_128x128_SPLIT) return sums + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * (1.2 * TILE_M[kind] / 256);
+      if (tiles * S <= chip) return sums + 0.72 * per;
+      const double r = (double)(tiles * S) / (2 * chip), whole = (double)(int64_t)r, part = r - whole;   // (two of them share a CU)
+      return sums + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * 0.95 * per;
+    }
+  }
+}
+// may partial sums of S slices on these tiles lie in `ws` bytes?  128 < M <= 320: one row tile may hold every row, so that a weight
+// crosses L2 -> LDS once
+template <TileKind kind>
+inline bool split_fits(int64_t M, int64_t N, int S, int64_t ws) {
+  if (kind == T_256x128_SPLIT && (M <= 128 || M > 256)) return false;
+  if (kind == T_320x128_SPLIT && (M <= 256 || M > 320)) return false;
+  return 4 * S * vy_cdiv(M, TILE_M[kind]) * vy_cdiv(N, TILE_N[kind]) * TILE_M[kind] * TILE_N[kind] <= ws;
+}
 // Slices of K whose sums a product adds up, in order: what fills the chip where every slice is a workgroup of its own (as many as
 // `target` workgroups in all, a power of two -- one per group of XCDs, splitk_block_of -- of at least two stages, none empty).  The
 // kernels below add up the same sums in the same order, so a result hangs neither on which of them the shape takes nor on a workspace
@@ -1692,37 +1750,24 @@ inline int sum_slices(int64_t M, int64_t N, int64_t K) {
 
 inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes) {
   const int KT = (int)vy_cdiv(K, BK), S = sum_slices(M, N, K);
-  Tiling best{T_256x256, S};
+  Tiling best{T_64x64, S};
   double least = 1e30;
   auto offer = [&](TileKind kind, double us) {
     if (us < least) { least = us; best.kind = kind; }
   };
-  auto tiles_of = [&](TileKind k) { return vy_cdiv(M, TILE_M[k]) * vy_cdiv(N, TILE_N[k]); };
-  // `fixed` per round, `stage` per stage of a round; the stages of a last round that leaves CUs idle run up to 30 % faster
-  auto one_shot = [&](TileKind k, int per_cu, double launch, double fixed, double stage) {
-    const double r = (double)tiles_of(k) / (chip * per_cu), whole = (double)(int64_t)r, part = r - whole;
-    offer(k, launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * stage * KT);
-  };
-  const double load = (double)tiles_of(T_64x64) / chip;
-  offer(T_64x64, 4.3 + KT * (0.22 * load > 0.295 ? 0.22 * load : 0.295));
+  offer(T_64x64, tile_cost<T_64x64>(M, N, KT, S, chip));
   if (S == 1) {
-    one_shot(T_256x256, 1, 2.5, 7.0, 1.55);
-    one_shot(T_256x192, 1, 2.3, 5.5, 1.30);
-    one_shot(T_256x128, 1, 4.5, 4.1, 0.97);
-    if (tiles_of(T_128x128) <= chip) offer(T_128x128, 8.5 + 0.72 * KT);
-    else one_shot(T_128x128, 2, 3.5, 5.0, 1.0);     // (two of them share a CU)
+    offer(T_256x256, tile_cost<T_256x256>(M, N, KT, S, chip));
+    offer(T_256x192, tile_cost<T_256x192>(M, N, KT, S, chip));
+    offer(T_256x128, tile_cost<T_256x128>(M, N, KT, S, chip));
+    offer(T_128x128, tile_cost<T_128x128>(M, N, KT, S, chip));
     return best;
   }
-  if (S == 2 || S == 4) offer(T_64x64_TWICE, 3.0 + (double)vy_cdiv(tiles_of(T_64x64_TWICE), chip) * (2.2 + 0.44 * ((KT + 1) / 2)));
-  // K over several workgroups: the partial sums' way through memory (about 8 TB/s there and back: mostly the Infinity Cache) and a second launch.
-  // 128 < M <= 320: one row tile holds every row, so a weight crosses L2 -> LDS once
-  const TileKind k = M > 256 && M <= 320 ? T_320x128_SPLIT : M > 128 && M <= 256 ? T_256x128_SPLIT : T_128x128_SPLIT;
-  const int64_t tiles = tiles_of(k);
-  const double bytes = 4.0 * S * tiles * TILE_M[k] * TILE_N[k];
-  if (bytes > (double)ws_bytes) return best;
-  const int per = (KT + S - 1) / S;
-  const double stage = k == T_128x128_SPLIT ? (tiles * S > chip ? 1.0 : 0.72) : 1.2 * TILE_M[k] / 256;
-  offer(k, 7.5 + (double)vy_cdiv(tiles * S, (int64_t)chip * (k == T_128x128_SPLIT ? 2 : 1)) * per * stage + 2 * bytes / 8e6);
+  if (S <= 4) offer(T_64x64_TWICE, tile_cost<T_64x64_TWICE>(M, N, KT, S, chip));
+  else offer(T_64x64_MANY, tile_cost<T_64x64_MANY>(M, N, KT, S, chip));
+  if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, tile_cost<T_128x128_SPLIT>(M, N, KT, S, chip));
+  if (split_fits<T_256x128_SPLIT>(M, N, S, ws_bytes)) offer(T_256x128_SPLIT, tile_cost<T_256x128_SPLIT>(M, N, KT, S, chip));
+  if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, tile_cost<T_320x128_SPLIT>(M, N, KT, S, chip));
   return best;
 }
 
@@ -2500,8 +2545,9 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
       case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>); break;
       case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, EPI, ACT, GRAD>); break;
       case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
-      case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, EPI, ACT, GRAD>); break;
-      case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, EPI, ACT, GRAD>); break;
+      case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, EPI, ACT, GRAD>); break;
+      case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, EPI, ACT, GRAD>); break;
+      case T_64x64_MANY: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, EPI, ACT, GRAD>); break;
       case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
       case T_256x128_SPLIT: launch_split<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
       case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
@@ -2527,8 +2573,9 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
     case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, 2, ACT, false>); break;
     case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, 2, ACT, false>); break;
     case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, 2, ACT, false>); break;
-    case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 2, ACT, false>); break;
-    case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, ACT, false>); break;
+    case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, 2, ACT, false>); break;
+    case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 2, ACT, false>); break;
+    case T_64x64_MANY: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, 2, ACT, false>); break;
     default: return VY_ERR_UNSUPPORTED;   // (K split over workgroups)
   }
 #undef VY_TILES
