@@ -535,7 +535,10 @@ struct DecAttnArgs {
   const bf16* k; const bf16* v; long long c_sb, c_sh, c_sl;
   bf16* out; long long o_sb;                // out[b][head * DH + d]
   const int* pos_dev; int S; int h, hk; float scale;
+  // PROJ: part[workgroup's heads][b][d] = their columns of wo times their results, 64 `passes` rows of wo per workgroup
+  const bf16* wo; float* part; int d, passes;
 };
+constexpr int PROJ_PASSES = 4;   // most
 
 template <int LPK>
 __device__ __forceinline__ float dec_group_sum(float v) {   // sum over the LPK lanes of a key group, in every lane
@@ -568,18 +571,36 @@ __device__ __forceinline__ float dec_stride_sum(float v) {
 // R > 1 (grouped-query attention): one workgroup per (batch row, KV head) serves the R query heads that share the head from
 // ONE read of its K and V rows -- with a workgroup per query head the K/V stream (non-temporal: it does not stay on chip)
 // was fetched R times, and a GQA step read as many bytes as the full-head model (0.492 against 0.484 ms per token step).
-template <int DH, int NW, int NP, bool NT, int R = 1>
+//
+// PROJ (few sequences): each result is multiplied with its columns of the output projection here, whose launch of its own falls away;
+// the product behind adds the heads' shares up (PARTS of vy_few.hip).  Every head is attended to by as many workgroups as the
+// projection's rows are spread over -- its keys come from L2 then, and no workgroup has more to read than before.
+// 12 layers of 768, prompt and 24 steps: one sequence behind 60 tokens 6700 -> 6120 us, behind 500 7200 -> 6580; 4 behind 500 11150 -> 10790,
+// with 4 key/value heads 11070 -> 9990.
+template <int DH, int NW, int NP, bool NT, int R = 1, bool PROJ = false>
 __global__ __launch_bounds__(64 * NW) void dec_attn_kernel(const DecAttnArgs p) {
   constexpr int LPK = DH / 8, KPW = 64 / LPK, KPP = NW * KPW;
   __shared__ float red_m[R][NW], red_l[R][NW];
   __shared__ float red_o[R][NW][DH];
+  __shared__ __attribute__((aligned(16))) bf16 result[PROJ ? R : 1][PROJ ? DH : 8];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int b = blockIdx.y;
-  // R == 1: blockIdx.x is the query head; R > 1: the KV head, query heads kvh * R .. + R - 1
-  const int head0 = R == 1 ? (int)blockIdx.x : (int)blockIdx.x * R;
-  const int kvh = R == 1 ? head0 / (p.h / p.hk) : (int)blockIdx.x;
+  // R == 1: `unit` is the query head; R > 1: the KV head, query heads kvh * R .. + R - 1
+  const int units = p.h / R, unit = PROJ ? (int)blockIdx.x % units : (int)blockIdx.x;
+  const int head0 = unit * R;
+  const int kvh = R == 1 ? head0 / (p.h / p.hk) : unit;
   const int g = lane / LPK, ch = lane % LPK;
+  bf16x8 wo8[PROJ ? PROJ_PASSES : 1][PROJ ? R : 1];
+  const int row0 = PROJ ? (int)blockIdx.x / units * p.passes * KPP + wave * KPW + g : 0;   // of wo, this lane's first
+  if constexpr (PROJ) {
+#pragma unroll
+    for (int i = 0; i < PROJ_PASSES; ++i)
+      if (i < p.passes)
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+          wo8[i][r] = *reinterpret_cast<const bf16x8*>(p.wo + (long long)(row0 + i * KPP) * p.d + (head0 + r) * DH + ch * 8);
+  }
   const int S = p.pos_dev ? *p.pos_dev + 1 : p.S;
   const bf16* kb = p.k + (long long)b * p.c_sb + (long long)kvh * p.c_sh + ch * 8;
   const bf16* vb = p.v + (long long)b * p.c_sb + (long long)kvh * p.c_sh + ch * 8;
@@ -650,20 +671,39 @@ __global__ __launch_bounds__(64 * NW) void dec_attn_kernel(const DecAttnArgs p) 
     float L = 0.f, o = 0.f;
 #pragma unroll
     for (int w = 0; w < NW; ++w) { L += red_l[r][w]; o += red_o[r][w][c]; }
-    p.out[(long long)b * p.o_sb + (head0 + r) * DH + c] = (bf16)(o / L);
+    if constexpr (PROJ) result[r][c] = (bf16)(o / L);
+    else p.out[(long long)b * p.o_sb + (head0 + r) * DH + c] = (bf16)(o / L);
+  }
+  if constexpr (PROJ) {
+    __syncthreads();
+    bf16x8 x[R];
+#pragma unroll
+    for (int r = 0; r < R; ++r) x[r] = *reinterpret_cast<const bf16x8*>(&result[r][ch * 8]);
+#pragma unroll
+    for (int i = 0; i < PROJ_PASSES; ++i)
+      if (i < p.passes) {
+        float v = 0.f;
+#pragma unroll
+        for (int r = 0; r < R; ++r)
+#pragma unroll
+          for (int e = 0; e < 8; e += 2)
+            v = __builtin_amdgcn_fdot2_f32_bf16(bf16x2{wo8[i][r][e], wo8[i][r][e + 1]}, bf16x2{x[r][e], x[r][e + 1]}, v, false);
+        v = dec_group_sum<LPK>(v);
+        if (ch == 0) p.part[((long long)unit * gridDim.y + b) * p.d + row0 + i * KPP] = v;
+      }
   }
 }
 
-template <int DH, int NW, bool NT, int R = 1>
+template <int DH, int NW, bool NT, int R = 1, bool PROJ = false>
 int dec_attn_go(const DecAttnArgs& a, int B, int Smax, hipStream_t st) {
   constexpr int KPP = NW * (64 / (DH / 8));
-  const dim3 grid((unsigned)(R == 1 ? a.h : a.hk), (unsigned)B), block(64 * NW);
+  const dim3 grid((unsigned)((R == 1 ? a.h : a.hk) * (PROJ ? a.d / (KPP * a.passes) : 1)), (unsigned)B), block(64 * NW);
   const int np = (Smax + KPP - 1) / KPP;
-  if (np <= 3) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 3, NT, R>), grid, block, 0, st, a);
-  else if (np <= 5) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 5, NT, R>), grid, block, 0, st, a);
-  else if (np <= 7) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 7, NT, R>), grid, block, 0, st, a);
-  else if (np <= 10) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 10, NT, R>), grid, block, 0, st, a);
-  else if (np <= 12) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 12, NT, R>), grid, block, 0, st, a);
+  if (np <= 3) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 3, NT, R, PROJ>), grid, block, 0, st, a);
+  else if (np <= 5) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 5, NT, R, PROJ>), grid, block, 0, st, a);
+  else if (np <= 7) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 7, NT, R, PROJ>), grid, block, 0, st, a);
+  else if (np <= 10) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 10, NT, R, PROJ>), grid, block, 0, st, a);
+  else if (np <= 12) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 12, NT, R, PROJ>), grid, block, 0, st, a);
   else return 1;
   return 0;
 }
@@ -985,4 +1025,33 @@ int vy_dec_attn(const void* q, int64_t q_sb, const void* k, const void* v, int64
   if (rc) return VY_ERR_UNSUPPORTED;
   VY_CHECK_LAUNCH("vy_dec_attn");
   return VY_OK;
+}
+
+// internal (vy_runtime.hip): attention of few sequences' steps and its output projection wo [h 64][h 64]: fp32 shares
+// part[returned][B][h 64], in `room` bytes, to be added up.  0: other sizes.
+int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, int64_t c_sh, int64_t c_sl, const void* wo, float* part,
+                    int64_t room, int B, int h, int hk, int64_t S, int64_t smax, const int* pos_dev, float scale, hipStream_t st) {
+  if (hk < 1 || h % hk || S < 1 || c_sl % 8 || c_sh % 8 || c_sb % 8 || ((uintptr_t)q % 16) || ((uintptr_t)k % 16) || ((uintptr_t)v % 16) ||
+      ((uintptr_t)wo % 16))
+    return 0;
+  DecAttnArgs a{};
+  a.q = (const bf16*)q; a.q_sb = h * 64; a.k = (const bf16*)k; a.v = (const bf16*)v; a.c_sb = c_sb; a.c_sh = c_sh; a.c_sl = c_sl;
+  a.pos_dev = pos_dev; a.S = (int)S; a.h = h; a.hk = hk; a.scale = scale; a.wo = (const bf16*)wo; a.part = part; a.d = h * 64;
+  // One sequence: a workgroup per query head also where several share a key head (12 layers of 768, 4 key/value heads, 24 steps and
+  // their prompt: behind 60 tokens 6113 against 6190 us, behind 500 6580 and 6990); more: one for all that share it, whose fewer shares the next
+  // product adds up sooner (4 sequences behind 30 tokens 9480 and 8990).
+  const int rep = B > 1 && h / hk >= 2 && h / hk <= 4 ? h / hk : 1, units = h / rep;
+  if (units > 16 || (int64_t)units * B * a.d * 4 > room) return 0;
+  if (rep == 4 && (pos_dev ? smax : S) > 640) return 0;   // (longer contexts in registers beside four heads' rows of wo: spills)
+  // rows of wo in as few passes as leave at most a workgroup a CU (h blocks of 64 rows)
+  for (int n = 1; n <= PROJ_PASSES && !a.passes; ++n)
+    if (h % n == 0 && (int64_t)units * B * (h / n) <= 256) a.passes = n;
+  if (!a.passes) return 0;
+  const int bound = (int)(pos_dev ? smax : S);
+  int rc;
+  if (rep == 2) rc = dec_attn_go<64, 8, false, 2, true>(a, B, bound, st);
+  else if (rep == 3) rc = dec_attn_go<64, 8, false, 3, true>(a, B, bound, st);
+  else if (rep == 4) rc = dec_attn_go<64, 8, false, 4, true>(a, B, bound, st);
+  else rc = dec_attn_go<64, 8, false, 1, true>(a, B, bound, st);
+  return rc ? 0 : units;
 }

@@ -51,6 +51,8 @@ template <int EPI, int PRO, int MR, int KC>
 __global__ __launch_bounds__(256) void few_kernel(Args a) {
   constexpr int K = 256 * KC, R = (EPI != STORE || KC % 2) ? 2 : 1, P = KC * R / 2;   // columns; weight rows and pieces per wave
   __shared__ __attribute__((aligned(16))) bf16 hs[PRO == PLAIN ? 8 : MR * K];
+  constexpr int SHARES = PRO == PARTS ? 4 / MR : 1;   // waves that add up a row
+  __shared__ __attribute__((aligned(16))) float sums[SHARES > 1 ? 4 * K : 4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int units = EPI == STORE ? (a.N + R - 1) / R : EPI == QKV ? a.N / 2 : a.N;   // of R weight rows
   const int step = gridDim.x * 4;
@@ -90,28 +92,71 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   };
   if constexpr (EPI == QKV) pos = a.pos_dev ? *a.pos_dev : a.pos;
   if (u < units) request(u);
-  if (u < units && (PRO == PLAIN || wave >= a.M)) request_rest(u);
+  const int row = wave / SHARES;   // of the operand, this wave's
+  const bool leads = wave % SHARES == 0 && row < a.M;
+  if (u < units && (PRO == PLAIN || !leads)) request_rest(u);
 
   if constexpr (PRO != PLAIN) {
     if (a.advance && blockIdx.x == 0)
       for (int i = threadIdx.x; i < a.n_adv; i += 256) a.advance[a.slots ? a.slots[i] : i] += 1;
-    if (wave < a.M) {
-      const int m = wave;
-      float v[KC][4], g[KC][4], b[KC][4];
-      if constexpr (PRO == LAYER) {
-        bf16x4 v4[KC], g4[KC], b4[KC];
+    bf16x4 v4[KC], g4[KC], b4[KC], xb4[KC];
+    if constexpr (PRO == LAYER || PRO == PARTS) {
+      if (leads) {
 #pragma unroll
         for (int c = 0; c < KC; ++c) {
           const int col = (64 * c + lane) * 4;
-          v4[c] = *reinterpret_cast<const bf16x4*>(a.x + m * a.ldx + col);
+          v4[c] = *reinterpret_cast<const bf16x4*>(a.x + row * a.ldx + col);
           g4[c] = *reinterpret_cast<const bf16x4*>(a.ln_g + col);
           b4[c] = *reinterpret_cast<const bf16x4*>(a.ln_b + col);
+          xb4[c] = bf16x4{(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
+          if (PRO == PARTS && a.x_bias) xb4[c] = *reinterpret_cast<const bf16x4*>(a.x_bias + col);
         }
         if (u < units) request_rest(u);
+      }
+    }
+    f32x4 mine[KC];   // PARTS: this wave's share of the row
+    if constexpr (PRO == PARTS) {
+      constexpr int AHEAD = MR == 4 ? 6 : 4;   // parts requested together: all that a wave has, of 12 heads' two times
+#pragma unroll
+      for (int c = 0; c < KC; ++c) mine[c] = f32x4{0.f, 0.f, 0.f, 0.f};
+      if (row < a.M)
+        for (int p0 = wave % SHARES; p0 < a.n_parts; p0 += AHEAD * SHARES) {
+          f32x4 part[AHEAD][KC];
+#pragma unroll
+          for (int i = 0; i < AHEAD; ++i)
+#pragma unroll
+            for (int c = 0; c < KC; ++c)
+              part[i][c] = *reinterpret_cast<const f32x4*>(a.parts + ((int64_t)min(p0 + i * SHARES, a.n_parts - 1) * a.M + row) * K + (64 * c + lane) * 4);
+#pragma unroll
+          for (int i = 0; i < AHEAD; ++i)
+            if (p0 + i * SHARES < a.n_parts)
+#pragma unroll
+              for (int c = 0; c < KC; ++c) mine[c] += part[i][c];
+        }
+      if constexpr (SHARES > 1) {
+        if (!leads)
+#pragma unroll
+          for (int c = 0; c < KC; ++c) *reinterpret_cast<f32x4*>(sums + wave * K + (64 * c + lane) * 4) = mine[c];
+      }
+    }
+    if constexpr (SHARES > 1) __syncthreads();
+    if (leads) {
+      const int m = row;
+      float v[KC][4], g[KC][4], b[KC][4];
+      if constexpr (PRO == LAYER || PRO == PARTS) {
 #pragma unroll
         for (int c = 0; c < KC; ++c)
 #pragma unroll
           for (int e = 0; e < 4; ++e) { v[c][e] = (float)v4[c][e]; g[c][e] = (float)g4[c][e]; b[c][e] = (float)b4[c][e]; }
+        if constexpr (PRO == PARTS) {
+#pragma unroll
+          for (int c = 0; c < KC; ++c) {
+#pragma unroll
+            for (int s = 1; s < SHARES; ++s) mine[c] += *reinterpret_cast<const f32x4*>(sums + (wave + s) * K + (64 * c + lane) * 4);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) v[c][e] = vy_round_bf16(mine[c][e] + (float)xb4[c][e] + v[c][e]);
+          }
+        }
       } else {
         f32x4 s4[KC], p4[KC], g4[KC];
         bf16x4 y4[KC];
@@ -150,7 +195,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
           for (int e = 0; e < 4; ++e) { g[c][e] = a.w_pre ? g4[c][e] : 1.f; b[c][e] = 0.f; }
       }
       float mean = 0.f, rstd = 1.f;
-      if (PRO == LAYER || a.w_pre) stats<KC>(v, lane, PRO == LAYER ? K : a.n, PRO == STREAM && a.rms, a.eps, mean, rstd);
+      if (PRO != STREAM || a.w_pre) stats<KC>(v, lane, PRO != STREAM ? K : a.n, PRO == STREAM && a.rms, a.eps, mean, rstd);
 #pragma unroll
       for (int c = 0; c < KC; ++c) {
         const int col = (64 * c + lane) * 4;
@@ -258,6 +303,7 @@ bool few_k(int epi, int pro, int64_t K) {
   const int kc = (int)(K / 256);
   if (pro == PLAIN) return epi == QKV ? kc >= 2 && kc <= 4 : epi == STORE && (kc == 2 || kc == 3 || kc == 4 || kc == 8 || kc == 12 || kc == 16);
   if (pro == LAYER) return epi != GATED && kc >= 2 && kc <= 4;
+  if (pro == PARTS) return epi == STORE && kc >= 2 && kc <= 4;
   return epi != QKV && (kc == 4 || kc == 8);
 }
 
@@ -268,6 +314,7 @@ int few_go(int epi, int pro, const Args& a, int64_t K, hipStream_t st) {
   if (pro == PLAIN && epi == QKV) switch (kc) { FEW(QKV, PLAIN, 2); FEW(QKV, PLAIN, 3); FEW(QKV, PLAIN, 4); }
   else if (pro == PLAIN) switch (kc) { FEW(STORE, PLAIN, 2); FEW(STORE, PLAIN, 3); FEW(STORE, PLAIN, 4); FEW(STORE, PLAIN, 8); FEW(STORE, PLAIN, 12); FEW(STORE, PLAIN, 16); }
   else if (pro == LAYER && epi == QKV) switch (kc) { FEW(QKV, LAYER, 2); FEW(QKV, LAYER, 3); FEW(QKV, LAYER, 4); }
+  else if (pro == PARTS) switch (kc) { FEW(STORE, PARTS, 2); FEW(STORE, PARTS, 3); FEW(STORE, PARTS, 4); }
   else if (pro == LAYER) switch (kc) { FEW(STORE, LAYER, 2); FEW(STORE, LAYER, 3); FEW(STORE, LAYER, 4); }
   else if (epi == STORE) switch (kc) { FEW(STORE, STREAM, 4); FEW(STORE, STREAM, 8); }
   else switch (kc) { FEW(GATED, STREAM, 4); FEW(GATED, STREAM, 8); }
@@ -278,15 +325,19 @@ int few_go(int epi, int pro, const Args& a, int64_t K, hipStream_t st) {
 
 }  // namespace vy_few
 
-// test aid, not part of include/vyom_hip.h: one product by itself on contiguous rows.  a, b: gamma and beta of LAYER (bf16), w_post and
-// w_pre of STREAM (fp32); y: QKV's queries [M][nq], k and v [M][nkv]
+// test aid, not part of include/vyom_hip.h: one product by itself on contiguous rows.  a, b: gamma and beta of LAYER and PARTS (bf16), w_post and
+// w_pre of STREAM (fp32); PARTS: n shares s_in [n][M][K] and their bias `residual`; y: QKV's queries [M][nq], k and v [M][nkv]
 extern "C" int vy_debug_few(int epi, int pro, const void* x, const void* a, const void* b, const float* s_in, float* s_out, void* h, int n,
                             int rms, float eps, const void* w, const void* bias, int act, float act_arg, const void* residual, void* y,
                             int64_t ldy, void* k, void* v, int nq, int nkv, const float* cos_tab, const float* sin_tab, int pos, int M,
                             int N, int64_t K, void* stream) {
   vy_few::Args f{};
   f.x = (const bf16*)x; f.ldx = K;
-  if (pro == vy_few::LAYER) { f.ln_g = (const bf16*)a; f.ln_b = (const bf16*)b; }
+  if (pro == vy_few::PARTS) {
+    f.parts = s_in; f.n_parts = n; f.x_bias = (const bf16*)residual;
+    residual = nullptr;
+  }
+  if (pro == vy_few::LAYER || pro == vy_few::PARTS) { f.ln_g = (const bf16*)a; f.ln_b = (const bf16*)b; }
   else { f.w_post = (const float*)a; f.w_pre = (const float*)b; }
   f.s_in = s_in; f.s_out = s_out; f.lds = K; f.n = n; f.rms = rms; f.eps = eps; f.h = (bf16*)h; f.ldh = K;
   f.w = (const bf16*)w; f.N = N; f.M = M; f.bias = (const bf16*)bias; f.act = act; f.act_arg = act_arg;

@@ -39,6 +39,8 @@ int vy_dec_qkv(const void* x, const void* w, const void* bias, const float* cos_
                int hk, hipStream_t st);
 int vy_dec_linear_ex(const void* x, int ldx, const void* w, const void* bias, const void* residual, int ldr, const void* ln_g,
                      const void* ln_b, float ln_eps, void* y, int ldy, int B, int N, int K, int act, hipStream_t st);
+int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, int64_t c_sh, int64_t c_sl, const void* wo, float* part,
+                    int64_t room, int B, int h, int hk, int64_t S, int64_t smax, const int* pos_dev, float scale, hipStream_t st);
 int vy_dec_linear(const void* x, int ldx, const void* w, const void* bias, void* y, int ldy, int B, int N, int K, int act,
                   hipStream_t st);
 int vy_dec_linear_res_ln(const void* x, int ldx, const void* w, const void* bias, const void* residual, int ldr,
@@ -94,7 +96,8 @@ static bool few_operands(const vy_decode_plan* p, const void* x, const void* hid
   return given && all % 16 == 0 && (!logits || p->vocab > 0);
 }
 
-// The step of 1 to 4 sequences on the kernels of vy_few.hip: five launches per layer, LayerNorms inside the products behind them.
+// The step of 1 to 4 sequences on the kernels of vy_few.hip: four launches per layer -- LayerNorms inside the products behind them, the
+// output projection inside the attention (longer contexts: five, the projection by itself).
 static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos, const int32_t* pos_dev, void* hidden_out, void* logits,
                             int64_t ldv, hipStream_t st) {
   using namespace vy_few;
@@ -105,6 +108,8 @@ static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos,
   bf16 *q = take(B * (int64_t)d), *ao = take(B * (int64_t)d), *s1 = take(B * (int64_t)d), *s2 = take(B * (int64_t)d);
   bf16* hb[2] = {take(B * (int64_t)d), take(B * (int64_t)d)};
   bf16* mid = take(B * (int64_t)p->ffn);
+  float* part = (float*)w;            // the attention heads' shares of the output projection
+  const int64_t part_bytes = 24 * 32 * (int64_t)d * 4;   // (vy_decode_ws_bytes)
   const bf16* cur = (const bf16*)x;   // the layer's input rows: of the first layer x, of the others LN2 of the layer before
   const vy_decode_layer* before = nullptr;
   int rc;
@@ -122,16 +127,26 @@ static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos,
       a.x = cur; a.ldx = d;
     }
     if ((rc = few_go(QKV, before ? LAYER : PLAIN, a, d, st))) return rc;
-    if ((rc = vy_attn_decode_ex(q, d, 64, L.kcache, L.c_sb, L.c_sh, L.c_sl, L.vcache, L.c_sb, L.c_sh, L.c_sl, ao, d, B, h, hk, pos + 1,
-                                pos_dev, 64, 0.125f, VY_BF16, st))) return rc;
-    Args o{};
-    o.M = B; o.x = ao; o.ldx = d; o.w = (const bf16*)L.wo; o.bias = (const bf16*)L.bo; o.N = d; o.residual = cur; o.ldr = d;
-    o.y = s1; o.ldy = d;
-    if ((rc = few_go(STORE, PLAIN, o, d, st))) return rc;
     Args f{};
-    f.M = B; f.x = s1; f.ldx = d; f.ln_g = (const bf16*)L.ln1_w; f.ln_b = (const bf16*)L.ln1_b; f.eps = p->eps_attn;
+    f.M = B; f.ln_g = (const bf16*)L.ln1_w; f.ln_b = (const bf16*)L.ln1_b; f.eps = p->eps_attn;
     f.w = (const bf16*)L.w1; f.bias = (const bf16*)L.b1; f.N = p->ffn; f.act = p->act; f.y = mid; f.ldy = p->ffn;
-    if ((rc = few_go(STORE, LAYER, f, d, st))) return rc;
+    const int shares = few_k(STORE, PARTS, d) && (uintptr_t)L.bo % 8 == 0
+                           ? vy_dec_attn_out(q, L.kcache, L.vcache, L.c_sb, L.c_sh, L.c_sl, L.wo, part, part_bytes, B, h, hk, pos + 1,
+                                             L.c_sh / (L.c_sl ? L.c_sl : 1), pos_dev, 0.125f, st)
+                           : 0;
+    if (shares) {
+      f.parts = part; f.n_parts = shares; f.x_bias = (const bf16*)L.bo; f.x = cur; f.ldx = d;
+      if ((rc = few_go(STORE, PARTS, f, d, st))) return rc;
+    } else {
+      if ((rc = vy_attn_decode_ex(q, d, 64, L.kcache, L.c_sb, L.c_sh, L.c_sl, L.vcache, L.c_sb, L.c_sh, L.c_sl, ao, d, B, h, hk, pos + 1,
+                                  pos_dev, 64, 0.125f, VY_BF16, st))) return rc;
+      Args o{};
+      o.M = B; o.x = ao; o.ldx = d; o.w = (const bf16*)L.wo; o.bias = (const bf16*)L.bo; o.N = d; o.residual = cur; o.ldr = d;
+      o.y = s1; o.ldy = d;
+      if ((rc = few_go(STORE, PLAIN, o, d, st))) return rc;
+      f.x = s1; f.ldx = d;
+      if ((rc = few_go(STORE, LAYER, f, d, st))) return rc;
+    }
     Args g{};
     g.M = B; g.x = mid; g.ldx = p->ffn; g.w = (const bf16*)L.w2; g.bias = (const bf16*)L.b2; g.N = d; g.residual = cur; g.ldr = d;
     g.y = s2; g.ldy = d;
