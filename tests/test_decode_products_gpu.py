@@ -282,3 +282,31 @@ def test_attention_into_its_output_projection(B, h, hk, S):
         w = wo.double()[:, cols].T.contiguous()
         bound = e @ w.abs() + 64 * together * 2.0 ** -24 * (x.abs() @ w.abs())
         assert ((part[u].double() - x @ w).abs() <= bound + 1e-30).all()
+
+
+@pytest.mark.parametrize("M", [1, 2, 4])
+@pytest.mark.parametrize("K,n,np_kv", [(512, 512, 256), (512, 500, 0), (1024, 1024, 8), (1024, 1000, 1024), (1024, 1001, 520)])
+def test_rms_norm_of_rows_and_cache_rows_beside_it(M, K, n, np_kv):
+    x, g = rnd(M, K, seed=K + n), rnd(K, seed=5, scale=0.3, dtype=torch.float32) + 1
+    x[:, n:] = 0
+    eye = torch.eye(K, dtype=BF, device=DEV)[: K - 3].contiguous()         # (the products are the operand rows themselves)
+    kv = rnd(M, K, seed=7) if np_kv else None                             # (rows of the stride of x; their first np_kv columns)
+    gk = rnd(max(np_kv, 1), seed=8, scale=0.3, dtype=torch.float32) + 1
+    cache = torch.full((M, 2, np_kv), NAN, dtype=BF, device=DEV) if np_kv else None
+    at = torch.tensor([1, 0, 2, 1][:M], dtype=torch.int32, device=DEV)    # (row 2 is past the capacity)
+    y = torch.full((M, K - 3), NAN, dtype=BF, device=DEV)
+    go = entry("vy_debug_few", i32, i32, p, p, p, p, p, p, i32, i32, f32, p, p, i32, f32, p, p, i64, p, p, i32, i32, p, p, i32, i32, i32, i64, p)
+    assert go(STORE, 4, ptr(x), None, ptr(gk), None, None, None, n, 1, 1e-5, ptr(eye), None, NONE, 0.0, None, ptr(y), K - 3, ptr(cache), ptr(kv),
+              2, np_kv, ptr(at), ptr(g), 0, M, K - 3, K, stream()) == 0
+    torch.cuda.synchronize()
+    want, e = normed(x, n, 1, g, None)
+    within(y, want[:, : K - 3], e[:, : K - 3] + 2.0 ** -18 * want[:, : K - 3].abs())
+    if not np_kv:
+        return
+    rows, ek = normed(kv[:, :np_kv], np_kv, 1, gk, None)
+    for m in range(M):
+        for r in (0, 1):
+            if r == int(at[m]):
+                within(cache[m, r], rows[m], ek[m])
+            else:
+                assert torch.isnan(cache[m, r]).all()

@@ -5,13 +5,17 @@
 namespace vy_few {
 
 enum { STORE, QKV, GATED };         // epilogues
-enum { PLAIN, LAYER, STREAM, PARTS };   // operand rows: as they are; LayerNorm of bf16 rows; the residual stream's next norm; LayerNorm of a sum
+enum { PLAIN, LAYER, STREAM, PARTS, RMS };   // operand rows: as they are; LayerNorm of bf16 rows; the residual stream's next norm; LayerNorm of a
+                                             // sum; RMS norm of bf16 rows
 
 struct Args {
   const bf16* x; int64_t ldx;                      // PLAIN, LAYER: rows of K; STREAM: the sublayer's output rows (nullable)
   const bf16 *ln_g, *ln_b;                         // LAYER, PARTS
   const float* parts; int n_parts;                 // PARTS: rows bf16(parts[0] + .. + x_bias + x), parts [n_parts][M][K]
   const bf16* x_bias;
+  // RMS: rows x / rms(x over n columns) w_pre, zeros behind column n of x
+  const bf16* kv; const float* w_kv; int n_kv, np_kv;   // beside it: rows kv (stride ldx) by the same norm into row start[slot] of a cache
+  bf16* cache; int64_t k_ss, k_st; int cap, ring; const int* start;
   const float* s_in; float* s_out; int64_t lds;    // STREAM: s_out = s_in + norm(x) w_post (workgroup 0 writes it); operand = norm(s_out) w_pre
   const float *w_post, *w_pre; int n, rms;         //   norms over the first n columns; w_post NULL: plain sum; w_pre NULL: s_out itself
   float eps;

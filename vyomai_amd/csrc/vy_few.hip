@@ -55,8 +55,37 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   __shared__ __attribute__((aligned(16))) float sums[SHARES > 1 ? 4 * K : 4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int units = EPI == STORE ? (a.N + R - 1) / R : EPI == QKV ? a.N / 2 : a.N;   // of R weight rows
-  const int step = gridDim.x * 4;
+  const int step = (PRO == RMS && a.cache ? gridDim.x - 1 : gridDim.x) * 4;
   int u = blockIdx.x * 4 + wave;
+
+  if constexpr (PRO == RMS) {
+    if (a.cache && blockIdx.x == gridDim.x - 1) {   // one workgroup more: the new tokens' cache rows, a wave each
+      if (wave >= a.M) return;
+      constexpr int CH = 2;
+      const bf16* src = a.kv + wave * a.ldx;
+      float v[CH][8], q = 0.f;
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        if ((lane + 64 * c) * 8 < a.np_kv) {
+          VyChunk<bf16>::load(src + (lane + 64 * c) * 8, v[c]);
+#pragma unroll
+          for (int e = 0; e < 8; ++e) q += v[c][e] * v[c][e];
+        }
+      const int slot = a.slots ? a.slots[wave] : wave, pos = a.start[slot];
+      const float rstd = rsqrt_refined(vy_wave_sum(q) / (float)a.n_kv + a.eps);
+      if (!a.ring && pos >= a.cap) return;
+      bf16* dst = a.cache + slot * a.k_ss + (a.ring ? pos % a.cap : pos) * a.k_st;
+#pragma unroll
+      for (int c = 0; c < CH; ++c)
+        if ((lane + 64 * c) * 8 < a.np_kv) {
+          float o[8];
+#pragma unroll
+          for (int e = 0; e < 8; ++e) o[e] = v[c][e] * rstd * a.w_kv[(lane + 64 * c) * 8 + e];
+          VyChunk<bf16>::store(dst + (lane + 64 * c) * 8, o);
+        }
+      return;
+    }
+  }
 
   auto row_of = [&](int unit, int r) {
     if constexpr (EPI == QKV) return (unit >> 5) * 64 + (unit & 31) + 32 * r;
@@ -140,7 +169,32 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
       }
     }
     if constexpr (SHARES > 1) __syncthreads();
-    if (leads) {
+    if constexpr (PRO == RMS) {
+      if (leads) {
+        // (a lane's quads two by two: the 16-byte chunks, and so the sum's order, of the norm's own kernel)
+        auto column = [&](int c) { return ((c >> 1) * 64 + lane) * 8 + (c & 1) * 4; };
+        f32x4 w4[KC];
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          v4[c] = *reinterpret_cast<const bf16x4*>(a.x + row * a.ldx + column(c));
+          w4[c] = *reinterpret_cast<const f32x4*>(a.w_pre + column(c));
+        }
+        if (u < units) request_rest(u);
+        float q = 0.f;
+#pragma unroll
+        for (int c = 0; c < KC; ++c)
+#pragma unroll
+          for (int e = 0; e < 4; ++e) q += (float)v4[c][e] * (float)v4[c][e];
+        const float rstd = rsqrt_refined(vy_wave_sum(q) / (float)a.n + a.eps);
+#pragma unroll
+        for (int c = 0; c < KC; ++c) {
+          bf16x4 o;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) o[e] = (bf16)((float)v4[c][e] * rstd * w4[c][e]);
+          *reinterpret_cast<bf16x4*>(hs + row * K + column(c)) = o;
+        }
+      }
+    } else if (leads) {
       const int m = row;
       float v[KC][4], g[KC][4], b[KC][4];
       if constexpr (PRO == LAYER || PRO == PARTS) {
@@ -290,7 +344,7 @@ void go_rows(const Args& a, hipStream_t st) {
   // every workgroup redoes the operand rows, so there are no more of them than fit on the chip at once (by registers): the waves of
   // wide products loop, with the next rows' weights requested ahead
   const int most = PRO != STREAM ? 2048 : KC <= 4 ? 1024 : 512;
-  const int grid = (units + 3) / 4 < most ? (units + 3) / 4 : most;
+  const int grid = ((units + 3) / 4 < most ? (units + 3) / 4 : most) + (PRO == RMS && a.cache ? 1 : 0);
   if (a.M == 1) hipLaunchKernelGGL((few_kernel<EPI, PRO, 1, KC>), dim3(grid), dim3(256), 0, st, a);
   else if (a.M == 2) hipLaunchKernelGGL((few_kernel<EPI, PRO, 2, KC>), dim3(grid), dim3(256), 0, st, a);
   else hipLaunchKernelGGL((few_kernel<EPI, PRO, 4, KC>), dim3(grid), dim3(256), 0, st, a);
@@ -303,6 +357,7 @@ bool few_k(int epi, int pro, int64_t K) {
   const int kc = (int)(K / 256);
   if (pro == PLAIN) return epi == QKV ? kc >= 2 && kc <= 4 : epi == STORE && (kc == 2 || kc == 3 || kc == 4 || kc == 8 || kc == 12 || kc == 16);
   if (pro == LAYER) return epi != GATED && kc >= 2 && kc <= 4;
+  if (pro == RMS) return epi == STORE && (kc == 2 || kc == 4);
   if (pro == PARTS) return epi == STORE && kc >= 2 && kc <= 4;
   return epi != QKV && (kc == 4 || kc == 8);
 }
@@ -314,6 +369,7 @@ int few_go(int epi, int pro, const Args& a, int64_t K, hipStream_t st) {
   if (pro == PLAIN && epi == QKV) switch (kc) { FEW(QKV, PLAIN, 2); FEW(QKV, PLAIN, 3); FEW(QKV, PLAIN, 4); }
   else if (pro == PLAIN) switch (kc) { FEW(STORE, PLAIN, 2); FEW(STORE, PLAIN, 3); FEW(STORE, PLAIN, 4); FEW(STORE, PLAIN, 8); FEW(STORE, PLAIN, 12); FEW(STORE, PLAIN, 16); }
   else if (pro == LAYER && epi == QKV) switch (kc) { FEW(QKV, LAYER, 2); FEW(QKV, LAYER, 3); FEW(QKV, LAYER, 4); }
+  else if (pro == RMS) switch (kc) { FEW(STORE, RMS, 2); FEW(STORE, RMS, 4); }
   else if (pro == PARTS) switch (kc) { FEW(STORE, PARTS, 2); FEW(STORE, PARTS, 3); FEW(STORE, PARTS, 4); }
   else if (pro == LAYER) switch (kc) { FEW(STORE, LAYER, 2); FEW(STORE, LAYER, 3); FEW(STORE, LAYER, 4); }
   else if (epi == STORE) switch (kc) { FEW(STORE, STREAM, 4); FEW(STORE, STREAM, 8); }
@@ -326,7 +382,7 @@ int few_go(int epi, int pro, const Args& a, int64_t K, hipStream_t st) {
 }  // namespace vy_few
 
 // test aid, not part of include/vyom_hip.h: one product by itself on contiguous rows.  a, b: gamma and beta of LAYER and PARTS (bf16), w_post and
-// w_pre of STREAM (fp32); PARTS: n shares s_in [n][M][K] and their bias `residual`; y: QKV's queries [M][nq], k and v [M][nkv]
+// w_pre of STREAM (fp32); PARTS: n shares s_in [n][M][K] and their bias `residual`; RMS: weights sin_tab; y: QKV's queries [M][nq], k and v [M][nkv]
 extern "C" int vy_debug_few(int epi, int pro, const void* x, const void* a, const void* b, const float* s_in, float* s_out, void* h, int n,
                             int rms, float eps, const void* w, const void* bias, int act, float act_arg, const void* residual, void* y,
                             int64_t ldy, void* k, void* v, int nq, int nkv, const float* cos_tab, const float* sin_tab, int pos, int M,
@@ -336,6 +392,13 @@ extern "C" int vy_debug_few(int epi, int pro, const void* x, const void* a, cons
   if (pro == vy_few::PARTS) {
     f.parts = s_in; f.n_parts = n; f.x_bias = (const bf16*)residual;
     residual = nullptr;
+  }
+  if (pro == vy_few::RMS) {
+    if (k) {   // rows v [M][K] of nkv columns, weights b, into row cos_tab[m] (integers; below nq) of k [M][2][nkv]
+      f.kv = (const bf16*)v; f.w_kv = (const float*)b; f.n_kv = f.np_kv = nkv; f.cache = (bf16*)k; f.k_ss = 2 * (int64_t)nkv; f.k_st = nkv;
+      f.cap = nq; f.ring = 0; f.start = (const int*)cos_tab;
+    }
+    b = sin_tab;
   }
   if (pro == vy_few::LAYER || pro == vy_few::PARTS) { f.ln_g = (const bf16*)a; f.ln_b = (const bf16*)b; }
   else { f.w_post = (const float*)a; f.w_pre = (const float*)b; }
