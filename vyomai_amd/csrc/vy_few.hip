@@ -106,7 +106,8 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   };
   // what the epilogue reads besides the product, one lane per (weight row, operand row), and none of it hangs on the product: requested
   // behind the norm's operands (behind the norm, the position and then the rotary factors were two more trips to memory: QKV of 768 columns
-  // 3.86 -> 3.68 us)
+  // 3.86 -> 3.68 us).  STREAM has a bias at most, which is there before the product is: requested ahead of its norm it
+  // cost 0.35 us a product (the 16 of a decoder of width 1024 and 8 layers, on average: 5.82 -> 6.16)
   const int er = R == 1 || lane >= R * MR ? 0 : lane / MR, em = R == 1 ? lane : lane % MR;
   float e_bias = 0.f, e_other = 0.f, e_res = 0.f, e_cos = 0.f, e_sin = 0.f;
   int pos = 0;
@@ -137,7 +138,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   }
   const int row = wave / SHARES;   // of the operand, this wave's
   const bool leads = wave % SHARES == 0 && row < a.M;
-  if (u < units && (PRO == PLAIN || !leads)) request_rest(u);
+  if (u < units && PRO != STREAM && (PRO == PLAIN || !leads)) request_rest(u);
 
   if constexpr (PRO != PLAIN) {
     if (a.advance && blockIdx.x == 0)
@@ -236,7 +237,6 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
           if (a.w_post) p4[c] = *reinterpret_cast<const f32x4*>(a.w_post + col);
           if (a.w_pre) g4[c] = *reinterpret_cast<const f32x4*>(a.w_pre + col);
         }
-        if (u < units) request_rest(u);
         if (a.x) {
           float mean = 0.f, rstd = 1.f, y[KC][4];
 #pragma unroll
@@ -278,6 +278,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   }
 
   for (; u < units; u += step) {
+    if constexpr (PRO == STREAM) request_rest(u);
     const bool mine = lane < R * MR && em < a.M;
     const int n = row_of(u, er);
     const bool real = mine && (EPI != STORE || u * R + er < a.N);
@@ -292,7 +293,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
     for (int p = 0; p < P; ++p) wv[p] = w[p];
     if (u + step < units) {
       request(u + step);
-      request_rest(u + step);
+      if constexpr (PRO != STREAM) request_rest(u + step);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
