@@ -14,7 +14,11 @@ template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3
 
 // acc[t][j] = 16 rows ws[t] x 16 rows xs[j] over the wave's share of K; a lane's pointers are its row (lane & 15) + 8 (lane >> 4).
 // D: a lane owns row lane & 15 of X and rows 4 (lane >> 4) .. + 3 of W.
-template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>>
+// APART: whole passes over K in code of their own, whose loads have no conditions.  dense() gains by it (decoder of width 2048, steps of 5 / 32
+// sequences 602 -> 572 us, 756 -> 690); the experts, whose kernels hold a dense product's code as well, lose (2 layers of width 2048 and 64
+// experts, 16 / 32 sequences: 321 -> 329 us, 411 -> 416).  Behind whole passes each load has a condition of its own: all of a step's
+// behind one branch came one step after the other (16 sequences 338 us, 32 433).
+template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>, bool APART = true>
 __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB]) {
   const int kq = (threadIdx.x & 63) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -35,19 +39,22 @@ __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* c
 #pragma unroll
       for (int j = 0; j < MB; ++j) x[u][j] = *reinterpret_cast<const bf16x8*>(xs[j] + k);
     };
-    // (all of the pass inside K, the common case: loads behind conditions of their own come one branch after the other)
-    if (k0 + 64 * NW * ((U - 1) >> 1) + 64 <= K) {
+    if (APART && k0 + 64 * NW * ((U - 1) >> 1) + 64 <= K) {
 #pragma unroll
       for (int u = 0; u < U; ++u) request(u, k0 + 64 * NW * (u >> 1) + 32 * (u & 1));
     } else {
 #pragma unroll
       for (int u = 0; u < U; ++u) {
         const int k = k0 + 64 * NW * (u >> 1) + 32 * (u & 1);
+        const bool in = k + 8 * kq < K;
 #pragma unroll
-        for (int t = 0; t < NT; ++t) w[u][t] = zero8;
+        for (int t = 0; t < NT; ++t) {
+          const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
+          if constexpr (ONCE) w[u][t] = in ? __builtin_nontemporal_load(at) : zero8;
+          else w[u][t] = in ? *at : zero8;
+        }
 #pragma unroll
-        for (int j = 0; j < MB; ++j) x[u][j] = zero8;
-        if (k + 8 * kq < K) request(u, k);
+        for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
       }
     }
 #pragma unroll
@@ -65,7 +72,7 @@ __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* 
                                        f32x4* red) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  share<NT, MB, ONCE, NW>(ws, xs, K, acc);
+  share<NT, MB, ONCE, NW, STEPS<NT, MB>, false>(ws, xs, K, acc);
   __syncthreads();   // (red may still be read from the pass before)
   if (wave)
 #pragma unroll
