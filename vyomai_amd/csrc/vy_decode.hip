@@ -992,13 +992,18 @@ int vy_dec_gemv1_qkv(const void* x, const void* w, const void* bias, void* q, vo
   return VY_OK;
 }
 
+// switches of the decode steps' attention, read at the first step: VY_DEC_ATTN = 0: the general kernel; VY_DEC_ATTN_NT = 0 / 1: keys and
+// values never / always streamed; VY_DEC_ATTN_GQ = 0: a workgroup for every query head
+static int dec_attn_on() { static const int v = [] { const char* e = getenv("VY_DEC_ATTN"); return e ? atoi(e) : 1; }(); return v; }
+static int dec_attn_nt() { static const int v = [] { const char* e = getenv("VY_DEC_ATTN_NT"); return e ? atoi(e) : -1; }(); return v; }
+static int dec_attn_gq() { static const int v = [] { const char* e = getenv("VY_DEC_ATTN_GQ"); return e ? atoi(e) : 1; }(); return v; }
+
 // single-query attention of the decode steps.  smax: an upper bound of the context length when it is read on the
 // device (pos_dev), else S.  Returns VY_ERR_UNSUPPORTED for shapes the resident-context kernel does not cover.
 int vy_dec_attn(const void* q, int64_t q_sb, const void* k, const void* v, int64_t c_sb, int64_t c_sh, int64_t c_sl, void* out,
                 int64_t o_sb, int B, int h, int hk, int64_t S, int64_t smax, const int* pos_dev, int dh, float scale,
                 hipStream_t st) {
-  static const int on = [] { const char* e = getenv("VY_DEC_ATTN"); return e ? atoi(e) : 1; }();
-  if (!on || (dh != 64 && dh != 256) || hk < 1 || h % hk || S < 1 || c_sl % 8 || c_sh % 8 || c_sb % 8 || q_sb % 8 ||
+  if (!dec_attn_on() || (dh != 64 && dh != 256) || hk < 1 || h % hk || S < 1 || c_sl % 8 || c_sh % 8 || c_sb % 8 || q_sb % 8 ||
       ((uintptr_t)q % 16) || ((uintptr_t)k % 16) || ((uintptr_t)v % 16))
     return VY_ERR_UNSUPPORTED;
   DecAttnArgs a{};
@@ -1009,13 +1014,11 @@ int vy_dec_attn(const void* q, int64_t q_sb, const void* k, const void* v, int64
   // d = 768 decoder, whose 170 MB of weights can stay in the Infinity Cache if the K/V stream does not push them out: nt is
   // ahead at every batch (B = 1 / 2 / 4 / 8 / 32: 349 / 360 / 380 / 368 / 485 us against 355 / 363 / 388 / 399 / 515); on
   // configs[4] (0.3 MB per layer, 5.8 GB of weights streaming through anyway) the default policy is 5 % ahead.
-  // VY_DEC_ATTN_NT = 0 / 1 forces it
-  static const int nt_env = [] { const char* e = getenv("VY_DEC_ATTN_NT"); return e ? atoi(e) : -1; }();
+  const int nt_env = dec_attn_nt(), gq_env = dec_attn_gq();
   const int64_t layer_bytes = 2ll * B * hk * (pos_dev ? smax : S) * dh * 2;
   const bool nt = nt_env < 0 ? layer_bytes > (1ll << 20) : nt_env != 0;
   int rc;
   // grouped-query heads of a 64-wide model: the query heads of one KV head in one workgroup (K/V read once, not h / hk times)
-  static const int gq_env = [] { const char* e = getenv("VY_DEC_ATTN_GQ"); return e ? atoi(e) : 1; }();
   const int rep = h / hk;
   if (dh == 64 && gq_env && nt && rep == 2) rc = dec_attn_go<64, 8, true, 2>(a, B, bound, st);
   else if (dh == 64 && gq_env && nt && rep == 3) rc = dec_attn_go<64, 8, true, 3>(a, B, bound, st);
@@ -1031,8 +1034,9 @@ int vy_dec_attn(const void* q, int64_t q_sb, const void* k, const void* v, int64
 // part[returned][B][h 64], in `room` bytes, to be added up.  0: other sizes.
 int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, int64_t c_sh, int64_t c_sl, const void* wo, float* part,
                     int64_t room, int B, int h, int hk, int64_t S, int64_t smax, const int* pos_dev, float scale, hipStream_t st) {
-  if (hk < 1 || h % hk || S < 1 || c_sl % 8 || c_sh % 8 || c_sb % 8 || ((uintptr_t)q % 16) || ((uintptr_t)k % 16) || ((uintptr_t)v % 16) ||
-      ((uintptr_t)wo % 16))
+  // (streamed keys are not for this kernel, whose workgroups share them through L2)
+  if (!dec_attn_on() || dec_attn_nt() > 0 || hk < 1 || h % hk || S < 1 || c_sl % 8 || c_sh % 8 || c_sb % 8 || ((uintptr_t)q % 16) ||
+      ((uintptr_t)k % 16) || ((uintptr_t)v % 16) || ((uintptr_t)wo % 16))
     return 0;
   DecAttnArgs a{};
   a.q = (const bf16*)q; a.q_sb = h * 64; a.k = (const bf16*)k; a.v = (const bf16*)v; a.c_sb = c_sb; a.c_sh = c_sh; a.c_sl = c_sl;
@@ -1040,7 +1044,7 @@ int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, i
   // One sequence: a workgroup per query head also where several share a key head (12 layers of 768, 4 key/value heads, 24 steps and
   // their prompt: behind 60 tokens 6113 against 6190 us, behind 500 6580 and 6990); more: one for all that share it, whose fewer shares the next
   // product adds up sooner (4 sequences behind 30 tokens 9480 and 8990).
-  const int rep = B > 1 && h / hk >= 2 && h / hk <= 4 ? h / hk : 1, units = h / rep;
+  const int rep = B > 1 && dec_attn_gq() && h / hk >= 2 && h / hk <= 4 ? h / hk : 1, units = h / rep;
   if (units > 16 || (int64_t)units * B * a.d * 4 > room) return 0;
   if (rep == 4 && (pos_dev ? smax : S) > 640) return 0;   // (longer contexts in registers beside four heads' rows of wo: spills)
   // rows of wo in as few passes as leave at most a workgroup a CU (h blocks of 64 rows)
