@@ -1031,7 +1031,7 @@ int vy_dec_attn(const void* q, int64_t q_sb, const void* k, const void* v, int64
 }
 
 // internal (vy_runtime.hip): attention of few sequences' steps and its output projection wo [h 64][h 64]: fp32 shares
-// part[returned][B][h 64], in `room` bytes, to be added up.  0: other sizes.
+// part[returned][B][h 64], in `room` bytes, to be added up.  0: other sizes; negative: an error.
 int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, int64_t c_sh, int64_t c_sl, const void* wo, float* part,
                     int64_t room, int B, int h, int hk, int64_t S, int64_t smax, const int* pos_dev, float scale, hipStream_t st) {
   // (streamed keys are not for this kernel, whose workgroups share them through L2)
@@ -1057,5 +1057,7 @@ int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, i
   else if (rep == 3) rc = dec_attn_go<64, 8, false, 3, true>(a, B, bound, st);
   else if (rep == 4) rc = dec_attn_go<64, 8, false, 4, true>(a, B, bound, st);
   else rc = dec_attn_go<64, 8, false, 1, true>(a, B, bound, st);
-  return rc ? 0 : units;
+  if (rc) return 0;
+  VY_CHECK_LAUNCH("vy_dec_attn_out");
+  return units;
 }

@@ -134,6 +134,7 @@ static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos,
                            ? vy_dec_attn_out(q, L.kcache, L.vcache, L.c_sb, L.c_sh, L.c_sl, L.wo, part, part_bytes, B, h, hk, pos + 1,
                                              L.c_sh / (L.c_sl ? L.c_sl : 1), pos_dev, 0.125f, st)
                            : 0;
+    if (shares < 0) return shares;
     if (shares) {
       f.parts = part; f.n_parts = shares; f.x_bias = (const bf16*)L.bo; f.x = cur; f.ldx = d;
       if ((rc = few_go(STORE, PARTS, f, d, st))) return rc;
