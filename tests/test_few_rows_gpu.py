@@ -160,3 +160,16 @@ def test_hidden_rows_at_any_address():
                       ops._raw_stream())
             got = room[off:off + 2 * 768].view(2, 768).float()
             assert (got - want.float()).norm() <= 18 * 2.0 ** -8 * want.float().norm() and room[:off].eq(0).all() and room[off + 1536:].eq(0).all()
+
+
+def test_what_four_sequences_cost():
+    """Width 1024: a step of four takes 1.2 times what a step of one takes; with the output projection inside the attention, whose sixteen
+    heads' shares every workgroup of the next product adds up, 1.65 times."""
+    from tests.test_decode_products_gpu import microseconds
+    us = {}
+    for B in (1, 4):
+        cfg, m = decoder(1024, "rope", None, BF, layers=6)
+        plan, cache = _plan(cfg, m, B, BF)
+        x, hidden = torch.randn(B, 1024, device=DEV).to(BF), torch.empty(B, 1024, dtype=BF, device=DEV)
+        us[B] = microseconds(lambda: plan._launch(x.data_ptr(), 60, None, hidden.data_ptr(), None), 4)
+    assert us[4] <= 1.4 * us[1], us

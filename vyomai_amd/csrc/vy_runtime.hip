@@ -96,8 +96,25 @@ static bool few_operands(const vy_decode_plan* p, const void* x, const void* hid
   return given && all % 16 == 0 && (!logits || p->vocab > 0);
 }
 
+// Does the output projection go into the attention (vy_dec_attn_out)?  That saves a launch, 1.2 us of a layer, but every workgroup of the
+// feed-forward's first product then adds up the heads' fp32 shares -- h B d of them, out of L2 -- and query heads that share a key head are
+// attended to by one workgroup, which three and four of them only repay where their keys are streamed otherwise (kv_bytes: one layer's keys
+// and values, against the 1 MB above which vy_dec_attn streams them).  A step with the projection inside / by itself, 12 layers, us:
+//   one sequence: 768 columns 196 / 209 behind 60 tokens, 212 / 245 behind 500, 1024 columns level
+//   two: 512 columns 181 / 198, 768 223 / 225 and 240 / 259, 1024 294 / 261;   four: 512 210 / 216, 768 268 / 250, 1024 406 / 298
+//   three query heads a key head, 768 columns: two sequences 219 / 221 behind 60, 250 / 240 behind 500, four 250 / 243 and 283 / 298; four
+//   heads: two sequences 230 / 220, behind 500 266 / 240, three behind 500 293 / 306; six: three sequences 251 / 240, behind 700 275 / 298
+bool vy_dec_shares_pay(int B, int h, int hk, int64_t kv_bytes) {
+  const int d = 64 * h, rep = hk > 0 ? h / hk : 1, units = rep >= 2 && rep <= 4 ? hk : h;
+  const bool streamed = kv_bytes > (1 << 20);
+  if (B == 1) return true;
+  if (d > 768) return false;   // (the product's sums of two and more rows of 1024 columns: registers)
+  if (rep == 3 || rep == 4) return streamed;
+  return units * B * d * 4 <= (72 << 10) || (rep > 4 && streamed);
+}
+
 // The step of 1 to 4 sequences on the kernels of vy_few.hip: four launches per layer -- LayerNorms inside the products behind them, the
-// output projection inside the attention (longer contexts: five, the projection by itself).
+// output projection inside the attention -- or five, the projection by itself (vy_dec_shares_pay; longer contexts).
 static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos, const int32_t* pos_dev, void* hidden_out, void* logits,
                             int64_t ldv, hipStream_t st) {
   using namespace vy_few;
@@ -130,9 +147,10 @@ static int few_decoder_step(const vy_decode_plan* p, const void* x, int64_t pos,
     Args f{};
     f.M = B; f.ln_g = (const bf16*)L.ln1_w; f.ln_b = (const bf16*)L.ln1_b; f.eps = p->eps_attn;
     f.w = (const bf16*)L.w1; f.bias = (const bf16*)L.b1; f.N = p->ffn; f.act = p->act; f.y = mid; f.ldy = p->ffn;
-    const int shares = few_k(STORE, PARTS, d) && (uintptr_t)L.bo % 8 == 0
-                           ? vy_dec_attn_out(q, L.kcache, L.vcache, L.c_sb, L.c_sh, L.c_sl, L.wo, part, part_bytes, B, h, hk, pos + 1,
-                                             L.c_sh / (L.c_sl ? L.c_sl : 1), pos_dev, 0.125f, st)
+    const int64_t smax = L.c_sh / (L.c_sl ? L.c_sl : 1), kv_bytes = 2ll * B * hk * (pos_dev ? smax : pos + 1) * 64 * 2;
+    const int shares = few_k(STORE, PARTS, d) && (uintptr_t)L.bo % 8 == 0 && vy_dec_shares_pay(B, h, hk, kv_bytes)
+                           ? vy_dec_attn_out(q, L.kcache, L.vcache, L.c_sb, L.c_sh, L.c_sl, L.wo, part, part_bytes, B, h, hk, pos + 1, smax,
+                                             pos_dev, 0.125f, st)
                            : 0;
     if (shares < 0) return shares;
     if (shares) {
