@@ -1,0 +1,28 @@
+"""Which kernel a product of more than 32 rows takes (pick_tiling of vyomai_amd/csrc/vy_gemm.hip), without a GPU."""
+import ctypes as C
+
+import pytest
+
+KINDS = ["256x256", "256x192", "256x128", "128x128", "64", "64 twice", "64 many", "128 split", "256 split", "320 split"]
+
+
+def tiling(M, N, K, ws=64 << 20):
+    from vyomai_amd import _lib
+    f = _lib.load().vy_debug_tiling
+    f.argtypes, f.restype = [C.c_int64] * 4, C.c_int
+    t = f(M, N, K, ws)
+    return KINDS[t % 16], t // 16
+
+
+#: rows, columns, K; slices of K; kernels within 5 % of the fastest (two builds of it on one box, weights out of the Infinity Cache)
+@pytest.mark.parametrize("M,N,K,slices,fastest", [
+    (257, 2048, 6144, 16, {"320 split"}), (290, 2048, 6144, 16, {"320 split"}), (320, 2048, 6144, 16, {"320 split"}),
+    (512, 1152, 4304, 8, {"128 split"}), (400, 1152, 4304, 8, {"128 split"}), (640, 1152, 4304, 8, {"128 split"}),
+    (1300, 1152, 4304, 4, {"128 split"}), (1024, 1152, 4304, 4, {"128 split"}), (33, 512, 1536, 8, {"128 split"}),
+    (100, 512, 1536, 8, {"128 split"}), (800, 1024, 6144, 8, {"128 split"}), (40, 3456, 3584, 14, {"128 split"}),
+    (39, 256, 1664, 7, {"128 split"}), (4096, 768, 2304, 2, {"64"}), (4096, 768, 3072, 2, {"64", "128 split"}),
+    (512, 768, 768, 4, {"64 twice"}), (512, 768, 3072, 16, {"64 many"}), (1000, 768, 3072, 8, {"64 many"}), (700, 1024, 1024, 8, {"64 many"}),
+    (700, 1152, 4304, 8, {"128 split"})])
+def test_kernel_is_a_fast_one(M, N, K, slices, fastest):
+    kind, S = tiling(M, N, K)
+    assert S == slices and kind in fastest

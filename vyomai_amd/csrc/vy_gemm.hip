@@ -31,6 +31,7 @@ int vy_rope_qk(void* q, int64_t q_sb, int64_t q_sh, int64_t q_sl, int hq, void* 
                int64_t k_sl, int hk, const float* cos_tab, const float* sin_tab, int64_t pos0, int64_t B, int64_t L, int dh,
                int dtype, hipStream_t st);
 
+#include <math.h>
 #include <stdlib.h>
 #include <mutex>
 
@@ -1679,10 +1680,12 @@ inline Scratch splitk_ws(hipStream_t st) {
 // own rate: 8192 x 2048 with K = 12288 is 352 tiles of 256 x 192 -- two rounds, the second a third full, 459 us -- or 256 tiles of
 // 256 x 256: 313 us; 8000 x 1024, K = 6144: 124 us on 256 x 192, 152 us on 256 x 256, 100 us on 256 x 128 (250 tiles).  So the
 // launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below; the constants
-// are fits to launches of 130 shapes from 40 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
-// output alone and so moves no choice), up to 4096 rows in graphs that walk through 170 MB of weights, as a model's layers do: products
-// that find their weights in L2, as a loop over one product does, made one launch look shorter than two groups in it.  90 shapes of
-// 40 to 4096 rows: the fastest kernel for 83, within 10 % of it for the others.
+// are fits to launches of 40 shapes from 48 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
+// output alone and so moves no choice), where K is sliced (up to 4096 rows) to 1100 of 33 to 4096 rows, 64 to 8192 columns and K = 256 to
+// 8192, each on all kernels that take it, in graphs that walk through 200 MB of weights, as a model's layers do: products that find
+// their weights in L2, as a loop over one product does, made one launch look shorter than two groups in it.  The kernel chosen takes
+// 0.2 % longer than the fastest on average, over 8 % for 5 of them.  (Fitted to 90 shapes, 8 % for 45: 300 x 2048, K = 6144, 31.5 us in two
+// groups, 25.6 with K over workgroups; 512 x 1152, K = 4304, 26.9 and 20.8.)
 // ------------------------------------------------------------------------------------------
 enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_64x64_MANY, T_128x128_SPLIT, T_256x128_SPLIT, T_320x128_SPLIT };
 constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 64, 128, 256, 320};
@@ -1692,9 +1695,11 @@ struct Tiling { TileKind kind; int slices; };
 
 // what a shape costs on a tile, S slices of K added up
 template <TileKind kind>
-inline double tile_cost(int64_t M, int64_t N, int KT, int S, int chip) {
+inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
   const int64_t tiles = vy_cdiv(M, TILE_M[kind]) * vy_cdiv(N, TILE_N[kind]);
+  const int KT = (int)vy_cdiv(K, BK);
   const double load = (double)tiles / chip;
+  const bool apart = K % BK != 0;   // (rows that start inside a 128-byte line: a stage touches more of them)
   // `fixed` per round, `stage` per stage of a round; the stages of a last round that leaves CUs idle run up to 30 % faster
   auto one_shot = [&](int per_cu, double launch, double fixed, double stage) {
     const double r = load / per_cu, whole = (double)(int64_t)r, part = r - whole;
@@ -1705,16 +1710,21 @@ inline double tile_cost(int64_t M, int64_t N, int KT, int S, int chip) {
     case T_256x192: return one_shot(1, 2.3, 5.5, 1.30);
     case T_256x128: return one_shot(1, 4.5, 4.1, 0.97);
     case T_128x128: return load <= 1 ? 8.5 + 0.72 * KT : one_shot(2, 3.5, 5.0, 1.0);     // (two of them share a CU)
-    case T_64x64: return (S > 1 ? 4.1 : 3.2) + (load > 1 ? 0.8 : 0.0) + KT * (0.25 * load > 0.335 ? 0.25 * load : 0.335);
-    case T_64x64_TWICE: case T_64x64_MANY: return 1.2 + (double)(int64_t)(load + 0.999) * (2.0 + 0.245 * KT + 0.13 * (S - 2));
-    default: {   // K over several workgroups: the partial sums' way through memory (about 6 TB/s there and back) and a second launch
-      const double bytes = 4.0 * S * tiles * TILE_M[kind] * TILE_N[kind];
+    case T_64x64: {
+      if (S == 1) return 3.2 + (load > 1 ? 0.8 : 0.0) + KT * (0.25 * load > 0.335 ? 0.25 * load : 0.335);
+      const double n = (double)vy_cdiv(tiles, (int64_t)chip), stage = 0.238 * n - 0.204;   // the fullest CU holds n (up to three at once)
+      return 4.0 + KT * (stage > 0.374 ? stage : 0.374) * (apart && n > 1 ? 1.3 : 1.0);
+    }
+    case T_64x64_TWICE: case T_64x64_MANY:
+      return 1.75 + (double)vy_cdiv(tiles, (int64_t)chip) * (2.2 + 0.238 * KT * (apart ? 1.25 : 1.0) + 0.13 * (S - 2));
+    default: {   // K over several workgroups: the partial sums' way through memory -- Infinity Cache for most of it -- and a second launch
+      const double padded = 4e-6 * S * tiles * TILE_M[kind] * TILE_N[kind], sums = 5.0 + 1.34 * sqrt(padded) + 0.18 * 4e-6 * S * M * N;
       const int per = (KT + S - 1) / S;
-      const double sums = 7.5 + 2 * bytes / 6e6;
-      if (kind != T_128x128_SPLIT) return sums + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * (1.2 * TILE_M[kind] / 256);
-      if (tiles * S <= chip) return sums + 0.72 * per;
+      if (kind != T_128x128_SPLIT) return sums + 1.6 + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * (0.688 * TILE_M[kind] / 256);
+      const double stage = per * (apart ? 1.16 : 1.0);
+      if (tiles * S <= chip) return sums + 0.66 * stage;
       const double r = (double)(tiles * S) / (2 * chip), whole = (double)(int64_t)r, part = r - whole;   // (two of them share a CU)
-      return sums + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * 0.95 * per;
+      return sums + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * 0.82 * stage;
     }
   }
 }
@@ -1749,25 +1759,25 @@ inline int sum_slices(int64_t M, int64_t N, int64_t K) {
 }
 
 inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes) {
-  const int KT = (int)vy_cdiv(K, BK), S = sum_slices(M, N, K);
+  const int S = sum_slices(M, N, K);
   Tiling best{T_64x64, S};
   double least = 1e30;
   auto offer = [&](TileKind kind, double us) {
     if (us < least) { least = us; best.kind = kind; }
   };
-  offer(T_64x64, tile_cost<T_64x64>(M, N, KT, S, chip));
+  offer(T_64x64, tile_cost<T_64x64>(M, N, K, S, chip));
   if (S == 1) {
-    offer(T_256x256, tile_cost<T_256x256>(M, N, KT, S, chip));
-    offer(T_256x192, tile_cost<T_256x192>(M, N, KT, S, chip));
-    offer(T_256x128, tile_cost<T_256x128>(M, N, KT, S, chip));
-    offer(T_128x128, tile_cost<T_128x128>(M, N, KT, S, chip));
+    offer(T_256x256, tile_cost<T_256x256>(M, N, K, S, chip));
+    offer(T_256x192, tile_cost<T_256x192>(M, N, K, S, chip));
+    offer(T_256x128, tile_cost<T_256x128>(M, N, K, S, chip));
+    offer(T_128x128, tile_cost<T_128x128>(M, N, K, S, chip));
     return best;
   }
-  if (S <= 4) offer(T_64x64_TWICE, tile_cost<T_64x64_TWICE>(M, N, KT, S, chip));
-  else offer(T_64x64_MANY, tile_cost<T_64x64_MANY>(M, N, KT, S, chip));
-  if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, tile_cost<T_128x128_SPLIT>(M, N, KT, S, chip));
-  if (split_fits<T_256x128_SPLIT>(M, N, S, ws_bytes)) offer(T_256x128_SPLIT, tile_cost<T_256x128_SPLIT>(M, N, KT, S, chip));
-  if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, tile_cost<T_320x128_SPLIT>(M, N, KT, S, chip));
+  if (S <= 4) offer(T_64x64_TWICE, tile_cost<T_64x64_TWICE>(M, N, K, S, chip));
+  else offer(T_64x64_MANY, tile_cost<T_64x64_MANY>(M, N, K, S, chip));
+  if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, tile_cost<T_128x128_SPLIT>(M, N, K, S, chip));
+  if (split_fits<T_256x128_SPLIT>(M, N, S, ws_bytes)) offer(T_256x128_SPLIT, tile_cost<T_256x128_SPLIT>(M, N, K, S, chip));
+  if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, tile_cost<T_320x128_SPLIT>(M, N, K, S, chip));
   return best;
 }
 
@@ -2713,6 +2723,13 @@ int qkv_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void*
 }
 
 }  // namespace
+
+// test aid, not part of include/vyom_hip.h: the kernel (TileKind) of a product of more than 32 rows with ws_bytes of workspace, and 16 times
+// the slices of K that it adds up
+extern "C" int vy_debug_tiling(int64_t M, int64_t N, int64_t K, int64_t ws_bytes) {
+  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes);
+  return (int)t.kind + 16 * t.slices;
+}
 
 extern "C" int vy_linear_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,
                              const void* residual, int64_t ldr, void* y, int64_t ldy, void* pre_out,
