@@ -59,6 +59,17 @@ def test_activation_and_its_saved_derivative_on_small_tiles(M, N, K):
     assert ((y.double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()       # 1e-5: the epilogue's fast erf
 
 
+def test_what_a_residual_behind_an_activation_costs():
+    """Requested ahead like a residual by itself, it costs as much: 1.02 times (requested where it is added: 1.13)."""
+    from tests.test_decode_products_gpu import microseconds
+    from vyomai_amd import ops, _lib
+    M, N, K = 30500, 768, 768
+    x, w, b, r = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5), rnd(N, seed=3), rnd(M, N, seed=4)
+    y = torch.empty(M, N, dtype=BF, device=DEV)
+    plain, behind = (microseconds(lambda: ops.linear(x, w, b, act=a, residual=r, out=y), 10) for a in (_lib.ACT_NONE, _lib.ACT_RELU2))
+    assert behind <= 1.08 * plain, (plain, behind)
+
+
 @pytest.mark.parametrize("B,L,h,hk", [(3, 37, 12, 12), (1, 65, 12, 4), (5, 333, 12, 4), (2, 1000, 12, 12)])
 def test_rotary_heads_on_small_tiles(B, L, h, hk):
     from vyomai_amd import ops

@@ -392,13 +392,14 @@ template <int BM, int BN, int WGM, int WGN, bool MF16> struct AccTile {
 
 // The second operand of a plain epilogue -- residual, or the pre-activation of a dgrad -- in the registers of the threads that will
 // combine it (16-byte chunks tid, tid + NT, ... of the tile), requested before the accumulators are staged: loaded in the loop over the
-// chunks, every iteration waits a full memory latency for it (22 k cycles per tile against 12 k without the operand).
-constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, int ACT, bool GRAD) {
-  return EPI == 0 && (GRAD || ACT == VY_ACT_NONE) && (BM * BN == 256 * 192 || BM * BN == 64 * 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
+// chunks, every iteration waits a full memory latency for it (22 k cycles per tile against 12 k without the operand; residual behind an
+// activation, squared ReLU, 30500 x 768: K = 768 51.4 -> 46.5 us, K = 3072 147 -> 138).
+constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, bool GRAD) {
+  return EPI == 0 && (BM * BN == 256 * 192 || BM * BN == 64 * 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
 }
-template <int BM, int BN, int NW, int EPI, int ACT, bool GRAD>
+template <int BM, int BN, int NW, int EPI, bool GRAD>
 struct EpiAhead {
-  static constexpr bool ON = epi_prefetches(BM, BN, NW, EPI, ACT, GRAD);
+  static constexpr bool ON = epi_prefetches(BM, BN, NW, EPI, GRAD);
   static constexpr int ITERS = ON ? BM * BN / 8 / (64 * NW) : 1;
   bf16x8 v[ITERS];
   bool on = false;
@@ -422,7 +423,7 @@ struct EpiAhead {
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD, int PASSES = 1, bool MF16 = false>
 __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN, MF16>::type& acc, char* smem,
                                               int m0, int n0, int M, int N, const EpiPlain<bf16>& ep,
-                                              const EpiQkv<bf16>& eq, const EpiAhead<BM, BN, WGM * WGN, EPI, ACT, GRAD>& ahead = EpiAhead<BM, BN, WGM * WGN, EPI, ACT, GRAD>{},
+                                              const EpiQkv<bf16>& eq, const EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>& ahead = EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>{},
                                               const unsigned* tab = nullptr) {
   constexpr bool TAB = MF16 && act_has_table(BM, BN, EPI, ACT, GRAD);
   static_assert(!MF16 || PASSES == 1, "the 16 x 16 accumulator layout is staged in one pass");
@@ -705,7 +706,7 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
       const std::integral_constant<bool, true> whole{};
       const std::integral_constant<bool, false> ragged{};
       const bf16x8 none{};
-      if constexpr (PASSES == 1 && EpiAhead<BM, BN, WGM * WGN, EPI, ACT, GRAD>::ON) {
+      if constexpr (PASSES == 1 && EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>::ON) {
         if (ahead.on) {
 #pragma unroll
           for (int it = 0; it < ITERS; ++it) do_chunk(whole, dst, dual, pass, tid + it * NT, staged(tid + it * NT), true, ahead.v[it]);
@@ -1150,7 +1151,7 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
     xbuf = xbuf == 2 ? 0 : xbuf + 1;
     if (kt + 1 < KT) read_frags(wa[0] + (WT - wo), xa[0] + xbuf * XT, wf[0], xf[0]);
   }
-  EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
+  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
   gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
 }
@@ -1281,7 +1282,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     asm volatile("" ::: "memory");
     if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
   }
-  EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
+  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
   gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
 }
@@ -1457,7 +1458,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
         for (int i = 0; i < TN * TM; ++i) acc[i / TM][i % TM] = acc[i / TM][i % TM] + other[(s * TN * TM + i) * 256];
     __syncthreads();
   }
-  EpiAhead<BM, BN, NW, EPI, ACT, GRAD> ahead;
+  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
   gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead);
 }
