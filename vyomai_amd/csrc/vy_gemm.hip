@@ -4,7 +4,7 @@
 //   * M > 32: the tile is chosen by what the shape costs on it (pick_tiling): 256 x 256 (gemm_nt_bf16_m16_kernel, two stages),
 //     256 x 192 or 256 x 128 (gemm_nt_bf16_x3m16_kernel, X in a three-deep ring), 128 x 128 (two workgroups per CU), 64 x 64 with a
 //     three-deep ring (gemm_nt_bf16_small_kernel), or K split over workgroups (gemm_nt_bf16_m16_splitk_kernel +
-//     gemm_splitk_finish_kernel; one row tile of 256 / 320 for 128 < M <= 320); all on mfma_f32_16x16x32_bf16.
+//     gemm_splitk_finish_kernel; one row tile of 320 for 256 < M <= 320); all on mfma_f32_16x16x32_bf16.
 //     gemm_nt_bf16_kernel is the same tile family on mfma_f32_32x32x16_bf16 (A/B knob, 32 x 128 fallback);
 //   * M <= 32 (decode): weight-streaming kernels without LDS staging (gemm_skinny*), M <= 4: one wave per output column
 //     (gemv_bf16_kernel); the decode driver's straight-line versions are in vy_decode.hip;
@@ -1495,11 +1495,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_splitk_kernel
   constexpr int GX = PX / NW, GW = PW / NW;
   static_assert(GX * NW == PX && GW * NW == PW, "pieces must divide over the waves");
   constexpr int STAGE = (BM + BN) * ROWB;
-  // a slice is 2-16 stages, each a full L2 / MALL round trip: where three stages fit in the CU's 160 KiB (the 256-row
-  // all-rows tile: 3 x 48 KiB) two of them stay in flight behind the one being multiplied (counted vmcnt), so a short slice
-  // is ONE round trip deep instead of one per stage; the other tiles keep two buffers (one stage ahead)
-  constexpr int NBUF = (3 * STAGE <= 160 * 1024 && BM * BN > 128 * 128) ? 3 : 2;
-  constexpr int PIECES = GX + GW;   // LDS-DMA instructions per wave and stage
+  constexpr int NBUF = 2;
   __shared__ __attribute__((aligned(16))) char smem[NBUF * STAGE];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -1590,16 +1586,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_splitk_kernel
   if (kt0 < kt1) {   // (workgroup-uniform; an empty slice stores zeros)
     const int n = kt1 - kt0;
     stage(kt0, 0);
-    if (NBUF >= 3 && n > 1) stage(kt0 + 1, 1);
     for (int i = 0; i < n; ++i) {
-      // stage i has landed for this wave (the younger stage, if any, may still be in flight) ...
-      if (NBUF >= 3 && i + 1 < n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PIECES) : "memory");
-      else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      // stage i has landed for this wave ...
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       // ... and for every wave once the barrier is passed; every wave has also finished reading the buffer of stage i - 1,
       // which the next request overwrites
       __builtin_amdgcn_s_barrier();
       asm volatile("" ::: "memory");
-      if (i + NBUF - 1 < n) stage(kt0 + i + NBUF - 1, (i + NBUF - 1) % NBUF);
+      if (i + 1 < n) stage(kt0 + i + 1, (i + 1) % NBUF);
       const unsigned boff = (unsigned)(i % NBUF) * STAGE;
       read_frags(wa[0] + boff, xa[0] + boff, wf[0], xf[0]);
       read_frags(wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
@@ -1688,10 +1682,10 @@ inline Scratch splitk_ws(hipStream_t st) {
 // 0.2 % longer than the fastest on average, over 8 % for 5 of them.  (Fitted to 90 shapes, 8 % for 45: 300 x 2048, K = 6144, 31.5 us in two
 // groups, 25.6 with K over workgroups; 512 x 1152, K = 4304, 26.9 and 20.8.)
 // ------------------------------------------------------------------------------------------
-enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_64x64_MANY, T_128x128_SPLIT, T_256x128_SPLIT, T_320x128_SPLIT };
-constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 64, 128, 256, 320};
-constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 64, 128, 128, 128};
-constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 512, 256, 512, 512};
+enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_64x64_MANY, T_128x128_SPLIT, T_320x128_SPLIT };
+constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 64, 128, 320};
+constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 64, 128, 128};
+constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 512, 256, 512};
 struct Tiling { TileKind kind; int slices; };
 
 // what a shape costs on a tile, S slices of K added up
@@ -1721,7 +1715,7 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     default: {   // K over several workgroups: the partial sums' way through memory -- Infinity Cache for most of it -- and a second launch
       const double padded = 4e-6 * S * tiles * TILE_M[kind] * TILE_N[kind], sums = 5.0 + 1.34 * sqrt(padded) + 0.18 * 4e-6 * S * M * N;
       const int per = (KT + S - 1) / S;
-      if (kind != T_128x128_SPLIT) return sums + 1.6 + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * (0.688 * TILE_M[kind] / 256);
+      if (kind == T_320x128_SPLIT) return sums + 1.6 + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * 0.86;
       const double stage = per * (apart ? 1.16 : 1.0);
       if (tiles * S <= chip) return sums + 0.66 * stage;
       const double r = (double)(tiles * S) / (2 * chip), whole = (double)(int64_t)r, part = r - whole;   // (two of them share a CU)
@@ -1729,11 +1723,10 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     }
   }
 }
-// may partial sums of S slices on these tiles lie in `ws` bytes?  128 < M <= 320: one row tile may hold every row, so that a weight
-// crosses L2 -> LDS once
+// may partial sums of S slices on these tiles lie in `ws` bytes?  256 < M <= 320: one row tile may hold every row, so that a weight
+// crosses L2 -> LDS once (three row tiles of 128: 300 x 2048, K = 6144, 30.8 us, one of 320 25.4.  Two of 128 are as fast as one of 256: 115 shapes)
 template <TileKind kind>
 inline bool split_fits(int64_t M, int64_t N, int S, int64_t ws) {
-  if (kind == T_256x128_SPLIT && (M <= 128 || M > 256)) return false;
   if (kind == T_320x128_SPLIT && (M <= 256 || M > 320)) return false;
   return 4 * S * vy_cdiv(M, TILE_M[kind]) * vy_cdiv(N, TILE_N[kind]) * TILE_M[kind] * TILE_N[kind] <= ws;
 }
@@ -1742,7 +1735,8 @@ inline bool split_fits(int64_t M, int64_t N, int S, int64_t ws) {
 // kernels below add up the same sums in the same order, so a result hangs neither on which of them the shape takes nor on a workspace
 // that the stream has or has not (in training the rounding of one product decides the noise of every gradient behind it).  Above 4096
 // rows, where the host layer registers none, K is not cut, and nothing is lost (two slices -> whole: 4200 x 1024, K = 6144, 92 -> 85 us;
-// 8192 x 512, K = 2048, 36 -> 29; 5000 x 768, K = 3072, 39.5 -> 39.8; the others of 15 shapes level or faster).
+// 8192 x 512, K = 2048, 36 -> 29; 5000 x 768, K = 3072, 39.5 -> 39.8; the others of 15 shapes level or faster).  (129 to 256 rows are cut as
+// for a row tile of 256: another number of slices would change the sums.)
 inline int sum_slices(int64_t M, int64_t N, int64_t K) {
   if (g_chains != 1 || M > 4096 || (M > 1024 && vy_cdiv(M, 256) * vy_cdiv(N, 192) >= 160)) return 1;
   const int bm = M > 128 && M <= 256 ? 256 : M > 256 && M <= 320 ? 320 : 128, target = bm == 128 ? 448 : 256;
@@ -1777,7 +1771,6 @@ inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_
   if (S <= 4) offer(T_64x64_TWICE, tile_cost<T_64x64_TWICE>(M, N, K, S, chip));
   else offer(T_64x64_MANY, tile_cost<T_64x64_MANY>(M, N, K, S, chip));
   if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, tile_cost<T_128x128_SPLIT>(M, N, K, S, chip));
-  if (split_fits<T_256x128_SPLIT>(M, N, S, ws_bytes)) offer(T_256x128_SPLIT, tile_cost<T_256x128_SPLIT>(M, N, K, S, chip));
   if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, tile_cost<T_320x128_SPLIT>(M, N, K, S, chip));
   return best;
 }
@@ -2560,7 +2553,6 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
       case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, EPI, ACT, GRAD>); break;
       case T_64x64_MANY: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, EPI, ACT, GRAD>); break;
       case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
-      case T_256x128_SPLIT: launch_split<256, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
       case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
     }
 #undef VY_TILES
