@@ -163,3 +163,44 @@ def test_bits_before_and_behind_a_smaller_product(M, N, K, act):
             call("vy_workspace_set", st, None, 0)
             ops._WS.pop(key, None)
     assert all(torch.equal(a, b) and torch.equal(a, c) for a, b, c in zip(first, behind, narrow))
+
+
+#: rows, columns, K, slices of K, kernel that adds them up inside a workgroup, kernels over which they are spread with a workspace
+SLICED = [(640, 1536, 6152, 4, "64 twice", "128 split"), (200, 384, 1096, 6, "64 many", "128 split"), (900, 576, 3080, 7, "64 many", "128 split"),
+          (900, 768, 4304, 8, "64 many", "128 split"), (257, 3072, 5000, 8, "64 many", "320 split"), (640, 384, 2056, 11, "64 many", "128 split"),
+          (900, 384, 4104, 13, "64 many", "128 split"), (65, 192, 4304, 14, "64 many", "128 split"), (640, 576, 5000, 16, "64 many", "128 split"),
+          (257, 1536, 5000, 16, "64 many", "320 split")]
+
+
+@pytest.mark.parametrize("M,N,K,S,inside,over", SLICED)
+def test_slices_inside_a_workgroup_and_over_workgroups(M, N, K, S, inside, over):
+    """Odd and even numbers of slices (the second group of waves has one less of the odd ones), last slices and stages that are short: plain,
+    behind a residual, gradient, gated and rotary products on the two kinds of kernels, bit by bit."""
+    from tests.test_product_tiles_cpu import tiling
+    from vyomai_amd import ops, _lib
+    from vyomai_amd._lib import call
+    assert tiling(M, N, K, 0) == (inside, S) and tiling(M, N, K) == (over, S)
+    x, w, b, r = rnd(M, K, seed=1), rnd(N, K, seed=2, scale=K ** -0.5), rnd(N, seed=3), rnd(M, N, seed=4)
+    heads = N // 192
+    cos, sin = ops.rope_tables(64, M, DEV)
+
+    def products():
+        out = [ops.linear(x, w), ops.linear(x, w, b, act=_lib.ACT_GELU_ERF, residual=r), ops.linear_dgrad(x, w, pre=r, act=_lib.ACT_GELU_ERF),
+               ops.linear_dgrad(x, w, add_to=r), ops.gated_linear(x, w, _lib.ACT_SILU)]
+        qkv = [torch.empty(1, heads, M, 64, dtype=BF, device=DEV) for _ in range(3)]
+        ops.qkv_rope(x.view(1, M, K), w, b, heads, heads, 64, cos, sin, 0, *qkv)
+        return out + qkv
+    st, key = torch.cuda.current_stream().cuda_stream, (torch.cuda.current_device(), torch.cuda.current_stream().cuda_stream)
+    register = ops._mid_ws
+    try:
+        spread = products()
+        ops._mid_ws = lambda rows: None
+        torch.cuda.synchronize()
+        call("vy_workspace_set", st, None, 0)
+        ops._WS.pop(key, None)
+        held = products()
+        torch.cuda.synchronize()
+    finally:
+        ops._mid_ws = register
+    close(held[0], x.double() @ w.double().T, x, w)
+    assert all(torch.equal(a, b) for a, b in zip(held, spread))
