@@ -312,6 +312,34 @@ def test_rms_norm_of_rows_and_cache_rows_beside_it(M, K, n, np_kv):
                 assert torch.isnan(cache[m, r]).all()
 
 
+@pytest.mark.parametrize("M", [1, 2, 3, 4])
+@pytest.mark.parametrize("K,n,np_kv,ring", [(512, 508, 256, 0), (512, 512, 504, 1), (1024, 1020, 512, 1), (1024, 1024, 1024, 0)])
+def test_rms_norm_of_rows_and_slots_of_a_cache(M, K, n, np_kv, ring):
+    """Slots that are not the rows' numbers, rings that have turned, three rows (a wave has none)."""
+    x, g = rnd(M, K, seed=K + n), rnd(K, seed=5, scale=0.3, dtype=torch.float32) + 1
+    x[:, n:] = 0
+    eye = torch.eye(K, dtype=BF, device=DEV)
+    kv, gk = rnd(M, K, seed=7), rnd(np_kv, seed=8, scale=0.3, dtype=torch.float32) + 1
+    cache = torch.full((M, 2, np_kv), NAN, dtype=BF, device=DEV)
+    slots = torch.tensor([[0], [1, 0], [2, 0, 1], [3, 1, 0, 2]][M - 1], dtype=torch.int32, device=DEV)
+    start = torch.tensor(([5, 2, 8, 3] if ring else [1, 0, 2, 1])[:M], dtype=torch.int32, device=DEV)     # of the slots
+    y = torch.full((M, K), NAN, dtype=BF, device=DEV)
+    go = entry("vy_debug_few", i32, i32, p, p, p, p, p, p, i32, i32, f32, p, p, i32, f32, p, p, i64, p, p, i32, i32, p, p, i32, i32, i32, i64, p)
+    assert go(STORE, 4, ptr(x), None, ptr(gk), None, None, ptr(slots), n, 1, 1e-5, ptr(eye), None, NONE, 0.0, None, ptr(y), K, ptr(cache), ptr(kv),
+              -2 if ring else 2, np_kv, ptr(start), ptr(g), 0, M, K, K, stream()) == 0
+    torch.cuda.synchronize()
+    want, e = normed(x, n, 1, g, None)
+    within(y, want, e + 2.0 ** -18 * want.abs())
+    rows, ek = normed(kv[:, :np_kv], np_kv, 1, gk, None)
+    at = {(int(slots[m]), int(start[slots[m]]) % 2): m for m in range(M) if ring or int(start[slots[m]]) < 2}
+    for s in range(M):
+        for r in (0, 1):
+            if (s, r) in at:
+                within(cache[s, r], rows[at[s, r]], ek[at[s, r]])
+            else:
+                assert torch.isnan(cache[s, r]).all()
+
+
 def microseconds(launch, n=50):
     """Of a launch among others: the least of several replays of a graph that holds n of them."""
     launch()

@@ -89,6 +89,41 @@ def test_hybrid_step(make, width, B):
         assert (got - want).norm() <= 8 * len(m.layers) * 2.0 ** -9 * want.norm(), float((got - want).norm() / want.norm())
 
 
+@pytest.mark.parametrize("B", [1, 2, 3, 4])
+@pytest.mark.parametrize("q_rank,kv_rank,window", [(512, 128, None), (512, 250, 5), (508, 128, 5), (1024, 512, None), (1020, 1000, 3), (1024, 64, 8)])
+def test_hybrid_step_with_wide_query_latents(q_rank, kv_rank, window, B):
+    """Query latents of 512 and 1024 columns (padded to them), which the queries' product norms itself: in slots that are not the rows'
+    numbers, with every earlier token in the cache and with rings that turn (the windows are shorter than the 12 tokens).  Bound: as above."""
+    from vyomai_amd import GisitarConfig, GisitarModel
+    from vyomai_amd.layers.latent_attention import LatentAttention
+    torch.manual_seed(q_rank + kv_rank)
+    mixer = {"heads": 4, "dim": 64, "vdim": 64, "q_rank": q_rank, "kv_rank": kv_rank, "scale": 0.125}
+    with torch.device(DEV):
+        torch.set_default_dtype(BF)
+        try:
+            m = GisitarModel(GisitarConfig(vocab=1003, width=1024, layers=[{"type": "latent_attention", "mixer": mixer, "mlp": {"kind": "dense", "ff": 1496}},
+                                                                           {"type": "latent_attention", "mixer": mixer, "mlp": None}]))
+            if window:
+                for layer in m.layers:
+                    layer.mixer = LatentAttention(1024, 4, 64, 64, q_rank, kv_rank, 0.125, 1e-5, window=window)
+        finally:
+            torch.set_default_dtype(torch.float32)
+    m = m.eval()
+    assert m.layers[0].mixer.packed().q_norm.numel() in (512, 1024)
+    ids = torch.randint(0, 1003, (B, 12), device=DEV, generator=torch.Generator(device=DEV).manual_seed(B))
+    cache = m.new_cache(B + 2, 16)
+    cache.allocate(2)
+    slots = cache.allocate(B)[::-1]
+    m.prefill(ids[:, :2].contiguous(), [2] * B, cache, slots)
+    for t in range(2, 12):
+        got = m.decode(ids[:, t].contiguous(), cache, slots).double()
+        other = m.new_cache(B, 16)
+        s = other.allocate(B)
+        want = m.logits(m.prefill(ids[:, :t + 1].contiguous(), [t + 1] * B, other, s)[:, -1]).double()
+        assert torch.isfinite(got).all()
+        assert (got - want).norm() <= 8 * len(m.layers) * 2.0 ** -9 * want.norm(), float((got - want).norm() / want.norm())
+
+
 @pytest.mark.parametrize("B", [1, 2, 4])
 def test_what_a_step_refuses(B):
     """Vocabulary weights that are not there and logits rows narrower than the vocabulary: errors, as from the general launchers, and the

@@ -373,7 +373,7 @@ bool few_k(int epi, int pro, int64_t K) {
   const int kc = (int)(K / 256);
   if (pro == PLAIN) return epi == QKV ? kc >= 2 && kc <= 4 : epi == STORE && (kc == 2 || kc == 3 || kc == 4 || kc == 8 || kc == 12 || kc == 16);
   if (pro == LAYER) return epi != GATED && kc >= 2 && kc <= 4;
-  if (pro == RMS) return epi == STORE && (kc == 2 || kc == 4);
+  if (pro == RMS) return epi == STORE && (kc == 2 || kc == 4);   // (an even kc: a lane's quads pair up to 16-byte chunks; the query latents of bench.py's models)
   if (pro == PARTS) return epi == STORE && kc >= 2 && kc <= 4;
   return epi != QKV && (kc == 4 || kc == 8);
 }
@@ -410,11 +410,11 @@ extern "C" int vy_debug_few(int epi, int pro, const void* x, const void* a, cons
     residual = nullptr;
   }
   if (pro == vy_few::RMS) {
-    if (k) {   // rows v [M][K] of nkv columns, weights b, into row cos_tab[m] (integers; below nq) of k [M][2][nkv]
+    if (k) {   // rows v [M][K] of nkv columns, weights b, into row cos_tab[slot] (integers; below nq, of a ring of -nq) of k [slot][2][nkv]; slots h
       f.kv = (const bf16*)v; f.w_kv = (const float*)b; f.n_kv = f.np_kv = nkv; f.cache = (bf16*)k; f.k_ss = 2 * (int64_t)nkv; f.k_st = nkv;
-      f.cap = nq; f.ring = 0; f.start = (const int*)cos_tab;
+      f.cap = nq < 0 ? -nq : nq; f.ring = nq < 0; f.start = (const int*)cos_tab; f.slots = (const int*)h;
     }
-    b = sin_tab;
+    b = sin_tab; h = nullptr;
   }
   if (pro == vy_few::LAYER || pro == vy_few::PARTS) { f.ln_g = (const bf16*)a; f.ln_b = (const bf16*)b; }
   else { f.w_post = (const float*)a; f.w_pre = (const float*)b; }
