@@ -104,10 +104,11 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
       else w[p] = *at;
     }
   };
-  // what the epilogue reads besides the product, one lane per (weight row, operand row), and none of it hangs on the product: requested
-  // behind the norm's operands (behind the norm, the position and then the rotary factors were two more trips to memory: QKV of 768 columns
-  // 3.86 -> 3.68 us).  STREAM has a bias at most, which is there before the product is: requested ahead of its norm it
-  // cost 0.35 us a product (the 16 of a decoder of width 1024 and 8 layers, on average: 5.82 -> 6.16)
+  // what the epilogue reads besides the product, one lane per (weight row, operand row), and none of it hangs on the product.  QKV requests
+  // it behind the norm's operands: behind the norm, the position and then the rotary factors were two more trips to memory (768 columns
+  // 3.86 -> 3.68 us).  The others have a bias and a residual at most, which are there before the product is if requested with it; ahead of
+  // it they delay weights and operands: text models of 12 layers, steps of 1 / 4 sequences 171.5 -> 168.5 / 207.7 -> 203 us at 512 columns,
+  // 194.5 -> 191.5 / 250 -> 244.5 at 768, 250 -> 247 / 302 -> 297 at 1024
   const int er = R == 1 || lane >= R * MR ? 0 : lane / MR, em = R == 1 ? lane : lane % MR;
   float e_bias = 0.f, e_other = 0.f, e_res = 0.f, e_cos = 0.f, e_sin = 0.f;
   int pos = 0;
@@ -138,7 +139,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   }
   const int row = wave / SHARES;   // of the operand, this wave's
   const bool leads = wave % SHARES == 0 && row < a.M;
-  if (u < units && PRO != STREAM && (PRO == PLAIN || !leads)) request_rest(u);
+  if (EPI == QKV && u < units && (PRO == PLAIN || !leads)) request_rest(u);
 
   if constexpr (PRO != PLAIN) {
     if (a.advance && blockIdx.x == 0)
@@ -155,7 +156,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
           xb4[c] = bf16x4{(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
           if (PRO == PARTS && a.x_bias) xb4[c] = *reinterpret_cast<const bf16x4*>(a.x_bias + col);
         }
-        if (u < units) request_rest(u);
+        if (EPI == QKV && u < units) request_rest(u);
       }
     }
     f32x4 mine[KC];   // PARTS: this wave's share of the row
@@ -194,7 +195,6 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
           v4[c] = *reinterpret_cast<const bf16x4*>(a.x + row * a.ldx + column(c));
           w4[c] = *reinterpret_cast<const f32x4*>(a.w_pre + column(c));
         }
-        if (u < units) request_rest(u);
         float q = 0.f;
 #pragma unroll
         for (int c = 0; c < KC; ++c)
@@ -278,7 +278,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   }
 
   for (; u < units; u += step) {
-    if constexpr (PRO == STREAM) request_rest(u);
+    if constexpr (EPI != QKV) request_rest(u);
     const bool mine = lane < R * MR && em < a.M;
     const int n = row_of(u, er);
     const bool real = mine && (EPI != STORE || u * R + er < a.N);
@@ -293,7 +293,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
     for (int p = 0; p < P; ++p) wv[p] = w[p];
     if (u + step < units) {
       request(u + step);
-      if constexpr (PRO != STREAM) request_rest(u + step);
+      if constexpr (EPI == QKV) request_rest(u + step);
     }
 #pragma unroll
     for (int p = 0; p < P; ++p) {
