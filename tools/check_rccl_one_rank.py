@@ -29,7 +29,7 @@ def train(**kw):
 
 # the weight gradients are summed with fp32 atomics and AdamW turns a sign flip of a noise-level gradient into a 2 lr
 # difference: runs of the SAME trainer set the noise floor the comparison is held to -- the largest difference between any two
-# of five, since two runs that happen to flip the same gradients are 1.5e-7 apart instead of 1.2e-6 to 3.2e-6 (seen in 3 of 40
+# of five, since two runs that happen to flip nearly the same gradients are 1.4e-7 to 6.7e-7 apart instead of 0.9e-6 to 3.2e-6 (3 of 53
 # pairs), while the exchange, which sums weight gradients layer by layer, is 3.8e-6 from either
 runs = [train()[:2] for _ in range(5)]
 ref, loss_ref = runs[0]
