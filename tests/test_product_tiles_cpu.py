@@ -6,11 +6,12 @@ import pytest
 KINDS = ["256x256", "256x192", "256x128", "128x128", "64", "64 twice", "64 many", "128 split", "320 split"]
 
 
-def tiling(M, N, K, ws=64 << 20):
+def tiling(M, N, K, ws=64 << 20, gated=False):
+    """gated: of M x N / 2 outputs, whose factors meet in a pass of their own where K is spread over workgroups"""
     from vyomai_amd import _lib
     f = _lib.load().vy_debug_tiling
-    f.argtypes, f.restype = [C.c_int64] * 4, C.c_int
-    t = f(M, N, K, ws)
+    f.argtypes, f.restype = [C.c_int64] * 4 + [C.c_double], C.c_int
+    t = f(M, N, K, ws, 3 if gated else 0)
     return KINDS[t % 16], t // 16
 
 
@@ -26,6 +27,12 @@ def tiling(M, N, K, ws=64 << 20):
 def test_kernel_is_a_fast_one(M, N, K, slices, fastest):
     kind, S = tiling(M, N, K)
     assert S == slices and kind in fastest
+
+
+@pytest.mark.parametrize("M,I,K,fastest", [(264, 8192, 2048, {"64"}), (129, 1024, 4096, {"64 many"}), (200, 1024, 4096, {"64 many"}),
+                                           (129, 512, 2048, {"64 many"}), (129, 768, 3072, {"64 many"}), (264, 16384, 2048, {"256x256"})])
+def test_gated_products_stay_in_one_launch(M, I, K, fastest):
+    assert tiling(M, 2 * I, K, gated=True)[0] in fastest
 
 
 def test_every_kernel_is_reached():

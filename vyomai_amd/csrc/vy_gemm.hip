@@ -1676,10 +1676,10 @@ inline Scratch splitk_ws(hipStream_t st) {
 // 256 x 256: 313 us; 8000 x 1024, K = 6144: 124 us on 256 x 192, 152 us on 256 x 256, 100 us on 256 x 128 (250 tiles).  So the
 // launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below; the constants
 // are fits to launches of 40 shapes from 48 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
-// output alone and so moves no choice), where K is sliced (up to 4096 rows) to 1100 of 33 to 4096 rows, 64 to 8192 columns and K = 256 to
-// 8192, each on all kernels that take it, in graphs that walk through 200 MB of weights, as a model's layers do: products that find
+// output alone and so moves no choice), where K is sliced (up to 4096 rows) to 1600 of 33 to 4096 rows, 64 to 40000 columns and K = 256 to
+// 16384, each on all kernels that take it, in graphs that walk through 200 MB of weights, as a model's layers do: products that find
 // their weights in L2, as a loop over one product does, made one launch look shorter than two groups in it.  The kernel chosen takes
-// 0.2 % longer than the fastest on average, over 8 % for 5 of them.  (Fitted to 90 shapes, 8 % for 45: 300 x 2048, K = 6144, 31.5 us in two
+// 0.2 % longer than the fastest on average, over 8 % for 12 of them.  (Fitted to 90 shapes, 8 % for 45 of 1100: 300 x 2048, K = 6144, 31.5 us in two
 // groups, 25.6 with K over workgroups; 512 x 1152, K = 4304, 26.9 and 20.8.)
 // ------------------------------------------------------------------------------------------
 enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWICE, T_64x64_MANY, T_128x128_SPLIT, T_320x128_SPLIT };
@@ -1715,7 +1715,7 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     default: {   // K over several workgroups: the partial sums' way through memory -- Infinity Cache for most of it -- and a second launch
       const double padded = 4e-6 * S * tiles * TILE_M[kind] * TILE_N[kind], sums = 5.0 + 1.34 * sqrt(padded) + 0.18 * 4e-6 * S * M * N;
       const int per = (KT + S - 1) / S;
-      if (kind == T_320x128_SPLIT) return sums + 1.6 + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * 0.86;
+      if (kind == T_320x128_SPLIT) return sums + 1.6 + (double)vy_cdiv(tiles * S, (int64_t)chip) * per * 0.95;
       const double stage = per * (apart ? 1.16 : 1.0);
       if (tiles * S <= chip) return sums + 0.66 * stage;
       const double r = (double)(tiles * S) / (2 * chip), whole = (double)(int64_t)r, part = r - whole;   // (two of them share a CU)
@@ -1753,7 +1753,8 @@ inline int sum_slices(int64_t M, int64_t N, int64_t K) {
   return (KT + per - 1) / per;
 }
 
-inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes) {
+// `behind`: microseconds that K over several workgroups costs besides
+inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes, double behind = 0.0) {
   const int S = sum_slices(M, N, K);
   Tiling best{T_64x64, S};
   double least = 1e30;
@@ -1770,8 +1771,8 @@ inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_
   }
   if (S <= 4) offer(T_64x64_TWICE, tile_cost<T_64x64_TWICE>(M, N, K, S, chip));
   else offer(T_64x64_MANY, tile_cost<T_64x64_MANY>(M, N, K, S, chip));
-  if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, tile_cost<T_128x128_SPLIT>(M, N, K, S, chip));
-  if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, tile_cost<T_320x128_SPLIT>(M, N, K, S, chip));
+  if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, behind + tile_cost<T_128x128_SPLIT>(M, N, K, S, chip));
+  if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, behind + tile_cost<T_320x128_SPLIT>(M, N, K, S, chip));
   return best;
 }
 
@@ -2566,7 +2567,9 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
 // 8000 x 2 x 4096, K = 1024: 163 -> 134; 700 x 2 x 4096, K = 1024: 25.8 -> 20.6; 100 rows: 10.3 -> 6.8.
 template <int ACT>
 int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N, int64_t K, const EpiPlain<bf16>& ep, hipStream_t st) {
-  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, splitk_ws(st).bytes);
+  // (with K over several workgroups the factors meet in a pass of their own over the product, 3 us: of 260 shapes none takes over 10 % longer
+  // than on the faster way.  Left out of the cost: 264 x 2 x 8192, K = 2048, 40 -> 47 us, 129 x 2 x 512, K = 2048, 12.2 -> 15.3)
+  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, splitk_ws(st).bytes, 3.0);
   const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, TILE_M[t.kind]) * tn;
   const int KT = (int)vy_cdiv(K, BK), per = (KT + t.slices - 1) / t.slices;
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
@@ -2718,9 +2721,9 @@ int qkv_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void*
 }  // namespace
 
 // test aid, not part of include/vyom_hip.h: the kernel (TileKind) of a product of more than 32 rows with ws_bytes of workspace, and 16 times
-// the slices of K that it adds up
-extern "C" int vy_debug_tiling(int64_t M, int64_t N, int64_t K, int64_t ws_bytes) {
-  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes);
+// the slices of K that it adds up; behind: as for pick_tiling
+extern "C" int vy_debug_tiling(int64_t M, int64_t N, int64_t K, int64_t ws_bytes, double behind) {
+  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes, behind);
   return (int)t.kind + 16 * t.slices;
 }
 
