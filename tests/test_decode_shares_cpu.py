@@ -14,7 +14,7 @@ def pays(B, h, hk, S):
 
 @pytest.mark.parametrize("h,hk,B,short,long", [
     # heads, key heads, sequences; behind 60 and behind 600 tokens
-    (12, 12, 1, True, True), (12, 4, 1, True, True), (16, 16, 1, True, True), (16, 2, 1, True, True),
+    (12, 12, 1, True, True), (12, 4, 1, True, True), (16, 16, 1, False, False), (16, 8, 1, False, True), (16, 2, 1, False, False),
     (8, 8, 4, True, True), (12, 12, 2, True, True), (12, 12, 3, False, False), (12, 12, 4, False, False), (12, 6, 4, True, True),
     (16, 16, 2, False, False), (16, 8, 2, False, False), (16, 4, 4, False, False), (16, 2, 3, False, False),
     (12, 4, 2, False, True), (12, 4, 4, False, True), (12, 3, 2, False, False), (12, 3, 3, False, True), (8, 2, 4, False, True),

@@ -574,9 +574,8 @@ __device__ __forceinline__ float dec_stride_sum(float v) {
 //
 // PROJ (few sequences): each result is multiplied with its columns of the output projection here, whose launch of its own falls away;
 // the product behind adds the heads' shares up (PARTS of vy_few.hip).  Every head is attended to by as many workgroups as the
-// projection's rows are spread over -- its keys come from L2 then, and no workgroup has more to read than before.
-// 12 layers of 768, prompt and 24 steps: one sequence behind 60 tokens 6700 -> 6120 us, behind 500 7200 -> 6580; 4 behind 500 11150 -> 10790,
-// with 4 key/value heads 11070 -> 9990.
+// projection's rows are spread over -- its keys come from L2 then, and no workgroup has more to read than before.  What that gives and
+// costs: vy_dec_shares_pay (vy_runtime.hip).
 template <int DH, int NW, int NP, bool NT, int R = 1, bool PROJ = false>
 __global__ __launch_bounds__(64 * NW) void dec_attn_kernel(const DecAttnArgs p) {
   constexpr int LPK = DH / 8, KPW = 64 / LPK, KPP = NW * KPW;
@@ -1043,7 +1042,8 @@ int vy_dec_attn_out(const void* q, const void* k, const void* v, int64_t c_sb, i
   a.pos_dev = pos_dev; a.S = (int)S; a.h = h; a.hk = hk; a.scale = scale; a.wo = (const bf16*)wo; a.part = part; a.d = h * 64;
   // One sequence: a workgroup per query head also where several share a key head (12 layers of 768, 4 key/value heads, 24 steps and
   // their prompt: behind 60 tokens 6113 against 6190 us, behind 500 6580 and 6990); more: one for all that share it, whose fewer shares the next
-  // product adds up sooner (4 sequences behind 30 tokens 9480 and 8990).
+  // product adds up sooner (a step of 12 layers of 768, 6 key/value heads, 3 / 4 sequences behind 60 tokens 235 / 240 us, with one for each
+  // query head 248 / 254, behind 500 260 / 265 and 266 / 275; two sequences 208 and 212, 232 and 230).
   const int rep = B > 1 && dec_attn_gq() && h / hk >= 2 && h / hk <= 4 ? h / hk : 1, units = h / rep;
   if (units > 16 || (int64_t)units * B * a.d * 4 > room) return 0;
   if (rep == 4 && (pos_dev ? smax : S) > 640) return 0;   // (longer contexts in registers beside four heads' rows of wo: spills)

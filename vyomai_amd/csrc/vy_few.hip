@@ -7,7 +7,7 @@
 // (rotary pairs and gate / up pairs are the two rows of a wave) in whole 1 KB pieces.
 //
 // 12 layers of 768, one sequence behind 70 tokens: 334 -> 249 us a step (62 launches instead of 75, and no products for 32 rows; with the
-// output projection inside the attention, PARTS, 50 launches and some 220 us);
+// output projection inside the attention, PARTS, 50 launches and 215 us);
 // 8 layers of width 1024 (latent and lightning attention), 700 tokens: 302 -> 267 us, 2 / 4 rows 414 -> 308 / 482 -> 398 us.
 #include "vy_few.h"
 

@@ -100,14 +100,17 @@ static bool few_operands(const vy_decode_plan* p, const void* x, const void* hid
 // feed-forward's first product then adds up the heads' fp32 shares -- h B d of them, out of L2 -- and query heads that share a key head are
 // attended to by one workgroup, which three and four of them only repay where their keys are streamed otherwise (kv_bytes: one layer's keys
 // and values, against the 1 MB above which vy_dec_attn streams them).  A step with the projection inside / by itself, 12 layers, us:
-//   one sequence: 768 columns 196 / 209 behind 60 tokens, 212 / 245 behind 500, 1024 columns level
-//   two: 512 columns 181 / 198, 768 223 / 225 and 240 / 259, 1024 294 / 261;   four: 512 210 / 216, 768 268 / 250, 1024 406 / 298
-//   three query heads a key head, 768 columns: two sequences 219 / 221 behind 60, 250 / 240 behind 500, four 250 / 243 and 283 / 298; four
-//   heads: two sequences 230 / 220, behind 500 266 / 240, three behind 500 293 / 306; six: three sequences 251 / 240, behind 700 275 / 298
+//   one sequence: 512 columns 168 / 184 behind 60 tokens, 768 191 / 206, behind 500 209 / 241; 1024 244 / 239, but 254 / 265 where two heads
+//   share streamed keys
+//   two: 512 columns 176 / 193, 768 217 / 221 and 235 / 256, 1024 291 / 255;   four: 512 204 / 207, 768 260 / 243, 1024 401 / 292
+//   two heads a key head, 768 columns: three sequences 233 / 235 and 259 / 272, four 239 / 237 and 265 / 275
+//   three: two sequences 215 / 217 behind 60, 245 / 236 behind 500, three 240 / 232 and 271 / 286, four 244 / 237 and 277 / 290
+//   four: two sequences 226 / 217, behind 500 262 / 236, three behind 500 288 / 302
+//   six: two sequences 212 / 217, three 247 / 234, behind 700 tokens 273 / 296
 bool vy_dec_shares_pay(int B, int h, int hk, int64_t kv_bytes) {
   const int d = 64 * h, rep = hk > 0 ? h / hk : 1, units = rep >= 2 && rep <= 4 ? hk : h;
   const bool streamed = kv_bytes > (1 << 20);
-  if (B == 1) return true;
+  if (B == 1) return d <= 768 || (rep > 1 && streamed);
   if (d > 768) return false;   // (the product's sums of two and more rows of 1024 columns: registers)
   if (rep == 3 || rep == 4) return streamed;
   return units * B * d * 4 <= (72 << 10) || (rep > 4 && streamed);
