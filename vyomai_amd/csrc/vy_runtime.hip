@@ -100,8 +100,8 @@ static bool few_operands(const vy_decode_plan* p, const void* x, const void* hid
 // feed-forward's first product then adds up the heads' fp32 shares -- h B d of them, out of L2 -- and query heads that share a key head are
 // attended to by one workgroup, which three and four of them only repay where their keys are streamed otherwise (kv_bytes: one layer's keys
 // and values, against the 1 MB above which vy_dec_attn streams them).  A step with the projection inside / by itself, 12 layers, us:
-//   one sequence: 512 columns 168 / 184 behind 60 tokens, 768 191 / 206, behind 500 209 / 241; 1024 244 / 239, but 254 / 265 where two heads
-//   share streamed keys
+//   one sequence: 512 columns 168 / 184 behind 60 tokens, 768 191 / 206, behind 500 209 / 241; 1024 244 / 239, but 264 / 275 behind 640 where
+//   two heads share streamed keys
 //   two: 512 columns 176 / 193, 768 217 / 221 and 235 / 256, 1024 291 / 255;   four: 512 204 / 207, 768 260 / 243, 1024 401 / 292
 //   two heads a key head, 768 columns: three sequences 233 / 235 and 259 / 272, four 239 / 237 and 265 / 275
 //   three: two sequences 215 / 217 behind 60, 245 / 236 behind 500, three 240 / 232 and 271 / 286, four 244 / 237 and 277 / 290
