@@ -3,7 +3,7 @@
  * behind vyomai_amd's mirror of the VyomAI layer API.
  *
  * The reference (Ajax0564/VyomAI) has no FFI: its hot path is the Python class API of
- * VyomAI/layers consumed by VyomAI/models (SURVEY.md section 8b).  Each entry point
+ * VyomAI/layers consumed by VyomAI/models.  Each entry point
  * below replaces the torch ops that one reference call site issues; the citation after
  * "replaces:" is path:line in the reference checkout.
  *
@@ -563,7 +563,7 @@ typedef struct vy_transpose_desc {
 int vy_transpose_batched(const vy_transpose_desc* descs_dev, int32_t n, int32_t total_tiles, int dtype,
                          void* stream);
 
-/* Sampling front end of the generate loops (SURVEY 8f-4).
+/* Sampling front end of the generate loops.
  * vy_greedy_step replaces reference models/decoder.py:478-507 (topk(k=1), the where() that forces prompt
  *   tokens, the token write, the isin()/or of the EOS bookkeeping and the all() reduction) for one
  *   generated position: for row b, next = argmax_v logits[b,v] (lowest index among equal maxima) unless
@@ -622,7 +622,7 @@ int vy_decoder_step(const vy_decode_plan* plan, const void* x, int64_t pos, cons
                     void* hidden_out, void* logits, int64_t ldv, void* stream);
 
 /* ------------------------------------------------------------------------------------------
- * vy_gemma_decoder_step: one single-token step of a Gemma-style decoder stack (BASELINE configs[4], the
+ * vy_gemma_decoder_step: one single-token step of a Gemma-style decoder stack (the
  * PaliGemma-shape language model; Examples/paligemma.ipynb cells 11-13): per layer
  *   n = RMSNorm(x) ; q,k,v = n Wqkv^T (+b) with RoPE, k/v written into the cache at `pos` ;
  *   x = x + attn(q, K[0..pos], V[0..pos]) Wo^T ; n = RMSNorm(x) ; x = x + (gelu_tanh(n Wg^T) * n Wu^T) Wd^T

@@ -674,7 +674,7 @@ def clm_loss(logits: Tensor, labels: Tensor) -> Tensor:
 
 
 # ----------------------------------------------------------------------------
-# sampling processors and speculative decoding (SURVEY 8f-4)
+# sampling processors and speculative decoding
 # ----------------------------------------------------------------------------
 
 

@@ -30,7 +30,7 @@ def close(got, want, x, w, extra=0.0):
 SHAPES = [(33, 8, 8), (63, 64, 64), (64, 72, 72), (65, 200, 136), (127, 64, 192), (129, 520, 200), (512, 768, 768), (300, 2304, 760),
           (1000, 776, 320), (2111, 1032, 448), (1665, 3080, 128), (4096, 768, 3072), (4100, 1000, 1024), (8000, 1024, 1600),
           (3000, 2048, 2048), (8193, 1030, 64), (9000, 776, 832), (130, 768, 6144), (257, 1024, 4160), (700, 1024, 6144),
-          # slices of K added up in order inside a tile: three, four with a short last one, eight, sixteen; two groups with two and four
+          # slices of K added up in order inside a tile, by one group of waves or two: two to eight, short last ones (more of them: SLICED, below)
           (512, 768, 576), (512, 776, 704), (700, 1024, 1024), (2112, 768, 3072), (1700, 1544, 392), (512, 768, 840)]
 
 

@@ -100,12 +100,12 @@ def _wt_cached(owner, key_fn, src_fn) -> torch.Tensor:
     return view
 
 
-_ROW_GRANULE = int(os.environ.get("VY_ROW_GRANULE", "64"))   # (8: the layout of rounds 1-2, for A/B runs)
+_ROW_GRANULE = int(os.environ.get("VY_ROW_GRANULE", "64"))   # (8: rows on 16 bytes, for A/B runs)
 
 
 def _row_stride(n: int) -> int:
     """Row stride (elements) of a matrix with n columns that a GEMM reads as an operand: whole 128-byte lines per row
-    (64 bf16), so that no row starts in the middle of a line.  With the 16-byte granule of rounds 1-2 the 50265-wide logits had a
+    (64 bf16), so that no row starts in the middle of a line.  With rows on 16 bytes the 50265-wide logits had a
     100,544-byte stride: every second row of the dgrad / wgrad operand began 64 bytes into a line and each 128-byte piece an
     LDS-DMA instruction fetches came from two lines."""
     g = _ROW_GRANULE
@@ -613,8 +613,7 @@ class LMHeadLossFn(torch.autograd.Function):
     labels[:, 1:] with ignore_index (Examples/vyom-ai-decoder_clm.ipynb cell 29).  The logits
     ([M, V] bf16, padded row stride) are produced by the vocabulary GEMM, then reduced AND
     overwritten IN PLACE by their unit gradient in one pass (vy_xent_fused; vy_xent_fwd + vy_xent_bwd
-    beyond 65536 columns) -- they are never copied, up-cast or re-materialised (SURVEY.md section 8f
-    item 1).  Backward multiplies by the upstream gradient through the GEMMs (a device scalar)."""
+    beyond 65536 columns) -- they are never copied, up-cast or re-materialised.  Backward multiplies by the upstream gradient through the GEMMs (a device scalar)."""
 
     @staticmethod
     def forward(ctx, hidden, labels, ignore_index, wd, bd, ln_w, ln_b, wv, bias, eps, err_flag=None):

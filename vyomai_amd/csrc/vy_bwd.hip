@@ -525,7 +525,7 @@ __device__ __forceinline__ void rope_bwd_quad(const BwdParams& p, int64_t pos, i
 }
 
 // chunk swizzle of a 128-B-row LDS image that is read BOTH by rows (ds_read_b128) and transposed
-// (ds_read_b64_tr_b16): conflict-free for both ("dual-use image")
+// (ds_read_b64_tr_b16): conflict-free for both
 __device__ __forceinline__ int dual_sw(int row) {
   const int v = (row >> 1) & 7;
   return ((v & 1) << 2) | (v >> 1);

@@ -1,4 +1,4 @@
-// Data-parallel gradient exchange on RCCL behind the C ABI (SURVEY.md section 8b's designed exports: the multi-GPU
+// Data-parallel gradient exchange on RCCL behind the C ABI (the multi-GPU
 // surface of the library).  The reference trains under accelerate / torch DDP (Examples/vyom-ai-decoder_clm.ipynb cell 31,
 // Examples/vyom-ai-accelerate-multimodel-2t4.ipynb cells 1-2): one process per GPU, gradients averaged by an all-reduce
 // while backward is still running.  Here: one communicator per process, the bucket all-reduce enqueued on a caller-given

@@ -40,7 +40,7 @@ struct DecDbg { unsigned long long* buf; int slot; int max_wg; };
 // 16 bytes of a stream too large to stay on chip until it is read again: the non-temporal policy
 // (`global_load_dwordx4 ... nt`).  Used for the K/V rows of a LARGE cache only (dec_attn_kernel<..., NT>): at B = 32 the
 // caches are 680 MB per step, and streamed with the default policy they push the 170 MB of weights out of the
-// Infinity Cache every step (step 514.5 -> 501 us with nt); a small cache (configs[4]: 5.5 MB) is served on chip from one
+// Infinity Cache every step (step 514.5 -> 501 us with nt); a small cache (18 layers with one key head of 256: 5.5 MB) is served on chip from one
 // step to the next and must keep the default policy (+5 % per token with nt).  The weight tiles keep the default policy
 // (nt on them alone: +1 %).
 __device__ __forceinline__ bf16x8 dec_load_stream(const bf16* p) {
@@ -509,7 +509,7 @@ int dec_part64_go(DecGemmArgs a, int K, hipStream_t st) {
 }
 
 // ------------------------------------------------------------------------------------------
-// Single-sequence matrix-vector products (Gemma-style decode, B = 1).  One wave per output
+// Single-sequence matrix-vector products (Gemma-style decode, B = 1: 18 layers of 2048, one key head of 256).  One wave per output
 // column, the row of the weight matrix in 16-byte pieces (1 KiB contiguous per wave instruction).  The general
 // gemv_bf16_kernel (vy_gemm.hip) serves up to 4 rows with run-time row guards, and its ISA shows what that costs:
 // the activation chunk of every k-piece is requested and waited for (vmcnt(0)) in the middle of the dot products,
@@ -1012,7 +1012,7 @@ int vy_dec_attn(const void* q, int64_t q_sb, const void* k, const void* v, int64
   // K/V policy (see dec_load_stream): streamed (nt) unless one layer's rows are under 1 MB.  Measured on the 12-layer
   // d = 768 decoder, whose 170 MB of weights can stay in the Infinity Cache if the K/V stream does not push them out: nt is
   // ahead at every batch (B = 1 / 2 / 4 / 8 / 32: 349 / 360 / 380 / 368 / 485 us against 355 / 363 / 388 / 399 / 515); on
-  // configs[4] (0.3 MB per layer, 5.8 GB of weights streaming through anyway) the default policy is 5 % ahead.
+  // the 18-layer Gemma-style decoder (0.3 MB per layer, 5.8 GB of weights streaming through anyway) the default policy is 5 % ahead.
   const int nt_env = dec_attn_nt(), gq_env = dec_attn_gq();
   const int64_t layer_bytes = 2ll * B * hk * (pos_dev ? smax : S) * dh * 2;
   const bool nt = nt_env < 0 ? layer_bytes > (1ll << 20) : nt_env != 0;

@@ -1012,7 +1012,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_kernel(
 // barrier that ends slice kt, and the barrier wait is a COUNTED vmcnt (the GX youngest LDS-DMA
 // instructions of the wave, slice kt+2 of X, may still be outstanding).
 //
-// On mfma_f32_16x16x32_bf16 (the 32 x 32 x 16 form of this kernel was removed in round 3 -- identical outputs, slower):
+// On mfma_f32_16x16x32_bf16 (on 32 x 32 x 16, with identical outputs, it was slower):
 // 4 x 6 blocks of 16 x 16 per wave (96 accumulator registers),
 // 24 MFMAs per 32-deep k-step, two k-steps per stage.  Same LDS image, same swizzle (conflict-free for this
 // fragment shape too: rows lane & 15, chunk 4 ks + (lane >> 4)), same ring, same epilogue (a lane still owns quads of 4

@@ -1,4 +1,4 @@
-// Sampling front end of the generate loops (SURVEY section 8f-4): the per-token work after the LM head.
+// Sampling front end of the generate loops: the per-token work after the LM head.
 //   vy_greedy_step     reference models/decoder.py:478-507 (top-1, prompt forcing, EOS bookkeeping)
 //   vy_sampling_probs  reference logits_processors.py:13-16, 59-63, 73-81, 92-102
 // One 1024-thread workgroup per row.  Selection (k-th largest value, nucleus cut) is a radix search over

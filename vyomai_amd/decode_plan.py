@@ -152,7 +152,7 @@ class DecodePlan:
         return logits[:, : self.vocab], hidden
 
 
-# ---- Gemma-style stack (PaliGemma-shape language model, BASELINE configs[4]) ---------------------------
+# ---- Gemma-style stack (PaliGemma-shape language model) ---------------------------
 
 class VyGemmaLayer(C.Structure):
     _fields_ = [(n, C.c_void_p) for n in ("wqkv", "bqkv", "wo", "bo", "ln_in", "ln_post", "wgu", "wdown", "kcache",

@@ -179,7 +179,7 @@ class _SelfAttentionBase(nn.Module):
         """The fused QKV kernel reads query/key/value.weight itself and never calls the sub-modules, so a projection that
         has been replaced by a wrapper -- the reference's adapters swap `attention.query` for a LoraLinear / DoraLinear
         whose weight lives at `.linear.weight` (VyomAI/layers/adapters.py:21-24, 58-62) -- would be ignored (or crash on
-        a missing attribute).  Adapters are outside SURVEY section 8; say so instead of computing without them."""
+        a missing attribute).  Adapters are not supported; say so instead of computing without them."""
         for name in (("qkv",) if self._fused_qkv else ("query", "key", "value")):
             m = self._modules[name] if name in self._modules else getattr(self, name)
             if not isinstance(m, nn.Linear):

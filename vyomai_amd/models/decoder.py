@@ -96,10 +96,10 @@ class DecoderLayer(nn.Module):
 
 
 def _two_lanes(model, rows: int) -> bool:
-    """Run the forward as two batch halves on two HIP streams (ops.lanes)?  Opt-in (VY_LANES=1): on configs[1] the two
+    """Run the forward as two batch halves on two HIP streams (ops.lanes)?  Opt-in (VY_LANES=1): on the 12-layer decoder, 32 x 512, the two
     half-size launch chains do overlap (two or more kernels resident 65-72 % of the time) but every half-size GEMM then
     takes as long as the full-size one did -- forward 6.63 against 6.49 ms, training step 18.71 against 18.56 ms, same box,
-    interleaved (tools/ab_env.py VY_LANES 0 1; DESIGN.md section 3, round 3)."""
+    interleaved (tools/ab_env.py VY_LANES 0 1)."""
     return os.environ.get("VY_LANES", "0") == "1"
 
 

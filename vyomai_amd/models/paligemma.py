@@ -7,7 +7,7 @@ wiring: pre-norm residual blocks, LayerNorm (SigLIP) / RMSNorm with (1+w) (Gemma
 GeGLU, grouped-query attention down to a single KV head, head_dim 72 (SigLIP) and 256 (Gemma), RoPE
 with theta 10000, embeddings scaled by sqrt(d), LM head tied to the embedding table.
 
-Inference only (config 5 of BASELINE.json is KV-cache decode).
+Inference only: prompts and KV-cache decode.
 """
 from __future__ import annotations
 

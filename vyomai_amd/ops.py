@@ -33,7 +33,7 @@ def _raw_stream() -> int:
 # What it buys on MI355X: a K = 768 GEMM launch is a k-loop bound by what the CUs take in from L2 followed by an
 # epilogue in which all 256 workgroups store at once (HBM-bound, matrix pipe idle) -- a third of the launch.  Two
 # independent half-size launch chains drift apart, so one chain's epilogue / LayerNorm / attention softmax runs
-# under the other's MFMA loop (DESIGN.md section 3, round 3).
+# under the other's MFMA loop.
 #
 # Ordering rules (correct by construction):
 #   * lane 1 waits, before each of its launches, for everything the host has enqueued on the main stream so far

@@ -1,4 +1,4 @@
-"""Parameter name -> shape tables of the reference models' state_dicts (SURVEY.md section 8b) and the
+"""Parameter name -> shape tables of the reference models' state_dicts and the
 configuration objects of the benchmark workloads.  Product-side so that bench.py and tools/ do not import the
 test tree; tests/golden/cases.py re-exports everything here."""
 from __future__ import annotations
@@ -22,12 +22,12 @@ class VitCfg:
 
 
 def vit_b16_config(num_hidden_layers: int = 12, hidden_dropout_prob: float = 0.0) -> VitCfg:
-    """ViT-B/16 of BASELINE.json configs[3]: 224x224 images, 16x16 patches, d = 768, 12 heads, 197 tokens."""
+    """ViT-B/16 of the captioning workload: 224x224 images, 16x16 patches, d = 768, 12 heads, 197 tokens."""
     return VitCfg(num_hidden_layers=num_hidden_layers, hidden_dropout_prob=hidden_dropout_prob)
 
 
 # ---------------------------------------------------------------------------
-# parameter name -> shape tables (reference state_dict layout, SURVEY.md section 8b)
+# parameter name -> shape tables (reference state_dict layout)
 # ---------------------------------------------------------------------------
 
 
@@ -124,7 +124,7 @@ def vit_shapes(cfg, p=""):
     return s
 
 
-# PaliGemma shapes (module dump in Examples/paligemma.ipynb cell 24 output; SURVEY.md section 2 row 21)
+# PaliGemma shapes (module dump in Examples/paligemma.ipynb cell 24 output)
 SIGLIP = dict(hidden_size=1152, intermediate_size=4304, num_hidden_layers=27, num_attention_heads=16,
               num_channels=3, image_size=224, patch_size=14, layer_norm_eps=1e-6, attention_dropout=0.0)
 GEMMA = dict(hidden_size=2048, intermediate_size=16384, num_hidden_layers=18, num_attention_heads=8,

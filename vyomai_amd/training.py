@@ -37,7 +37,7 @@ ALIGN = 8  # elements: keeps every bf16 parameter 16-byte aligned inside the sha
 # projections -- 64 bytes off a line: every 1536-byte weight row then straddled 13 lines instead of 12 and each 128-byte
 # row segment an LDS-DMA instruction fetches came from two lines (the decode step's vocabulary projection: 28.8 us inside
 # bench.py against 18.5 us on line-aligned weights, profiles/r03_*).
-LINE = int(os.environ.get("VY_ARENA_LINE", "64"))   # (8: the round-2 layout, for A/B runs)
+LINE = int(os.environ.get("VY_ARENA_LINE", "64"))   # (8: parameters on 16 bytes, for A/B runs)
 
 
 def _ordered_params(model: nn.Module) -> List[Tuple[str, nn.Parameter]]:
@@ -207,7 +207,7 @@ class BucketReducer:
     comm_dtype: None reduces the fp32 arena in place (652 MB per step for the 12-layer decoder);
     torch.bfloat16 reduces a bf16 copy of each bucket (326 MB) and writes the sum back in fp32 --
     a ring all-reduce over xGMI is bound by ONE ~153 GB/s link, so halving the bytes halves the
-    exchange (SURVEY.md section 5)."""
+    exchange."""
 
     def __init__(self, arena: FlatArena, process_group=None, bucket_bytes: int = 64 << 20,
                  average: bool = True, comm_dtype: Optional[torch.dtype] = None, native: Optional[NativeComm] = None):
