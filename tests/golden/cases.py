@@ -127,7 +127,7 @@ from vyomai_amd.shapes import (attn_shapes, aso_shapes, ffn_shapes, layer_shapes
 PG_SMALL_VOCAB, PG_IMAGE_TOKEN = 4099, 4000
 
 
-# ---- sampling processors / speculative decoding (SURVEY 8f-4) ----------------------------------
+# ---- sampling processors / speculative decoding ----------------------------------
 
 def sampling_logits() -> np.ndarray:
     """(3, 1531) fp32 logits: row 0 flat-ish, row 1 peaked, row 2 wide."""

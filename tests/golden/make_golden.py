@@ -238,7 +238,7 @@ def gradients():
 
 
 # ---------------------------------------------------------------------------
-# D2. configs[3] training: reference autograd through (i) a one-layer Vit (patchify conv, cls token, the
+# D2. caption training: reference autograd through (i) a one-layer Vit (patchify conv, cls token, the
 #     in-place double position add, VisionAttention with the fused qkv Linear at L = 197, FeedForward) and
 #     (ii) a VisionLanguageModel (1-layer Vit + 1-layer decoder, the image vector prepended as token 0) under
 #     the captioning notebooks' loss cross_entropy(logits[:, 1:-1], ids[:, 1:])
@@ -451,7 +451,7 @@ def paligemma_model():
 
 
 # ---------------------------------------------------------------------------
-# G. sampling processors and speculative decoding (SURVEY 8f-4)
+# G. sampling processors and speculative decoding
 # ---------------------------------------------------------------------------
 
 

@@ -60,7 +60,7 @@ def test_wgrad_grouped():
 
 
 @pytest.mark.parametrize("M,N,K,act", [(300, 768, 3072, 1), (1024, 768, 768, 0), (51, 3072, 768, 0),
-                                       # split-K launches (mid-size M, few tiles): the decoder rows of configs[3], a 264-row prefill
+                                       # split-K launches (mid-size M, few tiles): the captioning decoder's rows, a 264-row prefill
                                        (2112, 3072, 768, 0), (2112, 768, 3072, 1), (264, 2048, 2048, 0), (264, 16384, 2048, 0)])
 def test_dgrad(M, N, K, act):
     """dX[M,K] = dY[M,N] @ W[N,K] (* gelu'(pre)) (+ add)."""

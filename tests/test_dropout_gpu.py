@@ -275,7 +275,7 @@ def test_out_of_range_labels_are_ignored_and_flagged():
     assert torch.isfinite(loss)
     with pytest.raises(ValueError, match="outside"):
         m.lm_head.raise_on_label_error()
-    # ADVICE r2: the mean must not count the bad row on either path -- the same loss as with that label set to ignore_index
+    # the mean must not count the bad row on either path -- the same loss as with that label set to ignore_index
     asign = bad.clone()
     asign[0, 3] = -100
     m.eval()                                   # (the model was built with the default dropout: no random masks here)

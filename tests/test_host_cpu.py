@@ -287,7 +287,7 @@ def test_exchanged_weight_gradients_go_out_layer_by_layer(monkeypatch):
 
 
 def test_bench_starts_its_own_ranks_and_never_misreports_n_gpus():
-    """VERDICT r2: `python bench.py --gpus N` without a launcher used to run ONE rank and print n_gpus: 1.  Now it starts
+    """`python bench.py --gpus N` without a launcher used to run ONE rank and print n_gpus: 1.  Now it starts
     the N ranks itself (a child torch.distributed.run), and refuses a world size that differs from --gpus."""
     import json
     import subprocess

@@ -1,7 +1,7 @@
 """Kernel-level parity: every C-ABI entry point vs the CPU oracle / a plain fp32-fp64 torch
 restatement of the same op, on the same seeded inputs.  Runs on the MI355X box (-m gpu).
 
-Tolerances: f32 kernels 1e-5 (north_star); bf16 kernels are compared with the oracle evaluated on
+Tolerances: f32 kernels 1e-5; bf16 kernels are compared with the oracle evaluated on
 the bf16-rounded inputs, bar = a few bf16 ulps of the output scale.
 """
 import math
@@ -54,7 +54,7 @@ ACTS = {0: lambda x: x, 1: O.gelu_erf, 2: O.gelu_tanh}
                                    (2000, 768, 768), (4096, 1003, 768), (1500, 384, 72), (3072, 3072, 768),
                                    # mid-size M with few tiles: K split over workgroups (fp32 partial tiles + finish launch):
                                    # PaliGemma-shape prefill (264 rows; Gemma out-projection, SigLIP fc1 / fc2 with a K tail) and
-                                   # the 2112 rows of the captioning decoder (configs[3])
+                                   # the 2112 rows of the captioning decoder
                                    (264, 2048, 2048), (264, 2048, 16384), (256, 4304, 1152), (256, 1152, 4304), (2112, 768, 3072),
                                    (2112, 768, 768)])
 @pytest.mark.parametrize("act", [0, 1])

@@ -1,9 +1,8 @@
 """Model-level parity on the MI355X: vyomai_amd models (HIP kernels) vs the golden vectors the
 real reference produced (tests/golden/*.npz) and vs the CPU oracle on the same recipe weights.
 
-fp32 bar: 1e-5 on hidden states (north_star), token ids bit-exact in every cache mode.
-bf16 bar: error vs the fp32 reference no larger than the reference's own bf16-on-CPU gap
-("bf16 tolerance").
+fp32 bar: 1e-5 on hidden states, token ids bit-exact in every cache mode.
+bf16 bar: error vs the fp32 reference no larger than the reference's own bf16-on-CPU gap.
 """
 import numpy as np
 import pytest
@@ -37,7 +36,7 @@ def close(got, want, atol, what=""):
 
 @pytest.mark.parametrize("pos,at", [("absolute", None), ("rope", None), ("sinusoidal", "gqa"), ("rope", "gqa")])
 def test_encoder_config1(golden, pos, at):
-    """BASELINE.json configs[0] on the HIP path: EncoderModel default config, B=4, seq=128."""
+    """The text encoder on the HIP path: EncoderModel default config, B=4, seq=128."""
     import vyomai_amd as V
     g = golden("models_text")
     cfg = cases.with_kv(cases.test_cfg(), at)
@@ -104,7 +103,7 @@ def test_decoder_bf16_within_reference_gap(golden):
 
 
 def _bf16_bar(mine, ref32, refbf, keep=None, what=""):
-    """The bf16 bar of SURVEY section 7: the HIP bf16 error against the fp32 value is no larger than the gap the same
+    """The bf16 bar: the HIP bf16 error against the fp32 value is no larger than the gap the same
     model shows when its own op sequence runs in bf16 on the CPU (mean <= 1.5x + 1e-3, max <= 2x + 1e-2)."""
     gm, gr = np.abs(mine - ref32), np.abs(refbf - ref32)
     if keep is not None:

@@ -92,7 +92,7 @@ def test_modules(golden, tag):
 
 @pytest.mark.parametrize("pos,at", [("absolute", None), ("rope", None), ("sinusoidal", "gqa"), ("rope", "gqa")])
 def test_encoder_config1(golden, pos, at):
-    """BASELINE.json configs[0]: EncoderModel(EncoderConfig default) B=4 seq=128 on CPU."""
+    """EncoderModel(EncoderConfig default) B=4 seq=128 on CPU."""
     g = golden("models_text")
     cfg = cases.with_kv(cases.test_cfg(), at)
     sd = sd_from(cases.text_model_shapes(cfg, pos, at, head=False))
@@ -294,7 +294,7 @@ def test_paligemma_blocks(golden):
     close(cases.sub2(y.reshape(-1, y.shape[-1])), g["gemma.rmsnorm"], 2e-6, "rmsnorm")
 
 
-# ---- sampling processors and speculative decoding (SURVEY 8f-4) --------------------------------
+# ---- sampling processors and speculative decoding --------------------------------
 
 def _proc_args(cls, args):
     """(temperature, top_k, top_p) of a reference processor constructor call."""

@@ -1,4 +1,4 @@
-"""PaliGemma-shape path (BASELINE.json configs[4]) on the MI355X.
+"""PaliGemma-shape path on the MI355X.
 
 The layer blocks are pinned to the reference notebook's own classes (exec'd cells,
 tests/golden/paligemma_blocks.npz); the cached decode loop around them has no importable

@@ -1,4 +1,4 @@
-"""Sampling front end on the MI355X (SURVEY 8f-4): vy_greedy_step, vy_sampling_probs, the processor classes and
+"""Sampling front end on the MI355X: vy_greedy_step, vy_sampling_probs, the processor classes and
 speculative_generate against the reference's outputs (tests/golden/sampling.npz) and the CPU oracle.
 
 Bars: probabilities 1e-6 abs (fp32), support sets and token ids bit-exact, acceptance rate exact.

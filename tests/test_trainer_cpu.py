@@ -1,6 +1,6 @@
 """Host logic of the data-parallel trainer and of the compute-dtype weight copies, on CPU (no kernels):
 gradient accumulation with world_size 2 over gloo, frozen / unused parameters, the stale-state guards,
-and the two ways a cached bf16 copy of a parameter used to go stale (ADVICE r1)."""
+and the two ways a cached bf16 copy of a parameter used to go stale."""
 import os
 import socket
 
@@ -240,7 +240,7 @@ def _unused_on_one_rank_worker(rank, world, port, out):
 
 @pytest.mark.timeout(180)
 def test_parameter_unused_on_one_rank_keeps_the_replicas_identical():
-    """the touched set was rank-local, so a parameter one rank's batch skipped was updated on the other
+    """The touched set was rank-local, so a parameter one rank's batch skipped was updated on the other
     ranks only; and buckets went out in readiness order, which differs between such ranks."""
     ctx = mp.get_context("spawn")
     q = ctx.Queue()

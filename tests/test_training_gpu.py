@@ -325,7 +325,7 @@ def test_vlm_caption_loss_matches_cross_entropy_of_the_logits():
     got_m.backward()
 
 
-# ---- configs[3] training: ViT and vision-language gradients vs the REAL reference's autograd -------------
+# ---- caption training: ViT and vision-language gradients vs the REAL reference's autograd -------------
 
 def _grad_sample(g):
     g = g.detach().float().cpu()
