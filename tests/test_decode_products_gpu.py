@@ -372,3 +372,15 @@ def test_what_four_plain_rows_cost(K):
                       None, None, 0, M, 768, K, stream()) == 0
         us[M] = microseconds(launch)
     assert us[4] <= 1.7 * us[1], us
+
+
+@pytest.mark.parametrize("M", [5, 8])
+def test_what_the_bias_of_a_wide_product_costs(M):
+    """Nothing: it is there before the weights are (converted as it came, ahead of them, it took a tenth of the product's time)."""
+    go = entry("_Z14vy_rows_linearPKvS0_S0_ifPvllllP12ihipStream_t", p, p, p, i32, f32, p, i64, i64, i64, i64, p)
+    x, w, b, y = rnd(M, 1024, seed=1), rnd(32000, 1024, seed=2), rnd(32000, seed=3), torch.empty(M, 32000, dtype=BF, device=DEV)
+
+    def launch(bias):
+        assert go(ptr(x), ptr(w), ptr(bias), NONE, 0.0, ptr(y), 32000, M, 32000, 1024, stream()) == 0
+    without, beside = (microseconds(lambda: launch(bias), 20) for bias in (None, b))
+    assert beside <= 1.06 * without, (without, beside)

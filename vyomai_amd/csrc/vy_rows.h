@@ -118,12 +118,13 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int 
   const bf16* xs[MB];
 #pragma unroll
   for (int j = 0; j < MB; ++j) xs[j] = a.x + (int64_t)min(16 * j + r16, a.M - 1) * a.ldx + 8 * kq;
-  float bias[MINE][4];
+  bf16 bias[MINE][4];   // (as they come: a conversion here waits for them ahead of the stream)
   if (a.bias) {   // (uniform)
 #pragma unroll
     for (int b = 0; b < MINE; ++b)
+      if (wave + NW * b < BLOCKS)
 #pragma unroll
-      for (int r = 0; r < 4; ++r) bias[b][r] = (float)a.bias[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
+        for (int r = 0; r < 4; ++r) bias[b][r] = a.bias[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
   }
   f32x4 acc[NT][MB];
   share<NT, MB, true, NW, U>(ws, xs, K, acc);
@@ -157,7 +158,7 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int 
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float z = v[r];
-      if (a.bias) z += bias[b][r];
+      if (a.bias) z += (float)bias[b][r];
       if constexpr (ACT != VY_ACT_NONE) z = vy_act_fwd<ACT>(z, a.act_arg);
       w4[r] = (bf16)z;
     }
