@@ -18,10 +18,13 @@ template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3
 // sequences 602 -> 572 us, 756 -> 690); the experts, whose kernels hold a dense product's code as well, lose (2 layers of width 2048 and 64
 // experts, 16 / 32 sequences: 321 -> 329 us, 411 -> 416).  Behind whole passes each load has a condition of its own: all of a step's
 // behind one branch came one step after the other (16 sequences 338 us, 32 433).
-template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>, bool APART = true>
+// HALF: the last eight lanes of the last weight rows have none; up to 16 rows of X they load nothing (5 x 5984, K = 7424, 29.4 -> 26.7 us, 8 x 12511,
+// K = 7936, 74.5 -> 69.5), above that the other eight lanes' rows again (32 x 6144, K = 1024, 6.6 us either way, with conditions 6.8).
+template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>, bool APART = true, bool HALF = false>
 __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB]) {
   const int kq = (threadIdx.x & 63) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bool there = !HALF || MB > 1 || (threadIdx.x & 15) < 8;   // the last weight row, of this lane
   const bf16x8 zero8 = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -33,6 +36,9 @@ __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* c
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
+        if constexpr (HALF && MB == 1) {
+          if (t == NT - 1) { w[u][t] = there ? __builtin_nontemporal_load(at) : zero8; continue; }
+        }
         if constexpr (ONCE) w[u][t] = __builtin_nontemporal_load(at);
         else w[u][t] = *at;
       }
@@ -50,8 +56,9 @@ __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* c
 #pragma unroll
         for (int t = 0; t < NT; ++t) {
           const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
-          if constexpr (ONCE) w[u][t] = in ? __builtin_nontemporal_load(at) : zero8;
-          else w[u][t] = in ? *at : zero8;
+          const bool row = in && (t < NT - 1 || there);
+          if constexpr (ONCE) w[u][t] = row ? __builtin_nontemporal_load(at) : zero8;
+          else w[u][t] = row ? *at : zero8;
         }
 #pragma unroll
         for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
@@ -127,7 +134,7 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int 
         for (int r = 0; r < 4; ++r) bias[b][r] = a.bias[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
   }
   f32x4 acc[NT][MB];
-  share<NT, MB, true, NW, U>(ws, xs, K, acc);
+  share<NT, MB, true, NW, U, true, HALF>(ws, xs, K, acc);
   __syncthreads();   // (red may still be read from the pass before)
 #pragma unroll
   for (int i = 0; i < BLOCKS; ++i) red[(wave * BLOCKS + i) * 64 + lane] = acc[i / MB][i % MB];
