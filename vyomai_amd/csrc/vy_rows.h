@@ -19,7 +19,7 @@ template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3
 // experts, 16 / 32 sequences: 321 -> 329 us, 411 -> 416).  Behind whole passes each load has a condition of its own: all of a step's
 // behind one branch came one step after the other (16 sequences 338 us, 32 433).
 // HALF: the last eight lanes of the last weight rows have none; up to 16 rows of X they load nothing (5 x 5984, K = 7424, 29.4 -> 26.7 us, 8 x 12511,
-// K = 7936, 74.5 -> 69.5), above that the other eight lanes' rows again (32 x 6144, K = 1024, 6.6 us either way, with conditions 6.8).
+// K = 7936, 74.5 -> 69.5), above that the other eight lanes' rows again (32 x 6144, K = 1024, 6.9 us, with conditions 7.2).
 template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>, bool APART = true, bool HALF = false>
 __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB]) {
   const int kq = (threadIdx.x & 63) >> 4;
