@@ -1,0 +1,94 @@
+"""Weight gradients of which a launch adds one sum to an element -- read, added to and written, no atomics, for tiles inside the gradient --
+and the launches that few rows share: against fp64."""
+import pytest
+import torch
+
+BF, DEV = torch.bfloat16, "cuda"
+
+
+def check(dy, x, dw, db, before):
+    """Sums of M products in fp32: at most M rounding errors of 2^-24 of the sum of their magnitudes, and one of what was there."""
+    M, d = dy.shape[0], dy.double()
+    size = d.abs().T.contiguous() @ x.double().abs() + before.abs().double() + 1.0
+    assert ((dw.double() - (d.T.contiguous() @ x.double() + before.double())).abs() <= (M + 2) * 2.0 ** -24 * size).all()
+    if db is not None:
+        assert ((db.double() - (d.sum(0) - 0.25)).abs() <= (M + 2) * 2.0 ** -24 * (d.abs().sum(0) + 1.0)).all()
+
+
+def problem(g, M, N, K):
+    dy = torch.randn(M, (N + 7) // 8 * 8, device=DEV, generator=g).to(BF)[:, :N]
+    x = torch.randn(M, K, device=DEV, generator=g).to(BF)
+    before = torch.randn(N, K, device=DEV, generator=g)
+    return dy, x, before
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M", [1, 31, 64, 200, 257, 1000])
+def test_grouped(M):
+    """Whole tiles of 256 x 256, tiles that end in the last row or column but eight, and gradients smaller than a tile; up to 256 rows
+    every element gets one sum, beyond that the 11 tiles of the first launch take several pieces a tile and the 264 of the second one."""
+    from vyomai_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    for shapes in ([(256, 256), (248, 264), (768, 512), (255, 8), (520, 256)], [(4096, 4096), (264, 768), (512, 256)]):
+        items, olds = [], []
+        for i, (N, K) in enumerate(shapes):
+            dy, x, before = problem(g, M, N, K)
+            items.append((dy, x, before.clone(), torch.full((N,), -0.25, device=DEV) if i % 2 == 0 else None))
+            olds.append(before)
+        ops.linear_wgrad_grouped(items)
+        for (dy, x, dw, db), before in zip(items, olds):
+            check(dy, x, dw, db, before)
+
+
+@pytest.mark.gpu
+def test_two_sums_for_one_gradient():
+    """A weight that is used twice, and one whose gradient is a block of columns of another's, in one launch."""
+    from vyomai_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(3)
+    (dy, x, before), (dy2, x2, _), (dy3, x3, _) = problem(g, 100, 512, 768), problem(g, 77, 512, 768), problem(g, 200, 512, 256)
+    dw = before.clone()
+    ops.linear_wgrad_grouped([(dy, x, dw, None), (dy2, x2, dw, None), (dy3, x3, dw[:, 256:512], None)])
+    part = torch.zeros(512, 768, device=DEV, dtype=torch.float64)
+    size = before.abs().double() + 1.0
+    for a, b, cols in ((dy, x, slice(0, 768)), (dy2, x2, slice(0, 768)), (dy3, x3, slice(256, 512))):
+        part[:, cols] += a.double().T.contiguous() @ b.double()
+        size[:, cols] += a.double().abs().T.contiguous() @ b.double().abs()
+    assert ((dw.double() - before.double() - part).abs() <= 400 * 2.0 ** -24 * size).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(40, 50265, 256), (200, 16384, 264), (300, 8192, 768)])
+def test_by_itself(M, N, K):
+    """More tiles than the chip takes at once, one piece each: whole ones and the last of an odd count of rows."""
+    from vyomai_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(N)
+    dy, x, before = problem(g, M, N, K)
+    dw, db = before.clone(), torch.full((N,), -0.25, device=DEV)
+    ops.linear_wgrad(dy, x, dw, db, True)
+    check(dy, x, dw, db, before)
+
+
+def test_which_gradients_go_out_together():
+    """Any rows where launches take several layers' gradients; a launch per layer (exchanged gradients) begins at more."""
+    from vyomai_amd import autograd_train as AT
+    g = AT._WgradGroup()
+    p = torch.nn.Parameter(torch.zeros(4))
+    assert g.gathers((768, 768), (p, None)) and g.gathers((2304, 768), [p])
+    assert not g.gathers((50265, 768), (p,)) and not g.gathers((64, 64), (p,)) and not g.gathers((768, 4), (p,))
+    p._vy_exchanged = True
+    assert not g.gathers((768, 768), (p, None))
+
+
+def test_operands_of_another_type_go_out_by_themselves(monkeypatch):
+    from vyomai_amd import autograd_train as AT
+    alone, together = [], []
+    monkeypatch.setattr(AT.ops, "linear_wgrad", lambda dy, x, dw, db, accumulate: alone.append((dy.dtype, accumulate)))
+    monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", lambda items: together.append(len(items)))
+    monkeypatch.setattr(AT.ops, "_raw_stream", lambda: 7)
+    g = AT._WgradGroup()
+    g.armed = True   # (no backward pass to flush it)
+    dw = torch.empty(512, 512, device="meta")
+    for dt in (torch.bfloat16, torch.float32, torch.bfloat16):
+        g.add_tensors(torch.empty(4, 512, dtype=dt), None, dw, None, [])
+    g.flush()
+    assert alone == [(torch.float32, True)] and together == [2]

@@ -144,7 +144,7 @@ class _WgradGroup:
     EXCHANGED, EXCHANGED_MOST = 100, 8                           # exchanged gradients: as many tiles or gradients end a launch
 
     def __init__(self):
-        self.items, self.tiles, self.armed = [], 0, False
+        self.items, self.tiles, self.armed, self.key = [], 0, False, None
 
     def wants(self, dy, w, alpha) -> bool:
         if alpha is not None or not _GROUP_WGRADS:
@@ -152,17 +152,31 @@ class _WgradGroup:
         N, K = w.shape
         return dy.numel() // N >= _GROUP_MIN_ROWS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0
 
+    def gathers(self, shape, members) -> bool:
+        """Gradients that go out with other layers' (none of them exchanged): whatever the rows.  The four of a layer of width 768,
+        microseconds one by one / in launches of 256 tiles: 24 rows 34 / 15, 200 rows 43 / 18, 512 rows 70 / 21, 1665 rows 114 / 36,
+        2047 rows 120 / 40 (width 1024: 42 / 24 to 151 / 64), and half the host's time."""
+        N, K = shape
+        return _GROUP_WGRADS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0 and not any(getattr(p, "_vy_exchanged", False) for p in members)
+
     def add(self, dy, x, w, b) -> None:
         self.add_tensors(dy, x, w.grad, None if b is None else b.grad, [p for p in (w, b) if p is not None])
 
     def add_tensors(self, dy, x, dw, db, members) -> None:
         """dw / db: the fp32 gradient tensors the launch accumulates into (views of the arena); members: the
-        parameters to report ready once it has been enqueued (a packed projection has several)."""
+        parameters to report ready once it has been enqueued (a packed projection has several).  A gradient of another type or
+        on another stream than those that are waiting goes out by itself."""
+        key = dy is not None and (dy.dtype, ops._raw_stream())
+        if self.items and key != self.key:
+            ops.linear_wgrad(dy, x, dw, db, accumulate=True)
+            _notify(*members)
+            return
         tiles = -(-dw.shape[0] // 256) * -(-dw.shape[1] // 256)
         exchanged = any(getattr(p, "_vy_exchanged", False) for p in members)
         if self.tiles + tiles > self.TILES and not exchanged:
             self.flush()
         self.items.append((dy, x, dw, db, members))
+        self.key = key
         # autograd's own post-accumulate hook fires for these parameters as soon as this backward function
         # returns -- the reducer must not take that for "gradient written" (training.BucketReducer._hook)
         for p in members:
@@ -201,9 +215,8 @@ class _WgradGroup:
 
 _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
-_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 116 us one by one,
-# 73 in a launch of their own, 46 of one with its neighbours'.  (So it pays below as well, 1665 rows 109 / 67 / 41 and 1030 rows 94 / 60 / 35:
-# the line dates from launches of one layer.)
+_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # of a launch per layer (exchanged gradients): 2112 rows of width 768, a
+# layer's four gradients, 116 us one by one and 73 in a launch of their own
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group
 _wgrad_group = _WgradGroup()
 
@@ -211,7 +224,7 @@ _wgrad_group = _WgradGroup()
 def _wgrad(dy, x, w: torch.Tensor, b: Optional[torch.Tensor], alpha: Optional[torch.Tensor] = None):
     """-> (dw, db) to return to autograd (None when accumulated in place)."""
     if _direct(w) and (b is None or _direct(b)):
-        if _wgrad_group.wants(dy, w, alpha):
+        if _wgrad_group.wants(dy, w, alpha) or (alpha is None and _wgrad_group.gathers(w.shape, (w, b))):
             _wgrad_group.add(dy, x, w, b)
             return None, None
         ops.linear_wgrad(dy, x, w.grad, None if b is None else b.grad, accumulate=True, alpha=alpha)
@@ -525,10 +538,11 @@ def _packed_wgrad(mod, dy, x, w, b, params):
             ok = ok and all(p.grad.data_ptr() == db0.data_ptr() + off * 4 for p, off in zip(bs, _offsets(bs)))
         if ok:
             dy2 = dy.view(-1, dy.shape[-1])
-            if _GROUP_WGRADS and _GROUP_QKV and dy2.shape[0] >= _GROUP_MIN_ROWS and N * dw.shape[1] >= 512 * 512 and dw.shape[1] % 8 == 0:
+            if _GROUP_WGRADS and _GROUP_QKV and (_wgrad_group.gathers(dw.shape, members) or (
+                    dy2.shape[0] >= _GROUP_MIN_ROWS and N * dw.shape[1] >= 512 * 512 and dw.shape[1] % 8 == 0)):
                 # with the layer's other weight gradients in one grouped launch (27 of its 108 tiles: on its own
                 # this launch ran at 670 TFLOP/s, the group at 850)
-                _wgrad_group.add_tensors(dy2, x.view(-1, x.shape[-1]), dw, db, list(members))
+                _wgrad_group.add_tensors(dy2, x, dw, db, list(members))
             else:
                 ops.linear_wgrad(dy, x, dw, db, accumulate=True)
                 _notify(*members)

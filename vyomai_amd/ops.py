@@ -423,10 +423,11 @@ def linear_wgrad_grouped(items) -> None:
     n = len(items)
     assert 1 <= n <= 12
     arr = (_lib.VyWgradDesc * n)()
-    dt = None
+    dt, rows = None, []   # (rows: copies of operands without uniform rows live until the launch)
     for i, (dy, x, dw, db) in enumerate(items):
         _need_gpu(dy, x, dw, db)
         d2, x2 = _rows(dy), _rows(x)
+        rows.append((d2, x2))
         M, N = d2.shape
         K = x2.shape[1]
         assert x2.shape[0] == M and dw.dtype == torch.float32 and dw.shape == (N, K) and dw.stride(1) == 1
