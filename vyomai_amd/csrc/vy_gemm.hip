@@ -395,7 +395,7 @@ template <int BM, int BN, int WGM, int WGN, bool MF16> struct AccTile {
 // chunks, every iteration waits a full memory latency for it (22 k cycles per tile against 12 k without the operand; residual behind an
 // activation, squared ReLU, 30500 x 768: K = 768 51.4 -> 46.5 us, K = 3072 147 -> 138).
 constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, bool GRAD) {
-  return EPI == 0 && (BM * BN == 256 * 192 || BM * BN == 64 * 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
+  return EPI == 0 && (BM * BN == 256 * 192 || BN == 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
 }
 template <int BM, int BN, int NW, int EPI, bool GRAD>
 struct EpiAhead {
@@ -1288,7 +1288,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
-// 64 x 64 tiles for outputs that give the big tiles too few workgroups: KG groups of 4 waves (2 x 2, 32 x 32 outputs each), each
+// BM x 64 tiles for outputs that give the big tiles too few workgroups: KG groups of 4 waves (2 x 2, BM / 2 x 32 outputs each), each
 // with a ring of NBUF stages of its own, of which NBUF - 1 are on their way (counted vmcnt).  The sums of every `per` stages are added
 // up in order (sum_slices: as many as where K is split over workgroups, so that the result does not hang on the kernel); two groups
 // take half of the slices each -- up to MOST -- and keep each by itself in registers; the second group's go through LDS at the end.
@@ -1296,13 +1296,17 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
 // at most one, two groups in it (0.24 us a stage).  Weights out of the Infinity Cache: 512 x 768 x 768 8.1 us in one group, 6.6 in two;
 // 700 x 1024 x 1024, eight slices, 10.7 and 8.4; sixteen slices, 512 x 768 x 3072: 16.4 (K over workgroups and a second launch 18.1);
 // 256 x 2048 x 2048: 13.2 (18.4).  Four groups: no faster than two on any shape; a fourth and fifth stage: level.
+// Two groups bring a CU 65 KB a microsecond of operands (one group 48), and that is what a launch takes next to a fixed 5 us; so the rows of
+// a tile follow what the fullest CU has to take in, (rows + 64) K.  32 rows spread small outputs over the chip: 512 x 768 x 768 6.9 -> 5.8 us,
+// 512 x 768 x 3072 16.5 -> 12.9, 333 x 1024 x 1024 8.5 -> 6.9, 180 x 2048 x 2048 13.5 -> 10.0; 96 and 128 leave one tile on a CU where 64 leave
+// two on some: 512 x 2304 x 768 9.3 -> 8.3, 1665 x 768 x 768 9.6 -> 8.5, 700 x 2048 x 2048 16.9 -> 13.7 (the chip's 256 CUs, 288, 324 and 352 tiles).
 // ------------------------------------------------------------------------------------------
-template <int KG, int NBUF, int MOST, int EPI, int ACT, bool GRAD>
+template <int KG, int NBUF, int MOST, int BM, int EPI, int ACT, bool GRAD>
 __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
     int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob, int per) {
-  constexpr int BM = 64, BN = 64, WGM = 2, WGN = 2, NW = 4;
-  constexpr int TM = 2, TN = 2, PER = 2;               // 16 x 16 blocks and 1 KiB pieces of either operand per wave
+  constexpr int BN = 64, WGM = 2, WGN = 2, NW = 4;
+  constexpr int TM = BM / 32, TN = 2, PX = BM / 32, PW = 2;   // 16 x 16 blocks and 1 KiB pieces of X and W per wave
   constexpr int STAGE = (BM + BN) * ROWB, RING = NBUF * STAGE;
   static_assert(KG <= 2, "one group, or two");
   constexpr int LDS_BYTES = vy_cmax(vy_cmax(KG * RING, (KG - 1) * MOST * BM * BN * 4), epi_lds_bytes(BM, BN, EPI, 1));   // (MOST slices of the second group)
@@ -1325,16 +1329,20 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
   char* ring = smem + grp * RING;
 
   const int lrow = lane >> 3, slot = lane & 7;
-  const bf16 *xsrc[PER], *wsrc[PER];
-  int kcol[PER];
+  const bf16 *xsrc[PX], *wsrc[PW];
+  int xk[PX], wk[PW];
 #pragma unroll
-  for (int t = 0; t < PER; ++t) {
-    const int R = (wave + NW * t) * 8 + lrow;
-    const int g = slot ^ ((R >> 1) & 7);
+  for (int t = 0; t < PX; ++t) {
+    const int R = (wave + NW * t) * 8 + lrow, g = slot ^ ((R >> 1) & 7);
     int gm = m0 + R; gm = gm < M ? gm : M - 1;
     xsrc[t] = X + (int64_t)gm * ldx + g * 8;
+    xk[t] = g * 8;
+  }
+#pragma unroll
+  for (int t = 0; t < PW; ++t) {
+    const int R = (wave + NW * t) * 8 + lrow, g = slot ^ ((R >> 1) & 7);
     wsrc[t] = W + (int64_t)w_row<EPI>(n0, R, N) * ldw + g * 8;
-    kcol[t] = g * 8;
+    wk[t] = g * 8;
   }
   const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
   const int KT = (K + BK - 1) / BK;
@@ -1344,12 +1352,12 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     char* xb = ring + buf * STAGE;
     const int k0 = kt * BK;
 #pragma unroll
-    for (int t = 0; t < PER; ++t) {
-      const bool in = k0 + kcol[t] < K;
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(in ? xsrc[t] + k0 : zero), (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(in ? wsrc[t] + k0 : zero),
+    for (int t = 0; t < PX; ++t)
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(k0 + xk[t] < K ? xsrc[t] + k0 : zero), (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
+#pragma unroll
+    for (int t = 0; t < PW; ++t)
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(k0 + wk[t] < K ? wsrc[t] + k0 : zero),
                                        (VY_LDS void*)(xb + BM * ROWB + (wave + NW * t) * 1024), 16, 0, 0);
-    }
   };
 
   f32x4 acc[TN][TM];
@@ -1376,7 +1384,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
   auto stages_to = [&](int end) __attribute__((always_inline)) {
     for (; it < end; ++it) {
       // the slice has landed for this wave, NBUF - 2 younger ones may still be on their way (near the end: wait for all) ...
-      if (it + NBUF - 2 < n_it) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER * (NBUF - 2)) : "memory");
+      if (it + NBUF - 2 < n_it) asm volatile("s_waitcnt vmcnt(%0)" ::"n"((PX + PW) * (NBUF - 2)) : "memory");
       else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
       // ... and, behind the barrier, for every wave; every wave has also finished with the buffer that is filled next
       __builtin_amdgcn_s_barrier();
@@ -1389,16 +1397,19 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
         vy_static_for<TN>([&](auto i_c) { constexpr int i = decltype(i_c)::value; wf[ks][i] = vy_lds_read128_off<i * 16 * ROWB>(wa[ks] + boff); });
         vy_static_for<TM>([&](auto j_c) { constexpr int j = decltype(j_c)::value; xf[ks][j] = vy_lds_read128_off<j * 16 * ROWB>(xa[ks] + boff); });
       }
-      vy_lgkm_wait<TN + TM>(wf[0][0], wf[0][1], xf[0][0], xf[0][1]);
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TN + TM) : "memory");
 #pragma unroll
-      for (int i = 0; i < TN; ++i)
+      for (int ks = 0; ks < 2; ++ks) {
+        if (ks) asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
 #pragma unroll
-        for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[0][i], xf[0][j], acc[i][j], 0, 0, 0);
-      vy_lgkm_wait<0>(wf[1][0], wf[1][1], xf[1][0], xf[1][1]);
+        for (int i = 0; i < TN; ++i) vy_tie(wf[ks][i]);
 #pragma unroll
-      for (int i = 0; i < TN; ++i)
+        for (int j = 0; j < TM; ++j) vy_tie(xf[ks][j]);
 #pragma unroll
-        for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[1][i], xf[1][j], acc[i][j], 0, 0, 0);
+        for (int i = 0; i < TN; ++i)
+#pragma unroll
+          for (int j = 0; j < TM; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][i], xf[ks][j], acc[i][j], 0, 0, 0);
+      }
       buf = buf + 1 == NBUF ? 0 : buf + 1;
     }
   };
@@ -1686,7 +1697,7 @@ enum TileKind { T_256x256, T_256x192, T_256x128, T_128x128, T_64x64, T_64x64_TWI
 constexpr int TILE_M[] = {256, 256, 256, 128, 64, 64, 64, 128, 320};
 constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 64, 128, 128};
 constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 512, 256, 512};
-struct Tiling { TileKind kind; int slices; };
+struct Tiling { TileKind kind; int slices, rows; };   // (rows of a tile)
 
 // what a shape costs on a tile, S slices of K added up
 template <TileKind kind>
@@ -1723,6 +1734,15 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     }
   }
 }
+// the same of two groups on tiles of 32, 96 or 128 rows and 64 columns (fits to 450 to 680 shapes, 3 to 6 % added where 64 rows and K over
+// workgroups were as fast as predicted to be slower)
+template <int ROWS>
+inline double rows_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
+  const double n = (double)vy_cdiv(vy_cdiv(M, ROWS) * vy_cdiv(N, 64), (int64_t)chip), KT = (double)vy_cdiv(K, BK), apart = K % BK != 0;
+  if (ROWS == 32) return 3.0 + n * (0.6 + 0.02 * S + KT * (0.154 + 0.044 * apart)) + (S > 4 ? 0.11 * S : 0.0);
+  if (ROWS == 96) return 1.35 + n * (2.35 + 0.215 * S + KT * (0.289 + 0.073 * apart));
+  return 1.2 + n * (2.75 + 0.243 * S + KT * (0.352 + 0.084 * apart));
+}
 // may partial sums of S slices on these tiles lie in `ws` bytes?  256 < M <= 320: one row tile may hold every row, so that a weight
 // crosses L2 -> LDS once (three row tiles of 128: 300 x 2048, K = 6144, 30.8 us, one of 320 25.4.  Two of 128 are as fast as one of 256: 115 shapes)
 template <TileKind kind>
@@ -1756,10 +1776,10 @@ inline int sum_slices(int64_t M, int64_t N, int64_t K) {
 // `behind`: microseconds that K over several workgroups costs besides
 inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes, double behind = 0.0) {
   const int S = sum_slices(M, N, K);
-  Tiling best{T_64x64, S};
+  Tiling best{T_64x64, S, 64};
   double least = 1e30;
-  auto offer = [&](TileKind kind, double us) {
-    if (us < least) { least = us; best.kind = kind; }
+  auto offer = [&](TileKind kind, double us, int rows = 0) {
+    if (us < least) { least = us; best.kind = kind; best.rows = rows ? rows : TILE_M[kind]; }
   };
   offer(T_64x64, tile_cost<T_64x64>(M, N, K, S, chip));
   if (S == 1) {
@@ -1769,10 +1789,19 @@ inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_
     offer(T_128x128, tile_cost<T_128x128>(M, N, K, S, chip));
     return best;
   }
-  if (S <= 4) offer(T_64x64_TWICE, tile_cost<T_64x64_TWICE>(M, N, K, S, chip));
-  else offer(T_64x64_MANY, tile_cost<T_64x64_MANY>(M, N, K, S, chip));
+  const TileKind groups = S <= 4 ? T_64x64_TWICE : T_64x64_MANY;
+  offer(groups, tile_cost<T_64x64_TWICE>(M, N, K, S, chip));
   if (split_fits<T_128x128_SPLIT>(M, N, S, ws_bytes)) offer(T_128x128_SPLIT, behind + tile_cost<T_128x128_SPLIT>(M, N, K, S, chip));
   if (split_fits<T_320x128_SPLIT>(M, N, S, ws_bytes)) offer(T_320x128_SPLIT, behind + tile_cost<T_320x128_SPLIT>(M, N, K, S, chip));
+  // (a sixth faster than K over workgroups -- a quarter where rows of K start inside a line, which the fits tell least well --, or not
+  // at all: nearer to each other either may be the faster one.  39 x 256, K = 1664, 8.5 us on 32 rows, 8.3 over workgroups, but 33 x 512,
+  // K = 1536, 7.7 and 8.5; 152 x 240, K = 1848, 10.6 and 9.0)
+  const double ahead = best.kind == T_128x128_SPLIT || best.kind == T_320x128_SPLIT ? (K % BK ? 1.23 : 1.16) : 1.0;
+  offer(groups, ahead * rows_cost<32>(M, N, K, S, chip), 32);
+  if (S <= 4) {   // (more slices are of outputs that 64 rows a tile leave on part of the chip)
+    offer(groups, ahead * rows_cost<96>(M, N, K, S, chip), 96);
+    offer(groups, ahead * rows_cost<128>(M, N, K, S, chip), 128);
+  }
   return best;
 }
 
@@ -2533,9 +2562,9 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     Tiling t{};
     if (var < 0) {
       t = pick_tiling(M, N, K, chip, ws.bytes);
-      if (t.slices == 1 && (variant == 40 || variant == 41)) t.kind = variant == 40 ? T_256x192 : T_256x256;
+      if (t.slices == 1 && (variant == 40 || variant == 41)) t = {variant == 40 ? T_256x192 : T_256x256, 1, 256};
     }
-    const int bm = var >= 0 ? 256 : TILE_M[t.kind], bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
+    const int bm = var >= 0 ? 256 : t.rows, bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
     const int tn = (int)vy_cdiv(N, bn), tiles = (int)vy_cdiv(M, bm) * tn, threads = var >= 0 ? 512 : TILE_THREADS[t.kind];
     const int KT = (int)vy_cdiv(K, BK), per = t.slices ? (KT + t.slices - 1) / t.slices : KT;
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot)
@@ -2550,9 +2579,17 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
       case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>); break;
       case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, EPI, ACT, GRAD>); break;
       case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
-      case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, EPI, ACT, GRAD>); break;
-      case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, EPI, ACT, GRAD>); break;
-      case T_64x64_MANY: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, EPI, ACT, GRAD>); break;
+      case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, 64, EPI, ACT, GRAD>); break;
+      case T_64x64_TWICE:
+        if (t.rows == 32) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 32, EPI, ACT, GRAD>);
+        else if (t.rows == 96) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 96, EPI, ACT, GRAD>);
+        else if (t.rows == 128) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 128, EPI, ACT, GRAD>);
+        else VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 64, EPI, ACT, GRAD>);
+        break;
+      case T_64x64_MANY:
+        if (t.rows == 32) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, 32, EPI, ACT, GRAD>);
+        else VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, 64, EPI, ACT, GRAD>);
+        break;
       case T_128x128_SPLIT: launch_split<128, 128, 2, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
       case T_320x128_SPLIT: launch_split<320, 128, 4, 2, EPI, ACT, GRAD>(X, ldx, W, ldw, M, N, K, t.slices, ws.p, ep, eq, st); break;
     }
@@ -2570,7 +2607,7 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
   // (with K over several workgroups the factors meet in a pass of their own over the product, 3 us: of 260 shapes none takes over 10 % longer
   // than on the faster way.  Left out of the cost: 264 x 2 x 8192, K = 2048, 40 -> 47 us, 129 x 2 x 512, K = 2048, 12.2 -> 15.3)
   const Tiling t = pick_tiling(M, N, K, 256 / g_chains, splitk_ws(st).bytes, 3.0);
-  const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, TILE_M[t.kind]) * tn;
+  const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, t.rows) * tn;
   const int KT = (int)vy_cdiv(K, BK), per = (KT + t.slices - 1) / t.slices;
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
 #define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0, per)
@@ -2579,9 +2616,17 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
     case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, 2, ACT, false>); break;
     case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, 2, ACT, false>); break;
     case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, 2, ACT, false>); break;
-    case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, 2, ACT, false>); break;
-    case T_64x64_TWICE: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 2, ACT, false>); break;
-    case T_64x64_MANY: VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, 2, ACT, false>); break;
+    case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, 64, 2, ACT, false>); break;
+    case T_64x64_TWICE:
+      if (t.rows == 32) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 32, 2, ACT, false>);
+      else if (t.rows == 96) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 96, 2, ACT, false>);
+      else if (t.rows == 128) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 128, 2, ACT, false>);
+      else VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 2, 64, 2, ACT, false>);
+      break;
+    case T_64x64_MANY:
+      if (t.rows == 32) VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, 32, 2, ACT, false>);
+      else VY_SMALL(gemm_nt_bf16_small_kernel<2, 3, 8, 64, 2, ACT, false>);
+      break;
     default: return VY_ERR_UNSUPPORTED;   // (K split over workgroups)
   }
 #undef VY_TILES
@@ -2725,6 +2770,11 @@ int qkv_impl(const void* x, int64_t ldx, const void* w, int64_t ldw, const void*
 extern "C" int vy_debug_tiling(int64_t M, int64_t N, int64_t K, int64_t ws_bytes, double behind) {
   const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes, behind);
   return (int)t.kind + 16 * t.slices;
+}
+
+// test aid, not part of include/vyom_hip.h: the rows of a tile of that kernel
+extern "C" int vy_debug_tile_rows(int64_t M, int64_t N, int64_t K, int64_t ws_bytes, double behind) {
+  return pick_tiling(M, N, K, 256 / g_chains, ws_bytes, behind).rows;
 }
 
 extern "C" int vy_linear_fwd(const void* x, int64_t ldx, const void* w, int64_t ldw, const void* bias,
