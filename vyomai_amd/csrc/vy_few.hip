@@ -48,16 +48,16 @@ __device__ __forceinline__ void stats(const float (&v)[KC][4], int lane, int n, 
   rstd = rsqrt_refined(vy_wave_sum(q) / (float)n + eps);
 }
 
-template <int EPI, int PRO, int MR, int KC>
-__global__ __launch_bounds__(256) void few_kernel(Args a) {
+template <int EPI, int PRO, int MR, int KC, int NW>
+__global__ __launch_bounds__(64 * NW) void few_kernel(Args a) {
   constexpr int K = 256 * KC, R = (EPI != STORE || KC % 2) ? 2 : 1, P = KC * R / 2;   // columns; weight rows and pieces per wave
   __shared__ __attribute__((aligned(16))) bf16 hs[PRO == PLAIN ? 8 : MR * K];
-  constexpr int SHARES = PRO == PARTS ? 4 / MR : 1;   // waves that add up a row
+  constexpr int SHARES = PRO == PARTS ? 4 / MR : 1;   // waves that add up a row, of the first four
   __shared__ __attribute__((aligned(16))) float sums[SHARES > 1 ? 4 * K : 4];
   const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int units = EPI == STORE ? (a.N + R - 1) / R : EPI == QKV ? a.N / 2 : a.N;   // of R weight rows
-  const int step = (PRO == RMS && a.cache ? gridDim.x - 1 : gridDim.x) * 4;
-  int u = blockIdx.x * 4 + wave;
+  const int step = (PRO == RMS && a.cache ? gridDim.x - 1 : gridDim.x) * NW;
+  int u = blockIdx.x * NW + wave;
 
   if constexpr (PRO == RMS) {
     if (a.cache && blockIdx.x == gridDim.x - 1) {   // one workgroup more: the new tokens' cache rows, a wave each
@@ -143,7 +143,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
 
   if constexpr (PRO != PLAIN) {
     if (a.advance && blockIdx.x == 0)
-      for (int i = threadIdx.x; i < a.n_adv; i += 256) a.advance[a.slots ? a.slots[i] : i] += 1;
+      for (int i = threadIdx.x; i < a.n_adv; i += 64 * NW) a.advance[a.slots ? a.slots[i] : i] += 1;
     bf16x4 v4[KC], g4[KC], b4[KC], xb4[KC];
     if constexpr (PRO == LAYER || PRO == PARTS) {
       if (leads) {
@@ -179,7 +179,7 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
               for (int c = 0; c < KC; ++c) mine[c] += part[i][c];
         }
       if constexpr (SHARES > 1) {
-        if (!leads)
+        if (!leads && wave < 4)
 #pragma unroll
           for (int c = 0; c < KC; ++c) *reinterpret_cast<f32x4*>(sums + wave * K + (64 * c + lane) * 4) = mine[c];
       }
@@ -353,17 +353,33 @@ __global__ __launch_bounds__(256) void few_kernel(Args a) {
   }
 }
 
+template <int EPI, int PRO, int KC, int NW>
+void go_waves(const Args& a, int units, hipStream_t st) {
+  // every workgroup redoes the operand rows, so there are no more of them than fit on the chip at once (by registers): the waves of
+  // wide products loop, with the next rows' weights requested ahead
+  const int most = (PRO != STREAM ? 2048 : KC <= 4 ? 1024 : 512) * 4 / NW, wgs = (units + NW - 1) / NW;
+  const int grid = (wgs < most ? wgs : most) + (PRO == RMS && a.cache ? 1 : 0);
+  if (a.M == 1) hipLaunchKernelGGL((few_kernel<EPI, PRO, 1, KC, NW>), dim3(grid), dim3(64 * NW), 0, st, a);
+  else if (a.M == 2) hipLaunchKernelGGL((few_kernel<EPI, PRO, 2, KC, NW>), dim3(grid), dim3(64 * NW), 0, st, a);
+  else hipLaunchKernelGGL((few_kernel<EPI, PRO, 4, KC, NW>), dim3(grid), dim3(64 * NW), 0, st, a);
+}
 template <int EPI, int PRO, int KC>
 void go_rows(const Args& a, hipStream_t st) {
   constexpr int R = (EPI != STORE || KC % 2) ? 2 : 1;
   const int units = EPI == STORE ? (a.N + R - 1) / R : EPI == QKV ? a.N / 2 : a.N;
-  // every workgroup redoes the operand rows, so there are no more of them than fit on the chip at once (by registers): the waves of
-  // wide products loop, with the next rows' weights requested ahead
-  const int most = PRO != STREAM ? 2048 : KC <= 4 ? 1024 : 512;
-  const int grid = ((units + 3) / 4 < most ? (units + 3) / 4 : most) + (PRO == RMS && a.cache ? 1 : 0);
-  if (a.M == 1) hipLaunchKernelGGL((few_kernel<EPI, PRO, 1, KC>), dim3(grid), dim3(256), 0, st, a);
-  else if (a.M == 2) hipLaunchKernelGGL((few_kernel<EPI, PRO, 2, KC>), dim3(grid), dim3(256), 0, st, a);
-  else hipLaunchKernelGGL((few_kernel<EPI, PRO, 4, KC>), dim3(grid), dim3(256), 0, st, a);
+  // Operand rows that are made are made once a workgroup, so it has as many waves as leave no CU without one: what a CU takes in for them
+  // (the shares, or the stream, the sublayer and two weight rows, out of L2 behind the weights) falls with the workgroups on it.  Up to
+  // 1024 waves in all, which are a workgroup of four per CU at most: 4 (1152 columns of QKV, K = 768, 3.39 us, in workgroups of eight 3.46).
+  // One / four rows on four, eight and sixteen waves: PARTS, 3072 x 768, 5.0, 4.6, 4.9 / 7.9, 6.4, 6.9, 4096 x 1024 7.3, 6.0, 5.4 / 17.2,
+  // 13.3, 9.7; STREAM, 1792 x 1024, 4.1, 3.9, 4.0 / 5.3, 4.6, 4.9, 4096 x 1024 5.1, 4.9, 4.7 / 7.5, 6.3, 5.7; gated, 4096 x 1024, 6.4, 6.3,
+  // 6.2 / 9.0, 8.0, 7.5.  Sixteen waves of K = 2048 do not fit the registers (3584 rows 6.8, 6.5, 9.2).
+  if constexpr (KC <= 4 && (PRO == STREAM || PRO == PARTS)) {
+    if (units > 3072) return go_waves<EPI, PRO, KC, 16>(a, units, st);
+  }
+  if constexpr (PRO != PLAIN) {
+    if (units > 1024) return go_waves<EPI, PRO, KC, 8>(a, units, st);
+  }
+  go_waves<EPI, PRO, KC, 4>(a, units, st);
 }
 
 }  // namespace
