@@ -174,6 +174,26 @@ typedef struct vy_text_layer {
 } vy_text_layer;
 int64_t vy_text_layer_ws_bytes(int64_t B, int64_t L, int32_t h, int32_t dh, int32_t ffn, int dtype);
 int vy_text_layer_fwd(const vy_text_layer* l, const void* x, void* y, int64_t B, int64_t L, void* ws, int64_t ws_bytes, void* stream);
+/* The same layer in training, forward and backward as one call each.  vy_text_layer_kept: what the forward pass writes for the backward
+ * pass, all contiguous -- the rotated queries q [B][h][L][dh] (keys and values: k_new = k, v_new = v of the layer, S = L), the heads o,
+ * the rows ahead of both norms s1 and s2, a and the inner rows, the activation's derivative; lse [B][h][L], a mean and a 1 / deviation per
+ * row of both norms.  replaces: the autograd of the same modules.  vy_text_layer_bwd: dx from dy; the transposed weights [in][out] with
+ * row strides ld_*; dln* are added to, dln*_w and dln*_b fp32 [h dh]; ds2, dpre, ds1 and dqkv [B][L][dq | dk | dv] are what the weight
+ * gradients multiply with inner, a, o and x; da, dheads, ln_ws (2 vy_layernorm_bwd_ws_rows(B L) h dh fp32) and delta [B][h][L] are scratch. */
+typedef struct vy_text_layer_kept {
+  void *q, *o, *s1, *a, *deriv, *inner, *s2;
+  float *lse, *mean1, *rstd1, *mean2, *rstd2;
+} vy_text_layer_kept;
+typedef struct vy_text_layer_grads {
+  const void *wt_qkv, *wt_o, *wt_1, *wt_2;
+  int64_t ld_qkv, ld_o, ld_1, ld_2;
+  float *dln1_w, *dln1_b, *dln2_w, *dln2_b;
+  void *ds2, *dpre, *da, *ds1, *dheads, *dqkv;
+  float *ln_ws, *delta;
+} vy_text_layer_grads;
+int vy_text_layer_train_fwd(const vy_text_layer* l, const vy_text_layer_kept* t, const void* x, void* y, int64_t B, int64_t L, void* stream);
+int vy_text_layer_bwd(const vy_text_layer* l, const vy_text_layer_kept* t, const vy_text_layer_grads* g, const void* dy, void* dx, int64_t B,
+                      int64_t L, void* stream);
 
 /* vy_rmsnorm_fwd: y = x * rsqrt(mean(x^2) + eps) * (w_offset + w); Gemma uses w_offset = 1
  * (Examples/paligemma.ipynb cell 11, GemmaRMSNorm).  Statistics in fp32. */

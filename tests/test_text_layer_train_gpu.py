@@ -1,0 +1,101 @@
+"""A post-LN layer in training as one native call each way (vy_text_layer_train_fwd, vy_text_layer_bwd) against the modules one by one, whose
+launches it makes in their order: the same bits.  What keeps the modules: hooks, dropout, parameters that are not the trainer's."""
+import copy
+
+import pytest
+import torch
+
+from tests.golden import cases
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def model(kind, width, heads, kv=None, layers=2, dropout=0.0):
+    import vyomai_amd as V
+    cfg = cases.with_kv(cases.test_cfg(), kv)
+    cfg.num_hidden_layers, cfg.hidden_size, cfg.num_attention_heads, cfg.intermediate_size = layers, width, heads, 4 * width
+    cfg.hidden_dropout_prob, cfg.vocab_size, cfg.max_position_embeddings = dropout, 500, 512
+    torch.manual_seed(width + heads)
+    m = (V.EncoderModel if kind == "encoder" else V.DecoderModel)(cfg, "rope", "gqa" if kv else None)
+    return m.to(DEV).train()
+
+
+def step(m, ids, mask, dtype=torch.bfloat16, one_by_one=False):
+    """-> (states, gradients by name, native calls) of one backward pass of a fixed loss."""
+    from vyomai_amd import _lib, autograd
+    from vyomai_amd.models import decoder, encoder
+    from vyomai_amd.training import FlatTrainer
+    tr = FlatTrainer(m, lr=0.0, compute_dtype=dtype)
+    seen, real = [], _lib.call
+    _lib.call = lambda name, *a: (seen.append(name), real(name, *a))[1]
+    if one_by_one:
+        encoder.layer_train = decoder.layer_train = lambda *a: None
+    try:
+        tr.zero_grad()
+        out = m.forward_hidden(ids, mask)[0] if hasattr(m, "lm_head") else m(ids, mask).logits
+        w = torch.linspace(-1, 1, out.numel(), device=DEV).view(out.shape)
+        tr.backward((out.float() * w).mean())
+        torch.cuda.synchronize()
+    finally:
+        _lib.call = real
+        encoder.layer_train = decoder.layer_train = autograd.layer_train
+    return out.detach().clone(), {n: p.grad.clone() for n, p in m.named_parameters() if "all_layer" in n}, [n for n in seen if n.startswith("vy_text_layer")]
+
+
+def inputs(B, L, padded):
+    g = torch.Generator(device=DEV).manual_seed(B * L)
+    ids = torch.randint(3, 500, (B, L), generator=g, device=DEV)
+    mask = None
+    if padded:
+        mask = (torch.arange(L, device=DEV)[None] < torch.randint(1, L + 1, (B, 1), generator=g, device=DEV)).long()
+    return ids, mask
+
+
+@pytest.mark.parametrize("kind,width,heads,kv,B,L,padded,dtype", [
+    ("decoder", 512, 8, None, 3, 65, False, torch.bfloat16), ("decoder", 768, 12, 4, 5, 33, True, torch.bfloat16),
+    ("encoder", 512, 8, 4, 2, 128, True, torch.bfloat16), ("decoder", 512, 8, None, 1, 1, False, torch.bfloat16),
+    ("decoder", 256, 2, None, 2, 40, False, torch.bfloat16), ("encoder", 256, 4, None, 2, 19, True, torch.float32)])
+def test_bits_of_the_modules_one_by_one(kind, width, heads, kv, B, L, padded, dtype):
+    ids, mask = inputs(B, L, padded)
+    if kind == "encoder" and mask is None:
+        mask = torch.ones_like(ids)
+    a = model(kind, width, heads, kv)
+    b = copy.deepcopy(a)
+    y, grads, calls = step(a, ids, mask, dtype)
+    y2, grads2, calls2 = step(b, ids, mask, dtype, one_by_one=True)
+    assert calls == ["vy_text_layer_train_fwd"] * 2 + ["vy_text_layer_bwd"] * 2 and not calls2
+    assert torch.equal(y, y2)
+    for n in grads:
+        # (weight gradients of products smaller than 512 x 512, and all in fp32, are sums in atomics: any order)
+        close = (grads[n] - grads2[n]).abs().max() <= 2.0 ** -16 * grads2[n].abs().max() + 1e-12
+        assert torch.equal(grads[n], grads2[n]) or close, n
+        assert grads2[n].abs().max() > 0 or L == 1, n
+
+
+def test_what_keeps_the_modules():
+    ids, mask = inputs(2, 20, False)
+    m = model("decoder", 512, 8)
+    ran = []
+    handle = m.all_layer[0].feed_forward.register_forward_hook(lambda *a: ran.append(1))
+    calls = step(m, ids, mask)[2]
+    handle.remove()
+    assert ran == [1] and calls == ["vy_text_layer_train_fwd", "vy_text_layer_bwd"]      # (the other layer's)
+    assert not step(model("decoder", 512, 8, dropout=0.1), ids, mask)[2]
+    m = model("decoder", 512, 8)
+    m.all_layer[1].attention.out.dense.weight.requires_grad_(False)
+    assert step(m, ids, mask)[2] == ["vy_text_layer_train_fwd", "vy_text_layer_bwd"]
+    m = model("decoder", 512, 8).to(torch.bfloat16)      # (no trainer: gradients are returned)
+    m.forward_hidden(ids, None)[0].float().square().mean().backward()
+    assert all(p.grad is not None for n, p in m.named_parameters() if "all_layer" in n)
+
+
+def test_saved_tensors_go_through_their_hooks():
+    ids, mask = inputs(3, 50, False)
+    a = model("decoder", 512, 8)
+    b = copy.deepcopy(a)
+    want = step(a, ids, mask)
+    packed = []
+    with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.to(DEV)):
+        got = step(b, ids, mask)
+    assert len(packed) >= 6 and torch.equal(got[0], want[0]) and all(torch.equal(got[1][n], want[1][n]) for n in want[1])

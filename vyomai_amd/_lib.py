@@ -34,6 +34,8 @@ PROTOTYPES = {
                     _p, _i64, _i64, _p, _i, _i64, _p, _i64, _p, _i64, _i64,
                     _i64, _i, _i, _i64, _i64, _i, _f, _i, _p],
     "vy_text_layer_fwd": [_p, _p, _p, _i64, _i64, _p, _i64, _p],
+    "vy_text_layer_train_fwd": [_p, _p, _p, _p, _i64, _i64, _p],
+    "vy_text_layer_bwd": [_p, _p, _p, _p, _p, _i64, _i64, _p],
     "vy_attn_decode": [_p, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
                        _p, _i64, _i64, _i, _i, _i64, _i, _f, _i, _p],
     "vy_layernorm_fwd": [_p, _i64, _p, _p, _p, _i64, _p, _p, _i64, _i64, _f, _i, _p],
@@ -153,6 +155,17 @@ class VyTextLayer(C.Structure):
                                   "sin_tab")] + [("pos0", _i64), ("k_new", _p), ("v_new", _p)] + \
                [(n, _i64) for n in ("kn_sb", "kn_sh", "kn_sl", "vn_sb", "vn_sh", "vn_sl")] + [("k", _p), ("v", _p)] + \
                [(n, _i64) for n in ("k_sb", "k_sh", "k_sl", "v_sb", "v_sh", "v_sl", "S", "start_pos")] + [("keypad", _p), ("kp_sb", _i64)]
+
+
+class VyTextLayerKept(C.Structure):
+    """vy_text_layer_kept (include/vyom_hip.h)"""
+    _fields_ = [(n, _p) for n in ("q", "o", "s1", "a", "deriv", "inner", "s2", "lse", "mean1", "rstd1", "mean2", "rstd2")]
+
+
+class VyTextLayerGrads(C.Structure):
+    """vy_text_layer_grads (include/vyom_hip.h)"""
+    _fields_ = [(n, _p) for n in ("wt_qkv", "wt_o", "wt_1", "wt_2")] + [(n, _i64) for n in ("ld_qkv", "ld_o", "ld_1", "ld_2")] + \
+               [(n, _p) for n in ("dln1_w", "dln1_b", "dln2_w", "dln2_b", "ds2", "dpre", "da", "ds1", "dheads", "dqkv", "ln_ws", "delta")]
 
 
 _lib: Optional[C.CDLL] = None

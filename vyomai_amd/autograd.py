@@ -18,7 +18,7 @@ import torch
 
 from . import _lib, ops
 from ._lib import VyomHipError
-from .layers.attention import AttentionSelfOutput, _shadow as _param_shadow
+from .layers.attention import AttentionSelfOutput, _param, _shadow as _param_shadow
 from .layers.ffn import FeedForward
 from .layers.mask import AttnMask
 from .layers.positional_embeddings import resolve_freqs
@@ -137,58 +137,106 @@ def self_attention_block(mod, x, attention_mask, freqs, cache, cache_index, star
 _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks)
 
 
-def layer_forward(att, ff, x, mask, freqs, cache=None, start_pos: int = 0):
-    """ff(att(x), x) of one post-LN layer without gradients as ONE native call (vy_text_layer_fwd), the same launches in the same order:
-    a layer of a few short texts is 50 us of GPU work, and four times that in Python.  None: the modules are to be called one by one --
-    a module of another class, with a hook or with a forward of its own, active dropout, a dense mask, rows that are not contiguous."""
-    if type(ff) is not FeedForward or "_whole_layer" not in type(att).__dict__ or type(att.out) is not AttentionSelfOutput \
-            or not (mask is None or isinstance(mask, AttnMask)):
-        return None
-    aso = att.out
-    if _GLOBAL_HOOKS[0] or _GLOBAL_HOOKS[1]:
-        return None
+def _plain_layer(att, ff, x, mask) -> bool:
+    """May a post-LN layer be one native call?  Not with a module of another class, with a hook or with a forward of its own, active dropout,
+    a dense mask, rows that are not contiguous: the modules are then to be called one by one."""
+    if type(ff) is not FeedForward or "_whole_layer" not in type(att).__dict__ or not (mask is None or isinstance(mask, AttnMask)):
+        return False
+    aso = att._modules["out"]
+    if type(aso) is not AttentionSelfOutput or _GLOBAL_HOOKS[0] or _GLOBAL_HOOKS[1]:
+        return False
     for d in (att.__dict__, aso.__dict__, ff.__dict__):
         if d["_forward_hooks"] or d["_forward_pre_hooks"] or "forward" in d:
-            return None
-    if not x.is_cuda or x.dim() != 3 or not x.is_contiguous() or ops._Lanes.active or torch.is_grad_enabled() or type(x) is not torch.Tensor:
-        return None
-    if (aso.training and aso.dropout.p > 0.0) or (ff.training and ff.dropout.p > 0.0):
+            return False
+    if type(x) is not torch.Tensor or not x.is_cuda or x.dim() != 3 or not x.is_contiguous() or ops._Lanes.active:
+        return False
+    if (aso.training and aso._modules["dropout"].p > 0.0) or (ff.training and ff._modules["dropout"].p > 0.0):
+        return False
+    return (x.dtype is torch.bfloat16 or x.dtype is torch.float32) and x.shape[2] == att.num_attention_heads * att.head_dim and 0 not in x.shape
+
+
+def _layer_params(att, ff):
+    """Weights and biases of the output projection, its norm, the two projections of the feed-forward and its norm."""
+    aso, f = att._modules["out"]._modules, ff._modules
+    return [_param(m, n) for m in (aso["dense"], aso["layernorm"], f["intermediate"], f["out"], f["layernorm"]) for n in ("weight", "bias")]
+
+
+def _fits(keep, x, att, inner) -> bool:
+    """keep: [Wqkv, bqkv, *_layer_params] in the compute type."""
+    dev, d = x.device, x.shape[2]
+    for t in keep:
+        if t is not None and (t.device != dev or not t.is_contiguous()):
+            return False
+    return keep[0].shape == (d + 2 * att.num_key_value_heads * att.head_dim, d) and keep[2].shape == (d, d) and keep[6].shape == (inner, d) \
+        and keep[8].shape == (d, inner)
+
+
+def layer_forward(att, ff, x, mask, freqs, cache=None, start_pos: int = 0):
+    """ff(att(x), x) of one post-LN layer without gradients as ONE native call (vy_text_layer_fwd), the same launches in the same order:
+    a layer of a few short texts is 50 us of GPU work, and four times that in Python.  None: the modules are to be called one by one
+    (_plain_layer)."""
+    if torch.is_grad_enabled() or not _plain_layer(att, ff, x, mask):
         return None
     dt, dev = x.dtype, x.device
-    if dt is not torch.bfloat16 and dt is not torch.float32:
-        return None
     B, L, d = x.shape
     h, hk, dh = att.num_attention_heads, att.num_key_value_heads, att.head_dim
-    if d != h * dh or 0 in x.shape:
-        return None
-    w, b = att._packed_shadow(dt)
-    keep = [w, b] + [_shadow(p, dt) for p in (aso.dense.weight, aso.dense.bias, aso.layernorm.weight, aso.layernorm.bias, ff.intermediate.weight,
-                                              ff.intermediate.bias, ff.out.weight, ff.out.bias, ff.layernorm.weight, ff.layernorm.bias)]
-    inner = ff.intermediate.weight.shape[0]
-    if any(t is not None and (t.device != dev or not t.is_contiguous()) for t in keep) or w.shape != ((h + 2 * hk) * dh, d) \
-            or keep[2].shape != (d, d) or keep[6].shape != (inner, d) or keep[8].shape != (d, inner):
+    keep = [*att._packed_shadow(dt, None, att._params()), *[_shadow(p, dt) for p in _layer_params(att, ff)]]
+    inner = keep[6].shape[0]
+    if not _fits(keep, x, att, inner):
         return None
     cos, sin, pos0 = resolve_freqs(freqs, dev)
+    kv = None
     if cache is None:
         kv = torch.empty((2, B, hk, L, dh), dtype=dt, device=dev)
-        k_new, v_new = kv[0], kv[1]
-        k, v = k_new, v_new
+        k = kv.data_ptr()
+        v, S = k + kv.stride(0) * kv.element_size(), L
+        k_new, v_new, strides = k, v, (hk * L * dh, L * dh, dh) * 4
     else:
-        k_new, v_new = cache.reserve(att.layer_idx, B, hk, L, dh, start_pos, dt, dev)
-        k, v = cache.commit(att.layer_idx)
-    assert k_new.stride(3) == 1 and v_new.stride(3) == 1
-    S = k.shape[2]
+        kn, vn = cache.reserve(att.layer_idx, B, hk, L, dh, start_pos, dt, dev)
+        kc, vc = cache.commit(att.layer_idx)
+        assert kn.stride(3) == 1 and vn.stride(3) == 1
+        k_new, v_new, k, v, S = kn.data_ptr(), vn.data_ptr(), kc.data_ptr(), vc.data_ptr(), kc.shape[2]
+        strides = (*kn.stride()[:3], *vn.stride()[:3], *kc.stride()[:3], *vc.stride()[:3])
     m = _mask_args(mask, B, L, S, dev)
     kp = m["keypad"]
     kind = (_lib.MASK_CAUSAL if m["causal"] else 0) | (_lib.MASK_KEYPAD if kp is not None else 0)
     if kp is not None:
         assert kp.dtype == torch.uint8 and kp.shape == (B, S) and kp.stride(1) == 1
-    p = [ops._ptr(t) for t in keep]
-    desc = _lib.VyTextLayer(h, hk, dh, inner, ff.act, kind, _lib.dtype_code(dt), aso.layernorm.eps, ff.layernorm.eps, *p, ops._ptr(cos),
-                            ops._ptr(sin), pos0, k_new.data_ptr(), v_new.data_ptr(), *k_new.stride()[:3], *v_new.stride()[:3], k.data_ptr(),
-                            v.data_ptr(), *k.stride()[:3], *v.stride()[:3], S, m["start_pos"], ops._ptr(kp),
+    desc = _lib.VyTextLayer(h, hk, dh, inner, ff.act, kind, _lib.dtype_code(dt), att._modules["out"]._modules["layernorm"].eps,
+                            ff._modules["layernorm"].eps, *(None if t is None else t.data_ptr() for t in keep), ops._ptr(cos), ops._ptr(sin),
+                            pos0, k_new, v_new, *strides[:6], k, v, *strides[6:], S, m["start_pos"], ops._ptr(kp),
                             kp.stride(0) if kp is not None else 0)
     return ops.text_layer(desc, x)
+
+
+def layer_train(att, ff, x, mask, freqs):
+    """The same with gradients: one autograd function, whose forward and backward are a native call each (vy_text_layer_train_fwd,
+    vy_text_layer_bwd), where every gradient goes straight into the trainer's arena.  None: as above."""
+    if not torch.is_grad_enabled() or not _plain_layer(att, ff, x, mask):
+        return None
+    from .autograd_train import TextLayerFn, _direct
+    members = att._params()
+    params = [*_layer_params(att, ff), *members]
+    for p in params:
+        if p is not None and not (p.requires_grad and _direct(p)):
+            return None
+    if params[1] is None or params[3] is None or params[7] is None or params[9] is None:   # (biases of norms and projections)
+        return None
+    B, L, _ = x.shape
+    causal, kp, start = False, None, 0
+    if mask is not None:
+        causal, kp, start = mask.causal, mask.keypad, mask.start_pos
+        if kp is not None:
+            if not kp.is_cuda or kp.dtype is not torch.uint8 or kp.dim() != 2 or kp.shape[0] != B or kp.shape[1] < L:
+                return None
+            kp = kp[:, :L].contiguous() if kp.shape[1] != L else kp
+            if kp.stride(1) != 1:
+                return None
+    dt = x.dtype
+    keep = [*att._packed_shadow(dt, None, members), *[_shadow(p, dt) for p in params[:10]]]
+    if not _fits(keep, x, att, keep[6].shape[0]):
+        return None
+    return TextLayerFn.apply(x, kp, att, ff, keep, causal, start, resolve_freqs(freqs, x.device), *params)
 
 
 def _split(x2: torch.Tensor, heads: int, dh: int) -> torch.Tensor:

@@ -12,6 +12,7 @@ Gradient delivery has two modes per parameter:
 """
 from __future__ import annotations
 
+import ctypes
 import os
 
 import weakref
@@ -26,6 +27,7 @@ from .layers.mask import AttnMask
 from .layers.positional_embeddings import resolve_freqs
 
 BF16 = torch.bfloat16
+_ref = ctypes.addressof
 
 
 # bumped by FlatTrainer.step(): its AdamW kernel rewrites weights without touching tensor versions
@@ -54,21 +56,29 @@ class _WtRegistry:
         if self.epoch_done == ep:
             return
         self.epoch_done = ep
-        self.entries = [e for e in self.entries if e[0]() is not None]
-        live = [e for e in self.entries if e[4] >= ep - 1 and getattr(e[0](), "_vy_wt_key", None) != e[1](e[0]())]
+        entries, live = [], []
+        for e in self.entries:
+            owner = e[0]()
+            if owner is None:
+                continue
+            entries.append(e)
+            if e[4] >= ep - 1:
+                key = e[1](owner)
+                if getattr(owner, "_vy_wt_key", None) != key:
+                    live.append((owner, key, e[2](owner), e[3]))
+        self.entries = entries
         if not live:
             return
-        pairs = [(e[2](e[0]()), e[3]) for e in live]
         # one launch per dtype (a bf16 model and an fp32 one trained in the same process share this registry)
-        for dt in sorted({s_.dtype for s_, _ in pairs}, key=str):
-            sub = [(s_, d_) for s_, d_ in pairs if s_.dtype == dt]
+        for dt in sorted({src.dtype for _, _, src, _ in live}, key=str):
+            sub = [(src, dst) for _, _, src, dst in live if src.dtype == dt]
             keys = [(s_.data_ptr(), d_.data_ptr()) for s_, d_ in sub]
             batch = self.batches.get(dt)
             if batch is None or batch.keys != keys:
                 batch = self.batches[dt] = ops.TransposeBatch(sub)
             batch.run()
-        for e in live:
-            e[0]()._vy_wt_key = e[1](e[0]())
+        for owner, key, *_ in live:
+            owner._vy_wt_key = key
 
 
 _WT = _WtRegistry()
@@ -458,6 +468,97 @@ class SelfAttentionFn(torch.autograd.Function):
         return (dx, None, None, None, None, *grads)
 
 
+def _segments(*sizes):
+    """Where segments of so many elements begin in one buffer, each on a line of 128 bytes, and how long it is."""
+    at, out = 0, []
+    for n in sizes:
+        out.append(at)
+        at += (n + 63) // 64 * 64
+    return out, at
+
+
+class TextLayerFn(torch.autograd.Function):
+    """A whole post-LN layer (autograd.layer_train): the launches of SelfAttentionFn, LinearResidualLayerNormFn and FfnBlockFn in their order,
+    behind one native call each way; the gradients of the layer input's residual paths meet in the QKV dgrad's epilogue.  Every parameter's
+    gradient goes into the arena.  keep: [Wqkv, bqkv, Wo, bo, .., both norms, W1, b1, W2, b2] in the compute type."""
+
+    @staticmethod
+    def _layer(att, ff, x, kp, causal, start, rope, keep, kv):
+        """The descriptor; kv: where the keys and the values are."""
+        _, L, _ = x.shape
+        h, hk, dh = att.num_attention_heads, att.num_key_value_heads, att.head_dim
+        cos, sin, pos0 = rope
+        kind = (_lib.MASK_CAUSAL if causal else 0) | (_lib.MASK_KEYPAD if kp is not None else 0)
+        st = (hk * L * dh, L * dh, dh)
+        return _lib.VyTextLayer(h, hk, dh, keep[6].shape[0], ff.act, kind, _lib.dtype_code(x.dtype), att._modules["out"]._modules["layernorm"].eps,
+                                ff._modules["layernorm"].eps, *(None if t is None else t.data_ptr() for t in keep), ops._ptr(cos), ops._ptr(sin),
+                                pos0, *kv, *st, *st, *kv, *st, *st, L, start, ops._ptr(kp), kp.stride(0) if kp is not None else 0)
+
+    @staticmethod
+    def _kept(x, hk_dh, inner, h):
+        """Offsets of [q | o | s1 | a | deriv | inner | s2 | k | v] and of the statistics."""
+        B, L, d = x.shape
+        M = B * L
+        return _segments(M * d, M * d, M * d, M * d, M * inner, M * inner, M * d, M * hk_dh, M * hk_dh), _segments(B * h * L, M, M, M, M)
+
+    @staticmethod
+    def forward(ctx, x, kp, att, ff, keep, causal, start, rope, *params):
+        B, L, d = x.shape
+        h, hk, dh, inner = att.num_attention_heads, att.num_key_value_heads, att.head_dim, keep[6].shape[0]
+        (at, n), (sat, sn) = TextLayerFn._kept(x, hk * dh, inner, h)
+        rows = torch.empty(n, dtype=x.dtype, device=x.device)
+        stats = torch.empty(sn, dtype=torch.float32, device=x.device)
+        y = torch.empty_like(x)
+        e, r0, s0 = x.element_size(), rows.data_ptr(), stats.data_ptr()
+        kept = _lib.VyTextLayerKept(*(r0 + o * e for o in at[:7]), *(s0 + 4 * o for o in sat))
+        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, (r0 + at[7] * e, r0 + at[8] * e))
+        ops._mid_ws(B * L)
+        _lib.call("vy_text_layer_train_fwd", _ref(desc), _ref(kept), x.data_ptr(), y.data_ptr(), B, L, ops._stream())
+        ctx.save_for_backward(x, rows, stats, kp)
+        ctx.meta = (att, ff, causal, start, rope, params)
+        return y
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, rows, stats, kp = ctx.saved_tensors
+        att, ff, causal, start, rope, params = ctx.meta
+        B, L, d = x.shape
+        dt, dev, M = x.dtype, x.device, B * L
+        dy, rows, stats = dy.contiguous(), rows.contiguous(), stats.contiguous()
+        wo, bo, g1, b1, w1, c1, w2, c2, g2, b2 = params[:10]
+        members = att._params()
+        w, b = att._packed(members)
+        keep = [*att._packed_shadow(dt, (w, b), members), *[_shadow(p, dt) for p in params[:10]]]
+        h, hk, dh, inner = att.num_attention_heads, att.num_key_value_heads, att.head_dim, keep[6].shape[0]
+        W = d + 2 * hk * dh
+        (at, _), (sat, _) = TextLayerFn._kept(x, hk * dh, inner, h)
+        e, r0, s0 = x.element_size(), rows.data_ptr(), stats.data_ptr()
+        kept = _lib.VyTextLayerKept(*(r0 + o * e for o in at[:7]), *(s0 + 4 * o for o in sat))
+        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, (r0 + at[7] * e, r0 + at[8] * e))
+        wt = [_wt_packed(att, w, dt, members), _wt(wo, dt), _wt(w1, dt), _wt(w2, dt)]
+        to, n = _segments(M * d, M * inner, M * d, M * d, M * d, M * W)      # ds2, dpre, da, ds1, dheads, dqkv
+        work = torch.empty(n, dtype=dt, device=dev)
+        fo, fn = _segments(2 * _lib.load().vy_layernorm_bwd_ws_rows(M) * d, B * h * L)
+        scratch = torch.empty(fn, dtype=torch.float32, device=dev)
+        dx = torch.empty_like(x)
+        w0, f0 = work.data_ptr(), scratch.data_ptr()
+        # (a gradient that has left the arena since the forward pass is returned)
+        dln = [p.grad if _direct(p) else torch.zeros(d, dtype=torch.float32, device=dev) for p in (g1, b1, g2, b2)]
+        grads = _lib.VyTextLayerGrads(*(t.data_ptr() for t in wt), *(t.stride(0) for t in wt), *(t.data_ptr() for t in dln), *(w0 + o * e for o in to), *(f0 + 4 * o for o in fo))
+        ops._mid_ws(M)
+        _lib.call("vy_text_layer_bwd", _ref(desc), _ref(kept), _ref(grads), dy.data_ptr(), dx.data_ptr(), B, L, ops._stream())
+        dg1, db1, dg2, db2 = (None if _direct(p) else t.to(p.dtype) for p, t in zip((g1, b1, g2, b2), dln))
+        _notify(*(p for p in (g2, b2, g1, b1) if _direct(p)))
+
+        def of(t, o, cols):
+            return t.as_strided((M, cols), (cols, 1), t.storage_offset() + o)
+        dw2 = _wgrad(of(work, to[0], d), of(rows, at[5], inner), w2, c2)
+        dw1 = _wgrad(of(work, to[1], inner), of(rows, at[3], d), w1, c1)
+        dwo = _wgrad(of(work, to[3], d), of(rows, at[1], d), wo, bo)
+        dqkv = _packed_wgrad(att, of(work, to[5], W), x, w, b, params[10:], members)
+        return (dx, *[None] * 7, *dwo, dg1, db1, *dw1, *dw2, dg2, db2, *dqkv)
+
+
 class CrossAttentionFn(torch.autograd.Function):
     """o = merge_heads(softmax(q k^T / sqrt(dh) + key-padding mask) v), q = x Wq^T + bq,
     k/v = enc Wk/v^T + b: the encoder-decoder attention of the seq2seq decoder layer
@@ -514,14 +615,20 @@ def _heads(x2: torch.Tensor, heads: int, dh: int) -> torch.Tensor:
     return x2.view(B, L, heads, dh).permute(0, 2, 1, 3)
 
 
-def _wt_packed(mod, w, dtype):
-    """W^T of the packed projection: keyed on the versions of the member parameters."""
+def _wt_packed(mod, w, dtype, members=None):
+    """W^T of the packed projection: keyed on the versions of the member parameters.  (members: what mod._params() has just returned)"""
+    if members is not None:   # what _wt_cached finds first
+        view = getattr(mod, "_vy_wt_view", None)
+        if view is not None and getattr(mod, "_vy_wt_key", None) == tuple([p._version for p in members]) + (WEIGHT_EPOCH[0], dtype):
+            mod._vy_wt_entry[4] = WEIGHT_EPOCH[0]
+            return view
     return _wt_cached(mod, lambda m: tuple(p._version for p in m._params()) + (WEIGHT_EPOCH[0], dtype),
                       lambda m: m._packed_shadow(dtype)[0])
 
 
-def _packed_wgrad(mod, dy, x, w, b, params):
-    members = mod._params()
+def _packed_wgrad(mod, dy, x, w, b, params, members=None):
+    if members is None:
+        members = mod._params()
     nw = 1 if mod._fused_qkv else 3
     ws, bs = members[:nw], members[nw:]
     if all(_direct(p) for p in members):

@@ -68,6 +68,14 @@ def _shadow(param: torch.Tensor, dtype: torch.dtype) -> torch.Tensor:
     return cache[1]
 
 
+def _param(m: nn.Module, name: str):
+    """m.name, past nn.Module.__getattr__ (a microsecond on every layer and step) where it is a plain parameter."""
+    try:
+        return m._parameters[name]
+    except KeyError:
+        return getattr(m, name)
+
+
 class AttentionSelfOutput(nn.Module):
     """LN(dropout(dense(hidden)) + input).  Reference :42-72."""
 
@@ -123,14 +131,15 @@ class _SelfAttentionBase(nn.Module):
         self._fused_qkv = fused_qkv
 
     # ---- packed [Wq; Wk; Wv] ------------------------------------------------------------------
-    def _packed(self) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    def _packed(self, members=None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
         """The three projection weights as ONE (Nq+2Nkv, K) matrix for the fused kernel.  The
         nn.Linear parameters stay (state_dict names, LoRA wrapping) but are re-pointed to be
         views of one packed buffer the first time, or after .to()/load_state_dict moved them."""
-        self._plain_projections()
+        if members is None:     # (members: what _params() has just returned)
+            members = self._params()
         if self._fused_qkv:
-            return self.qkv.weight, self.qkv.bias
-        ws = [self._modules[n].weight for n in ("query", "key", "value")]
+            return members[0], members[1]
+        ws, bs = members[:3], members[3:]
         packed = getattr(self, "_packed_w", None)
         ok = packed is not None and packed.device == ws[0].device and packed.dtype == ws[0].dtype
         if ok:
@@ -149,7 +158,6 @@ class _SelfAttentionBase(nn.Module):
                     off += w.shape[0]
                 self._packed_w = packed
                 if self.attention_bias:
-                    bs = [self.query.bias, self.key.bias, self.value.bias]
                     pb = torch.cat([b.detach() for b in bs], dim=0).contiguous()
                     off = 0
                     for b in bs:
@@ -159,7 +167,6 @@ class _SelfAttentionBase(nn.Module):
                 else:
                     self._packed_b = None
         elif self.attention_bias:
-            bs = [self.query.bias, self.key.bias, self.value.bias]
             pb = self._packed_b
             off = 0
             for b in bs:
@@ -189,18 +196,18 @@ class _SelfAttentionBase(nn.Module):
                     "Adapter wrappers (LoRA / DoRA) are out of scope here -- merge the low-rank update into "
                     f"`{name}.weight` (W + alpha * B A) and restore the nn.Linear before running on the HIP path.")
 
-    def _packed_shadow(self, dtype: torch.dtype, packed=None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
+    def _packed_shadow(self, dtype: torch.dtype, packed=None, members=None) -> Tuple[torch.Tensor, Optional[torch.Tensor]]:
         """_packed() in the compute dtype.  The packed buffer has a version counter of its own that
         in-place writes to query/key/value.weight (optimizer.step() of a torch optimizer,
         load_state_dict) never bump, so the copy is keyed on the MEMBER parameters' versions (as the
         transposed copy for the backward GEMMs is).  Entry: (key, w, b, packed data_ptr, pinned);
         pinned = views of the trainer's shadow arena, refreshed in place (see _shadow)."""
-        w, b = self._packed() if packed is None else packed     # (packed: what _packed() has just returned)
+        w, b = self._packed(members) if packed is None else packed     # (packed, members: what _packed(), _params() have just returned)
         if w.dtype == dtype:
             return w, b
         if self._fused_qkv:
             return _shadow(w, dtype), _shadow(b, dtype)
-        key = tuple(p._version for p in self._params())
+        key = tuple([p._version for p in (self._params() if members is None else members)])
         c = getattr(self, "_vy_pshadow", None)
         if c is not None and c[1].dtype == dtype and c[1].device == w.device and c[3] == w.data_ptr() \
                 and (c[2] is None) == (b is None):
@@ -219,11 +226,10 @@ class _SelfAttentionBase(nn.Module):
 
     def _params(self):
         self._plain_projections()
-        if self._fused_qkv:
-            return [self.qkv.weight, self.qkv.bias]
-        ps = [self.query.weight, self.key.weight, self.value.weight]
-        if self.attention_bias:
-            ps += [self.query.bias, self.key.bias, self.value.bias]
+        mods = [self._modules[n] if n in self._modules else getattr(self, n) for n in (("qkv",) if self._fused_qkv else ("query", "key", "value"))]
+        ps = [_param(m, "weight") for m in mods]
+        if self._fused_qkv or self.attention_bias:
+            ps += [_param(m, "bias") for m in mods]
         return ps
 
     def _attend(self, hidden_state: torch.Tensor, attention_mask, freqs, cache=None,

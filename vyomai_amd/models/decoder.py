@@ -17,7 +17,7 @@ from ..layers.attention import _SelfAttentionBase
 from ..layers.ffn import FeedForward
 from ..layers.kv_cache import DynamicCacheOne, StaticCacheOne
 from ..layers.mask import AttnMask
-from ..autograd import layer_forward
+from ..autograd import layer_forward, layer_train
 from ..autograd_train import defer_residual_grads as _defer
 from .common import LMHead, PositionMixin
 
@@ -87,6 +87,10 @@ class DecoderLayer(nn.Module):
         if not torch.is_grad_enabled() and (kv_cache is not None or not use_cache):
             y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs,
                               kv_cache if use_cache else None, start_pos)
+            if y is not None:
+                return y, kv_cache
+        if not use_cache:
+            y = layer_train(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
             if y is not None:
                 return y, kv_cache
         _defer(hidden_state)  # training: its residual-path gradients are added in the QKV dgrad epilogue

@@ -10,7 +10,7 @@ import torch.nn as nn
 from ..layers.attention import EncoderAttention, EncoderAttentionGqa
 from ..layers.ffn import FeedForward
 from ..layers.mask import AttnMask
-from ..autograd import layer_forward
+from ..autograd import layer_forward, layer_train
 from ..autograd_train import defer_residual_grads as _defer
 from .common import LMHead, PositionMixin
 
@@ -43,6 +43,9 @@ class EncoderLayer(nn.Module):
             y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
             if y is not None:
                 return y
+        y = layer_train(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
+        if y is not None:
+            return y
         _defer(hidden_state)  # training: its residual-path gradients are added in the QKV dgrad epilogue
         out = self.attention(hidden_state=hidden_state, attention_mask=attention_mask, freqs=freqs)
         return self.feed_forward(out, hidden_state)

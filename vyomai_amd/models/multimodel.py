@@ -9,7 +9,7 @@ from typing import Optional
 import torch
 import torch.nn as nn
 
-from ..autograd import layer_forward
+from ..autograd import layer_forward, layer_train
 from ..autograd_train import defer_residual_grads as _defer
 from ..layers.attention import DecoderAttention, DecoderAttentionGqa
 from ..layers.ffn import FeedForward
@@ -39,6 +39,10 @@ class DecoderLayer(nn.Module):
                 start_pos: Optional[int] = 0) -> torch.Tensor:
         if not torch.is_grad_enabled() and not use_cache:
             y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
+            if y is not None:
+                return y
+        if not use_cache:
+            y = layer_train(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
             if y is not None:
                 return y
         _defer(hidden_state)  # training: its residual-path gradients are added in the QKV dgrad epilogue

@@ -8,7 +8,7 @@ import torch
 import torch.nn as nn
 
 from .. import ops
-from ..autograd import layer_forward
+from ..autograd import layer_forward, layer_train
 from ..autograd_train import defer_residual_grads as _defer
 from ..layers.attention import VisionAttention, _shadow
 from ..layers.ffn import FeedForward
@@ -37,6 +37,9 @@ class EncoderLayer(nn.Module):
             y = layer_forward(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
             if y is not None:
                 return y
+        y = layer_train(self.attention, self.feed_forward, hidden_state, attention_mask, freqs)
+        if y is not None:
+            return y
         _defer(hidden_state)  # training: its residual-path gradients are added in the qkv dgrad epilogue
         out = self.attention(hidden_state=hidden_state, attention_mask=attention_mask, freqs=freqs)
         return self.feed_forward(out, hidden_state)

@@ -72,6 +72,9 @@ def _ordered_params(model: nn.Module) -> List[Tuple[str, nn.Parameter]]:
     return out
 
 
+_DEBUG_READY = bool(os.environ.get("VY_DEBUG_READY"))
+
+
 class FlatArena:
     """fp32 master + fp32 grad (+ optional bf16 shadow) arenas; parameters and their .grad become
     views."""
@@ -276,18 +279,19 @@ class BucketReducer:
         self.dirty = False
 
     def mark_ready(self, p) -> None:
-        self.touched.add(id(p))
+        i = id(p)
+        self.touched.add(i)
         if not self.enabled:
             return
         self.dirty = True
-        b = self.bucket_of[id(p)]
+        b = self.bucket_of[i]
         if self._launched[b]:
             return
-        if id(p) in self._seen:   # a parameter reports once per backward, however many ops fed it
-            if os.environ.get("VY_DEBUG_READY"):
+        if i in self._seen:   # a parameter reports once per backward, however many ops fed it
+            if _DEBUG_READY:
                 print("double ready:", [n for n, q in self.arena.items if q is p])
             return
-        self._seen.add(id(p))
+        self._seen.add(i)
         self._pending[b] += 1
         if self._pending[b] >= self.expect[b]:
             self._ready[b] = True
