@@ -25,8 +25,8 @@ __global__ __launch_bounds__(256) void parallel_in_kernel(Dense in, Dense router
   if constexpr (MB == 0) {
     vy_rows::dense1(first ? in : router, tile);
   } else {
-    __shared__ f32x4 red[vy_rows::DENSE_RED<1, MB>];
-    vy_rows::dense<MB>(first ? in : router, red, tile);
+    __shared__ __attribute__((aligned(16))) char lds[vy_rows::DENSE<MB, 4, 1, false, 2>];
+    vy_rows::dense<MB>(first ? in : router, lds, tile);
   }
 }
 
@@ -98,8 +98,8 @@ __global__ __launch_bounds__(256) void parallel_out_kernel(Dense out, int n_out,
     if (id < n_out) vy_rows::dense1(out, id);
     else expert_rows1<DOWN>(ex, (id - n_out) % tiles, (id - n_out) / tiles);
   } else {
-    __shared__ union { ExpertLds<NT> ex; f32x4 red[vy_rows::DENSE_RED<1, MB>]; } lds;
-    if (id < n_out) vy_rows::dense<MB>(out, lds.red, id);
+    __shared__ __attribute__((aligned(16))) union { ExpertLds<NT> ex; char out[vy_rows::DENSE<MB, 4, 1, false, 2>]; } lds;
+    if (id < n_out) vy_rows::dense<MB>(out, lds.out, id);
     else expert_rows<DOWN, NT>(ex, lds.ex, (id - n_out) % tiles, (id - n_out) / tiles);
   }
 }

@@ -1,8 +1,9 @@
 // Weight-streaming products of few rows (decode): a workgroup of NW = 4 (or 8) waves takes 16 NT rows of W [N][K] against 16 MB rows of X
-// on mfma_f32_16x16x32_bf16 (A = weight rows, B = rows of X), both straight from memory into operand registers: a weight is used
-// once, and X is small enough for L2.  The waves split K by whole 128-byte lines (two k-steps of 32); every wave requests its
-// loads of up to STEPS k-steps before the first product, so a pass over K = 32 NW STEPS costs one memory latency.  W is streamed
-// past the caches (non-temporal) unless other workgroups read it too.
+// on mfma_f32_16x16x32_bf16 (A = weight rows, B = rows of X).  The waves split K by whole 128-byte lines (two k-steps of 32).  Two ways for
+// the operands: through LDS, line by line (share_lds), or straight from memory into operand registers (share) -- every wave requests
+// its loads of up to STEPS k-steps before the first product, W past the caches (non-temporal) unless other workgroups read it too.  A
+// load into registers is 16 rows with 16 bytes a lane, no two neighbouring lanes on a line, and a CU takes in 25 to 30 KB of them a
+// microsecond; of whole lines, 8 lanes each, 60.
 #pragma once
 #include "vy_common.h"
 
@@ -10,21 +11,17 @@ namespace vy_rows {
 
 template <int NT, int MB, int NW = 4> constexpr int RED = (NW - 1) * NT * MB * 64;   // f32x4 of LDS that stream() needs
 template <int NT, int MB, int NW = 4> constexpr int DENSE_RED = NW * NT * MB * 64;   // and dense()
+constexpr int vy_max2(int a, int b) { return a > b ? a : b; }
 template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3 ? 8 : 4;
 
 // acc[t][j] = 16 rows ws[t] x 16 rows xs[j] over the wave's share of K; a lane's pointers are its row (lane & 15) + 8 (lane >> 4).
-// D: a lane owns row lane & 15 of X and rows 4 (lane >> 4) .. + 3 of W.
-// APART: whole passes over K in code of their own, whose loads have no conditions.  dense() gains by it (decoder of width 2048, steps of 5 / 32
-// sequences 602 -> 572 us, 756 -> 690); the experts, whose kernels hold a dense product's code as well, lose (2 layers of width 2048 and 64
-// experts, 16 / 32 sequences: 321 -> 329 us, 411 -> 416).  Behind whole passes each load has a condition of its own: all of a step's
-// behind one branch came one step after the other (16 sequences 338 us, 32 433).
-// HALF: the last eight lanes of the last weight rows have none; up to 16 rows of X they load nothing (5 x 5984, K = 7424, 29.4 -> 26.7 us, 8 x 12511,
-// K = 7936, 74.5 -> 69.5), above that the other eight lanes' rows again (32 x 6144, K = 1024, 6.9 us, with conditions 7.2).
-template <int NT, int MB, bool ONCE, int NW, int U = STEPS<NT, MB>, bool APART = true, bool HALF = false>
+// D: a lane owns row lane & 15 of X and rows 4 (lane >> 4) .. + 3 of W.  Each load has a condition of its own: all of a step's behind one
+// branch came one step after the other (experts of 16 sequences 338 us, 32 433, instead of 321 and 411).
+template <int NT, int MB, bool ONCE, int NW>
 __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB]) {
+  constexpr int U = STEPS<NT, MB>;
   const int kq = (threadIdx.x & 63) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bool there = !HALF || MB > 1 || (threadIdx.x & 15) < 8;   // the last weight row, of this lane
   const bf16x8 zero8 = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
 #pragma unroll
   for (int t = 0; t < NT; ++t)
@@ -32,37 +29,18 @@ __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* c
     for (int j = 0; j < MB; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
   for (int k0 = 64 * wave; k0 < K; k0 += 32 * NW * U) {
     bf16x8 w[U][NT], x[U][MB];
-    auto request = [&](int u, int k) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + 64 * NW * (u >> 1) + 32 * (u & 1);
+      const bool in = k + 8 * kq < K;
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
-        if constexpr (HALF && MB == 1) {
-          if (t == NT - 1) { w[u][t] = there ? __builtin_nontemporal_load(at) : zero8; continue; }
-        }
-        if constexpr (ONCE) w[u][t] = __builtin_nontemporal_load(at);
-        else w[u][t] = *at;
+        if constexpr (ONCE) w[u][t] = in ? __builtin_nontemporal_load(at) : zero8;
+        else w[u][t] = in ? *at : zero8;
       }
 #pragma unroll
-      for (int j = 0; j < MB; ++j) x[u][j] = *reinterpret_cast<const bf16x8*>(xs[j] + k);
-    };
-    if (APART && k0 + 64 * NW * ((U - 1) >> 1) + 64 <= K) {
-#pragma unroll
-      for (int u = 0; u < U; ++u) request(u, k0 + 64 * NW * (u >> 1) + 32 * (u & 1));
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int k = k0 + 64 * NW * (u >> 1) + 32 * (u & 1);
-        const bool in = k + 8 * kq < K;
-#pragma unroll
-        for (int t = 0; t < NT; ++t) {
-          const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
-          const bool row = in && (t < NT - 1 || there);
-          if constexpr (ONCE) w[u][t] = row ? __builtin_nontemporal_load(at) : zero8;
-          else w[u][t] = row ? *at : zero8;
-        }
-#pragma unroll
-        for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
-      }
+      for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
     }
 #pragma unroll
     for (int u = 0; u < U; ++u)
@@ -73,13 +51,95 @@ __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* c
   }
 }
 
+// share() with the operands' way through LDS: a wave's share of K is whole 128-byte lines, and it brings each line of its rows -- 8 rows a
+// load, 8 lanes side by side on a row's line -- into a ring of its own, D lines deep, and multiplies out of it.  No other wave is waited
+// for, and the products and their order are share()'s.  first, rows, count: rows of W from `first`, R of them, below count.
+template <int MB, int R> constexpr int LINE = (2 * MB + R / 8) * 1024;   // bytes of a line of all rows
+template <int NT, int MB, int NW, int D, int R>
+__device__ __forceinline__ void share_lds(const bf16* x, int64_t ldx, int M, const bf16* w, int64_t ldw, int first, int count, int K, char* ring,
+                                          f32x4 (&acc)[NT][MB]) {
+  constexpr int PX = 2 * MB, PW = R / 8, P = PX + PW;
+  static_assert(R % 8 == 0 && R > 16 * (NT - 1) && P * (D - 1) < 64, "vmcnt counts to 63");
+  const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const bf16* at[P];
+  int col[P];
+#pragma unroll
+  for (int p = 0; p < P; ++p) {
+    const int row = 8 * (p < PX ? p : p - PX) + (lane >> 3);
+    col[p] = 8 * ((lane & 7) ^ ((row >> 1) & 7));
+    at[p] = (p < PX ? x + min(row, M - 1) * ldx : w + min(first + row, count - 1) * ldw) + col[p];
+  }
+  const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
+  const int lines = K > 64 * wave ? (K - 64 * wave + 64 * NW - 1) / (64 * NW) : 0;
+  char* mine = ring + wave * D * P * 1024;
+  auto request = [&](int i, int slot) {
+    const int k = 64 * wave + 64 * NW * i;
+#pragma unroll
+    for (int p = 0; p < P; ++p)
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(k + col[p] < K ? at[p] + k : zero), (VY_LDS void*)(mine + (slot * P + p) * 1024), 16, 0, 0);
+  };
+#pragma unroll
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int i = 0; i < D; ++i)
+    if (i < lines) request(i, i);
+  unsigned xa[2][MB], wa[2][NT];   // of the two k-steps of a line in slot 0
+#pragma unroll
+  for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+    for (int j = 0; j < MB; ++j) xa[ks][j] = vy_lds_addr(mine) + (16 * j + r16) * 128 + (((4 * ks + kq) ^ ((r16 >> 1) & 7)) << 4);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+      const int r = 16 * t + (16 * t + 16 > R ? r16 & 7 : r16);
+      wa[ks][t] = vy_lds_addr(mine) + PX * 1024 + r * 128 + (((4 * ks + kq) ^ ((r >> 1) & 7)) << 4);
+    }
+  }
+  int slot = 0;
+  for (int i = 0; i < lines; ++i) {
+    // line i has landed: the younger ones, D - 1 of them or what is left, may be on their way
+    const int younger = min(D - 1, lines - 1 - i);
+    vy_static_for<D>([&](auto n_c) {
+      constexpr int n = decltype(n_c)::value;
+      if (younger == n) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(P * n) : "memory");
+    });
+    const unsigned off = (unsigned)slot * P * 1024;
+    bf16x8 xf[2][MB], wf[2][NT];
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) wf[ks][t] = vy_lds_read128_off<0>(wa[ks][t] + off);
+#pragma unroll
+      for (int j = 0; j < MB; ++j) xf[ks][j] = vy_lds_read128_off<0>(xa[ks][j] + off);
+    }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks) {
+#pragma unroll
+      for (int t = 0; t < NT; ++t) vy_tie(wf[ks][t]);
+#pragma unroll
+      for (int j = 0; j < MB; ++j) vy_tie(xf[ks][j]);
+    }
+    if (i + D < lines) request(i + D, slot);
+#pragma unroll
+    for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+      for (int t = 0; t < NT; ++t)
+#pragma unroll
+        for (int j = 0; j < MB; ++j) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][t], xf[ks][j], acc[t][j], 0, 0, 0);
+    slot = slot + 1 == D ? 0 : slot + 1;
+  }
+}
+
 // share() and, in wave 0, the waves' sums
 template <int NT, int MB, bool ONCE = true, int NW = 4>
 __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB],
                                        f32x4* red) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  share<NT, MB, ONCE, NW, STEPS<NT, MB>, false>(ws, xs, K, acc);
+  share<NT, MB, ONCE, NW>(ws, xs, K, acc);
   __syncthreads();   // (red may still be read from the pass before)
   if (wave)
 #pragma unroll
@@ -111,20 +171,14 @@ struct Dense {
 // LDS, and each wave finishes blocks of its own, biases requested ahead of the stream: finished by the first wave alone, element by
 // element with a wait for each bias and a switch over the activations, a workgroup ran through 3300 instructions behind its last
 // product, 3 of 8.6 us (32 rows, 6144 x 1024).
-template <int MB, int NW = 4, int NT = 1, bool HALF = false, int ACT = VY_ACT_NONE, int U = STEPS<NT, MB>>
-__device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int K) {   // K: columns of x and w that count
+// red: LDS of DENSE bytes, the ring of share_lds before what the waves add up.
+template <int MB, int NW, int NT, bool HALF, int D> constexpr int DENSE = vy_max2(D * NW * LINE<MB, 16 * NT - (HALF ? 8 : 0)>, DENSE_RED<NT, MB, NW> * 16);
+template <int MB, int NW = 4, int NT = 1, bool HALF = false, int ACT = VY_ACT_NONE, int D = 2>
+__device__ __forceinline__ void dense(const Dense& a, char* lds, int tile, int K) {   // K: columns of x and w that count
   constexpr int R = 16 * NT - (HALF ? 8 : 0), BLOCKS = NT * MB, MINE = (BLOCKS + NW - 1) / NW;
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const bf16* ws[NT];
-#pragma unroll
-  for (int t = 0; t < NT; ++t) {
-    const int r = HALF && t == NT - 1 ? r16 & 7 : r16;
-    ws[t] = a.w + (int64_t)min(R * tile + 16 * t + r, a.N - 1) * a.K + 8 * kq;
-  }
-  const bf16* xs[MB];
-#pragma unroll
-  for (int j = 0; j < MB; ++j) xs[j] = a.x + (int64_t)min(16 * j + r16, a.M - 1) * a.ldx + 8 * kq;
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
   bf16 bias[MINE][4];   // (as they come: a conversion here waits for them ahead of the stream)
   if (a.bias) {   // (uniform)
 #pragma unroll
@@ -134,8 +188,8 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int 
         for (int r = 0; r < 4; ++r) bias[b][r] = a.bias[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
   }
   f32x4 acc[NT][MB];
-  share<NT, MB, true, NW, U, true, HALF>(ws, xs, K, acc);
-  __syncthreads();   // (red may still be read from the pass before)
+  share_lds<NT, MB, NW, D, R>(a.x, a.ldx, a.M, a.w, a.K, R * tile, a.N, K, lds, acc);
+  __syncthreads();   // (red lies over the other waves' rings)
 #pragma unroll
   for (int i = 0; i < BLOCKS; ++i) red[(wave * BLOCKS + i) * 64 + lane] = acc[i / MB][i % MB];
   __syncthreads();
@@ -180,8 +234,8 @@ __device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile, int 
   }
 }
 
-template <int MB, int NW = 4, int NT = 1>
-__device__ __forceinline__ void dense(const Dense& a, f32x4* red, int tile) { dense<MB, NW, NT>(a, red, tile, a.K); }
+template <int MB>
+__device__ __forceinline__ void dense(const Dense& a, char* lds, int tile) { dense<MB>(a, lds, tile, a.K); }
 
 // ---- one row of X: a wave per two weight rows ---------------------------------------------------
 // Whole 1 KiB pieces of a row per instruction and no sharing between waves: many small, even pieces of work, which a single

@@ -5,53 +5,49 @@ namespace {
 
 using vy_rows::Dense;
 
-// (32 and 48 rows: eight k-steps ahead instead of four, 6144 x 1024 7.1 -> 6.7 us)
-template <int ACT, int MB, int NW, int NT, bool HALF = false>
+// D: lines of K that a wave has on their way (vy_rows::share_lds)
+template <int ACT, int MB, int NW, int NT, bool HALF, int D>
 __global__ __launch_bounds__(64 * NW) void rows_linear_kernel(Dense a) {
-  __shared__ f32x4 red[vy_rows::DENSE_RED<NT, MB, NW>];
-  vy_rows::dense<MB, NW, NT, HALF, ACT, NT == 2 || NT == 3 ? 8 : vy_rows::STEPS<NT, MB>>(a, red, blockIdx.x, a.K);
+  __shared__ __attribute__((aligned(16))) char lds[vy_rows::DENSE<MB, NW, NT, HALF, D>];
+  vy_rows::dense<MB, NW, NT, HALF, ACT, D>(a, lds, blockIdx.x, a.K);
 }
 
 // K cut into slices of `len` columns: fp32 partial sums [slice][M][N]
 template <int MB, int NT>
 __global__ __launch_bounds__(256) void rows_parts_kernel(Dense a, int len, int tiles) {
-  __shared__ f32x4 red[vy_rows::DENSE_RED<NT, MB>];
+  __shared__ __attribute__((aligned(16))) char lds[vy_rows::DENSE<MB, 4, NT, false, 2>];
   const int slice = blockIdx.x / tiles, tile = blockIdx.x - slice * tiles, k0 = slice * len;
   a.x += k0;
   a.w += k0;
   a.y = (float*)a.y + (int64_t)slice * a.M * a.N;
-  vy_rows::dense<MB, 4, NT>(a, red, tile, min(len, a.K - k0));
+  vy_rows::dense<MB, 4, NT>(a, lds, tile, min(len, a.K - k0));
 }
 
-// Weight rows of a workgroup.  What one CU takes in (25 to 40 GB/s) sets the time, and a workgroup reads x -- 16 MB rows of K -- beside
-// its weights: so the rows that make the fullest CU read least.  24 are one workgroup a CU where 16 are two on half of them.  32 rows,
-// weights from HBM: 6144 x 1024 8.3 us on 16, 6.7 on 24, 6.9 on 32 (8.6 before dense() spread its last part over the waves); 8192 x 1024
-// 8.4, 10.3, 6.9 (9.3); 6144 x 2048 14.5, 11.0, 11.5 (12.9); 12288 x 2048 15.7 on 48, 18.9 on 24 (19.4); 32000 x 1024 18.7 on 64, 20.1 on
-// 32 (23.0).  Up to 16 rows x weighs half and wide products stream from HBM, so only 24 in place of 16 pays, up to 16384: 8 rows,
-// 6144 x 1024 6.1 -> 5.2, 6144 x 2048 9.3 -> 8.5, 32000 x 1024 16.3 (24: 17.6).
+// Weight rows of a workgroup.  What one CU takes in sets the time, and a workgroup reads x -- 16 MB rows of K -- beside its weights: so the
+// rows that make the fullest CU read least, as long as 64 of them bring everything in one round; wider products (vocabularies) have 64
+// rows, beside 32 rows of x 48, and two lines on their way instead of three, so that two workgroups share a CU.  With the operands by
+// whole lines through LDS instead of 16 rows a load straight into the product's registers (which a CU takes in at 25 to 30 KB a
+// microsecond: 4.5 of the 6.8 us below): 32 rows, 6144 x 1024 6.8 -> 5.2 us, 8192 x 1024 7.1 -> 5.7, 2048 x 1024 5.5 -> 3.7, 6144 x 2048
+// 11.5 -> 7.8, 12288 x 2048 16.7 -> 12.6, 16384 x 2048 21.5 -> 14.6, 32000 x 1024 20.0 -> 15.3 (64 rows a workgroup 17.6), 32000 x 2048 38.2 ->
+// 27.7; 8 rows 5.4 -> 4.6, 6.6 -> 5.2, 4.3 -> 3.4, 8.8 -> 6.9, 14.7 -> 12.0, 20.1 -> 13.8, 18.8 -> 13.9, 34.9 -> 24.8.  The same bits.
 template <int ACT, int MB>
 void rows_go(const Dense& a, hipStream_t st) {
-  // few workgroups with long rows: twice the waves each
+  // few workgroups with long rows: twice the waves each (32 rows, 2048 x 2048 8.2 -> 4.9 us)
   if (a.N <= 4096 && a.K >= 2048) {
-    hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 8, 1>), dim3((unsigned)vy_cdiv(a.N, 16)), dim3(512), 0, st, a);
+    hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 8, 1, false, 2>), dim3((unsigned)vy_cdiv(a.N, 16)), dim3(512), 0, st, a);
     return;
   }
   auto rounds = [&](int r) { return vy_cdiv(vy_cdiv(a.N, r), 256); };
   int best = 16;
-  if constexpr (MB == 1) {
-    if (a.N <= 16384 && rounds(24) < rounds(16)) best = 24;
-  } else {
-    for (const int r : {24, 32, 48, 64})
-      if (rounds(r) * (16 * MB + r) < rounds(best) * (16 * MB + best)) best = r;
-  }
+  for (const int r : {24, 32, 48, 64})
+    if (rounds(r) * (16 * MB + r) < rounds(best) * (16 * MB + best)) best = r;
+  if (rounds(64) > 1) best = MB == 1 ? 64 : 48;
   const dim3 grid((unsigned)vy_cdiv(a.N, best)), block(256);
-  if (best == 16) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 1>), grid, block, 0, st, a);
-  else if (best == 24) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 2, true>), grid, block, 0, st, a);
-  else if constexpr (MB > 1) {
-    if (best == 32) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 2>), grid, block, 0, st, a);
-    else if (best == 48) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 3>), grid, block, 0, st, a);
-    else hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 4>), grid, block, 0, st, a);
-  }
+  if (best == 16) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 1, false, 3>), grid, block, 0, st, a);
+  else if (best == 24) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 2, true, 3>), grid, block, 0, st, a);
+  else if (best == 32) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 2, false, 3>), grid, block, 0, st, a);
+  else if (best == 48) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 3, false, 2>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 4, false, 2>), grid, block, 0, st, a);
 }
 
 template <int ACT>
@@ -81,7 +77,8 @@ int vy_rows_linear(const void* x, const void* w, const void* bias, int act, floa
 // or 64 workgroups of 32 columns, and what one CU takes in (25 to 40 GB/s) sets its time; slices bring the workgroups to 256, and
 // wider tiles halve the times x is read: 64 columns where they still are 256 workgroups.  32 rows, 1024 x 6144: 23.3 -> 6.8 us;
 // 2048 x 8192: 11.4 (32 columns: 12.7); 2048 x 12288: 43.2 -> 16.6 (17.9); 1024 x 1024: 6.1 -> 3.5; 8 rows: 13.3 -> 5.4, 24.8 -> 14.2,
-// 4.2 -> 3.2 (weights from HBM).  A slice keeps at least 128 columns: 8 waves' lines.
+// 4.2 -> 3.2 (weights from HBM); with whole lines through LDS 5.1, 9.4, 12.7, 3.3 and 4.6, 11.3, 3.0.  A slice keeps at least 128 columns:
+// 8 waves' lines.
 int vy_rows_parts(const void* x, const void* w, float* parts, int64_t M, int64_t N, int64_t K, hipStream_t st) {
   if (M < 5 || M > 32 || N < 512 || N > 4096 || K > INT32_MAX || K < 1024 || K % 8 || (uintptr_t)x % 16 || (uintptr_t)w % 16 ||
       (uintptr_t)parts % 16)
