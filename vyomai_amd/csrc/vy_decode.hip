@@ -31,9 +31,9 @@ struct DecDbg { unsigned long long* buf; int slot; int max_wg; };
   if constexpr (DBG) { __builtin_amdgcn_sched_barrier(0); dbg_t[i] = wall_clock64(); __builtin_amdgcn_sched_barrier(0); }
 #define DEC_STAMP_FLUSH()                                                                                     \
   if constexpr (DBG) {                                                                                        \
-    if (threadIdx.x == 0 && (int)(blockIdx.x + gridDim.x * blockIdx.y) < dbg.max_wg) {                        \
-      for (int i_ = 0; i_ < 8; ++i_)                                                                          \
-        dbg.buf[((long long)dbg.slot * dbg.max_wg + blockIdx.x + gridDim.x * blockIdx.y) * 8 + i_] = dbg_t[i_]; \
+    const int wg_ = (int)(blockIdx.x + gridDim.x * (blockIdx.y + gridDim.y * blockIdx.z));                    \
+    if (threadIdx.x == 0 && wg_ < dbg.max_wg) {                                                               \
+      for (int i_ = 0; i_ < 8; ++i_) dbg.buf[((long long)dbg.slot * dbg.max_wg + wg_) * 8 + i_] = dbg_t[i_];  \
     }                                                                                                         \
   }
 
@@ -125,24 +125,42 @@ __device__ __forceinline__ float dec_swap32(float v, bool upper) {
   return __builtin_bit_cast(float, upper ? (unsigned)s[0] : (unsigned)s[1]);
 }
 
+// The operands come by whole lines: 8 rows a load, 8 lanes side by side on the 128 bytes of a row, straight into LDS.  A CU takes in about
+// 60 KB of these a microsecond and 25 to 30 of MFMA fragments requested by the lanes that need them (16 rows and 16 bytes a lane).
+// 16-byte chunk c of row r lies at c ^ (r / 2 & 7) of its line, so that the fragment reads (16 rows, 4 chunks) meet no bank twice.
+// With the tiles and the LayerNorm operands below, 32 sequences of width 768: a layer's projections 5.6 (QKV), 4.3, 6.9 (LayerNorm and
+// GELU), 4.5 -> 4.2, 4.0, 4.7, 3.7 us, of which a launch alone is 2.4; 12 layers, prompts of 512 and 24 tokens, all of it 15.9 -> 14.2 ms.
+__device__ __forceinline__ void dec_line(const bf16* g, char* l) {
+  __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)g, (VY_LDS void*)l, 16, 0, 0);
+}
+__device__ __forceinline__ bf16x8 dec_frag(const char* line, int r, int chunk) {
+  return *reinterpret_cast<const bf16x8*>(line + r * 128 + ((chunk ^ ((r >> 1) & 7)) << 4));
+}
+
 // ------------------------------------------------------------------------------------------
-// 16 output columns x 32 rows per workgroup, the K range of the workgroup (4 * U k-steps of 32) split over the
-// 4 waves: wave w takes k-steps w, w + 4, ... -- the four waves together read whole 128-byte lines of every
-// weight row.  mfma_f32_16x16x32_bf16 with A = 16 weight rows, B = 16 batch rows (two row blocks); D[n][m]: a
-// lane owns batch row lane & 15 (and + 16) and the 4 consecutive columns 4 * (lane >> 4) .. + 3.  With fused RoPE
-// a workgroup takes columns {d0 .. d0+7} and {d0+32 .. d0+39} of one 64-wide head: a rotary pair sits in lanes l
-// and l ^ 32.  Same arithmetic as gemm_skinny16_bf16_kernel (vy_gemm.hip).
+// 16 NT output columns x 16 MB rows per workgroup, its K range (4 * U k-steps of 32) split over the 4 waves: the waves bring the lines
+// in turn, wave w multiplies k-steps w, w + 4, ...  mfma_f32_16x16x32_bf16 with A = 16 weight rows, B = 16 batch rows; D[n][m]: a lane
+// owns batch row lane & 15 and the 4 consecutive columns 4 * (lane >> 4) .. + 3.  What the waves add up goes through LDS and a wave a
+// block finishes it, the waves' sums in their order.  With fused RoPE a workgroup takes columns {d0 .. d0+7} and {d0+32 .. d0+39} of one
+// 64-wide head: a rotary pair sits in lanes l and l ^ 32.  Same arithmetic as gemm_skinny16_bf16_kernel (vy_gemm.hip).
 // ------------------------------------------------------------------------------------------
 // LNP: the rows of X are normalised on the way in -- y = act(LayerNorm(x) W^T + b) without a LayerNorm launch in front.
-// A workgroup holds every element of all 32 rows anyway (its four waves split K), so the row statistics are two
+// A workgroup holds every element of its rows anyway (its four waves split K), so the row statistics are two
 // reductions over values already in registers: over the 4 lane rows of a wave (permlane swaps), then over the 4 waves
 // through LDS (one barrier each: mean, then the sum of squared deviations -- the two-pass form of dec_finish_ln_kernel,
 // same rsqrt refinement, the normalised value rounded to bf16 exactly where that kernel stores it).  The launch this
-// saves is a ~4.3 us link of the step's dependent chain; every workgroup redoes the statistics (25 k elements: noise).
-template <int EPI, int ACT, int U, bool DBG, bool LNP = false>
+// saves is a ~4.3 us link of the step's dependent chain.  Every workgroup redoes the statistics and the normalisation, some ten
+// vector instructions an element: 16 rows x 32 columns instead of 32 x 16 halve them for the same bytes (768 x 3072, 32 rows: 6.15 ->
+// 5.3 us), and gamma and beta come into LDS once instead of to every lane (-> 4.7).
+template <int EPI, int ACT, int U, bool DBG, bool LNP, int MB, int NT>
 __global__ __launch_bounds__(256) void dec_gemm16_kernel(const DecGemmArgs p, const DecDbg dbg) {
-  __shared__ float red[3][8][64];
-  __shared__ float lnred[2][4][32];
+  constexpr int XG = 2 * MB, GROUPS = XG + 2 * NT, LINE = GROUPS * 1024;   // groups of 8 rows of a line in LDS: of X, of W
+  constexpr int BLOCKS = MB * NT;
+  static_assert(BLOCKS <= 4 && (EPI != DEC_QKV || NT == 1), "a wave finishes one block; a rotary pair is of one block");
+  __shared__ __align__(16) char lines[2 * U * LINE];   // K range: 128 U columns
+  __shared__ f32x4 red[4][BLOCKS][64];
+  __shared__ float lnred[2][4][16 * MB];
+  __shared__ __align__(16) bf16 lnp[LNP ? 2 * 128 * U : 8];   // gamma, beta
   unsigned long long dbg_t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   DEC_STAMP(0)
   if constexpr (DBG) { asm volatile("" ::"s"(p.M), "s"(p.ldw)); }
@@ -150,42 +168,42 @@ __global__ __launch_bounds__(256) void dec_gemm16_kernel(const DecGemmArgs p, co
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
-  const int nb = blockIdx.x;
+  const int row0 = (int)blockIdx.z * 16 * MB, rows = min(p.M - row0, 16 * MB);
   const bool rope_map = EPI == DEC_QKV && p.rope;
-  int col = nb * 16 + r16;
-  if (rope_map) col = (nb >> 2) * 64 + (nb & 3) * 8 + (r16 < 8 ? r16 : 24 + r16);
-  const int m0 = r16 < p.M ? r16 : p.M - 1, m1 = 16 + r16 < p.M ? 16 + r16 : p.M - 1;
-  const int kbase = ((int)blockIdx.y * 4 * U + wave) * 32 + kq * 8;
-  const bf16* wp = p.W + (long long)col * p.ldw + kbase;
-  const bf16* xp0 = p.X + (long long)m0 * p.ldx + kbase;
-  const bf16* xp1 = p.X + (long long)m1 * p.ldx + kbase;
-  if constexpr (DBG) { asm volatile("" ::"v"(wp), "v"(xp0), "v"(xp1)); }
+  // a lane's places of the loads: row lane / 8 of each group, 16 bytes of a line
+  const bf16* at[GROUPS];
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const int row = 8 * g + (lane >> 3);
+    const int k = (int)blockIdx.y * 128 * U + 64 * wave + 8 * ((lane & 7) ^ ((row >> 1) & 7));
+    int n = row - 16 * MB;
+    n = rope_map ? ((int)blockIdx.x >> 2) * 64 + ((int)blockIdx.x & 3) * 8 + (n < 8 ? n : 24 + n) : (int)blockIdx.x * 16 * NT + n;
+    at[g] = g < XG ? p.X + (long long)(row0 + min(row, rows - 1)) * p.ldx + k : p.W + (long long)n * p.ldw + k;
+  }
+  if constexpr (DBG) { asm volatile("" ::"v"(at[0]), "v"(at[XG]), "v"(at[XG + 1])); }
   DEC_STAMP(6)
-  // this lane's output quad: columns nq0 .. nq0 + 3
+  // the block that this wave finishes: rows m of X, four columns a lane from nq0
+  const int nb = (int)blockIdx.x * NT + (wave % BLOCKS) / MB;
   const int nq0 = rope_map ? (nb >> 2) * 64 + (nb & 3) * 8 + 4 * (kq & 1) + (kq >= 2 ? 32 : 0) : nb * 16 + 4 * kq;
+  const int mr = 16 * ((wave % BLOCKS) % MB) + r16, m = row0 + min(mr, rows - 1);
 
-  // every load of the launch, oldest first: bias, the weight / activation fragments, then what depends on the
-  // position (read on the device under a graph)
+  // every load of the launch: bias, the operands' lines, then what depends on the position (read on the device under a graph)
   bf16x4 bias4 = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
   if (EPI != DEC_PART && p.bias) bias4 = *reinterpret_cast<const bf16x4*>(p.bias + nq0);
-  bf16x8 a[U], b0[U], b1[U];
-  bf16x8 lg[LNP ? U : 1], lb[LNP ? U : 1];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    a[u] = *reinterpret_cast<const bf16x8*>(wp + 128 * u);
-    b0[u] = *reinterpret_cast<const bf16x8*>(xp0 + 128 * u);
-    b1[u] = *reinterpret_cast<const bf16x8*>(xp1 + 128 * u);
-    if constexpr (LNP) {
-      lg[u] = *reinterpret_cast<const bf16x8*>(p.ln_g + kbase + 128 * u);
-      lb[u] = *reinterpret_cast<const bf16x8*>(p.ln_b + kbase + 128 * u);
+  for (int i = 0; i < U / 2; ++i)
+#pragma unroll
+    for (int g = GROUPS - 1; g >= 0; --g)
+      if (g >= XG || 8 * g < rows) dec_line(at[g] + 256 * i, lines + (wave + 4 * i) * LINE + g * 1024);
+  if constexpr (LNP) {
+    if (wave < U / 2) {
+      const int c = 64 * wave + lane;
+      dec_line(c < 16 * U ? p.ln_g + 8 * c : p.ln_b + 8 * (c - 16 * U), reinterpret_cast<char*>(lnp) + 1024 * wave);
     }
   }
-  bf16x4 res0 = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f}, res1 = res0;
+  bf16x4 res = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
   if constexpr (EPI == DEC_STORE) {
-    if (p.residual) {   // (workgroup-uniform; requested with everything else, used by wave 0 at the very end)
-      res0 = *reinterpret_cast<const bf16x4*>(p.residual + (long long)m0 * p.ldr + nq0);
-      res1 = *reinterpret_cast<const bf16x4*>(p.residual + (long long)m1 * p.ldr + nq0);
-    }
+    if (p.residual) res = *reinterpret_cast<const bf16x4*>(p.residual + (long long)m * p.ldr + nq0);   // (workgroup-uniform)
   }
   int pos = 0;
   f32x4 cos4 = {1.f, 1.f, 1.f, 1.f}, sin4 = {0.f, 0.f, 0.f, 0.f};
@@ -199,86 +217,107 @@ __global__ __launch_bounds__(256) void dec_gemm16_kernel(const DecGemmArgs p, co
     }
   }
   DEC_STAMP(1)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
+  bf16x8 a[U][NT], b[U][MB];
+#pragma unroll
+  for (int u = 0; u < U; ++u) {   // k-step wave + 4 u: half a line
+    const char* line = lines + ((wave + 4 * u) >> 1) * LINE;
+    const int ch = 4 * (wave & 1) + kq;
+#pragma unroll
+    for (int j = 0; j < MB; ++j) b[u][j] = dec_frag(line, 16 * j + r16, ch);
+#pragma unroll
+    for (int t = 0; t < NT; ++t) a[u][t] = dec_frag(line, 16 * (MB + t) + r16, ch);
+  }
   if constexpr (LNP) {
     const float inv_n = 1.0f / (float)(128 * U);   // K = 4 waves x U k-steps x 32
-    float s0 = 0.f, s1 = 0.f;
+    float mean[MB], rstd[MB];
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int j = 0; j < MB; ++j) {
+      float s = 0.f;
 #pragma unroll
-      for (int e = 0; e < 8; ++e) { s0 += (float)b0[u][e]; s1 += (float)b1[u][e]; }
-    s0 = dec_rows_sum(s0); s1 = dec_rows_sum(s1);
-    if (kq == 0) { lnred[0][wave][r16] = s0; lnred[0][wave][16 + r16] = s1; }
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) s += (float)b[u][j][e];
+      s = dec_rows_sum(s);
+      if (kq == 0) lnred[0][wave][16 * j + r16] = s;
+    }
     __syncthreads();
-    const float mean0 = (lnred[0][0][r16] + lnred[0][1][r16] + lnred[0][2][r16] + lnred[0][3][r16]) * inv_n;
-    const float mean1 = (lnred[0][0][16 + r16] + lnred[0][1][16 + r16] + lnred[0][2][16 + r16] + lnred[0][3][16 + r16]) * inv_n;
-    float q0 = 0.f, q1 = 0.f;
 #pragma unroll
-    for (int u = 0; u < U; ++u)
+    for (int j = 0; j < MB; ++j) {
+      const int r = 16 * j + r16;
+      mean[j] = (lnred[0][0][r] + lnred[0][1][r] + lnred[0][2][r] + lnred[0][3][r]) * inv_n;
+      float q = 0.f;
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          const float d = (float)b[u][j][e] - mean[j];
+          q += d * d;
+        }
+      q = dec_rows_sum(q);
+      if (kq == 0) lnred[1][wave][r] = q;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < MB; ++j) {
+      const int r = 16 * j + r16;
+      const float var = (lnred[1][0][r] + lnred[1][1][r] + lnred[1][2][r] + lnred[1][3][r]) * inv_n + p.ln_eps;
+      rstd[j] = rsqrtf(var);
+      rstd[j] = rstd[j] * (1.5f - 0.5f * var * rstd[j] * rstd[j]);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const bf16x8 lg = *reinterpret_cast<const bf16x8*>(lnp + (wave + 4 * u) * 32 + kq * 8);
+      const bf16x8 lb = *reinterpret_cast<const bf16x8*>(lnp + 128 * U + (wave + 4 * u) * 32 + kq * 8);
 #pragma unroll
       for (int e = 0; e < 8; ++e) {
-        const float d0 = (float)b0[u][e] - mean0, d1 = (float)b1[u][e] - mean1;
-        q0 += d0 * d0; q1 += d1 * d1;
+        const float g = (float)lg[e], be = (float)lb[e];
+#pragma unroll
+        for (int j = 0; j < MB; ++j) b[u][j][e] = (bf16)(((float)b[u][j][e] - mean[j]) * rstd[j] * g + be);
       }
-    q0 = dec_rows_sum(q0); q1 = dec_rows_sum(q1);
-    if (kq == 0) { lnred[1][wave][r16] = q0; lnred[1][wave][16 + r16] = q1; }
-    __syncthreads();
-    const float var0 = (lnred[1][0][r16] + lnred[1][1][r16] + lnred[1][2][r16] + lnred[1][3][r16]) * inv_n + p.ln_eps;
-    const float var1 = (lnred[1][0][16 + r16] + lnred[1][1][16 + r16] + lnred[1][2][16 + r16] + lnred[1][3][16 + r16]) * inv_n + p.ln_eps;
-    float r0 = rsqrtf(var0), r1 = rsqrtf(var1);
-    r0 = r0 * (1.5f - 0.5f * var0 * r0 * r0);
-    r1 = r1 * (1.5f - 0.5f * var1 * r1 * r1);
-#pragma unroll
-    for (int u = 0; u < U; ++u)
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        const float g = (float)lg[u][e], be = (float)lb[u][e];
-        b0[u][e] = (bf16)(((float)b0[u][e] - mean0) * r0 * g + be);
-        b1[u][e] = (bf16)(((float)b1[u][e] - mean1) * r1 * g + be);
-      }
+    }
   }
-  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
+  f32x4 acc[NT][MB];
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b0[u], acc0, 0, 0, 0);
-    acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b1[u], acc1, 0, 0, 0);
-  }
-  if constexpr (DBG) { asm volatile("" :: "v"(acc0), "v"(acc1)); }
+  for (int t = 0; t < NT; ++t)
+#pragma unroll
+    for (int j = 0; j < MB; ++j) acc[t][j] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+  for (int u = 0; u < U; ++u)
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+#pragma unroll
+      for (int j = 0; j < MB; ++j) acc[t][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u][t], b[u][j], acc[t][j], 0, 0, 0);
+  if constexpr (DBG) { asm volatile("" :: "v"(acc[0][0]), "v"(acc[NT - 1][MB - 1])); }
   DEC_STAMP(2)
-  if (wave > 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) { red[wave - 1][r][lane] = acc0[r]; red[wave - 1][4 + r][lane] = acc1[r]; }
-  }
+  for (int i = 0; i < BLOCKS; ++i) red[wave][i][lane] = acc[i / MB][i % MB];
   __syncthreads();
-  if (wave != 0) return;
+  if (wave >= BLOCKS) return;
   DEC_STAMP(3)
+  f32x4 v = red[0][wave][lane];
+  {
+    const f32x4 s1 = red[1][wave][lane], s2 = red[2][wave][lane], s3 = red[3][wave][lane];
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    acc0[r] += red[0][r][lane] + red[1][r][lane] + red[2][r][lane];
-    acc1[r] += red[0][4 + r][lane] + red[1][4 + r][lane] + red[2][4 + r][lane];
+    for (int r = 0; r < 4; ++r) v[r] += s1[r] + s2[r] + s3[r];
   }
   if constexpr (EPI == DEC_PART) {
-    float* dst = p.part + ((long long)blockIdx.y * 32 + r16) * p.N + nq0;
-    if (r16 < p.M) dec_store(dst, acc0, p.wt);
-    if (16 + r16 < p.M) dec_store(dst + 16ll * p.N, acc1, p.wt);
+    if (mr < rows) dec_store(p.part + ((long long)blockIdx.y * 32 + m) * p.N + nq0, v, p.wt);
   } else if constexpr (EPI == DEC_STORE) {
-    bf16x4 o0, o1;
+    bf16x4 o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      // (+ residual in fp32, one rounding: the value dec_finish_ln_kernel normalises)
-      o0[i] = (bf16)(vy_act_fwd_fast<ACT>(acc0[i] + (float)bias4[i]) + (float)res0[i]);
-      o1[i] = (bf16)(vy_act_fwd_fast<ACT>(acc1[i] + (float)bias4[i]) + (float)res1[i]);
-    }
-    bf16* dst = p.y + (long long)r16 * p.ldy + nq0;
-    if (r16 < p.M) dec_store(dst, o0, p.wt);
-    if (16 + r16 < p.M) dec_store(dst + 16ll * p.ldy, o1, p.wt);
+    for (int i = 0; i < 4; ++i)   // (+ residual in fp32, one rounding: the value dec_finish_ln_kernel normalises)
+      o[i] = (bf16)(vy_act_fwd_fast<ACT>(v[i] + (float)bias4[i]) + (float)res[i]);
+    if (mr < rows) dec_store(p.y + (long long)m * p.ldy + nq0, o, p.wt);
   } else {
     // head and offset inside the head of this lane's quad; section q / k / v is workgroup-uniform
     const int hd = nb >> 2;                       // 64-wide heads: 4 workgroups per head under either column map
     const int dcol = nq0 & 63;
     const int hq = p.nq >> 6, hkv = p.nkv >> 6;
-    float v0[4], v1[4];
+    bf16x4 o;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { v0[i] = acc0[i] + (float)bias4[i]; v1[i] = acc1[i] + (float)bias4[i]; }
+    for (int i = 0; i < 4; ++i) v[i] += (float)bias4[i];
     if (rope_map && hd < hq + hkv) {
       // reference op order (layers/positional_embeddings.py:173-181), every product rounded to bf16; the other
       // half of each rotary pair is in lane ^ 32
@@ -286,22 +325,19 @@ __global__ __launch_bounds__(256) void dec_gemm16_kernel(const DecGemmArgs p, co
 #pragma unroll
       for (int i = 0; i < 4; ++i) {
         const float c = vy_round_bf16(cos4[i]), sn = vy_round_bf16(sin4[i]);
-        const float o0 = dec_swap32(v0[i], hi_half), o1 = dec_swap32(v1[i], hi_half);
-        const float a0 = vy_round_bf16(v0[i]), a1 = vy_round_bf16(v1[i]);
-        const float t0 = vy_round_bf16(vy_round_bf16(o0) * sn), t1 = vy_round_bf16(vy_round_bf16(o1) * sn);
-        v0[i] = hi_half ? vy_round_bf16(a0 * c) + t0 : vy_round_bf16(a0 * c) - t0;
-        v1[i] = hi_half ? vy_round_bf16(a1 * c) + t1 : vy_round_bf16(a1 * c) - t1;
+        const float other = dec_swap32(v[i], hi_half);
+        const float own = vy_round_bf16(v[i]);
+        const float turn = vy_round_bf16(vy_round_bf16(other) * sn);
+        v[i] = hi_half ? vy_round_bf16(own * c) + turn : vy_round_bf16(own * c) - turn;
       }
     }
-    bf16x4 o0, o1;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) { o0[i] = (bf16)v0[i]; o1[i] = (bf16)v1[i]; }
+    for (int i = 0; i < 4; ++i) o[i] = (bf16)v[i];
     bf16* base; long long rs;   // destination of row 0 and the row stride
     if (hd < hq) { base = p.q + hd * 64 + dcol; rs = p.nq; }
     else if (hd < hq + hkv) { base = p.k + (hd - hq) * p.c_sh + (long long)pos * p.c_sl + dcol; rs = p.c_sb; }
     else { base = p.v + (hd - hq - hkv) * p.c_sh + (long long)pos * p.c_sl + dcol; rs = p.c_sb; }
-    if (r16 < p.M) dec_store(base + r16 * rs, o0, p.wt);
-    if (16 + r16 < p.M) dec_store(base + (16 + r16) * rs, o1, p.wt);
+    if (mr < rows) dec_store(base + m * rs, o, p.wt);
   }
   if constexpr (DBG) { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
   DEC_STAMP(4)
@@ -311,34 +347,44 @@ __global__ __launch_bounds__(256) void dec_gemm16_kernel(const DecGemmArgs p, co
 // ------------------------------------------------------------------------------------------
 // Partial tiles of the two N = d projections (out-projection, FFN2) for the split-K finish below: 64 output
 // columns x 32 rows x a SHORT K range (U k-steps of 32) per workgroup, one 16-column block per WAVE, all four
-// waves on the same K range.  The timeline (tools/decode_timeline.py) shows what a launch of dec_gemm16_kernel
-// waits for: its 73 KB per workgroup (49 KB of it the activations, re-read by every workgroup) arrive at the
-// ~30 GB/s one CU takes in -- 2.4 us.  Bytes per workgroup for a (c columns, k range) tile are 2k(32 + c) against
-// k c of work: wide and short is cheapest, and costs nothing here because these projections are split over K
-// anyway.  12 KB of activations (shared by the four waves through L1) + 24 KB of weights per workgroup, no
-// cross-wave reduction, no LDS, no barrier.  part[gridDim.y][32][N] as in dec_gemm16_kernel<DEC_PART>.
+// waves on the same K range.  Bytes per workgroup for a (c columns, k range) tile are 2k(32 + c) against k c of work: wide and
+// short is cheapest, and costs nothing here because these projections are split over K anyway.  12 KB of activations and
+// 24 KB of weights per workgroup (U = 6), no cross-wave reduction.  part[gridDim.y][32][N] as in dec_gemm16_kernel<DEC_PART>.
 // ------------------------------------------------------------------------------------------
 template <int U, bool DBG>
 __global__ __launch_bounds__(256) void dec_gemm64p_kernel(const DecGemmArgs p, const DecDbg dbg) {
+  constexpr int L = U / 2, GROUPS = 4 + 8;   // lines of the K range; groups of 8 rows: of X, of W
+  __shared__ __align__(16) char lines[L * GROUPS * 1024];
   unsigned long long dbg_t[8] = {0, 0, 0, 0, 0, 0, 0, 0};
   DEC_STAMP(0)
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
-  const int col = (int)blockIdx.x * 64 + wave * 16 + r16;
-  const int m0 = r16 < p.M ? r16 : p.M - 1, m1 = 16 + r16 < p.M ? 16 + r16 : p.M - 1;
-  const int kbase = (int)blockIdx.y * U * 32 + kq * 8;
-  const bf16* wp = p.W + (long long)col * p.ldw + kbase;
-  const bf16* xp0 = p.X + (long long)m0 * p.ldx + kbase;
-  const bf16* xp1 = p.X + (long long)m1 * p.ldx + kbase;
+  // a wave loads the lines of its 16 rows of W and of one group of 8 rows of X
+  const int row = lane >> 3, k = (int)blockIdx.y * U * 32;
+  auto at = [&](const bf16* base, int ld, int n, int r) { return base + (long long)n * ld + k + 8 * ((lane & 7) ^ ((r >> 1) & 7)); };
+  const bf16* xp = at(p.X, p.ldx, min(8 * wave + row, p.M - 1), 8 * wave + row);
+  const bf16* wp0 = at(p.W, p.ldw, (int)blockIdx.x * 64 + wave * 16 + row, row);
+  const bf16* wp1 = at(p.W, p.ldw, (int)blockIdx.x * 64 + wave * 16 + 8 + row, 8 + row);
+#pragma unroll
+  for (int l = 0; l < L; ++l) {
+    char* line = lines + l * GROUPS * 1024;
+    dec_line(wp0 + 64 * l, line + (4 + 2 * wave) * 1024);
+    dec_line(wp1 + 64 * l, line + (5 + 2 * wave) * 1024);
+    if (8 * wave < p.M) dec_line(xp + 64 * l, line + wave * 1024);
+  }
+  DEC_STAMP(1)
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  __syncthreads();
   bf16x8 a[U], b0[U], b1[U];
 #pragma unroll
   for (int u = 0; u < U; ++u) {
-    a[u] = *reinterpret_cast<const bf16x8*>(wp + 32 * u);
-    b0[u] = *reinterpret_cast<const bf16x8*>(xp0 + 32 * u);
-    b1[u] = *reinterpret_cast<const bf16x8*>(xp1 + 32 * u);
+    const char* line = lines + (u >> 1) * GROUPS * 1024;
+    const int ch = 4 * (u & 1) + kq;
+    b0[u] = dec_frag(line, r16, ch);
+    b1[u] = dec_frag(line, 16 + r16, ch);
+    a[u] = dec_frag(line, 32 + 16 * wave + r16, ch);
   }
-  DEC_STAMP(1)
   f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int u = 0; u < U; ++u) {
@@ -457,34 +503,41 @@ int dec_wt() {
   return v;
 }
 
-template <int EPI, int ACT>
-int dec_gemm_go(DecGemmArgs a, int K, int chunks, hipStream_t st) {
-  a.wt = dec_wt();
-  const int u4 = K / chunks / 128;   // k-steps per wave
-  const dim3 grid((unsigned)(a.N / 16), (unsigned)chunks), block(256);
-  if constexpr (EPI == DEC_STORE) {
-    if (a.ln_g) {   // LayerNorm prologue: the workgroup must hold whole rows (one K chunk)
-      if (chunks != 1) return 1;
-      if (u4 == 6) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 6, false, true>), grid, block, 0, st, a, g_dbg);
-      else if (u4 == 8) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 8, false, true>), grid, block, 0, st, a, g_dbg);
-      else if (u4 == 4) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 4, false, true>), grid, block, 0, st, a, g_dbg);
-      else return 1;
-      return 0;
-    }
-  }
-  if (g_dbg.buf && g_dbg.slot < g_dbg_launches) {
-    if (u4 == 6) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 6, true>), grid, block, 0, st, a, g_dbg);
-    else if (u4 == 8) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 8, true>), grid, block, 0, st, a, g_dbg);
-    else if (u4 == 4) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 4, true>), grid, block, 0, st, a, g_dbg);
+template <int EPI, int ACT, bool LNP, int MB, int NT>
+int dec_gemm_tile(const DecGemmArgs& a, int u4, int chunks, hipStream_t st) {   // u4: k-steps per wave
+  const dim3 grid((unsigned)(a.N / (16 * NT)), (unsigned)chunks, (unsigned)vy_cdiv(a.M, 16 * MB)), block(256);
+  if (!LNP && g_dbg.buf && g_dbg.slot < g_dbg_launches) {
+    if (u4 == 6) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 6, !LNP, LNP, MB, NT>), grid, block, 0, st, a, g_dbg);
+    else if (u4 == 8) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 8, !LNP, LNP, MB, NT>), grid, block, 0, st, a, g_dbg);
+    else if (u4 == 4) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 4, !LNP, LNP, MB, NT>), grid, block, 0, st, a, g_dbg);
     else return 1;
     ++g_dbg.slot;
     return 0;
   }
-  if (u4 == 6) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 6, false>), grid, block, 0, st, a, g_dbg);
-  else if (u4 == 8) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 8, false>), grid, block, 0, st, a, g_dbg);
-  else if (u4 == 4) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 4, false>), grid, block, 0, st, a, g_dbg);
+  if (u4 == 6) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 6, false, LNP, MB, NT>), grid, block, 0, st, a, g_dbg);
+  else if (u4 == 8) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 8, false, LNP, MB, NT>), grid, block, 0, st, a, g_dbg);
+  else if (u4 == 4) hipLaunchKernelGGL((dec_gemm16_kernel<EPI, ACT, 4, false, LNP, MB, NT>), grid, block, 0, st, a, g_dbg);
   else return 1;
   return 0;
+}
+
+// Rows in blocks of 16, two of them to a workgroup where blocks by themselves are more workgroups than CUs: two on a CU take in 98 KB in
+// turn (K = 768), one with both 73.  768 x 768, 32 rows: 48 workgroups 4.2 us, 96 of one block 3.9 to 4.0.
+template <int EPI, int ACT>
+int dec_gemm_go(DecGemmArgs a, int K, int chunks, hipStream_t st) {
+  a.wt = dec_wt();
+  const int u4 = K / chunks / 128;
+  const bool one = a.M <= 16 || a.N / 16 * chunks * 2 <= 256;
+  if constexpr (EPI == DEC_STORE) {
+    if (a.ln_g) {   // LayerNorm prologue: the workgroup must hold whole rows (one K chunk)
+      if (chunks != 1) return 1;
+      if (one) return dec_gemm_tile<EPI, ACT, true, 1, 1>(a, u4, chunks, st);
+      if (a.N % 32 == 0) return dec_gemm_tile<EPI, ACT, true, 1, 2>(a, u4, chunks, st);
+      return dec_gemm_tile<EPI, ACT, true, 2, 1>(a, u4, chunks, st);
+    }
+  }
+  if (one) return dec_gemm_tile<EPI, ACT, false, 1, 1>(a, u4, chunks, st);
+  return dec_gemm_tile<EPI, ACT, false, 2, 1>(a, u4, chunks, st);
 }
 
 // partial tiles with 64-column workgroups: k-steps per workgroup U in {6, 8, 4}; returns the number of K chunks or 0
