@@ -148,22 +148,33 @@ __global__ __launch_bounds__(256) void latent_scan_kernel(LatentArgs p) {
     }
   };
   const int kblk = KH == 2 ? wave & 1 : wave, khalf = KH == 2 ? wave >> 1 : 0;
-  bf16x8 qh[KS], ql[KS];
-  const int64_t qo = ((int64_t)b * p.h + (head < p.h ? head : 0)) * p.R;
-  const bf16x8 zero8 = {};
+  // The latent queries come by whole lines into the ring's last buffer, free until the loop's first tile has been waited for, once for
+  // all four waves: as fragments from memory, 16 rows and 16 bytes a lane and every wave all of them, they were the longest part of a
+  // slice of one tile (one sequence, 16 heads, latents of 256: 5.7 -> 5.3 us)
+  constexpr int QP = 2 * 16 * RB / 1024 / 4;  // pieces per wave: the rows of 16 heads, hi and then lo
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) {
-    const int k = 32 * (khalf * KS + ks) + 8 * kq;
-    const bool ok = k < p.R && head < p.h;
-    qh[ks] = ok ? *reinterpret_cast<const bf16x8*>(p.qhi + qo + k) : zero8;
-    ql[ks] = ok ? *reinterpret_cast<const bf16x8*>(p.qlo + qo + k) : zero8;
+  for (int i = 0; i < QP; ++i) {
+    const int P = (wave * QP + i) * 1024 + lane * 16, row = P / RB;
+    const int k = 8 * (((P % RB) >> 4) ^ (row & SWZ));
+    const bf16* q = (row < 16 ? p.qhi : p.qlo) + ((int64_t)b * p.h + min((int)blockIdx.y * 16 + (row & 15), p.h - 1)) * p.R + k;
+    __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(k < p.R ? q : reinterpret_cast<const bf16*>(vy_zero16)),
+                                     (VY_LDS void*)(smem + (NS - 1) * TILE + (wave * QP + i) * 1024), 16, 0, 0);
   }
-  // The ring is filled behind the query loads (without conditions, so that their wait can be counted: rows past the end are
-  // clamped), and the queries are retired before the loop: a wait for them inside it would drain the ring.
 #pragma unroll
   for (int t = 0; t < NS - 1; ++t) stage(t);
+  asm volatile("s_waitcnt vmcnt(%0)" ::"n"((NS - 1) * NP) : "memory");
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+  bf16x8 qh[KS], ql[KS];
 #pragma unroll
-  for (int ks = 0; ks < KS; ++ks) { asm volatile("" ::"v"(qh[ks])); asm volatile("" ::"v"(ql[ks])); }
+  for (int ks = 0; ks < KS; ++ks) {
+    const unsigned at = vy_lds_addr(smem) + (NS - 1) * TILE + r16 * RB + (((4 * (khalf * KS + ks) + kq) ^ (r16 & SWZ)) << 4);
+    qh[ks] = lds_read16(at);
+    ql[ks] = lds_read16(at + 16 * RB);
+  }
+  asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) { vy_tie(qh[ks]); vy_tie(ql[ks]); }
 
   const unsigned base = vy_lds_addr(smem), sbase = base + NS * TILE;
   const int krow = 16 * kblk + r16;
@@ -293,38 +304,38 @@ __device__ __forceinline__ void slice_weights(const LatentArgs& p, int b, int he
   if (lane < p.nsplit) w[lane] = e / L;
 }
 
-// out[b][h][n] = (W_uv,h u_bh)_n * sigmoid(gate): workgroup = 64 value columns of one head x p.seqs (<= 16) sequences; the
+// out[b][h][n] = (W_uv,h u_bh)_n * sigmoid(gate): workgroup = 16 NB value columns of one head x p.seqs (<= 16) sequences; the
 // mean latents are added up from the slices into LDS first (few sequences: the slices are shared out over the threads)
 // (RP: padded latent width.  The weights of the product are requested before anything else: one memory latency beside the
-// slices', not one after another behind them.)
-template <int RP>
+// slices', not one after another behind them -- by whole 128-byte lines into LDS: as fragments, 16 rows and 16 bytes a lane, a CU takes
+// in half as much.)
+template <int RP, int NB> constexpr int VALUE_LINES = RP / 64 * 2 * NB * 1024;
+template <int RP, int NB>
 __global__ __launch_bounds__(256) void latent_value_kernel(LatentArgs p) {
   extern __shared__ __attribute__((aligned(16))) char dyn[];
-  constexpr int PITCH = (RP + 8) * 2, KS = RP / 32;
-  float* sw = reinterpret_cast<float*>(dyn);                       // [seqs][MAX_SPLIT]
-  f32x4* acc4 = reinterpret_cast<f32x4*>(dyn + p.seqs * MAX_SPLIT * 4);   // [256]
-  char* xh = dyn + p.seqs * MAX_SPLIT * 4 + 4096;
+  constexpr int PITCH = (RP + 8) * 2, KS = RP / 32, LINES = VALUE_LINES<RP, NB>;
+  float* sw = reinterpret_cast<float*>(dyn + LINES);               // [seqs][MAX_SPLIT]
+  f32x4* acc4 = reinterpret_cast<f32x4*>(dyn + LINES + p.seqs * MAX_SPLIT * 4);   // [256]
+  char* xh = dyn + LINES + p.seqs * MAX_SPLIT * 4 + 4096;
   char* xl = xh + p.seqs * PITCH;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
   const int head = blockIdx.y, b0 = (int)blockIdx.z * p.seqs;
   const int nb = min(p.seqs, p.B - b0);
   const bf16x8 zero8 = {};
-  const int n0 = (int)blockIdx.x * 64 + wave * 16;
-  const bool wok = n0 + r16 < p.dv;
-  bf16x8 wf[KS];
-  {
-    const bf16* w = (const bf16*)p.wuv + ((int64_t)head * p.dv + (wok ? n0 + r16 : 0)) * p.R;
+  const int first = (int)blockIdx.x * 16 * NB, n0 = first + wave * 16;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) {
-      const int k = 32 * ks + 8 * kq;
-      wf[ks] = wok && k < p.R ? *reinterpret_cast<const bf16x8*>(w + k) : zero8;
-    }
+  for (int i = 0; i < (LINES / 1024 + 3) / 4; ++i) {   // 8 rows of a line each; 16-byte chunk c of row r at c ^ (r / 2 & 7)
+    const int piece = wave + 4 * i, row = 8 * (piece % (2 * NB)) + (lane >> 3);
+    const int k = piece / (2 * NB) * 64 + 8 * ((lane & 7) ^ ((row >> 1) & 7));
+    const bf16* w = (const bf16*)p.wuv + ((int64_t)head * p.dv + min(first + row, p.dv - 1)) * p.R + k;
+    if (piece < LINES / 1024)   // (wave-uniform)
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(k < p.R ? w : reinterpret_cast<const bf16*>(vy_zero16)), (VY_LDS void*)(dyn + piece * 1024), 16, 0, 0);
   }
   // the gates and the first slices' sums do not wait for the weights of the slices (8 sequences, 16 heads, latents of 256 of 720 keys,
   // all three kernels: 14.55 -> 14.2 us)
   const int nn = n0 + 4 * kq;
-  const bool out_ok = r16 < nb && nn < p.dv;
+  const bool out_ok = wave < NB && r16 < nb && nn < p.dv;
   bf16x4 g4 = {};
   if (out_ok && p.gate) {
     const bf16* gr = (const bf16*)p.gate + (int64_t)(b0 + r16) * p.ldg;
@@ -385,8 +396,9 @@ __global__ __launch_bounds__(256) void latent_value_kernel(LatentArgs p) {
       *reinterpret_cast<bf16x4*>(xl + i * PITCH + col * 2) = lo;
     }
   }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");   // (the lines)
   __syncthreads();
-  if (n0 >= p.dv) return;
+  if (wave >= NB || n0 >= p.dv) return;
   f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acl = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
   for (int ks = 0; ks < KS; ++ks) {
@@ -394,8 +406,9 @@ __global__ __launch_bounds__(256) void latent_value_kernel(LatentArgs p) {
     const bool ok = r16 < nb;
     const bf16x8 a = ok ? *reinterpret_cast<const bf16x8*>(xl + r16 * PITCH + k * 2) : zero8;
     const bf16x8 c = ok ? *reinterpret_cast<const bf16x8*>(xh + r16 * PITCH + k * 2) : zero8;
-    acl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks], a, acl, 0, 0, 0);
-    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks], c, acc, 0, 0, 0);
+    const bf16x8 w = *reinterpret_cast<const bf16x8*>(dyn + (ks >> 1) * 2 * NB * 1024 + (16 * wave + r16) * 128 + (((4 * (ks & 1) + kq) ^ ((r16 >> 1) & 7)) << 4));
+    acl = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, acl, 0, 0, 0);
+    acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, c, acc, 0, 0, 0);
   }
   acc += acl;
   if (out_ok) {
@@ -580,15 +593,21 @@ extern "C" int vy_latent_decode(const void* q, int64_t ldq, const void* wukt, co
     else if (R <= 128) hipLaunchKernelGGL(latent_scan_kernel<128>, grid, block, 0, st, p);
     else if (R <= 256) hipLaunchKernelGGL(latent_scan_kernel<256>, grid, block, 0, st, p);
     else hipLaunchKernelGGL(latent_scan_kernel<512>, grid, block, 0, st, p);
-    const int nv = (int)vy_cdiv(dv, 64);
+    // 64 value columns a workgroup; 16 where those are 64 workgroups at most, so that these are no more than the CUs (one sequence, 8 heads of 128,
+    // latents of 256: 16 workgroups 5.6 us, 64 of 16 columns 4.7)
+    const bool narrow = B * h * vy_cdiv(dv, 64) <= 64;
+    const int nv = (int)vy_cdiv(dv, narrow ? 16 : 64);
     const int64_t per = vy_cdiv((int64_t)B * h * nv, 256);         // sequences per workgroup: fill the CUs first
     p.seqs = (int)(per > 16 ? 16 : per);
     const dim3 vgrid(nv, h, (unsigned)vy_cdiv(B, p.seqs));
-    auto lds = [&](int RP) { return p.seqs * MAX_SPLIT * 4 + 4096 + 2 * p.seqs * (RP + 8) * 2; };
-    if (R <= 64) hipLaunchKernelGGL(latent_value_kernel<64>, vgrid, block, lds(64), st, p);
-    else if (R <= 128) hipLaunchKernelGGL(latent_value_kernel<128>, vgrid, block, lds(128), st, p);
-    else if (R <= 256) hipLaunchKernelGGL(latent_value_kernel<256>, vgrid, block, lds(256), st, p);
-    else hipLaunchKernelGGL(latent_value_kernel<512>, vgrid, block, lds(512), st, p);
+#define VALUE_NB(RP, NB) hipLaunchKernelGGL((latent_value_kernel<RP, NB>), vgrid, block, (VALUE_LINES<RP, NB> + p.seqs * MAX_SPLIT * 4 + 4096 + 2 * p.seqs * (RP + 8) * 2), st, p)
+#define VALUE(RP) do { if (narrow) VALUE_NB(RP, 1); else VALUE_NB(RP, 4); } while (0)
+    if (R <= 64) VALUE(64);
+    else if (R <= 128) VALUE(128);
+    else if (R <= 256) VALUE(256);
+    else VALUE(512);
+#undef VALUE
+#undef VALUE_NB
   }
   VY_CHECK_LAUNCH(who);
   return VY_OK;
