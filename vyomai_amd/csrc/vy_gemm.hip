@@ -332,7 +332,7 @@ __device__ __forceinline__ int w_row(int n0, int R, int N) {
 // division), 8192 x 2 x 8192, K = 2048: 508 -> 501 us, 8192 x 2 x 4096, K = 1024: 135 -> 132.
 constexpr unsigned ACT_TAB_LOW = (127 - 20) << 7, ACT_TAB_HALF = 24 << 7;   // first magnitude's bits, entries per sign
 constexpr bool act_has_table(int BM, int BN, int EPI, int ACT, bool GRAD) {
-  return BM == 256 && BN != 192 && !GRAD && (EPI == 0 ? ACT == VY_ACT_GELU_ERF || ACT == VY_ACT_GELU_TANH : EPI == 2);
+  return (BN == 256 || (BM == 256 && BN == 128)) && !GRAD && (EPI == 0 ? ACT == VY_ACT_GELU_ERF || ACT == VY_ACT_GELU_TANH : EPI == 2);
 }
 constexpr int act_table_bytes(int BM, int BN, int EPI, int ACT, bool GRAD) {
   return act_has_table(BM, BN, EPI, ACT, GRAD) ? 2 * ACT_TAB_HALF * 4 : 0;
@@ -395,7 +395,7 @@ template <int BM, int BN, int WGM, int WGN, bool MF16> struct AccTile {
 // chunks, every iteration waits a full memory latency for it (22 k cycles per tile against 12 k without the operand; residual behind an
 // activation, squared ReLU, 30500 x 768: K = 768 51.4 -> 46.5 us, K = 3072 147 -> 138).
 constexpr bool epi_prefetches(int BM, int BN, int NW, int EPI, bool GRAD) {
-  return EPI == 0 && (BM * BN == 256 * 192 || BN == 64 || (BM * BN == 256 * 256 && GRAD)) && (BM * BN / 8) % (64 * NW) == 0;
+  return EPI == 0 && (BN == 192 || BN == 64 || (BN == 256 && (GRAD || BM < 256))) && (BM * BN / 8) % (64 * NW) == 0;
 }
 template <int BM, int BN, int NW, int EPI, bool GRAD>
 struct EpiAhead {
@@ -1160,6 +1160,10 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
 // BM x BN x 64 tiles, two whole stages, on mfma_f32_16x16x32_bf16.  256 x 256 (8 waves, 128 KiB): the wide launches (FFN1,
 // the dgrad of FFN2, the vocabulary projection), where the tile's fewer operand bytes per FLOP matter more than a third X
 // stage; 4 x 8 blocks of 16 x 16 per wave (128 accumulator registers), 32 MFMAs per k-step, fragments double-buffered.
+// 224 and 160 x 256 (2 x 4 waves): where these heights fill the last round of the CUs better, which is what ragged rows lose to.  Under
+// load, 12608 x 3072, K = 768: 600 tiles 76.4 us, 684 of 224 rows 71.2; 6000 x 3072, K = 768: 288 tiles 47.1, 456 of 160 rows 37.0 (operands from
+// beyond the Infinity Cache: 77.4 and 75.8, 49.8 and 42.7).  A third stage of X for them: 3 to 6 % slower, or where X comes from far 3 to 7 % faster
+// and then as fast as 256 x 192; 192 rows 0.2 % on average beside these, 192 x 192 0.5 %, 224, 288 and 320 x 192 0.1 %.
 // 128 x 128 (4 waves, 64 KiB, two workgroups per CU): mid-size M.
 // ------------------------------------------------------------------------------------------
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD>
@@ -1167,10 +1171,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
     int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob) {
   constexpr int NW = WGM * WGN;
-  constexpr int TM = BM / (16 * WGM), TN = BN / (16 * WGN);   // 256 x 256, 4 x 2 waves: 4, 8;  128 x 128, 2 x 2 waves: 4, 4
+  constexpr int TM = BM / (16 * WGM), TN = BN / (16 * WGN);   // 256 x 256, 4 x 2 waves: 4, 8;  224 x 256, 2 x 4 waves: 7, 4;  128 x 128, 2 x 2 waves: 4, 4
   constexpr int PX = BM / 8, PW = BN / 8;
-  constexpr int GX = PX / NW, GW = PW / NW;
-  static_assert(GX * NW == PX && GW * NW == PW, "pieces must divide over the waves");
+  constexpr int GX = (PX + NW - 1) / NW, GW = PW / NW, REST = PX % NW;   // (of X, the last piece of a wave may be missing)
+  static_assert(TM * 16 * WGM == BM && TN * 16 * WGN == BN && GW * NW == PW, "whole blocks, and pieces of W divide over the waves");
   constexpr int STAGE = (BM + BN) * ROWB;
   constexpr int LDS_BYTES = vy_cmax(2 * STAGE, epi_lds_bytes(BM, BN, EPI, 1)), TABLE = act_table_bytes(BM, BN, EPI, ACT, GRAD);
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES + TABLE];
@@ -1212,7 +1216,8 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     for (int t = 0; t < GX; ++t) {
       const bf16* s = xsrc[t] + k0;
       if (ktail && k0 + xk[t] >= K) s = zero;
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
+      if (REST == 0 || t + 1 < GX || wave < REST)
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
     }
 #pragma unroll
     for (int t = 0; t < GW; ++t) {
@@ -1685,9 +1690,9 @@ inline Scratch splitk_ws(hipStream_t st) {
 // Tiles of a product of more than 32 rows.  What a shape costs depends on how its tiles fill the 256 CUs as much as on the tile's
 // own rate: 8192 x 2048 with K = 12288 is 352 tiles of 256 x 192 -- two rounds, the second a third full, 459 us -- or 256 tiles of
 // 256 x 256: 313 us; 8000 x 1024, K = 6144: 124 us on 256 x 192, 152 us on 256 x 256, 100 us on 256 x 128 (250 tiles).  So the
-// launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below; the constants
-// are fits to launches of 40 shapes from 48 to 30500 rows on one box (mostly within 10 %; a GELU epilogue's extra time grows with the
-// output alone and so moves no choice), where K is sliced (up to 4096 rows) to 1600 of 33 to 4096 rows, 64 to 40000 columns and K = 256 to
+// launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below (a GELU epilogue's
+// extra time grows with the output alone and so moves no choice); the constants are fits: whole_cost, and where K is sliced (up to 4096
+// rows) 1600 shapes of 33 to 4096 rows, 64 to 40000 columns and K = 256 to
 // 16384, each on all kernels that take it, in graphs that walk through 200 MB of weights, as a model's layers do: products that find
 // their weights in L2, as a loop over one product does, made one launch look shorter than two groups in it.  The kernel chosen takes
 // 0.2 % longer than the fastest on average, over 8 % for 12 of them.  (Fitted to 90 shapes, 8 % for 45 of 1100: 300 x 2048, K = 6144, 31.5 us in two
@@ -1699,6 +1704,17 @@ constexpr int TILE_N[] = {256, 192, 128, 128, 64, 64, 64, 128, 128};
 constexpr int TILE_THREADS[] = {512, 512, 512, 256, 256, 512, 512, 256, 512};
 struct Tiling { TileKind kind; int slices, rows; };   // (rows of a tile)
 
+// a shape on tiles of rows x cols, all of K in one workgroup, `places` of them at a time: `fixed` per round, `stage` per 64 columns of K (`apart` more
+// of it where rows start inside a 128-byte line: a stage touches more of them), less of it for a last round that leaves CUs idle.  Fits to
+// 440 shapes of 1100 to 33000 rows, each on every kernel, launched back to back for 25 ms on operands that stay in the Infinity Cache and on ones
+// that do not (the root of the product of both; 224 rows 1 %, 160 rows 4 and 128 x 128 1.5 % on top, which lose most where X comes from far).
+// One launch at a time on a cool chip, 160 rows looked 7 % better than they are beside 256 x 192: the chip's power and its memory decide between them.
+// Against the choice before, 1.8 % on average where operands are near and 1.1 % where they are not.
+inline double whole_cost(int64_t M, int64_t N, int64_t K, int places, int rows, int cols, double launch, double fixed, double stage, double idle, double apart) {
+  const double r = (double)(vy_cdiv(M, rows) * vy_cdiv(N, cols)) / places, whole = (double)(int64_t)r, part = r - whole;
+  const int KT = (int)vy_cdiv(K, BK);
+  return launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? idle + (1 - idle) * part : 0.0)) * stage * KT * (K % BK ? 1 + apart : 1.0);
+}
 // what a shape costs on a tile, S slices of K added up
 template <TileKind kind>
 inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
@@ -1706,16 +1722,11 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
   const int KT = (int)vy_cdiv(K, BK);
   const double load = (double)tiles / chip;
   const bool apart = K % BK != 0;   // (rows that start inside a 128-byte line: a stage touches more of them)
-  // `fixed` per round, `stage` per stage of a round; the stages of a last round that leaves CUs idle run up to 30 % faster
-  auto one_shot = [&](int per_cu, double launch, double fixed, double stage) {
-    const double r = load / per_cu, whole = (double)(int64_t)r, part = r - whole;
-    return launch + (whole + (part > 0)) * fixed + (whole + (part > 0 ? 0.7 + 0.3 * part : 0.0)) * stage * KT;
-  };
   switch (kind) {
-    case T_256x256: return one_shot(1, 2.5, 7.0, 1.55);
-    case T_256x192: return one_shot(1, 2.3, 5.5, 1.30);
-    case T_256x128: return one_shot(1, 4.5, 4.1, 0.97);
-    case T_128x128: return load <= 1 ? 8.5 + 0.72 * KT : one_shot(2, 3.5, 5.0, 1.0);     // (two of them share a CU)
+    case T_256x256: return whole_cost(M, N, K, chip, 256, 256, 1.71, 7.15, 1.633, 0.714, 0.2);
+    case T_256x192: return whole_cost(M, N, K, chip, 256, 192, 2.57, 5.53, 1.278, 0.755, 0.18);
+    case T_256x128: return whole_cost(M, N, K, chip, 256, 128, 2.86, 3.91, 0.993, 0.644, 0.2);
+    case T_128x128: return load <= 1 ? 2.76 + 0.84 * KT * (apart ? 1.3 : 1.0) : whole_cost(M, N, K, 2 * chip, 128, 128, 2.46, 3.65, 1.115, 0.417, 0.23);   // (two of them share a CU)
     case T_64x64: {
       if (S == 1) return 3.2 + (load > 1 ? 0.8 : 0.0) + KT * (0.25 * load > 0.335 ? 0.25 * load : 0.335);
       const double n = (double)vy_cdiv(tiles, (int64_t)chip), stage = 0.238 * n - 0.204;   // the fullest CU holds n (up to three at once)
@@ -1784,6 +1795,8 @@ inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_
   offer(T_64x64, tile_cost<T_64x64>(M, N, K, S, chip));
   if (S == 1) {
     offer(T_256x256, tile_cost<T_256x256>(M, N, K, S, chip));
+    offer(T_256x256, whole_cost(M, N, K, chip, 224, 256, 2.07, 6.19, 1.524, 0.726, 0.22), 224);
+    offer(T_256x256, whole_cost(M, N, K, chip, 160, 256, 1.92, 4.73, 1.326, 0.683, 0.25), 160);
     offer(T_256x192, tile_cost<T_256x192>(M, N, K, S, chip));
     offer(T_256x128, tile_cost<T_256x128>(M, N, K, S, chip));
     offer(T_128x128, tile_cost<T_128x128>(M, N, K, S, chip));
@@ -2575,7 +2588,11 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
         else VY_TILES(gemm_nt_bf16_kernel<256, 192, 4, 2, EPI, ACT, GRAD>);
       }
     } else switch (t.kind) {
-      case T_256x256: VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>); break;
+      case T_256x256:
+        if (t.rows == 224) VY_TILES(gemm_nt_bf16_m16_kernel<224, 256, 2, 4, EPI, ACT, GRAD>);
+        else if (t.rows == 160) VY_TILES(gemm_nt_bf16_m16_kernel<160, 256, 2, 4, EPI, ACT, GRAD>);
+        else VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>);
+        break;
       case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>); break;
       case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, EPI, ACT, GRAD>); break;
       case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
@@ -2612,7 +2629,11 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
 #define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
 #define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0, per)
   switch (t.kind) {
-    case T_256x256: VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, 2, ACT, false>); break;
+    case T_256x256:
+      if (t.rows == 224) VY_TILES(gemm_nt_bf16_m16_kernel<224, 256, 2, 4, 2, ACT, false>);
+      else if (t.rows == 160) VY_TILES(gemm_nt_bf16_m16_kernel<160, 256, 2, 4, 2, ACT, false>);
+      else VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, 2, ACT, false>);
+      break;
     case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, 2, ACT, false>); break;
     case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, 2, ACT, false>); break;
     case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, 2, ACT, false>); break;
