@@ -22,34 +22,37 @@ using namespace vy_moe_dev;
 constexpr int COUNT_STRIDE = 32;   // the experts' counters, one per 128-byte line: adds to one line queue up
 
 // ---- router -----------------------------------------------------------------------------------
-// logits[m][e] = sum_k h[m][k] w[e][k], fp32 accumulation and result.  One workgroup: 16 ET experts x 16 MT tokens.
-template <int ET, int MT, int NW>
+// logits[m][e] = sum_k h[m][k] w[e][k], fp32 accumulation and result.  One workgroup: 16 ET experts x 16 MT tokens, whose lines go through
+// LDS (share_lds: a CU takes in twice as much of whole lines as of fragments, 16 rows and 16 bytes a lane).  8193 x 64, K = 2048: 26.9 -> 14.2 us.
+template <int ET, int MT, int NW, int D>
 __global__ __launch_bounds__(64 * NW) void router_logits_kernel(const bf16* __restrict__ h, int64_t ldh, const bf16* __restrict__ w,
                                                             float* __restrict__ logits, int64_t M, int K, int E) {
-  __shared__ f32x4 red[vy_rows::RED<ET, MT, NW>];
+  constexpr int BLOCKS = ET * MT;
+  __shared__ __attribute__((aligned(16))) char lds[vy_rows::vy_max2(D * NW * vy_rows::LINE<MT, 16 * ET>, vy_rows::DENSE_RED<ET, MT, NW> * 16)];
+  f32x4* red = reinterpret_cast<f32x4*>(lds);
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int e0 = blockIdx.x * 16 * ET;
   const int64_t m0 = (int64_t)blockIdx.y * 16 * MT;
-  const bf16* ws[ET];
-  const bf16* hs[MT];
-#pragma unroll
-  for (int i = 0; i < ET; ++i) ws[i] = w + (int64_t)min(e0 + 16 * i + r16, E - 1) * K + 8 * kq;
-#pragma unroll
-  for (int j = 0; j < MT; ++j) hs[j] = h + (m0 + 16 * j + r16 < M ? m0 + 16 * j + r16 : M - 1) * ldh + 8 * kq;
+  const int rows = (int)(M - m0 < 16 * MT ? M - m0 : 16 * MT);
   f32x4 acc[ET][MT];
-  vy_rows::stream<ET, MT, false, NW>(ws, hs, K, acc, red);
-  if (threadIdx.x >= 64) return;
+  vy_rows::share_lds<ET, MT, NW, D, 16 * ET>(h + m0 * ldh, ldh, rows, w, K, e0, E, K, lds, acc);
+  __syncthreads();   // (red lies over the other waves' rings)
 #pragma unroll
-  for (int i = 0; i < ET; ++i)
+  for (int i = 0; i < BLOCKS; ++i) red[(wave * BLOCKS + i) * 64 + lane] = acc[i / MT][i % MT];
+  __syncthreads();
 #pragma unroll
-    for (int j = 0; j < MT; ++j) {
-      const int64_t m = m0 + 16 * j + r16;
-      const int e = e0 + 16 * i + 4 * kq;   // a lane: token r16, experts 4 kq .. + 3
-      if (m < M)
+  for (int i = 0; i < BLOCKS; ++i) {
+    if (i % NW != wave) continue;
+    const int m = 16 * (i % MT) + r16, e = e0 + 16 * (i / MT) + 4 * kq;   // a lane: token r16, experts 4 kq .. + 3
+    f32x4 v = red[i * 64 + lane];
 #pragma unroll
-        for (int r = 0; r < 4; ++r)
-          if (e + r < E) logits[m * E + e + r] = acc[i][j][r];
-    }
+    for (int s = 1; s < NW; ++s) v += red[(s * BLOCKS + i) * 64 + lane];
+    if (m < rows)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (e + r < E) logits[(m0 + m) * E + e + r] = v[r];
+  }
 }
 
 __global__ __launch_bounds__(256) void router_logits_f32_kernel(const float* __restrict__ h, int64_t ldh, const float* __restrict__ w,
@@ -533,12 +536,16 @@ extern "C" int vy_moe_fwd(const vy_moe* d, const void* h, int64_t ldh, int64_t M
   if (dtype == VY_F32) {
     hipLaunchKernelGGL(router_logits_f32_kernel, dim3((unsigned)M, (unsigned)vy_cdiv(E, 4)), dim3(256), 0, st, (const float*)h, ldh,
                        (const float*)d->w_router, p.logits, K, E);
-  } else if (M <= 256) {
-    hipLaunchKernelGGL((router_logits_kernel<1, 1, 4>), dim3((unsigned)vy_cdiv(E, 16), (unsigned)vy_cdiv(M, 16)), dim3(256), 0, st,
-                       (const bf16*)h, ldh, (const bf16*)d->w_router, p.logits, M, K, E);
   } else {
-    hipLaunchKernelGGL((router_logits_kernel<4, 2, 8>), dim3((unsigned)vy_cdiv(E, 64), (unsigned)vy_cdiv(M, 32)), dim3(512), 0, st,
-                       (const bf16*)h, ldh, (const bf16*)d->w_router, p.logits, M, K, E);
+    // many tokens: 32, 48 or 64 a workgroup, one workgroup on a CU, by what the rounds of the 256 CUs take in
+    const int64_t cols = vy_cdiv(E, 64);
+    auto taken = [&](int rows) { return vy_cdiv(vy_cdiv(M, rows) * cols, 256) * (rows + 64); };
+#define LOGITS(ET, MT, NW, D) hipLaunchKernelGGL((router_logits_kernel<ET, MT, NW, D>), dim3((unsigned)vy_cdiv(E, 16 * ET), (unsigned)vy_cdiv(M, 16 * MT)), dim3(64 * NW), 0, st, (const bf16*)h, ldh, (const bf16*)d->w_router, p.logits, M, K, E)
+    if (M <= 256) LOGITS(1, 1, 4, 4);
+    else if (taken(32) <= taken(48) && taken(32) <= taken(64)) LOGITS(4, 2, 8, 1);
+    else if (taken(48) <= taken(64)) LOGITS(4, 3, 8, 1);
+    else LOGITS(4, 4, 8, 1);
+#undef LOGITS
   }
   ChooseArgs c{p.logits, M, E, d->top, d->groups, d->keep, d->score == VY_SCORE_SIGMOID, d->group_best, d->normalize, d->scale, count, (int)L, ids, weight, small ? pos : nullptr, small ? nullptr : p.counts, p.rank};
   // few tokens: a wave each, spread over the CUs; many: several per workgroup, so that few global adds count them
@@ -549,7 +556,7 @@ extern "C" int vy_moe_fwd(const vy_moe* d, const void* h, int64_t ldh, int64_t M
     else if (E <= 128) CHOOSE(2, 4, 1);
     else if (E <= 256) CHOOSE(4, 4, 1);
     else CHOOSE(16, 4, 2);
-  } else if (E <= 64) CHOOSE(1, 16, 2);
+  } else if (E <= 64) CHOOSE(1, 8, 2);   // (8193 tokens: 18.4 us; 16 waves 22.5, one token a wave 19.6 and 24.8, four 25.2 and 28.5)
   else if (E <= 128) CHOOSE(2, 16, 2);
   else CHOOSE(4, 16, 2);
 #undef CHOOSE
