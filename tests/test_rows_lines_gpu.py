@@ -21,3 +21,18 @@ def test_stored(M, K, N):
     assert torch.isnan(y[:, N:]).all()
     want, e = sums(x, w)
     within(y[:, :N], want + bias.double(), e + 2.0 ** -23 * want.abs())
+
+
+@pytest.mark.parametrize("M", [5, 32])
+@pytest.mark.parametrize("N", [40, 4100, 12300])
+def test_biases_that_start_anywhere(N, M):
+    x, w, bias = rnd(M, 512, seed=N), rnd(N, 512, seed=12, scale=512 ** -0.5), rnd(N + 3, seed=13, scale=0.5)
+    go = entry("_Z14vy_rows_linearPKvS0_S0_ifPvllllP12ihipStream_t", p, p, p, i32, f32, p, i64, i64, i64, i64, p)
+    ldy = (N + 7) // 8 * 8
+    y = torch.empty(4, M, ldy, dtype=BF, device=DEV)
+    for at in range(4):
+        same = torch.cat([bias[:0], bias[at:at + N]])          # (the same numbers at an aligned place)
+        assert go(ptr(x), ptr(w), bias.data_ptr() + 2 * at, 0, 0.0, ptr(y[0]), ldy, M, N, 512, stream()) == 0
+        assert go(ptr(x), ptr(w), ptr(same), 0, 0.0, ptr(y[1]), ldy, M, N, 512, stream()) == 0
+        torch.cuda.synchronize()
+        assert torch.equal(y[0, :, :N], y[1, :, :N]), at

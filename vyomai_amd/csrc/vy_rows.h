@@ -1,7 +1,7 @@
 // Weight-streaming products of few rows (decode): a workgroup of NW = 4 (or 8) waves takes 16 NT rows of W [N][K] against 16 MB rows of X
 // on mfma_f32_16x16x32_bf16 (A = weight rows, B = rows of X).  The waves split K by whole 128-byte lines (two k-steps of 32).  Two ways for
 // the operands: through LDS, line by line (share_lds), or straight from memory into operand registers (share) -- every wave requests
-// its loads of up to STEPS k-steps before the first product, W past the caches (non-temporal) unless other workgroups read it too.  A
+// its loads of up to STEPS k-steps before the first product, W past the caches (non-temporal).  A
 // load into registers is 16 rows with 16 bytes a lane, no two neighbouring lanes on a line, and a CU takes in 25 to 30 KB of them a
 // microsecond; of whole lines, 8 lanes each, 60.
 #pragma once
@@ -9,7 +9,7 @@
 
 namespace vy_rows {
 
-template <int NT, int MB, int NW = 4> constexpr int RED = (NW - 1) * NT * MB * 64;   // f32x4 of LDS that stream() needs
+template <int NT, int MB> constexpr int RED = 3 * NT * MB * 64;   // f32x4 of LDS that stream() needs
 template <int NT, int MB, int NW = 4> constexpr int DENSE_RED = NW * NT * MB * 64;   // and dense()
 constexpr int vy_max2(int a, int b) { return a > b ? a : b; }
 template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3 ? 8 : 4;
@@ -17,9 +17,9 @@ template <int NT, int MB> constexpr int STEPS = NT * MB == 1 ? 16 : NT + MB <= 3
 // acc[t][j] = 16 rows ws[t] x 16 rows xs[j] over the wave's share of K; a lane's pointers are its row (lane & 15) + 8 (lane >> 4).
 // D: a lane owns row lane & 15 of X and rows 4 (lane >> 4) .. + 3 of W.  Each load has a condition of its own: all of a step's behind one
 // branch came one step after the other (experts of 16 sequences 338 us, 32 433, instead of 321 and 411).
-template <int NT, int MB, bool ONCE, int NW>
+template <int NT, int MB>
 __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB]) {
-  constexpr int U = STEPS<NT, MB>;
+  constexpr int U = STEPS<NT, MB>, NW = 4;
   const int kq = (threadIdx.x & 63) >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const bf16x8 zero8 = {(bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f, (bf16)0.f};
@@ -36,8 +36,7 @@ __device__ __forceinline__ void share(const bf16* const (&ws)[NT], const bf16* c
 #pragma unroll
       for (int t = 0; t < NT; ++t) {
         const bf16x8* at = reinterpret_cast<const bf16x8*>(ws[t] + k);
-        if constexpr (ONCE) w[u][t] = in ? __builtin_nontemporal_load(at) : zero8;
-        else w[u][t] = in ? *at : zero8;
+        w[u][t] = in ? __builtin_nontemporal_load(at) : zero8;
       }
 #pragma unroll
       for (int j = 0; j < MB; ++j) x[u][j] = in ? *reinterpret_cast<const bf16x8*>(xs[j] + k) : zero8;
@@ -134,12 +133,12 @@ __device__ __forceinline__ void share_lds(const bf16* x, int64_t ldx, int M, con
 }
 
 // share() and, in wave 0, the waves' sums
-template <int NT, int MB, bool ONCE = true, int NW = 4>
+template <int NT, int MB>
 __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* const (&xs)[MB], int K, f32x4 (&acc)[NT][MB],
                                        f32x4* red) {
   const int lane = threadIdx.x & 63;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  share<NT, MB, ONCE, NW>(ws, xs, K, acc);
+  share<NT, MB>(ws, xs, K, acc);
   __syncthreads();   // (red may still be read from the pass before)
   if (wave)
 #pragma unroll
@@ -153,7 +152,7 @@ __device__ __forceinline__ void stream(const bf16* const (&ws)[NT], const bf16* 
 #pragma unroll
       for (int j = 0; j < MB; ++j)
 #pragma unroll
-        for (int s = 0; s < NW - 1; ++s) {
+        for (int s = 0; s < 3; ++s) {
           const f32x4 v = red[(s * NT * MB + t * MB + j) * 64 + lane];
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc[t][j][r] += v[r];
@@ -179,13 +178,21 @@ __device__ __forceinline__ void dense(const Dense& a, char* lds, int tile, int K
   const int lane = threadIdx.x & 63, r16 = lane & 15, kq = lane >> 4;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   f32x4* red = reinterpret_cast<f32x4*>(lds);
-  bf16 bias[MINE][4];   // (as they come: a conversion here waits for them ahead of the stream)
-  if (a.bias) {   // (uniform)
+  // biases of the wave's blocks, a quad each: as they come, since what unpacks them here waits for them ahead of the stream
+  uint2 bias[MINE];
+  if (a.bias && (uintptr_t)a.bias % 8 == 0 && R * tile + 16 * NT <= a.N) {   // (uniform)
 #pragma unroll
     for (int b = 0; b < MINE; ++b)
-      if (wave + NW * b < BLOCKS)
+      if (wave + NW * b < BLOCKS) bias[b] = *reinterpret_cast<const uint2*>(a.bias + R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq);
+  } else if (a.bias) {
 #pragma unroll
-        for (int r = 0; r < 4; ++r) bias[b][r] = a.bias[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
+    for (int b = 0; b < MINE; ++b)
+      if (wave + NW * b < BLOCKS) {
+        unsigned v[4];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) v[r] = reinterpret_cast<const unsigned short*>(a.bias)[min(R * tile + 16 * ((wave + NW * b) / MB) + 4 * kq + r, a.N - 1)];
+        bias[b] = make_uint2(v[0] | v[1] << 16, v[2] | v[3] << 16);
+      }
   }
   f32x4 acc[NT][MB];
   share_lds<NT, MB, NW, D, R>(a.x, a.ldx, a.M, a.w, a.K, R * tile, a.N, K, lds, acc);
@@ -219,7 +226,10 @@ __device__ __forceinline__ void dense(const Dense& a, char* lds, int tile, int K
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       float z = v[r];
-      if (a.bias) z += (float)bias[b][r];
+      if (a.bias) {
+        const unsigned two = r < 2 ? bias[b].x : bias[b].y;
+        z += __builtin_bit_cast(float, r & 1 ? two & 0xffff0000u : two << 16);
+      }
       if constexpr (ACT != VY_ACT_NONE) z = vy_act_fwd<ACT>(z, a.act_arg);
       w4[r] = (bf16)z;
     }
