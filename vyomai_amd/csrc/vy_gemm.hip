@@ -2164,8 +2164,8 @@ __global__ __launch_bounds__(256) void splitk_finish_ln_row_kernel(const float* 
 
 // ------------------------------------------------------------------------------------------
 // 16 output columns per workgroup (M <= 32): the decode projections with N/32 < ~200 workgroups leave most
-// of the 256 CUs without a weight stream, and ONE CU pulls only ~25-40 GB/s (what its L1 keeps in flight
-// over a memory latency), so such a launch runs at a quarter of the chip's bandwidth.  Halving the tile
+// of the 256 CUs without a weight stream, and ONE CU takes in only 25 to 30 KB of such
+// fragments a microsecond, so such a launch runs at a quarter of the chip's bandwidth.  Halving the tile
 // doubles the CUs that stream: mfma_f32_16x16x32_bf16, A = 16 weight rows x 32 k, B = 16 batch rows x 32 k
 // (two row blocks), K split over the workgroup's 4 waves, partial sums through LDS.  D[n][m]: a lane owns
 // batch row lane & 15 and the 4 consecutive columns 4 * (lane >> 4) .. + 3.  With fused RoPE a workgroup

@@ -74,7 +74,7 @@ int vy_rows_linear(const void* x, const void* w, const void* bias, int act, floa
 
 // internal (vy_hybrid.hip): the product of a sublayer's output, whose rows vy_residual_norm_parts adds to the stream: fp32 partial sums
 // parts[slice][M][N] of K cut into that many slices (returned; 0: other sizes).  A product with as few columns as the stream has 32
-// or 64 workgroups of 32 columns, and what one CU takes in (25 to 40 GB/s) sets its time; slices bring the workgroups to 256, and
+// or 64 workgroups of 32 columns, and what one CU takes in sets its time; slices bring the workgroups to 256, and
 // wider tiles halve the times x is read: 64 columns where they still are 256 workgroups.  32 rows, 1024 x 6144: 23.3 -> 6.8 us;
 // 2048 x 8192: 11.4 (32 columns: 12.7); 2048 x 12288: 43.2 -> 16.6 (17.9); 1024 x 1024: 6.1 -> 3.5; 8 rows: 13.3 -> 5.4, 24.8 -> 14.2,
 // 4.2 -> 3.2 (weights from HBM); with whole lines through LDS 5.1, 9.4, 12.7, 3.3 and 4.6, 11.3, 3.0.  A slice keeps at least 128 columns:
