@@ -2164,36 +2164,39 @@ __global__ __launch_bounds__(256) void splitk_finish_ln_row_kernel(const float* 
 
 // ------------------------------------------------------------------------------------------
 // 16 output columns per workgroup (M <= 32): the decode projections with N/32 < ~200 workgroups leave most
-// of the 256 CUs without a weight stream, and ONE CU takes in only 25 to 30 KB of such
-// fragments a microsecond, so such a launch runs at a quarter of the chip's bandwidth.  Halving the tile
+// of the 256 CUs without a weight stream, and what one CU takes in sets the time.  Halving the tile
 // doubles the CUs that stream: mfma_f32_16x16x32_bf16, A = 16 weight rows x 32 k, B = 16 batch rows x 32 k
-// (two row blocks), K split over the workgroup's 4 waves, partial sums through LDS.  D[n][m]: a lane owns
+// (MB row blocks), K split over the workgroup's 4 waves, partial sums through LDS.  The operands come by whole 128-byte lines into
+// LDS, 512 columns of K at a time and the next 512 on their way: of MFMA fragments requested by the lanes that need them (16 rows
+// and 16 bytes a lane) a CU takes in 25 to 30 KB a microsecond, of lines 60.  28 rows: 768 x 3072 13.5 -> 7.6 us,
+// 2304 x 768 with RoPE 6.8 -> 5.5, 3072 x 768 with GELU 6.4 -> 5.2, 768 x 768 4.1 -> 3.2.  D[n][m]: a lane owns
 // batch row lane & 15 and the 4 consecutive columns 4 * (lane >> 4) .. + 3.  With fused RoPE a workgroup
 // takes columns {d0 .. d0+7} and {d0+32 .. d0+39} of one head: a rotary pair sits in lanes l and l ^ 32.
 // ------------------------------------------------------------------------------------------
-template <int EPI, int ACT>
+template <int EPI, int ACT, int MB>
 __global__ __launch_bounds__(256) void gemm_skinny16_bf16_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
-    int K, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int dbg) {
-  __shared__ float red[3][8][64];
+    int K, EpiPlain<bf16> ep, EpiQkv<bf16> eq) {
+  constexpr int XG = 2 * MB, GROUPS = XG + 2, LINE = GROUPS * 1024, CHUNK = 8 * LINE;   // groups of 8 rows of a line: of X, of W
+  __shared__ __attribute__((aligned(16))) char smem[2 * CHUNK];
+  __shared__ f32x4 red[3][MB][64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int r16 = lane & 15, kq = lane >> 4;
   const int nb = blockIdx.x;
   const bool rope_map = (EPI == 1) && eq.rope;
-  int col = nb * 16 + r16;
-  if (rope_map) col = (nb >> 2) * 64 + (nb & 3) * 8 + (r16 < 8 ? r16 : 24 + r16);
-  const int wr = col < N ? col : N - 1;
-  const int m0r = r16 < M ? r16 : M - 1, m1r = 16 + r16 < M ? 16 + r16 : M - 1;
-  const bf16* wp = W + (int64_t)wr * ldw + kq * 8;
-  const bf16* xp0 = X + (int64_t)m0r * ldx + kq * 8;
-  const bf16* xp1 = X + (int64_t)m1r * ldx + kq * 8;
-  // measurement knobs (VY_SKINNY_DBG; wrong results): 1 = every lane reads X row 0, 2 = every workgroup reads the
-  // weight rows of tile 0, 4 = one k-step only, 8 = no epilogue, 16 = return at once
-  if (dbg & 16) return;
-  if (dbg & 1) { xp0 = X + kq * 8; xp1 = xp0; }
-  if (dbg & 2) wp = W + (int64_t)r16 * ldw + kq * 8;
-  const bool two = M > 16;   // (wave-uniform) a second block of batch rows exists
+  const int rows[2] = {r16 < M ? r16 : M - 1, 16 + r16 < M ? 16 + r16 : M - 1};
+  // a lane's places of the loads: row lane / 8 of each group, 16 bytes of a line; chunk c of row r lies at c ^ (r / 2 & 7)
+  const bf16* at[GROUPS];
+  int kat[GROUPS];
+#pragma unroll
+  for (int g = 0; g < GROUPS; ++g) {
+    const int row = 8 * g + (lane >> 3);
+    int n = row - 16 * MB;
+    n = rope_map ? (nb >> 2) * 64 + (nb & 3) * 8 + (n < 8 ? n : 24 + n) : nb * 16 + n;
+    kat[g] = 64 * wave + 8 * ((lane & 7) ^ ((row >> 1) & 7));
+    at[g] = (g < XG ? X + (int64_t)(row < M ? row : M - 1) * ldx : W + (int64_t)(n < N ? n : N - 1) * ldw) + kat[g];
+  }
   // the epilogue's operands that do not depend on the product (bias, residual, rotary cos / sin) are requested
   // up front, under the weight stream: loaded after the reduction they are one more dependent memory round
   // trip in a kernel that is nothing but round trips (measured: the epilogue was 2 of this kernel's ~5 us)
@@ -2204,66 +2207,86 @@ __global__ __launch_bounds__(256) void gemm_skinny16_bf16_kernel(
   if (biasp && fast) bias4 = *reinterpret_cast<const bf16x4*>(biasp + nq0);
   bf16x4 res4[2];
   if (EPI == 0 && fast && ep.residual) {
-    res4[0] = *reinterpret_cast<const bf16x4*>(ep.residual + (int64_t)m0r * ep.ldr + nq0);
-    res4[1] = *reinterpret_cast<const bf16x4*>(ep.residual + (int64_t)m1r * ep.ldr + nq0);
+    res4[0] = *reinterpret_cast<const bf16x4*>(ep.residual + (int64_t)rows[0] * ep.ldr + nq0);
+    if (MB == 2) res4[1] = *reinterpret_cast<const bf16x4*>(ep.residual + (int64_t)rows[1] * ep.ldr + nq0);
   }
   f32x4 cos4[2], sin4[2];
   if (rope_map) {
     const int64_t pbase = eq.pos_dev ? (int64_t)*eq.pos_dev : eq.pos0;
     const int dcol = (nb & 3) * 8 + 4 * (kq & 1);
 #pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      const int64_t mm = blk == 0 ? m0r : m1r;
+    for (int blk = 0; blk < MB; ++blk) {
+      const int64_t mm = rows[blk];
       const int64_t pp = pbase + (mm - (mm / eq.L) * eq.L);
       cos4[blk] = *reinterpret_cast<const f32x4*>(eq.cos_tab + pp * 32 + dcol);
       sin4[blk] = *reinterpret_cast<const f32x4*>(eq.sin_tab + pp * 32 + dcol);
     }
   }
-  const int nsteps = (dbg & 4) ? 4 : K >> 5;
-  f32x4 acc0 = {0.f, 0.f, 0.f, 0.f}, acc1 = {0.f, 0.f, 0.f, 0.f};
-  int s = wave;
-  constexpr int U = 6;   // K = 768: the wave's 6 k-steps in one trip, 18 loads in flight per lane
-  for (; s + 4 * (U - 1) < nsteps; s += 4 * U) {
-    bf16x8 a[U], b0[U], b1[U];
+  const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
+  const int chunks = (K + 511) / 512;
+  auto stage = [&](int c) {   // lines wave and wave + 4 of the chunk
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      a[u] = *reinterpret_cast<const bf16x8*>(wp + 32 * (s + 4 * u));
-      b0[u] = *reinterpret_cast<const bf16x8*>(xp0 + 32 * (s + 4 * u));
-      b1[u] = *reinterpret_cast<const bf16x8*>(xp1 + 32 * (s + 4 * u));
-    }
-    __builtin_amdgcn_sched_barrier(0);
+    for (int i = 0; i < 2; ++i)
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b0[u], acc0, 0, 0, 0);
-      if (two) acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b1[u], acc1, 0, 0, 0);
+      for (int g = GROUPS - 1; g >= 0; --g) {
+        const int k = 512 * c + 256 * i;
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(kat[g] + k < K ? at[g] + k : zero), (VY_LDS void*)(smem + (c & 1) * CHUNK + (wave + 4 * i) * LINE + g * 1024), 16, 0, 0);
+      }
+  };
+  f32x4 acc[MB];
+#pragma unroll
+  for (int j = 0; j < MB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
+  const unsigned frag = vy_lds_addr(smem) + r16 * 128 + (((4 * (wave & 1) + kq) ^ ((r16 >> 1) & 7)) << 4) + (wave >> 1) * LINE;   // k-step `wave`
+  stage(0);
+  if (chunks > 1) stage(1);
+  for (int c = 0; c < chunks; ++c) {
+    if (c + 1 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * GROUPS) : "memory");
+    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const unsigned from = frag + (c & 1) * CHUNK;
+    bf16x8 a[4], b[4][MB];
+    vy_static_for<4>([&](auto u_c) {   // k-steps wave + 4 u of the chunk
+      constexpr int u = decltype(u_c)::value;
+      a[u] = vy_lds_read128_off<2 * u * LINE + 16 * MB * 128>(from);
+      b[u][0] = vy_lds_read128_off<2 * u * LINE>(from);
+      if constexpr (MB == 2) b[u][MB - 1] = vy_lds_read128_off<2 * u * LINE + 16 * 128>(from);
+    });
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      vy_tie(a[u]);
+#pragma unroll
+      for (int j = 0; j < MB; ++j) {
+        vy_tie(b[u][j]);
+        acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u][j], acc[j], 0, 0, 0);
+      }
     }
-  }
-  for (; s < nsteps; s += 4) {
-    const bf16x8 a = *reinterpret_cast<const bf16x8*>(wp + 32 * s);
-    const bf16x8 b0 = *reinterpret_cast<const bf16x8*>(xp0 + 32 * s);
-    const bf16x8 b1 = *reinterpret_cast<const bf16x8*>(xp1 + 32 * s);
-    acc0 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b0, acc0, 0, 0, 0);
-    if (two) acc1 = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b1, acc1, 0, 0, 0);
+    if (c + 2 < chunks) {
+      __builtin_amdgcn_s_barrier();   // the buffer has been read
+      asm volatile("" ::: "memory");
+      stage(c + 2);
+    }
   }
   if (wave > 0) {
 #pragma unroll
-    for (int r = 0; r < 4; ++r) { red[wave - 1][r][lane] = acc0[r]; red[wave - 1][4 + r][lane] = acc1[r]; }
+    for (int j = 0; j < MB; ++j) red[wave - 1][j][lane] = acc[j];
   }
   __syncthreads();
   if (wave != 0) return;
-  if (dbg & 8) { if (acc0[0] == 12345.678f) ep.y[0] = (bf16)acc1[0]; return; }
 #pragma unroll
-  for (int r = 0; r < 4; ++r) {
-    acc0[r] += red[0][r][lane] + red[1][r][lane] + red[2][r][lane];
-    acc1[r] += red[0][4 + r][lane] + red[1][4 + r][lane] + red[2][4 + r][lane];
+  for (int j = 0; j < MB; ++j) {
+    const f32x4 v1 = red[0][j][lane], v2 = red[1][j][lane], v3 = red[2][j][lane];
+#pragma unroll
+    for (int r = 0; r < 4; ++r) acc[j][r] += v1[r] + v2[r] + v3[r];
   }
 #pragma unroll
-  for (int blk = 0; blk < 2; ++blk) {
+  for (int blk = 0; blk < MB; ++blk) {
     const int64_t m = blk * 16 + r16;
     if (m >= M) continue;
     float v[4];
 #pragma unroll
-    for (int r = 0; r < 4; ++r) v[r] = blk == 0 ? acc0[r] : acc1[r];
+    for (int r = 0; r < 4; ++r) v[r] = acc[blk][r];
     if constexpr (EPI == 0) {
       if (fast && !ep.pre && !ep.residual2 && !ep.drop.thr) {   // epi_plain_quad on the prefetched operands
 #pragma unroll
@@ -2555,9 +2578,8 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
   } else if (M <= 32 && K % 32 == 0 && !GRAD && N % 16 == 0 && N / 32 < 200 && skinny16_on &&
              (EPI == 0 || !eq.rope || (N % 64 == 0 && eq.dh == 64))) {
     // few 32-column workgroups: 16-column ones, so that twice as many CUs stream weights
-    static const int sk_dbg = [] { const char* e = getenv("VY_SKINNY_DBG"); return e ? atoi(e) : 0; }();
-    hipLaunchKernelGGL((gemm_skinny16_bf16_kernel<EPI, ACT>), dim3((unsigned)(N / 16)), dim3(256), 0, st, X, ldx,
-                       W, ldw, (int)M, (int)N, (int)K, ep, eq, sk_dbg);
+    if (M <= 16) hipLaunchKernelGGL((gemm_skinny16_bf16_kernel<EPI, ACT, 1>), dim3((unsigned)(N / 16)), dim3(256), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, ep, eq);
+    else hipLaunchKernelGGL((gemm_skinny16_bf16_kernel<EPI, ACT, 2>), dim3((unsigned)(N / 16)), dim3(256), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, ep, eq);
   } else if (M <= 32 && K % 16 == 0 && !GRAD && (EPI == 0 || !eq.rope || N % 64 == 0) && N <= skinny_max_n) {
     hipLaunchKernelGGL((gemm_skinny_bf16_kernel<EPI, ACT>), dim3((unsigned)vy_cdiv(N, 32)), dim3(256), 0, st, X, ldx,
                        W, ldw, (int)M, (int)N, (int)K, ep, eq);
