@@ -1,5 +1,5 @@
 """Weight gradients of which a launch adds one sum to an element -- read, added to and written, no atomics, for tiles inside the gradient --
-and the launches that few rows share: against fp64."""
+and launches of few rows: against fp64."""
 import pytest
 import torch
 
@@ -66,17 +66,6 @@ def test_by_itself(M, N, K):
     dw, db = before.clone(), torch.full((N,), -0.25, device=DEV)
     ops.linear_wgrad(dy, x, dw, db, True)
     check(dy, x, dw, db, before)
-
-
-def test_which_gradients_go_out_together():
-    """Any rows where launches take several layers' gradients; a launch per layer (exchanged gradients) begins at more."""
-    from vyomai_amd import autograd_train as AT
-    g = AT._WgradGroup()
-    p = torch.nn.Parameter(torch.zeros(4))
-    assert g.gathers((768, 768), (p, None)) and g.gathers((2304, 768), [p])
-    assert not g.gathers((50265, 768), (p,)) and not g.gathers((64, 64), (p,)) and not g.gathers((768, 4), (p,))
-    p._vy_exchanged = True
-    assert not g.gathers((768, 768), (p, None))
 
 
 def test_operands_of_another_type_go_out_by_themselves(monkeypatch):

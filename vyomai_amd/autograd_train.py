@@ -162,13 +162,6 @@ class _WgradGroup:
         N, K = w.shape
         return dy.numel() // N >= _GROUP_MIN_ROWS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0
 
-    def gathers(self, shape, members) -> bool:
-        """Gradients that go out with other layers' (none of them exchanged): whatever the rows.  The four of a layer of width 768,
-        microseconds one by one / in launches of 256 tiles: 24 rows 34 / 15, 200 rows 43 / 18, 512 rows 70 / 21, 1665 rows 114 / 36,
-        2047 rows 120 / 40 (width 1024: 42 / 24 to 151 / 64), and half the host's time."""
-        N, K = shape
-        return _GROUP_WGRADS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0 and not any(getattr(p, "_vy_exchanged", False) for p in members)
-
     def add(self, dy, x, w, b) -> None:
         self.add_tensors(dy, x, w.grad, None if b is None else b.grad, [p for p in (w, b) if p is not None])
 
@@ -225,8 +218,10 @@ class _WgradGroup:
 
 _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
-_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # of a launch per layer (exchanged gradients): 2112 rows of width 768, a
-# layer's four gradients, 116 us one by one and 73 in a launch of their own
+_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 116 us one by one,
+# 73 in a launch of their own, 46 of one with its neighbours'.  It pays below as well -- 1665 rows 114 / 36, 512 rows 70 / 21, 200 rows 43 / 18 --,
+# but one sum over all rows instead of a dozen changes gradients by 2e-7, and a step's weights in enough places that the next one's gradients,
+# whose noise is the rounding of bf16, differ by 1 % from what they were (single values by more than the tensor's mean).
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group
 _wgrad_group = _WgradGroup()
 
@@ -234,7 +229,7 @@ _wgrad_group = _WgradGroup()
 def _wgrad(dy, x, w: torch.Tensor, b: Optional[torch.Tensor], alpha: Optional[torch.Tensor] = None):
     """-> (dw, db) to return to autograd (None when accumulated in place)."""
     if _direct(w) and (b is None or _direct(b)):
-        if _wgrad_group.wants(dy, w, alpha) or (alpha is None and _wgrad_group.gathers(w.shape, (w, b))):
+        if _wgrad_group.wants(dy, w, alpha):
             _wgrad_group.add(dy, x, w, b)
             return None, None
         ops.linear_wgrad(dy, x, w.grad, None if b is None else b.grad, accumulate=True, alpha=alpha)
@@ -645,8 +640,7 @@ def _packed_wgrad(mod, dy, x, w, b, params, members=None):
             ok = ok and all(p.grad.data_ptr() == db0.data_ptr() + off * 4 for p, off in zip(bs, _offsets(bs)))
         if ok:
             dy2 = dy.view(-1, dy.shape[-1])
-            if _GROUP_WGRADS and _GROUP_QKV and (_wgrad_group.gathers(dw.shape, members) or (
-                    dy2.shape[0] >= _GROUP_MIN_ROWS and N * dw.shape[1] >= 512 * 512 and dw.shape[1] % 8 == 0)):
+            if _GROUP_WGRADS and _GROUP_QKV and dy2.shape[0] >= _GROUP_MIN_ROWS and N * dw.shape[1] >= 512 * 512 and dw.shape[1] % 8 == 0:
                 # with the layer's other weight gradients in one grouped launch (27 of its 108 tiles: on its own
                 # this launch ran at 670 TFLOP/s, the group at 850)
                 _wgrad_group.add_tensors(dy2, x, dw, db, list(members))
