@@ -99,3 +99,44 @@ def test_saved_tensors_go_through_their_hooks():
     with torch.autograd.graph.saved_tensors_hooks(lambda t: (packed.append(t.shape), t.cpu())[1], lambda t: t.to(DEV)):
         got = step(b, ids, mask)
     assert len(packed) >= 6 and torch.equal(got[0], want[0]) and all(torch.equal(got[1][n], want[1][n]) for n in want[1])
+
+
+def hooked(kind, ff, att):
+    """A hook of that kind that changes a gradient -> handles"""
+    from torch.nn.modules import module as M
+    half = lambda g: tuple(None if t is None else 0.5 * t for t in g)
+    if kind == "full":
+        return [ff.register_full_backward_hook(lambda m, gi, go: half(gi))]
+    if kind == "pre":
+        return [att.register_full_backward_pre_hook(lambda m, go: half(go))]
+    if kind == "old":
+        return [ff.register_backward_hook(lambda m, gi, go: None)]
+    if kind == "global":
+        return [M.register_module_full_backward_hook(lambda m, gi, go: half(gi) if m is ff else None)]
+    return [M.register_module_full_backward_pre_hook(lambda m, go: half(go) if m is att else None)]
+
+
+@pytest.mark.parametrize("kind", ["full", "pre", "old", "global", "global pre"])
+def test_backward_hooks_see_their_modules(kind):
+    """A hook that halves a gradient: what the modules one by one make of it."""
+    ids, mask = inputs(2, 20, False)
+    plain = model("decoder", 512, 8)
+    results = []
+    for one_by_one in (False, True):
+        m = copy.deepcopy(plain)
+        handles = hooked(kind, m.all_layer[1].feed_forward, m.all_layer[1].attention)
+        try:
+            results.append(step(m, ids, mask, one_by_one=one_by_one))
+        finally:
+            for h in handles:
+                h.remove()
+    (y, grads, calls), (y2, grads2, _) = results
+    assert calls == ([] if "global" in kind else ["vy_text_layer_train_fwd", "vy_text_layer_bwd"])      # (the other layer's)
+    assert torch.equal(y, y2)
+    unhooked = step(plain, ids, mask)[1]
+    changed = False
+    for n in grads:
+        bound = 2.0 ** -16 * grads2[n].abs().max() + 1e-12      # (as above: sums in atomics)
+        assert (grads[n] - grads2[n]).abs().max() <= bound, n
+        changed |= bool((grads[n] - unhooked[n]).abs().max() > bound)
+    assert changed == (kind != "old"), kind

@@ -135,6 +135,7 @@ def self_attention_block(mod, x, attention_mask, freqs, cache, cache_index, star
 
 
 _GLOBAL_HOOKS = (torch.nn.modules.module._global_forward_hooks, torch.nn.modules.module._global_forward_pre_hooks)
+_GLOBAL_BACKWARD_HOOKS = (torch.nn.modules.module._global_backward_hooks, torch.nn.modules.module._global_backward_pre_hooks)
 
 
 def _plain_layer(att, ff, x, mask) -> bool:
@@ -209,10 +210,18 @@ def layer_forward(att, ff, x, mask, freqs, cache=None, start_pos: int = 0):
     return ops.text_layer(desc, x)
 
 
+def _backward_hooks(att, ff) -> bool:
+    """Is there a hook on the gradients of the two modules' outputs or inputs?"""
+    if _GLOBAL_BACKWARD_HOOKS[0] or _GLOBAL_BACKWARD_HOOKS[1]:
+        return True
+    return any(d["_backward_hooks"] or d["_backward_pre_hooks"] for d in (att.__dict__, ff.__dict__))
+
+
 def layer_train(att, ff, x, mask, freqs):
     """The same with gradients: one autograd function, whose forward and backward are a native call each (vy_text_layer_train_fwd,
-    vy_text_layer_bwd), where every gradient goes straight into the trainer's arena.  None: as above."""
-    if not torch.is_grad_enabled() or not _plain_layer(att, ff, x, mask):
+    vy_text_layer_bwd), where every gradient goes straight into the trainer's arena.  None: as above, and with a backward hook, which only
+    a call of its module sees."""
+    if not torch.is_grad_enabled() or not _plain_layer(att, ff, x, mask) or _backward_hooks(att, ff):
         return None
     from .autograd_train import TextLayerFn, _direct
     members = att._params()
