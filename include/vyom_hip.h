@@ -422,6 +422,8 @@ int vy_linear_dgrad(const void* dy, int64_t lddy, const void* wt, int64_t ldwt, 
 /* dW[N,K] (fp32, accumulate when beta != 0) = alpha * dY[M,N]^T . X[M,K];  db[N] (fp32) likewise
  * alpha * colsum(dY).  alpha_dev: optional DEVICE fp32 scalar (NULL = 1), e.g. the upstream
  * gradient of a loss whose unit gradient is already stored in dY -- no host sync to read it.
+ * With beta != 0 every sum is added by an atomic: launches on any streams, of this call and of the two below, may add to one
+ * gradient at the same time.
  * dtype VY_BF16: MFMA kernels (K, lddy, ldx multiples of 8).  VY_F32: the parity path, plain FMAs
  * (any K; the reference's autograd of nn.Linear in full precision). */
 int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int64_t ldx, float* dw,

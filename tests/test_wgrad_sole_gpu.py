@@ -1,5 +1,5 @@
-"""Weight gradients of which a launch adds one sum to an element -- read, added to and written, no atomics, for tiles inside the gradient --
-and launches of few rows: against fp64."""
+"""Weight gradients of which a launch adds one sum to an element, by themselves and several in one launch: against fp64; and launches on two
+streams that add to one gradient."""
 import pytest
 import torch
 
@@ -66,6 +66,34 @@ def test_by_itself(M, N, K):
     dw, db = before.clone(), torch.full((N,), -0.25, device=DEV)
     ops.linear_wgrad(dy, x, dw, db, True)
     check(dy, x, dw, db, before)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(64, 512, 512), (200, 16384, 256), (4096, 32768, 520)])
+def test_two_streams_add_to_one_gradient(M, N, K):
+    """Launches of one and of several gradients on two streams at once, with nothing between them.  Whole numbers: the sums, up to
+    12 * 2 * 4096 * 6, and every sum on the way are exact in fp32, in whatever order they are added."""
+    from vyomai_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    streams = [torch.cuda.Stream(), torch.cuda.Stream()]
+    operands = []
+    for _ in streams:
+        dy = torch.randint(-2, 3, (M, N), device=DEV, generator=g).to(BF)
+        x = torch.randint(-3, 4, (M, K), device=DEV, generator=g).to(BF)
+        operands.append((dy, x))
+    once = [a.float().T.contiguous() @ b.float() for a, b in operands]
+    dw, db = torch.full((N, K), 5.0, device=DEV), torch.full((N,), -7.0, device=DEV)
+    torch.cuda.synchronize()
+    for _ in range(6):
+        for s, (dy, x) in zip(streams, operands):
+            with torch.cuda.stream(s):
+                ops.linear_wgrad(dy, x, dw, db, True)
+                if N < 16384:
+                    ops.linear_wgrad_grouped([(dy, x, dw, db)])
+    torch.cuda.synchronize()
+    n = 12 if N < 16384 else 6
+    assert torch.equal(dw, 5.0 + n * (once[0] + once[1]))
+    assert torch.equal(db, -7.0 + n * sum(a.float().sum(0) for a, _ in operands))
 
 
 def test_operands_of_another_type_go_out_by_themselves(monkeypatch):

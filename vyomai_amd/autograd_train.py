@@ -218,8 +218,8 @@ class _WgradGroup:
 
 _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
-_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 116 us one by one,
-# 73 in a launch of their own, 46 of one with its neighbours'.  It pays below as well -- 1665 rows 114 / 36, 512 rows 70 / 21, 200 rows 43 / 18 --,
+_GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 121 us one by one,
+# 52 of a launch with its neighbours'.  It pays below as well -- 1665 rows 114 / 47, 512 rows 71 / 32, 200 rows 49 / 28 --,
 # but one sum over all rows instead of a dozen changes gradients by 2e-7, and a step's weights in enough places that the next one's gradients,
 # whose noise is the rounding of bf16, differ by 1 % from what they were (single values by more than the tensor's mean).
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group

@@ -55,15 +55,11 @@ __device__ __forceinline__ bf16x8 tr_pair(const char* base, int row_bytes) {
 // columns: the source-side swizzle gets a second bit ((row >> 2) & 1) << 5 that puts them in the two 32-byte halves of a
 // 64-byte slot (conflict-free).  The atomic epilogue exchanges lane halves of two neighbouring k blocks
 // (v_permlane32_swap) so that a wave instruction is again two 128-byte row segments.
-// sole: the launch adds one sum to each element of dW -- read, added to and written with plain loads and stores, a batch of loads
-// ahead of the stores, for tiles inside dW (atomics, which run in L2 at 1.6 to 3 TB/s, elsewhere; the same bits for alpha = 1).  252
-// tiles of 256 x 256, 64 MB of sums, 24 rows: 56 -> 33 us; four gradients of a layer of width 768, 2112 rows: 51.7 -> 40.4, 12608 rows
-// 171 -> 167; 50265 x 768: 64 rows 121 -> 51 us, 2112 rows 255 -> 223, 16384 rows 1264 -> 1254.
 template <int BN, int BKW, int MS, int NS, bool MF16 = false>
 __device__ __forceinline__ void wgrad_tn_bf16_body(
     const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
     float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
-    int M, int N, int K, int tiles_k, int m_chunk, int diag, int split, int t2, bool sole) {
+    int M, int N, int K, int tiles_k, int m_chunk, int diag, int split, int t2) {
   constexpr int NW = BN / 32;                 // waves: (BN/64) x 2
   constexpr int WKT = BKW / 2, TJ = WKT / 32; // k extent of a wave, 32-wide fragments along k
   constexpr int AROW = BN * 2, BROW = BKW * 2;  // LDS row bytes of the dY and X tiles
@@ -246,40 +242,6 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
     // D[n][k] of block (i, j): lane = k index (lane & 15), register r = n row 4 kq + r.  Blocks j and j + 1 trade lane
     // halves so that one wave instruction adds rows {r, 4 + r} (then {8 + r, 12 + r}) x 32 consecutive k
     const bool hi = lane >= 32;
-    // halves of (j, j + 1) traded: rows r (0) or 8 + r (1) of the lane's four
-    auto pair = [&](int i, int jp, int r, float (&v)[2]) {
-      auto sw = __builtin_amdgcn_permlane32_swap(__builtin_bit_cast(unsigned, acc[i][2 * jp][r] * alpha),
-                                                 __builtin_bit_cast(unsigned, acc[i][2 * jp + 1][r] * alpha), false, false);
-      v[0] = __builtin_bit_cast(float, (unsigned)sw[0]);
-      v[1] = __builtin_bit_cast(float, (unsigned)sw[1]);
-    };
-    if (sole && n0 + BN <= N && k0 + BKW <= K) {
-      float* at = dW + (int64_t)(n0 + wn * 64 + 4 * (kq & 1)) * lddw + k0 + wk * WKT + (hi ? 16 : 0) + r16;
-      float old[2][JH][4][2];
-      auto request = [&](int i) {
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int e = 0; e < 2; ++e)
-#pragma unroll
-            for (int jp = 0; jp < JH; ++jp) old[i & 1][jp][r][e] = at[(int64_t)(16 * i + r + 8 * e) * lddw + 32 * jp];
-      };
-      request(0);
-#pragma unroll
-      for (int i = 0; i < TI; ++i) {
-        if (i + 1 < TI) request(i + 1);
-#pragma unroll
-        for (int r = 0; r < 4; ++r)
-#pragma unroll
-          for (int jp = 0; jp < JH; ++jp) {
-            float v[2];
-            pair(i, jp, r, v);
-#pragma unroll
-            for (int e = 0; e < 2; ++e) at[(int64_t)(16 * i + r + 8 * e) * lddw + 32 * jp] = old[i & 1][jp][r][e] + v[e];
-          }
-      }
-      return;
-    }
 #pragma unroll
     for (int i = 0; i < TI; ++i)
 #pragma unroll
@@ -287,12 +249,13 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
         const int k = k0 + wk * WKT + 16 * (2 * jp + (hi ? 1 : 0)) + r16;
 #pragma unroll
         for (int r = 0; r < 4; ++r) {
-          float v[2];
-          pair(i, jp, r, v);
+          const unsigned x = __builtin_bit_cast(unsigned, acc[i][2 * jp][r] * alpha);
+          const unsigned y = __builtin_bit_cast(unsigned, acc[i][2 * jp + 1][r] * alpha);
+          auto sw = __builtin_amdgcn_permlane32_swap(x, y, false, false);
           const int nlo = n0 + wn * 64 + 16 * i + 4 * (kq & 1) + r;
           if (k < K) {
-            if (nlo < N) atomicAdd(dW + (int64_t)nlo * lddw + k, v[0]);
-            if (nlo + 8 < N) atomicAdd(dW + (int64_t)(nlo + 8) * lddw + k, v[1]);
+            if (nlo < N) atomicAdd(dW + (int64_t)nlo * lddw + k, __builtin_bit_cast(float, (unsigned)sw[0]));
+            if (nlo + 8 < N) atomicAdd(dW + (int64_t)(nlo + 8) * lddw + k, __builtin_bit_cast(float, (unsigned)sw[1]));
           }
         }
       }
@@ -421,27 +384,6 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
       if (fh == 0 && n < N) atomicAdd(db + n, t_);
     }
   }
-  if (sole && n0 + BN <= N && k0 + BKW <= K) {
-    float* at = dW + (int64_t)(n0 + wn * 64 + 4 * fh) * lddw + k0 + wk * WKT + fr;
-    float old[2][TJ][16];
-    auto row = [](int i, int r) { return 32 * i + (r & 3) + 8 * (r >> 2); };
-    auto request = [&](int i) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) old[i][j][r] = at[(int64_t)row(i, r) * lddw + 32 * j];
-    };
-    request(0);
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-      if (i == 0) request(1);
-#pragma unroll
-      for (int r = 0; r < 16; ++r)
-#pragma unroll
-        for (int j = 0; j < TJ; ++j) at[(int64_t)row(i, r) * lddw + 32 * j] = old[i][j][r] + acc[i][j][r] * alpha;
-    }
-    return;
-  }
 #pragma unroll
   for (int i = 0; i < 2; ++i)
 #pragma unroll
@@ -461,10 +403,10 @@ template <int BN, int BKW, int MS, int NS, bool MF16 = false>
 __global__ __launch_bounds__(BN * 2, BN == 128 ? 2 : 1) void wgrad_tn_bf16_kernel(
     const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
     float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
-    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag, bool sole) {
+    int M, int N, int K, int tiles_k, int tiles_nk, int m_chunk, int diag) {
   const int wg = xcd_remap(blockIdx.x, gridDim.x), split = wg / tiles_nk;
   wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, tiles_k, m_chunk, diag, split,
-                                            wg - split * tiles_nk, sole);
+                                            wg - split * tiles_nk);
 }
 
 // The 256 x 256 tiles (tiles_k of them side by side) from `first` on, four workgroups of 128 x 128 each, two on a CU.  An element is
@@ -478,7 +420,7 @@ __global__ __launch_bounds__(256, 2) void wgrad_quarters_kernel(
   const int tile_n = 2 * tile + ((wg >> 1) & 1), tile_k = 2 * (t - tile * tiles_k) + (wg & 1);
   if (tile_n * 128 >= N || tile_k * 128 >= K) return;
   wgrad_tn_bf16_body<128, 128, 64, 2, true>(dY, lddy, X, ldx, dW, lddw, db, alpha_dev, M, N, K, 2 * tiles_k, m_chunk, diag, 0,
-                                            tile_n * 2 * tiles_k + tile_k, true);
+                                            tile_n * 2 * tiles_k + tile_k);
 }
 
 // Several weight gradients in ONE launch (vy_linear_wgrad_grouped, vy_linear_wgrad_batch): the four GEMMs of a transformer layer
@@ -489,7 +431,6 @@ struct WgradItem {
   const bf16* dY; const bf16* X; float* dW; float* db;
   int64_t lddy, ldx, lddw;
   int M, N, K, tiles_k, tiles_nk, m_chunk, item0;   // item0: first work item of this GEMM
-  bool sole;
 };
 constexpr int MOST_WGRADS = 12;
 struct WgradGroup { WgradItem g[MOST_WGRADS]; int n; };
@@ -507,7 +448,7 @@ __global__ __launch_bounds__(BN * 2, 1) void wgrad_tn_bf16_grouped_kernel(WgradG
   for (int i = 1; i < MOST_WGRADS; ++i)
     if (d == i) it = grp.g[i];
   wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(it.dY, it.lddy, it.X, it.ldx, it.dW, it.lddw, it.db, nullptr, it.M, it.N, it.K,
-                                      it.tiles_k, it.m_chunk, diag, (id - it.item0) / it.tiles_nk, (id - it.item0) % it.tiles_nk, it.sole);
+                                      it.tiles_k, it.m_chunk, diag, (id - it.item0) / it.tiles_nk, (id - it.item0) % it.tiles_nk);
 }
 
 // db[n] += sum_m dY[m,n]: block = 64 lanes x 8 columns, 256 rows per block
@@ -1175,15 +1116,14 @@ extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int6
   // the others.  50265 x 768 over 16384 rows, 591 tiles: 1543 -> 1478 us; 8192 rows 742 -> 700; 22016 x 768 over 8192 rows, 258 tiles:
   // 461 -> 380; 11008 x 2048, 344 tiles: 482 -> 411.  (Halves of 256 x 128, one on a CU: 1490, 712, 410, 427.)
   const int whole = var == 8 && w16 && splits == 1 && tiles > 256 && tiles % 256 > 0 && tiles % 256 <= 128 ? tiles / 256 * 256 : tiles;
-  const bool sole = splits == 1;
 #define WG_GO(BN_, BK_, MS_, NS_)                                                                          \
   hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_>), dim3((unsigned)(whole * splits)), dim3(BN_ * 2), 0, \
                      st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
-                     (int)K, tiles_k, whole, (int)m_chunk, diag, sole)
+                     (int)K, tiles_k, whole, (int)m_chunk, diag)
 #define WG_GO16(BN_, BK_, MS_, NS_)                                                                        \
   hipLaunchKernelGGL((wgrad_tn_bf16_kernel<BN_, BK_, MS_, NS_, true>), dim3((unsigned)(whole * splits)), dim3(BN_ * 2), 0, \
                      st, (const bf16*)dy, lddy, (const bf16*)x, ldx, dw, lddw, db, alpha_dev, (int)M, (int)N, \
-                     (int)K, tiles_k, whole, (int)m_chunk, diag, sole)
+                     (int)K, tiles_k, whole, (int)m_chunk, diag)
   if (var == 1) { if (ns == 3) WG_GO(256, 128, 64, 3); else WG_GO(256, 128, 64, 2); }
   else if (var == 2) WG_GO(128, 256, 32, 2);
   else if (var == 4) WG_GO(128, 256, 32, 3);
@@ -1238,9 +1178,6 @@ static int wgrad_together(const char* who, const vy_wgrad_desc* descs, int32_t n
     it.lddy = d.lddy; it.ldx = d.ldx; it.lddw = d.lddw;
     it.M = (int)d.M; it.N = (int)d.N; it.K = (int)d.K;
     it.tiles_k = (int)tiles_k; it.tiles_nk = (int)tiles; it.m_chunk = (int)m_chunk; it.item0 = (int)items;
-    it.sole = splits == 1;
-    for (int j = 0; j < n; ++j)   // (two sums for one gradient meet in atomics)
-      if (j != i && descs[j].dw < d.dw + (d.N - 1) * d.lddw + d.K && d.dw < descs[j].dw + (descs[j].N - 1) * descs[j].lddw + descs[j].K) it.sole = false;
     items += tiles * splits;
   }
   for (int i = n; i < MOST_WGRADS; ++i) grp.g[i] = grp.g[0];
