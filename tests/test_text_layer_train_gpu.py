@@ -140,3 +140,21 @@ def test_backward_hooks_see_their_modules(kind):
         assert (grads[n] - grads2[n]).abs().max() <= bound, n
         changed |= bool((grads[n] - unhooked[n]).abs().max() > bound)
     assert changed == (kind != "old"), kind
+
+
+def test_what_waiting_weight_gradients_hold(monkeypatch):
+    """Their operands and nothing else of the layer, 16 numbers of a row's width a token: x, o, a and the inner rows of four widths, and
+    the gradients of both norms' inputs, of the inner rows and of the projections of three widths."""
+    from vyomai_amd import autograd_train as AT
+    B, L, d, layers = 8, 256, 512, 2
+    ids, mask = inputs(B, L, False)
+    held, real = [], AT.ops.linear_wgrad_grouped
+
+    def launch(items):
+        held.extend(t for dy, x, *_ in items for t in (dy, x))
+        real(items)
+    monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", launch)
+    calls = step(model("decoder", d, 8, layers=layers), ids, mask)[2]
+    assert len(calls) == 2 * layers and len(held) >= 2 * 4 * layers
+    storages = {t.untyped_storage().data_ptr(): t.untyped_storage().nbytes() for t in held}
+    assert sum(storages.values()) <= layers * (16 * d * B * L * 2 + 16 * 128)     # (a segment is filled up to a line)

@@ -491,55 +491,68 @@ class TextLayerFn(torch.autograd.Function):
 
     @staticmethod
     def _kept(x, hk_dh, inner, h):
-        """Offsets of [q | o | s1 | a | deriv | inner | s2 | k | v] and of the statistics."""
+        """Offsets of what the weight gradients multiply with, [o | a | inner], of the rest, [q | s1 | deriv | s2 | k | v], and of the
+        statistics: waiting weight gradients hold their operands' buffer, so the rest has one of its own."""
         B, L, d = x.shape
         M = B * L
-        return _segments(M * d, M * d, M * d, M * d, M * inner, M * inner, M * d, M * hk_dh, M * hk_dh), _segments(B * h * L, M, M, M, M)
+        return _segments(M * d, M * d, M * inner), _segments(M * d, M * d, M * inner, M * d, M * hk_dh, M * hk_dh), _segments(B * h * L, M, M, M, M)
+
+    @staticmethod
+    def _places(x, rows, rest, stats, operands, others, numbers):
+        """-> vy_text_layer_kept, and where the keys and the values are."""
+        e, r0, t0, s0 = x.element_size(), rows.data_ptr(), rest.data_ptr(), stats.data_ptr()
+        o, a, inner = (r0 + n * e for n in operands)
+        q, s1, deriv, s2, k, v = (t0 + n * e for n in others)
+        return _lib.VyTextLayerKept(q, o, s1, a, deriv, inner, s2, *(s0 + 4 * n for n in numbers)), (k, v)
 
     @staticmethod
     def forward(ctx, x, kp, att, ff, keep, causal, start, rope, *params):
         B, L, d = x.shape
         h, hk, dh, inner = att.num_attention_heads, att.num_key_value_heads, att.head_dim, keep[6].shape[0]
-        (at, n), (sat, sn) = TextLayerFn._kept(x, hk * dh, inner, h)
+        (operands, n), (others, m), (numbers, sn) = TextLayerFn._kept(x, hk * dh, inner, h)
         rows = torch.empty(n, dtype=x.dtype, device=x.device)
+        rest = torch.empty(m, dtype=x.dtype, device=x.device)
         stats = torch.empty(sn, dtype=torch.float32, device=x.device)
         y = torch.empty_like(x)
-        e, r0, s0 = x.element_size(), rows.data_ptr(), stats.data_ptr()
-        kept = _lib.VyTextLayerKept(*(r0 + o * e for o in at[:7]), *(s0 + 4 * o for o in sat))
-        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, (r0 + at[7] * e, r0 + at[8] * e))
+        kept, kv = TextLayerFn._places(x, rows, rest, stats, operands, others, numbers)
+        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, kv)
         ops._mid_ws(B * L)
         _lib.call("vy_text_layer_train_fwd", _ref(desc), _ref(kept), x.data_ptr(), y.data_ptr(), B, L, ops._stream())
-        ctx.save_for_backward(x, rows, stats, kp)
+        ctx.save_for_backward(x, rows, rest, stats, kp)
         ctx.meta = (att, ff, causal, start, rope, params)
         return y
 
     @staticmethod
     def backward(ctx, dy):
-        x, rows, stats, kp = ctx.saved_tensors
+        x, rows, rest, stats, kp = ctx.saved_tensors
         att, ff, causal, start, rope, params = ctx.meta
         B, L, d = x.shape
         dt, dev, M = x.dtype, x.device, B * L
-        dy, rows, stats = dy.contiguous(), rows.contiguous(), stats.contiguous()
+        dy, rows, rest, stats = dy.contiguous(), rows.contiguous(), rest.contiguous(), stats.contiguous()
         wo, bo, g1, b1, w1, c1, w2, c2, g2, b2 = params[:10]
         members = att._params()
         w, b = att._packed(members)
         keep = [*att._packed_shadow(dt, (w, b), members), *[_shadow(p, dt) for p in params[:10]]]
         h, hk, dh, inner = att.num_attention_heads, att.num_key_value_heads, att.head_dim, keep[6].shape[0]
         W = d + 2 * hk * dh
-        (at, _), (sat, _) = TextLayerFn._kept(x, hk * dh, inner, h)
-        e, r0, s0 = x.element_size(), rows.data_ptr(), stats.data_ptr()
-        kept = _lib.VyTextLayerKept(*(r0 + o * e for o in at[:7]), *(s0 + 4 * o for o in sat))
-        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, (r0 + at[7] * e, r0 + at[8] * e))
+        (operands, _), (others, _), (numbers, _) = TextLayerFn._kept(x, hk * dh, inner, h)
+        kept, kv = TextLayerFn._places(x, rows, rest, stats, operands, others, numbers)
+        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, kv)
         wt = [_wt_packed(att, w, dt, members), _wt(wo, dt), _wt(w1, dt), _wt(w2, dt)]
-        to, n = _segments(M * d, M * inner, M * d, M * d, M * d, M * W)      # ds2, dpre, da, ds1, dheads, dqkv
+        to, n = _segments(M * d, M * inner, M * d, M * W)      # ds2, dpre, ds1, dqkv: the weight gradients' other operands
         work = torch.empty(n, dtype=dt, device=dev)
+        oo, on = _segments(M * d, M * d)                       # da, dheads
+        own = torch.empty(on, dtype=dt, device=dev)
         fo, fn = _segments(2 * _lib.load().vy_layernorm_bwd_ws_rows(M) * d, B * h * L)
         scratch = torch.empty(fn, dtype=torch.float32, device=dev)
         dx = torch.empty_like(x)
-        w0, f0 = work.data_ptr(), scratch.data_ptr()
+        e, f0 = x.element_size(), scratch.data_ptr()
+        ds2, dpre, ds1, dqkv = (work.data_ptr() + o * e for o in to)
+        da, dheads = (own.data_ptr() + o * e for o in oo)
         # (a gradient that has left the arena since the forward pass is returned)
         dln = [p.grad if _direct(p) else torch.zeros(d, dtype=torch.float32, device=dev) for p in (g1, b1, g2, b2)]
-        grads = _lib.VyTextLayerGrads(*(t.data_ptr() for t in wt), *(t.stride(0) for t in wt), *(t.data_ptr() for t in dln), *(w0 + o * e for o in to), *(f0 + 4 * o for o in fo))
+        grads = _lib.VyTextLayerGrads(*(t.data_ptr() for t in wt), *(t.stride(0) for t in wt), *(t.data_ptr() for t in dln), ds2, dpre, da, ds1,
+                                      dheads, dqkv, *(f0 + 4 * o for o in fo))
         ops._mid_ws(M)
         _lib.call("vy_text_layer_bwd", _ref(desc), _ref(kept), _ref(grads), dy.data_ptr(), dx.data_ptr(), B, L, ops._stream())
         dg1, db1, dg2, db2 = (None if _direct(p) else t.to(p.dtype) for p, t in zip((g1, b1, g2, b2), dln))
@@ -547,11 +560,11 @@ class TextLayerFn(torch.autograd.Function):
 
         def of(t, o, cols):
             return t.as_strided((M, cols), (cols, 1), t.storage_offset() + o)
-        dw2 = _wgrad(of(work, to[0], d), of(rows, at[5], inner), w2, c2)
-        dw1 = _wgrad(of(work, to[1], inner), of(rows, at[3], d), w1, c1)
-        dwo = _wgrad(of(work, to[3], d), of(rows, at[1], d), wo, bo)
-        dqkv = _packed_wgrad(att, of(work, to[5], W), x, w, b, params[10:], members)
-        return (dx, *[None] * 7, *dwo, dg1, db1, *dw1, *dw2, dg2, db2, *dqkv)
+        dw2 = _wgrad(of(work, to[0], d), of(rows, operands[2], inner), w2, c2)
+        dw1 = _wgrad(of(work, to[1], inner), of(rows, operands[1], d), w1, c1)
+        dwo = _wgrad(of(work, to[2], d), of(rows, operands[0], d), wo, bo)
+        dqkv_w = _packed_wgrad(att, of(work, to[3], W), x, w, b, params[10:], members)
+        return (dx, *[None] * 7, *dwo, dg1, db1, *dw1, *dw2, dg2, db2, *dqkv_w)
 
 
 class CrossAttentionFn(torch.autograd.Function):
