@@ -2173,12 +2173,15 @@ __global__ __launch_bounds__(256) void splitk_finish_ln_row_kernel(const float* 
 // batch row lane & 15 and the 4 consecutive columns 4 * (lane >> 4) .. + 3.  With fused RoPE a workgroup
 // takes columns {d0 .. d0+7} and {d0+32 .. d0+39} of one head: a rotary pair sits in lanes l and l ^ 32.
 // ------------------------------------------------------------------------------------------
-template <int EPI, int ACT, int MB>
+// HELD: chunks in LDS.  Two of 32 rows are 96 KB and one workgroup on a CU, so a K of one chunk holds one, and up to 160 columns (one or two
+// k-steps a wave) none: a line's way through LDS takes longer there than the fragments' requests.  With two, one and none, 32 rows x 4096
+// columns K = 64 3.2, 2.9, 2.7 us, 160 3.4, 3.3, 3.1, 256 3.6, 3.6, -; x 4608, more workgroups than CUs, 4.8, 3.2, 2.8; 5.2, 3.8, 3.3; 5.2, 3.8, -.
+template <int EPI, int ACT, int MB, int HELD>
 __global__ __launch_bounds__(256) void gemm_skinny16_bf16_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
     int K, EpiPlain<bf16> ep, EpiQkv<bf16> eq) {
   constexpr int XG = 2 * MB, GROUPS = XG + 2, LINE = GROUPS * 1024, CHUNK = 8 * LINE;   // groups of 8 rows of a line: of X, of W
-  __shared__ __attribute__((aligned(16))) char smem[2 * CHUNK];
+  __shared__ __attribute__((aligned(16))) char smem[HELD ? HELD * CHUNK : 16];
   __shared__ f32x4 red[3][MB][64];
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -2237,10 +2240,23 @@ __global__ __launch_bounds__(256) void gemm_skinny16_bf16_kernel(
 #pragma unroll
   for (int j = 0; j < MB; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
   const unsigned frag = vy_lds_addr(smem) + r16 * 128 + (((4 * (wave & 1) + kq) ^ ((r16 >> 1) & 7)) << 4) + (wave >> 1) * LINE;   // k-step `wave`
-  stage(0);
-  if (chunks > 1) stage(1);
-  for (int c = 0; c < chunks; ++c) {
-    if (c + 1 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * GROUPS) : "memory");
+  if constexpr (HELD == 0) {
+    const int n = rope_map ? (nb >> 2) * 64 + (nb & 3) * 8 + (r16 < 8 ? r16 : 24 + r16) : nb * 16 + r16;
+    const bf16* wp = W + (int64_t)(n < N ? n : N - 1) * ldw + 8 * kq;
+    for (int k = 32 * wave; k < K; k += 128) {
+      const bf16x8 a = *reinterpret_cast<const bf16x8*>(wp + k);
+      bf16x8 b[MB];
+#pragma unroll
+      for (int j = 0; j < MB; ++j) b[j] = *reinterpret_cast<const bf16x8*>(X + (int64_t)rows[j] * ldx + 8 * kq + k);
+#pragma unroll
+      for (int j = 0; j < MB; ++j) acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b[j], acc[j], 0, 0, 0);
+    }
+  } else {
+    stage(0);
+    if (HELD == 2) stage(1);
+  }
+  for (int c = 0; c < (HELD == 2 ? chunks : HELD); ++c) {
+    if (HELD == 2 && c + 1 < chunks) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * GROUPS) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
@@ -2262,7 +2278,7 @@ __global__ __launch_bounds__(256) void gemm_skinny16_bf16_kernel(
         acc[j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[u], b[u][j], acc[j], 0, 0, 0);
       }
     }
-    if (c + 2 < chunks) {
+    if (HELD == 2 && c + 2 < chunks) {
       __builtin_amdgcn_s_barrier();   // the buffer has been read
       asm volatile("" ::: "memory");
       stage(c + 2);
@@ -2578,8 +2594,11 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
   } else if (M <= 32 && K % 32 == 0 && !GRAD && N % 16 == 0 && N / 32 < 200 && skinny16_on &&
              (EPI == 0 || !eq.rope || (N % 64 == 0 && eq.dh == 64))) {
     // few 32-column workgroups: 16-column ones, so that twice as many CUs stream weights
-    if (M <= 16) hipLaunchKernelGGL((gemm_skinny16_bf16_kernel<EPI, ACT, 1>), dim3((unsigned)(N / 16)), dim3(256), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, ep, eq);
-    else hipLaunchKernelGGL((gemm_skinny16_bf16_kernel<EPI, ACT, 2>), dim3((unsigned)(N / 16)), dim3(256), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, ep, eq);
+#define VY_SKINNY16(MB, HELD) hipLaunchKernelGGL((gemm_skinny16_bf16_kernel<EPI, ACT, MB, HELD>), dim3((unsigned)(N / 16)), dim3(256), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, ep, eq)
+    const int held = K <= 160 ? 0 : K <= 512 ? 1 : 2;
+    if (M <= 16) { if (held == 0) VY_SKINNY16(1, 0); else if (held == 1) VY_SKINNY16(1, 1); else VY_SKINNY16(1, 2); }
+    else { if (held == 0) VY_SKINNY16(2, 0); else if (held == 1) VY_SKINNY16(2, 1); else VY_SKINNY16(2, 2); }
+#undef VY_SKINNY16
   } else if (M <= 32 && K % 16 == 0 && !GRAD && (EPI == 0 || !eq.rope || N % 64 == 0) && N <= skinny_max_n) {
     hipLaunchKernelGGL((gemm_skinny_bf16_kernel<EPI, ACT>), dim3((unsigned)vy_cdiv(N, 32)), dim3(256), 0, st, X, ldx,
                        W, ldw, (int)M, (int)N, (int)K, ep, eq);
