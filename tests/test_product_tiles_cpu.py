@@ -29,6 +29,15 @@ def test_kernel_is_a_fast_one(M, N, K, slices, fastest):
     assert S == slices and kind in fastest
 
 
+#: all of K in one workgroup, few stages of it: kernels within 8 % of the fastest
+@pytest.mark.parametrize("M,N,K,fastest", [
+    (530, 2432, 128, {"64"}), (430, 4224, 192, {"64"}), (1167, 1856, 192, {"64"}), (139, 8192, 64, {"64"}), (4181, 280, 64, {"64"}), (1019, 2056, 88, {"64"}),
+    (29760, 64, 192, {"64"}), (23937, 128, 384, {"64"}), (30506, 72, 1792, {"64", "128x128"}), (1825, 5120, 224, {"256x256"}), (13215, 384, 816, {"128x128", "256x128"})])
+def test_short_and_ragged_k(M, N, K, fastest):
+    kind, S = tiling(M, N, K)
+    assert S == 1 and kind in fastest
+
+
 @pytest.mark.parametrize("M,I,K,fastest", [(264, 8192, 2048, {"64"}), (129, 1024, 4096, {"64 many"}), (200, 1024, 4096, {"64 many"}),
                                            (129, 512, 2048, {"64 many"}), (129, 768, 3072, {"64 many"}), (264, 16384, 2048, {"256x256"})])
 def test_gated_products_stay_in_one_launch(M, I, K, fastest):

@@ -1726,9 +1726,10 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     case T_256x256: return whole_cost(M, N, K, chip, 256, 256, 1.71, 7.15, 1.633, 0.714, 0.2);
     case T_256x192: return whole_cost(M, N, K, chip, 256, 192, 2.57, 5.53, 1.278, 0.755, 0.18);
     case T_256x128: return whole_cost(M, N, K, chip, 256, 128, 2.86, 3.91, 0.993, 0.644, 0.2);
-    case T_128x128: return load <= 1 ? 2.76 + 0.84 * KT * (apart ? 1.3 : 1.0) : whole_cost(M, N, K, 2 * chip, 128, 128, 2.46, 3.65, 1.115, 0.417, 0.23);   // (two of them share a CU)
+    // (up to one on a CU: 272 shapes of K = 64 to 8192, 6 %.  Fitted to K from 256 on, it had 4.4 us for 530 x 2432, K = 128, which take 7.2, on 64 x 64 4.3)
+    case T_128x128: return load <= 1 ? 4.5 + 2.2 * load + 0.75 * KT * (apart ? 1.05 : 1.0) : whole_cost(M, N, K, 2 * chip, 128, 128, 2.46, 3.65, 1.115, 0.417, 0.23);   // (two of them share a CU)
     case T_64x64: {
-      if (S == 1) return 3.2 + (load > 1 ? 0.8 : 0.0) + KT * (0.25 * load > 0.335 ? 0.25 * load : 0.335);
+      if (S == 1) return 3.2 + (load > 1 ? 0.8 : 0.0) + KT * (0.25 * load > 0.335 ? 0.25 * load : 0.335) * (apart ? 1.08 : 1.0);
       const double n = (double)vy_cdiv(tiles, (int64_t)chip), stage = 0.238 * n - 0.204;   // the fullest CU holds n (up to three at once)
       return 4.0 + KT * (stage > 0.374 ? stage : 0.374) * (apart && n > 1 ? 1.3 : 1.0);
     }
