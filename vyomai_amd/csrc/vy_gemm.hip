@@ -1690,8 +1690,8 @@ inline Scratch splitk_ws(hipStream_t st) {
 // Tiles of a product of more than 32 rows.  What a shape costs depends on how its tiles fill the 256 CUs as much as on the tile's
 // own rate: 8192 x 2048 with K = 12288 is 352 tiles of 256 x 192 -- two rounds, the second a third full, 459 us -- or 256 tiles of
 // 256 x 256: 313 us; 8000 x 1024, K = 6144: 124 us on 256 x 192, 152 us on 256 x 256, 100 us on 256 x 128 (250 tiles).  So the
-// launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below (a GELU epilogue's
-// extra time grows with the output alone and so moves no choice); the constants are fits: whole_cost, and where K is sliced (up to 4096
+// launcher compares, in microseconds, rounds x (fixed part + stages x time per 64-deep stage) over the kernels below (and a GELU epilogue's
+// time, gelu_cost); the constants are fits: whole_cost, and where K is sliced (up to 4096
 // rows) 1600 shapes of 33 to 4096 rows, 64 to 40000 columns and K = 256 to
 // 16384, each on all kernels that take it, in graphs that walk through 200 MB of weights, as a model's layers do: products that find
 // their weights in L2, as a loop over one product does, made one launch look shorter than two groups in it.  The kernel chosen takes
@@ -1746,6 +1746,14 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     }
   }
 }
+// What a GELU adds on tiles of `rows` rows that take all of K: 2 us a tile of a CU, 6 where the tile has no table (256 x 192), and little on 64 x 64
+// tiles, which share a CU (medians over 150 shapes: 2.6, 2.2 and 1.8 us on 256, 224 and 160 x 256, 1.9 on 256 x 128, 2.3 on 128 x 128, 6.0, 0.3).
+// 32237 x 1920, K = 432: 100.9 us on 256 x 192, 79.8 on 256 x 256.
+inline double gelu_cost(TileKind kind, int64_t M, int64_t N, int rows, int chip) {
+  const int64_t tiles = vy_cdiv(M, rows) * vy_cdiv(N, TILE_N[kind]);
+  if (kind == T_64x64) return 0.3 * (double)tiles / chip;
+  return (kind == T_256x192 ? 6.0 : 2.0) * (double)vy_cdiv(tiles, (int64_t)chip);
+}
 // the same of two groups on tiles of 32, 96 or 128 rows and 64 columns (fits to 450 to 680 shapes, 3 to 6 % added where 64 rows and K over
 // workgroups were as fast as predicted to be slower)
 template <int ROWS>
@@ -1786,21 +1794,22 @@ inline int sum_slices(int64_t M, int64_t N, int64_t K) {
 }
 
 // `behind`: microseconds that K over several workgroups costs besides
-inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes, double behind = 0.0) {
+inline Tiling pick_tiling(int64_t M, int64_t N, int64_t K, int chip, int64_t ws_bytes, double behind = 0.0, bool gelu = false) {
   const int S = sum_slices(M, N, K);
   Tiling best{T_64x64, S, 64};
   double least = 1e30;
   auto offer = [&](TileKind kind, double us, int rows = 0) {
     if (us < least) { least = us; best.kind = kind; best.rows = rows ? rows : TILE_M[kind]; }
   };
-  offer(T_64x64, tile_cost<T_64x64>(M, N, K, S, chip));
+  offer(T_64x64, tile_cost<T_64x64>(M, N, K, S, chip) + (S == 1 && gelu ? gelu_cost(T_64x64, M, N, 64, chip) : 0.0));
   if (S == 1) {
-    offer(T_256x256, tile_cost<T_256x256>(M, N, K, S, chip));
-    offer(T_256x256, whole_cost(M, N, K, chip, 224, 256, 2.07, 6.19, 1.524, 0.726, 0.22), 224);
-    offer(T_256x256, whole_cost(M, N, K, chip, 160, 256, 1.92, 4.73, 1.326, 0.683, 0.25), 160);
-    offer(T_256x192, tile_cost<T_256x192>(M, N, K, S, chip));
-    offer(T_256x128, tile_cost<T_256x128>(M, N, K, S, chip));
-    offer(T_128x128, tile_cost<T_128x128>(M, N, K, S, chip));
+    auto whole = [&](TileKind kind, double us, int rows) { offer(kind, us + (gelu ? gelu_cost(kind, M, N, rows, chip) : 0.0), rows); };
+    whole(T_256x256, tile_cost<T_256x256>(M, N, K, S, chip), 256);
+    whole(T_256x256, whole_cost(M, N, K, chip, 224, 256, 2.07, 6.19, 1.524, 0.726, 0.22), 224);
+    whole(T_256x256, whole_cost(M, N, K, chip, 160, 256, 1.92, 4.73, 1.326, 0.683, 0.25), 160);
+    whole(T_256x192, tile_cost<T_256x192>(M, N, K, S, chip), 256);
+    whole(T_256x128, tile_cost<T_256x128>(M, N, K, S, chip), 256);
+    whole(T_128x128, tile_cost<T_128x128>(M, N, K, S, chip), 128);
     return best;
   }
   const TileKind groups = S <= 4 ? T_64x64_TWICE : T_64x64_MANY;
@@ -2616,7 +2625,7 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     const Scratch ws = splitk_ws(st);
     Tiling t{};
     if (var < 0) {
-      t = pick_tiling(M, N, K, chip, ws.bytes);
+      t = pick_tiling(M, N, K, chip, ws.bytes, 0.0, EPI == 0 && !GRAD && (ACT == VY_ACT_GELU_ERF || ACT == VY_ACT_GELU_TANH));
       if (t.slices == 1 && (variant == 40 || variant == 41)) t = {variant == 40 ? T_256x192 : T_256x256, 1, 256};
     }
     const int bm = var >= 0 ? 256 : t.rows, bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
@@ -2835,7 +2844,11 @@ extern "C" int vy_debug_tiling(int64_t M, int64_t N, int64_t K, int64_t ws_bytes
   return (int)t.kind + 16 * t.slices;
 }
 
-// test aid, not part of include/vyom_hip.h: the rows of a tile of that kernel
+// test aids, not part of include/vyom_hip.h: the same for a GELU, and the rows of a tile of that kernel
+extern "C" int vy_debug_tiling_gelu(int64_t M, int64_t N, int64_t K, int64_t ws_bytes) {
+  const Tiling t = pick_tiling(M, N, K, 256 / g_chains, ws_bytes, 0.0, true);
+  return (int)t.kind + 16 * t.slices;
+}
 extern "C" int vy_debug_tile_rows(int64_t M, int64_t N, int64_t K, int64_t ws_bytes, double behind) {
   return pick_tiling(M, N, K, 256 / g_chains, ws_bytes, behind).rows;
 }
