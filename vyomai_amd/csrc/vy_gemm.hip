@@ -707,9 +707,11 @@ __device__ __forceinline__ void gemm_epilogue(typename AccTile<BM, BN, WGM, WGN,
       const std::integral_constant<bool, false> ragged{};
       const bf16x8 none{};
       if constexpr (PASSES == 1 && EpiAhead<BM, BN, WGM * WGN, EPI, GRAD>::ON) {
-        if (ahead.on) {
-#pragma unroll
-          for (int it = 0; it < ITERS; ++it) do_chunk(whole, dst, dual, pass, tid + it * NT, staged(tid + it * NT), true, ahead.v[it]);
+        if (ahead.on) {   // (a register each: 14 chunks with the tanh GELU were left a loop, and the operand in scratch memory)
+          vy_static_for<ITERS>([&](auto it_c) __attribute__((always_inline)) {
+            constexpr int c = decltype(it_c)::value;
+            do_chunk(whole, dst, dual, pass, tid + c * NT, staged(tid + c * NT), true, ahead.v[c]);
+          });
           return;
         }
       }
@@ -1748,7 +1750,7 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
 }
 // What a GELU adds on tiles of `rows` rows that take all of K: 2 us a tile of a CU, 6 where the tile has no table (256 x 192), and little on 64 x 64
 // tiles, which share a CU (medians over 150 shapes: 2.6, 2.2 and 1.8 us on 256, 224 and 160 x 256, 1.9 on 256 x 128, 2.3 on 128 x 128, 6.0, 0.3).
-// 32237 x 1920, K = 432: 100.9 us on 256 x 192, 79.8 on 256 x 256.
+// 32237 x 1920, K = 432: 100.9 us on 256 x 192, 79.8 on 256 x 256.  (Not beside a residual, where nobody looks up: 12.5, 10.2, 7.4; 6.7; 3.1; 8.1.)
 inline double gelu_cost(TileKind kind, int64_t M, int64_t N, int rows, int chip) {
   const int64_t tiles = vy_cdiv(M, rows) * vy_cdiv(N, TILE_N[kind]);
   if (kind == T_64x64) return 0.3 * (double)tiles / chip;
@@ -2625,7 +2627,7 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     const Scratch ws = splitk_ws(st);
     Tiling t{};
     if (var < 0) {
-      t = pick_tiling(M, N, K, chip, ws.bytes, 0.0, EPI == 0 && !GRAD && (ACT == VY_ACT_GELU_ERF || ACT == VY_ACT_GELU_TANH));
+      t = pick_tiling(M, N, K, chip, ws.bytes, 0.0, EPI == 0 && !GRAD && (ACT == VY_ACT_GELU_ERF || ACT == VY_ACT_GELU_TANH) && !ep.residual);
       if (t.slices == 1 && (variant == 40 || variant == 41)) t = {variant == 40 ? T_256x192 : T_256x256, 1, 256};
     }
     const int bm = var >= 0 ? 256 : t.rows, bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
