@@ -23,6 +23,13 @@ def test_stored(M, K, N):
     within(y[:, :N], want + bias.double(), e + 2.0 ** -23 * want.abs())
 
 
+@pytest.mark.parametrize("M", [17, 32])
+@pytest.mark.parametrize("K", [8, 64, 248, 256, 264])
+def test_wide_products_of_few_columns(M, K):
+    """16400 weight rows are more than a round of 64 a workgroup: one line a wave, the last one short or not there, and more."""
+    test_stored(M, K, 16400)
+
+
 @pytest.mark.parametrize("M", [5, 32])
 @pytest.mark.parametrize("N", [40, 4100, 12300])
 def test_biases_that_start_anywhere(N, M):

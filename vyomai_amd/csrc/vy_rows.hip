@@ -30,6 +30,8 @@ __global__ __launch_bounds__(256) void rows_parts_kernel(Dense a, int len, int t
 // microsecond: 4.5 of the 6.8 us below): 32 rows, 6144 x 1024 6.8 -> 5.2 us, 8192 x 1024 7.1 -> 5.7, 2048 x 1024 5.5 -> 3.7, 6144 x 2048
 // 11.5 -> 7.8, 12288 x 2048 16.7 -> 12.6, 16384 x 2048 21.5 -> 14.6, 32000 x 1024 20.0 -> 15.3 (64 rows a workgroup 17.6), 32000 x 2048 38.2 ->
 // 27.7; 8 rows 5.4 -> 4.6, 6.6 -> 5.2, 4.3 -> 3.4, 8.8 -> 6.9, 14.7 -> 12.0, 20.1 -> 13.8, 18.8 -> 13.9, 34.9 -> 24.8.  The same bits.
+// Wide and beside 32 rows of x, up to 256 columns of K are one line a wave, so room for one: 40 KB, four workgroups on a CU.  32 rows, 38360 x 64,
+// 6.4 -> 4.8 us (5.5 straight into registers), 27072 x 168 6.5 -> 5.2 (6.6), 17000 x 256 5.2 -> 4.9 (6.6).
 template <int ACT, int MB>
 void rows_go(const Dense& a, hipStream_t st) {
   // few workgroups with long rows: twice the waves each (32 rows, 2048 x 2048 8.2 -> 4.9 us)
@@ -46,7 +48,15 @@ void rows_go(const Dense& a, hipStream_t st) {
   if (best == 16) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 1, false, 3>), grid, block, 0, st, a);
   else if (best == 24) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 2, true, 3>), grid, block, 0, st, a);
   else if (best == 32) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 2, false, 3>), grid, block, 0, st, a);
-  else if (best == 48) hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 3, false, 2>), grid, block, 0, st, a);
+  else if (best == 48) {
+    if constexpr (MB == 2) {
+      if (rounds(64) > 1 && a.K <= 256) {
+        hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 3, false, 1>), grid, block, 0, st, a);
+        return;
+      }
+    }
+    hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 3, false, 2>), grid, block, 0, st, a);
+  }
   else hipLaunchKernelGGL((rows_linear_kernel<ACT, MB, 4, 4, false, 2>), grid, block, 0, st, a);
 }
 
