@@ -108,7 +108,7 @@ def test_vision_and_captioning_layers():
     """A packed projection with one bias, rows without a mask, and keys of an image ahead of padded ones."""
     (y, grads, calls), (y2, grads2, calls2) = vision_step(False), vision_step(True)
     assert calls == ["vy_text_layer_train_fwd"] * 4 + ["vy_text_layer_bwd"] * 4 and not calls2
-    assert torch.equal(y, y2) and any("qkv" in n for n in grads)
+    assert (y - y2).abs() <= 36 * 2.0 ** -24 * y2 and any("qkv" in n for n in grads)      # (a sum over 36 tokens in atomics)
     for n in grads:
         assert grads2[n].abs().max() > 0 and (grads[n] - grads2[n]).abs().max() <= 2.0 ** -16 * grads2[n].abs().max(), n      # (sums in atomics)
 

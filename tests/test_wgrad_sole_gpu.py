@@ -1,5 +1,7 @@
 """Weight gradients of which a launch adds one sum to an element, by themselves and several in one launch: against fp64; and launches on two
 streams that add to one gradient."""
+import types
+
 import pytest
 import torch
 
@@ -109,3 +111,63 @@ def test_operands_of_another_type_go_out_by_themselves(monkeypatch):
         g.add_tensors(torch.empty(4, 512, dtype=dt), None, dw, None, [])
     g.flush()
     assert alone == [(torch.float32, True)] and together == [2]
+
+
+def test_what_waits_goes_out_on_the_stream_of_its_operands(monkeypatch):
+    """The end of a backward pass that was called on another stream than the forward pass ran on."""
+    import contextlib
+    from vyomai_amd import autograd_train as AT
+    now, done = [5], []
+
+    class Stream:
+        def __init__(self, raw):
+            self.raw = raw
+
+        def wait_stream(self, other):
+            done.append(("wait", self.raw, other.raw))
+
+    @contextlib.contextmanager
+    def inside(s):
+        before, now[0] = now[0], s.raw
+        yield
+        now[0] = before
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: Stream(now[0]))
+    monkeypatch.setattr(torch.cuda, "stream", inside)
+    monkeypatch.setattr(AT.ops, "_raw_stream", lambda: now[0])
+    monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", lambda items: done.append(("launch", now[0])))
+    g = AT._WgradGroup()
+    g.armed = True
+    dy = types.SimpleNamespace(dtype=torch.bfloat16, is_cuda=True)
+    for caller, want in ((0, [("launch", 5), ("wait", 0, 5)]), (5, [("launch", 5)])):
+        now[0] = 5
+        g.add_tensors(dy, None, torch.empty(512, 512, device="meta"), None, [])
+        now[0] = caller
+        g._end_of_backward()
+        assert done == want and not g.items
+        done.clear()
+        g.armed = True
+
+
+@pytest.mark.gpu
+def test_backward_called_on_another_stream():
+    from vyomai_amd import autograd_train as AT
+    from vyomai_amd.training import FlatTrainer
+    from tests.test_text_layer_train_gpu import inputs, model
+    ids, _ = inputs(8, 256, False)
+    grads = []
+    for apart in (False, True):
+        m = model("decoder", 512, 8)
+        tr = FlatTrainer(m, lr=0.0)
+        tr.zero_grad()
+        side = torch.cuda.Stream() if apart else torch.cuda.current_stream()
+        side.wait_stream(torch.cuda.current_stream())
+        with torch.cuda.stream(side):
+            out = m.forward_hidden(ids, None)[0]
+            loss = (out.float() * torch.randn(out.shape, device=DEV, generator=torch.Generator(device=DEV).manual_seed(9))).mean()
+        torch.cuda.current_stream().wait_stream(side)
+        loss.backward()
+        grads.append({n: p.grad.clone() for n, p in m.named_parameters() if "all_layer" in n})
+        assert not AT._wgrad_group.items
+        torch.cuda.synchronize()
+    for n, a in grads[0].items():
+        assert a.abs().max() > 0 and (a - grads[1][n]).abs().max() <= 2.0 ** -16 * a.abs().max(), n      # (sums in atomics)

@@ -154,7 +154,7 @@ class _WgradGroup:
     EXCHANGED, EXCHANGED_MOST = 100, 8                           # exchanged gradients: as many tiles or gradients end a launch
 
     def __init__(self):
-        self.items, self.tiles, self.armed, self.key = [], 0, False, None
+        self.items, self.tiles, self.armed, self.key, self.stream = [], 0, False, None, None
 
     def wants(self, dy, w, alpha) -> bool:
         if alpha is not None or not _GROUP_WGRADS:
@@ -178,8 +178,9 @@ class _WgradGroup:
         exchanged = any(getattr(p, "_vy_exchanged", False) for p in members)
         if self.tiles + tiles > self.TILES and not exchanged:
             self.flush()
+        if not self.items:
+            self.key, self.stream = key, torch.cuda.current_stream() if dy is not None and dy.is_cuda else None
         self.items.append((dy, x, dw, db, members))
-        self.key = key
         # autograd's own post-accumulate hook fires for these parameters as soon as this backward function
         # returns -- the reducer must not take that for "gradient written" (training.BucketReducer._hook)
         for p in members:
@@ -206,8 +207,16 @@ class _WgradGroup:
             _notify(*members)
 
     def _end_of_backward(self) -> None:
+        """On the stream that the backward pass was called on.  What waits may be of another one, the forward pass's: it goes out there, where
+        its operands were made, and the caller's stream waits for it."""
         self.armed = False
-        self.flush()
+        if not self.items or self.stream is None or self.key[1] == ops._raw_stream():
+            self.flush()
+            return
+        here, there = torch.cuda.current_stream(), self.stream
+        with torch.cuda.stream(there):
+            self.flush()
+        here.wait_stream(there)
 
     def discard(self) -> None:
         for *_, members in self.items:
