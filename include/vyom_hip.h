@@ -639,7 +639,7 @@ int64_t vy_decode_ws_bytes(int32_t B, int32_t d, int32_t h, int32_t hk, int32_t 
  * attended); hidden_out (nullable): (B, d) last hidden state; logits (nullable): (B, ldv).
  * pos_dev (nullable): device int32 holding the position -- when given, every kernel reads the
  * position on the device and `pos` is ignored, so one captured hipGraph of this call can be
- * replayed for every token (bf16, head_dim 64 models). */
+ * replayed for every token (bf16, head_dim 64 models).  x and the weight matrices start on 16 bytes. */
 int vy_decoder_step(const vy_decode_plan* plan, const void* x, int64_t pos, const int32_t* pos_dev,
                     void* hidden_out, void* logits, int64_t ldv, void* stream);
 

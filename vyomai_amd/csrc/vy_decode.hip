@@ -900,9 +900,16 @@ bool vy_dec_supported(int B, int d, int h, int hk, int dh, int ffn, int dtype) {
          (h + 2 * hk) * dh % 16 == 0 && dec_chunks(d, false) == 1 && dec_chunks(ffn, true) > 0;
 }
 
+// lines go to LDS in 16-byte pieces from places that are multiples of them
+static int dec_operands(const char* who, const void* x, const void* w) {
+  if (((uintptr_t)x | (uintptr_t)w) % 16) VY_FAIL(VY_ERR_ARG, "%s: operand rows must be 16-byte aligned", who);
+  return VY_OK;
+}
+
 int vy_dec_qkv(const void* x, const void* w, const void* bias, const float* cos_tab, const float* sin_tab, int64_t pos0,
                const int* pos_dev, void* q, void* k, void* v, int64_t c_sb, int64_t c_sh, int64_t c_sl, int B, int d, int h,
                int hk, hipStream_t st) {
+  if (int rc = dec_operands("vy_dec_qkv", x, w)) return rc;
   DecGemmArgs a{};
   a.X = (const bf16*)x; a.W = (const bf16*)w; a.bias = (const bf16*)bias;
   a.ldx = d; a.ldw = d; a.M = B; a.N = (h + 2 * hk) * 64;
@@ -917,6 +924,7 @@ int vy_dec_qkv(const void* x, const void* w, const void* bias, const float* cos_
 // y[B][N] = bf16(act(LN(x) W^T + b) + residual), K one chunk.  residual / ln_g / ln_b may be NULL (no residual / x as is)
 int vy_dec_linear_ex(const void* x, int ldx, const void* w, const void* bias, const void* residual, int ldr, const void* ln_g,
                      const void* ln_b, float ln_eps, void* y, int ldy, int B, int N, int K, int act, hipStream_t st) {
+  if (int rc = dec_operands("vy_dec_linear_ex", x, w)) return rc;
   DecGemmArgs a{};
   a.X = (const bf16*)x; a.W = (const bf16*)w; a.bias = (const bf16*)bias;
   a.ldx = ldx; a.ldw = K; a.M = B; a.N = N; a.y = (bf16*)y; a.ldy = ldy;
@@ -935,6 +943,7 @@ int vy_dec_linear_ex(const void* x, int ldx, const void* w, const void* bias, co
 // y[B][N] = act(x W^T + b), K one chunk
 int vy_dec_linear(const void* x, int ldx, const void* w, const void* bias, void* y, int ldy, int B, int N, int K, int act,
                   hipStream_t st) {
+  if (int rc = dec_operands("vy_dec_linear", x, w)) return rc;
   DecGemmArgs a{};
   a.X = (const bf16*)x; a.W = (const bf16*)w; a.bias = (const bf16*)bias;
   a.ldx = ldx; a.ldw = K; a.M = B; a.N = N; a.y = (bf16*)y; a.ldy = ldy;
@@ -952,6 +961,7 @@ int vy_dec_linear_res_ln(const void* x, int ldx, const void* w, const void* bias
                          const void* gamma, const void* beta, float eps, void* y, int ldy, float* part, int B, int N, int K,
                          int act, hipStream_t st) {
   const char* who = "vy_dec_linear_res_ln";
+  if (int rc = dec_operands(who, x, w)) return rc;
   if (N % 16 || N % 4 || N > 8192) VY_FAIL(VY_ERR_UNSUPPORTED, "%s: N = %d", who, N);
   DecGemmArgs a{};
   a.X = (const bf16*)x; a.W = (const bf16*)w; a.ldx = ldx; a.ldw = K; a.M = B; a.N = N; a.part = part;

@@ -600,6 +600,12 @@ extern "C" int vy_latent_decode(const void* q, int64_t ldq, const void* wukt, co
     const int64_t per = vy_cdiv((int64_t)B * h * nv, 256);         // sequences per workgroup: fill the CUs first
     p.seqs = (int)(per > 16 ? 16 : per);
     const dim3 vgrid(nv, h, (unsigned)vy_cdiv(B, p.seqs));
+    // (lines go to LDS in 16-byte pieces from places that are multiples of them; weights that start elsewhere are read a number at a time)
+    if ((uintptr_t)wuv % 16) {
+      hipLaunchKernelGGL(latent_value_gen_kernel<bf16>, dim3((unsigned)vy_cdiv(dv, 64), h, B), block, 0, st, p);
+      VY_CHECK_LAUNCH(who);
+      return VY_OK;
+    }
 #define VALUE_NB(RP, NB) hipLaunchKernelGGL((latent_value_kernel<RP, NB>), vgrid, block, (VALUE_LINES<RP, NB> + p.seqs * MAX_SPLIT * 4 + 4096 + 2 * p.seqs * (RP + 8) * 2), st, p)
 #define VALUE(RP) do { if (narrow) VALUE_NB(RP, 1); else VALUE_NB(RP, 4); } while (0)
     if (R <= 64) VALUE(64);

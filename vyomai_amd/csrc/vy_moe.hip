@@ -55,16 +55,22 @@ __global__ __launch_bounds__(64 * NW) void router_logits_kernel(const bf16* __re
   }
 }
 
-__global__ __launch_bounds__(256) void router_logits_f32_kernel(const float* __restrict__ h, int64_t ldh, const float* __restrict__ w,
-                                                                float* __restrict__ logits, int K, int E) {
+// a wave per logit: fp32, and bf16 rows that do not start on 16 bytes, from where lines go to LDS
+template <typename T>
+__global__ __launch_bounds__(256) void router_logits_plain_kernel(const T* __restrict__ h, int64_t ldh, const T* __restrict__ w,
+                                                                  float* __restrict__ logits, int K, int E) {
   const int lane = threadIdx.x & 63, e = blockIdx.y * 4 + (threadIdx.x >> 6);
   const int64_t m = blockIdx.x;
   if (e >= E) return;
   float s = 0.f;
-  for (int k = lane * 4; k < K; k += 256) {
-    const f32x4 a = *reinterpret_cast<const f32x4*>(h + m * ldh + k), b = *reinterpret_cast<const f32x4*>(w + (int64_t)e * K + k);
+  if constexpr (sizeof(T) == 4) {
+    for (int k = lane * 4; k < K; k += 256) {
+      const f32x4 a = *reinterpret_cast<const f32x4*>(h + m * ldh + k), b = *reinterpret_cast<const f32x4*>(w + (int64_t)e * K + k);
 #pragma unroll
-    for (int c = 0; c < 4; ++c) s = fmaf(a[c], b[c], s);
+      for (int c = 0; c < 4; ++c) s = fmaf(a[c], b[c], s);
+    }
+  } else {
+    for (int k = lane; k < K; k += 64) s = fmaf(VyT<T>::ld(h + m * ldh + k), VyT<T>::ld(w + (int64_t)e * K + k), s);
   }
   s = vy_wave_sum(s);
   if (lane == 0) logits[m * E + e] = s;
@@ -534,8 +540,11 @@ extern "C" int vy_moe_fwd(const vy_moe* d, const void* h, int64_t ldh, int64_t M
   const int up_rows = gated ? 2 * d->ff : d->ff;
   if (!small) hipLaunchKernelGGL(zero_kernel, dim3((unsigned)vy_cdiv((int64_t)E * COUNT_STRIDE, 256)), dim3(256), 0, st, p.counts, E * COUNT_STRIDE);
   if (dtype == VY_F32) {
-    hipLaunchKernelGGL(router_logits_f32_kernel, dim3((unsigned)M, (unsigned)vy_cdiv(E, 4)), dim3(256), 0, st, (const float*)h, ldh,
+    hipLaunchKernelGGL(router_logits_plain_kernel<float>, dim3((unsigned)M, (unsigned)vy_cdiv(E, 4)), dim3(256), 0, st, (const float*)h, ldh,
                        (const float*)d->w_router, p.logits, K, E);
+  } else if (((uintptr_t)h | (uintptr_t)d->w_router) % 16) {
+    hipLaunchKernelGGL(router_logits_plain_kernel<bf16>, dim3((unsigned)M, (unsigned)vy_cdiv(E, 4)), dim3(256), 0, st, (const bf16*)h, ldh,
+                       (const bf16*)d->w_router, p.logits, K, E);
   } else {
     // many tokens: 32, 48 or 64 a workgroup, one workgroup on a CU, by what the rounds of the 256 CUs take in
     const int64_t cols = vy_cdiv(E, 64);
