@@ -143,7 +143,7 @@ def _plain_layer(att, ff, x, mask) -> bool:
     a dense mask, rows that are not contiguous: the modules are then to be called one by one."""
     if type(ff) is not FeedForward or "_whole_layer" not in type(att).__dict__ or not (mask is None or isinstance(mask, AttnMask)):
         return False
-    aso = att._modules["out"]
+    aso = att._modules.get("out")
     if type(aso) is not AttentionSelfOutput or _GLOBAL_HOOKS[0] or _GLOBAL_HOOKS[1]:
         return False
     for d in (att.__dict__, aso.__dict__, ff.__dict__):
