@@ -47,6 +47,7 @@ PROTOTYPES = {
     "vy_linear_wgrad": [_p, _i64, _p, _i64, _p, _i64, _p, _f, _p, _i64, _i64, _i64, _i, _p],
     "vy_linear_wgrad_grouped": [_p, _i, _i, _p],
     "vy_linear_wgrad_batch": [_p, _i, _i, _p],
+    "vy_linear_wgrad_rows": [_p, _i, _i, _p],
     "vy_layernorm_bwd": [_p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p, _p, _f, _p, _i64, _i64, _i, _p],
     "vy_attn_bwd": [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
                     _p, _p, _i64, _i64, _p, _p,

@@ -200,11 +200,14 @@ class _WgradGroup:
         items, self.items, self.tiles = self.items, [], 0
         if not items:
             return
-        ops.linear_wgrad_grouped([(dy, x, dw, db) for dy, x, dw, db, _ in items])
+        self._launch([(dy, x, dw, db) for dy, x, dw, db, _ in items])
         for *_, members in items:
             for p in members:
                 p._vy_deferred = False
             _notify(*members)
+
+    def _launch(self, items) -> None:
+        ops.linear_wgrad_grouped(items)
 
     def _end_of_backward(self) -> None:
         """On the stream that the backward pass was called on.  What waits may be of another one, the forward pass's: it goes out there, where
@@ -225,14 +228,32 @@ class _WgradGroup:
         self.items, self.tiles, self.armed = [], 0, False
 
 
+class _WgradRows(_WgradGroup):
+    """The same for gradients over fewer rows than those: four layers' in a launch that sums each up as a launch of its own does
+    (ops.linear_wgrad_rows), so they keep their bits.  Exchanged gradients go out one by one."""
+
+    TILES, MOST = 1 << 30, 16
+
+    def gathers(self, dy, shape, members, alpha=None) -> bool:
+        if alpha is not None or not _GROUP_WGRADS or dy.dtype != torch.bfloat16:
+            return False
+        N, K = shape
+        return (dy.numel() // N < _GROUP_MIN_ROWS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0
+                and not any(getattr(p, "_vy_exchanged", False) for p in members))
+
+    def _launch(self, items) -> None:
+        ops.linear_wgrad_rows(items)
+
+
 _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
 _GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 121 us one by one,
-# 52 of a launch with its neighbours'.  It pays below as well -- 1665 rows 114 / 47, 512 rows 71 / 32, 200 rows 49 / 28 --,
-# but one sum over all rows instead of a dozen changes gradients by 2e-7, and a step's weights in enough places that the next one's gradients,
-# whose noise is the rounding of bf16, differ by 1 % from what they were (single values by more than the tensor's mean).
+# 58 of a launch with its neighbours'.  Below, tiles of 128 x 128 that sum the rows up as launches one by one do are faster (2047 rows 50,
+# 1665 rows 45 / 52 / 113 one by one) and keep the bits: another order changes gradients by 2e-7, and a step's weights in enough places that the
+# next one's gradients, whose noise is the rounding of bf16, differ by 1 % from what they were (single values by more than the tensor's mean).
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group
 _wgrad_group = _WgradGroup()
+_wgrad_rows = _WgradRows()
 
 
 def _wgrad(dy, x, w: torch.Tensor, b: Optional[torch.Tensor], alpha: Optional[torch.Tensor] = None):
@@ -240,6 +261,9 @@ def _wgrad(dy, x, w: torch.Tensor, b: Optional[torch.Tensor], alpha: Optional[to
     if _direct(w) and (b is None or _direct(b)):
         if _wgrad_group.wants(dy, w, alpha):
             _wgrad_group.add(dy, x, w, b)
+            return None, None
+        if _wgrad_rows.gathers(dy, w.shape, [p for p in (w, b) if p is not None], alpha):
+            _wgrad_rows.add(dy, x, w, b)
             return None, None
         ops.linear_wgrad(dy, x, w.grad, None if b is None else b.grad, accumulate=True, alpha=alpha)
         _notify(w, b)
@@ -666,6 +690,8 @@ def _packed_wgrad(mod, dy, x, w, b, params, members=None):
                 # with the layer's other weight gradients in one grouped launch (27 of its 108 tiles: on its own
                 # this launch ran at 670 TFLOP/s, the group at 850)
                 _wgrad_group.add_tensors(dy2, x, dw, db, list(members))
+            elif _GROUP_QKV and _wgrad_rows.gathers(dy2, dw.shape, members):
+                _wgrad_rows.add_tensors(dy2, x, dw, db, list(members))
             else:
                 ops.linear_wgrad(dy, x, dw, db, accumulate=True)
                 _notify(*members)

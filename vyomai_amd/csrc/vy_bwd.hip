@@ -55,7 +55,9 @@ __device__ __forceinline__ bf16x8 tr_pair(const char* base, int row_bytes) {
 // columns: the source-side swizzle gets a second bit ((row >> 2) & 1) << 5 that puts them in the two 32-byte halves of a
 // 64-byte slot (conflict-free).  The atomic epilogue exchanges lane halves of two neighbouring k blocks
 // (v_permlane32_swap) so that a wave instruction is again two 128-byte row segments.
-template <int BN, int BKW, int MS, int NS, bool MF16 = false>
+// FOLD: all rows in one workgroup, but summed up in slices of m_chunk rows (a multiple of MS), the slices' sums added up in their order:
+// one of the orders in which the atomics of workgroups of a slice each arrive (wgrad_tn_bf16_rows_kernel).
+template <int BN, int BKW, int MS, int NS, bool MF16 = false, bool FOLD = false>
 __device__ __forceinline__ void wgrad_tn_bf16_body(
     const bf16* __restrict__ dY, int64_t lddy, const bf16* __restrict__ X, int64_t ldx,
     float* __restrict__ dW, int64_t lddw, float* __restrict__ db, const float* __restrict__ alpha_dev,
@@ -75,8 +77,8 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
   const int wn = wave >> 1, wk = wave & 1;
   const int tile_n = t2 / tiles_k, tile_k = t2 - tile_n * tiles_k;
   const int n0 = tile_n * BN, k0 = tile_k * BKW;
-  const int m_begin = split * m_chunk;
-  const int m_end = min(M, m_begin + m_chunk);
+  const int m_begin = FOLD ? 0 : split * m_chunk;
+  const int m_end = FOLD ? M : min(M, m_begin + m_chunk);
   if (m_begin >= m_end) return;
   const int nst = (m_end - m_begin + MS - 1) / MS;
 
@@ -275,6 +277,17 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
   typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2_t;
   const bf16x2_t ones2 = {(__bf16)1.0f, (__bf16)1.0f};
   float sdb[2] = {0.f, 0.f};
+  f32x16 total[FOLD ? 2 : 1][FOLD ? TJ : 1];   // of the slices that are done
+  float tdb[2] = {0.f, 0.f};
+  int left = m_chunk / MS;                     // stages of this slice
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) total[i][j][r] = 0.f;
+  }
 
   const int li = lane & 15, g16 = (lane >> 4) & 1, fh = lane >> 5;
   const int tr_row = 4 * fh + (li >> 2);                  // + 16*s (second read +8)
@@ -369,6 +382,26 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
       }
     };
     vy_static_for<KS>(kstep);
+    if constexpr (FOLD) {
+      if (--left == 0 || s == nst - 1) {
+        left = m_chunk / MS;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+#pragma unroll
+          for (int j = 0; j < TJ; ++j)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) { total[i][j][r] += acc[i][j][r]; acc[i][j][r] = 0.f; }
+          tdb[i] += sdb[i] + __shfl_xor(sdb[i], 32, 64);
+          sdb[i] = 0.f;
+        }
+      }
+    }
+  }
+  if constexpr (FOLD) {
+#pragma unroll
+    for (int i = 0; i < 2; ++i)
+#pragma unroll
+      for (int j = 0; j < TJ; ++j) acc[i][j] = total[i][j];
   }
   const int fr = lane & 31;
   if (diag == 1) {  // timing-only: no atomic epilogue (results wrong)
@@ -379,7 +412,7 @@ __device__ __forceinline__ void wgrad_tn_bf16_body(
   if (do_db) {
 #pragma unroll
     for (int i = 0; i < 2; ++i) {
-      const float t_ = (sdb[i] + __shfl_xor(sdb[i], 32, 64)) * alpha;
+      const float t_ = (FOLD ? tdb[i] : sdb[i] + __shfl_xor(sdb[i], 32, 64)) * alpha;
       const int n = n0 + wn * 64 + 32 * i + fr;
       if (fh == 0 && n < N) atomicAdd(db + n, t_);
     }
@@ -449,6 +482,28 @@ __global__ __launch_bounds__(BN * 2, 1) void wgrad_tn_bf16_grouped_kernel(WgradG
     if (d == i) it = grp.g[i];
   wgrad_tn_bf16_body<BN, BKW, MS, NS, MF16>(it.dY, it.lddy, it.X, it.ldx, it.dW, it.lddw, it.db, nullptr, it.M, it.N, it.K,
                                       it.tiles_k, it.m_chunk, diag, (id - it.item0) / it.tiles_nk, (id - it.item0) % it.tiles_nk);
+}
+
+// The weight gradients of several layers over few rows (vy_linear_wgrad_rows): a workgroup a tile of 128 x 128, all rows.  One by one, a
+// launch has 36 to 144 tiles and fills the chip with slices of rows, up to 7 of them, whose fp32 atomics bound it (1.2 TB/s); with
+// four layers in a launch -- 1728 tiles, two on a CU -- an element is added to once, and the slices live on as the order of its sum, so the
+// bits stay.  The four gradients of a layer of width 768, one by one / here, us: 24 rows 37.6 / 23.9 (the atomics of one sum), 180 rows
+// 45.2 / 24.8, 512 rows 69.6 / 27.9, 1000 rows 97.9 / 35.2, 1665 rows 113 / 45.5, 2047 rows 121 / 50.2 (tiles of 256 x 128 50.5 at 1665 rows).
+struct WgradRowsItem {
+  const bf16* dY; const bf16* X; float* dW; float* db;
+  int lddy, ldx, lddw, M, N, K, m_chunk, item0;
+};
+constexpr int MOST_ROWS_WGRADS = 16;
+struct WgradRows { WgradRowsItem g[MOST_ROWS_WGRADS]; int n; };
+
+__global__ __launch_bounds__(256, 2) void wgrad_tn_bf16_rows_kernel(WgradRows grp) {
+  const int id = xcd_remap(blockIdx.x, gridDim.x);
+  WgradRowsItem it = grp.g[0];
+#pragma unroll
+  for (int i = 1; i < MOST_ROWS_WGRADS; ++i)
+    if (i < grp.n && id >= grp.g[i].item0) it = grp.g[i];
+  wgrad_tn_bf16_body<128, 128, 64, 2, false, true>(it.dY, it.lddy, it.X, it.ldx, it.dW, it.lddw, it.db, nullptr, it.M, it.N, it.K,
+                                                   (it.K + 127) / 128, it.m_chunk, 0, 0, id - it.item0);
 }
 
 // db[n] += sum_m dY[m,n]: block = 64 lanes x 8 columns, 256 rows per block
@@ -1061,6 +1116,13 @@ int wgrad_f32(const char* who, const void* dy, int64_t lddy, const void* x, int6
 
 }  // namespace
 
+// Rows of the slices that a gradient over M rows is summed up in, for the workgroups that `goal` asks for and so many tiles
+static int64_t wgrad_slice(int64_t M, int64_t tiles, int64_t goal) {
+  const int64_t most = vy_cdiv(M, 256), splits = vy_cdiv(goal, tiles);   // (a slice has 256 rows at least: 4 stages of 64)
+  return vy_cdiv(vy_cdiv(M, splits < 1 ? 1 : splits > most ? most : splits), 64) * 64;
+}
+constexpr int WGRAD_GOAL = 384;   // ~1.5 workgroups of 128 x 128 per CU
+
 extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int64_t ldx, float* dw,
                                int64_t lddw, float* db, float beta, const float* alpha_dev, int64_t M,
                                int64_t N, int64_t K, int dtype, void* stream) {
@@ -1100,13 +1162,9 @@ extern "C" int vy_linear_wgrad(const void* dy, int64_t lddy, const void* x, int6
   const int BNt = (var == 1 || big) ? 256 : 128, BKt = (var == 2 || var == 4 || big) ? 256 : 128;
   const int tiles_n = (int)vy_cdiv(N, BNt), tiles_k = (int)vy_cdiv(K, BKt);
   const int tiles = tiles_n * tiles_k;
-  int64_t splits = vy_cdiv(tgt > 0 ? tgt : (var == 1 ? 256 : (var == 5 ? 704 : 384)), tiles);  // ~1.5 workgroups per CU
-  if (big && tgt <= 0) splits = 256 / tiles;                 // at most one round of 256 workgroups
-  const int64_t max_splits = vy_cdiv(M, 256);                // >= 4 stages of 64 rows each
-  if (splits > max_splits) splits = max_splits;
-  if (splits < 1) splits = 1;
-  int64_t m_chunk = vy_cdiv(vy_cdiv(M, splits), 64) * 64;
-  splits = vy_cdiv(M, m_chunk);
+  // (256 x 256 tiles: at most one round of 256 workgroups)
+  const int64_t m_chunk = wgrad_slice(M, tiles, tgt > 0 ? tgt : var == 1 ? 256 : var == 5 ? 704 : big ? (int64_t)(256 / tiles) * tiles : WGRAD_GOAL);
+  const int64_t splits = vy_cdiv(M, m_chunk);
   static const int ns = [] { const char* e = getenv("VY_WGRAD_STAGES"); return e ? atoi(e) : 2; }();
   // 16 x 16 x 32 MFMAs: 3 % faster on the 256 x 256 tiles (vocabulary projection 1.62 -> 1.57 ms, +0.25 % on the training
   // step), 2-8 % SLOWER on the 128 x 128 tiles (these kernels are bound by the transposing LDS reads and the atomic
@@ -1201,6 +1259,34 @@ extern "C" int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, in
 
 extern "C" int vy_linear_wgrad_batch(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream) {
   return wgrad_together("vy_linear_wgrad_batch", descs, n, MOST_WGRADS, dtype, stream);
+}
+
+extern "C" int vy_linear_wgrad_rows(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream) {
+  const char* who = "vy_linear_wgrad_rows";
+  if (dtype != VY_BF16) VY_FAIL(VY_ERR_ARG, "%s: bad dtype %d", who, dtype);
+  if (!descs || n <= 0 || n > MOST_ROWS_WGRADS) VY_FAIL(VY_ERR_ARG, "%s: 1..%d descriptors", who, MOST_ROWS_WGRADS);
+  WgradRows grp;
+  grp.n = n;
+  int64_t items = 0;
+  for (int i = 0; i < n; ++i) {
+    const vy_wgrad_desc& d = descs[i];
+    if (!d.dy || !d.x || !d.dw || d.M <= 0 || d.N <= 0 || d.K <= 0) VY_FAIL(VY_ERR_ARG, "%s: descriptor %d: bad arguments", who, i);
+    if (d.K % 8 || d.lddy % 8 || d.ldx % 8 || d.lddy < vy_cdiv(d.N, 8) * 8 || (uintptr_t)d.dy % 16 || (uintptr_t)d.x % 16)
+      VY_FAIL(VY_ERR_ARG, "%s: descriptor %d: K and leading dimensions must be multiples of 8, operands 16-byte aligned", who, i);
+    if ((d.lddy | d.ldx | d.lddw | d.M | d.N | d.K) >> 31) VY_FAIL(VY_ERR_ARG, "%s: descriptor %d: sizes of 32 bits", who, i);
+    WgradRowsItem& it = grp.g[i];
+    it.dY = (const bf16*)d.dy; it.X = (const bf16*)d.x; it.dW = d.dw; it.db = d.db;
+    it.lddy = (int)d.lddy; it.ldx = (int)d.ldx; it.lddw = (int)d.lddw;
+    it.M = (int)d.M; it.N = (int)d.N; it.K = (int)d.K;
+    const int64_t tiles = vy_cdiv(d.N, 128) * vy_cdiv(d.K, 128);
+    it.m_chunk = (int)wgrad_slice(d.M, tiles, WGRAD_GOAL);
+    it.item0 = (int)items;
+    items += tiles;
+  }
+  for (int i = n; i < MOST_ROWS_WGRADS; ++i) grp.g[i] = grp.g[0];
+  hipLaunchKernelGGL(wgrad_tn_bf16_rows_kernel, dim3((unsigned)items), dim3(256), 0, (hipStream_t)stream, grp);
+  VY_CHECK_LAUNCH(who);
+  return VY_OK;
 }
 
 // ------------------------------------------------------------------------------------------

@@ -419,9 +419,17 @@ def linear_wgrad_grouped(items) -> None:
     """items: up to 12 tuples (dy, x, dw, db|None): dw += dy^T @ x, db += colsum(dy), ONE launch
     (vy_linear_wgrad_grouped, vy_linear_wgrad_batch).  The tensors must stay alive until the launch has been enqueued (they do:
     the caller holds them)."""
-    import ctypes as C
+    _wgrads("vy_linear_wgrad_grouped" if len(items) <= 8 else "vy_linear_wgrad_batch", 12, items)
+
+
+def linear_wgrad_rows(items) -> None:
+    """The same for up to 16 bf16 gradients over few rows, each with the sums of linear_wgrad (vy_linear_wgrad_rows)."""
+    _wgrads("vy_linear_wgrad_rows", 16, items)
+
+
+def _wgrads(entry: str, most: int, items) -> None:
     n = len(items)
-    assert 1 <= n <= 12
+    assert 1 <= n <= most
     arr = (_lib.VyWgradDesc * n)()
     dt, rows = None, []   # (rows: copies of operands without uniform rows live until the launch)
     for i, (dy, x, dw, db) in enumerate(items):
@@ -438,7 +446,7 @@ def linear_wgrad_grouped(items) -> None:
         a.dy, a.lddy, a.x, a.ldx = d2.data_ptr(), d2.stride(0), x2.data_ptr(), x2.stride(0)
         a.dw, a.lddw, a.db = dw.data_ptr(), dw.stride(0), _ptr(db)
         a.M, a.N, a.K = M, N, K
-    call("vy_linear_wgrad_grouped" if n <= 8 else "vy_linear_wgrad_batch", C.cast(arr, C.c_void_p), n, dtype_code(dt), _stream())
+    call(entry, C.cast(arr, C.c_void_p), n, dtype_code(dt), _stream())
 
 
 def layernorm_bwd(dy: Tensor, x: Tensor, gamma: Tensor, mean: Tensor, rstd: Tensor, dgamma: Tensor,
