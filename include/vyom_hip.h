@@ -179,7 +179,9 @@ int vy_text_layer_fwd(const vy_text_layer* l, const void* x, void* y, int64_t B,
  * the rows ahead of both norms s1 and s2, a and the inner rows, the activation's derivative; lse [B][h][L], a mean and a 1 / deviation per
  * row of both norms.  replaces: the autograd of the same modules.  vy_text_layer_bwd: dx from dy; the transposed weights [in][out] with
  * row strides ld_*; dln* are added to, dln*_w and dln*_b fp32 [h dh]; ds2, dpre, ds1 and dqkv [B][L][dq | dk | dv] are what the weight
- * gradients multiply with inner, a, o and x; da, dheads, ln_ws (2 vy_layernorm_bwd_ws_rows(B L) h dh fp32) and delta [B][h][L] are scratch. */
+ * gradients multiply with inner, a, o and x; da, dheads, ln_ws (2 vy_layernorm_bwd_ws_rows(B L) h dh fp32) and delta [B][h][L] are scratch.
+ * ln_ws1: NULL, or as much again: the partials of the first norm stay there, those of the second in ln_ws, for vy_layernorm_sums, and dln*
+ * are not touched. */
 typedef struct vy_text_layer_kept {
   void *q, *o, *s1, *a, *deriv, *inner, *s2;
   float *lse, *mean1, *rstd1, *mean2, *rstd2;
@@ -189,7 +191,7 @@ typedef struct vy_text_layer_grads {
   int64_t ld_qkv, ld_o, ld_1, ld_2;
   float *dln1_w, *dln1_b, *dln2_w, *dln2_b;
   void *ds2, *dpre, *da, *ds1, *dheads, *dqkv;
-  float *ln_ws, *delta;
+  float *ln_ws, *delta, *ln_ws1;
 } vy_text_layer_grads;
 int vy_text_layer_train_fwd(const vy_text_layer* l, const vy_text_layer_kept* t, const void* x, void* y, int64_t B, int64_t L, void* stream);
 int vy_text_layer_bwd(const vy_text_layer* l, const vy_text_layer_kept* t, const vy_text_layer_grads* g, const void* dy, void* dx, int64_t B,
@@ -451,12 +453,19 @@ int vy_linear_wgrad_rows(const vy_wgrad_desc* descs, int32_t n, int dtype, void*
 
 /* LayerNorm backward: dx = rstd*(g - mean(g) - xhat*mean(g*xhat)), g = dy*gamma;
  * dgamma/dbeta fp32 [N] accumulated (beta) from per-block partials in `ws`
- * (ws: fp32, at least 2 * ws_rows * N elements; ws_rows = vy_layernorm_bwd_ws_rows(M)). */
+ * (ws: fp32, at least 2 * ws_rows * N elements; ws_rows = vy_layernorm_bwd_ws_rows(M)).  With neither of them the partials
+ * stay in ws, for vy_layernorm_sums: the column sums of 1..16 norms' partials in one launch, added to dgamma and dbeta. */
 int64_t vy_layernorm_bwd_ws_rows(int64_t M);
 int vy_layernorm_bwd(const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* gamma,
                      const float* mean, const float* rstd, void* dx, int64_t lddx, float* dgamma,
                      float* dbeta, float beta, float* ws, int64_t M, int64_t N, int dtype,
                      void* stream);
+
+typedef struct vy_norm_sums {
+  const float* ws; float* dgamma; float* dbeta;
+  int32_t rows, N;      /* rows: vy_layernorm_bwd_ws_rows of the norm's rows */
+} vy_norm_sums;
+int vy_layernorm_sums(const vy_norm_sums* descs, int32_t n, void* stream);
 
 /* Flash attention backward.  dO/O are (B,L,h*dh) (strides {sb,sl}); dq/dk/dv use q/k/v layouts.
  * delta_ws: fp32 [B,h,L] scratch.  dk/dv are (B,hk,S,dh): the n_rep query heads of one kv head

@@ -48,6 +48,7 @@ PROTOTYPES = {
     "vy_linear_wgrad_grouped": [_p, _i, _i, _p],
     "vy_linear_wgrad_batch": [_p, _i, _i, _p],
     "vy_linear_wgrad_rows": [_p, _i, _i, _p],
+    "vy_layernorm_sums": [_p, _i, _p],
     "vy_layernorm_bwd": [_p, _i64, _p, _i64, _p, _p, _p, _p, _i64, _p, _p, _f, _p, _i64, _i64, _i, _p],
     "vy_attn_bwd": [_p, _i64, _i64, _i64, _p, _i64, _i64, _i64, _p, _i64, _i64, _i64,
                     _p, _p, _i64, _i64, _p, _p,
@@ -166,7 +167,13 @@ class VyTextLayerKept(C.Structure):
 class VyTextLayerGrads(C.Structure):
     """vy_text_layer_grads (include/vyom_hip.h)"""
     _fields_ = [(n, _p) for n in ("wt_qkv", "wt_o", "wt_1", "wt_2")] + [(n, _i64) for n in ("ld_qkv", "ld_o", "ld_1", "ld_2")] + \
-               [(n, _p) for n in ("dln1_w", "dln1_b", "dln2_w", "dln2_b", "ds2", "dpre", "da", "ds1", "dheads", "dqkv", "ln_ws", "delta")]
+               [(n, _p) for n in ("dln1_w", "dln1_b", "dln2_w", "dln2_b", "ds2", "dpre", "da", "ds1", "dheads", "dqkv", "ln_ws", "delta",
+                                "ln_ws1")]
+
+
+class VyNormSums(C.Structure):
+    """vy_norm_sums (include/vyom_hip.h)"""
+    _fields_ = [(n, _p) for n in ("ws", "dgamma", "dbeta")] + [(n, C.c_int32) for n in ("rows", "N")]
 
 
 _lib: Optional[C.CDLL] = None

@@ -178,9 +178,13 @@ class _WgradGroup:
         exchanged = any(getattr(p, "_vy_exchanged", False) for p in members)
         if self.tiles + tiles > self.TILES and not exchanged:
             self.flush()
+        self._hold((dy, x, dw, db, members), tiles, key, exchanged)
+
+    def _hold(self, item, tiles, key, exchanged) -> None:
+        members = item[4]
         if not self.items:
-            self.key, self.stream = key, torch.cuda.current_stream() if dy is not None and dy.is_cuda else None
-        self.items.append((dy, x, dw, db, members))
+            self.key, self.stream = key, torch.cuda.current_stream() if item[0] is not None and item[0].is_cuda else None
+        self.items.append(item)
         # autograd's own post-accumulate hook fires for these parameters as soon as this backward function
         # returns -- the reducer must not take that for "gradient written" (training.BucketReducer._hook)
         for p in members:
@@ -200,7 +204,9 @@ class _WgradGroup:
         items, self.items, self.tiles = self.items, [], 0
         if not items:
             return
-        self._launch([(dy, x, dw, db) for dy, x, dw, db, _ in items])
+        self._launch([item[:4] for item in items])
+        if _norm_sums.items and _norm_sums.key[1] == ops._raw_stream():   # (so that whole buckets of parameters are ready)
+            _norm_sums.flush()
         for *_, members in items:
             for p in members:
                 p._vy_deferred = False
@@ -245,6 +251,28 @@ class _WgradRows(_WgradGroup):
         ops.linear_wgrad_rows(items)
 
 
+class _NormSums(_WgradGroup):
+    """Column sums of the gradients of norms, whose partials lie in buffers of their own: they go out with the weight gradients of their
+    layers, up to sixteen in a launch (ops.layernorm_sums); exchanged ones, and those on another stream than others that wait, at once."""
+
+    MOST = 16
+
+    def add_norms(self, norms) -> None:
+        """norms: (ws, rows, weight, bias) each."""
+        items = [(ws, rows, w.grad, b.grad, (w, b)) for ws, rows, w, b in norms]
+        key = (torch.float32, ops._raw_stream())
+        if (self.items and key != self.key) or any(getattr(p, "_vy_exchanged", False) for item in items for p in item[4]):
+            self._launch([item[:4] for item in items])
+            for item in items:
+                _notify(*item[4])
+            return
+        for item in items:
+            self._hold(item, 0, key, False)
+
+    def _launch(self, items) -> None:
+        ops.layernorm_sums(items)
+
+
 _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
 _GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 121 us one by one,
@@ -254,6 +282,7 @@ _GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 ro
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group
 _wgrad_group = _WgradGroup()
 _wgrad_rows = _WgradRows()
+_norm_sums = _NormSums()
 
 
 def _wgrad(dy, x, w: torch.Tensor, b: Optional[torch.Tensor], alpha: Optional[torch.Tensor] = None):
@@ -576,20 +605,28 @@ class TextLayerFn(torch.autograd.Function):
         work = torch.empty(n, dtype=dt, device=dev)
         oo, on = _segments(M * d, M * d)                       # da, dheads
         own = torch.empty(on, dtype=dt, device=dev)
-        fo, fn = _segments(2 * _lib.load().vy_layernorm_bwd_ws_rows(M) * d, B * h * L)
+        slabs = _lib.load().vy_layernorm_bwd_ws_rows(M)
+        wait = _GROUP_WGRADS and all(_direct(p) for p in (g1, b1, g2, b2))     # the norms' column sums go out with other layers'
+        fo, fn = _segments(B * h * L, 0 if wait else 2 * slabs * d)
         scratch = torch.empty(fn, dtype=torch.float32, device=dev)
+        sums = torch.empty((2, 2 * slabs * d), dtype=torch.float32, device=dev) if wait else None
         dx = torch.empty_like(x)
         e, f0 = x.element_size(), scratch.data_ptr()
         ds2, dpre, ds1, dqkv = (work.data_ptr() + o * e for o in to)
         da, dheads = (own.data_ptr() + o * e for o in oo)
         # (a gradient that has left the arena since the forward pass is returned)
-        dln = [p.grad if _direct(p) else torch.zeros(d, dtype=torch.float32, device=dev) for p in (g1, b1, g2, b2)]
-        grads = _lib.VyTextLayerGrads(*(t.data_ptr() for t in wt), *(t.stride(0) for t in wt), *(t.data_ptr() for t in dln), ds2, dpre, da, ds1,
-                                      dheads, dqkv, *(f0 + 4 * o for o in fo))
+        dln = [] if wait else [p.grad if _direct(p) else torch.zeros(d, dtype=torch.float32, device=dev) for p in (g1, b1, g2, b2)]
+        at = sums.data_ptr() if wait else f0 + 4 * fo[1]
+        grads = _lib.VyTextLayerGrads(*(t.data_ptr() for t in wt), *(t.stride(0) for t in wt), *((None,) * 4 if wait else (t.data_ptr() for t in dln)),
+                                      ds2, dpre, da, ds1, dheads, dqkv, at, f0 + 4 * fo[0], at + 8 * slabs * d if wait else None)
         ops._mid_ws(M)
         _lib.call("vy_text_layer_bwd", _ref(desc), _ref(kept), _ref(grads), dy.data_ptr(), dx.data_ptr(), B, L, ops._stream())
-        dg1, db1, dg2, db2 = (None if _direct(p) else t.to(p.dtype) for p, t in zip((g1, b1, g2, b2), dln))
-        _notify(*(p for p in (g2, b2, g1, b1) if _direct(p)))
+        if wait:
+            dg1 = db1 = dg2 = db2 = None
+            _norm_sums.add_norms([(sums[0], slabs, g2, b2), (sums[1], slabs, g1, b1)])
+        else:
+            dg1, db1, dg2, db2 = (None if _direct(p) else t.to(p.dtype) for p, t in zip((g1, b1, g2, b2), dln))
+            _notify(*(p for p in (g2, b2, g1, b1) if _direct(p)))
 
         def of(t, o, cols):
             return t.as_strided((M, cols), (cols, 1), t.storage_offset() + o)

@@ -82,20 +82,22 @@ extern "C" int vy_text_layer_bwd(const vy_text_layer* l, const vy_text_layer_kep
                                  int64_t B, int64_t L, void* stream) {
   const char* who = "vy_text_layer_bwd";
   if (int rc = kept_layer(who, l, t, B, L)) return rc;
-  if (!g || !dy || !dx || !g->wt_qkv || !g->wt_o || !g->wt_1 || !g->wt_2 || !g->dln1_w || !g->dln1_b || !g->dln2_w || !g->dln2_b || !g->ds2 ||
-      !g->dpre || !g->da || !g->ds1 || !g->dheads || !g->dqkv || !g->ln_ws || !g->delta)
+  if (!g || !dy || !dx || !g->wt_qkv || !g->wt_o || !g->wt_1 || !g->wt_2 || (!g->ln_ws1 && (!g->dln1_w || !g->dln1_b || !g->dln2_w || !g->dln2_b)) ||
+      !g->ds2 || !g->dpre || !g->da || !g->ds1 || !g->dheads || !g->dqkv || !g->ln_ws || !g->delta)
     VY_FAIL(VY_ERR_ARG, "%s: null tensor", who);
   const int64_t d = (int64_t)l->h * l->dh, kv = (int64_t)l->hk * l->dh, W = d + 2 * kv, M = B * L, e = l->dtype == VY_BF16 ? 2 : 4, dh = l->dh;
   const float scale = (float)(1.0 / sqrt((double)l->dh));
   char *dq = (char*)g->dqkv, *dk = dq + d * e, *dv = dk + kv * e;
+  const bool later = g->ln_ws1 != nullptr;   // the norms' column sums, with other layers'
+  float *ln1_w = later ? nullptr : g->dln1_w, *ln1_b = later ? nullptr : g->dln1_b, *ln2_w = later ? nullptr : g->dln2_w, *ln2_b = later ? nullptr : g->dln2_b;
   int rc;
-  if ((rc = vy_layernorm_bwd(dy, d, t->s2, d, l->ln2_w, t->mean2, t->rstd2, g->ds2, d, g->dln2_w, g->dln2_b, 1.f, g->ln_ws, M, d, l->dtype, stream))) return rc;
+  if ((rc = vy_layernorm_bwd(dy, d, t->s2, d, l->ln2_w, t->mean2, t->rstd2, g->ds2, d, ln2_w, ln2_b, 1.f, g->ln_ws, M, d, l->dtype, stream))) return rc;
   if ((rc = vy_linear_dgrad(g->ds2, d, g->wt_2, g->ld_2, t->deriv, l->ffn, l->act | VY_ACT_SAVE_DERIV, nullptr, 0, nullptr, 0, g->dpre, l->ffn, M, d,
                             l->ffn, l->dtype, stream)))
     return rc;
   if ((rc = vy_linear_dgrad(g->dpre, l->ffn, g->wt_1, g->ld_1, nullptr, 0, VY_ACT_NONE, nullptr, 0, nullptr, 0, g->da, d, M, l->ffn, d, l->dtype, stream)))
     return rc;
-  if ((rc = vy_layernorm_bwd(g->da, d, t->s1, d, l->ln1_w, t->mean1, t->rstd1, g->ds1, d, g->dln1_w, g->dln1_b, 1.f, g->ln_ws, M, d, l->dtype, stream)))
+  if ((rc = vy_layernorm_bwd(g->da, d, t->s1, d, l->ln1_w, t->mean1, t->rstd1, g->ds1, d, ln1_w, ln1_b, 1.f, later ? g->ln_ws1 : g->ln_ws, M, d, l->dtype, stream)))
     return rc;
   if ((rc = vy_linear_dgrad(g->ds1, d, g->wt_o, g->ld_o, nullptr, 0, VY_ACT_NONE, nullptr, 0, nullptr, 0, g->dheads, d, M, d, d, l->dtype, stream))) return rc;
   if ((rc = vy_attn_bwd(t->q, L * d, L * dh, dh, l->k, l->k_sb, l->k_sh, l->k_sl, l->v, l->v_sb, l->v_sh, l->v_sl, t->o, g->dheads, L * d, d, t->lse,

@@ -249,16 +249,22 @@ __global__ __launch_bounds__(256) void layernorm_bwd_kernel(
   }
 }
 
-// column sums of the [W, N] partial slabs, accumulated into out0/out1 (zeroed by the launcher
-// when beta == 0): grid = (column blocks of 64) x (row slices), 4 row groups per block reduced
-// through LDS, one fp32 atomic per column per block
-__global__ __launch_bounds__(256) void colsum_partials_kernel(const float* __restrict__ ws, int W, int N,
-                                                              float* __restrict__ out0, float* __restrict__ out1,
-                                                              int rows_per_slice) {
+// Column sums of the [rows, N] partial slabs of one or several norms (one launch of 5 to 10 us for each of them was 1 % of a training step of
+// 32 x 512 tokens and 2 % of shorter ones: a few MB, all latency), added to out0 / out1 (zeroed by the launcher when beta == 0):
+// grid = (column blocks of 64) x (row slices) x (norms), 4 row groups per block reduced through LDS, one fp32 atomic per column per block
+struct ColsumItem { const float* ws; float* out0; float* out1; int rows, N; };
+constexpr int MOST_COLSUMS = 16;
+struct Colsums { ColsumItem g[MOST_COLSUMS]; };
+
+__global__ __launch_bounds__(256) void colsum_partials_kernel(Colsums all) {
   __shared__ float red[2][4][64];
+  const ColsumItem it = all.g[blockIdx.z];
+  const float* __restrict__ ws = it.ws;
+  const int N = it.N, W = it.rows, slice = W >= 64 ? (W + 15) / 16 : W;
   const int c = threadIdx.x & 63, g = threadIdx.x >> 6;
   const int n = blockIdx.x * 64 + c;
-  const int w0 = blockIdx.y * rows_per_slice, w1 = min(W, w0 + rows_per_slice);
+  const int w0 = blockIdx.y * slice, w1 = min(W, w0 + slice);
+  if (w0 >= W || (int)blockIdx.x * 64 >= N) return;
   float a = 0.f, b = 0.f;
   if (n < N) {
     // eight rows of both slabs requested at once (one round trip for the usual 32-row slice; a loop of dependent
@@ -282,8 +288,8 @@ __global__ __launch_bounds__(256) void colsum_partials_kernel(const float* __res
   if (g == 0 && n < N) {
     a = red[0][0][c] + red[0][1][c] + red[0][2][c] + red[0][3][c];
     b = red[1][0][c] + red[1][1][c] + red[1][2][c] + red[1][3][c];
-    if (out0) atomicAdd(out0 + n, a);
-    if (out1) atomicAdd(out1 + n, b);
+    if (it.out0) atomicAdd(it.out0 + n, a);
+    if (it.out1) atomicAdd(it.out1 + n, b);
   }
 }
 
@@ -701,16 +707,16 @@ int ln_bwd_dispatch(const void* dy, int64_t lddy, const void* x, int64_t ldx, co
   else VY_FAIL(VY_ERR_UNSUPPORTED, "vy_layernorm_bwd: N=%ld too wide", (long)N);
 #undef LN_GO
   VY_CHECK_LAUNCH("vy_layernorm_bwd");
+  if (!dgamma && !dbeta) return VY_OK;   // (the partial sums stay in ws: vy_layernorm_sums)
   if (beta == 0.f) {
     if (dgamma && hipMemsetAsync(dgamma, 0, N * sizeof(float), st) != hipSuccess) VY_FAIL(VY_ERR_LAUNCH, "vy_layernorm_bwd: memset failed");
     if (dbeta && hipMemsetAsync(dbeta, 0, N * sizeof(float), st) != hipSuccess) VY_FAIL(VY_ERR_LAUNCH, "vy_layernorm_bwd: memset failed");
   } else if (beta != 1.f) {
     VY_FAIL(VY_ERR_ARG, "vy_layernorm_bwd: beta must be 0 or 1");
   }
-  const int slices = WB >= 64 ? 16 : 1;
-  const int rps = (int)vy_cdiv(WB, slices);
-  hipLaunchKernelGGL(colsum_partials_kernel, dim3((unsigned)vy_cdiv(N, 64), (unsigned)slices), dim3(256), 0, st, ws, WB,
-                     (int)N, dgamma, dbeta, rps);
+  Colsums one{};
+  one.g[0] = {ws, dgamma, dbeta, WB, (int)N};
+  hipLaunchKernelGGL(colsum_partials_kernel, dim3((unsigned)vy_cdiv(N, 64), WB >= 64 ? 16 : 1), dim3(256), 0, st, one);
   VY_CHECK_LAUNCH("vy_layernorm_bwd(colsum)");
   return VY_OK;
 }
@@ -779,6 +785,22 @@ extern "C" int64_t vy_layernorm_bwd_ws_rows(int64_t M) {
   static const int64_t cap = [] { const char* e = getenv("VY_LNBWD_WB"); return e ? (int64_t)atoi(e) : (int64_t)512; }();   // measured at M = 16384, N = 768: 256: 27.8 us, 512: 24.3, 1024: 27.6, 2048: 36.3
   const int64_t b = (M + 3) / 4;  // one wave per row at least
   return b < 1 ? 1 : (b > cap ? cap : b);
+}
+
+extern "C" int vy_layernorm_sums(const vy_norm_sums* descs, int32_t n, void* stream) {
+  if (!descs || n <= 0 || n > MOST_COLSUMS) VY_FAIL(VY_ERR_ARG, "vy_layernorm_sums: 1..%d descriptors", MOST_COLSUMS);
+  Colsums all{};
+  int64_t columns = 0, slices = 1;
+  for (int i = 0; i < n; ++i) {
+    const vy_norm_sums& d = descs[i];
+    if (!d.ws || !d.dgamma || !d.dbeta || d.rows <= 0 || d.N <= 0) VY_FAIL(VY_ERR_ARG, "vy_layernorm_sums: descriptor %d: bad arguments", i);
+    all.g[i] = {d.ws, d.dgamma, d.dbeta, d.rows, d.N};
+    if (d.N > columns) columns = d.N;
+    if (d.rows >= 64) slices = 16;
+  }
+  hipLaunchKernelGGL(colsum_partials_kernel, dim3((unsigned)vy_cdiv(columns, 64), (unsigned)slices, (unsigned)n), dim3(256), 0, (hipStream_t)stream, all);
+  VY_CHECK_LAUNCH("vy_layernorm_sums");
+  return VY_OK;
 }
 
 extern "C" int vy_layernorm_bwd(const void* dy, int64_t lddy, const void* x, int64_t ldx, const void* gamma,

@@ -463,6 +463,18 @@ def layernorm_bwd(dy: Tensor, x: Tensor, gamma: Tensor, mean: Tensor, rstd: Tens
     return dx.view(x.shape)
 
 
+def layernorm_sums(items) -> None:
+    """items: up to 16 tuples (ws, rows, dgamma, dbeta): the column sums of the partials that a norm's backward pass left in ws, added to
+    dgamma and dbeta, ONE launch (vy_layernorm_sums)."""
+    arr = (_lib.VyNormSums * len(items))()
+    for a, (ws, rows, dg, db) in zip(arr, items):
+        _need_gpu(ws, dg, db)
+        assert ws.is_contiguous() and ws.numel() >= 2 * rows * dg.numel() and dg.numel() == db.numel()
+        assert ws.dtype == dg.dtype == db.dtype == torch.float32 and dg.is_contiguous() and db.is_contiguous()
+        a.ws, a.rows, a.dgamma, a.dbeta, a.N = ws.data_ptr(), rows, dg.data_ptr(), db.data_ptr(), dg.numel()
+    call("vy_layernorm_sums", C.cast(arr, C.c_void_p), len(items), _stream())
+
+
 def attention_bwd(q, k, v, out, dout, lse, dq, dk, dv, *, causal: bool, start_pos: int = 0,
                   keypad: Optional[Tensor] = None, scale: Optional[float] = None,
                   cos: Optional[Tensor] = None, sin: Optional[Tensor] = None, rope_pos0: int = 0) -> None:
