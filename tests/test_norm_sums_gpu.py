@@ -51,7 +51,7 @@ def test_when_sums_go_out(monkeypatch):
     from vyomai_amd import autograd_train as AT
     out, ready, stream = [], [], [1]
     monkeypatch.setattr(AT.ops, "layernorm_sums", lambda items: out.append(len(items)))
-    monkeypatch.setattr(AT.ops, "linear_wgrad_rows", lambda items: None)
+    monkeypatch.setattr(AT.ops, "wgrad_rows", lambda descs: None)
     monkeypatch.setattr(AT.ops, "_raw_stream", lambda: stream[0])
     sums, rows = AT._NormSums(), AT._WgradRows()
     monkeypatch.setattr(AT, "_norm_sums", sums)
@@ -61,17 +61,17 @@ def test_when_sums_go_out(monkeypatch):
         ps = [torch.nn.Parameter(torch.zeros(4)) for _ in range(2)]
         for p in ps:
             p.grad, p._vy_ready, p._vy_exchanged = torch.zeros(4), ready.append, exchanged
-        return (torch.empty(8), 1, *ps)
+        return (torch.empty(8), 1, ps[0].grad, ps[1].grad, ps)
     sums.add_norms([norm(), norm()])
     assert not out and not ready and all(p._vy_deferred for item in sums.items for p in item[4])
     stream[0] = 2
     sums.add_norms([norm()])
     assert out == [1] and len(ready) == 2
-    rows.add_tensors(torch.empty(4, 512, dtype=BF), None, torch.empty(512, 512, device="meta"), None, [])
+    rows.add_descs([(None, [])], (torch.empty(4, dtype=BF),))
     rows.flush()                    # (of the other stream)
     assert out == [1]
     stream[0] = 1
-    rows.add_tensors(torch.empty(4, 512, dtype=BF), None, torch.empty(512, 512, device="meta"), None, [])
+    rows.add_descs([(None, [])], (torch.empty(4, dtype=BF),))
     rows.flush()
     assert out == [1, 2] and len(ready) == 6 and not any(p._vy_deferred for p in ready if hasattr(p, "_vy_deferred"))
     sums.add_norms([norm(True), norm(True)])

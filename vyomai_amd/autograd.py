@@ -223,11 +223,11 @@ def layer_train(att, ff, x, mask, freqs):
     a call of its module sees."""
     if not torch.is_grad_enabled() or not _plain_layer(att, ff, x, mask) or _backward_hooks(att, ff):
         return None
-    from .autograd_train import TextLayerFn, _direct
+    from .autograd_train import TextLayerFn
     members = att._params()
-    params = [*_layer_params(att, ff), *members]
+    params = _layer_params(att, ff) + members
     for p in params:
-        if p is not None and not (p.requires_grad and _direct(p)):
+        if p is not None and not (getattr(p, "_vy_direct", False) and p.requires_grad and p.grad is not None):
             return None
     if params[1] is None or params[3] is None or params[7] is None or params[9] is None:   # (biases of norms and projections)
         return None

@@ -13,8 +13,9 @@ Gradient delivery has two modes per parameter:
 from __future__ import annotations
 
 import ctypes
+import functools
+import itertools
 import os
-
 import weakref
 from typing import Optional
 
@@ -30,73 +31,77 @@ BF16 = torch.bfloat16
 _ref = ctypes.addressof
 
 
-# bumped by FlatTrainer.step(): its AdamW kernel rewrites weights without touching tensor versions
-WEIGHT_EPOCH = [0]
+_EPOCHS = itertools.count()
 
 
 class _WtRegistry:
-    """Every W^T the dgrad GEMMs read.  The first backward transposes each matrix as it meets it; from
-    then on ONE vy_transpose_batched launch per weight epoch refreshes all that were used in the
-    previous epoch (the per-matrix launches are latency-bound: ~8 us each, 50 per step).  Owners are
-    held weakly: a model that is dropped, or no longer trained, falls out of the batch."""
+    """Every W^T the dgrad GEMMs read, of the parameters of one trainer (and one registry for parameters without).  The first backward
+    transposes each matrix as it meets it; from then on ONE vy_transpose_batched launch per weight epoch refreshes all that were used
+    in the previous epoch (the per-matrix launches are latency-bound: ~8 us each, 50 per step).  An epoch ends with a step of
+    the trainer, whose AdamW kernel rewrites weights without touching tensor versions; its number is used once in a process.  Models that
+    are trained in turn have an epoch each: one for all had the other models' matrices transposed at every step, and this one's
+    one by one.  Owners are held weakly: a model that is dropped, or no longer trained, falls out of the batch."""
 
     def __init__(self) -> None:
-        self.entries = []      # [weakref(owner), key_fn, src_fn, dst_view, last_used_epoch]
+        self.entries = []      # [weakref(owner), key_fn, src_fn, dst_view, last_used_epoch, number of the registry]
         self.batches = {}
-        self.epoch_done = -1
+        self.number = self.epoch = next(_EPOCHS)
+        self.before = self.epoch_done = -1
+
+    def bump(self) -> None:
+        self.before, self.epoch = self.epoch, next(_EPOCHS)
 
     def register(self, owner, key_fn, src_fn, dst):
-        e = [weakref.ref(owner), key_fn, src_fn, dst, WEIGHT_EPOCH[0]]
+        e = [weakref.ref(owner), key_fn, src_fn, dst, self.epoch, self.number]
         self.entries.append(e)
         return e
 
     def refresh(self) -> None:
-        """Re-transpose the recently used matrices for the current WEIGHT_EPOCH (once per epoch)."""
-        ep = WEIGHT_EPOCH[0]
+        """Re-transpose the recently used matrices for the current epoch (once per epoch)."""
+        ep = self.epoch
         if self.epoch_done == ep:
             return
         self.epoch_done = ep
-        entries, live = [], []
+        entries, live = [], {}
         for e in self.entries:
             owner = e[0]()
-            if owner is None:
+            if owner is None or owner._vy_wt_entry is not e:
                 continue
             entries.append(e)
-            if e[4] >= ep - 1:
-                key = e[1](owner)
-                if getattr(owner, "_vy_wt_key", None) != key:
-                    live.append((owner, key, e[2](owner), e[3]))
+            if e[4] == ep or e[4] == self.before:
+                key, members = e[1](owner)
+                if owner._vy_wt_key != key:
+                    src = e[2](owner, members)
+                    live.setdefault(src.dtype, []).append((owner, key, src, e[3]))
         self.entries = entries
-        if not live:
-            return
-        # one launch per dtype (a bf16 model and an fp32 one trained in the same process share this registry)
-        for dt in sorted({src.dtype for _, _, src, _ in live}, key=str):
-            sub = [(src, dst) for _, _, src, dst in live if src.dtype == dt]
-            keys = [(s_.data_ptr(), d_.data_ptr()) for s_, d_ in sub]
+        # one launch per dtype (a bf16 model and an fp32 one that no trainer owns share a registry)
+        for dt, sub in live.items():
+            keys = [(src.data_ptr(), dst.data_ptr()) for _, _, src, dst in sub]
             batch = self.batches.get(dt)
             if batch is None or batch.keys != keys:
-                batch = self.batches[dt] = ops.TransposeBatch(sub)
+                batch = self.batches[dt] = ops.TransposeBatch([(src, dst) for _, _, src, dst in sub])
             batch.run()
-        for owner, key, *_ in live:
-            owner._vy_wt_key = key
+            for owner, key, *_ in sub:
+                owner._vy_wt_key = key
 
 
 _WT = _WtRegistry()
 
 
-def _wt_cached(owner, key_fn, src_fn) -> torch.Tensor:
+def _wt_cached(owner, reg: _WtRegistry, key, key_fn, src_fn, members=None) -> torch.Tensor:
     """Shared body of _wt / _wt_packed: owner carries _vy_wt_key / _vy_wt_view / _vy_wt_entry.
-    key_fn / src_fn take the owner as their argument (the registry must not keep it alive)."""
+    key_fn / src_fn take the owner as their argument (the registry must not keep it alive); key, members: what key_fn returns now."""
     view = getattr(owner, "_vy_wt_view", None)
-    key = key_fn(owner)
-    entry = getattr(owner, "_vy_wt_entry", None)
-    if entry is not None:
-        entry[4] = WEIGHT_EPOCH[0]
-    if view is not None and getattr(owner, "_vy_wt_key", None) == key:
-        return view
-    src = src_fn(owner)
+    if view is not None:
+        entry = owner._vy_wt_entry
+        if entry[5] != reg.number or entry[0]() is not owner:      # (the parameter has gone over to another trainer; a copy of a module)
+            entry = owner._vy_wt_entry = reg.register(owner, key_fn, src_fn, view)
+        entry[4] = reg.epoch
+        if owner._vy_wt_key == key:
+            return view
+    src = src_fn(owner, members)
     if view is not None and view.dtype == src.dtype and view.device == src.device:
-        _WT.refresh()   # weights changed: all recently used matrices in one launch
+        reg.refresh()   # weights changed: all recently used matrices in one launch
         if owner._vy_wt_key != key:
             ops.transpose(src, view)   # not in the batch (first use after a pause, or an in-place edit)
             owner._vy_wt_key = key
@@ -106,7 +111,7 @@ def _wt_cached(owner, key_fn, src_fn) -> torch.Tensor:
     view = torch.zeros((K, ld), dtype=src.dtype, device=src.device)[:, :N]  # pad columns stay zero
     ops.transpose(src, view)
     owner._vy_wt_view, owner._vy_wt_key = view, key
-    owner._vy_wt_entry = _WT.register(owner, key_fn, src_fn, view)
+    owner._vy_wt_entry = reg.register(owner, key_fn, src_fn, view)
     return view
 
 
@@ -124,7 +129,9 @@ def _row_stride(n: int) -> int:
 
 def _wt(param: torch.Tensor, dtype) -> torch.Tensor:
     """W^T ([K, N], row stride padded to 8) of a 2-D parameter in `dtype`, cached per version."""
-    return _wt_cached(param, lambda p: (p._version, WEIGHT_EPOCH[0], dtype), lambda p: _shadow(p, dtype))
+    reg = getattr(param, "_vy_weights", _WT)
+    return _wt_cached(param, reg, (param._version, reg.epoch, dtype), lambda p: ((p._version, getattr(p, "_vy_weights", _WT).epoch, dtype), None),
+                      lambda p, _: _shadow(p, dtype))
 
 
 def _direct(p: Optional[torch.Tensor]) -> bool:
@@ -236,19 +243,37 @@ class _WgradGroup:
 
 class _WgradRows(_WgradGroup):
     """The same for gradients over fewer rows than those: four layers' in a launch that sums each up as a launch of its own does
-    (ops.linear_wgrad_rows), so they keep their bits.  Exchanged gradients go out one by one."""
+    (ops.wgrad_rows), so they keep their bits.  Exchanged gradients go out one by one."""
 
-    TILES, MOST = 1 << 30, 16
+    MOST = 16
 
     def gathers(self, dy, shape, members, alpha=None) -> bool:
-        if alpha is not None or not _GROUP_WGRADS or dy.dtype != torch.bfloat16:
+        if alpha is not None or dy.dtype != torch.bfloat16 or any(getattr(p, "_vy_exchanged", False) for p in members):
             return False
-        N, K = shape
-        return (dy.numel() // N < _GROUP_MIN_ROWS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0
-                and not any(getattr(p, "_vy_exchanged", False) for p in members))
+        return _few_rows(dy.numel() // shape[0], *shape)
+
+    def add_tensors(self, dy, x, dw, db, members) -> None:
+        desc, operands = ops.wgrad_desc(dy, x, dw, db)
+        self.add_descs([(desc, members)], (dy, dw, db, *operands))
+
+    def add_descs(self, products, keep) -> None:
+        """products: (vy_wgrad_desc, members) each; keep: every tensor they point into, the first one a bf16 operand."""
+        key = (keep[0].dtype, ops._raw_stream())
+        if self.items and key != self.key:
+            ops.wgrad_rows([desc for desc, _ in products])
+            for _, members in products:
+                _notify(*members)
+            return
+        for desc, members in products:
+            self._hold((keep[0], desc, keep, None, members), 0, key, False)
 
     def _launch(self, items) -> None:
-        ops.linear_wgrad_rows(items)
+        ops.wgrad_rows([item[1] for item in items])
+
+
+def _few_rows(M, N, K) -> bool:
+    """Does a weight gradient N x K over M rows wait for those of other layers with few rows?"""
+    return _GROUP_WGRADS and M < _GROUP_MIN_ROWS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0
 
 
 class _NormSums(_WgradGroup):
@@ -257,9 +282,8 @@ class _NormSums(_WgradGroup):
 
     MOST = 16
 
-    def add_norms(self, norms) -> None:
-        """norms: (ws, rows, weight, bias) each."""
-        items = [(ws, rows, w.grad, b.grad, (w, b)) for ws, rows, w, b in norms]
+    def add_norms(self, items) -> None:
+        """items: (ws, rows, gradients of weight and bias, (weight, bias)) each."""
         key = (torch.float32, ops._raw_stream())
         if (self.items and key != self.key) or any(getattr(p, "_vy_exchanged", False) for item in items for p in item[4]):
             self._launch([item[:4] for item in items])
@@ -518,7 +542,7 @@ class SelfAttentionFn(torch.autograd.Function):
         a2 = adds[1] if len(adds) > 1 else None
         if extra is not None:
             a2 = a2 + extra
-        dx = ops.linear_dgrad(packed, _wt_packed(mod, w, dt), add_to=a1, add_to2=a2)
+        dx = ops.linear_dgrad(packed, _wt_packed(mod, dt), add_to=a1, add_to2=a2)
         if ctx.defer is not None:
             ctx.defer.clear()
         grads = _packed_wgrad(mod, packed, x, w, b, params)
@@ -534,55 +558,87 @@ def _segments(*sizes):
     return out, at
 
 
+@functools.lru_cache(maxsize=256)
+def _kept_segments(B, L, d, hk_dh, inner, h):
+    """Offsets of what the weight gradients of a layer multiply with, [o | a | inner], of the rest, [q | s1 | deriv | s2 | k | v], and of the
+    statistics: waiting weight gradients hold their operands' buffer, so the rest has one of its own."""
+    M = B * L
+    return _segments(M * d, M * d, M * inner), _segments(M * d, M * d, M * inner, M * d, M * hk_dh, M * hk_dh), _segments(B * h * L, M, M, M, M)
+
+
+@functools.lru_cache(maxsize=256)
+def _work_segments(B, L, d, W, inner, h, slabs):
+    """Of the weight gradients' other operands, [ds2 | dpre | ds1 | dqkv], of [da | dheads], and of the scratch [delta | ln_ws]."""
+    M = B * L
+    return _segments(M * d, M * inner, M * d, M * W), _segments(M * d, M * d), _segments(B * h * L, 2 * slabs * d)
+
+
 class TextLayerFn(torch.autograd.Function):
     """A whole post-LN layer (autograd.layer_train): the launches of SelfAttentionFn, LinearResidualLayerNormFn and FfnBlockFn in their order,
     behind one native call each way; the gradients of the layer input's residual paths meet in the QKV dgrad's epilogue.  Every parameter's
-    gradient goes into the arena.  keep: [Wqkv, bqkv, Wo, bo, .., both norms, W1, b1, W2, b2] in the compute type."""
+    gradient goes into the arena.  keep: [Wqkv, bqkv, Wo, bo, .., both norms, W1, b1, W2, b2] in the compute type.
+
+    Steps of a few hundred tokens are the host's, so it does here what they need and no more: 12 layers, 186 tokens, 4.9 -> 4.4 ms a step,
+    captions of 3 images, 24 layers, 8.8 -> 6.6."""
 
     @staticmethod
-    def _layer(att, ff, x, kp, causal, start, rope, keep, kv):
+    def _layer(att, ff, x, kp, causal, start, rope, keep, inner, kv):
         """The descriptor; kv: where the keys and the values are."""
-        _, L, _ = x.shape
-        h, hk, dh = att.num_attention_heads, att.num_key_value_heads, att.head_dim
+        L = x.shape[1]
+        hk, dh = att.num_key_value_heads, att.head_dim
         cos, sin, pos0 = rope
         kind = (_lib.MASK_CAUSAL if causal else 0) | (_lib.MASK_KEYPAD if kp is not None else 0)
         st = (hk * L * dh, L * dh, dh)
-        return _lib.VyTextLayer(h, hk, dh, keep[6].shape[0], ff.act, kind, _lib.dtype_code(x.dtype), att._modules["out"]._modules["layernorm"].eps,
-                                ff._modules["layernorm"].eps, *(None if t is None else t.data_ptr() for t in keep), ops._ptr(cos), ops._ptr(sin),
-                                pos0, *kv, *st, *st, *kv, *st, *st, L, start, ops._ptr(kp), kp.stride(0) if kp is not None else 0)
-
-    @staticmethod
-    def _kept(x, hk_dh, inner, h):
-        """Offsets of what the weight gradients multiply with, [o | a | inner], of the rest, [q | s1 | deriv | s2 | k | v], and of the
-        statistics: waiting weight gradients hold their operands' buffer, so the rest has one of its own."""
-        B, L, d = x.shape
-        M = B * L
-        return _segments(M * d, M * d, M * inner), _segments(M * d, M * d, M * inner, M * d, M * hk_dh, M * hk_dh), _segments(B * h * L, M, M, M, M)
+        return _lib.VyTextLayer(att.num_attention_heads, hk, dh, inner, ff.act, kind, _lib.dtype_code(x.dtype),
+                                att._modules["out"]._modules["layernorm"].eps, ff._modules["layernorm"].eps,
+                                *[None if t is None else t.data_ptr() for t in keep], None if cos is None else cos.data_ptr(),
+                                None if sin is None else sin.data_ptr(), pos0, *kv, *st, *st, *kv, *st, *st, L, start,
+                                None if kp is None else kp.data_ptr(), 0 if kp is None else kp.stride(0))
 
     @staticmethod
     def _places(x, rows, rest, stats, operands, others, numbers):
         """-> vy_text_layer_kept, and where the keys and the values are."""
         e, r0, t0, s0 = x.element_size(), rows.data_ptr(), rest.data_ptr(), stats.data_ptr()
-        o, a, inner = (r0 + n * e for n in operands)
-        q, s1, deriv, s2, k, v = (t0 + n * e for n in others)
-        return _lib.VyTextLayerKept(q, o, s1, a, deriv, inner, s2, *(s0 + 4 * n for n in numbers)), (k, v)
+        o, a, inner = [r0 + n * e for n in operands]
+        q, s1, deriv, s2, k, v = [t0 + n * e for n in others]
+        return _lib.VyTextLayerKept(q, o, s1, a, deriv, inner, s2, *[s0 + 4 * n for n in numbers]), (k, v)
 
     @staticmethod
     def forward(ctx, x, kp, att, ff, keep, causal, start, rope, *params):
         B, L, d = x.shape
-        h, hk, dh, inner = att.num_attention_heads, att.num_key_value_heads, att.head_dim, keep[6].shape[0]
-        (operands, n), (others, m), (numbers, sn) = TextLayerFn._kept(x, hk * dh, inner, h)
-        rows = torch.empty(n, dtype=x.dtype, device=x.device)
-        rest = torch.empty(m, dtype=x.dtype, device=x.device)
-        stats = torch.empty(sn, dtype=torch.float32, device=x.device)
+        inner, dt, dev = keep[6].shape[0], x.dtype, x.device
+        (operands, n), (others, m), (numbers, sn) = _kept_segments(B, L, d, att.num_key_value_heads * att.head_dim, inner, att.num_attention_heads)
+        rows = torch.empty(n, dtype=dt, device=dev)
+        rest = torch.empty(m, dtype=dt, device=dev)
+        stats = torch.empty(sn, dtype=torch.float32, device=dev)
         y = torch.empty_like(x)
         kept, kv = TextLayerFn._places(x, rows, rest, stats, operands, others, numbers)
-        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, kv)
+        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, inner, kv)
         ops._mid_ws(B * L)
         _lib.call("vy_text_layer_train_fwd", _ref(desc), _ref(kept), x.data_ptr(), y.data_ptr(), B, L, ops._stream())
         ctx.save_for_backward(x, rows, rest, stats, kp)
         ctx.meta = (att, ff, causal, start, rope, params)
         return y
+
+    @staticmethod
+    def _waiting(M, d, W, inner, dt, params, nw):
+        """The gradients of the parameters, [Wo, bo, first norm, W1, b1, W2, b2, second norm, projections], if every weight gradient of the
+        layer waits for those of other layers with few rows (_WgradRows) and the projections' lie one behind the other."""
+        if dt is not torch.bfloat16 or not _GROUP_QKV or not (_few_rows(M, d, d) and _few_rows(M, W, d) and _few_rows(M, inner, d) and _few_rows(M, d, inner)):
+            return None
+        grads = []
+        for p in params:
+            g = p.grad if getattr(p, "_vy_direct", False) else None
+            if g is None or g.dtype is not torch.float32 or not g.is_contiguous() or getattr(p, "_vy_exchanged", False):
+                return None
+            grads.append(g)
+        for group in (grads[10:10 + nw], grads[10 + nw:]):
+            at = group[0].data_ptr() if group else 0
+            for g in group:
+                if g.data_ptr() != at:
+                    return None
+                at += 4 * g.numel()
+        return grads
 
     @staticmethod
     def backward(ctx, dy):
@@ -593,37 +649,46 @@ class TextLayerFn(torch.autograd.Function):
         dy, rows, rest, stats = dy.contiguous(), rows.contiguous(), rest.contiguous(), stats.contiguous()
         wo, bo, g1, b1, w1, c1, w2, c2, g2, b2 = params[:10]
         members = att._params()
-        w, b = att._packed(members)
-        keep = [*att._packed_shadow(dt, (w, b), members), *[_shadow(p, dt) for p in params[:10]]]
-        h, hk, dh, inner = att.num_attention_heads, att.num_key_value_heads, att.head_dim, keep[6].shape[0]
-        W = d + 2 * hk * dh
-        (operands, _), (others, _), (numbers, _) = TextLayerFn._kept(x, hk * dh, inner, h)
+        h, hk_dh, inner = att.num_attention_heads, att.num_key_value_heads * att.head_dim, w1.shape[0]
+        W = d + 2 * hk_dh
+        (operands, _), (others, _), (numbers, _) = _kept_segments(B, L, d, hk_dh, inner, h)
         kept, kv = TextLayerFn._places(x, rows, rest, stats, operands, others, numbers)
-        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, kv)
-        wt = [_wt_packed(att, w, dt, members), _wt(wo, dt), _wt(w1, dt), _wt(w2, dt)]
-        to, n = _segments(M * d, M * inner, M * d, M * W)      # ds2, dpre, ds1, dqkv: the weight gradients' other operands
-        work = torch.empty(n, dtype=dt, device=dev)
-        oo, on = _segments(M * d, M * d)                       # da, dheads
-        own = torch.empty(on, dtype=dt, device=dev)
+        # (of the weights only the norms' are read here, the others transposed)
+        keep = (None, None, None, None, _shadow(g1, dt), None, None, None, None, None, _shadow(g2, dt), None)
+        desc = TextLayerFn._layer(att, ff, x, kp, causal, start, rope, keep, inner, kv)
+        wt = (_wt_packed(att, dt, members), _wt(wo, dt), _wt(w1, dt), _wt(w2, dt))
         slabs = _lib.load().vy_layernorm_bwd_ws_rows(M)
-        wait = _GROUP_WGRADS and all(_direct(p) for p in (g1, b1, g2, b2))     # the norms' column sums go out with other layers'
-        fo, fn = _segments(B * h * L, 0 if wait else 2 * slabs * d)
-        scratch = torch.empty(fn, dtype=torch.float32, device=dev)
-        sums = torch.empty((2, 2 * slabs * d), dtype=torch.float32, device=dev) if wait else None
+        (to, n), (oo, on), (fo, fn) = _work_segments(B, L, d, W, inner, h, slabs)
+        work = torch.empty(n, dtype=dt, device=dev)
+        own = torch.empty(on, dtype=dt, device=dev)
         dx = torch.empty_like(x)
-        e, f0 = x.element_size(), scratch.data_ptr()
-        ds2, dpre, ds1, dqkv = (work.data_ptr() + o * e for o in to)
-        da, dheads = (own.data_ptr() + o * e for o in oo)
+        nw = 1 if att._fused_qkv else 3
+        waiting = TextLayerFn._waiting(M, d, W, inner, dt, (*params[:10], *members), nw) if x.is_contiguous() else None
+        wait = waiting is not None or (_GROUP_WGRADS and all(_direct(p) for p in (g1, b1, g2, b2)))    # the norms' column sums go out with other layers'
+        scratch = torch.empty(fo[1] if wait else fn, dtype=torch.float32, device=dev)
+        sums = torch.empty((2, 2 * slabs * d), dtype=torch.float32, device=dev) if wait else None
+        e, f0, w0, o0 = x.element_size(), scratch.data_ptr(), work.data_ptr(), own.data_ptr()
+        ds2, dpre, ds1, dqkv = [w0 + o * e for o in to]
         # (a gradient that has left the arena since the forward pass is returned)
         dln = [] if wait else [p.grad if _direct(p) else torch.zeros(d, dtype=torch.float32, device=dev) for p in (g1, b1, g2, b2)]
         at = sums.data_ptr() if wait else f0 + 4 * fo[1]
-        grads = _lib.VyTextLayerGrads(*(t.data_ptr() for t in wt), *(t.stride(0) for t in wt), *((None,) * 4 if wait else (t.data_ptr() for t in dln)),
-                                      ds2, dpre, da, ds1, dheads, dqkv, at, f0 + 4 * fo[0], at + 8 * slabs * d if wait else None)
+        grads = _lib.VyTextLayerGrads(*[t.data_ptr() for t in wt], *[t.stride(0) for t in wt], *((None,) * 4 if wait else [t.data_ptr() for t in dln]),
+                                      ds2, dpre, o0 + oo[0] * e, ds1, o0 + oo[1] * e, dqkv, at, f0, at + 8 * slabs * d if wait else None)
         ops._mid_ws(M)
         _lib.call("vy_text_layer_bwd", _ref(desc), _ref(kept), _ref(grads), dy.data_ptr(), dx.data_ptr(), B, L, ops._stream())
+        if waiting is not None:
+            _norm_sums.add_norms([(sums[0], slabs, waiting[8], waiting[9], (g2, b2)), (sums[1], slabs, waiting[2], waiting[3], (g1, b1))])
+            gwo, gbo, _, _, gw1, gc1, gw2, gc2, _, _, gq = [g.data_ptr() for g in waiting[:11]]
+            gbq = waiting[10 + nw].data_ptr() if len(members) > nw else None
+            D, kept_o, kept_a, kept_inner = _lib.VyWgradDesc, kept.o, kept.a, kept.inner
+            _wgrad_rows.add_descs([(D(ds2, d, kept_inner, inner, gw2, inner, gc2, M, d, inner), (w2, c2)),
+                                   (D(dpre, inner, kept_a, d, gw1, d, gc1, M, inner, d), (w1, c1)),
+                                   (D(ds1, d, kept_o, d, gwo, d, gbo, M, d, d), (wo, bo)),
+                                   (D(dqkv, W, x.data_ptr(), d, gq, d, gbq, M, W, d), members)], (work, rows, x, *waiting))
+            return (dx, *[None] * (7 + len(params)))
         if wait:
             dg1 = db1 = dg2 = db2 = None
-            _norm_sums.add_norms([(sums[0], slabs, g2, b2), (sums[1], slabs, g1, b1)])
+            _norm_sums.add_norms([(sums[0], slabs, g2.grad, b2.grad, (g2, b2)), (sums[1], slabs, g1.grad, b1.grad, (g1, b1))])
         else:
             dg1, db1, dg2, db2 = (None if _direct(p) else t.to(p.dtype) for p, t in zip((g1, b1, g2, b2), dln))
             _notify(*(p for p in (g2, b2, g1, b1) if _direct(p)))
@@ -633,7 +698,7 @@ class TextLayerFn(torch.autograd.Function):
         dw2 = _wgrad(of(work, to[0], d), of(rows, operands[2], inner), w2, c2)
         dw1 = _wgrad(of(work, to[1], inner), of(rows, operands[1], d), w1, c1)
         dwo = _wgrad(of(work, to[2], d), of(rows, operands[0], d), wo, bo)
-        dqkv_w = _packed_wgrad(att, of(work, to[3], W), x, w, b, params[10:], members)
+        dqkv_w = _packed_wgrad(att, of(work, to[3], W), x, *att._packed(members), params[10:], members)
         return (dx, *[None] * 7, *dwo, dg1, db1, *dw1, *dw2, dg2, db2, *dqkv_w)
 
 
@@ -693,15 +758,18 @@ def _heads(x2: torch.Tensor, heads: int, dh: int) -> torch.Tensor:
     return x2.view(B, L, heads, dh).permute(0, 2, 1, 3)
 
 
-def _wt_packed(mod, w, dtype, members=None):
+def _wt_packed(mod, dtype, members=None):
     """W^T of the packed projection: keyed on the versions of the member parameters.  (members: what mod._params() has just returned)"""
-    if members is not None:   # what _wt_cached finds first
-        view = getattr(mod, "_vy_wt_view", None)
-        if view is not None and getattr(mod, "_vy_wt_key", None) == tuple([p._version for p in members]) + (WEIGHT_EPOCH[0], dtype):
-            mod._vy_wt_entry[4] = WEIGHT_EPOCH[0]
-            return view
-    return _wt_cached(mod, lambda m: tuple(p._version for p in m._params()) + (WEIGHT_EPOCH[0], dtype),
-                      lambda m: m._packed_shadow(dtype)[0])
+    def key(members):
+        return (*[p._version for p in members], getattr(members[0], "_vy_weights", _WT).epoch, dtype)
+
+    def key_of(m):
+        members = m._params()
+        return key(members), members
+    if members is None:
+        members = mod._params()
+    return _wt_cached(mod, getattr(members[0], "_vy_weights", _WT), key(members), key_of, lambda m, members: m._packed_shadow(dtype, None, members)[0],
+                      members)
 
 
 def _packed_wgrad(mod, dy, x, w, b, params, members=None):

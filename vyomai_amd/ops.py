@@ -419,34 +419,38 @@ def linear_wgrad_grouped(items) -> None:
     """items: up to 12 tuples (dy, x, dw, db|None): dw += dy^T @ x, db += colsum(dy), ONE launch
     (vy_linear_wgrad_grouped, vy_linear_wgrad_batch).  The tensors must stay alive until the launch has been enqueued (they do:
     the caller holds them)."""
-    _wgrads("vy_linear_wgrad_grouped" if len(items) <= 8 else "vy_linear_wgrad_batch", 12, items)
+    n = len(items)
+    assert 1 <= n <= 12
+    dt = items[0][0].dtype
+    assert all(dy.dtype == dt for dy, *_ in items)
+    made = [wgrad_desc(*item) for item in items]   # (copies of operands without uniform rows live until the launch)
+    arr = (_lib.VyWgradDesc * n)(*[desc for desc, _ in made])
+    call("vy_linear_wgrad_grouped" if n <= 8 else "vy_linear_wgrad_batch", C.cast(arr, C.c_void_p), n, dtype_code(dt), _stream())
+
+
+def wgrad_desc(dy: Tensor, x: Tensor, dw: Tensor, db: Optional[Tensor]):
+    """-> (vy_wgrad_desc, the operands as rows, which it points into)"""
+    _need_gpu(dy, x, dw, db)
+    d2, x2 = _rows(dy), _rows(x)
+    M, N = d2.shape
+    K = x2.shape[1]
+    assert x2.shape[0] == M and dw.dtype == torch.float32 and dw.shape == (N, K) and dw.stride(1) == 1
+    assert db is None or (db.dtype == torch.float32 and db.numel() == N)
+    return _lib.VyWgradDesc(d2.data_ptr(), d2.stride(0), x2.data_ptr(), x2.stride(0), dw.data_ptr(), dw.stride(0), _ptr(db), M, N, K), (d2, x2)
+
+
+def wgrad_rows(descs) -> None:
+    """The same for up to 16 bf16 gradients over few rows, each with the sums of linear_wgrad (vy_linear_wgrad_rows); descs: wgrad_desc's."""
+    n = len(descs)
+    assert 1 <= n <= 16
+    call("vy_linear_wgrad_rows", C.cast((_lib.VyWgradDesc * n)(*descs), C.c_void_p), n, _lib.VY_BF16, _stream())
 
 
 def linear_wgrad_rows(items) -> None:
-    """The same for up to 16 bf16 gradients over few rows, each with the sums of linear_wgrad (vy_linear_wgrad_rows)."""
-    _wgrads("vy_linear_wgrad_rows", 16, items)
-
-
-def _wgrads(entry: str, most: int, items) -> None:
-    n = len(items)
-    assert 1 <= n <= most
-    arr = (_lib.VyWgradDesc * n)()
-    dt, rows = None, []   # (rows: copies of operands without uniform rows live until the launch)
-    for i, (dy, x, dw, db) in enumerate(items):
-        _need_gpu(dy, x, dw, db)
-        d2, x2 = _rows(dy), _rows(x)
-        rows.append((d2, x2))
-        M, N = d2.shape
-        K = x2.shape[1]
-        assert x2.shape[0] == M and dw.dtype == torch.float32 and dw.shape == (N, K) and dw.stride(1) == 1
-        assert db is None or (db.dtype == torch.float32 and db.numel() == N)
-        assert dt is None or dt == dy.dtype
-        dt = dy.dtype
-        a = arr[i]
-        a.dy, a.lddy, a.x, a.ldx = d2.data_ptr(), d2.stride(0), x2.data_ptr(), x2.stride(0)
-        a.dw, a.lddw, a.db = dw.data_ptr(), dw.stride(0), _ptr(db)
-        a.M, a.N, a.K = M, N, K
-    call(entry, C.cast(arr, C.c_void_p), n, dtype_code(dt), _stream())
+    """items: as linear_wgrad_grouped's."""
+    assert all(dy.dtype == torch.bfloat16 for dy, *_ in items)
+    made = [wgrad_desc(*item) for item in items]
+    wgrad_rows([desc for desc, _ in made])
 
 
 def layernorm_bwd(dy: Tensor, x: Tensor, gamma: Tensor, mean: Tensor, rstd: Tensor, dgamma: Tensor,
@@ -501,18 +505,21 @@ def attention_bwd(q, k, v, out, dout, lse, dq, dk, dv, *, causal: bool, start_po
 
 def adamw_step(p: Tensor, g: Tensor, m: Tensor, v: Tensor, p_bf16: Optional[Tensor], lr: float,
                beta1: float, beta2: float, eps: float, weight_decay: float, step: int,
-               grad_scale: float = 1.0, scale_dev: Optional[Tensor] = None, gate: Optional[Tensor] = None) -> None:
+               grad_scale: float = 1.0, scale_dev: Optional[Tensor] = None, gate: Optional[Tensor] = None,
+               stream: Optional[int] = None) -> None:
     """scale_dev: optional fp32 device scalar multiplied into grad_scale by the kernel (clip coefficient).
-    gate: optional fp32 device scalar; when it is 0 the launch changes nothing (vy_adamw_step_gated)."""
+    gate: optional fp32 device scalar; when it is 0 the launch changes nothing (vy_adamw_step_gated).
+    stream: a stream's handle (None: the current stream)."""
     _need_gpu(p, g, m, v, p_bf16, scale_dev, gate)
     assert scale_dev is None or (scale_dev.dtype == torch.float32 and scale_dev.numel() == 1)
+    stream = _stream() if stream is None else stream
     if gate is None:
         call("vy_adamw_step", p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), _ptr(p_bf16), p.numel(),
-             lr, beta1, beta2, eps, weight_decay, step, grad_scale, _ptr(scale_dev), _stream())
+             lr, beta1, beta2, eps, weight_decay, step, grad_scale, _ptr(scale_dev), stream)
     else:
         assert gate.dtype == torch.float32 and gate.numel() == 1
         call("vy_adamw_step_gated", p.data_ptr(), g.data_ptr(), m.data_ptr(), v.data_ptr(), _ptr(p_bf16), p.numel(),
-             lr, beta1, beta2, eps, weight_decay, step, grad_scale, _ptr(scale_dev), gate.data_ptr(), _stream())
+             lr, beta1, beta2, eps, weight_decay, step, grad_scale, _ptr(scale_dev), gate.data_ptr(), stream)
 
 
 def sumsq(x: Tensor) -> Tensor:

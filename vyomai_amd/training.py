@@ -229,6 +229,7 @@ class BucketReducer:
         # parameters that require gradients are waited for; a frozen one never reports.
         self.buckets: List[Tuple[int, int]] = []      # (start, end) element ranges
         self.bucket_of: Dict[int, int] = {}
+        self.members: List[List[nn.Parameter]] = []   # parameters of each
         self.expect: List[int] = []
         cap = max(1, bucket_bytes // 4)
         end = arena.numel
@@ -244,6 +245,7 @@ class BucketReducer:
             if end - cur_start >= cap or idx == 0:
                 b = len(self.buckets)
                 self.buckets.append((cur_start, end))
+                self.members.append([arena.params[m] for m in members])
                 self.expect.append(count)
                 for m in members:
                     self.bucket_of[id(arena.params[m])] = b
@@ -421,6 +423,10 @@ class FlatTrainer:
                 m.compute_dtype = compute_dtype
         # fp32 compute (the parity path) reads the masters themselves: no shadow arena
         self.arena = FlatArena(model, shadow_dtype=None if compute_dtype == torch.float32 else compute_dtype)
+        from .autograd_train import _WtRegistry
+        self.weights = _WtRegistry()
+        for p in self.arena.params:
+            p._vy_weights = self.weights
         self.m = torch.zeros_like(self.arena.master)
         self.v = torch.zeros_like(self.arena.master)
         # native_rccl: the exchange goes through the library's own RCCL communicator (vy_ddp_*) instead of
@@ -446,6 +452,7 @@ class FlatTrainer:
             overlap_optimizer = False
         self._side = torch.cuda.Stream() if (overlap_optimizer and self.arena.master.is_cuda) else None
         self._stepped: set = set()
+        self._events: Dict[int, torch.cuda.Event] = {}
         self._scale = (1.0 / self.reducer.world) if (self.reducer.average and self.reducer.world > 1) else 1.0
         if self._side is not None:
             self.reducer.on_bucket = self._bucket_final
@@ -509,14 +516,14 @@ class FlatTrainer:
         self.reducer.enabled = True
 
     def _adamw(self, lo: int, hi: int, step: int, scale_dev: Optional[torch.Tensor] = None,
-               gate: Optional[torch.Tensor] = None) -> None:
+               gate: Optional[torch.Tensor] = None, stream: Optional[int] = None) -> None:
         """gate: one fp32 on the device; the launch leaves the range alone when it is 0 (a parameter without a gradient
-        on this rank whose fate depends on the other ranks: BucketReducer._exchange_flags)."""
+        on this rank whose fate depends on the other ranks: BucketReducer._exchange_flags).  stream: None, the current one."""
         from . import ops
         a = self.arena
         ops.adamw_step(a.master[lo:hi], a.grad[lo:hi], self.m[lo:hi], self.v[lo:hi],
                        None if a.shadow is None else a.shadow[lo:hi], self.lr, self.betas[0], self.betas[1],
-                       self.eps, self.weight_decay, step, self._scale, scale_dev=scale_dev, gate=gate)
+                       self.eps, self.weight_decay, step, self._scale, scale_dev=scale_dev, gate=gate, stream=stream)
 
     def _step_range(self, lo: int, hi: int, step: int, scale_dev: Optional[torch.Tensor] = None) -> None:
         """AdamW over the trainable parameters inside [lo, hi) that received a gradient -- on this rank (merged plain
@@ -539,13 +546,20 @@ class FlatTrainer:
     def _bucket_final(self, b: int, work) -> None:
         """Reducer callback (during backward): step bucket b on the side stream."""
         lo, hi = self.reducer.buckets[b]
-        ev = torch.cuda.current_stream().record_event()   # after the kernels that wrote its gradients
+        ev = self._events.get(b)
+        if ev is None:
+            ev = self._events[b] = torch.cuda.Event()
+        ev.record(torch.cuda.current_stream())             # after the kernels that wrote its gradients
         self._side.wait_event(ev)
-        with torch.cuda.stream(self._side):
-            if work is not None:
-                work.wait()                                # the side stream waits for the all-reduce
-                self.reducer.writeback(b)
-            self._step_range(lo, hi, self.step_count + 1)
+        r = self.reducer
+        if work is None and r.global_flags is None and all([p.requires_grad and id(p) in r.touched for p in r.members[b]]):
+            self._adamw(lo, hi, self.step_count + 1, stream=self._side.cuda_stream)      # (what _step_range makes of it)
+        else:
+            with torch.cuda.stream(self._side):
+                if work is not None:
+                    work.wait()                            # the side stream waits for the all-reduce
+                    r.writeback(b)
+                self._step_range(lo, hi, self.step_count + 1)
         self._stepped.add(b)
 
     def _sumsq(self) -> torch.Tensor:
@@ -558,8 +572,6 @@ class FlatTrainer:
 
     def optimizer_step(self) -> bool:
         """-> True when an update was applied (False inside an accumulation window)."""
-        from .autograd_train import WEIGHT_EPOCH
-
         if self._micro < self.accumulate_steps:
             return False
         self._micro = 0
@@ -579,9 +591,15 @@ class FlatTrainer:
                 if b not in self._stepped:
                     self._step_range(lo, hi, self.step_count)
             torch.cuda.current_stream().wait_stream(self._side)
-        WEIGHT_EPOCH[0] += 1
+        self._new_weights()
         self._needs_zero = True
         return True
+
+    def _new_weights(self) -> None:
+        """The W^T copies of this trainer's matrices are old, and those of matrices that no trainer owns (they may be views of its arena)."""
+        from .autograd_train import _WT
+        self.weights.bump()
+        _WT.bump()
 
     def train_step(self, loss_fn: Callable[[], torch.Tensor]) -> torch.Tensor:
         """zero_grad -> loss_fn() -> backward (overlapped all-reduce) -> fused AdamW.  With
@@ -597,14 +615,13 @@ class FlatTrainer:
         """After anything but this trainer wrote the parameters in place (load_state_dict, a manual
         re-initialisation): recast the fp32 masters into the compute-dtype arena the kernels read and
         invalidate every cached W^T."""
-        from .autograd_train import WEIGHT_EPOCH
         self.arena.refresh_shadow(install=True)
         self.arena._install_packed(self.model)
         if reset_moments:
             self.m.zero_()
             self.v.zero_()
             self.step_count = 0
-        WEIGHT_EPOCH[0] += 1
+        self._new_weights()
 
     def load_state_dict(self, state_dict, strict: bool = True, reset_moments: bool = False):
         """model.load_state_dict() into the master arena (the parameters are views of it), then resync()."""
