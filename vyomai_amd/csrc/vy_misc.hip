@@ -20,6 +20,9 @@ namespace {
 // ---- LayerNorm forward: one wave per row, CH chunks per lane -------------------------------
 // mean, then variance about the mean (two reductions on registers): the same two-pass
 // formulation as aten's CPU LayerNorm closely enough for 1e-6 agreement.
+// Weight and bias are requested with the row, not behind the reductions (512 rows of 768: 3.7 -> 3.2 us, an encoder of 4 x 128 tokens
+// 708 -> 699 us); the rows, which only this launch and perhaps the backward pass read, pass by the caches (30500 rows 19.8 -> 19.6 us, the encoder
+// behind them 7452 -> 7419: the products around find more of their operands).
 template <typename T, int CH>
 __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const T* __restrict__ x, int64_t ldx,
                                                             const T* __restrict__ gamma,
@@ -32,18 +35,39 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const T* __restrict_
   const int64_t row = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
   if (row >= M) return;
   const int nch = N / VEC;
+  typedef typename VyChunk<T>::Raw Raw;
+  constexpr bool AHEAD = CH <= 4;
+  Raw gr[AHEAD ? CH : 1], br[AHEAD ? CH : 1];
   float v[CH][VEC];
   float s = 0.f;
+  {
+    Raw xr[CH];
 #pragma unroll
-  for (int c = 0; c < CH; ++c) {
-    const int ch = lane + 64 * c;
-    if (ch < nch) {
-      VyChunk<T>::load(x + row * ldx + (int64_t)ch * VEC, v[c]);
+    for (int c = 0; c < CH; ++c) {
+      const int ch = lane + 64 * c;
+      if (ch < nch) xr[c] = __builtin_nontemporal_load(reinterpret_cast<const Raw*>(x + row * ldx + (int64_t)ch * VEC));
+    }
+    if constexpr (AHEAD) {
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) s += v[c][e];
-    } else {
+      for (int c = 0; c < CH; ++c) {
+        const int ch = lane + 64 * c;
+        if (ch < nch) {
+          gr[c] = *reinterpret_cast<const Raw*>(gamma + (int64_t)ch * VEC);
+          br[c] = *reinterpret_cast<const Raw*>(beta + (int64_t)ch * VEC);
+        }
+      }
+    }
 #pragma unroll
-      for (int e = 0; e < VEC; ++e) v[c][e] = 0.f;
+    for (int c = 0; c < CH; ++c) {
+      const int ch = lane + 64 * c;
+      if (ch < nch) {
+        VyChunk<T>::unpack(xr[c], v[c]);
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) s += v[c][e];
+      } else {
+#pragma unroll
+        for (int e = 0; e < VEC; ++e) v[c][e] = 0.f;
+      }
     }
   }
   const float mean = vy_wave_sum(s) / (float)N;
@@ -65,8 +89,13 @@ __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const T* __restrict_
     const int ch = lane + 64 * c;
     if (ch < nch) {
       float g[VEC], b[VEC], o[VEC];
-      VyChunk<T>::load(gamma + (int64_t)ch * VEC, g);
-      VyChunk<T>::load(beta + (int64_t)ch * VEC, b);
+      if constexpr (AHEAD) {
+        VyChunk<T>::unpack(gr[c], g);
+        VyChunk<T>::unpack(br[c], b);
+      } else {
+        VyChunk<T>::load(gamma + (int64_t)ch * VEC, g);
+        VyChunk<T>::load(beta + (int64_t)ch * VEC, b);
+      }
 #pragma unroll
       for (int e = 0; e < VEC; ++e) o[e] = (v[c][e] - mean) * rstd_r * g[e] + b[e];
       VyChunk<T>::store(y + row * ldy + (int64_t)ch * VEC, o);

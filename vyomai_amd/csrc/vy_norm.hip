@@ -41,6 +41,14 @@ template <> __device__ __forceinline__ void load4<bf16>(const bf16* p, float (&v
 #pragma unroll
   for (int e = 0; e < 4; ++e) v[e] = (float)t[e];
 }
+// what a launch over many rows reads or writes once
+template <bool ONCE, typename T> __device__ __forceinline__ void load4_once(const T* p, float (&v)[4]) {
+  if constexpr (!ONCE) return load4<T>(p, v);
+  typedef __attribute__((ext_vector_type(4))) T T4;
+  const T4 q = __builtin_nontemporal_load(reinterpret_cast<const T4*>(p));
+#pragma unroll
+  for (int e = 0; e < 4; ++e) v[e] = (float)q[e];
+}
 template <typename T> __device__ __forceinline__ void store4(T* p, const float (&v)[4]);
 template <> __device__ __forceinline__ void store4<float>(float* p, const float (&v)[4]) {
   *reinterpret_cast<f32x4*>(p) = f32x4{v[0], v[1], v[2], v[3]};
@@ -93,6 +101,9 @@ __device__ __forceinline__ void row_stats(const float (&v)[CH][4], int t, int N,
 // A step of few rows (TPR = 256: a workgroup per row) is a chain of memory round trips and reductions and nothing else: the norms'
 // weights are requested with the row (not behind the reductions) and a row that arrives in PARTS slices has all of them in flight.
 // 32 rows of 1024: 4.2 -> 3.1 us, one row with layer norms: 3.8 -> 2.6 us.
+// Many rows (TPR = 64: a wave per row) are bound by memory, 200 MB for 8192 rows of 2048: the stream and the sublayer's rows pass by the
+// caches, which then still hold what the products around the norm read (40.9 -> 40.2 us here, prompts of 8 x 1024 tokens 9723 -> 9602 us, of
+// 8192 tokens through plain feed-forwards 10094 -> 9998).
 template <typename T, int TPR, int CH, bool RMS, bool ROUTED, int PARTS = 0>
 __global__ __launch_bounds__(256) void residual_norm_kernel(ResNormArgs p) {
   constexpr bool AHEAD = TPR == 256 && CH <= 4;
@@ -138,9 +149,9 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResNormArgs p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) y[c][e] += v[s][e];
       } else {
-        if (p.ids || p.y) load4<T>(src + col, y[c]);
+        if (p.ids || p.y) load4_once<TPR == 64>(src + col, y[c]);
       }
-      if (!p.ids) load4<float>(xr + col, x[c]);
+      if (!p.ids) load4_once<TPR == 64>(xr + col, x[c]);
     }
   }
   if (p.ids) {
@@ -184,7 +195,8 @@ __global__ __launch_bounds__(256) void residual_norm_kernel(ResNormArgs p) {
 #pragma unroll
           for (int e = 0; e < 4; ++e) x[c][e] += bad ? 0.f : y[c][e];
         }
-        store4<float>(xr + col, x[c]);
+        if constexpr (TPR == 64) __builtin_nontemporal_store(f32x4{x[c][0], x[c][1], x[c][2], x[c][3]}, reinterpret_cast<f32x4*>(xr + col));
+        else store4<float>(xr + col, x[c]);
       }
     }
   }
