@@ -447,7 +447,7 @@ typedef struct vy_wgrad_desc {
 int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
 /* vy_linear_wgrad_batch: the same for up to 12. */
 int vy_linear_wgrad_batch(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
-/* vy_linear_wgrad_rows: the same for up to 16 bf16 gradients over few rows, each summed up in the slices of rows that
+/* vy_linear_wgrad_rows: the same for up to 20 bf16 gradients over few rows, each summed up in the slices of rows that
  * vy_linear_wgrad takes for its shape; the slices' sums are added up in their order and added to dW_i once. */
 int vy_linear_wgrad_rows(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
 

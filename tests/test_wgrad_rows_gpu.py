@@ -10,11 +10,11 @@ SHAPES = [(768, 3072), (3072, 768), (768, 768), (2304, 768), (512, 520), (255, 1
 @pytest.mark.parametrize("M", [1, 24, 63, 256, 257, 512, 700, 1665, 2047])
 def test_rows(M):
     """Slices of 64 to 256 rows and their remainders, tiles that end in the last row or column but eight, gradients smaller than a tile, 1 to
-    16 gradients.  Up to two slices the sums of a launch of its own arrive in either order with the same result; more of them are added in
+    20 gradients.  Up to two slices the sums of a launch of its own arrive in either order with the same result; more of them are added in
     their order here, in any there: a rounding each, at most 8, of the sum of magnitudes."""
     from vyomai_amd import ops
     g = torch.Generator(device=DEV).manual_seed(M)
-    for shapes in (SHAPES, (SHAPES * 3)[:16], SHAPES[:1]):
+    for shapes in (SHAPES, (SHAPES * 3)[:20], SHAPES[:1]):
         items, alone = [], []
         for i, (N, K) in enumerate(shapes):
             dy = torch.randn(M, (N + 7) // 8 * 8, device=DEV, generator=g).to(BF)[:, :N]
@@ -55,7 +55,7 @@ def test_rows_are_added_to_what_is_there():
 
 def test_refused_on_the_host():
     from vyomai_amd import _lib
-    d = (_lib.VyWgradDesc * 17)()
+    d = (_lib.VyWgradDesc * 21)()
     import ctypes as C
     buf = (C.c_char * 64)()
     a = (C.addressof(buf) + 15) // 16 * 16
@@ -64,11 +64,14 @@ def test_refused_on_the_host():
         d[i].dy, d[i].lddy, d[i].x, d[i].ldx, d[i].dw, d[i].lddw, d[i].db = dy, lddy, a, 8, a, 8, None
         d[i].M, d[i].N, d[i].K = 1, 8, K
     ref = C.cast(d, C.c_void_p)
-    for n, kind, match in ((0, _lib.dtype_code(BF), "1..16"), (17, _lib.dtype_code(BF), "1..16"), (1, _lib.dtype_code(torch.float32), "dtype")):
+    for n, kind, match in ((0, _lib.dtype_code(BF), "1..20"), (21, _lib.dtype_code(BF), "1..20"), (1, _lib.dtype_code(torch.float32), "dtype")):
         with pytest.raises(_lib.VyomHipError, match=match):
             _lib.call("vy_linear_wgrad_rows", ref, n, kind, None)
+    fill(1)
     for bad in ({"K": 12}, {"lddy": 12}, {"dy": a + 2}, {"lddy": 0}):
         fill(0, **bad)
+        with pytest.raises(_lib.VyomHipError, match="multiples of 8"):
+            _lib.call("vy_linear_wgrad_rows", ref, 2, _lib.dtype_code(BF), None)
         with pytest.raises(_lib.VyomHipError, match="multiples of 8"):
             _lib.call("vy_linear_wgrad_rows", ref, 1, _lib.dtype_code(BF), None)
 
@@ -83,3 +86,22 @@ def test_which_gradients_wait():
     assert not g.gathers(rows(24, 768), (768, 772), [p]) and not g.gathers(rows(24, 768), (768, 768), [p], torch.ones(1))
     p._vy_exchanged = True
     assert not g.gathers(rows(24, 768), (768, 768), [p])
+
+
+def test_a_launch_takes_whole_layers(monkeypatch):
+    """Four layers' gradients, or what comes before them and four layers'; never more than twenty."""
+    from vyomai_amd import autograd_train as AT
+    sizes = []
+    monkeypatch.setattr(AT.ops, "wgrad_rows", lambda descs: sizes.append(len(descs)))
+    monkeypatch.setattr(AT.ops, "_raw_stream", lambda: 1)
+    g = AT._WgradRows()
+    g.armed = True   # (no backward pass to flush it)
+    keep = (torch.empty(4, dtype=BF),)
+    g.add_descs([(None, [])], keep)
+    for _ in range(12):
+        g.add_descs([(None, [])] * 4, keep)
+    assert sizes == [17, 16, 16] and not g.items
+    for _ in range(15):
+        g.add_descs([(None, [])], keep)
+    g.add_descs([(None, [])] * 6, keep)
+    assert sizes == [17, 16, 16, 15] and len(g.items) == 6

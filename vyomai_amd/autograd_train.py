@@ -245,7 +245,7 @@ class _WgradRows(_WgradGroup):
     """The same for gradients over fewer rows than those: four layers' in a launch that sums each up as a launch of its own does
     (ops.wgrad_rows), so they keep their bits.  Exchanged gradients go out one by one."""
 
-    MOST = 16
+    MOST, FULL = 20, 16     # gradients of a launch; four layers' (with the language model head's dense layer before them: 17) fill it
 
     def gathers(self, dy, shape, members, alpha=None) -> bool:
         if alpha is not None or dy.dtype != torch.bfloat16 or any(getattr(p, "_vy_exchanged", False) for p in members):
@@ -264,8 +264,12 @@ class _WgradRows(_WgradGroup):
             for _, members in products:
                 _notify(*members)
             return
+        if len(self.items) + len(products) > self.MOST:
+            self.flush()
         for desc, members in products:
             self._hold((keep[0], desc, keep, None, members), 0, key, False)
+        if len(self.items) >= self.FULL:
+            self.flush()
 
     def _launch(self, items) -> None:
         ops.wgrad_rows([item[1] for item in items])
