@@ -567,15 +567,21 @@ __global__ __launch_bounds__(256) void attn_delta_kernel(BwdParams p) {
 // RoPE is an orthogonal map, so its backward is the transposed rotation of the gradient pair
 // (d, d+32): lo' = lo*c + hi*s, hi' = hi*c - lo*s, with the same storage-rounded cos/sin the forward
 // used.  pos = token position, d0 = first of the 4 consecutive d (< 32) of this quad.
-__device__ __forceinline__ void rope_bwd_quad(const BwdParams& p, int64_t pos, int d0, float (&lo)[4], float (&hi)[4]) {
-  const f32x4 c4 = *reinterpret_cast<const f32x4*>(p.cos_tab + pos * 32 + d0);
-  const f32x4 s4 = *reinterpret_cast<const f32x4*>(p.sin_tab + pos * 32 + d0);
+__device__ __forceinline__ void rope_bwd_quad(const f32x4& c4, const f32x4& s4, float (&lo)[4], float (&hi)[4]) {
 #pragma unroll
   for (int e = 0; e < 4; ++e) {
     const float c = vy_round_bf16(c4[e]), s = vy_round_bf16(s4[e]);
     const float a = lo[e], b = hi[e];
-    lo[e] = a * c + b * s;
-    hi[e] = b * c - a * s;
+    lo[e] = fmaf(a, c, b * s);
+    hi[e] = fmaf(b, c, -(a * s));
+  }
+}
+// a lane's eight quads of cos and sin for one position, all requested at once
+__device__ __forceinline__ void rope_bwd_tables(const BwdParams& p, int64_t pos, int fh, f32x4 (&c4)[4], f32x4 (&s4)[4]) {
+#pragma unroll
+  for (int rg = 0; rg < 4; ++rg) {
+    c4[rg] = *reinterpret_cast<const f32x4*>(p.cos_tab + pos * 32 + 8 * rg + 4 * fh);
+    s4[rg] = *reinterpret_cast<const f32x4*>(p.sin_tab + pos * 32 + 8 * rg + 4 * fh);
   }
 }
 
@@ -584,6 +590,11 @@ __device__ __forceinline__ void rope_bwd_quad(const BwdParams& p, int64_t pos, i
 __device__ __forceinline__ int dual_sw(int row) {
   const int v = (row >> 1) & 7;
   return ((v & 1) << 2) | (v >> 1);
+}
+
+// v where bit `bit` of word is set, else 0
+__device__ __forceinline__ float masked(float v, unsigned word, int bit) {
+  return __builtin_bit_cast(float, __builtin_bit_cast(int, v) & ((int)(word << (31 - bit)) >> 31));
 }
 
 // visibility bits [lo, hi) of a 32- or 64-wide index range (lo/hi may lie outside it)
@@ -596,18 +607,24 @@ __device__ __forceinline__ unsigned long long range_bits64(int lo, int hi) {
 // ---- dq kernel: forward structure, no online softmax --------------------------------------
 // K/V tiles of 64 keys run through a 3-deep LDS-DMA ring with counted vmcnt waits (as in the
 // forward kernel); masks are per-lane bit words, P is recomputed as exp2(fma(s, c, -lse*log2e)).
-__global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
-  constexpr int DH = 64, RB = 128, TILE = 64 * RB, NS = 3, KPW = 256;
-  __shared__ __attribute__((aligned(16))) char smem[2 * NS * TILE + KPW * 8 + 32];  // K ring, V ring, key-padding words, their ends
+// PAIR: two waves have the same 32 queries; each takes 32 keys of a tile up to dS, the dS are exchanged through LDS, and each sums
+// one 32-wide half of d, in the order of a wave that does all of it.  Where workgroups are few a wave has its SIMD to itself and a
+// tile takes what one wave issues for it (about 1.2 us) however little the matrix cores are used: 12 heads x 5 x 333 14.1 -> 12.0 us.
+template <bool PAIR>
+__global__ __launch_bounds__(256, PAIR ? 2 : 3) void attn_bwd_dq_kernel(BwdParams p) {
+  constexpr int DH = 64, RB = 128, TILE = 64 * RB, NS = 3, KPW = 256, ROWS = PAIR ? 64 : 128;
+  constexpr int XCH = 2 * NS * TILE + KPW * 8 + 32;   // PAIR: dS of [query group][key block][k-step], 1 KiB each
+  __shared__ __attribute__((aligned(16))) char smem[XCH + (PAIR ? 8192 : 0)];  // K ring, V ring, key-padding words, their ends
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int nqb = (p.L + 127) / 128;
+  const int qw = PAIR ? wave >> 1 : wave, half = PAIR ? wave & 1 : 0;   // the wave's 32 queries; of a pair, its key block and d block
+  const int nqb = (p.L + ROWS - 1) / ROWS;
   const int qb = nqb - 1 - (int)blockIdx.y;  // grid (h*B, query blocks): heaviest blocks of ALL heads first
   const int head = (int)blockIdx.x % p.h, b = (int)blockIdx.x / p.h;
   const int kvh = head / (p.h / p.hk);
-  const int q0 = qb * 128;
+  const int q0 = qb * ROWS;
   const int fr = lane & 31, fh = lane >> 5;
-  const int qi = q0 + wave * 32 + fr;
+  const int qi = q0 + qw * 32 + fr;
   const int qrow = qi < p.L ? qi : p.L - 1;
   const bf16* Q = p.q + (int64_t)b * p.q_sb + (int64_t)head * p.q_sh + (int64_t)qrow * p.q_sl;
   const bf16* dO = p.dout + (int64_t)b * p.o_sb + (int64_t)qrow * p.o_sl + head * DH;
@@ -622,6 +639,9 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
   const int64_t stat = ((int64_t)b * p.h + head) * p.L + qrow;
   const float c = p.scale * LOG2E;
   float neg_lse = -p.lse[stat] * LOG2E;  // p = exp2(c*s + neg_lse)
+  const bool rotates = p.cos_tab != nullptr;
+  f32x4 rc[4], rs[4];
+  if (PAIR && half == 0 && rotates) rope_bwd_tables(p, (int64_t)p.rope_pos0 + qrow, fh, rc, rs);   // (registers to spare)
   // -delta = -sum_d dO*O of this lane's query row: the dO fragments are already here, O costs four
   // more 16-byte loads, the two lane halves (d 8fh..8fh+7 of every 16) are added by one exchange.
   // Written to the workspace for the dK/dV kernel, which is launched after this one.
@@ -637,7 +657,7 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
     }
     acc_ += __shfl_xor(acc_, 32, 64);
     neg_delta = -acc_;
-    if (fh == 0 && qi < p.L) p.delta[stat] = neg_delta;
+    if (fh == 0 && half == 0 && qi < p.L) p.delta[stat] = neg_delta;
   }
   const bool causal = p.mask_kind & VY_MASK_CAUSAL;
   const bool haskp = p.mask_kind & VY_MASK_KEYPAD;
@@ -665,6 +685,12 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
     }
   };
   const int k_sw = dual_sw(fr), v_sw = (fr >> 1) & 7;
+  unsigned row_lds[2][4];   // PAIR: row fragments of the wave's 32 keys, ring buffer 0
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) {
+    row_lds[0][ks] = vy_lds_addr(smem) + (32 * half + fr) * RB + (((2 * ks + fh) ^ k_sw) << 4);
+    row_lds[1][ks] = vy_lds_addr(smem) + (32 * half + fr) * RB + (((2 * ks + fh) ^ v_sw) << 4);
+  }
   const int li = lane & 15, g16 = (lane >> 4) & 1;
   const int t_row = 4 * fh + (li >> 2);
   const int t_chunk = 2 * g16 + ((li & 3) >> 1), t_byte = 8 * (li & 1);
@@ -684,8 +710,8 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
     for (int r = 0; r < 16; ++r) dq[n][r] = 0.f;
 
   int nt = (p.S + 63) / 64;
-  if (causal) nt = max(1, min(nt, (min(p.S, p.start_pos + q0 + 128) + 63) / 64));
-  const int wave_first = q0 + wave * 32, wave_last = wave_first + 31;
+  if (causal) nt = max(1, min(nt, (min(p.S, p.start_pos + q0 + ROWS) + 63) / 64));
+  const int wave_first = q0 + qw * 32, wave_last = wave_first + 31;
 
   // only the tiles from the first with a visible key to the last: hidden keys pass nothing on (with the dK/dV kernel's hidden blocks,
   // 61 sequences of 167 .. 500 of 500 tokens, 12 heads: 258 -> 219 us for both kernels; 16 of 600 .. 2000 834 -> 657)
@@ -713,28 +739,42 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
     nt = __builtin_amdgcn_readfirstlane(max(max(ends[4], ends[5]), max(ends[6], ends[7])));   // (no visible key: 0, below u0)
   }
 
-  auto compute = [&](int tile, int buf) {
+  auto compute = [&](int tile, int buf, bool more) {
     const int k0 = tile * 64;
-    if (causal && k0 > p.start_pos + wave_last) return;
+    const bool hidden = causal && k0 > p.start_pos + wave_last;
+    if (!PAIR && hidden) return;
     const char* kb_ = smem + buf * TILE;
     const char* vb_ = smem + (NS + buf) * TILE;
     unsigned long long vis = ~0ull;
-    if (haskp) vis = kpbits[tile];
+    if (haskp) {
+      const unsigned long long bits = kpbits[tile];   // (the same in every lane)
+      vis = (unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(bits >> 32)) << 32 |
+            (unsigned)__builtin_amdgcn_readfirstlane((int)bits);
+    }
     const bool need_mask = (k0 + 64 > p.S) || (causal && k0 + 63 > p.start_pos + wave_first) || vis != ~0ull;
     // key of register r: k0 + 4fh + kofs, kofs = 32kb + (r&3) + 8(r>>2); visible iff kofs <= klim
     int klim = p.S - 1 - k0 - 4 * fh;
     if (causal) klim = min(klim, qi + p.start_pos - k0 - 4 * fh);
     const unsigned long long lm = need_mask ? (range_bits64(0, klim + 1) & (vis >> (4 * fh))) : ~0ull;
     const unsigned lmw[2] = {(unsigned)lm, (unsigned)(lm >> 32)};
-    // one 32-key block at a time: scores and dP of a block are turned into dS (8 registers) before the next block's
-    // accumulators exist -- both blocks' st / dp tiles live at once cost 32 more registers, the difference between two
-    // and three waves per SIMD
-    bf16x8 ds[2][2];
-#pragma unroll
-    for (int kb = 0; kb < 2; ++kb) {
-      f32x16 st, dp;
+    auto products = [&](int kb, f32x16& st, f32x16& dp) {
 #pragma unroll
       for (int r = 0; r < 16; ++r) { st[r] = 0.f; dp[r] = neg_delta; }
+      if constexpr (PAIR) {   // all requested at once: one wave on a SIMD waits for each pair by itself otherwise
+        bf16x8 kf[4], vf[4];
+        vy_static_for<4>([&](auto i_c) {
+          constexpr int i = decltype(i_c)::value;
+          kf[i] = vy_lds_read128_off<0>(row_lds[0][i] + buf * TILE);
+          vf[i] = vy_lds_read128_off<NS * TILE>(row_lds[1][i] + buf * TILE);
+        });
+        vy_static_for<4>([&](auto i_c) {
+          constexpr int i = decltype(i_c)::value;
+          vy_lgkm_wait<6 - 2 * i>(kf[i], vf[i]);
+          st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf[i], qf[i], st, 0, 0, 0);
+          dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf[i], gf[i], dp, 0, 0, 0);
+        });
+        return;
+      }
 #pragma unroll
       for (int ks = 0; ks < 4; ++ks) {
         const bf16x8 kf = *reinterpret_cast<const bf16x8*>(kb_ + (32 * kb + fr) * RB + (((2 * ks + fh) ^ k_sw) << 4));
@@ -742,12 +782,58 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
         st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kf, qf[ks], st, 0, 0, 0);
         dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(vf, gf[ks], dp, 0, 0, 0);
       }
+    };
+    auto score_grads = [&](unsigned visible, const f32x16& st, const f32x16& dp, bf16x8 (&ds)[2]) {
+      if (!PAIR || need_mask) {
 #pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        float pr = __builtin_amdgcn_exp2f(fmaf(st[r], c, neg_lse));
-        pr = ((lmw[kb] >> ((r & 3) + 8 * (r >> 2))) & 1u) ? pr : 0.f;
-        ds[kb][r >> 3][r & 7] = (bf16)(pr * dp[r]);
+        for (int r = 0; r < 16; ++r) {
+          const float pr = masked(__builtin_amdgcn_exp2f(fmaf(st[r], c, neg_lse)), visible, (r & 3) + 8 * (r >> 2));
+          ds[r >> 3][r & 7] = (bf16)(pr * dp[r]);
+        }
+      } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) ds[r >> 3][r & 7] = (bf16)(__builtin_amdgcn_exp2f(fmaf(st[r], c, neg_lse)) * dp[r]);
       }
+    };
+    if constexpr (PAIR) {
+      f32x16 st, dp;
+      bf16x8 ds[2][2], kfr[4];
+      const unsigned xch = vy_lds_addr(smem) + XCH + qw * 4096 + lane * 16;
+      if (!hidden) products(half, st, dp);
+      if (more) stage(tile + NS - 1, buf ? buf - 1 : NS - 1);
+      const unsigned kbase[2] = {k_lds[half][0] + buf * TILE, k_lds[half][1] + buf * TILE};
+      vy_static_for<4>([&](auto f_c) {
+        constexpr int f = decltype(f_c)::value, ro = 16 * f * RB;
+        union { struct { s16x4 a, b; } s_; bf16x8 v; } u;
+        u.s_.a = vy_lds_tr16_off<ro>(kbase[0]);
+        u.s_.b = vy_lds_tr16_off<ro>(kbase[1]);
+        kfr[f] = u.v;
+      });
+      if (!hidden) {
+        score_grads(half ? lmw[1] : lmw[0], st, dp, ds[0]);
+#pragma unroll
+        for (int j = 0; j < 2; ++j) *reinterpret_cast<bf16x8*>(smem + XCH + qw * 4096 + (half * 2 + j) * 1024 + lane * 16) = ds[0][j];
+      }
+      vy_lgkm_wait<0>(kfr[0], kfr[1], kfr[2], kfr[3]);
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (!hidden) {
+        vy_static_for<4>([&](auto f_c) { constexpr int f = decltype(f_c)::value; ds[f >> 1][f & 1] = vy_lds_read128_off<f * 1024>(xch); });
+        vy_lgkm_wait<0>(ds[0][0], ds[0][1], ds[1][0], ds[1][1]);
+#pragma unroll
+        for (int f = 0; f < 4; ++f) dq[0] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(kfr[f], ds[f >> 1][f & 1], dq[0], 0, 0, 0);
+      }
+      return;
+    }
+    // one 32-key block at a time: scores and dP of a block are turned into dS (8 registers) before the next block's
+    // accumulators exist -- both blocks' st / dp tiles live at once cost 32 more registers, the difference between two
+    // and three waves per SIMD
+    bf16x8 ds[2][2];
+#pragma unroll
+    for (int kb = 0; kb < 2; ++kb) {
+      f32x16 st, dp;
+      products(kb, st, dp);
+      score_grads(lmw[kb], st, dp, ds[kb]);
     }
     // dQ^T[d][q] += K^T[d][key] . dS^T[key][q]; K^T fragments by asm transposing reads, one ahead.
     // Base addresses per (d block, row / row+8); key block and k-step go into the offset field.
@@ -787,14 +873,29 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) { vy_tie(qf[ks]); vy_tie(gf[ks]); }
   vy_tie(neg_lse); vy_tie(neg_delta);
+  int buf = 0;
   for (int t = u0; t < nt; ++t) {
     if (t + 1 < nt) asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (t + NS - 1 < nt) stage(t + NS - 1, (t - u0 + NS - 1) % NS);
-    compute(t, (t - u0) % NS);
+    const bool more = t + NS - 1 < nt;
+    if (!PAIR && more) stage(t + NS - 1, buf ? buf - 1 : NS - 1);
+    compute(t, buf, more);
+    buf = buf + 1 < NS ? buf + 1 : 0;
   }
+  if constexpr (PAIR) {   // (the rotation needs both d blocks in one lane)
+    float* other = reinterpret_cast<float*>(smem + XCH + qw * 4096) + lane;
+    __syncthreads();
+    if (half == 1)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) other[64 * r] = dq[0][r];
+    __syncthreads();
+    if (half == 1) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) dq[1][r] = other[64 * r];
+  }
+  if (!PAIR && rotates) rope_bwd_tables(p, (int64_t)p.rope_pos0 + qrow, fh, rc, rs);
   if (qi < p.L) {
     bf16* D = p.dq + (int64_t)b * p.dq_sb + (int64_t)head * p.dq_sh + (int64_t)qi * p.dq_sl;
 #pragma unroll
@@ -802,7 +903,7 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
       float lo[4], hi[4];
 #pragma unroll
       for (int e = 0; e < 4; ++e) { lo[e] = dq[0][4 * rg + e] * p.scale; hi[e] = dq[1][4 * rg + e] * p.scale; }
-      if (p.cos_tab) rope_bwd_quad(p, (int64_t)p.rope_pos0 + qi, 8 * rg + 4 * fh, lo, hi);
+      if (rotates) rope_bwd_quad(rc[rg], rs[rg], lo, hi);
       bf16x4 wl, wh;
 #pragma unroll
       for (int e = 0; e < 4; ++e) { wl[e] = (bf16)lo[e]; wh[e] = (bf16)hi[e]; }
@@ -818,17 +919,27 @@ __global__ __launch_bounds__(256, 3) void attn_bwd_dq_kernel(BwdParams p) {
 // tile).  Q and dO tiles are staged by LDS-DMA into dual-use images (row + transposed reads)
 // through a 3-deep ring; the tile's row statistics (lse, -delta) ride along as one 4-byte-per-lane
 // LDS-DMA per wave, so the loop holds no ordinary load and is paced by counted vmcnt waits only.
-__global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
-  constexpr int DH = 64, RB = 128, QR = 64, QT = QR * RB, NS = 3;  // one 64-row tile = 8 KiB
-  constexpr int ST_OFF = 2 * NS * QT;                              // NS x [lse 64 floats][-delta 64 floats]
-  __shared__ __attribute__((aligned(16))) char smem[2 * NS * QT + NS * 512 + 16];   // .., a word per wave
+// What a tile costs beside its products: the addresses of the next one (kept as running pointers) and the waits for its fragments
+// (requested all at once); 32 x 512, 12 heads: 72.2 -> 63.8 us, rotation included.
+// SPLIT 2 or 4: that many waves have the same 32 keys; each takes 32 of a tile's 64 or 128 rows up to P and dS, these are exchanged
+// through LDS, and each wave sums dV (even ones) or dK (odd ones), of 4 one 32-wide half of d, in the order of a wave that does all
+// of it.  A sweep is a chain of tiles of about 1.4 us each where a wave has its SIMD to itself (by what it issues, the products are
+// a third); with two waves it is 1.0 us, with four 1.0 us for twice the rows: 4 kv heads of 12, 5 x 333: 35.4 -> 17.2 us.
+template <int SPLIT>
+__global__ __launch_bounds__(256, SPLIT == 4 ? 1 : 2) void attn_bwd_dkdv_kernel(BwdParams p) {
+  constexpr int DH = 64, RB = 128, QR = SPLIT == 4 ? 128 : 64, QT = QR * RB, NS = 3, PIECES = QR / 32;
+  constexpr int KEYS = 128 / SPLIT, NR = SPLIT == 4 ? 1 : 2;       // keys of a workgroup; 32-wide parts of d that a wave sums
+  constexpr int ST_OFF = 2 * NS * QT, SB = QR * 8;                 // NS x [lse of the rows][-delta of the rows]
+  constexpr int XCH = ST_OFF + NS * SB + 16;                       // SPLIT: [32 keys][P, dS][32 rows][k-step], 1 KiB each
+  __shared__ __attribute__((aligned(16))) char smem[XCH + (SPLIT > 1 ? 16384 : 0)];   // .., a word per wave, ..
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int kw = wave / SPLIT, part = wave % SPLIT;
   // grid (hk*B, key blocks): key block 0 sees every query row under a causal mask -> all of them first
   const int kblk = blockIdx.y, kvh = (int)blockIdx.x % p.hk, b = (int)blockIdx.x / p.hk;
   const int n_rep = p.h / p.hk;
   const int fr = lane & 31, fh = lane >> 5;
-  const int key0 = kblk * 128 + wave * 32;
+  const int key0 = kblk * KEYS + kw * 32;
   const int kj = key0 + fr;                       // this lane's key (column of S)
   const int krow = kj < p.S ? kj : p.S - 1;
   const bf16* Kp = p.k + (int64_t)b * p.k_sb + (int64_t)kvh * p.k_sh + (int64_t)krow * p.k_sl;
@@ -842,20 +953,14 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
   const bool causal = p.mask_kind & VY_MASK_CAUSAL;
   const bool haskp = p.mask_kind & VY_MASK_KEYPAD;
   const bool key_dead = (kj >= p.S) || (haskp && !p.keypad[(int64_t)b * p.kp_sb + krow]);
-  const bool any_dead = __any(key_dead), all_dead = __all(key_dead);
-  // hidden keys get zero gradients: a block of them sweeps no query row, a wave of them multiplies nothing
-  bool block_dead = false;
-  if (haskp) {
-    int* dead = reinterpret_cast<int*>(smem + ST_OFF + NS * 512);
-    if (lane == 0) dead[wave] = all_dead;
-    __syncthreads();
-    block_dead = __builtin_amdgcn_readfirstlane(dead[0] & dead[1] & dead[2] & dead[3]) != 0;
-  }
+  const bool rotates = (SPLIT == 1 || (part & 1)) && p.cos_tab;
+  f32x4 rc[4], rs[4];
+  if (SPLIT > 1 && rotates) rope_bwd_tables(p, (int64_t)p.rope_pos0 + krow, fh, rc, rs);   // (registers to spare)
   const float c = p.scale * LOG2E;
 
-  f32x16 dk[2], dv[2];
+  f32x16 dk[NR], dv[NR];   // (SPLIT: an odd wave's dv is dK)
 #pragma unroll
-  for (int n = 0; n < 2; ++n)
+  for (int n = 0; n < NR; ++n)
 #pragma unroll
     for (int r = 0; r < 16; ++r) { dk[n][r] = 0.f; dv[n][r] = 0.f; }
 
@@ -863,113 +968,191 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
   const int nqt = (p.L + QR - 1) / QR;
   int qt_first = 0;
   if (causal) {
-    const int first_row = kblk * 128 - p.start_pos;
+    const int first_row = kblk * KEYS - p.start_pos;
     qt_first = first_row > 0 ? first_row / QR : 0;
   }
-  const int per_head = nqt > qt_first && !block_dead ? nqt - qt_first : 0;
-  const int total = per_head * n_rep;
+  int total = max(nqt - qt_first, 0) * n_rep;
 
-  // LDS-DMA: tile = 8 pieces of 1 KiB; wave w loads pieces 2w, 2w+1 of the Q tile and of the dO tile
-  int ld_row[2], ld_eoff[2];
+  // LDS-DMA: a tile is QR / 8 pieces of 1 KiB; each wave loads PIECES of the Q tile and of the dO tile
+  int ld_row[PIECES], ld_eoff[PIECES];
+  unsigned q_off[PIECES], g_off[PIECES];   // a lane's bytes of a whole tile, from its first row
+  const bool near = p.q_sl < (1 << 24) && p.o_sl < (1 << 24);   // (a tile's rows within 32 bits)
 #pragma unroll
-  for (int t = 0; t < 2; ++t) {
-    const int P = (wave * 2 + t) * 1024 + lane * 16;
+  for (int t = 0; t < PIECES; ++t) {
+    const int P = (wave * PIECES + t) * 1024 + lane * 16;
     const int row = P / RB, off = P % RB;
     ld_row[t] = row;
     ld_eoff[t] = (((off >> 4) ^ dual_sw(row)) << 4) >> 1;
+    q_off[t] = 2 * (row * (unsigned)p.q_sl + ld_eoff[t]);
+    g_off[t] = 2 * (row * (unsigned)p.o_sl + ld_eoff[t]);
   }
-  const float* stat_src = (wave & 1) ? p.delta : p.lse;
-  auto stage = [&](int it, int buf) {
-    const int hh = it / per_head, qt = qt_first + (it - hh * per_head);
-    const int head = kvh * n_rep + hh;
+  // row statistics: even waves bring lse, odd waves -delta, 64 rows each (of 64 rows both pairs write the same bytes)
+  const int st_row = (SPLIT == 4 ? wave >> 1 : 0) * 64;
+  // the tile to be staged next, head by head, rows from the first one
+  int next_row = qt_first * QR;
+  const int64_t back = (int64_t)(nqt - 1 - qt_first) * QR;   // from a head's last tile to its first
+  const char* Qt = reinterpret_cast<const char*>(p.q + (int64_t)b * p.q_sb + (int64_t)kvh * n_rep * p.q_sh + next_row * p.q_sl);
+  const char* Gt = reinterpret_cast<const char*>(p.dout + (int64_t)b * p.o_sb + kvh * n_rep * DH + next_row * p.o_sl);
+  const float* St = ((wave & 1) ? p.delta : p.lse) + ((int64_t)b * p.h + kvh * n_rep) * p.L + next_row;
+  auto stage = [&](int buf) {
+    char* qd = smem + buf * QT + wave * PIECES * 1024;
+    char* gd = smem + (NS + buf) * QT + wave * PIECES * 1024;
+    if (near && next_row + QR <= p.L) {
 #pragma unroll
-    for (int t = 0; t < 2; ++t) {
-      int qr = qt * QR + ld_row[t];
-      qr = qr < p.L ? qr : p.L - 1;
-      const bf16* qs = p.q + (int64_t)b * p.q_sb + (int64_t)head * p.q_sh + (int64_t)qr * p.q_sl + ld_eoff[t];
-      const bf16* gs = p.dout + (int64_t)b * p.o_sb + (int64_t)qr * p.o_sl + head * DH + ld_eoff[t];
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)qs, (VY_LDS void*)(smem + buf * QT + (wave * 2 + t) * 1024), 16, 0, 0);
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)gs, (VY_LDS void*)(smem + (NS + buf) * QT + (wave * 2 + t) * 1024), 16, 0, 0);
+      for (int t = 0; t < PIECES; ++t) {
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(Qt + q_off[t]), (VY_LDS void*)(qd + t * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(Gt + g_off[t]), (VY_LDS void*)(gd + t * 1024), 16, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int t = 0; t < PIECES; ++t) {
+        const int64_t qr = min(ld_row[t], p.L - 1 - next_row);
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(Qt + 2 * (qr * p.q_sl + ld_eoff[t])), (VY_LDS void*)(qd + t * 1024), 16, 0, 0);
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(Gt + 2 * (qr * p.o_sl + ld_eoff[t])), (VY_LDS void*)(gd + t * 1024), 16, 0, 0);
+      }
     }
-    // row statistics: even waves bring lse, odd waves -delta (both pairs write the same bytes)
-    int sr = qt * QR + lane;
-    sr = sr < p.L ? sr : p.L - 1;
-    __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(stat_src + ((int64_t)b * p.h + head) * p.L + sr),
-                                     (VY_LDS void*)(smem + ST_OFF + buf * 512 + (wave & 1) * 256), 4, 0, 0);
+    __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)(St + min(st_row + lane, p.L - 1 - next_row)),
+                                     (VY_LDS void*)(smem + ST_OFF + buf * SB + (wave & 1) * QR * 4 + st_row * 4), 4, 0, 0);
+    next_row += QR;
+    const bool wrap = next_row >= p.L;
+    Qt += 2 * (wrap ? p.q_sh - back * p.q_sl : QR * p.q_sl);
+    Gt += 2 * (wrap ? DH - back * p.o_sl : QR * p.o_sl);
+    St += wrap ? p.L - back : QR;
+    if (wrap) next_row = qt_first * QR;
   };
+#pragma unroll
+  for (int s_ = 0; s_ < NS - 1; ++s_)
+    if (s_ < total) stage(s_);
+  const bool any_dead = __any(key_dead), all_dead = __all(key_dead);
   const int r_sw = dual_sw(fr);
   const int li = lane & 15, g16 = (lane >> 4) & 1;
   const int t_row = 4 * fh + (li >> 2);
   const int t_chunk = 2 * g16 + ((li & 3) >> 1), t_byte = 8 * (li & 1);
-  unsigned t_lds[2][2];  // transposed fragment of d block n, rows t_row (+8), ring buffer 0
+  unsigned t_lds[NR][2];  // transposed fragment of d block n, rows t_row (+8), ring buffer 0 (SPLIT: of the wave's operand)
 #pragma unroll
-  for (int n = 0; n < 2; ++n)
+  for (int n = 0; n < NR; ++n)
 #pragma unroll
     for (int u = 0; u < 2; ++u) {
-      const int row = t_row + 8 * u;
-      t_lds[n][u] = vy_lds_addr(smem) + row * RB + (((4 * n + t_chunk) ^ dual_sw(row)) << 4) + t_byte;
+      const int row = t_row + 8 * u, d = NR == 2 ? n : part >> 1;
+      t_lds[n][u] = vy_lds_addr(smem) + row * RB + (((4 * d + t_chunk) ^ dual_sw(row)) << 4) + t_byte;
+      if (SPLIT > 1 && (part & 1) == 0) t_lds[n][u] += NS * QT;
     }
 
-  auto compute = [&](int it, int buf) {
+  // register r <-> query row qbase + (r&3) + 8(r>>2) + 4fh: row constants straight from LDS.  All the reads of a block are requested
+  // at once and awaited one pair at a time (left to the compiler, each pair is requested when the one before has arrived).
+  unsigned row_lds[4];
+  const unsigned stat_lds = vy_lds_addr(smem) + ST_OFF + 128 * part + 16 * fh;
+#pragma unroll
+  for (int ks = 0; ks < 4; ++ks) row_lds[ks] = vy_lds_addr(smem) + (32 * part + fr) * RB + (((2 * ks + fh) ^ r_sw) << 4);
+  auto products = [&](auto blk_c, int buf, f32x16& st, f32x16& dp, f32x16& nl) {
+    constexpr int blk = decltype(blk_c)::value;   // (SPLIT: 0, the wave's block lies in the addresses)
+    const unsigned sa = stat_lds + buf * SB;
+    bf16x8 d4[4], l4[4], qa[4], ga[4];
+    vy_static_for<4>([&](auto i_c) { constexpr int i = decltype(i_c)::value; d4[i] = vy_lds_read128_off<QR * 4 + 128 * blk + 32 * i>(sa); });
+    vy_static_for<4>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      qa[i] = vy_lds_read128_off<32 * blk * RB>(row_lds[i] + buf * QT);
+      ga[i] = vy_lds_read128_off<32 * blk * RB + NS * QT>(row_lds[i] + buf * QT);
+    });
+    vy_static_for<4>([&](auto i_c) { constexpr int i = decltype(i_c)::value; l4[i] = vy_lds_read128_off<128 * blk + 32 * i>(sa); });
+    vy_lgkm_wait<10>(d4[0], d4[1], d4[2], d4[3], qa[0], ga[0]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+      st[r] = 0.f;
+      dp[r] = __builtin_bit_cast(f32x4, d4[r >> 2])[r & 3];
+    }
+    vy_static_for<4>([&](auto i_c) {
+      constexpr int i = decltype(i_c)::value;
+      if constexpr (i > 0) vy_lgkm_wait<10 - 2 * i>(qa[i], ga[i]);
+      st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa[i], kf[i], st, 0, 0, 0);
+      dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga[i], vf[i], dp, 0, 0, 0);
+    });
+    vy_lgkm_wait<0>(l4[0], l4[1], l4[2], l4[3]);
+#pragma unroll
+    for (int r = 0; r < 16; ++r) nl[r] = __builtin_bit_cast(f32x4, l4[r >> 2])[r & 3] * -LOG2E;
+  };
+  auto score_grads = [&](int qbase, const f32x16& st, const f32x16& dp, const f32x16& nl, bf16x8 (&pf)[2], bf16x8 (&dsf)[2]) {
+    const bool need_mask = any_dead || qbase + 32 > p.L || (causal && key0 + 31 > qbase + p.start_pos);
+    if (need_mask) {
+      // rows of this block the lane's key may see: [kj - start_pos - qbase, L - qbase)
+      unsigned rm = (unsigned)range_bits64(causal ? kj - p.start_pos - qbase : 0, min(32, p.L - qbase));
+      rm = key_dead ? 0u : rm >> (4 * fh);
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float pr = masked(__builtin_amdgcn_exp2f(fmaf(st[r], c, nl[r])), rm, (r & 3) + 8 * (r >> 2));
+        pf[r >> 3][r & 7] = (bf16)pr;
+        dsf[r >> 3][r & 7] = (bf16)(pr * dp[r]);
+      }
+    } else {
+#pragma unroll
+      for (int r = 0; r < 16; ++r) {
+        const float pr = __builtin_amdgcn_exp2f(fmaf(st[r], c, nl[r]));
+        pf[r >> 3][r & 7] = (bf16)pr;
+        dsf[r >> 3][r & 7] = (bf16)(pr * dp[r]);
+      }
+    }
+  };
+  // wave-uniform skips: block beyond L, or every key of this wave above the block's last diagonal
+  auto skips = [&](int qbase) { return qbase >= p.L || (causal && key0 > qbase + 31 + p.start_pos); };
+
+  auto compute_split = [&](int row0, int buf, bool more) {
+    const bool mine = !all_dead && !skips(row0 + 32 * part);
+    f32x16 st, dp, nl;
+    if (mine) products(std::integral_constant<int, 0>{}, buf, st, dp, nl);
+    if (more) stage(buf ? buf - 1 : NS - 1);
+    bf16x8 fr_[8];   // [32 rows][d block][k-step]
+    vy_static_for<8>([&](auto f_c) {
+      constexpr int f = decltype(f_c)::value, n = NR == 2 ? (f >> 1) & 1 : 0, ro = (32 * (f / (2 * NR)) + 16 * (f & 1)) * RB;
+      union { struct { s16x4 a, b; } s_; bf16x8 v; } u;
+      u.s_.a = vy_lds_tr16_off<ro>(t_lds[n][0] + buf * QT);
+      u.s_.b = vy_lds_tr16_off<ro>(t_lds[n][1] + buf * QT);
+      fr_[f] = u.v;
+    });
+    if (mine) {
+      bf16x8 pf[2], dsf[2];
+      score_grads(row0 + 32 * part, st, dp, nl, pf, dsf);
+      char* x = smem + XCH + kw * SPLIT * 4096 + part * 2048 + lane * 16;
+#pragma unroll
+      for (int j = 0; j < 2; ++j) {
+        *reinterpret_cast<bf16x8*>(x + j * 1024) = pf[j];
+        *reinterpret_cast<bf16x8*>(x + SPLIT * 2048 + j * 1024) = dsf[j];
+      }
+    }
+    vy_lgkm_wait<0>(fr_[0], fr_[1], fr_[2], fr_[3], fr_[4], fr_[5], fr_[6], fr_[7]);
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    const unsigned xch = vy_lds_addr(smem) + XCH + kw * SPLIT * 4096 + (part & 1) * SPLIT * 2048 + lane * 16;
+    bf16x8 g[2 * SPLIT];
+    vy_static_for<2 * SPLIT>([&](auto f_c) { constexpr int f = decltype(f_c)::value; g[f] = vy_lds_read128_off<f * 1024>(xch); });
+    vy_static_for<SPLIT>([&](auto blk_c) {
+      constexpr int blk = decltype(blk_c)::value;
+      vy_lgkm_wait<2 * (SPLIT - 1 - blk)>(g[2 * blk], g[2 * blk + 1]);
+      if (all_dead || skips(row0 + 32 * blk)) return;
+#pragma unroll
+      for (int j = 0; j < 2; ++j)
+#pragma unroll
+        for (int n = 0; n < NR; ++n)
+          dv[n] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(fr_[blk * 2 * NR + n * 2 + j], g[2 * blk + j], dv[n], 0, 0, 0);
+    });
+  };
+  auto compute = [&](int row0, int buf) {
     if (all_dead) return;
-    const int hh = it / per_head, qt = qt_first + (it - hh * per_head);
-    const char* qb_ = smem + buf * QT;
-    const char* gb_ = smem + (NS + buf) * QT;
-    const float* stl = reinterpret_cast<const float*>(smem + ST_OFF + buf * 512);
     unsigned qbase_[2][2], gbase[2][2];  // transposed-read bases of this buffer (Q ring / dO ring)
 #pragma unroll
     for (int n = 0; n < 2; ++n)
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        qbase_[n][u] = t_lds[n][u] + buf * QT;
-        gbase[n][u] = t_lds[n][u] + (NS + buf) * QT;
+        qbase_[n][u] = t_lds[n % NR][u] + buf * QT;
+        gbase[n][u] = t_lds[n % NR][u] + (NS + buf) * QT;
       }
-#pragma unroll
-    for (int blk = 0; blk < 2; ++blk) {
-      const int qbase = qt * QR + 32 * blk;
-      // wave-uniform skips: block beyond L, or every key of this wave above the block's last diagonal
-      if (qbase >= p.L || (causal && key0 > qbase + 31 + p.start_pos)) continue;
-      // register r <-> query row qbase + (r&3) + 8(r>>2) + 4fh: row constants straight from LDS
+    vy_static_for<2>([&](auto blk_c) {
+      constexpr int blk = decltype(blk_c)::value;
+      const int qbase = row0 + 32 * blk;
+      if (skips(qbase)) return;
       f32x16 st, dp, nl;
-#pragma unroll
-      for (int rg = 0; rg < 4; ++rg) {
-        const f32x4 l4 = *reinterpret_cast<const f32x4*>(stl + 32 * blk + 8 * rg + 4 * fh);
-        const f32x4 d4 = *reinterpret_cast<const f32x4*>(stl + 64 + 32 * blk + 8 * rg + 4 * fh);
-#pragma unroll
-        for (int e = 0; e < 4; ++e) {
-          st[4 * rg + e] = 0.f;
-          nl[4 * rg + e] = l4[e] * -LOG2E;
-          dp[4 * rg + e] = d4[e];
-        }
-      }
-#pragma unroll
-      for (int ks = 0; ks < 4; ++ks) {
-        const bf16x8 qa = *reinterpret_cast<const bf16x8*>(qb_ + (32 * blk + fr) * RB + (((2 * ks + fh) ^ r_sw) << 4));
-        const bf16x8 ga = *reinterpret_cast<const bf16x8*>(gb_ + (32 * blk + fr) * RB + (((2 * ks + fh) ^ r_sw) << 4));
-        st = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qa, kf[ks], st, 0, 0, 0);
-        dp = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ga, vf[ks], dp, 0, 0, 0);
-      }
-      const bool need_mask = any_dead || qbase + 32 > p.L || (causal && key0 + 31 > qbase + p.start_pos);
       bf16x8 pf[2], dsf[2];
-      if (need_mask) {
-        // rows of this block the lane's key may see: [kj - start_pos - qbase, L - qbase)
-        unsigned rm = (unsigned)range_bits64(causal ? kj - p.start_pos - qbase : 0, min(32, p.L - qbase));
-        rm = key_dead ? 0u : rm >> (4 * fh);
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          float pr = __builtin_amdgcn_exp2f(fmaf(st[r], c, nl[r]));
-          pr = ((rm >> ((r & 3) + 8 * (r >> 2))) & 1u) ? pr : 0.f;
-          pf[r >> 3][r & 7] = (bf16)pr;
-          dsf[r >> 3][r & 7] = (bf16)(pr * dp[r]);
-        }
-      } else {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const float pr = __builtin_amdgcn_exp2f(fmaf(st[r], c, nl[r]));
-          pf[r >> 3][r & 7] = (bf16)pr;
-          dsf[r >> 3][r & 7] = (bf16)(pr * dp[r]);
-        }
-      }
+      products(blk_c, buf, st, dp, nl);
+      score_grads(qbase, st, dp, nl, pf, dsf);
       // dV^T[d][key] += dO^T[d][q] . P[q][key];   dK^T[d][key] += Q^T[d][q] . dS[q][key]
       auto frag = [&](auto f_c, const unsigned (&base)[2][2]) {
         constexpr int f = decltype(f_c)::value;
@@ -991,45 +1174,85 @@ __global__ __launch_bounds__(256, 2) void attn_bwd_dkdv_kernel(BwdParams p) {
         } else {
           vy_lgkm_wait<0>(gfr[f & 1], qfr[f & 1]);
         }
-        dv[f >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gfr[f & 1], pf[f & 1], dv[f >> 1], 0, 0, 0);
-        dk[f >> 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfr[f & 1], dsf[f & 1], dk[f >> 1], 0, 0, 0);
+        dv[(f >> 1) % NR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(gfr[f & 1], pf[f & 1], dv[(f >> 1) % NR], 0, 0, 0);
+        dk[(f >> 1) % NR] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(qfr[f & 1], dsf[f & 1], dk[(f >> 1) % NR], 0, 0, 0);
       };
       vy_static_for<4>(step);
-    }
+    });
   };
 
-#pragma unroll
-  for (int s_ = 0; s_ < NS - 1; ++s_)
-    if (s_ < total) stage(s_, s_);
+  // hidden keys get zero gradients: a block of them sweeps no query row, a wave of them multiplies nothing
+  if (haskp) {
+    int* dead = reinterpret_cast<int*>(smem + ST_OFF + NS * SB);
+    if (lane == 0) dead[wave] = all_dead;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (and not for the tiles under way)
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    if (__builtin_amdgcn_readfirstlane(dead[0] & dead[1] & dead[2] & dead[3])) {
+      total = 0;
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    }
+  }
 #pragma unroll
   for (int ks = 0; ks < 4; ++ks) { vy_tie(kf[ks]); vy_tie(vf[ks]); }
+  int buf = 0, row0 = qt_first * QR;
   for (int it = 0; it < total; ++it) {
-    if (it + 1 < total) asm volatile("s_waitcnt vmcnt(5)" ::: "memory");
+    if (it + 1 < total) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PIECES + 1) : "memory");
     else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (it + NS - 1 < total) stage(it + NS - 1, (it + NS - 1) % NS);
-    compute(it, it % NS);
+    const bool more = it + NS - 1 < total;
+    if constexpr (SPLIT > 1) {
+      compute_split(row0, buf, more);
+    } else {
+      if (more) stage(buf ? buf - 1 : NS - 1);
+      compute(row0, buf);
+    }
+    buf = buf + 1 < NS ? buf + 1 : 0;
+    row0 = row0 + QR < p.L ? row0 + QR : qt_first * QR;
+  }
+  if (SPLIT == 1 && rotates) rope_bwd_tables(p, (int64_t)p.rope_pos0 + krow, fh, rc, rs);
+  f32x16 hi;
+  if constexpr (SPLIT == 4) {   // (the rotation needs both parts of d in one lane)
+    float* other = reinterpret_cast<float*>(smem + XCH) + lane;
+    __syncthreads();
+    if (part == 3)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) other[64 * r] = dv[0][r];
+    __syncthreads();
+    if (part == 3) return;
+    if (part == 1)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) hi[r] = other[64 * r];
   }
   if (kj < p.S) {
     bf16* DK = p.dk + (int64_t)b * p.dk_sb + (int64_t)kvh * p.dk_sh + (int64_t)kj * p.dk_sl;
     bf16* DV = p.dv + (int64_t)b * p.dv_sb + (int64_t)kvh * p.dv_sh + (int64_t)kj * p.dv_sl;
+    if (SPLIT == 1 || (part & 1) == 1) {
+      const f32x16 &k_lo = SPLIT == 1 ? dk[0] : dv[0], &k_hi = SPLIT == 1 ? dk[NR - 1] : SPLIT == 2 ? dv[NR - 1] : hi;
 #pragma unroll
-    for (int rg = 0; rg < 4; ++rg) {
-      float lo[4], hi[4];
+      for (int rg = 0; rg < 4; ++rg) {
+        float lo[4], up[4];
 #pragma unroll
-      for (int e = 0; e < 4; ++e) { lo[e] = dk[0][4 * rg + e] * p.scale; hi[e] = dk[1][4 * rg + e] * p.scale; }
-      if (p.cos_tab) rope_bwd_quad(p, (int64_t)p.rope_pos0 + kj, 8 * rg + 4 * fh, lo, hi);
-      bf16x4 wl, wh, vl, vh;
+        for (int e = 0; e < 4; ++e) { lo[e] = k_lo[4 * rg + e] * p.scale; up[e] = k_hi[4 * rg + e] * p.scale; }
+        if (rotates) rope_bwd_quad(rc[rg], rs[rg], lo, up);
+        bf16x4 wl, wh;
 #pragma unroll
-      for (int e = 0; e < 4; ++e) {
-        wl[e] = (bf16)lo[e]; wh[e] = (bf16)hi[e];
-        vl[e] = (bf16)dv[0][4 * rg + e]; vh[e] = (bf16)dv[1][4 * rg + e];
+        for (int e = 0; e < 4; ++e) { wl[e] = (bf16)lo[e]; wh[e] = (bf16)up[e]; }
+        *reinterpret_cast<bf16x4*>(DK + 8 * rg + 4 * fh) = wl;
+        *reinterpret_cast<bf16x4*>(DK + 32 + 8 * rg + 4 * fh) = wh;
       }
-      *reinterpret_cast<bf16x4*>(DK + 8 * rg + 4 * fh) = wl;
-      *reinterpret_cast<bf16x4*>(DK + 32 + 8 * rg + 4 * fh) = wh;
-      *reinterpret_cast<bf16x4*>(DV + 8 * rg + 4 * fh) = vl;
-      *reinterpret_cast<bf16x4*>(DV + 32 + 8 * rg + 4 * fh) = vh;
+    }
+    if (SPLIT == 1 || (part & 1) == 0) {
+#pragma unroll
+      for (int n = 0; n < NR; ++n)
+#pragma unroll
+        for (int rg = 0; rg < 4; ++rg) {
+          bf16x4 w;
+#pragma unroll
+          for (int e = 0; e < 4; ++e) w[e] = (bf16)dv[n][4 * rg + e];
+          *reinterpret_cast<bf16x4*>(DV + 32 * (NR == 2 ? n : part >> 1) + 8 * rg + 4 * fh) = w;
+        }
     }
   }
 }
@@ -1853,9 +2076,23 @@ extern "C" int vy_attn_bwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_
   }
   // (delta = rowsum(dO * O) is computed by the dQ kernel for its own rows and left in delta_ws for the
   // dK/dV kernel; attn_delta_kernel remains for reference)
-  hipLaunchKernelGGL(attn_bwd_dq_kernel, dim3((unsigned)(h * B), (unsigned)((L + 127) / 128), 1), dim3(256), 0, st, p);
+  // with at most one workgroup a CU a wave has its SIMD to itself and the kernels are as long as one workgroup's chain: then the waves
+  // share the tiles (dQ by two, dK/dV by two or four; 4 needs more than one tile of rows and all its workgroups at once, a CU holds one.
+  // Under a causal mask the later half of many rows is short and fills in).  us of dQ / dK,dV at 12 heads, whole | by two | by four:
+  // 5 x 333, 4 kv heads 14.1 / 30.9 | 12.2 / 25.3 | 18.2; 1 x 700, 4 kv heads 18.4 / 50.2 | 13.8 / 38.3 | 26.6; causal 2 x 512 15.2 / 16.0
+  // | 11.4 / 12.3 | 11.4; 8 x 256 10.7 / 11.1 | 10.7 / 11.4 | 17.1; 12 x 197 14.2 / 13.4 | 16.4 / 15.8 | -; 32 x 512 45.7 / 60.8 |
+  // 68.2 / 71.4 | 154; both kernels, 8 x 44 11.9 | 11.1 | 11.9
+  constexpr int64_t CUS = 256;
+  const int64_t wq = B * h * ((L + 127) / 128), wkv = B * hk * ((S + 127) / 128), wkv4 = B * hk * ((S + 31) / 32);
+  if (wq <= CUS) hipLaunchKernelGGL(attn_bwd_dq_kernel<true>, dim3((unsigned)(h * B), (unsigned)((L + 63) / 64), 1), dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(attn_bwd_dq_kernel<false>, dim3((unsigned)(h * B), (unsigned)((L + 127) / 128), 1), dim3(256), 0, st, p);
   VY_CHECK_LAUNCH("vy_attn_bwd(dq)");
-  hipLaunchKernelGGL(attn_bwd_dkdv_kernel, dim3((unsigned)(hk * B), (unsigned)((S + 127) / 128), 1), dim3(256), 0, st, p);
+  const int64_t at_once = (mask_kind & VY_MASK_CAUSAL) && L >= 512 ? 2 * CUS : CUS;
+  const int split = L > 64 && wkv4 <= at_once ? 4 : wkv <= CUS ? 2 : 1;
+  const dim3 gkv((unsigned)(hk * B), (unsigned)((S * split + 127) / 128), 1);
+  if (split == 4) hipLaunchKernelGGL(attn_bwd_dkdv_kernel<4>, gkv, dim3(256), 0, st, p);
+  else if (split == 2) hipLaunchKernelGGL(attn_bwd_dkdv_kernel<2>, gkv, dim3(256), 0, st, p);
+  else hipLaunchKernelGGL(attn_bwd_dkdv_kernel<1>, gkv, dim3(256), 0, st, p);
   VY_CHECK_LAUNCH("vy_attn_bwd(dkdv)");
   return VY_OK;
 }
