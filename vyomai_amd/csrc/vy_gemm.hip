@@ -278,9 +278,26 @@ __device__ __forceinline__ int xcd_remap(int bid, int nwg) {
 // L2): 113 MB of weight re-fetch per launch against 30 MB of algorithmic reads (PMC, profiles/r01_gemm_pmc.json).
 // Here an XCD keeps ONE band of W (half the matrix) in its L2 for the whole launch and streams its row panels
 // past it; every X panel is read by two XCDs instead of one: fetch ~ 2 X + 8 * W/2 = 69 MB instead of 138 MB.
-__device__ __forceinline__ void tile_of(int bid, int nwg, int tiles_n, int band_on, int& tile_m, int& tile_n) {
+// 16 to 64 column tiles whose bands are far beyond L2, or that do not divide into bands: an XCD's run walks strips of up to STRIP row panels
+// column by column, so that its 32 CUs share 6 panels of X and 5 or 6 of W, not one panel and 32 -- what a stage brings in from beyond
+// L2 is what bounds it.  K = 2048: 8192 x 16384 510 -> 470 us, 2500 x 16384 182 -> 165, 12608 x 6144 301 -> 282, 1665 x 4096 38.4 -> 36.3;
+// 6300 x 8192, K = 1024 125.6 -> 112.3.  (Level where bands reach up to 12 MB, 8192 x 4096 and 6144; with 12 column tiles or fewer a run is as
+// square by rows; the vocabulary's 197 from 8 % slower to 5 % faster.  Strips of 4 panels 0.5 % behind 6, of 8 2 %.)
+constexpr int STRIP = 6;
+__device__ __forceinline__ void tile_of(int bid, int nwg, int tiles_n, int64_t w_panel, int& tile_m, int& tile_n) {
   const int tiles_m = nwg / tiles_n;
-  if (band_on && tiles_n >= 8 && (tiles_n & 1) == 0 && (tiles_m & 3) == 0 && tiles_m * tiles_n == nwg) {
+  const bool bands = tiles_n >= 8 && (tiles_n & 1) == 0 && (tiles_m & 3) == 0;
+  if (tiles_n >= 16 && tiles_n <= 64 && !(bands && tiles_n * w_panel <= (25 << 20))) {
+    const int strips = (tiles_m + STRIP - 1) / STRIP, q = tiles_m / strips, r = tiles_m - q * strips;
+    int wg = xcd_remap(bid, nwg);
+    const int high = r * (q + 1) * tiles_n;   // tiles in the strips of q + 1 panels, which come first
+    const bool low = wg >= high;
+    const int rows = low ? q : q + 1;
+    wg -= low ? high : 0;
+    const int strip = wg / (rows * tiles_n), i = wg - strip * rows * tiles_n;
+    tile_n = i / rows;
+    tile_m = (low ? r * (q + 1) : 0) + strip * rows + i - tile_n * rows;
+  } else if (bands) {
     const int xcd = bid & 7, i = bid >> 3;
     const int band = xcd & 1, grp = xcd >> 1;
     const int bw = tiles_n >> 1, pg = tiles_m >> 2;
@@ -865,7 +882,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   int tile_m, tile_n;
-  tile_of(blockIdx.x, gridDim.x, tiles_n, !(rot_on & 32), tile_m, tile_n);
+  tile_of(blockIdx.x, gridDim.x, tiles_n, (int64_t)BN * K * 2, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   // ---- per-lane LDS-DMA source pointers (row clamped for M/N tails, chunk pre-swizzled) ----
@@ -1042,7 +1059,7 @@ __global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   int tile_m, tile_n;
-  tile_of(blockIdx.x, gridDim.x, tiles_n, !(knob & 32), tile_m, tile_n);
+  tile_of(blockIdx.x, gridDim.x, tiles_n, (int64_t)BN * K * 2, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   const int lrow = lane >> 3, slot = lane & 7;
@@ -1186,7 +1203,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave / WGN, wn = wave % WGN;
   int tile_m, tile_n;
-  tile_of(blockIdx.x, gridDim.x, tiles_n, !(knob & 32), tile_m, tile_n);
+  tile_of(blockIdx.x, gridDim.x, tiles_n, (int64_t)BN * K * 2, tile_m, tile_n);
   const int m0 = tile_m * BM, n0 = tile_n * BN;
 
   const int lrow = lane >> 3, slot = lane & 7;
@@ -1330,7 +1347,7 @@ __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     tile_n = wg / tiles_m;
     tile_m = wg - tile_n * tiles_m;
   } else {
-    tile_of(blockIdx.x, gridDim.x, tiles_n, !(knob & 32), tile_m, tile_n);
+    tile_of(blockIdx.x, gridDim.x, tiles_n, (int64_t)BN * K * 2, tile_m, tile_n);
   }
   const int m0 = tile_m * BM, n0 = tile_n * BN;
   char* ring = smem + grp * RING;
