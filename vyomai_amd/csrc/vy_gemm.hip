@@ -1,8 +1,8 @@
 // GEMM family for the projection / feed-forward path:  Y[M,N] = epi(X[M,K] . W[N,K]^T)
 //
 // bf16 kernels (the product path): MFMA, fp32 accumulate, LDS-DMA staging, by size of M:
-//   * M > 32: the tile is chosen by what the shape costs on it (pick_tiling): 256 x 256 (gemm_nt_bf16_m16_kernel, two stages),
-//     256 x 192 or 256 x 128 (gemm_nt_bf16_x3m16_kernel, X in a three-deep ring), 128 x 128 (two workgroups per CU), 64 x 64 with a
+//   * M > 32: the tile is chosen by what the shape costs on it (pick_tiling): 160, 224 or 256 x 256, 256 x 192 or 256 x 128
+//     (gemm_nt_bf16_m16_kernel, two stages) or 128 x 128 (the same, two workgroups per CU), 64 x 64 with a
 //     three-deep ring (gemm_nt_bf16_small_kernel), or K split over workgroups (gemm_nt_bf16_m16_splitk_kernel +
 //     gemm_splitk_finish_kernel; one row tile of 320 for 256 < M <= 320); all on mfma_f32_16x16x32_bf16.
 //     gemm_nt_bf16_kernel is the same tile family on mfma_f32_32x32x16_bf16 (A/B knob, 32 x 128 fallback);
@@ -344,7 +344,7 @@ __device__ __forceinline__ int w_row(int n0, int R, int N) {
 // table in LDS while its first stage is on its way, with the very expressions that it replaces (the same bits), for 2^-20 <= |x| < 16
 // and both signs; a wave with any other value in its chunk evaluates them.  Evaluated, the erf GELU's 21 vector instructions an element
 // (two at a quarter of the rate) were 9 of the 15 us that the epilogue of a 256 x 256 tile took next to a loop of 19 us (K = 768).
-// Tile sizes whose stages leave no room for it (256 x 192, and the smaller ones that share a CU) evaluate.
+// 256 x 192 tiles and the smaller ones, which share a CU, evaluate.
 // 16384 x 3072, K = 768: 107 -> 95 us, with the derivative saved 112 -> 95; 30500 rows 195 -> 171 and 218 -> 181; gated SiLU (there the
 // division), 8192 x 2 x 8192, K = 2048: 508 -> 501 us, 8192 x 2 x 4096, K = 1024: 135 -> 132.
 constexpr unsigned ACT_TAB_LOW = (127 - 20) << 7, ACT_TAB_HALF = 24 << 7;   // first magnitude's bits, entries per sign
@@ -1022,168 +1022,24 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_kernel(
 }
 
 // ------------------------------------------------------------------------------------------
-// 256 x BN x 64 tile, 8 waves (4 x 2), with the X operand in a THREE-deep LDS ring and W in two
-// buffers (3*32 + 2*BN/8 KiB = 144 KiB at BN = 192).  Why: with two whole stages every workgroup
-// barrier drains the memory pipe (all waves issue, then all wait), and the pipe is busy about half
-// the time; tools/probe/ldsdma_probe shows free-running waves take in twice as much.  A third whole
-// stage does not fit in 160 KiB, but X -- 57 % of the bytes and the operand that streams from
-// HBM/MALL rather than from L2 -- does: its loads for k-slice kt+2 stay in flight across the
-// barrier that ends slice kt, and the barrier wait is a COUNTED vmcnt (the GX youngest LDS-DMA
-// instructions of the wave, slice kt+2 of X, may still be outstanding).
-//
-// On mfma_f32_16x16x32_bf16 (on 32 x 32 x 16, with identical outputs, it was slower):
-// 4 x 6 blocks of 16 x 16 per wave (96 accumulator registers),
-// 24 MFMAs per 32-deep k-step, two k-steps per stage.  Same LDS image, same swizzle (conflict-free for this
-// fragment shape too: rows lane & 15, chunk 4 ks + (lane >> 4)), same ring, same epilogue (a lane still owns quads of 4
-// consecutive columns of one row).  Why: the chip holds a higher clock on this MFMA shape and the loop needs fewer
-// cycles per stage (tools/probe/gemm_loop_probe.hip, QUICK=1: 2250-2270 against 2380; MI355X_MICROARCH.md, DVFS
-// give-back item 7).  Per output element the k order is unchanged (one chain over k in steps of 32 instead of 16),
-// so results can differ from the 32 x 32 x 16 kernel only in the rounding of the fp32 chain.
-// ------------------------------------------------------------------------------------------
-template <int BN, int EPI, int ACT, bool GRAD>
-__global__ __launch_bounds__(512) void gemm_nt_bf16_x3m16_kernel(
-    const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
-    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob) {
-  constexpr int BM = 256, WGM = 4, WGN = 2, NW = 8;
-  constexpr int TM = BM / (16 * WGM), TN = BN / (16 * WGN);   // 4, 6
-  constexpr int PX = BM / 8, PW = BN / 8;
-  constexpr int GX = PX / NW, GW = PW / NW;
-  static_assert(GX * NW == PX && GW * NW == PW, "pieces must divide over the waves");
-  constexpr int XT = BM * ROWB, WT = BN * ROWB;
-  constexpr int WOFF = 3 * XT;
-  constexpr int LDS_BYTES = vy_cmax(3 * XT + 2 * WT, epi_lds_bytes(BM, BN, EPI, 1)), TABLE = act_table_bytes(BM, BN, EPI, ACT, GRAD);
-  __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES + TABLE];
-  unsigned* tab = reinterpret_cast<unsigned*>(smem + LDS_BYTES);
-
-  const int tid = threadIdx.x, lane = tid & 63;
-  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-  const int wm = wave / WGN, wn = wave % WGN;
-  int tile_m, tile_n;
-  tile_of(blockIdx.x, gridDim.x, tiles_n, (int64_t)BN * K * 2, tile_m, tile_n);
-  const int m0 = tile_m * BM, n0 = tile_n * BN;
-
-  const int lrow = lane >> 3, slot = lane & 7;
-  const bf16* xsrc[GX]; int xk[GX];
-  const bf16* wsrc[GW]; int wk[GW];
-#pragma unroll
-  for (int t = 0; t < GX; ++t) {
-    const int R = (wave + NW * t) * 8 + lrow;
-    const int g = slot ^ ((R >> 1) & 7);
-    int gm = m0 + R; gm = gm < M ? gm : M - 1;
-    xsrc[t] = X + (int64_t)gm * ldx + g * 8;
-    xk[t] = g * 8;
-  }
-#pragma unroll
-  for (int t = 0; t < GW; ++t) {
-    const int R = (wave + NW * t) * 8 + lrow;
-    const int g = slot ^ ((R >> 1) & 7);
-    wsrc[t] = W + (int64_t)w_row<EPI>(n0, R, N) * ldw + g * 8;
-    wk[t] = g * 8;
-  }
-  const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
-  const bool ktail = (K % BK) != 0;
-  const int KT = (K + BK - 1) / BK;
-  auto stage_x = [&](int kt) {
-    char* xb = smem + (kt % 3) * XT;
-    const int k0 = kt * BK;
-#pragma unroll
-    for (int t = 0; t < GX; ++t) {
-      const bf16* s = xsrc[t] + k0;
-      if (ktail && k0 + xk[t] >= K) s = zero;
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
-    }
-  };
-  auto stage_w = [&](int kt) {
-    char* wb = smem + WOFF + (kt & 1) * WT;
-    const int k0 = kt * BK;
-#pragma unroll
-    for (int t = 0; t < GW; ++t) {
-      const bf16* s = wsrc[t] + k0;
-      if (ktail && k0 + wk[t] >= K) s = zero;
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(wb + (wave + NW * t) * 1024), 16, 0, 0);
-    }
-  };
-
-  f32x4 acc[TN][TM];
-#pragma unroll
-  for (int i = 0; i < TN; ++i)
-#pragma unroll
-    for (int j = 0; j < TM; ++j) acc[i][j] = f32x4{0.f, 0.f, 0.f, 0.f};
-
-  const int r16 = lane & 15, kq = lane >> 4, fsw = (r16 >> 1) & 7;
-  unsigned xa[2], wa[2];
-#pragma unroll
-  for (int ks = 0; ks < 2; ++ks) {
-    const int coff = (((ks * 4 + kq) ^ fsw) << 4);
-    xa[ks] = vy_lds_addr(smem) + (wm * 16 * TM + r16) * ROWB + coff;
-    wa[ks] = vy_lds_addr(smem) + WOFF + (wn * 16 * TN + r16) * ROWB + coff;
-  }
-  bf16x8 wf[2][TN], xf[2][TM];
-  auto read_frags = [&](unsigned wbase, unsigned xbase, bf16x8 (&w_)[TN], bf16x8 (&x_)[TM]) {
-    vy_static_for<TN>([&](auto i_c) { constexpr int i = decltype(i_c)::value; w_[i] = vy_lds_read128_off<i * 16 * ROWB>(wbase); });
-    vy_static_for<TM>([&](auto j_c) { constexpr int j = decltype(j_c)::value; x_[j] = vy_lds_read128_off<j * 16 * ROWB>(xbase); });
-  };
-  auto tie_frags = [&](bf16x8 (&w_)[TN], bf16x8 (&x_)[TM]) {
-#pragma unroll
-    for (int i = 0; i < TN; ++i) vy_tie(w_[i]);
-#pragma unroll
-    for (int j = 0; j < TM; ++j) vy_tie(x_[j]);
-  };
-  auto mma = [&](bf16x8 (&w_)[TN], bf16x8 (&x_)[TM]) {
-    __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-    for (int i = 0; i < TN; ++i)
-#pragma unroll
-      for (int j = 0; j < TM; ++j)
-        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_[i], x_[j], acc[i][j], 0, 0, 0);
-    __builtin_amdgcn_s_setprio(0);
-  };
-
-  stage_x(0);
-  stage_w(0);
-  if (KT > 1) stage_x(1);
-  if constexpr (TABLE > 0) {
-    fill_act_table<EPI, ACT>(tab, ep.pre_deriv);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-  }
-  if (KT > 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GX) : "memory");
-  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-  __builtin_amdgcn_s_barrier();
-  asm volatile("" ::: "memory");
-  read_frags(wa[0], xa[0], wf[0], xf[0]);
-  int xbuf = 0;   // kt % 3
-  for (int kt = 0; kt < KT; ++kt) {
-    if (kt + 1 < KT) stage_w(kt + 1);
-    if (kt + 2 < KT) stage_x(kt + 2);
-    const unsigned xo = xbuf * XT, wo = (kt & 1) * WT;
-    read_frags(wa[1] + wo, xa[1] + xo, wf[1], xf[1]);
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TN + TM) : "memory");
-    tie_frags(wf[0], xf[0]);
-    mma(wf[0], xf[0]);
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    tie_frags(wf[1], xf[1]);
-    mma(wf[1], xf[1]);
-    if (kt + 2 < KT) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GX) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __builtin_amdgcn_s_barrier();
-    asm volatile("" ::: "memory");
-    xbuf = xbuf == 2 ? 0 : xbuf + 1;
-    if (kt + 1 < KT) read_frags(wa[0] + (WT - wo), xa[0] + xbuf * XT, wf[0], xf[0]);
-  }
-  EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
-  ahead.request(ep, m0, n0, M, N);
-  gemm_epilogue<BM, BN, WGM, WGN, EPI, ACT, GRAD, 1, true>(acc, smem, m0, n0, M, N, ep, eq, ahead, tab);
-}
-
-// ------------------------------------------------------------------------------------------
-// BM x BN x 64 tiles, two whole stages, on mfma_f32_16x16x32_bf16.  256 x 256 (8 waves, 128 KiB): the wide launches (FFN1,
-// the dgrad of FFN2, the vocabulary projection), where the tile's fewer operand bytes per FLOP matter more than a third X
-// stage; 4 x 8 blocks of 16 x 16 per wave (128 accumulator registers), 32 MFMAs per k-step, fragments double-buffered.
-// 224 and 160 x 256 (2 x 4 waves): where these heights fill the last round of the CUs better, which is what ragged rows lose to.  Under
-// load, 12608 x 3072, K = 768: 600 tiles 76.4 us, 684 of 224 rows 71.2; 6000 x 3072, K = 768: 288 tiles 47.1, 456 of 160 rows 37.0 (operands from
-// beyond the Infinity Cache: 77.4 and 75.8, 49.8 and 42.7).  A third stage of X for them: 3 to 6 % slower, or where X comes from far 3 to 7 % faster
-// and then as fast as 256 x 192; 192 rows 0.2 % on average beside these, 192 x 192 0.5 %, 224, 288 and 320 x 192 0.1 %.
+// BM x BN x 64 tiles, two whole stages, on mfma_f32_16x16x32_bf16 (on 32 x 32 x 16, with the same sums but for the rounding of their
+// chains, it was slower: the chip holds a higher clock on this shape).  256 x 256 (8 waves, 128 KiB): the wide launches, where
+// the tile's fewer operand bytes per FLOP matter most; 4 x 8 blocks of 16 x 16 per wave (128 accumulator registers), 32 products per
+// k-step, fragments double-buffered.  256 x 192 and 256 x 128: outputs that these divide into whole rounds of the 256 CUs.
+// 224 and 160 x 256 (2 x 4 waves): where these heights fill the last round of the CUs better, which is what ragged rows lose to.
 // 128 x 128 (4 waves, 64 KiB, two workgroups per CU): mid-size M.
+//
+// Eight waves, ORDERED: products, LDS reads and requests in the order written.  A stage's fragments are all in registers a third
+// into its products; behind a barrier there, the requests of the stage after next go out into its place, one every few products (W's
+// first, which more workgroups of the XCD ask for), and the next stage has to be there only two thirds into the products, behind a second
+// barrier, with the fragments of its first half read under the remaining ones.  So a request has 1.2 to 1.6 stages of time, a wave
+// is not held up by a burst of requests, and no wave waits for LDS at a stage's start.  One barrier a stage and its requests in
+// a burst at the start (as 128 x 128 does, where the other workgroup fills the gaps), 256 x 256: 8192 x 2048, K = 8192, 222 -> 207 us; 16384
+// x 768, K = 3072, 87 -> 78.5; 30500 x 3072, K = 768, 171.5 -> 162.4; 160 x 256, 8192 x 8192, K = 1024: 183 -> 170; 256 x 192 against
+// three stages of X and two of W: 4096 x 4096, K = 4096, 161 -> 149; 16384 x 768, K = 768, 23.9 -> 23.0.  X's requests first: half of the gain.
+// A stage of 256 x 256 takes 1.5 us, 0.95 without its requests: data from beyond L2, shared by 4 to 8 CUs that ask at the same time (from
+// L2 alone 1.2), and the chip's power (zeros as data 1.35).  No faster: stages of 32 columns in a ring of four, one of them half a line (four waves
+// of 128 x 128 or eight: 1.7), five slots of X or W (1.7), four waves with two stages (1.65), tiles in a loop with the epilogue through LDS by wave.
 // ------------------------------------------------------------------------------------------
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
@@ -1195,6 +1051,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   constexpr int GX = (PX + NW - 1) / NW, GW = PW / NW, REST = PX % NW;   // (of X, the last piece of a wave may be missing)
   static_assert(TM * 16 * WGM == BM && TN * 16 * WGN == BN && GW * NW == PW, "whole blocks, and pieces of W divide over the waves");
   constexpr int STAGE = (BM + BN) * ROWB;
+  constexpr bool ORDERED = NW == 8;
   constexpr int LDS_BYTES = vy_cmax(2 * STAGE, epi_lds_bytes(BM, BN, EPI, 1)), TABLE = act_table_bytes(BM, BN, EPI, ACT, GRAD);
   __shared__ __attribute__((aligned(16))) char smem[LDS_BYTES + TABLE];
   unsigned* tab = reinterpret_cast<unsigned*>(smem + LDS_BYTES);
@@ -1227,23 +1084,27 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   const bf16* zero = reinterpret_cast<const bf16*>(vy_zero16);
   const bool ktail = (K % BK) != 0;
   const int KT = (K + BK - 1) / BK;
-  auto stage = [&](int kt, int buf) {
-    char* xb = smem + buf * STAGE;
-    char* wb = xb + BM * ROWB;
+  // piece t of a wave: W's first, then X's
+  auto request = [&](auto t_c, int kt, char* stage) {
+    constexpr int t = decltype(t_c)::value;
     const int k0 = kt * BK;
-#pragma unroll
-    for (int t = 0; t < GX; ++t) {
-      const bf16* s = xsrc[t] + k0;
-      if (ktail && k0 + xk[t] >= K) s = zero;
-      if (REST == 0 || t + 1 < GX || wave < REST)
-        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(xb + (wave + NW * t) * 1024), 16, 0, 0);
+    if constexpr (t < GW) {
+      const bf16* p = wsrc[t] + k0;
+      if (ktail && k0 + wk[t] >= K) p = zero;
+      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)p, (VY_LDS void*)(stage + BM * ROWB + (wave + NW * t) * 1024), 16, 0, 0);
+    } else {
+      constexpr int x = t - GW;
+      const bf16* p = xsrc[x] + k0;
+      if (ktail && k0 + xk[x] >= K) p = zero;
+      if (REST == 0 || x + 1 < GX || wave < REST)
+        __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)p, (VY_LDS void*)(stage + (wave + NW * x) * 1024), 16, 0, 0);
     }
-#pragma unroll
-    for (int t = 0; t < GW; ++t) {
-      const bf16* s = wsrc[t] + k0;
-      if (ktail && k0 + wk[t] >= K) s = zero;
-      __builtin_amdgcn_global_load_lds((const VY_GLOBAL void*)s, (VY_LDS void*)(wb + (wave + NW * t) * 1024), 16, 0, 0);
-    }
+  };
+  auto stage = [&](int kt, int buf) { vy_static_for<GX + GW>([&](auto t_c) { request(t_c, kt, smem + buf * STAGE); }); };
+  // the requests of one stage may be under way
+  auto wait_but_one_stage = [&]() {
+    if (REST == 0 || wave < REST) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GX + GW) : "memory");
+    else asm volatile("s_waitcnt vmcnt(%0)" ::"n"(GX + GW - 1) : "memory");
   };
 
   f32x4 acc[TN][TM];
@@ -1282,29 +1143,81 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
   };
 
   stage(0, 0);
+  if constexpr (ORDERED) {
+    if (KT > 1) stage(1, 1);
+  }
   if constexpr (TABLE > 0) {
     fill_act_table<EPI, ACT>(tab, ep.pre_deriv);
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
   }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+  if (ORDERED && KT > 1) wait_but_one_stage();
+  else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   __builtin_amdgcn_s_barrier();
   asm volatile("" ::: "memory");
   read_frags(wa[0], xa[0], wf[0], xf[0]);
-  for (int kt = 0; kt < KT; ++kt) {
-    const int cur = kt & 1;
-    if (kt + 1 < KT) stage(kt + 1, cur ^ 1);
-    const unsigned boff = cur * STAGE;
-    read_frags(wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
-    asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TN + TM) : "memory");
-    tie_frags(wf[0], xf[0]);
-    mma(wf[0], xf[0]);
+  if constexpr (ORDERED) {
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-    tie_frags(wf[1], xf[1]);
-    mma(wf[1], xf[1]);
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    tie_frags(wf[0], xf[0]);
+    auto read_one = [&](auto q_c, unsigned wbase, unsigned xbase, bf16x8 (&w_)[TN], bf16x8 (&x_)[TM]) {
+      constexpr int q = decltype(q_c)::value;
+      if constexpr (q < TN) w_[q] = vy_lds_read128_off<q * 16 * ROWB>(wbase);
+      else x_[q - TN] = vy_lds_read128_off<(q - TN) * 16 * ROWB>(xbase);
+    };
+    constexpr int HALF = TM * TN, READS = TM + TN, LOADS = GX + GW;
+    constexpr int FREE = READS + (HALF < 20 ? 3 : 6), LANDED = 2 * HALF - READS - (HALF < 20 ? 2 : 4), STEP = (LANDED - 2 - FREE) / (LOADS - 1);
+    static_assert(STEP >= 1 && FREE + 1 + STEP * (LOADS - 1) < LANDED, "the requests fit between the two barriers");
+    for (int kt = 0; kt < KT; ++kt) {
+      const unsigned boff = (kt & 1) * STAGE, noff = STAGE - boff;
+      char* mine = smem + boff;
+      const bool more = kt + 2 < KT;
+      vy_static_for<2 * HALF>([&](auto m_c) {
+        constexpr int m = decltype(m_c)::value, f = m / HALF, i = m % HALF / TM, j = m % TM;
+        asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(wf[f][i]), "v"(xf[f][j]));
+        if constexpr (m < READS) read_one(m_c, wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
+        if constexpr (m == FREE) {   // every wave has its fragments of this stage: the next but one may come into its place
+          asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+          tie_frags(wf[1], xf[1]);
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+        }
+        if constexpr (m > FREE && (m - FREE - 1) % STEP == 0 && (m - FREE - 1) / STEP < LOADS) {
+          if (more) request(std::integral_constant<int, (m - FREE - 1) / STEP>{}, kt + 2, mine);
+        }
+        if constexpr (m == LANDED) {   // the next stage is there
+          if (more) wait_but_one_stage();
+          else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+          __builtin_amdgcn_s_barrier();
+          asm volatile("" ::: "memory");
+        }
+        if constexpr (m > LANDED && m - LANDED - 1 < READS) read_one(std::integral_constant<int, m - LANDED - 1>{}, wa[0] + noff, xa[0] + noff, wf[0], xf[0]);
+      });
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (behind the last stage: of the one before, for nothing)
+      tie_frags(wf[0], xf[0]);
+    }
+    asm volatile("s_nop 15\n\ts_nop 15" ::: "memory");   // (the compiler does not know that the accumulators are a matrix product's)
+#pragma unroll
+    for (int i = 0; i < TN; ++i)
+#pragma unroll
+      for (int j = 0; j < TM; ++j) vy_tie(acc[i][j]);
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
-    if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
+  } else {
+    for (int kt = 0; kt < KT; ++kt) {
+      const int cur = kt & 1;
+      if (kt + 1 < KT) stage(kt + 1, cur ^ 1);
+      const unsigned boff = cur * STAGE;
+      read_frags(wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
+      asm volatile("s_waitcnt lgkmcnt(%0)" ::"n"(TN + TM) : "memory");
+      tie_frags(wf[0], xf[0]);
+      mma(wf[0], xf[0]);
+      asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+      tie_frags(wf[1], xf[1]);
+      mma(wf[1], xf[1]);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+      __builtin_amdgcn_s_barrier();
+      asm volatile("" ::: "memory");
+      if (kt + 1 < KT) read_frags(wa[0] + (STAGE - boff), xa[0] + (STAGE - boff), wf[0], xf[0]);
+    }
   }
   EpiAhead<BM, BN, NW, EPI, GRAD> ahead;
   ahead.request(ep, m0, n0, M, N);
@@ -2663,8 +2576,8 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
         else if (t.rows == 160) VY_TILES(gemm_nt_bf16_m16_kernel<160, 256, 2, 4, EPI, ACT, GRAD>);
         else VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>);
         break;
-      case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, EPI, ACT, GRAD>); break;
-      case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, EPI, ACT, GRAD>); break;
+      case T_256x192: VY_TILES(gemm_nt_bf16_m16_kernel<256, 192, 4, 2, EPI, ACT, GRAD>); break;
+      case T_256x128: VY_TILES(gemm_nt_bf16_m16_kernel<256, 128, 4, 2, EPI, ACT, GRAD>); break;
       case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, EPI, ACT, GRAD>); break;
       case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, 64, EPI, ACT, GRAD>); break;
       case T_64x64_TWICE:
@@ -2704,8 +2617,8 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
       else if (t.rows == 160) VY_TILES(gemm_nt_bf16_m16_kernel<160, 256, 2, 4, 2, ACT, false>);
       else VY_TILES(gemm_nt_bf16_m16_kernel<256, 256, 4, 2, 2, ACT, false>);
       break;
-    case T_256x192: VY_TILES(gemm_nt_bf16_x3m16_kernel<192, 2, ACT, false>); break;
-    case T_256x128: VY_TILES(gemm_nt_bf16_x3m16_kernel<128, 2, ACT, false>); break;
+    case T_256x192: VY_TILES(gemm_nt_bf16_m16_kernel<256, 192, 4, 2, 2, ACT, false>); break;
+    case T_256x128: VY_TILES(gemm_nt_bf16_m16_kernel<256, 128, 4, 2, 2, ACT, false>); break;
     case T_128x128: VY_TILES(gemm_nt_bf16_m16_kernel<128, 128, 2, 2, 2, ACT, false>); break;
     case T_64x64: VY_SMALL(gemm_nt_bf16_small_kernel<1, 3, 1, 64, 2, ACT, false>); break;
     case T_64x64_TWICE:
