@@ -1164,8 +1164,14 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
       else x_[q - TN] = vy_lds_read128_off<(q - TN) * 16 * ROWB>(xbase);
     };
     constexpr int HALF = TM * TN, READS = TM + TN, LOADS = GX + GW;
-    constexpr int FREE = READS + (HALF < 20 ? 3 : 6), LANDED = 2 * HALF - READS - (HALF < 20 ? 2 : 4), STEP = (LANDED - 2 - FREE) / (LOADS - 1);
+    // fragments read per product, and the products behind which a stage is free, its requests go out and the next has to be there.  Trials: 256 x
+    // 256 with the others' distances 2 to 4 % slower, 256 x 192 with one read a product 3 to 5, the others with 256 x 256's 3 to 7
+    constexpr bool WHOLE = BM * BN == 65536;
+    constexpr int PER = BN == 192 ? 2 : 1, ROUNDS = (READS + PER - 1) / PER;
+    constexpr int FREE = ROUNDS + (WHOLE ? 2 : HALF < 20 ? 3 : 6), LANDED = 2 * HALF - ROUNDS - (WHOLE ? 1 : HALF < 20 ? 2 : 4);
+    constexpr int STEP = (LANDED - 2 - FREE) / (LOADS - 1);
     static_assert(STEP >= 1 && FREE + 1 + STEP * (LOADS - 1) < LANDED, "the requests fit between the two barriers");
+    static_assert(LANDED + ROUNDS < 2 * HALF && ROUNDS <= FREE, "and the reads beside them");
     for (int kt = 0; kt < KT; ++kt) {
       const unsigned boff = (kt & 1) * STAGE, noff = STAGE - boff;
       char* mine = smem + boff;
@@ -1173,7 +1179,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
       vy_static_for<2 * HALF>([&](auto m_c) {
         constexpr int m = decltype(m_c)::value, f = m / HALF, i = m % HALF / TM, j = m % TM;
         asm volatile("v_mfma_f32_16x16x32_bf16 %0, %1, %2, %0" : "+v"(acc[i][j]) : "v"(wf[f][i]), "v"(xf[f][j]));
-        if constexpr (m < READS) read_one(m_c, wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
+        vy_static_for<PER>([&](auto p_c) {
+          constexpr int q = PER * m + decltype(p_c)::value;
+          if constexpr (q < READS) read_one(std::integral_constant<int, q>{}, wa[1] + boff, xa[1] + boff, wf[1], xf[1]);
+        });
         if constexpr (m == FREE) {   // every wave has its fragments of this stage: the next but one may come into its place
           asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
           tie_frags(wf[1], xf[1]);
@@ -1189,7 +1198,10 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
           __builtin_amdgcn_s_barrier();
           asm volatile("" ::: "memory");
         }
-        if constexpr (m > LANDED && m - LANDED - 1 < READS) read_one(std::integral_constant<int, m - LANDED - 1>{}, wa[0] + noff, xa[0] + noff, wf[0], xf[0]);
+        vy_static_for<PER>([&](auto p_c) {
+          constexpr int q = PER * (m - LANDED - 1) + decltype(p_c)::value;
+          if constexpr (m > LANDED && q < READS) read_one(std::integral_constant<int, q>{}, wa[0] + noff, xa[0] + noff, wf[0], xf[0]);
+        });
       });
       asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");   // (behind the last stage: of the one before, for nothing)
       tie_frags(wf[0], xf[0]);
