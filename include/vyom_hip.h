@@ -569,6 +569,11 @@ int vy_xent_bwd(void* logits, int64_t ld, const int64_t* labels, int64_t ignore_
 int vy_xent_fused(void* logits, int64_t ld, const int64_t* labels, int64_t ignore_index, float* lse,
                   float* loss_sum, const float* count, const float* gscale, int64_t M, int64_t V,
                   int32_t* err_flag, int dtype, void* stream);
+/* What a loss shifted by one position gives vy_xent_fused besides the logits, in one launch: shifted[b L + l] = labels[b][l + 1]
+ * (elements sb, sl apart; ignore_index for the last of a row), acc = {0, the number of labels in [0, V) that are not ignore_index}, and
+ * the columns V .. ld - 1 of the B L rows of bf16 logits cleared. */
+int vy_shift_labels(const int64_t* labels, int64_t sb, int64_t sl, int64_t* shifted, float* acc, void* logits, int64_t ld,
+                    int64_t ignore_index, int64_t B, int64_t L, int64_t V, void* stream);
 /* A label that is neither ignore_index nor inside [0, V) (torch.cross_entropy device-asserts on it) is
  * never dereferenced: the row counts as ignored (zero loss, zero gradient) and *err_flag (nullable,
  * device int32) is set to 1 for the host to report. */

@@ -899,22 +899,28 @@ class LMHeadLossFn(torch.autograd.Function):
         V = wv.shape[0]
         ld = _row_stride(V)
         buf = torch.empty((B * L, ld), dtype=dt, device=dev)
-        if ld != V:
-            buf[:, V:].zero_()  # only the pad columns: the GEMM writes the rest
         logits = buf[:, :V]
-        ops.linear(n.view(B * L, -1), _shadow(wv, dt), _shadow(bias, dt), out=logits)
-        shifted = torch.full((B, L), ignore_index, dtype=torch.long, device=dev)
-        shifted[:, :-1] = labels[:, 1:]
-        shifted = shifted.view(-1)
-        lse = torch.empty(B * L, dtype=torch.float32, device=dev)
-        acc = torch.zeros(2, dtype=torch.float32, device=dev)  # [loss_sum, count]
         fused = V <= 65536 and dt == BF16   # (vy_xent_fused is a bf16 kernel; fp32 takes the two-pass pair)
+        together = fused and labels.dtype == torch.long and labels.device == dev and labels.shape == (B, L)
+        if not together and ld != V:
+            buf[:, V:].zero_()  # only the pad columns: the GEMM writes the rest
+        ops.linear(n.view(B * L, -1), _shadow(wv, dt), _shadow(bias, dt), out=logits)
+        # acc: [loss_sum, count]
+        if together:
+            shifted, acc = ops.shift_labels(labels, ignore_index, logits, ld)
+        else:
+            shifted = torch.full((B, L), ignore_index, dtype=torch.long, device=dev)
+            shifted[:, :-1] = labels[:, 1:]
+            shifted = shifted.view(-1)
+            acc = torch.zeros(2, dtype=torch.float32, device=dev)
+        lse = torch.empty(B * L, dtype=torch.float32, device=dev)
         if fused:
             # one pass: loss AND the unit gradient (d loss / d logits for an upstream gradient of 1),
             # written over the logits; backward scales by the actual upstream gradient (linearity)
             # (rows with an out-of-range label contribute neither loss nor gradient -- the kernel raises err_flag for
             # them -- so they must not count in the mean either, exactly as on the two-pass path)
-            acc[1] = ((shifted != ignore_index) & (shifted >= 0) & (shifted < V)).sum()
+            if not together:
+                acc[1] = ((shifted != ignore_index) & (shifted >= 0) & (shifted < V)).sum()
             ops.xent_fused_(logits, shifted, ignore_index, lse, acc[0:1], acc[1:2], _one(dev), err_flag)
         else:
             ops.xent_fwd(logits, shifted, ignore_index, lse, acc[0:1], acc[1:2], err_flag)

@@ -952,6 +952,52 @@ extern "C" int vy_xent_fused(void* logits, int64_t ld, const int64_t* labels, in
   return VY_OK;
 }
 
+// Labels of a shifted loss and what its kernel is given besides, in one launch: shifted[b][l] = labels[b][l + 1] (the last of a row: ignore),
+// the rows of logits' padding columns cleared, acc = {0, rows that count}.  The first workgroup counts, the others do the rest.  (As eleven
+// launches of a few bytes each it was 60 us of a training step of 5 x 333, 4.65 ms.)
+__global__ __launch_bounds__(1024) void shift_labels_kernel(const int64_t* __restrict__ labels, int64_t sb, int64_t sl, int64_t* __restrict__ shifted,
+                                                            float* __restrict__ acc, bf16* __restrict__ logits, int64_t ld, int64_t ignore,
+                                                            unsigned M, unsigned L, int64_t V) {
+  auto label = [&](unsigned m) {
+    const unsigned b = m / L, l = m - b * L;
+    return l + 1 < L ? labels[b * sb + (l + 1) * sl] : ignore;
+  };
+  if (blockIdx.x == 0) {
+    __shared__ unsigned counts[16];
+    unsigned n = 0;
+    for (unsigned m = threadIdx.x; m < M; m += 1024) {
+      const int64_t t = label(m);
+      n += t != ignore && t >= 0 && t < V;
+    }
+#pragma unroll
+    for (int o = 32; o; o >>= 1) n += __shfl_xor(n, o, 64);
+    if ((threadIdx.x & 63) == 0) counts[threadIdx.x >> 6] = n;
+    __syncthreads();
+    if (threadIdx.x == 0) {
+#pragma unroll
+      for (int w = 1; w < 16; ++w) n += counts[w];
+      acc[0] = 0.f;
+      acc[1] = (float)n;
+    }
+    return;
+  }
+  for (unsigned m = (blockIdx.x - 1) * 1024 + threadIdx.x; m < M; m += (gridDim.x - 1) * 1024) {
+    shifted[m] = label(m);
+    for (int64_t c = V; c < ld; ++c) logits[m * ld + c] = (bf16)0.f;
+  }
+}
+
+extern "C" int vy_shift_labels(const int64_t* labels, int64_t sb, int64_t sl, int64_t* shifted, float* acc, void* logits, int64_t ld,
+                               int64_t ignore_index, int64_t B, int64_t L, int64_t V, void* stream) {
+  if (!labels || !shifted || !acc || !logits || B <= 0 || L <= 0 || V <= 0) VY_FAIL(VY_ERR_ARG, "vy_shift_labels: bad arguments");
+  if (ld < V || B * L >= (int64_t)1 << 31) VY_FAIL(VY_ERR_ARG, "vy_shift_labels: rows of %ld for %ld columns, %ld rows", (long)ld, (long)V, (long)(B * L));
+  const int64_t want = vy_cdiv(B * L, 1024);
+  hipLaunchKernelGGL(shift_labels_kernel, dim3((unsigned)(1 + (want < 256 ? want : 256))), dim3(1024), 0, (hipStream_t)stream, labels, sb, sl, shifted,
+                     acc, (bf16*)logits, ld, ignore_index, (unsigned)(B * L), (unsigned)L, V);
+  VY_CHECK_LAUNCH("vy_shift_labels");
+  return VY_OK;
+}
+
 extern "C" int vy_cast(const void* src, void* dst, int64_t n, int src_dtype, int dst_dtype, void* stream) {
   if (!src || !dst || n < 0) VY_FAIL(VY_ERR_ARG, "vy_cast: bad arguments");
   if (n == 0) return VY_OK;

@@ -691,6 +691,20 @@ def xent_fused_(logits2d: Tensor, labels: Tensor, ignore_index: int, lse: Tensor
          _stream())
 
 
+def shift_labels(labels: Tensor, ignore_index: int, logits2d: Tensor, ld: int):
+    """Labels (B, L) int64 of a loss shifted by one position -> ((B L,) int64, the last of a row ignored, and [0, rows that count] fp32); the
+    columns of logits2d's rows behind its own, up to ld, are cleared  (vy_shift_labels)."""
+    _need_gpu(labels, logits2d)
+    assert labels.dtype == torch.long and labels.dim() == 2 and logits2d.dtype == torch.bfloat16 and logits2d.stride() == (ld, 1)
+    B, L = labels.shape
+    assert logits2d.shape[0] == B * L
+    shifted = torch.empty(B * L, dtype=torch.long, device=labels.device)
+    acc = torch.empty(2, dtype=torch.float32, device=labels.device)
+    call("vy_shift_labels", labels.data_ptr(), labels.stride(0), labels.stride(1), shifted.data_ptr(), acc.data_ptr(), logits2d.data_ptr(),
+         ld, ignore_index, B, L, logits2d.shape[1], _stream())
+    return shifted, acc
+
+
 def rmsnorm(x: Tensor, w: Tensor, eps: float, w_offset: float = 1.0) -> Tensor:
     """x * rsqrt(mean x^2 + eps) * (w_offset + w)  (vy_rmsnorm_fwd; Gemma: w_offset = 1)."""
     _need_gpu(x, w)
