@@ -1,6 +1,6 @@
 // One post-LN layer of the text and vision models (host code): the seven launches of vy_text_layer_fwd, and the seven and nine of a
 // layer in training, behind one call each.  A few short texts keep the GPU busy for about 50 us per layer, and enqueueing the launches one
-// by one from Python took four times that; a training step of 5 x 333 tokens, 12 layers, is 5.9 ms of kernels, and its layers one operation at
+// by one from Python took four times that; a training step of 5 x 333 tokens, 12 layers, is 4.5 ms of kernels, and its layers one operation at
 // a time took the host 6.5 and more.
 #include "vy_common.h"
 
