@@ -1,5 +1,5 @@
-"""Decode attention whose softmax goes by two parts of the keys: contexts at the edges of the register counts (64 keys a pass of 64-wide heads, 32
-of 256-wide ones, parts from the sixth pass on), the largest score in either part, parts that weigh nothing, streamed and cached keys, shared
+"""Decode attention's softmax over keys of any place: contexts at the edges of the register counts (64 keys a pass of 64-wide heads, 32
+of 256-wide ones), the largest score in the first, a middle or the last key, keys that weigh nothing, streamed and cached keys, shared
 key heads; against fp64."""
 import pytest
 import torch
@@ -44,7 +44,7 @@ def test_heads_of_256(B, h, hk, S):
 
 @pytest.mark.parametrize("S", [5, 400, 700])
 def test_values_without_a_finite_weight(S):
-    """A NaN or an infinite score in either part: NaN in its head's result, and nowhere else."""
+    """A NaN or an infinite score of the first or the last key: NaN in its head's result, and nowhere else."""
     from vyomai_amd import ops
     g = torch.Generator(device=DEV).manual_seed(S)
     for at in (0, S - 1):

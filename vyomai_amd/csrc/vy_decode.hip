@@ -577,10 +577,8 @@ int dec_part64_go(DecGemmArgs a, int K, hipStream_t st) {
 // Single-query attention against the KV cache (reference models/decoder.py:107 / layers/attention.py with L = 1 and
 // mask = None): one workgroup per (batch row, query head), every K and V chunk of the row's context requested
 // BEFORE the first dot product (NP passes of NW * 64 / (DH / 8) keys: a compile-time count, no loop around the
-// loads), reductions on the DPP / permlane path, one barrier.  The softmax goes by two parts of the keys, the second rescaling the
-// first, and by groups of LPK lanes, whose sums meet at the end: while the second part arrives the first is done, where one maximum
-// over all keys left every exponential and every value to do behind the last byte (32 x 12 heads behind 524 tokens, 52 MB, of which a
-// bare read takes 9 us: 13.1 -> 12.0 us; parts of four keys or the last two or three by themselves 12.1 to 12.6).  The general attn_rowwise_kernel walks the context in
+// loads), plain two-pass softmax over the scores held in registers (no online rescaling: the whole context is
+// resident), reductions on the DPP / permlane path, two barriers.  The general attn_rowwise_kernel walks the context in
 // dependent trips with ds_bpermute reductions: 11.9 us for the 8 x 300-key rows of a PaliGemma-shape step, 14.7 us for
 // 384 rows x 577 keys -- this one is bound by the K/V stream alone.
 //   lane = (key group g, 16-byte chunk ch of the head): LPK = DH / 8 lanes per key, KPW = 64 / LPK keys per wave pass.
@@ -632,8 +630,8 @@ __device__ __forceinline__ float dec_stride_sum(float v) {
 // projection's rows are spread over -- its keys come from L2 then, and no workgroup has more to read than before.  What that gives and
 // costs: vy_dec_shares_pay (vy_runtime.hip).
 template <int DH, int NW, int NP, bool NT, int R = 1, bool PROJ = false>
-__global__ __launch_bounds__(64 * NW, R == 1 && !PROJ ? 4 : 1) void dec_attn_kernel(const DecAttnArgs p) {
-  constexpr int LPK = DH / 8, KPW = 64 / LPK, KPP = NW * KPW, FIRST = NP <= 5 ? NP : (NP + 1) / 2;
+__global__ __launch_bounds__(64 * NW) void dec_attn_kernel(const DecAttnArgs p) {
+  constexpr int LPK = DH / 8, KPW = 64 / LPK, KPP = NW * KPW;
   __shared__ float red_m[R][NW], red_l[R][NW];
   __shared__ float red_o[R][NW][DH];
   __shared__ __attribute__((aligned(16))) bf16 result[PROJ ? R : 1][PROJ ? DH : 8];
@@ -669,63 +667,51 @@ __global__ __launch_bounds__(64 * NW, R == 1 && !PROJ ? 4 : 1) void dec_attn_ker
     if constexpr (NT) { kr[i] = dec_load_stream(kb + jo); vr[i] = dec_load_stream(vb + jo); }
     else { kr[i] = *reinterpret_cast<const bf16x8*>(kb + jo); vr[i] = *reinterpret_cast<const bf16x8*>(vb + jo); }
   }
-  asm volatile("" ::: "memory");   // (everything is requested ahead of the first dot product: left to itself the compiler moves loads down to save registers)
-  float m[R], l[R], acc[R][8];
+  float sc[R][NP];
+  float m[R];
 #pragma unroll
   for (int r = 0; r < R; ++r) {
+    float qf[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) qf[e] = (float)q8[r][e];
     m[r] = -FLT_MAX;
+#pragma unroll
+    for (int i = 0; i < NP; ++i) {
+      float d = 0.f;
+#pragma unroll
+      for (int e = 0; e < 8; ++e) d = fmaf(qf[e], (float)kr[i][e], d);
+      d = dec_group_sum<LPK>(d) * p.scale;
+      const int j = i * KPP + wave * KPW + g;
+      sc[r][i] = j < S ? d : -FLT_MAX;
+      m[r] = fmaxf(m[r], sc[r][i]);
+    }
+    m[r] = dec_wave_max(m[r]);
+    if (lane == 0) red_m[r][wave] = m[r];
+  }
+  __syncthreads();
+  float l[R], acc[R][8];
+#pragma unroll
+  for (int r = 0; r < R; ++r) {
+    float M = red_m[r][0];
+#pragma unroll
+    for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[r][w]);
     l[r] = 0.f;
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[r][e] = 0.f;
-  }
-  // two parts of the keys, the first's softmax ahead of the second's arrival: by groups of LPK lanes, whose maximum needs no other lane's
-  auto keys = [&](auto from_c, auto to_c) {
-    constexpr int FROM = decltype(from_c)::value, TO = decltype(to_c)::value;
-    float sc[R][TO - FROM], top[R];
 #pragma unroll
-    for (int r = 0; r < R; ++r) top[r] = m[r];
+    for (int i = 0; i < NP; ++i) {
+      const int j = i * KPP + wave * KPW + g;
+      const float ev = j < S ? __expf(sc[r][i] - M) : 0.f;
+      l[r] += ev;
 #pragma unroll
-    for (int i = FROM; i < TO; ++i)
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        float d = 0.f;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) d = fmaf((float)q8[r][e], (float)kr[i][e], d);
-        d = dec_group_sum<LPK>(d) * p.scale;
-        sc[r][i - FROM] = i * KPP + wave * KPW + g < S ? d : -FLT_MAX;
-        top[r] = fmaxf(top[r], sc[r][i - FROM]);
-      }
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      if constexpr (FROM > 0) {
-        const float keep = __expf(m[r] - top[r]);
-        l[r] *= keep;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[r][e] *= keep;
-      }
-      m[r] = top[r];
+      for (int e = 0; e < 8; ++e) acc[r][e] = fmaf(ev, (float)vr[i][e], acc[r][e]);
     }
-#pragma unroll
-    for (int i = FROM; i < TO; ++i)
-#pragma unroll
-      for (int r = 0; r < R; ++r) {
-        const float ev = i * KPP + wave * KPW + g < S ? __expf(sc[r][i - FROM] - top[r]) : 0.f;
-        l[r] += ev;
-#pragma unroll
-        for (int e = 0; e < 8; ++e) acc[r][e] = fmaf(ev, (float)vr[i][e], acc[r][e]);
-      }
-  };
-  keys(std::integral_constant<int, 0>{}, std::integral_constant<int, FIRST>{});
-  if constexpr (FIRST < NP) keys(std::integral_constant<int, FIRST>{}, std::integral_constant<int, NP>{});
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
     // per wave: the weights of its keys (each key counted once: chunk 0 of its group) and, per chunk, the sum over
     // the wave's key groups
-    const float M = dec_wave_max(m[r]), keep = __expf(m[r] - M);
-    l[r] = dec_wave_sum(ch == 0 ? l[r] * keep : 0.f);
+    l[r] = dec_wave_sum(ch == 0 ? l[r] : 0.f);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) acc[r][e] = dec_stride_sum<LPK>(acc[r][e] * keep);
-    if (lane == 0) { red_m[r][wave] = M; red_l[r][wave] = l[r]; }
+    for (int e = 0; e < 8; ++e) acc[r][e] = dec_stride_sum<LPK>(acc[r][e]);
+    if (lane == 0) red_l[r][wave] = l[r];
     if (g == 0) {
 #pragma unroll
       for (int e = 0; e < 8; ++e) red_o[r][wave][ch * 8 + e] = acc[r][e];
@@ -734,15 +720,9 @@ __global__ __launch_bounds__(64 * NW, R == 1 && !PROJ ? 4 : 1) void dec_attn_ker
   __syncthreads();
   for (int t = tid; t < R * DH; t += 64 * NW) {
     const int r = t / DH, c = t - r * DH;
-    float M = red_m[r][0], L = 0.f, o = 0.f;
+    float L = 0.f, o = 0.f;
 #pragma unroll
-    for (int w = 1; w < NW; ++w) M = fmaxf(M, red_m[r][w]);
-#pragma unroll
-    for (int w = 0; w < NW; ++w) {
-      const float keep = __expf(red_m[r][w] - M);
-      L += red_l[r][w] * keep;
-      o += red_o[r][w][c] * keep;
-    }
+    for (int w = 0; w < NW; ++w) { L += red_l[r][w]; o += red_o[r][w][c]; }
     if constexpr (PROJ) result[r][c] = (bf16)(o / L);
     else p.out[(long long)b * p.o_sb + (head0 + r) * DH + c] = (bf16)(o / L);
   }
