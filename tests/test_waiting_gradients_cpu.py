@@ -1,0 +1,177 @@
+"""Weight gradients and norms' sums that wait for others belong to their backward pass.  Real backward passes on the CPU, the launches replaced by
+the sums that they stand for."""
+import gc
+import threading
+import weakref
+
+import pytest
+import torch
+
+from vyomai_amd import autograd_train as AT
+
+BF = torch.bfloat16
+KINDS = ["rows", "many rows", "norms"]
+M = {"rows": 8, "many rows": 2048}
+
+
+@pytest.fixture(autouse=True)
+def launches(monkeypatch):
+    """Sizes of the launches; a descriptor is the gradient's tensors."""
+    out = []
+
+    def add(items):
+        out.append(len(items))
+        for dy, x, dw, db in items:
+            dw.add_(dy.float().T @ x.float())
+
+    def norms(items):
+        out.append(len(items))
+        for _, _, dg, db in items:
+            dg.add_(1.0), db.add_(1.0)
+    monkeypatch.setattr(AT.ops, "_raw_stream", lambda: 0)
+    monkeypatch.setattr(AT.ops, "wgrad_desc", lambda dy, x, dw, db: ((dy, x, dw, db), (dy, x)))
+    monkeypatch.setattr(AT.ops, "wgrad_rows", add)
+    monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", add)
+    monkeypatch.setattr(AT.ops, "linear_wgrad", lambda dy, x, dw, db, accumulate, alpha=None: add([(dy, x, dw, db)]))
+    monkeypatch.setattr(AT.ops, "layernorm_sums", norms)
+    return out
+
+
+class Product(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w):
+        ctx.save_for_backward(x, w)
+        return x @ w.to(x.dtype).T
+
+    @staticmethod
+    def backward(ctx, dy):
+        x, w = ctx.saved_tensors
+        dw, _ = AT._wgrad(dy.contiguous(), x, w, None)
+        return dy @ w.to(dy.dtype), dw
+
+
+class Norm(torch.autograd.Function):
+    @staticmethod
+    def forward(ctx, x, w, b):
+        ctx.params = w, b
+        return x * 1.0
+
+    @staticmethod
+    def backward(ctx, dy):
+        w, b = ctx.params
+        AT._norm_sums.add_norms([(torch.zeros(2), 1, w.grad, b.grad, (w, b))])
+        return dy, None, None
+
+
+class Then(torch.autograd.Function):
+    """Calls something in the middle of the backward pass."""
+    @staticmethod
+    def forward(ctx, x, act):
+        ctx.act = act
+        return x * 1.0
+
+    @staticmethod
+    def backward(ctx, dy):
+        ctx.act()
+        return dy, None
+
+
+def parameter(shape, ready=None):
+    p = torch.nn.Parameter(torch.ones(shape))
+    p.grad, p._vy_direct = torch.zeros(shape), True
+    if ready is not None:
+        p._vy_ready = lambda q: ready.append(q)
+    return p
+
+
+def layer(kind, ready=None):
+    """-> its parameters, and what it makes of a tensor (of no tensor: of an input of its size)."""
+    if kind == "norms":
+        w, b = parameter((4,), ready), parameter((4,), ready)
+        return (w, b), lambda x=None: Norm.apply(torch.ones(2, 4, requires_grad=True) if x is None else x, w, b)
+    w = parameter((512, 512), ready)
+    return (w,), lambda x=None: Product.apply(torch.ones(M[kind], 512, dtype=BF, requires_grad=True) if x is None else x, w)
+
+
+def written(params):
+    return all(bool((p.grad != 0).all()) for p in params) and not any(getattr(p, "_vy_deferred", False) for p in params)
+
+
+def untouched(params):
+    return all(bool((p.grad == 0).all()) for p in params)
+
+
+@pytest.mark.parametrize("other", KINDS)
+@pytest.mark.parametrize("kind", KINDS)
+def test_two_passes_at_a_time(kind, other):
+    """One holds a gradient while the other begins and ends, and a trainer of the other clears its gradients."""
+    ready = []
+    pa, fa = layer(kind, ready)
+    pb, fb = layer(other, ready)
+    held, go, errors = threading.Event(), threading.Event(), []
+
+    def wait():
+        held.set()
+        assert go.wait(60)
+
+    def first():
+        try:
+            fa(Then.apply(torch.ones(M.get(kind, 2), 512 if kind in M else 4, dtype=BF if kind in M else None, requires_grad=True), wait)).float().sum().backward()
+        except BaseException as e:
+            errors.append(e)
+    t = threading.Thread(target=first)
+    t.start()
+    assert held.wait(60)
+    assert untouched(pa) and all(p._vy_deferred for p in pa)
+    fb().float().sum().backward()
+    assert written(pb) and {id(p) for p in ready} == {id(p) for p in pb}
+    assert untouched(pa) and all(p._vy_deferred for p in pa)
+    go.set()
+    t.join(60)
+    assert not errors and written(pa) and {id(p) for p in ready} == {id(p) for p in pa + pb}
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_pass_that_raises(kind, launches):
+    """It launches nothing, holds nothing, and the next one's gradients are written, those of the same parameters too."""
+    def fail():
+        raise RuntimeError("out of memory")
+    ready = []
+    p1, f1 = layer(kind, ready)
+    p2, f2 = layer(kind, ready)
+    x = Then.apply(torch.ones(M.get(kind, 2), 512 if kind in M else 4, dtype=BF if kind in M else None, requires_grad=True), fail)
+    kept = weakref.ref(x)
+    with pytest.raises(RuntimeError, match="out of memory"):
+        f1(x).float().sum().backward()
+    del x
+    gc.collect()
+    assert kept() is None and not launches and not ready and untouched(p1) and not any(p._vy_deferred for p in p1)
+    f2().float().sum().backward()
+    assert written(p2) and launches == [1]
+    f1().float().sum().backward()
+    assert written(p1) and launches == [1, 1] and len(ready) == len(p1) + len(p2)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_pass_inside_another(kind):
+    """A checkpoint that runs its own backward pass in the middle of one."""
+    from torch.utils.checkpoint import checkpoint
+    (p1, f1), (p2, f2), (p3, f3) = layer(kind), layer(kind), layer(kind)
+    y = f1()
+    f3(checkpoint(f2, y, use_reentrant=True)).float().sum().backward()
+    assert written(p1) and written(p2) and written(p3)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_backward_function_called_by_hand(kind):
+    """There is no end of a pass to wait for."""
+    class Ctx:
+        pass
+    ctx, (params, _) = Ctx(), layer(kind)
+    if kind == "norms":
+        ctx.params = params
+        Norm.backward(ctx, torch.ones(2, 4))
+    else:
+        ctx.saved_tensors = torch.ones(M[kind], 512, dtype=BF), params[0]
+        Product.backward(ctx, torch.ones(M[kind], 512, dtype=BF))
+    assert written(params)

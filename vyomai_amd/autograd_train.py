@@ -146,6 +146,30 @@ def _notify(*params) -> None:
                 cb(p)
 
 
+_graph_task = torch._C._current_graph_task_id
+
+
+class _Waiting:
+    """What waits of one backward pass in one group.  The pass's callback alone holds it, so it goes with its pass, whether that ends
+    or raises."""
+
+    __slots__ = ("at", "number", "items", "tiles", "armed", "key", "stream", "__weakref__")
+    numbers = itertools.count(1)
+
+    def __init__(self, at=None):
+        self.at, self.number = at, next(self.numbers)     # the backward pass (None: of none); what its parameters are marked with
+        self.items, self.tiles, self.armed, self.key, self.stream = [], 0, False, None, None
+
+    def unmark(self, items) -> None:
+        for *_, members in items:
+            for p in members:
+                if getattr(p, "_vy_deferred", False) == self.number:     # (not of a later pass)
+                    p._vy_deferred = False
+
+    def __del__(self):
+        self.unmark(self.items)
+
+
 class _WgradGroup:
     """Weight gradients that accumulate straight into the gradient arena do not have to be launched where
     autograd reaches them: the projections of a layer are small wgrad problems (9-36 tiles of 256 x 256),
@@ -154,14 +178,49 @@ class _WgradGroup:
     (per-bucket AdamW) when that launch has been enqueued, and its operands live until then (0.4 GB a layer at 16384 rows of
     768).  Parameters whose gradients are exchanged between ranks (training.BucketReducer) go out layer by layer: their buckets
     wait for the launch, and the exchange is what has to begin early.  Whatever is still pending when the backward pass ends is
-    flushed by an autograd-engine callback."""
+    flushed by an autograd-engine callback.
+
+    Every backward pass has its own (_Waiting): two threads' passes end at different times, and one that raises launches nothing and leaves
+    nothing to the next."""
 
     TILES = int(os.environ.get("VY_WGRAD_GROUP_TILES", "256"))   # most 256 x 256 output tiles of a launch: a CU each (a post-LN layer of 768: 108)
     MOST = 12                                                    # gradients of a launch
     EXCHANGED, EXCHANGED_MOST = 100, 8                           # exchanged gradients: as many tiles or gradients end a launch
 
     def __init__(self):
-        self.items, self.tiles, self.armed, self.key, self.stream = [], 0, False, None, None
+        self.passes = weakref.WeakValueDictionary()   # backward pass -> _Waiting
+        self.outside = _Waiting()                     # of no pass (nothing flushes it)
+
+    def _now(self) -> _Waiting:
+        task = _graph_task()
+        if task < 0:
+            return self.outside
+        w = self.passes.get(task)
+        if w is None:
+            w = self.passes[task] = _Waiting(task)
+            torch.autograd.Variable._execution_engine.queue_callback(functools.partial(self._end_of_backward, w))
+            w.armed = True
+        return w
+
+    def _here(self) -> _Waiting:
+        """Of the backward pass that asks; of none, if nothing of it waits."""
+        return self.passes.get(_graph_task(), self.outside)
+
+    @property
+    def items(self) -> list:
+        return self._here().items
+
+    @property
+    def tiles(self) -> int:
+        return self._here().tiles
+
+    @property
+    def armed(self) -> bool:
+        return self._here().armed
+
+    @armed.setter
+    def armed(self, value: bool) -> None:
+        self._here().armed = value
 
     def wants(self, dy, w, alpha) -> bool:
         if alpha is not None or not _GROUP_WGRADS:
@@ -175,70 +234,73 @@ class _WgradGroup:
     def add_tensors(self, dy, x, dw, db, members) -> None:
         """dw / db: the fp32 gradient tensors the launch accumulates into (views of the arena); members: the
         parameters to report ready once it has been enqueued (a packed projection has several).  A gradient of another type or
-        on another stream than those that are waiting goes out by itself."""
+        on another stream than those that are waiting, or of a backward function called by hand, goes out by itself."""
         key = dy is not None and (dy.dtype, ops._raw_stream())
-        if self.items and key != self.key:
+        w = self._now()
+        if not w.armed or (w.items and key != w.key):
             ops.linear_wgrad(dy, x, dw, db, accumulate=True)
             _notify(*members)
             return
         tiles = -(-dw.shape[0] // 256) * -(-dw.shape[1] // 256)
         exchanged = any(getattr(p, "_vy_exchanged", False) for p in members)
-        if self.tiles + tiles > self.TILES and not exchanged:
-            self.flush()
-        self._hold((dy, x, dw, db, members), tiles, key, exchanged)
+        if w.tiles + tiles > self.TILES and not exchanged:
+            self._flush(w)
+        self._hold(w, (dy, x, dw, db, members), tiles, key, exchanged)
 
-    def _hold(self, item, tiles, key, exchanged) -> None:
+    def _hold(self, w, item, tiles, key, exchanged) -> None:
         members = item[4]
-        if not self.items:
-            self.key, self.stream = key, torch.cuda.current_stream() if item[0] is not None and item[0].is_cuda else None
-        self.items.append(item)
+        if not w.items:
+            w.key, w.stream = key, torch.cuda.current_stream() if item[0] is not None and item[0].is_cuda else None
+        w.items.append(item)
         # autograd's own post-accumulate hook fires for these parameters as soon as this backward function
         # returns -- the reducer must not take that for "gradient written" (training.BucketReducer._hook)
         for p in members:
-            p._vy_deferred = True
-        self.tiles += tiles
-        if not self.armed:
-            torch.autograd.Variable._execution_engine.queue_callback(self._end_of_backward)
-            self.armed = True
+            p._vy_deferred = w.number
+        w.tiles += tiles
         if exchanged:
-            full = self.tiles >= min(self.TILES, self.EXCHANGED) or len(self.items) >= self.EXCHANGED_MOST
+            full = w.tiles >= min(self.TILES, self.EXCHANGED) or len(w.items) >= self.EXCHANGED_MOST
         else:
-            full = self.tiles >= self.TILES or len(self.items) >= self.MOST
+            full = w.tiles >= self.TILES or len(w.items) >= self.MOST
         if full:
-            self.flush()
+            self._flush(w)
 
     def flush(self) -> None:
-        items, self.items, self.tiles = self.items, [], 0
+        self._flush(self._here())
+
+    def _flush(self, w) -> None:
+        items, w.items, w.tiles = w.items, [], 0
         if not items:
             return
         self._launch([item[:4] for item in items])
-        if _norm_sums.items and _norm_sums.key[1] == ops._raw_stream():   # (so that whole buckets of parameters are ready)
-            _norm_sums.flush()
-        for *_, members in items:
-            for p in members:
-                p._vy_deferred = False
-            _notify(*members)
+        sums = _norm_sums.outside if w.at is None else _norm_sums.passes.get(w.at)
+        if sums is not None and sums.items and sums.key[1] == ops._raw_stream():   # (so that whole buckets of parameters are ready)
+            _norm_sums._flush(sums)
+        for item in items:
+            w.unmark((item,))
+            _notify(*item[4])
 
     def _launch(self, items) -> None:
         ops.linear_wgrad_grouped(items)
 
-    def _end_of_backward(self) -> None:
+    def _end_of_backward(self, w=None) -> None:
         """On the stream that the backward pass was called on.  What waits may be of another one, the forward pass's: it goes out there, where
         its operands were made, and the caller's stream waits for it."""
-        self.armed = False
-        if not self.items or self.stream is None or self.key[1] == ops._raw_stream():
-            self.flush()
+        w = self.outside if w is None else w
+        w.armed = False
+        if not w.items or w.stream is None or w.key[1] == ops._raw_stream():
+            self._flush(w)
             return
-        here, there = torch.cuda.current_stream(), self.stream
+        here, there = torch.cuda.current_stream(), w.stream
         with torch.cuda.stream(there):
-            self.flush()
+            self._flush(w)
         here.wait_stream(there)
 
     def discard(self) -> None:
-        for *_, members in self.items:
-            for p in members:
-                p._vy_deferred = False
-        self.items, self.tiles, self.armed = [], 0, False
+        for w in (self.outside, *[ref() for ref in self.passes.valuerefs()]):
+            if w is None:
+                continue
+            items, w.items, w.tiles = w.items, [], 0
+            w.unmark(items)
 
 
 class _WgradRows(_WgradGroup):
@@ -259,17 +321,18 @@ class _WgradRows(_WgradGroup):
     def add_descs(self, products, keep) -> None:
         """products: (vy_wgrad_desc, members) each; keep: every tensor they point into, the first one a bf16 operand."""
         key = (keep[0].dtype, ops._raw_stream())
-        if self.items and key != self.key:
+        w = self._now()
+        if not w.armed or (w.items and key != w.key):
             ops.wgrad_rows([desc for desc, _ in products])
             for _, members in products:
                 _notify(*members)
             return
-        if len(self.items) + len(products) > self.MOST:
-            self.flush()
+        if len(w.items) + len(products) > self.MOST:
+            self._flush(w)
         for desc, members in products:
-            self._hold((keep[0], desc, keep, None, members), 0, key, False)
-        if len(self.items) >= self.FULL:
-            self.flush()
+            self._hold(w, (keep[0], desc, keep, None, members), 0, key, False)
+        if len(w.items) >= self.FULL:
+            self._flush(w)
 
     def _launch(self, items) -> None:
         ops.wgrad_rows([item[1] for item in items])
@@ -289,13 +352,14 @@ class _NormSums(_WgradGroup):
     def add_norms(self, items) -> None:
         """items: (ws, rows, gradients of weight and bias, (weight, bias)) each."""
         key = (torch.float32, ops._raw_stream())
-        if (self.items and key != self.key) or any(getattr(p, "_vy_exchanged", False) for item in items for p in item[4]):
+        w = self._now()
+        if not w.armed or (w.items and key != w.key) or any(getattr(p, "_vy_exchanged", False) for item in items for p in item[4]):
             self._launch([item[:4] for item in items])
             for item in items:
                 _notify(*item[4])
             return
         for item in items:
-            self._hold(item, 0, key, False)
+            self._hold(w, item, 0, key, False)
 
     def _launch(self, items) -> None:
         ops.layernorm_sums(items)
