@@ -175,3 +175,32 @@ def test_a_backward_function_called_by_hand(kind):
         ctx.saved_tensors = torch.ones(M[kind], 512, dtype=BF), params[0]
         Product.backward(ctx, torch.ones(M[kind], 512, dtype=BF))
     assert written(params)
+
+
+@pytest.mark.parametrize("accumulate", [1, 3])
+@pytest.mark.parametrize("kind", KINDS)
+def test_trainers_that_clear_their_gradients(kind, accumulate):
+    """Another trainer's zero_grad() in the middle of a backward pass takes nothing away from it, and a micro-batch whose pass raised, nothing from
+    the next one, whether zero_grad() comes between them at the start of an accumulation window or inside of one."""
+    from vyomai_amd.training import FlatTrainer
+
+    def fail():
+        raise RuntimeError("out of memory")
+    mine = torch.nn.ParameterList(layer(kind)[0])
+    other = FlatTrainer(torch.nn.Linear(8, 8), compute_dtype=torch.float32)
+    tr = FlatTrainer(mine, compute_dtype=torch.float32, accumulate_steps=accumulate)
+
+    def loss(act):
+        x = Then.apply(torch.ones(M.get(kind, 2), 512 if kind in M else 4, dtype=BF if kind in M else None, requires_grad=True), act)
+        return (Norm.apply(x, *mine) if kind == "norms" else Product.apply(x, mine[0])).float().sum()
+    tr.zero_grad()
+    tr.backward(loss(other.zero_grad))
+    assert written(mine) and len(tr.reducer.touched) == len(mine)
+    tr.zero_grad()
+    before = [p.grad.clone() for p in mine]
+    with pytest.raises(RuntimeError, match="out of memory"):
+        tr.backward(loss(fail))
+    assert all(torch.equal(p.grad, g) for p, g in zip(mine, before))
+    tr.zero_grad()
+    tr.backward(loss(lambda: None))
+    assert written(mine) and all(bool((p.grad != g).all()) for p, g in zip(mine, before))

@@ -295,13 +295,6 @@ class _WgradGroup:
             self._flush(w)
         here.wait_stream(there)
 
-    def discard(self) -> None:
-        for w in (self.outside, *[ref() for ref in self.passes.valuerefs()]):
-            if w is None:
-                continue
-            items, w.items, w.tiles = w.items, [], 0
-            w.unmark(items)
-
 
 class _WgradRows(_WgradGroup):
     """The same for gradients over fewer rows than those: four layers' in a launch that sums each up as a launch of its own does

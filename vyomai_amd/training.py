@@ -482,9 +482,6 @@ class FlatTrainer:
         if 0 < self._micro < self.accumulate_steps:   # in the middle of an accumulation window: keep adding
             return
         self._micro = 0            # (a finished window that was never stepped is dropped here: its gradients are cleared)
-        from .autograd_train import _norm_sums, _wgrad_group, _wgrad_rows
-        for group in (_wgrad_group, _wgrad_rows, _norm_sums):
-            group.discard()   # (only an aborted backward can have left deferred weight gradients behind)
         self.arena.zero_grad()
         self.reducer.reset()
         self._stepped = set()
