@@ -204,3 +204,28 @@ def test_trainers_that_clear_their_gradients(kind, accumulate):
     tr.zero_grad()
     tr.backward(loss(lambda: None))
     assert written(mine) and all(bool((p.grad != g).all()) for p, g in zip(mine, before))
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_two_devices_in_a_pass(kind, monkeypatch):
+    """A launch has the gradients of one device: streams of two have the same handles, and the engine calls each one's backward functions in a
+    thread of its own."""
+    out = []
+    of = lambda items: {t.device.type for item in items for t in (item if kind != "norms" else item[2:])}
+    for name in ("wgrad_rows", "linear_wgrad_grouped", "layernorm_sums"):
+        monkeypatch.setattr(AT.ops, name, lambda items: out.append((len(items), *of(items))))
+
+    def hold():
+        for device in ("cpu", "meta") * 3:
+            if kind == "norms":
+                AT._norm_sums.add_norms([(None, 1, torch.zeros(4, device=device), torch.zeros(4, device=device), ())])
+            else:
+                dy, x, dw = (torch.zeros(512, 512, dtype=t, device=device) for t in (BF, BF, None))
+                (AT._wgrad_rows if kind == "rows" else AT._wgrad_group).add_tensors(dy, x, dw, None, [])
+    if kind == "rows":
+        monkeypatch.setattr(AT.ops, "wgrad_desc", lambda dy, x, dw, db: ((dy, x, dw), (dy, x)))
+    else:
+        real = AT.ops.linear_wgrad_grouped
+        monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", lambda items: real([item[:3] for item in items]))
+    Then.apply(torch.ones(2, requires_grad=True), hold).sum().backward()
+    assert sorted(out) == [(3, "cpu"), (3, "meta")]

@@ -150,14 +150,14 @@ _graph_task = torch._C._current_graph_task_id
 
 
 class _Waiting:
-    """What waits of one backward pass in one group.  The pass's callback alone holds it, so it goes with its pass, whether that ends
+    """What waits of one backward pass on one device, in one group.  The pass's callback alone holds it, so it goes with its pass, whether that ends
     or raises."""
 
     __slots__ = ("at", "number", "items", "tiles", "armed", "key", "stream", "__weakref__")
     numbers = itertools.count(1)
 
     def __init__(self, at=None):
-        self.at, self.number = at, next(self.numbers)     # the backward pass (None: of none); what its parameters are marked with
+        self.at, self.number = at, next(self.numbers)     # (backward pass, device), None: of none; what its parameters are marked with
         self.items, self.tiles, self.armed, self.key, self.stream = [], 0, False, None, None
 
     def unmark(self, items) -> None:
@@ -180,47 +180,51 @@ class _WgradGroup:
     wait for the launch, and the exchange is what has to begin early.  Whatever is still pending when the backward pass ends is
     flushed by an autograd-engine callback.
 
-    Every backward pass has its own (_Waiting): two threads' passes end at different times, and one that raises launches nothing and leaves
-    nothing to the next."""
+    Every backward pass has its own (_Waiting): two threads' passes end at different times, one that raises launches nothing and leaves
+    nothing to the next, and the engine calls a pass's backward functions in a thread for each device."""
 
     TILES = int(os.environ.get("VY_WGRAD_GROUP_TILES", "256"))   # most 256 x 256 output tiles of a launch: a CU each (a post-LN layer of 768: 108)
     MOST = 12                                                    # gradients of a launch
     EXCHANGED, EXCHANGED_MOST = 100, 8                           # exchanged gradients: as many tiles or gradients end a launch
 
     def __init__(self):
-        self.passes = weakref.WeakValueDictionary()   # backward pass -> _Waiting
+        self.passes = weakref.WeakValueDictionary()   # (backward pass, device) -> _Waiting
         self.outside = _Waiting()                     # of no pass (nothing flushes it)
 
-    def _now(self) -> _Waiting:
+    def _now(self, device) -> _Waiting:
         task = _graph_task()
         if task < 0:
             return self.outside
-        w = self.passes.get(task)
+        w = self.passes.get((task, device))
         if w is None:
-            w = self.passes[task] = _Waiting(task)
+            w = self.passes[(task, device)] = _Waiting((task, device))
             torch.autograd.Variable._execution_engine.queue_callback(functools.partial(self._end_of_backward, w))
             w.armed = True
         return w
 
-    def _here(self) -> _Waiting:
-        """Of the backward pass that asks; of none, if nothing of it waits."""
-        return self.passes.get(_graph_task(), self.outside)
+    def _here(self) -> list:
+        """Of the backward pass that asks, on every device."""
+        task = _graph_task()
+        if task < 0:
+            return [self.outside]
+        return [w for w in [ref() for ref in self.passes.valuerefs()] if w is not None and w.at[0] == task]
 
     @property
     def items(self) -> list:
-        return self._here().items
+        return [item for w in self._here() for item in w.items]
 
     @property
     def tiles(self) -> int:
-        return self._here().tiles
+        return sum(w.tiles for w in self._here())
 
     @property
     def armed(self) -> bool:
-        return self._here().armed
+        return any(w.armed for w in self._here())
 
     @armed.setter
     def armed(self, value: bool) -> None:
-        self._here().armed = value
+        for w in self._here():
+            w.armed = value
 
     def wants(self, dy, w, alpha) -> bool:
         if alpha is not None or not _GROUP_WGRADS:
@@ -236,7 +240,7 @@ class _WgradGroup:
         parameters to report ready once it has been enqueued (a packed projection has several).  A gradient of another type or
         on another stream than those that are waiting, or of a backward function called by hand, goes out by itself."""
         key = dy is not None and (dy.dtype, ops._raw_stream())
-        w = self._now()
+        w = self._now(dw.device)
         if not w.armed or (w.items and key != w.key):
             ops.linear_wgrad(dy, x, dw, db, accumulate=True)
             _notify(*members)
@@ -265,7 +269,8 @@ class _WgradGroup:
             self._flush(w)
 
     def flush(self) -> None:
-        self._flush(self._here())
+        for w in self._here():
+            self._flush(w)
 
     def _flush(self, w) -> None:
         items, w.items, w.tiles = w.items, [], 0
@@ -283,11 +288,11 @@ class _WgradGroup:
         ops.linear_wgrad_grouped(items)
 
     def _end_of_backward(self, w=None) -> None:
-        """On the stream that the backward pass was called on.  What waits may be of another one, the forward pass's: it goes out there, where
-        its operands were made, and the caller's stream waits for it."""
+        """On the stream that the backward pass was called on.  What waits may be of another one, the forward pass's, or of another device: it goes
+        out there, where its operands were made, and the caller's stream waits for it."""
         w = self.outside if w is None else w
         w.armed = False
-        if not w.items or w.stream is None or w.key[1] == ops._raw_stream():
+        if not w.items or w.stream is None or (w.key[1] == ops._raw_stream() and (w.at is None or w.at[1].index == torch.cuda.current_device())):
             self._flush(w)
             return
         here, there = torch.cuda.current_stream(), w.stream
@@ -314,7 +319,7 @@ class _WgradRows(_WgradGroup):
     def add_descs(self, products, keep) -> None:
         """products: (vy_wgrad_desc, members) each; keep: every tensor they point into, the first one a bf16 operand."""
         key = (keep[0].dtype, ops._raw_stream())
-        w = self._now()
+        w = self._now(keep[0].device)
         if not w.armed or (w.items and key != w.key):
             ops.wgrad_rows([desc for desc, _ in products])
             for _, members in products:
@@ -345,7 +350,7 @@ class _NormSums(_WgradGroup):
     def add_norms(self, items) -> None:
         """items: (ws, rows, gradients of weight and bias, (weight, bias)) each."""
         key = (torch.float32, ops._raw_stream())
-        w = self._now()
+        w = self._now(items[0][2].device)
         if not w.armed or (w.items and key != w.key) or any(getattr(p, "_vy_exchanged", False) for item in items for p in item[4]):
             self._launch([item[:4] for item in items])
             for item in items:
