@@ -229,3 +229,32 @@ def test_two_devices_in_a_pass(kind, monkeypatch):
         monkeypatch.setattr(AT.ops, "linear_wgrad_grouped", lambda items: real([item[:3] for item in items]))
     Then.apply(torch.ones(2, requires_grad=True), hold).sum().backward()
     assert sorted(out) == [(3, "cpu"), (3, "meta")]
+
+
+@pytest.mark.parametrize("which", ["dy", "x"])
+@pytest.mark.parametrize("kind", ["rows", "many rows"])
+def test_operands_that_no_launch_takes(kind, which, launches, monkeypatch):
+    """Rows that do not start on 16 bytes are refused where their layer is reached, not with those of other layers that waited."""
+    def refuse(dy, x, dw, db, accumulate, alpha=None):
+        assert accumulate and any(t.data_ptr() % 16 or t.stride(0) % 8 for t in (dy, x))
+        raise AT._lib.VyomHipError("vy_linear_wgrad: operands")
+    monkeypatch.setattr(AT.ops, "linear_wgrad", refuse)
+    w = parameter((512, 512))
+    odd, even = torch.ones(M[kind], 520, dtype=BF)[:, 1:513], torch.ones(M[kind], 512, dtype=BF)
+    for pair in ((odd, even), (torch.ones(M[kind], 513, dtype=BF)[:, :512], even)):
+        with pytest.raises(AT._lib.VyomHipError, match="operands"):
+            Then.apply(torch.ones(2, requires_grad=True), lambda: AT._wgrad(*(pair if which == "dy" else pair[::-1]), w, None)).sum().backward()
+    assert not launches and not getattr(w, "_vy_deferred", False)
+
+
+@pytest.mark.parametrize("kind", KINDS)
+def test_a_launch_that_fails(kind, monkeypatch):
+    """Nothing is left marked as waiting."""
+    def fail(items):
+        raise AT._lib.VyomHipError("launch failed")
+    for name in ("wgrad_rows", "linear_wgrad_grouped", "layernorm_sums"):
+        monkeypatch.setattr(AT.ops, name, fail)
+    params, apply = layer(kind)
+    with pytest.raises(AT._lib.VyomHipError, match="launch failed"):
+        apply().float().sum().backward()
+    assert not any(p._vy_deferred for p in params)

@@ -276,13 +276,15 @@ class _WgradGroup:
         items, w.items, w.tiles = w.items, [], 0
         if not items:
             return
-        self._launch([item[:4] for item in items])
+        try:
+            self._launch([item[:4] for item in items])
+        finally:
+            w.unmark(items)
         sums = _norm_sums.outside if w.at is None else _norm_sums.passes.get(w.at)
         if sums is not None and sums.items and sums.key[1] == ops._raw_stream():   # (so that whole buckets of parameters are ready)
             _norm_sums._flush(sums)
-        for item in items:
-            w.unmark((item,))
-            _notify(*item[4])
+        for *_, members in items:
+            _notify(*members)
 
     def _launch(self, items) -> None:
         ops.linear_wgrad_grouped(items)
@@ -336,6 +338,12 @@ class _WgradRows(_WgradGroup):
         ops.wgrad_rows([item[1] for item in items])
 
 
+def _aligned(dy, x) -> bool:
+    """Does a launch take these operands, as rows on 16 bytes (or as copies)?  One that does not would take others with it: it is launched, and
+    refused, where its layer is reached."""
+    return all(t.dtype != BF16 or t.stride(-1) != 1 or (t.data_ptr() % 16 == 0 and t.stride(-2) % 8 == 0 and t.stride(-2) >= t.shape[-1]) for t in (dy, x))
+
+
 def _few_rows(M, N, K) -> bool:
     """Does a weight gradient N x K over M rows wait for those of other layers with few rows?"""
     return _GROUP_WGRADS and M < _GROUP_MIN_ROWS and N < 8192 and N * K >= 512 * 512 and K % 8 == 0
@@ -378,11 +386,13 @@ _norm_sums = _NormSums()
 def _wgrad(dy, x, w: torch.Tensor, b: Optional[torch.Tensor], alpha: Optional[torch.Tensor] = None):
     """-> (dw, db) to return to autograd (None when accumulated in place)."""
     if _direct(w) and (b is None or _direct(b)):
+        group = None
         if _wgrad_group.wants(dy, w, alpha):
-            _wgrad_group.add(dy, x, w, b)
-            return None, None
-        if _wgrad_rows.gathers(dy, w.shape, [p for p in (w, b) if p is not None], alpha):
-            _wgrad_rows.add(dy, x, w, b)
+            group = _wgrad_group
+        elif _wgrad_rows.gathers(dy, w.shape, [p for p in (w, b) if p is not None], alpha):
+            group = _wgrad_rows
+        if group is not None and _aligned(dy, x):
+            group.add(dy, x, w, b)
             return None, None
         ops.linear_wgrad(dy, x, w.grad, None if b is None else b.grad, accumulate=True, alpha=alpha)
         _notify(w, b)
@@ -729,7 +739,7 @@ class TextLayerFn(torch.autograd.Function):
         own = torch.empty(on, dtype=dt, device=dev)
         dx = torch.empty_like(x)
         nw = 1 if att._fused_qkv else 3
-        waiting = TextLayerFn._waiting(M, d, W, inner, dt, (*params[:10], *members), nw) if x.is_contiguous() else None
+        waiting = TextLayerFn._waiting(M, d, W, inner, dt, (*params[:10], *members), nw) if x.is_contiguous() and x.data_ptr() % 16 == 0 else None
         wait = waiting is not None or (_GROUP_WGRADS and all(_direct(p) for p in (g1, b1, g2, b2)))    # the norms' column sums go out with other layers'
         scratch = torch.empty(fo[1] if wait else fn, dtype=torch.float32, device=dev)
         sums = torch.empty((2, 2 * slabs * d), dtype=torch.float32, device=dev) if wait else None
@@ -857,11 +867,12 @@ def _packed_wgrad(mod, dy, x, w, b, params, members=None):
             ok = ok and all(p.grad.data_ptr() == db0.data_ptr() + off * 4 for p, off in zip(bs, _offsets(bs)))
         if ok:
             dy2 = dy.view(-1, dy.shape[-1])
-            if _GROUP_WGRADS and _GROUP_QKV and dy2.shape[0] >= _GROUP_MIN_ROWS and N * dw.shape[1] >= 512 * 512 and dw.shape[1] % 8 == 0:
+            may = _GROUP_QKV and _aligned(dy2, x)
+            if _GROUP_WGRADS and may and dy2.shape[0] >= _GROUP_MIN_ROWS and N * dw.shape[1] >= 512 * 512 and dw.shape[1] % 8 == 0:
                 # with the layer's other weight gradients in one grouped launch (27 of its 108 tiles: on its own
                 # this launch ran at 670 TFLOP/s, the group at 850)
                 _wgrad_group.add_tensors(dy2, x, dw, db, list(members))
-            elif _GROUP_QKV and _wgrad_rows.gathers(dy2, dw.shape, members):
+            elif may and _wgrad_rows.gathers(dy2, dw.shape, members):
                 _wgrad_rows.add_tensors(dy2, x, dw, db, list(members))
             else:
                 ops.linear_wgrad(dy, x, dw, db, accumulate=True)
