@@ -755,7 +755,9 @@ __global__ __launch_bounds__(256, PAIR ? 2 : 3) void attn_bwd_dq_kernel(BwdParam
     // key of register r: k0 + 4fh + kofs, kofs = 32kb + (r&3) + 8(r>>2); visible iff kofs <= klim
     int klim = p.S - 1 - k0 - 4 * fh;
     if (causal) klim = min(klim, qi + p.start_pos - k0 - 4 * fh);
-    const unsigned long long lm = need_mask ? (range_bits64(0, klim + 1) & (vis >> (4 * fh))) : ~0ull;
+    // (a choice of two scalar words, not a shift by 4 fh: its register pair was spilled, and the reload waited for every request under way:
+    // both kernels, causal 32 x 512 112.2 -> 110.7 us, with padding 106.0 -> 104.4)
+    const unsigned long long lm = need_mask ? (range_bits64(0, klim + 1) & (fh ? vis >> 4 : vis)) : ~0ull;
     const unsigned lmw[2] = {(unsigned)lm, (unsigned)(lm >> 32)};
     auto products = [&](int kb, f32x16& st, f32x16& dp) {
 #pragma unroll
