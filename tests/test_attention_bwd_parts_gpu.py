@@ -13,6 +13,7 @@ CASES = [
     (1, 3, 1, 127, 96, False, 0, None, False), (1, 4, 2, 128, 128, True, 0, "end", True), (1, 6, 2, 129, 129, True, 0, "start", True),
     (2, 6, 2, 200, 200, True, 0, "end", True), (1, 2, 1, 256, 257, True, 1, None, False), (1, 2, 2, 333, 333, False, 0, "end", True),
     (1, 12, 4, 700, 700, True, 0, "all", True), (2, 12, 12, 512, 512, True, 0, None, False),   # (the last: 384 workgroups of 32 keys)
+    (10, 12, 12, 128, 128, False, 0, "end", True), (11, 12, 12, 128, 128, False, 0, "end", True),   # (up to and past half of the CUs)
 ]
 
 

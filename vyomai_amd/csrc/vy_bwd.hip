@@ -2080,17 +2080,20 @@ extern "C" int vy_attn_bwd(const void* q, int64_t q_sb, int64_t q_sh, int64_t q_
   // dK/dV kernel; attn_delta_kernel remains for reference)
   // with at most one workgroup a CU a wave has its SIMD to itself and the kernels are as long as one workgroup's chain: then the waves
   // share the tiles (dQ by two, dK/dV by two or four; 4 needs more than one tile of rows and all its workgroups at once, a CU holds one.
-  // Under a causal mask the later half of many rows is short and fills in).  us of dQ / dK,dV at 12 heads, whole | by two | by four:
+  // Under a causal mask the later half of many rows is short and fills in.  Two tiles of rows in all are as soon done by whole waves where
+  // more than half of the CUs have a workgroup).  us of dQ / dK,dV at 12 heads, whole | by two | by four:
   // 5 x 333, 4 kv heads 14.1 / 30.9 | 12.2 / 25.3 | 18.2; 1 x 700, 4 kv heads 18.4 / 50.2 | 13.8 / 38.3 | 26.6; causal 2 x 512 15.2 / 16.0
-  // | 11.4 / 12.3 | 11.4; 8 x 256 10.7 / 11.1 | 10.7 / 11.4 | 17.1; 12 x 197 14.2 / 13.4 | 16.4 / 15.8 | -; 32 x 512 45.7 / 60.8 |
-  // 68.2 / 71.4 | 154; both kernels, 8 x 44 11.9 | 11.1 | 11.9
+  // | 11.4 / 12.3 | 11.4; 12 x 197 14.2 / 13.4 | 16.4 / 15.8 | -; 32 x 512 45.7 / 60.8 | 68.2 / 71.4 | 154; both kernels, dK/dV whole and what
+  // it gains or loses by two: 8 x 256 23.2 -0.1, causal 22.9 -1.0; 21 x 128 20.2 +0.5 and 19.6 +0.3, 10 x 128 16.7 -1.3 and 16.0 -1.1;
+  // 8 x 197 22.0 +0.4 and 20.8 -0.8, 10 x 197 23.3 +0.1 and 21.8 -1.0; 7 x 333 30.2 -0.6 and 27.6 -1.5
   constexpr int64_t CUS = 256;
   const int64_t wq = B * h * ((L + 127) / 128), wkv = B * hk * ((S + 127) / 128), wkv4 = B * hk * ((S + 31) / 32);
   if (wq <= CUS) hipLaunchKernelGGL(attn_bwd_dq_kernel<true>, dim3((unsigned)(h * B), (unsigned)((L + 63) / 64), 1), dim3(256), 0, st, p);
   else hipLaunchKernelGGL(attn_bwd_dq_kernel<false>, dim3((unsigned)(h * B), (unsigned)((L + 127) / 128), 1), dim3(256), 0, st, p);
   VY_CHECK_LAUNCH("vy_attn_bwd(dq)");
   const int64_t at_once = (mask_kind & VY_MASK_CAUSAL) && L >= 512 ? 2 * CUS : CUS;
-  const int split = L > 64 && wkv4 <= at_once ? 4 : wkv <= CUS ? 2 : 1;
+  const int64_t at_most = (h / hk) * L > 128 ? CUS : CUS / 2;
+  const int split = L > 64 && wkv4 <= at_once ? 4 : wkv <= at_most ? 2 : 1;
   const dim3 gkv((unsigned)(hk * B), (unsigned)((S * split + 127) / 128), 1);
   if (split == 4) hipLaunchKernelGGL(attn_bwd_dkdv_kernel<4>, gkv, dim3(256), 0, st, p);
   else if (split == 2) hipLaunchKernelGGL(attn_bwd_dkdv_kernel<2>, gkv, dim3(256), 0, st, p);
