@@ -448,7 +448,9 @@ int vy_linear_wgrad_grouped(const vy_wgrad_desc* descs, int32_t n, int dtype, vo
 /* vy_linear_wgrad_batch: the same for up to 12. */
 int vy_linear_wgrad_batch(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
 /* vy_linear_wgrad_rows: the same for up to 20 bf16 gradients over few rows, each summed up in the slices of rows that
- * vy_linear_wgrad takes for its shape; the slices' sums are added up in their order and added to dW_i once. */
+ * vy_linear_wgrad takes for its shape; the slices' sums are added up in their order and added to dW_i once, where vy_linear_wgrad adds
+ * each to dW as it is done: the same bits for one slice, and for two into a gradient of zeros; else a rounding for each slice apart, as two
+ * runs of vy_linear_wgrad with three slices are.  n = 1 is vy_linear_wgrad itself. */
 int vy_linear_wgrad_rows(const vy_wgrad_desc* descs, int32_t n, int dtype, void* stream);
 
 /* LayerNorm backward: dx = rstd*(g - mean(g) - xhat*mean(g*xhat)), g = dy*gamma;

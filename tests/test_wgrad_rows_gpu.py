@@ -37,6 +37,31 @@ def test_rows(M):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M", [200, 400, 1665])
+def test_rows_are_added_to_fractions(M):
+    """Gradients that are not zero: g + (s1 + s2) here, (g + s1) + s2 or (g + s2) + s1 by launches of their own.  The same bits from one slice; else
+    a rounding for each slice and its sum, at most 8 slices, apart, and so is the only gradient of a launch."""
+    from vyomai_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    for shapes in (SHAPES, SHAPES[:1]):
+        items, alone = [], []
+        for N, K in shapes:
+            dy = torch.randn(M, (N + 7) // 8 * 8, device=DEV, generator=g).to(BF)[:, :N]
+            x, start = torch.randn(M, K, device=DEV, generator=g).to(BF), torch.randn(N, K, device=DEV, generator=g)
+            items.append((dy, x, start.clone(), None))
+            alone.append((start, start.clone()))
+            ops.linear_wgrad(dy, x, alone[-1][1], None, True)
+        ops.linear_wgrad_rows(items)
+        for (dy, x, dw, _), (start, dw1) in zip(items, alone):
+            d = dy.double()
+            size, want = d.abs().T.contiguous() @ x.double().abs() + start.double().abs(), start.double() + d.T.contiguous() @ x.double()
+            assert ((dw.double() - want).abs() <= (M + 3) * 2.0 ** -24 * size).all()
+            assert ((dw - dw1).double().abs() <= 16 * 2.0 ** -24 * size).all()
+            if M <= 256:
+                assert torch.equal(dw, dw1)
+
+
+@pytest.mark.gpu
 def test_rows_are_added_to_what_is_there():
     """Two gradients of one weight in one launch, and launches on two streams: whole numbers, exact in any order."""
     from vyomai_amd import ops

@@ -304,8 +304,9 @@ class _WgradGroup:
 
 
 class _WgradRows(_WgradGroup):
-    """The same for gradients over fewer rows than those: four layers' in a launch that sums each up as a launch of its own does
-    (ops.wgrad_rows), so they keep their bits.  Exchanged gradients go out one by one."""
+    """The same for gradients over fewer rows than those: four layers' in a launch that sums each up in the slices of rows of a launch of its own
+    (ops.wgrad_rows), in one of the orders in which their sums may arrive there: the same bits up to 256 rows, and up to 512 into a gradient
+    of zeros; beyond, and where one is left alone in a launch, they differ as two runs of one by one do.  Exchanged gradients go out one by one."""
 
     MOST, FULL = 20, 16     # gradients of a launch; four layers' (with the language model head's dense layer before them: 17) fill it
 
@@ -375,7 +376,7 @@ _GROUP_WGRADS = os.environ.get("VY_WGRAD_GROUP", "1") != "0"
 _DEFER_RESIDUALS = os.environ.get("VY_DEFER_RESIDUALS", "1") != "0"
 _GROUP_MIN_ROWS = int(os.environ.get("VY_WGRAD_GROUP_ROWS", "2048"))   # 2112 rows of width 768, a layer's four gradients: 121 us one by one,
 # 58 of a launch with its neighbours'.  Below, tiles of 128 x 128 that sum the rows up as launches one by one do are faster (2047 rows 50,
-# 1665 rows 45 / 52 / 113 one by one) and keep the bits: another order changes gradients by 2e-7, and a step's weights in enough places that the
+# 1665 rows 45 / 52 / 113 one by one) and keep the slices: other sums change gradients by 2e-7, and a step's weights in enough places that the
 # next one's gradients, whose noise is the rounding of bf16, differ by 1 % from what they were (single values by more than the tensor's mean).
 _GROUP_QKV = os.environ.get("VY_WGRAD_GROUP_QKV", "1") != "0"              # the packed QKV gradient joins the group
 _wgrad_group = _WgradGroup()

@@ -486,8 +486,8 @@ __global__ __launch_bounds__(BN * 2, 1) void wgrad_tn_bf16_grouped_kernel(WgradG
 
 // The weight gradients of several layers over few rows (vy_linear_wgrad_rows): a workgroup a tile of 128 x 128, all rows.  One by one, a
 // launch has 36 to 144 tiles and fills the chip with slices of rows, up to 7 of them, whose fp32 atomics bound it (1.2 TB/s); with
-// four layers in a launch -- 1728 tiles, two on a CU -- an element is added to once, and the slices live on as the order of its sum, so the
-// bits stay.  The four gradients of a layer of width 768, one by one / here, us: 24 rows 37.6 / 23.9 (the atomics of one sum), 180 rows
+// four layers in a launch -- 1728 tiles, two on a CU -- an element is added to once, and the slices live on as the order of its sum (one of
+// those in which the atomics may come).  The four gradients of a layer of width 768, one by one / here, us: 24 rows 37.6 / 23.9 (the atomics of one sum), 180 rows
 // 45.2 / 24.8, 512 rows 69.6 / 27.9, 1000 rows 97.9 / 35.2, 1665 rows 113 / 45.5, 2047 rows 121 / 50.2 (tiles of 256 x 128 50.5 at 1665 rows).
 struct WgradRowsItem {
   const bf16* dY; const bf16* X; float* dW; float* db;
@@ -1343,7 +1343,7 @@ int wgrad_f32(const char* who, const void* dy, int64_t lddy, const void* x, int6
 
 // Rows of the slices that a gradient over M rows is summed up in, for the workgroups that `goal` asks for and so many tiles
 static int64_t wgrad_slice(int64_t M, int64_t tiles, int64_t goal) {
-  const int64_t most = vy_cdiv(M, 256), splits = vy_cdiv(goal, tiles);   // (a slice has 256 rows at least: 4 stages of 64)
+  const int64_t most = vy_cdiv(M, 256), splits = vy_cdiv(goal, tiles);   // (one slice for every 256 rows begun, of whole stages: 257 rows 192 and 65)
   return vy_cdiv(vy_cdiv(M, splits < 1 ? 1 : splits > most ? most : splits), 64) * 64;
 }
 constexpr int WGRAD_GOAL = 384;   // ~1.5 workgroups of 128 x 128 per CU

@@ -440,7 +440,8 @@ def wgrad_desc(dy: Tensor, x: Tensor, dw: Tensor, db: Optional[Tensor]):
 
 
 def wgrad_rows(descs) -> None:
-    """The same for up to 20 bf16 gradients over few rows, each with the sums of linear_wgrad (vy_linear_wgrad_rows); descs: wgrad_desc's."""
+    """The same for up to 20 bf16 gradients over few rows, each with the slices of linear_wgrad in their order (vy_linear_wgrad_rows); descs:
+    wgrad_desc's."""
     n = len(descs)
     assert 1 <= n <= 20
     call("vy_linear_wgrad_rows", C.cast((_lib.VyWgradDesc * n)(*descs), C.c_void_p), n, _lib.VY_BF16, _stream())
