@@ -344,7 +344,8 @@ __device__ __forceinline__ int w_row(int n0, int R, int N) {
 // table in LDS while its first stage is on its way, with the very expressions that it replaces (the same bits), for 2^-20 <= |x| < 16
 // and both signs; a wave with any other value in its chunk evaluates them.  Evaluated, the erf GELU's 21 vector instructions an element
 // (two at a quarter of the rate) were 9 of the 15 us that the epilogue of a 256 x 256 tile took next to a loop of 19 us (K = 768).
-// 256 x 192 tiles and the smaller ones, which share a CU, evaluate.
+// 128 x 128 tiles and smaller ones, which share a CU, evaluate, and so do 256 x 192 (which would have room: 16384 x 768, K = 768, 30.3 -> 27.4 us,
+// 3072 wide 103.6 -> 91.9; the tiles chosen there take 27.9 and 87.5, and so on at five more sizes, so a table would change next to nothing).
 // 16384 x 3072, K = 768: 107 -> 95 us, with the derivative saved 112 -> 95; 30500 rows 195 -> 171 and 218 -> 181; gated SiLU (there the
 // division), 8192 x 2 x 8192, K = 2048: 508 -> 501 us, 8192 x 2 x 4096, K = 1024: 135 -> 132.
 constexpr unsigned ACT_TAB_LOW = (127 - 20) << 7, ACT_TAB_HALF = 24 << 7;   // first magnitude's bits, entries per sign
@@ -1044,7 +1045,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_kernel(
 template <int BM, int BN, int WGM, int WGN, int EPI, int ACT, bool GRAD>
 __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
-    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob) {
+    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq) {
   constexpr int NW = WGM * WGN;
   constexpr int TM = BM / (16 * WGM), TN = BN / (16 * WGN);   // 256 x 256, 4 x 2 waves: 4, 8;  224 x 256, 2 x 4 waves: 7, 4;  128 x 128, 2 x 2 waves: 4, 4
   constexpr int PX = BM / 8, PW = BN / 8;
@@ -1253,7 +1254,7 @@ __global__ __launch_bounds__(64 * WGM * WGN) void gemm_nt_bf16_m16_kernel(
 template <int KG, int NBUF, int MOST, int BM, int EPI, int ACT, bool GRAD>
 __global__ __launch_bounds__(256 * KG) void gemm_nt_bf16_small_kernel(
     const bf16* __restrict__ X, int64_t ldx, const bf16* __restrict__ W, int64_t ldw, int M, int N,
-    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int knob, int per) {
+    int K, int tiles_n, EpiPlain<bf16> ep, EpiQkv<bf16> eq, int per) {
   constexpr int BN = 64, WGM = 2, WGN = 2, NW = 4;
   constexpr int TM = BM / 32, TN = 2, PX = BM / 32, PW = 2;   // 16 x 16 blocks and 1 KiB pieces of X and W per wave
   constexpr int STAGE = (BM + BN) * ROWB, RING = NBUF * STAGE;
@@ -1690,7 +1691,7 @@ inline double tile_cost(int64_t M, int64_t N, int64_t K, int S, int chip) {
     }
   }
 }
-// What a GELU adds on tiles of `rows` rows that take all of K: 2 us a tile of a CU, 6 where the tile has no table (256 x 192), and little on 64 x 64
+// What a GELU adds on tiles of `rows` rows that take all of K: 2 us a tile of a CU, 6 on 256 x 192, which has no table, and little on 64 x 64
 // tiles, which share a CU (medians over 150 shapes: 2.6, 2.2 and 1.8 us on 256, 224 and 160 x 256, 1.9 on 256 x 128, 2.3 on 128 x 128, 6.0, 0.3).
 // 32237 x 1920, K = 432: 100.9 us on 256 x 192, 79.8 on 256 x 256.  (Not beside a residual, where nobody looks up: 12.5, 10.2, 7.4; 6.7; 3.1; 8.1.)
 inline double gelu_cost(TileKind kind, int64_t M, int64_t N, int rows, int chip) {
@@ -2536,7 +2537,7 @@ __global__ __launch_bounds__(256) void gemv_bf16_kernel(const bf16* __restrict__
 template <int EPI, int ACT, bool GRAD>
 int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t M, int64_t N,
                 int64_t K, const EpiPlain<bf16>& ep, const EpiQkv<bf16>& eq, hipStream_t st) {
-  static const int rot = [] { const char* e = getenv("VY_GEMM_ROT"); return e ? atoi(e) : 0; }();  // rotated k order: measured 1-5 % slower
+  static const int rot = [] { const char* e = getenv("VY_GEMM_ROT"); return e ? atoi(e) : 0; }();  // gemm_nt_bf16_kernel's rotated k order: measured 1-5 % slower
   static const int gemv_on = [] { const char* e = getenv("VY_GEMV"); return e ? atoi(e) : 1; }();
   static const int skinny16_on = [] { const char* e = getenv("VY_SKINNY16"); return e ? atoi(e) : 1; }();
   static const int64_t skinny_max_n = [] { const char* e = getenv("VY_SKINNY_MAXN"); return e ? (int64_t)atoll(e) : (int64_t)8192; }();   // wider (the vocabulary): 32 x 128 tiles with X staged once per workgroup -- 15.5 vs 31.1 us at N = 50265
@@ -2575,12 +2576,14 @@ int launch_bf16(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t 
     const int bm = var >= 0 ? 256 : t.rows, bn = var == 8 ? 256 : var == 9 ? 192 : TILE_N[t.kind];
     const int tn = (int)vy_cdiv(N, bn), tiles = (int)vy_cdiv(M, bm) * tn, threads = var >= 0 ? 512 : TILE_THREADS[t.kind];
     const int KT = (int)vy_cdiv(K, BK), per = t.slices ? (KT + t.slices - 1) / t.slices : KT;
-#define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot)
-#define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot, per)
+#define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq)
+#define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, per)
     if (var >= 0) {
       if constexpr (EPI == 0 && !GRAD) {
-        if (var == 8) VY_TILES(gemm_nt_bf16_kernel<256, 256, 4, 2, EPI, ACT, GRAD>);
-        else VY_TILES(gemm_nt_bf16_kernel<256, 192, 4, 2, EPI, ACT, GRAD>);
+#define VY_WIDE(BN) hipLaunchKernelGGL((gemm_nt_bf16_kernel<256, BN, 4, 2, EPI, ACT, GRAD>), dim3(tiles), dim3(threads), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, eq, rot)
+        if (var == 8) VY_WIDE(256);
+        else VY_WIDE(192);
+#undef VY_WIDE
       }
     } else switch (t.kind) {
       case T_256x256:
@@ -2621,8 +2624,8 @@ int launch_gated(const bf16* X, int64_t ldx, const bf16* W, int64_t ldw, int64_t
   const Tiling t = pick_tiling(M, N, K, 256 / g_chains, splitk_ws(st).bytes, 3.0);
   const int tn = (int)vy_cdiv(N, TILE_N[t.kind]), tiles = (int)vy_cdiv(M, t.rows) * tn;
   const int KT = (int)vy_cdiv(K, BK), per = (KT + t.slices - 1) / t.slices;
-#define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0)
-#define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, 0, per)
+#define VY_TILES(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{})
+#define VY_SMALL(...) hipLaunchKernelGGL((__VA_ARGS__), dim3(tiles), dim3(TILE_THREADS[t.kind]), 0, st, X, ldx, W, ldw, (int)M, (int)N, (int)K, tn, ep, EpiQkv<bf16>{}, per)
   switch (t.kind) {
     case T_256x256:
       if (t.rows == 224) VY_TILES(gemm_nt_bf16_m16_kernel<224, 256, 2, 4, 2, ACT, false>);
