@@ -755,8 +755,9 @@ int dec_attn_go(const DecAttnArgs& a, int B, int Smax, hipStream_t st) {
   else if (np <= 5) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 5, NT, R, PROJ>), grid, block, 0, st, a);
   else if (np <= 7) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 7, NT, R, PROJ>), grid, block, 0, st, a);
   else if (np <= 10) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 10, NT, R, PROJ>), grid, block, 0, st, a);
-  else if (np <= 12) hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 12, NT, R, PROJ>), grid, block, 0, st, a);
-  else return 1;
+  else if (np > 12) return 1;
+  else if constexpr (PROJ && R == 4) return 1;   // (spills: vy_dec_attn_out)
+  else hipLaunchKernelGGL((dec_attn_kernel<DH, NW, 12, NT, R, PROJ>), grid, block, 0, st, a);
   return 0;
 }
 
