@@ -133,21 +133,7 @@ def roofline_probe(cfg, B, L, dev):
     t_blk = event_time_us(block, 10, st)
     f_gemm = 24.0 * d * d * M
     f_blk = block_flops_per_token(d, L) * M
-    # HBM-side bytes per launch come from a rocprofv3 --pmc run of the same four launches (rocprofv3 cannot wrap
-    # this process from the inside): tools/regen_profiles.sh writes profiles/rNN_gemm_pmc.json every round; the
-    # newest one is reported, with its name
-    traffic, traffic_file, alg_bytes = None, None, None
-    import glob
-    for fn in sorted(glob.glob(os.path.join(ROOT, "profiles", "r*_gemm_pmc.json")), reverse=True):
-        try:
-            with open(fn) as f:
-                j = json.load(f)
-            traffic = round(j["avg_hbm_bytes_per_launch"])
-            alg_bytes = round(j.get("algorithmic_bytes_per_launch", 0)) or None
-            traffic_file = os.path.relpath(fn, ROOT)
-            break
-        except (OSError, KeyError, ValueError):
-            continue
+    traffic, alg_bytes, traffic_file = product_traffic()
     return {
         "bound": "mfma", "kernel": "gemm_nt_bf16_m16_kernel<256,192> / <256,256> (4 launches of one layer: qkv+rope, out+res, "
                                    "ffn1+gelu, ffn2+res)",
@@ -161,6 +147,23 @@ def roofline_probe(cfg, B, L, dev):
                           "frac": round(f_blk / t_blk * 1e-6 / PEAK_BF16_TFLOPS, 4),
                           "flops": f_blk, "convention": "24 d^2 + 2 S d per token (causal)"},
     }
+
+
+def product_traffic():
+    """HBM-side and algorithmic bytes of a launch of roofline_probe's products, and the file that has them: counted by rocprofv3 --pmc runs of
+    tools/roofline_probe.py (it cannot wrap this process from the inside).  Nothing where the library has other kernels than those counted."""
+    from vyomai_amd import _lib
+    fn = os.path.join("profiles", "gemm_pmc.json")
+    try:
+        with open(os.path.join(ROOT, fn)) as f:
+            j = json.load(f)
+        with open(_lib.LIB_PATH, "rb") as f:
+            lib = f.read()
+        if j["kernels"] and all(name.encode() in lib for name in j["kernels"]):
+            return round(j["avg_hbm_bytes_per_launch"]), round(j["algorithmic_bytes_per_launch"]), fn
+    except (OSError, KeyError, ValueError):
+        pass
+    return None, None, None
 
 
 def measured_ceilings(dev):

@@ -286,6 +286,20 @@ def test_exchanged_weight_gradients_go_out_layer_by_layer(monkeypatch):
     assert launches(False) == [9, 9, 2]
 
 
+def test_bench_reports_bytes_of_its_own_kernels_alone(monkeypatch, tmp_path):
+    """roofline's bytes a launch were counted in another run: they are those of kernels that the library has, or none."""
+    import json
+    import bench
+    traffic, algorithmic, fn = bench.product_traffic()
+    assert traffic >= algorithmic > 0 and fn == os.path.join("profiles", "gemm_pmc.json")
+    counted = json.load(open(os.path.join(bench.ROOT, fn)))
+    counted["kernels"]["gemm_of_an_older_library"] = counted["kernels"].popitem()[1]
+    (tmp_path / "profiles").mkdir()
+    (tmp_path / fn).write_text(json.dumps(counted))
+    monkeypatch.setattr(bench, "ROOT", str(tmp_path))
+    assert bench.product_traffic() == (None, None, None)
+
+
 def test_bench_starts_its_own_ranks_and_never_misreports_n_gpus():
     """`python bench.py --gpus N` without a launcher used to run ONE rank and print n_gpus: 1.  Now it starts
     the N ranks itself (a child torch.distributed.run), and refuses a world size that differs from --gpus."""

@@ -28,8 +28,8 @@ dirs = [os.path.join(src, d) for d in ("pmc_fetch", "pmc_write", "pmc_hit")]
 if all(os.path.isdir(d) for d in dirs):
     out = subprocess.run([sys.executable, os.path.join(root, "tools", "gemm_pmc_json.py")] + dirs, capture_output=True, text=True)
     if out.returncode == 0:
-        open(os.path.join(dst, f"{R}_gemm_pmc.json"), "w").write(out.stdout)
-        print("wrote", f"{R}_gemm_pmc.json")
+        open(os.path.join(dst, "gemm_pmc.json"), "w").write(out.stdout)
+        print("wrote", "gemm_pmc.json")
     else:
         print(out.stderr[-2000:])
 tl = os.path.join(src, "decode_timeline.log")

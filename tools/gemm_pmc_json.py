@@ -1,4 +1,4 @@
-"""profiles/r01_gemm_pmc.json from three rocprofv3 --pmc passes over tools/roofline_probe.py:
+"""profiles/gemm_pmc.json from three rocprofv3 --pmc passes over tools/roofline_probe.py:
 
     python tools/gemm_pmc_json.py <dir FETCH_SIZE> <dir WRITE_SIZE> <dir TCC_HIT_sum TCC_MISS_sum>
 

@@ -281,7 +281,8 @@ __device__ __forceinline__ int xcd_remap(int bid, int nwg) {
 // 16 to 64 column tiles whose bands are far beyond L2, or that do not divide into bands: an XCD's run walks strips of up to STRIP row panels
 // column by column, so that its 32 CUs share 6 panels of X and 5 or 6 of W, not one panel and 32 -- what a stage brings in from beyond
 // L2 is what bounds it.  K = 2048: 8192 x 16384 510 -> 470 us, 2500 x 16384 182 -> 165, 12608 x 6144 301 -> 282, 1665 x 4096 38.4 -> 36.3;
-// 6300 x 8192, K = 1024 125.6 -> 112.3.  (Level where bands reach up to 12 MB, 8192 x 4096 and 6144; with 12 column tiles or fewer a run is as
+// 6300 x 8192, K = 1024 125.6 -> 112.3; what leaves L2 for them falls from 2215 MB to 814, 826 to 274, 1079 to 522 and 512 to 187
+// (101, 77, 77 and 30 MB of operands; profiles/product_strips_pmc.txt).  (Level where bands reach up to 12 MB, 8192 x 4096 and 6144; with 12 column tiles or fewer a run is as
 // square by rows; the vocabulary's 197 from 8 % slower to 5 % faster.  Strips of 4 panels 0.5 % behind 6, of 8 2 %.)
 constexpr int STRIP = 6;
 __device__ __forceinline__ void tile_of(int bid, int nwg, int tiles_n, int64_t w_panel, int& tile_m, int& tile_n) {
