@@ -46,6 +46,18 @@ def test_refused_on_the_host():
         _lib.call("vy_layernorm_sums", ref, 1, None)
 
 
+def test_backward_refuses_other_factors():
+    """Of what is there, all or nothing is kept; without gradients to add to as well."""
+    import ctypes as C
+    from vyomai_amd import _lib
+    buf = (C.c_char * 256)()
+    a = (C.addressof(buf) + 63) // 64 * 64
+    for grads in ((None, None), (a, a)):
+        for beta in (0.5, -1.0, float("nan")):
+            with pytest.raises(_lib.VyomHipError, match="beta must be 0 or 1"):
+                _lib.call("vy_layernorm_bwd", a, 8, a, 8, a, a, a, a, 8, *grads, beta, a, 1, 8, _lib.dtype_code(BF), None)
+
+
 def test_when_sums_go_out(monkeypatch):
     """With the weight gradients of their layers, sixteen at the most; on another stream, or exchanged, at once; never reported ready before."""
     from vyomai_amd import autograd_train as AT

@@ -754,8 +754,6 @@ int ln_bwd_dispatch(const void* dy, int64_t lddy, const void* x, int64_t ldx, co
   if (beta == 0.f) {
     if (dgamma && hipMemsetAsync(dgamma, 0, N * sizeof(float), st) != hipSuccess) VY_FAIL(VY_ERR_LAUNCH, "vy_layernorm_bwd: memset failed");
     if (dbeta && hipMemsetAsync(dbeta, 0, N * sizeof(float), st) != hipSuccess) VY_FAIL(VY_ERR_LAUNCH, "vy_layernorm_bwd: memset failed");
-  } else if (beta != 1.f) {
-    VY_FAIL(VY_ERR_ARG, "vy_layernorm_bwd: beta must be 0 or 1");
   }
   Colsums one{};
   one.g[0] = {ws, dgamma, dbeta, WB, (int)N};
@@ -852,6 +850,7 @@ extern "C" int vy_layernorm_bwd(const void* dy, int64_t lddy, const void* x, int
                                 void* stream) {
   if (!dy || !x || !gamma || !mean || !rstd || !dx || !ws || M <= 0 || N <= 0)
     VY_FAIL(VY_ERR_ARG, "vy_layernorm_bwd: bad arguments");
+  if (beta != 0.f && beta != 1.f) VY_FAIL(VY_ERR_ARG, "vy_layernorm_bwd: beta must be 0 or 1");
   hipStream_t st = (hipStream_t)stream;
   if (dtype == VY_BF16) return ln_bwd_dispatch<bf16>(dy, lddy, x, ldx, gamma, mean, rstd, dx, lddx, dgamma, dbeta, beta, ws, M, N, st);
   if (dtype == VY_F32) return ln_bwd_dispatch<float>(dy, lddy, x, ldx, gamma, mean, rstd, dx, lddx, dgamma, dbeta, beta, ws, M, N, st);
