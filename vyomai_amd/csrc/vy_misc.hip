@@ -20,9 +20,9 @@ namespace {
 // ---- LayerNorm forward: one wave per row, CH chunks per lane -------------------------------
 // mean, then variance about the mean (two reductions on registers): the same two-pass
 // formulation as aten's CPU LayerNorm closely enough for 1e-6 agreement.
-// Weight and bias are requested with the row, not behind the reductions (512 rows of 768: 3.7 -> 3.2 us, an encoder of 4 x 128 tokens
-// 708 -> 699 us); the rows, which only this launch and perhaps the backward pass read, pass by the caches (30500 rows 19.8 -> 19.6 us, the encoder
-// behind them 7452 -> 7419: the products around find more of their operands).
+// Weight and bias are requested with the row, not behind the reductions (back to back, 64 rows of 768 3.03 -> 2.81 us, 512 rows
+// 3.07 -> 2.91; an encoder of 4 x 128 tokens is level, 710 us); the rows, which only this launch and perhaps the backward pass read, pass by the
+// caches (30500 rows 20.2 -> 19.6 us).
 template <typename T, int CH>
 __global__ __launch_bounds__(256) void layernorm_fwd_kernel(const T* __restrict__ x, int64_t ldx,
                                                             const T* __restrict__ gamma,
